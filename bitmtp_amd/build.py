@@ -1,5 +1,5 @@
-"""Builds the gfx950 shared libraries of this package with hipcc, in-tree, and the PyTorch
-operator library on top of them with g++.
+"""Builds the gfx950 shared libraries of this package with hipcc, in-tree, and the host
+libraries on top of them (PyTorch operators, Python extension) with g++.
 
     python -m bitmtp_amd.build            # build what is missing or out of date
     python -m bitmtp_amd.build --force    # rebuild everything
@@ -82,22 +82,24 @@ def build_all(force: bool = False, verbose: bool = True) -> list[str]:
     return [lib_path(s) for s in TARGETS if os.path.exists(lib_path(s))]
 
 
-# ---- the PyTorch operator library (host code only, g++) ---------------------------------
+# ---- host libraries on top of them (g++, no device code) -----------------------------------
 TORCH_OPS_SOURCE = "torch_ops.cpp"
 TORCH_OPS_LIB = os.path.join("torch_ops", "libbonsai_torch.so")
+PY_OPS_SOURCE = "py_ops.cpp"
+PY_OPS_LIB = os.path.join("torch_ops", "_bonsai_py.so")
 
 
 def torch_ops_path() -> str:
     return os.path.join(HERE, TORCH_OPS_LIB)
 
 
-def build_torch_ops(force: bool = False, verbose: bool = True) -> str:
-    """Compiles csrc/torch_ops.cpp against the installed PyTorch and links it to the three C-ABI
-    libraries it calls (found at run time next to it through $ORIGIN).  No device code."""
-    out = torch_ops_path()
-    if not force and not _stale(out):
-        return out
-    build_all(verbose=verbose)  # the libraries it links to
+def py_ops_path() -> str:
+    return os.path.join(HERE, PY_OPS_LIB)
+
+
+def _build_host(source: str, out: str, extra: list[str]) -> None:
+    """Compiles a host source against the installed PyTorch and links it to the three C-ABI
+    libraries it calls (found at run time next to it through $ORIGIN)."""
     import torch
     tdir = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
@@ -107,16 +109,30 @@ def build_torch_ops(force: bool = False, verbose: bool = True) -> str:
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include", f"-I{rocm}/include",
-           os.path.join(CSRC, TORCH_OPS_SOURCE), "-o", out,
-           f"-L{tdir}/lib", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip"]
+           os.path.join(CSRC, source), "-o", out,
+           f"-L{tdir}/lib", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip"] + extra
     cmd += [f"-L{d}" for d in libdirs] + ["-lbonsai_t2", "-lbonsai_q1", "-lbonsai_actq",
             "-Wl,-rpath,$ORIGIN/../t2g128_kernels:$ORIGIN/../q1g128_kernels:$ORIGIN/../act_quant"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
-        raise RuntimeError(f"g++ failed for {TORCH_OPS_SOURCE}:\n{proc.stdout}")
+        raise RuntimeError(f"g++ failed for {source}:\n{proc.stdout}")
+
+
+def build_torch_ops(force: bool = False, verbose: bool = True) -> str:
+    """Builds the registered PyTorch operators (csrc/torch_ops.cpp) and the Python extension the
+    operator layer calls (csrc/py_ops.cpp); returns the path of the former."""
+    import sysconfig
+    build_all(verbose=verbose)  # the libraries they link to
+    todo = [(src, out, extra) for src, out, extra in (
+        (TORCH_OPS_SOURCE, torch_ops_path(), []),
+        (PY_OPS_SOURCE, py_ops_path(), [f"-I{sysconfig.get_paths()['include']}", "-ltorch_python"]))
+        if force or _stale(out)]
+    with ThreadPoolExecutor(max_workers=max(1, len(todo))) as pool:
+        list(pool.map(lambda t: _build_host(*t), todo))
     if verbose:
-        print(f"[bitmtp_amd.build] built {os.path.relpath(out, HERE)}")
-    return out
+        for _, out, _ in todo:
+            print(f"[bitmtp_amd.build] built {os.path.relpath(out, HERE)}")
+    return torch_ops_path()
 
 
 if __name__ == "__main__":

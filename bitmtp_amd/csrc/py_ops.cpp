@@ -1,0 +1,307 @@
+// _bonsai_py: the operators of bitmtp_amd/ops.py from the tensors' handles to the C ABI without
+// Python in between.  A decode-width projection runs 3-8 us on the GPU; with checks, allocation,
+// device guard and ctypes conversion in Python a call cost 11.4 us of host time (37.9 us for a
+// grouped call of seven, 46.9 us for the five launches of an MLP), so back-to-back calls were
+// bound by the host.  Here a call is one allocation per result plus the launch.
+//
+// Every function returns None when its operands are anything but the plain case (tensor
+// subclasses, other devices, dtypes or layouts, shapes the checks refuse, an active dispatch
+// mode): the caller then takes its own checked path, which raises the error messages of the
+// operator contract.  Nothing is launched before that decision.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <optional>
+#include <string>
+
+#include "../../include/bonsai_gemv.h"
+
+namespace {
+
+constexpr int64_t kMaxOutputs = 1 << 30, kMaxK = 65536;  // the native launchers' limits
+
+// The tensor behind a Python object that is exactly torch.Tensor (or a Parameter), else null.
+const at::Tensor *plain(PyObject *o) {
+    return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr;
+}
+
+bool on_gpu(const at::Tensor &t, c10::Device dev) {
+    return t.is_cuda() && t.device() == dev && t.is_contiguous();
+}
+
+at::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType dtype, c10::Device dev) {
+    return at::Tensor(at::detail::empty_cuda(sizes, dtype, dev, std::nullopt));
+}
+
+// The current device moved to `dev` for the call, where it is another one.
+struct OnDevice {
+    c10::OptionalDeviceGuard guard;
+    explicit OnDevice(c10::Device dev) {
+        if (c10::hip::current_device() != dev.index()) guard.reset_device(dev);
+    }
+    void *stream() const { return c10::hip::getCurrentHIPStream().stream(); }
+};
+
+struct ReleaseGil {
+    PyThreadState *state = PyEval_SaveThread();
+    ~ReleaseGil() { PyEval_RestoreThread(state); }
+};
+
+struct Problem {
+    int64_t m, n, k;
+    bool f16_scales;
+};
+
+// The operand checks of a packed projection (bf16 result); false = take the caller's path.
+bool gemv_ok(int bits, const at::Tensor &a, const at::Tensor &b, const at::Tensor &s, const at::Tensor &ws,
+             bool allow_f16_scales, Problem &p) {
+    const int64_t rank = a.dim();
+    if ((rank != 2 && rank != 3) || b.dim() != 2 || ws.dim() != 2 || s.dim() < 1) return false;
+    const c10::Device dev = a.device();
+    if (!on_gpu(a, dev) || !on_gpu(b, dev) || !on_gpu(s, dev) || !on_gpu(ws, dev)) return false;
+    if (a.scalar_type() != at::kChar || b.scalar_type() != at::kChar || s.scalar_type() != at::kFloat) return false;
+    p.f16_scales = ws.scalar_type() == at::kHalf;
+    if (!(ws.scalar_type() == at::kBFloat16 || (allow_f16_scales && p.f16_scales))) return false;
+    p.k = a.size(-1);
+    p.n = b.size(0);
+    if (p.k < 128 || p.k % 128 != 0 || p.k > kMaxK || p.n < 1 || b.size(1) * (8 / bits) != p.k) return false;
+    p.m = a.numel() / p.k;
+    if (p.m < 1 || p.m * p.n > kMaxOutputs) return false;
+    return ws.size(0) == p.n && ws.size(1) == p.k / 128 && s.size(-1) == 1 && s.numel() == p.m;
+}
+
+PyObject *fail(const std::string &what) {
+    PyErr_SetString(PyExc_RuntimeError, what.c_str());
+    return nullptr;
+}
+
+const char *kind_name(int bits) { return bits == 2 ? "t2g128" : "q1"; }
+
+// linear(bits, a_int8, b_packed, s, ws, allow_f16_scales) -> bf16 [.., N] or None
+PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 6 || c10::impl::dispatch_mode_enabled()) Py_RETURN_NONE;
+    const int bits = (int)PyLong_AsLong(args[0]);
+    const at::Tensor *a = plain(args[1]), *b = plain(args[2]), *s = plain(args[3]), *ws = plain(args[4]);
+    Problem p;
+    if (!a || !b || !s || !ws || !gemv_ok(bits, *a, *b, *s, *ws, args[5] == Py_True, p)) Py_RETURN_NONE;
+    if (args[5] == Py_True && a->dim() != 2) Py_RETURN_NONE;
+    int64_t shape[3] = {a->size(0), p.n, p.n};
+    if (a->dim() == 3) shape[1] = a->size(1);
+    at::Tensor out = new_tensor(at::IntArrayRef(shape, a->dim()), at::kBFloat16, a->device());
+    const OnDevice on(a->device());
+    int rc;
+    {
+        ReleaseGil unlocked;
+        rc = (bits == 2 ? t2g128_gemv_ex : q1g128_gemv_ex)(
+            static_cast<const int8_t *>(a->const_data_ptr()), static_cast<const uint8_t *>(b->const_data_ptr()),
+            out.mutable_data_ptr(), static_cast<const float *>(s->const_data_ptr()), ws->const_data_ptr(), (int)p.m,
+            (int)p.n, (int)p.k, BONSAI_OUT_BF16, p.f16_scales ? BONSAI_SCALE_F16 : BONSAI_SCALE_BF16, on.stream());
+    }
+    if (rc != 0)
+        return fail(std::string(kind_name(bits)) + ": native launch failed with status " + std::to_string(rc) + " (M=" +
+                    std::to_string(p.m) + ", N=" + std::to_string(p.n) + ", K=" + std::to_string(p.k) + ")");
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// grouped(bits, problems) -> list of bf16 [M_i, N_i] or None; problems: a list or tuple of 4-tuples
+PyObject *grouped(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 2 || c10::impl::dispatch_mode_enabled()) Py_RETURN_NONE;
+    const int bits = (int)PyLong_AsLong(args[0]);
+    PyObject *seq = args[1];
+    if (!PyList_CheckExact(seq) && !PyTuple_CheckExact(seq)) Py_RETURN_NONE;
+    const Py_ssize_t count = PySequence_Fast_GET_SIZE(seq);
+    if (count < 1 || count > BONSAI_GROUPED_MAX) Py_RETURN_NONE;
+    bonsai_gemv_desc descs[BONSAI_GROUPED_MAX];
+    const at::Tensor *first = nullptr;
+    bool f16 = false;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject *t = PySequence_Fast_GET_ITEM(seq, i);
+        if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 4) Py_RETURN_NONE;
+        const at::Tensor *a = plain(PyTuple_GET_ITEM(t, 0)), *b = plain(PyTuple_GET_ITEM(t, 1)),
+                         *s = plain(PyTuple_GET_ITEM(t, 2)), *ws = plain(PyTuple_GET_ITEM(t, 3));
+        Problem p;
+        if (!a || !b || !s || !ws || a->dim() != 2 || !gemv_ok(bits, *a, *b, *s, *ws, true, p)) Py_RETURN_NONE;
+        if (i == 0) {
+            first = a;
+            f16 = p.f16_scales;
+        } else if (a->device() != first->device() || p.f16_scales != f16) {
+            Py_RETURN_NONE;
+        }
+        descs[i] = {static_cast<const int8_t *>(a->const_data_ptr()), static_cast<const uint8_t *>(b->const_data_ptr()),
+                    nullptr, static_cast<const float *>(s->const_data_ptr()), ws->const_data_ptr(), (int32_t)p.m,
+                    (int32_t)p.n, (int32_t)p.k, 0};
+    }
+    PyObject *list = PyList_New(count);
+    if (list == nullptr) return nullptr;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        const int64_t shape[2] = {descs[i].M, descs[i].N};
+        at::Tensor out = new_tensor(at::IntArrayRef(shape, 2), at::kBFloat16, first->device());
+        descs[i].out = out.mutable_data_ptr();
+        PyList_SET_ITEM(list, i, THPVariable_Wrap(std::move(out)));
+    }
+    const OnDevice on(first->device());
+    int rc;
+    {
+        ReleaseGil unlocked;
+        rc = (bits == 2 ? t2g128_gemv_grouped : q1g128_gemv_grouped)(
+            descs, (int)count, BONSAI_OUT_BF16, f16 ? BONSAI_SCALE_F16 : BONSAI_SCALE_BF16, on.stream());
+    }
+    if (rc != 0) {
+        Py_DECREF(list);
+        return fail(std::string(kind_name(bits)) + ": grouped native launch failed with status " + std::to_string(rc));
+    }
+    return list;
+    END_HANDLE_TH_ERRORS
+}
+
+// q int8 [.., K] and s fp32 [.., 1] of a row-wise quantiser over `x`, K columns kept of each row
+struct Quantised {
+    at::Tensor q, s;
+    Quantised(const at::Tensor &x, int64_t k) {
+        c10::SmallVector<int64_t, 4> shape(x.sizes().begin(), x.sizes().end());
+        shape.back() = k;
+        q = new_tensor(shape, at::kChar, x.device());
+        shape.back() = 1;
+        s = new_tensor(shape, at::kFloat, x.device());
+    }
+    int8_t *qp() { return static_cast<int8_t *>(q.mutable_data_ptr()); }
+    float *sp() { return static_cast<float *>(s.mutable_data_ptr()); }
+};
+
+PyObject *tuple2(at::Tensor a, at::Tensor b) {
+    PyObject *t = PyTuple_New(2);
+    if (t == nullptr) return nullptr;
+    PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(a)));
+    PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(b)));
+    return t;
+}
+
+bool rows_ok(const at::Tensor &x, int64_t multiple, int64_t &m, int64_t &k) {
+    if (x.dim() < 1 || !x.is_cuda() || !x.is_contiguous()) return false;
+    k = x.size(-1);
+    if (k < 1 || k % multiple != 0 || k > (1 << 30)) return false;
+    m = x.numel() / k;
+    return m >= 1 && m <= (1 << 30);
+}
+
+// quant_input(x) -> (q, s) or None
+PyObject *quant_input(PyObject *, PyObject *x_obj) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = plain(x_obj);
+    int64_t m, k;
+    if (!x || c10::impl::dispatch_mode_enabled() || !rows_ok(*x, 8, m, k)) Py_RETURN_NONE;
+    int kind;
+    switch (x->scalar_type()) {
+        case at::kBFloat16: kind = BONSAI_X_BF16; break;
+        case at::kHalf: kind = BONSAI_X_F16; break;
+        case at::kFloat: kind = BONSAI_X_F32; break;
+        default: Py_RETURN_NONE;
+    }
+    Quantised out(*x, k);
+    const OnDevice on(x->device());
+    int rc;
+    {
+        ReleaseGil unlocked;
+        rc = bonsai_act_quant_int8(x->const_data_ptr(), kind, out.qp(), out.sp(), (int)m, (int)k, on.stream());
+    }
+    if (rc != 0) return fail("quant_input: native launch failed with status " + std::to_string(rc));
+    return tuple2(std::move(out.q), std::move(out.s));
+    END_HANDLE_TH_ERRORS
+}
+
+bool bf16_on(const at::Tensor &t, c10::Device dev) { return t.scalar_type() == at::kBFloat16 && on_gpu(t, dev); }
+
+// norm_quant(x, w, eps) -> (q, s) or None
+PyObject *norm_quant(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 3 || c10::impl::dispatch_mode_enabled() || !PyFloat_CheckExact(args[2])) Py_RETURN_NONE;
+    const at::Tensor *x = plain(args[0]), *w = plain(args[1]);
+    int64_t m, k;
+    if (!x || !w || !rows_ok(*x, 8, m, k) || !bf16_on(*x, x->device()) || !bf16_on(*w, x->device()) || w->dim() != 1 ||
+        w->size(0) != k)
+        Py_RETURN_NONE;
+    Quantised out(*x, k);
+    const OnDevice on(x->device());
+    int rc;
+    {
+        ReleaseGil unlocked;
+        rc = bonsai_rmsnorm_quant_int8(x->const_data_ptr(), w->const_data_ptr(), (float)PyFloat_AS_DOUBLE(args[2]),
+                                       out.qp(), out.sp(), (int)m, (int)k, on.stream());
+    }
+    if (rc != 0) return fail("fused_norm_quant: native launch failed with status " + std::to_string(rc));
+    return tuple2(std::move(out.q), std::move(out.s));
+    END_HANDLE_TH_ERRORS
+}
+
+// add_norm_quant(x, residual, w, eps) -> (h, q, s) or None
+PyObject *add_norm_quant(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 4 || c10::impl::dispatch_mode_enabled() || !PyFloat_CheckExact(args[3])) Py_RETURN_NONE;
+    const at::Tensor *x = plain(args[0]), *r = plain(args[1]), *w = plain(args[2]);
+    int64_t m, k;
+    if (!x || !r || !w || !rows_ok(*x, 8, m, k) || !bf16_on(*x, x->device()) || !bf16_on(*r, x->device()) ||
+        !bf16_on(*w, x->device()) || r->sizes() != x->sizes() || w->dim() != 1 || w->size(0) != k)
+        Py_RETURN_NONE;
+    at::Tensor h = new_tensor(x->sizes(), at::kBFloat16, x->device());
+    Quantised out(*x, k);
+    const OnDevice on(x->device());
+    int rc;
+    {
+        ReleaseGil unlocked;
+        rc = bonsai_add_rmsnorm_quant_int8(x->const_data_ptr(), r->const_data_ptr(), w->const_data_ptr(),
+                                           (float)PyFloat_AS_DOUBLE(args[3]), h.mutable_data_ptr(), out.qp(), out.sp(),
+                                           (int)m, (int)k, on.stream());
+    }
+    if (rc != 0) return fail("fused_add_norm_quant: native launch failed with status " + std::to_string(rc));
+    PyObject *t = PyTuple_New(3);
+    if (t == nullptr) return nullptr;
+    PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(h)));
+    PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(out.q)));
+    PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(std::move(out.s)));
+    return t;
+    END_HANDLE_TH_ERRORS
+}
+
+// silu_mul_quant(gate_up) -> (q, s) or None
+PyObject *silu_mul_quant(PyObject *, PyObject *x_obj) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = plain(x_obj);
+    int64_t m, f2;
+    if (!x || c10::impl::dispatch_mode_enabled() || !rows_ok(*x, 16, m, f2) || !bf16_on(*x, x->device())) Py_RETURN_NONE;
+    Quantised out(*x, f2 / 2);
+    const OnDevice on(x->device());
+    int rc;
+    {
+        ReleaseGil unlocked;
+        rc = bonsai_silu_mul_quant_int8(x->const_data_ptr(), out.qp(), out.sp(), (int)m, (int)(f2 / 2), on.stream());
+    }
+    if (rc != 0) return fail("silu_mul_quant: native launch failed with status " + std::to_string(rc));
+    return tuple2(std::move(out.q), std::move(out.s));
+    END_HANDLE_TH_ERRORS
+}
+
+#define FASTCALL(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)), METH_FASTCALL
+PyMethodDef kMethods[] = {
+    {"linear", FASTCALL(linear), "(bits, a_int8, b_packed, s, ws, allow_f16_scales) -> bf16 or None"},
+    {"grouped", FASTCALL(grouped), "(bits, [(a_int8, b_packed, s, ws), ...]) -> [bf16, ...] or None"},
+    {"quant_input", quant_input, METH_O, "(x) -> (q, s) or None"},
+    {"norm_quant", FASTCALL(norm_quant), "(x, w, eps) -> (q, s) or None"},
+    {"add_norm_quant", FASTCALL(add_norm_quant), "(x, residual, w, eps) -> (h, q, s) or None"},
+    {"silu_mul_quant", silu_mul_quant, METH_O, "(gate_up) -> (q, s) or None"},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_bonsai_py", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__bonsai_py(void) { return PyModule_Create(&kModule); }

@@ -8,11 +8,13 @@ There is no CPU or PyTorch fallback: if a library is missing the loaders raise.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from typing import List, Optional, Sequence, Tuple
 
 import torch
 
+from . import contracts
 from .contracts import require_kernel_shape
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -195,6 +197,31 @@ def load_torch_ops():
     return torch.ops.bonsai
 
 
+# The operators below that take plain contiguous GPU tensors go through csrc/py_ops.cpp, which
+# checks, allocates and launches without Python in between (an operator call is a few
+# microseconds of GPU work; the checked ctypes path costs 11 us of host time).  It declines
+# anything but the plain case, and the checked path then decides and words the error.  It is
+# loaded by the first call that path has accepted, so a refused call still loads nothing.
+_native = None
+
+
+def py_ops_lib_path() -> str:
+    return os.path.join(_HERE, "torch_ops", "_bonsai_py.so")
+
+
+def _load_native() -> None:
+    global _native
+    so = py_ops_lib_path()
+    if not os.path.exists(so):
+        raise RuntimeError(
+            f"{so} is missing: build it with `python -m bitmtp_amd.build` "
+            "(there is no fallback implementation)")
+    spec = importlib.util.spec_from_file_location("_bonsai_py", so)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    _native = module
+
+
 def t2_lib() -> ctypes.CDLL:
     if _t2_lib is None:
         load_t2_kernel()
@@ -297,6 +324,10 @@ def t2g128_int8xint2_linear(a_int8: torch.Tensor, b_packed: torch.Tensor, s: tor
                             ws: torch.Tensor) -> torch.Tensor:
     """``[..., K] int8 x [N, K/4] packed ternary -> [..., N] bf16`` on the current
     stream (reference: model.py:222-256)."""
+    if _native is not None and not contracts._strict:
+        out = _native.linear(2, a_int8, b_packed, s, ws, False)
+        if out is not None:
+            return out
     _validate_packed_inputs(a_int8, b_packed, s, ws, kind="t2g128", bits=2,
                             activation_dtype=torch.int8)
     n, k = b_packed.shape[0], b_packed.shape[1] * 4
@@ -310,6 +341,8 @@ def t2g128_int8xint2_linear(a_int8: torch.Tensor, b_packed: torch.Tensor, s: tor
                                 m, n, k, OUT_BF16, SCALE_BF16, _stream(a_int8.device))
     if rc != 0:
         raise RuntimeError(f"t2g128: native launch failed with status {rc} (M={m}, N={n}, K={k})")
+    if _native is None:
+        _load_native()
     return out
 
 
@@ -317,6 +350,10 @@ def q1g128_int8xint1_linear(a_int8: torch.Tensor, b_packed: torch.Tensor, s: tor
                             ws: torch.Tensor) -> torch.Tensor:
     """``[..., K] int8 x [N, K/8] packed signs -> [..., N] bf16`` (reference:
     model.py:118-153)."""
+    if _native is not None and not contracts._strict:
+        out = _native.linear(1, a_int8, b_packed, s, ws, False)
+        if out is not None:
+            return out
     _validate_packed_inputs(a_int8, b_packed, s, ws, kind="q1", bits=1,
                             activation_dtype=torch.int8)
     n, k = b_packed.shape[0], b_packed.shape[1] * 8
@@ -328,6 +365,8 @@ def q1g128_int8xint1_linear(a_int8: torch.Tensor, b_packed: torch.Tensor, s: tor
                                 m, n, k, OUT_BF16, SCALE_BF16, _stream(a_int8.device))
     if rc != 0:
         raise RuntimeError(f"q1: native launch failed with status {rc} (M={m}, N={n}, K={k})")
+    if _native is None:
+        _load_native()
     return out
 
 
@@ -369,6 +408,11 @@ def packed_gemv_ex(a_int8: torch.Tensor, b_packed: torch.Tensor, s: Optional[tor
     before the bf16 rounding, or the exact int32 group sums ``[M,N,K/128]``.
     ``ws`` may be bf16 or fp16.  Rank-2 activations only.  ``out`` supplies a preallocated
     result (so that a captured graph allocates nothing)."""
+    if _native is not None and out_kind == OUT_BF16 and out is None and not contracts._strict \
+            and (bits == 1 or bits == 2):
+        got = _native.linear(bits, a_int8, b_packed, s, ws, True)
+        if got is not None:
+            return got
     if bits not in (1, 2):
         raise ValueError("bits must be 1 (Q1) or 2 (T2)")
     kind = "t2g128" if bits == 2 else "q1"
@@ -402,6 +446,8 @@ def packed_gemv_ex(a_int8: torch.Tensor, b_packed: torch.Tensor, s: Optional[tor
                 scale_kind, _stream(dev))
     if rc != 0:
         raise RuntimeError(f"{kind}: native launch failed with status {rc} (M={m}, N={n}, K={k})")
+    if _native is None:
+        _load_native()
     return out
 
 
@@ -532,6 +578,11 @@ def packed_gemv_grouped(problems: Sequence[Tuple[torch.Tensor, torch.Tensor, Opt
     calls reach the same kernel with the same geometry (otherwise equal within the tolerance
     of the fp32 summation order).  ``outs`` supplies preallocated outputs (so that a captured graph
     allocates nothing); otherwise fresh tensors are returned."""
+    if _native is not None and out_kind == OUT_BF16 and outs is None and not contracts._strict \
+            and (bits == 1 or bits == 2):
+        got = _native.grouped(bits, problems)
+        if got is not None:
+            return got
     if bits not in (1, 2):
         raise ValueError("bits must be 1 (Q1) or 2 (T2)")
     if not 1 <= len(problems) <= GROUPED_MAX:
@@ -578,6 +629,8 @@ def packed_gemv_grouped(problems: Sequence[Tuple[torch.Tensor, torch.Tensor, Opt
         rc = fn(descs, len(problems), out_kind, scale_kind, _stream(dev))
     if rc != 0:
         raise RuntimeError(f"{kind}: grouped native launch failed with status {rc}")
+    if _native is None:
+        _load_native()
     return results
 
 
@@ -586,6 +639,10 @@ def quant_input(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     s fp32 [..., 1])`` with ``s = reciprocal(clamp_min(absmax, 1e-5)) * 127`` -- what
     PyTorch computes for the reference's ``127.0 / absmax.clamp_(min=1e-5)``
     (model.py:632-636)."""
+    if _native is not None:
+        got = _native.quant_input(x)
+        if got is not None:
+            return got
     if x.dtype not in _X_KIND:
         raise RuntimeError("quant_input: activation must be bfloat16, float16 or float32")
     if not (x.is_cuda and x.is_contiguous()) or x.dim() < 1:
@@ -603,6 +660,8 @@ def quant_input(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
                                               _stream(x.device))
     if rc != 0:
         raise RuntimeError(f"quant_input: native launch failed with status {rc}")
+    if _native is None:
+        _load_native()
     return q, s
 
 
@@ -615,6 +674,10 @@ def _check_bf16_rows(name: str, *tensors: torch.Tensor) -> None:
 def fused_norm_quant(x: torch.Tensor, w: torch.Tensor, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """RMSNorm then per-token INT8 quantisation: ``(q int8 [..., K], s fp32 [..., 1])``
     (reference: ``_fused_norm_quant``, model.py:307-319)."""
+    if _native is not None:
+        got = _native.norm_quant(x, w, eps)
+        if got is not None:
+            return got
     _check_bf16_rows("fused_norm_quant", x, w)
     k = x.shape[-1]
     if w.shape != (k,) or k % 8 != 0:
@@ -627,6 +690,8 @@ def fused_norm_quant(x: torch.Tensor, w: torch.Tensor, eps: float) -> Tuple[torc
                                                   _stream(x.device))
     if rc != 0:
         raise RuntimeError(f"fused_norm_quant: native launch failed with status {rc}")
+    if _native is None:
+        _load_native()
     return q, s
 
 
@@ -634,6 +699,10 @@ def fused_add_norm_quant(x: torch.Tensor, residual: torch.Tensor, w: torch.Tenso
                          eps: float) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``h = x + residual``; returns ``(h, q, s)`` with ``(q, s)`` the quantised RMSNorm of h
     (reference: ``_fused_add_norm_quant``, model.py:322-336)."""
+    if _native is not None:
+        got = _native.add_norm_quant(x, residual, w, eps)
+        if got is not None:
+            return got
     _check_bf16_rows("fused_add_norm_quant", x, residual, w)
     k = x.shape[-1]
     if residual.shape != x.shape or w.shape != (k,) or k % 8 != 0:
@@ -648,6 +717,8 @@ def fused_add_norm_quant(x: torch.Tensor, residual: torch.Tensor, w: torch.Tenso
                                                       _stream(x.device))
     if rc != 0:
         raise RuntimeError(f"fused_add_norm_quant: native launch failed with status {rc}")
+    if _native is None:
+        _load_native()
     return h, q, s
 
 
@@ -676,6 +747,10 @@ def silu_mul_quant(gate_up: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """``inner = silu(gate) * up`` of a merged gate/up projection ``[..., 2F]`` followed by
     per-token quantisation: ``(q int8 [..., F], s fp32 [..., 1])`` (reference:
     model.py:1058-1061)."""
+    if _native is not None:
+        got = _native.silu_mul_quant(gate_up)
+        if got is not None:
+            return got
     _check_bf16_rows("silu_mul_quant", gate_up)
     f2 = gate_up.shape[-1]
     if f2 % 16 != 0:
@@ -689,4 +764,6 @@ def silu_mul_quant(gate_up: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
                                                    _stream(gate_up.device))
     if rc != 0:
         raise RuntimeError(f"silu_mul_quant: native launch failed with status {rc}")
+    if _native is None:
+        _load_native()
     return q, s
