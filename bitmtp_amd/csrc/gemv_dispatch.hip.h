@@ -18,12 +18,14 @@
 #include "gemv_mxl.hip.h"
 #include "gemv_mxs.hip.h"
 #include "gemv_rowreg.hip.h"
+#include "gemv_wide.hip.h"
 #include "packed_gemv.hip.h"
 
 namespace bonsai {
 
 constexpr int kDefaultMfmaMinWidth = 3;       // layer-sized matrices (dot4 wins at 1 and 2 tokens)
 constexpr int kDirectMaxRows = 16384;         // up to here the staging-free matrix-core kernel
+constexpr int kWideMinRagged = 5;             // K not a multiple of 512: the wide kernel instead of dot4
 constexpr int kLongMatrixRows = 32768;        // from here on the matrix cores pay off at M >= 2
 
 // Every kernel reads A and B with 16-byte vector loads and the scales as 16-bit words.
@@ -182,6 +184,8 @@ int init_all_kernels() {
         if (rc6 != 0) return rc6;
         const int rc7 = mxl_init_device<BITS>(st.lds_limit[dev]);
         if (rc7 != 0) return rc7;
+        const int rc8 = wide_init_device<BITS>(st.lds_limit[dev]);
+        if (rc8 != 0) return rc8;
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             cus <= 0)
@@ -348,7 +352,24 @@ int launch_grouped_mx_only(const GemvProblem &q, int out_kind, int scale_kind, i
             if (rc != -1) return rc;
         }
     }
+    if (!mx_problem_ok(q, out_kind == OUT_G32)) return -1;
     return launch_mx<BITS>(batch, nb, out_kind, scale_kind, lds_limit, n_cus, stream);
+}
+
+// K for which the lean kernel stands in for the matrix-core kernels that want whole 512-wide tiles and for
+// the dot4 kernel they leave (12288 x 1920 at nine tokens: dot4 9.2 us).
+inline bool lean_any_k(int K) { return K % 512 != 0 && K > 512; }
+
+// Blocks the wide kernel takes.  The lean kernel's 16-token tiles are ahead up to about six of its
+// workgroups per CU (12288 x 2048 at 32 tokens 7.2 us against 7.3, at 48 12.7 / 9.3; 2048 x 2048 at 128
+// 5.8 / 7.2, at 256 10.3 / 7.6; 2560 x 9728 at 128 18.4 / 20.3, at 192 26.6 / 21.2), and at a few tokens
+// over 16 also above that (19456 x 2560 at 24 tokens 9.9 / 11.9, at 32 12.9 / 12.1).  What the lean kernel
+// does not take leaves only the dot4 kernel where K is not a multiple of 512 (19000 x 2688: dot4 9.1 us at
+// four tokens, 15.5 at nine, against 10.6 at any width up to 32).
+inline bool wide_default(int M, int N, int K, int n_cus) {
+    const long lean_tiles = (long)((M + kMfmaTokens - 1) / kMfmaTokens) * ((N + 15) / 16);
+    if (K % 512 != 0 && (lean_tiles > 8L * n_cus || N > kLongMatrixRows || K < 512)) return M >= kWideMinRagged;
+    return M > 24 && lean_tiles > 6L * n_cus;
 }
 
 template <int BITS>
@@ -371,6 +392,13 @@ int launch_gemv(const int8_t *A, const uint8_t *B, void *out, const float *s, co
     const int lds_limit = st.lds_limit[dev];
 
     const MfmaTuning &mtu = mfma_tuning<BITS>();
+    if (mtu.engine == 7 || (mtu.engine == 0 && mtu.min_width <= 0 && wide_default(M, N, K, st.n_cus[dev]))) {
+        const GemvProblem q{A, B, out, s, ws, M, N, K};
+        const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % kWideVariants
+                                                           : wide_pick(M, N, K, st.n_cus[dev]);
+        const int rc = launch_wide<BITS>(v, q, out_kind, scale_kind, lds_limit, stream);
+        if (rc != -1) return rc;
+    }
     // two tokens go to the matrix cores for very long matrices and for long rows (K >= 4096: at
     // two tokens 2048 x 6144 takes 3.74 us there against 4.23 us on the dot4 kernel, 2560 x 9728
     // 4.77 against 5.91; K = 2048 and 2560 are level or slower)
@@ -403,7 +431,7 @@ int launch_gemv(const int8_t *A, const uint8_t *B, void *out, const float *s, co
     if ((mtu.engine == 4 || lean_default) && M >= min_width) {
         // the grouped kernel with a single descriptor
         const GemvProblem q{A, B, out, s, ws, M, N, K};
-        if (mx_problem_ok(q, out_kind == OUT_G32)) {
+        if (mx_problem_ok(q, out_kind == OUT_G32) || (lean_default && lean_any_k(K))) {
             const int rc = launch_grouped_mx_only<BITS>(q, out_kind, scale_kind, lds_limit, st.n_cus[dev],
                                                         stream);
             if (rc >= 0) return rc;
@@ -566,7 +594,8 @@ int launch_grouped(const GemvProblem *probs, int count, int out_kind, int scale_
         }
         // token tiles of at most 16 (the staged activations are chunked along K: they always fit)
         const int cap = q.M < kMfmaTokens ? q.M : kMfmaTokens;
-        if (q.M < min_width || !mx_problem_ok(q, out_kind == OUT_G32)) {
+        if (q.M < min_width || !mx_problem_ok(q, out_kind == OUT_G32) ||
+            (tu.row_tiles == 0 && tu.max_wgs == 0 && wide_default(q.M, q.N, q.K, st.n_cus[dev]))) {
             const int rc = launch_gemv<BITS>(q.A, q.B, q.out, q.s, q.ws, q.M, q.N, q.K, out_kind,
                                              scale_kind, stream);
             if (rc != 0) return rc;

@@ -76,10 +76,10 @@ __host__ __device__ constexpr size_t mxl_lds_bytes(int mmax, int waves) {
 // 7.6 us), so the host picks per launch.
 // G32: store the exact int32 group sums G[m][n][g] (what the matrix cores return, before any
 // scale) instead of the scaled result; the scales and multipliers are not read.
-template <int BITS, int MR, bool SF16, int W, int NB, int OCC, bool G32 = false>
-__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
-gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8, int e9,
-                int e10, int e11, int out_f32, int mmax, const MxlTable tbl) {
+// RAGGED: some problem's K is not a multiple of 512 (kernel gemv_mxl_ragged_kernel).
+template <int BITS, int MR, bool SF16, int W, int NB, bool G32, bool RAGGED>
+__device__ __forceinline__ void gemv_mxl_body(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8,
+                                              int e9, int e10, int e11, int out_f32, int mmax, const MxlTable &tbl) {
     using MF = MfmaFmt<BITS>;
     extern __shared__ __align__(16) unsigned char smem[];
 
@@ -91,7 +91,7 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
     const MxlDesc d = tbl.d[di];
     const int K = d.K, N = d.N, M = d.M;
     const int G = K >> 7;
-    const int KT = K >> 9;  // K % 512 == 0 and K >= 2048 (host)
+    const int KT = RAGGED ? (K + 511) >> 9 : K >> 9;  // (ragged: the last tile may hold one to three groups)
     const int row_bytes = K * BITS / 8;
     const int n0 = (wg - d.wg_begin) << 4;
 
@@ -122,6 +122,10 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
     for (int h = 0; h < MF::kLoads; ++h)
         w_off[h] = (uint32_t)(n0 + h * MF::kRowsPerLoad + ld_row) * (uint32_t)row_bytes +
                    (uint32_t)(ld_col * 16);
+    // (where K is not a multiple of 512 the scale rows are 2-byte aligned, which buffer loads take; a last
+    // tile of fewer than four groups loads the last four scales of the row and shifts, so that nothing past
+    // the matrix is read and the groups that do not exist have scale zero; the weights loaded there are the
+    // next row's and meet zero activations)
     const uint32_t s_off = (uint32_t)(n0 + op_row) * (uint32_t)(G * 2);
     u32x4 w[MF::kLoads];
     uint2 scr;
@@ -129,7 +133,8 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
 #pragma unroll
         for (int h = 0; h < MF::kLoads; ++h) w[h] = mxl_load_b128(rB, w_off[h], (uint32_t)(kt * MF::kTileBytes));
         typedef unsigned int v2u __attribute__((ext_vector_type(2)));
-        const v2u sv = __builtin_amdgcn_raw_buffer_load_b64(rS, (int)s_off, kt * 8, 0);
+        const int first = !RAGGED || kt * kMxTileGroups < G - kMxTileGroups ? kt * kMxTileGroups : G - kMxTileGroups;
+        const v2u sv = __builtin_amdgcn_raw_buffer_load_b64(rS, (int)s_off, first * 2, 0);
         scr = make_uint2(sv.x, sv.y);
     };
 
@@ -149,12 +154,14 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
         u32x4 v[kSt][QW];
     };
     auto act_load = [&](ActRegs &ar, int kt, int batch) {
+        // activations past K read as zero: an offset outside the buffer
+        const uint32_t a_lane = !RAGGED || kt * kMxTileK + sq * QB < K ? a_off : 0x80000000u;
 #pragma unroll
         for (int i = 0; i < kSt; ++i) {
             if (TSTEP * i + 8 * batch >= M) break;  // uniform: no lane of this task has a token
 #pragma unroll
             for (int q = 0; q < QW; ++q)
-                ar.v[i][q] = mxl_load_b128(rA, a_off + (uint32_t)((TSTEP * i + 8 * batch) * K + q * 16),
+                ar.v[i][q] = mxl_load_b128(rA, a_lane + (uint32_t)((TSTEP * i + 8 * batch) * K + q * 16),
                                            (uint32_t)(kt * kMxTileK));
         }
     };
@@ -200,7 +207,12 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
             d2[0] = make_uint2(w[h].x, w[h].y);
             d2[1] = make_uint2(w[h].z, w[h].w);
         }
-        const uint2 sc = scr;
+        const int left = G - kt * kMxTileGroups;  // groups of this tile that exist (four or more: all)
+        uint2 sc = scr;
+        if (RAGGED) {
+            const uint64_t sc64 = (((uint64_t)scr.y << 32) | scr.x) >> (left < kMxTileGroups ? 16 * (kMxTileGroups - left) : 0);
+            sc = make_uint2((uint32_t)sc64, (uint32_t)(sc64 >> 32));
+        }
         if (kt + 1 < te) {  // uniform: the next tile of this slice travels during the arithmetic
             act_load(acur, kt + 1, 0);
             if (NB > 1 && nbatch > 1) act_load(amore, kt + 1, 1);
@@ -234,7 +246,7 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
 #pragma unroll
                 for (int r = 0; r < MR; ++r) {
                     const int tk = 4 * kb + r;
-                    if (row < N && tk < M)
+                    if (row < N && tk < M && (!RAGGED || gi < left))
                         reinterpret_cast<int32_t *>(d.out)[((size_t)tk * N + row) * G + (kt * kMxTileGroups + gi)] = dd[r];
                 }
                 continue;
@@ -268,6 +280,23 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
     }
 }
 
+template <int BITS, int MR, bool SF16, int W, int NB, int OCC, bool G32 = false>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
+gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8, int e9,
+                int e10, int e11, int out_f32, int mmax, const MxlTable tbl) {
+    gemv_mxl_body<BITS, MR, SF16, W, NB, G32, false>(e0, e1, e2, e3, e4, e5, e6, e7, e8, e9, e10, e11, out_f32, mmax, tbl);
+}
+
+// Rows of any whole number of groups from four on: the dot4 kernel, the only other one that takes them, walks
+// them once per eight tokens (12288 x 1920 at nine tokens 9.2 us against 4.3 here, 2500 x 9600 at 16 23.6
+// against 5.9).  A build of its own: the checks of the last tile cost the others 0.1 us a launch.
+template <int BITS, int MR, bool SF16, int W, int NB, int OCC, bool G32 = false>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
+gemv_mxl_ragged_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8, int e9,
+                       int e10, int e11, int out_f32, int mmax, const MxlTable tbl) {
+    gemv_mxl_body<BITS, MR, SF16, W, NB, G32, true>(e0, e1, e2, e3, e4, e5, e6, e7, e8, e9, e10, e11, out_f32, mmax, tbl);
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -278,24 +307,26 @@ constexpr int kMxlWideWaves = 12;
 
 // width class: 0 = every block has one token, 1 = at most eight tokens, 2 = up to sixteen;
 // dense: more than four workgroups per CU to place (only matters for width class 2)
-template <int BITS, int W, int OCC1, int OCC2>
-MxlKernelFn mxl_kernel_w(int scale_kind, int width_class) {
-    if (scale_kind == 2) {  // int32 group sums from the same builds
-        if (width_class == 0) return gemv_mxl_kernel<BITS, 1, false, W, 1, OCC1, true>;
-        if (width_class == 1) return gemv_mxl_kernel<BITS, 4, false, W, 1, OCC1, true>;
-        return gemv_mxl_kernel<BITS, 4, false, W, 2, OCC2, true>;
+template <int BITS, int MR, int W, int NB, int OCC>
+MxlKernelFn mxl_kernel_n(int scale_kind, bool ragged) {
+    if (ragged) {
+        if (scale_kind == 2) return gemv_mxl_ragged_kernel<BITS, MR, false, W, NB, OCC, true>;
+        return scale_kind == 1 ? gemv_mxl_ragged_kernel<BITS, MR, true, W, NB, OCC> : gemv_mxl_ragged_kernel<BITS, MR, false, W, NB, OCC>;
     }
-    if (width_class == 0)
-        return scale_kind == 1 ? gemv_mxl_kernel<BITS, 1, true, W, 1, OCC1> : gemv_mxl_kernel<BITS, 1, false, W, 1, OCC1>;
-    if (width_class == 1)
-        return scale_kind == 1 ? gemv_mxl_kernel<BITS, 4, true, W, 1, OCC1> : gemv_mxl_kernel<BITS, 4, false, W, 1, OCC1>;
-    return scale_kind == 1 ? gemv_mxl_kernel<BITS, 4, true, W, 2, OCC2> : gemv_mxl_kernel<BITS, 4, false, W, 2, OCC2>;
+    if (scale_kind == 2) return gemv_mxl_kernel<BITS, MR, false, W, NB, OCC, true>;  // int32 group sums from the same builds
+    return scale_kind == 1 ? gemv_mxl_kernel<BITS, MR, true, W, NB, OCC> : gemv_mxl_kernel<BITS, MR, false, W, NB, OCC>;
+}
+template <int BITS, int W, int OCC1, int OCC2>
+MxlKernelFn mxl_kernel_w(int scale_kind, int width_class, bool ragged) {
+    if (width_class == 0) return mxl_kernel_n<BITS, 1, W, 1, OCC1>(scale_kind, ragged);
+    if (width_class == 1) return mxl_kernel_n<BITS, 4, W, 1, OCC1>(scale_kind, ragged);
+    return mxl_kernel_n<BITS, 4, W, 2, OCC2>(scale_kind, ragged);
 }
 template <int BITS>
-MxlKernelFn mxl_kernel(int scale_kind, int width_class, bool wide, bool dense) {
-    if (wide) return mxl_kernel_w<BITS, kMxlWideWaves, 3, 3>(scale_kind, width_class);
-    return dense ? mxl_kernel_w<BITS, kMxWaves, 5, 5>(scale_kind, width_class)
-                 : mxl_kernel_w<BITS, kMxWaves, 5, 4>(scale_kind, width_class);
+MxlKernelFn mxl_kernel(int scale_kind, int width_class, bool wide, bool dense, bool ragged) {
+    if (wide) return mxl_kernel_w<BITS, kMxlWideWaves, 3, 3>(scale_kind, width_class, ragged);
+    return dense ? mxl_kernel_w<BITS, kMxWaves, 5, 5>(scale_kind, width_class, ragged)
+                 : mxl_kernel_w<BITS, kMxWaves, 5, 4>(scale_kind, width_class, ragged);
 }
 
 template <int BITS>
@@ -303,20 +334,21 @@ int mxl_init_device(int max_lds) {
     for (int sk = 0; sk < 3; ++sk)
         for (int wc = 0; wc < 3; ++wc)
             for (int wide = 0; wide < 2; ++wide)
-                for (int dense = 0; dense < 2; ++dense)
+                for (int k = 0; k < 4; ++k)
                     if (hipFuncSetAttribute(
-                            reinterpret_cast<const void *>(mxl_kernel<BITS>(sk, wc, wide != 0, dense != 0)),
+                            reinterpret_cast<const void *>(mxl_kernel<BITS>(sk, wc, wide != 0, (k & 1) != 0, (k & 2) != 0)),
                             hipFuncAttributeMaxDynamicSharedMemorySize, max_lds) != hipSuccess)
                         return 2;
     return 0;
 }
 
-// True when this kernel takes the problem: what gemv_mx.hip.h takes, with at most 16 tokens and
-// operand sizes within the 32-bit buffer range (q.ws may be null when group sums are wanted).
+// True when this kernel takes the problem: at most 16 tokens, whole groups from four on, 16-byte aligned
+// operands whose sizes are within the 32-bit buffer range (q.ws may be null when group sums are wanted).
 template <int BITS>
 bool mxl_problem_ok(const GemvProblem &q) {
-    return mx_problem_ok(q, false) && q.M <= 16 && (long)q.N * (q.K * BITS / 8) < (1L << 31) &&
-           (long)q.M * q.K < (1L << 31);
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(q.A) | reinterpret_cast<uintptr_t>(q.B);
+    return (bits & 15) == 0 && q.K >= kMxTileK && q.M <= 16 && (long)q.N * (q.K * BITS / 8) < (1L << 31) - 1024 &&
+           (long)q.M * q.K < (1L << 31) - 1024;
 }
 
 // Launches up to kMxlMaxDesc problems, one workgroup per 16 rows.  Returns 0, -1 when the launch
@@ -327,8 +359,9 @@ int launch_mxl(const GemvProblem *probs, int count, int out_kind, int scale_kind
     if (count < 1 || count > kMxlMaxDesc) return -1;
     long wgs = 0;
     int mmax = 1;
-    bool one_token = true;
+    bool one_token = true, ragged = false;
     for (int i = 0; i < count; ++i) {
+        ragged = ragged || probs[i].K % kMxTileK != 0;
         wgs += (probs[i].N + 15) / 16;
         mmax = probs[i].M > mmax ? probs[i].M : mmax;
         one_token = one_token && probs[i].M == 1;
@@ -375,12 +408,12 @@ int launch_mxl(const GemvProblem *probs, int count, int out_kind, int scale_kind
     for (int i = count; i < kMxlMaxDesc; ++i) ends[i] = 0x7fffffff;
     const int width_class = one_token ? 0 : (mmax <= 8 ? 1 : 2);
     const int variant = out_kind == OUT_G32 ? 2 : scale_kind;
-    hipLaunchKernelGGL(mxl_kernel<BITS>(variant, width_class, wide, dense), dim3(wg, 1, 1), dim3(waves * 64, 1, 1),
+    hipLaunchKernelGGL(mxl_kernel<BITS>(variant, width_class, wide, dense, ragged), dim3(wg, 1, 1), dim3(waves * 64, 1, 1),
                        lds, stream, ends[0], ends[1], ends[2], ends[3], ends[4], ends[5], ends[6],
                        ends[7], ends[8], ends[9], ends[10], ends[11], out_kind == OUT_F32 ? 1 : 0,
                        mmax, tbl);
     // <BITS, MR, SF16, W, NB, OCC, G32> as instantiated by mxl_kernel
-    note_kernel("gemv_mxl_kernel", BITS, width_class == 0 ? 1 : 4, scale_kind == 1 && variant != 2, waves,
+    note_kernel(ragged ? "gemv_mxl_ragged_kernel" : "gemv_mxl_kernel", BITS, width_class == 0 ? 1 : 4, scale_kind == 1 && variant != 2, waves,
                 width_class == 2 ? 2 : 1, wide ? 3 : (width_class == 2 && !dense ? 4 : 5), variant == 2);
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }

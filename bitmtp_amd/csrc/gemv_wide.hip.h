@@ -1,0 +1,459 @@
+// Matrix-core kernel for wide blocks (prompts, batches of requests): more than 16 tokens.
+//
+// Below 16 tokens a packed projection streams its weights and is bound by latency and bytes; here
+// every weight is multiplied with tens to thousands of tokens, and what bounds the kernel is the
+// vector ALU: per scale group (128 of K) and 16 x 16 results, two v_mfma_i32_16x16x64_i8 (32 clocks)
+// leave exact int32 group sums that must become fp32 and meet the group's scale -- eight vector
+// operations, 32 clocks as well -- beside the unpacking of the weights.  The token-tiled decode
+// kernels unpack every weight once per 16 tokens (14 operations per 16 x 16 results and group) and
+// re-read the activations for every 16 rows.  Here a wave holds MT x NT tiles of 16 tokens x 16 rows:
+// an unpacked operand serves MT tiles, an activation operand read from LDS serves NT, and the offset
+// term (two more MFMAs per 16 tokens and group against an operand of all -2 / -1, as in
+// gemv_mxl.hip.h) serves NT as well.
+//
+//   WM x WN waves share a staged block of WM*MT*16 tokens x WN*NT*16 rows; KS such sets of waves
+//   split K and add their fp32 results up in slice order (narrower blocks and few rows, where a
+//   tile per workgroup would leave most CUs idle).
+//
+// Per group a set stages 128 bytes of K for its tokens (4 x 4 byte transposes: operand order, see
+// gemv_core.h; 16-byte units XORed with the row number, so that a ds_read_b128 of 16 rows meets every
+// bank once) and the packed rows as they are (a wave's operand read is 512 contiguous bytes).  The
+// loads of group g + 2 are in flight and group g + 1 is being parked while group g is multiplied: one
+// barrier per group, none where a set is a single wave.  All scales of the row block (G x rows,
+// transposed) and the multipliers are staged once.  Rows past N and tokens past M read as zero through
+// the buffer range check.
+//
+// Arithmetic and rounding points are those of the other kernels: exact G, fp32 scale-accumulate with
+// groups in ascending order inside a slice, slices in order, division by s[m], bf16 RNE.
+//
+// Block numbers go round the eight XCDs, so an XCD takes a contiguous range of tiles, eight token
+// tiles by consecutive row tiles: its L2 sees the same activations and the same rows again.
+//
+// Replaces, for these widths, the launch-per-projection path of
+// src/bonsai_sft/gpu/t2g128_kernels/t2g128_kernels.cu:94-148 (any M).
+#ifndef BONSAI_GEMV_WIDE_HIP_H
+#define BONSAI_GEMV_WIDE_HIP_H
+
+#include <type_traits>
+
+#include "gemv_mxl.hip.h"
+
+namespace bonsai {
+
+constexpr int kWideXcds = 8;
+constexpr int kWideTokenGroup = 8;  // token tiles walked before the next row tile
+
+template <int BITS, int WM, int WN, int KS, int MT, int NT>
+struct WideShape {
+    static constexpr int kTokens = WM * MT * 16, kRows = WN * NT * 16;
+    static constexpr int kSet = 64 * WM * WN;  // threads that share a staged block
+    static constexpr int kThreads = kSet * KS;
+    static constexpr bool kPrivate = WM * WN == 1;  // a set is one wave: program order is enough
+    static constexpr int kBufs = kPrivate ? 1 : 2;
+    static constexpr int kAhead = kPrivate && MT <= 2 ? 2 : 1;  // register sets of staging loads in flight
+    static constexpr int kABytes = kTokens * 128, kBBytes = kRows * 16 * BITS;
+    static constexpr int kSetBytes = kBufs * (kABytes + kBBytes);
+    static constexpr int kElems = MT * NT * 4;  // results per lane
+    static constexpr int kOutPitch = kRows * 2 + 16;
+    static constexpr int kShare = kElems / KS;  // results per lane that a K slice finishes
+    static constexpr int kRedBytes = (KS - 1) * kSet * kElems * 4;
+    // scales [G][rows] u16, then multipliers [tokens] fp32 (they stay), then the staged blocks, whose
+    // space the K slices' partial sums and the outgoing tile take over
+    static size_t lds_bytes(int K) {
+        const size_t keep = (size_t)(K / kGroup) * kRows * 2 + kTokens * 4;
+        const size_t stage = (size_t)KS * kSetBytes;
+        const size_t after = kRedBytes + (size_t)kTokens * kOutPitch;
+        return keep + (stage > after ? stage : after);
+    }
+};
+
+// The barrier of the staging pipeline: LDS traffic of the group is done, loads for later ones stay
+// in flight (a __syncthreads() would wait for them as well).
+__device__ __forceinline__ void wide_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <int BITS, int WM, int WN, int KS, int MT, int NT, bool SF16, bool G32>
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(2)))
+gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
+                 int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
+    using S = WideShape<BITS, WM, WN, KS, MT, NT>;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int G = K >> 7;
+    const int row_bytes = K * BITS / 8;
+
+    // ---- tile of this workgroup
+    const int total = tiles_m * tiles_n;
+    const int per = (total + kWideXcds - 1) / kWideXcds;
+    const int t = ((int)blockIdx.x & (kWideXcds - 1)) * per + ((int)blockIdx.x >> 3);
+    if (t >= total) return;
+    const int band = kWideTokenGroup * tiles_n;
+    const int mg = t / band, rem = t - mg * band;
+    const int gm = tiles_m - mg * kWideTokenGroup < kWideTokenGroup ? tiles_m - mg * kWideTokenGroup : kWideTokenGroup;
+    const int tn = rem / gm;
+    const int m0 = (mg * kWideTokenGroup + rem - tn * gm) * S::kTokens;
+    const int n0 = tn * S::kRows;
+    const int mv = M - m0 < S::kTokens ? M - m0 : S::kTokens;
+    const int nv = N - n0 < S::kRows ? N - n0 : S::kRows;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int set = wave / (WM * WN), wsub = wave % (WM * WN);
+    const int stid = tid - set * S::kSet;
+    const int wm = wsub / WN, wn = wsub % WN;
+    const int op_row = lane & 15, kb = lane >> 4;
+
+    uint16_t *scales = reinterpret_cast<uint16_t *>(smem);
+    float *mult = reinterpret_cast<float *>(smem + (size_t)G * S::kRows * 2);
+    unsigned char *work = reinterpret_cast<unsigned char *>(mult + S::kTokens);
+    unsigned char *abuf = work + set * S::kSetBytes;
+    unsigned char *bbuf = abuf + S::kBufs * S::kABytes;
+
+    const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t *>(A + (size_t)m0 * K), 0, mv * K, kMxlBufferWord3);
+    const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(B + (size_t)n0 * row_bytes), 0, nv * row_bytes, kMxlBufferWord3);
+
+    // ---- K slice of this set (whole 512-wide tiles where K has them: the slices of gemv_mxl.hip.h)
+    const int unit = (G & 3) == 0 ? 4 : 1;
+    const int units = G / unit;
+    const int gb = KS == 1 ? 0 : (units * set / KS) * unit;
+    const int ge = KS == 1 ? G : (units * (set + 1) / KS) * unit;
+    const int iters = KS == 1 ? G : ((units + KS - 1) / KS) * unit;  // of the longest slice
+
+    // ---- staging roles
+    constexpr int QB = mfma_quarter_bytes<BITS>();
+    constexpr int QW = QB / 16;
+    constexpr int QPR = 128 / QB;                       // quarters of a token row
+    constexpr int AL = S::kTokens * QPR / S::kSet;      // quarters a thread stages
+    constexpr int BCH = BITS;                           // 16-byte chunks of a packed row
+    constexpr int BN_TASKS = S::kRows * BCH;
+    constexpr int BL = (BN_TASKS + S::kSet - 1) / S::kSet;
+    static_assert(AL * S::kSet == S::kTokens * QPR && AL >= 1, "staging tasks divide evenly");
+    uint32_t a_off[AL], b_off[BL];
+#pragma unroll
+    for (int i = 0; i < AL; ++i) {
+        const int task = stid + i * S::kSet;
+        a_off[i] = (uint32_t)(task / QPR) * (uint32_t)K + (uint32_t)((task % QPR) * QB);
+    }
+#pragma unroll
+    for (int i = 0; i < BL; ++i) {
+        const int task = stid + i * S::kSet;
+        b_off[i] = (uint32_t)(task / BCH) * (uint32_t)row_bytes + (uint32_t)((task % BCH) * 16);
+    }
+    u32x4 ars[S::kAhead][AL][QW], brs[S::kAhead][BL];
+    auto load = [&](auto &ar, auto &br, int g) {
+#pragma unroll
+        for (int i = 0; i < AL; ++i)
+#pragma unroll
+            for (int q = 0; q < QW; ++q) ar[i][q] = mxl_load_b128(rA, a_off[i] + q * 16, (uint32_t)(g * 128));
+#pragma unroll
+        for (int i = 0; i < BL; ++i)
+            if (BN_TASKS % S::kSet == 0 || stid + i * S::kSet < BN_TASKS)
+                br[i] = mxl_load_b128(rB, b_off[i], (uint32_t)(g * 16 * BITS));
+    };
+    auto park = [&](const auto &ar, const auto &br, int buf) {
+        u32x4 *a = reinterpret_cast<u32x4 *>(abuf + buf * S::kABytes);
+#pragma unroll
+        for (int i = 0; i < AL; ++i) {
+            const int task = stid + i * S::kSet;
+            const int row = task / QPR, q = task % QPR;
+            u32x4 *dst = a + row * 8;
+            const int x = row & 7;
+            if (BITS == 2) {
+                const u32x4 v = ar[i][0];
+                dst[q ^ x] = transpose4x4_bytes(v.x, v.y, v.z, v.w);
+            } else {
+                const u32x4 lo = ar[i][0], hi = ar[i][QW - 1];
+                dst[(2 * q) ^ x] = transpose4x4_bytes(lo.x, lo.z, hi.x, hi.z);
+                dst[(2 * q + 1) ^ x] = transpose4x4_bytes(lo.y, lo.w, hi.y, hi.w);
+            }
+        }
+        u32x4 *b = reinterpret_cast<u32x4 *>(bbuf + buf * S::kBBytes);
+#pragma unroll
+        for (int i = 0; i < BL; ++i)
+            if (BN_TASKS % S::kSet == 0 || stid + i * S::kSet < BN_TASKS) b[stid + i * S::kSet] = br[i];
+    };
+
+    load(ars[0], brs[0], gb < ge ? gb : 0);
+
+    // ---- scales of the row block, transposed, and the multipliers
+    if (!G32) {
+        const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t *>(ws + (size_t)n0 * G), 0, nv * G * 2, kMxlBufferWord3);
+        if (flags & 1) {  // whole quads of groups, aligned
+            const int quads = G >> 2;
+            for (int i = tid; i < S::kRows * quads; i += S::kThreads) {
+                const int row = i / quads, q = i - row * quads;
+                typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+                const v2u v = __builtin_amdgcn_raw_buffer_load_b64(rS, i * 8, 0, 0);
+                uint16_t *d = scales + (q * 4) * S::kRows + row;
+                d[0] = (uint16_t)v.x;
+                d[S::kRows] = (uint16_t)(v.x >> 16);
+                d[2 * S::kRows] = (uint16_t)v.y;
+                d[3 * S::kRows] = (uint16_t)(v.y >> 16);
+            }
+        } else {
+            for (int i = tid; i < S::kRows * G; i += S::kThreads) {
+                const int row = i / G, g = i - row * G;
+                scales[g * S::kRows + row] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rS, i * 2, 0, 0);
+            }
+        }
+        for (int i = tid; i < S::kTokens; i += S::kThreads) mult[i] = s[m0 + (i < mv ? i : mv - 1)];
+    }
+
+    float acc[MT][NT][4];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
+    constexpr int kNegs = BITS == 2 ? (int)0xFEFEFEFEu : (int)0xFFFFFFFFu;
+    const v4i negs = {kNegs, kNegs, kNegs, kNegs};
+    // The accumulators start from the bits of 1.5 * 2^23 (|G| < 2^22): the sums then ARE floats,
+    // 12582912 + G, and one exact subtraction at full rate takes the place of an int-to-float conversion.
+    constexpr int kBias = 0x4B400000;
+    constexpr float kBiasF = 12582912.0f;
+    const v4i bias4 = {kBias, kBias, kBias, kBias};
+
+    if (S::kPrivate) {
+        if (S::kAhead > 1 && gb + 1 < ge) load(ars[S::kAhead - 1], brs[S::kAhead - 1], gb + 1);
+    } else {
+        park(ars[0], brs[0], 0);
+        if (gb + 1 < ge) load(ars[0], brs[0], gb + 1);
+    }
+    __syncthreads();
+
+    const auto step = [&](int it, auto set_of) {
+        constexpr int R = decltype(set_of)::value;  // register set of this group
+        const int g = gb + it;
+        const int buf = S::kPrivate ? 0 : (it & 1);
+        if (S::kPrivate) {
+            if (g < ge) park(ars[R], brs[R], 0);
+            if (g + S::kAhead < ge) load(ars[R], brs[R], g + S::kAhead);
+        } else {
+            if (it > 0) wide_barrier();  // group g is parked; group g - 1 is no longer read
+            if (g + 1 < ge) park(ars[0], brs[0], buf ^ 1);
+            if (g + 2 < ge) load(ars[0], brs[0], g + 2);
+        }
+        if (g >= ge) return;  // (uniform in a set)
+        const u32x4 *a = reinterpret_cast<const u32x4 *>(abuf + buf * S::kABytes) + (wm * MT * 16 + op_row) * 8;
+        const unsigned char *b = bbuf + buf * S::kBBytes + (wn * NT * 16 + op_row) * (16 * BITS) + kb * (4 * BITS);
+        const int x = op_row & 7;
+        v4i va0[MT], va1[MT], vc[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const u32x4 u0 = a[i * 128 + ((2 * kb) ^ x)], u1 = a[i * 128 + ((2 * kb + 1) ^ x)];
+            va0[i] = v4i{(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w};
+            va1[i] = v4i{(int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) vc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va0[i], negs, bias4, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) vc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va1[i], negs, vc[i], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            uint32_t p0, p1 = 0;
+            if (BITS == 2) {
+                const uint2 pp = *reinterpret_cast<const uint2 *>(b + j * 16 * 16 * BITS);
+                p0 = pp.x;
+                p1 = pp.y;
+            } else {
+                p0 = *reinterpret_cast<const uint32_t *>(b + j * 16 * 16 * BITS);
+            }
+            float w = 0.0f;
+            if (!G32) w = scale_to_f32<SF16>(scales[g * S::kRows + (wn * NT + j) * 16 + op_row]);
+            uint32_t b0[4], b1[4];
+            mfma_unpack<BITS>(p0, p1, b0, b1);
+            const v4i vb0 = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3]};
+            const v4i vb1 = {(int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
+            v4i dd[MT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) dd[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va0[i], vb0, vc[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) dd[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va1[i], vb1, dd[i], 0, 0, 0);
+            if (G32) {
+                const int n = (wn * NT + j) * 16 + op_row;
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int m = (wm * MT + i) * 16 + 4 * kb + r;
+                        if (m < mv && n < nv)
+                            reinterpret_cast<int32_t *>(out)[((size_t)(m0 + m) * N + n0 + n) * G + g] = dd[i][r] - kBias;
+                    }
+                continue;
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][j][r] += (__int_as_float(dd[i][r]) - kBiasF) * w;
+        }
+    };
+    for (int it = 0; it < iters; it += S::kAhead) {
+        step(it, std::integral_constant<int, 0>{});
+        if (S::kAhead > 1) step(it + 1, std::integral_constant<int, S::kAhead - 1>{});
+    }
+    if (G32) return;
+
+    // ---- y / s: the reciprocal is correctly rounded and one residual step makes the quotient so
+    const auto divide = [&](float y, float d, float inv) {
+        const float q = y * inv;
+        const float c = fmaf(fmaf(-q, d, y), inv, q);
+        return c == c ? c : q;  // (infinite or NaN y)
+    };
+    __syncthreads();  // the staged blocks are free
+    unsigned char *tile = work + S::kRedBytes;
+    const auto finish = [&](int i, int j, int r, float y, float d, float inv) {
+        const int m = (wm * MT + i) * 16 + 4 * kb + r, n = (wn * NT + j) * 16 + op_row;
+        y = divide(y, d, inv);
+        if (out_f32) {
+            if (m < mv && n < nv) reinterpret_cast<float *>(out)[(size_t)(m0 + m) * N + n0 + n] = y;
+        } else {
+            *reinterpret_cast<uint16_t *>(tile + m * S::kOutPitch + n * 2) = f32_to_bf16_rne_nobranch(y);
+        }
+    };
+    if (KS > 1) {
+        // slice z finishes the results [z * kShare, ..) of every lane and takes the other slices'
+        // values of them, slot by slot, from red[z]
+        static_assert(S::kShare * KS == S::kElems, "results divide among the slices");
+        float *red = reinterpret_cast<float *>(work) + stid;
+        const auto slot = [&](int dst, int src, int k) -> float & {
+            return red[((dst * (KS - 1) + (src < dst ? src : src - 1)) * S::kShare + k) * S::kSet];
+        };
+#pragma unroll
+        for (int z = 0; z < KS; ++z)
+            if (z != set) {
+#pragma unroll
+                for (int k = 0; k < S::kShare; ++k) {
+                    const int e = z * S::kShare + k;
+                    slot(z, set, k) = acc[e / (NT * 4)][e / 4 % NT][e % 4];
+                }
+            }
+        __syncthreads();
+#pragma unroll
+        for (int z = 0; z < KS; ++z)
+            if (z == set) {
+#pragma unroll
+                for (int k = 0; k < S::kShare; ++k) {
+                    const int e = z * S::kShare + k;
+                    const float own = acc[e / (NT * 4)][e / 4 % NT][e % 4];
+                    float y = z == 0 ? own : slot(z, 0, k);
+#pragma unroll
+                    for (int src = 1; src < KS; ++src) y += src == z ? own : slot(z, src, k);
+                    const float d = mult[(wm * MT + e / (NT * 4)) * 16 + 4 * kb + e % 4];
+                    finish(e / (NT * 4), e / 4 % NT, e % 4, y, d, 1.0f / d);
+                }
+            }
+    } else {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float d = mult[(wm * MT + i) * 16 + 4 * kb + r], inv = 1.0f / d;
+#pragma unroll
+                for (int j = 0; j < NT; ++j) finish(i, j, r, acc[i][j][r], d, inv);
+            }
+    }
+    if (out_f32) return;
+    __syncthreads();
+    // ---- the tile leaves in 16-byte pieces of whole rows
+    constexpr int CPR = S::kRows / 8;
+    uint16_t *o = reinterpret_cast<uint16_t *>(out);
+    for (int i = tid; i < S::kTokens * CPR; i += S::kThreads) {
+        const int m = i / CPR, c = (i % CPR) * 8;
+        if (m >= mv || c >= nv) continue;
+        const unsigned char *src = tile + m * S::kOutPitch + c * 2;
+        uint16_t *dst = o + (size_t)(m0 + m) * N + n0 + c;
+        if (flags & 2) {  // N a multiple of 8, rows 16-byte aligned
+            *reinterpret_cast<u32x4 *>(dst) = *reinterpret_cast<const u32x4 *>(src);
+        } else {
+            for (int k = 0; k < 8 && c + k < nv; ++k) dst[k] = reinterpret_cast<const uint16_t *>(src)[k];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Host side
+// ---------------------------------------------------------------------------
+using WideKernelFn = void (*)(const int8_t *, const uint8_t *, void *, const float *, const uint16_t *, int, int,
+                              int, int, int, int, int);
+
+struct WideVariant {
+    WideKernelFn fn[3];  // bf16 scales, fp16 scales, group sums
+    int tokens, rows, threads;
+    size_t (*lds)(int K);
+    int t[5];  // template arguments, for the launch record
+};
+
+template <int BITS, int WM, int WN, int KS, int MT, int NT>
+constexpr WideVariant wide_variant() {
+    using S = WideShape<BITS, WM, WN, KS, MT, NT>;
+    return WideVariant{{gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false>,
+                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, true, false>,
+                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, true>},
+                       S::kTokens, S::kRows, S::kThreads, S::lds_bytes, {WM, WN, KS, MT, NT}};
+}
+
+enum : int { WIDE_128x128 = 0, WIDE_32x64, kWideVariants };
+
+template <int BITS>
+const WideVariant &wide_kernel(int v) {
+    static const WideVariant t[kWideVariants] = {wide_variant<BITS, 2, 2, 1, 4, 4>(),
+                                                 wide_variant<BITS, 1, 1, 4, 2, 4>()};
+    return t[v];
+}
+
+template <int BITS>
+int wide_init_device(int max_lds) {
+    for (int v = 0; v < kWideVariants; ++v)
+        for (int k = 0; k < 3; ++k)
+            if (hipFuncSetAttribute(reinterpret_cast<const void *>(wide_kernel<BITS>(v).fn[k]),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, max_lds) != hipSuccess)
+                return 2;
+    return 0;
+}
+
+// Which variant a shape gets: the smaller of the two estimates, in microseconds, of fixed cost plus
+// scale groups times tiles per CU in the fullest CU.  The constants are fits to sweeps over the 1.7B- and
+// 4B-shaped matrices at 17-3000 tokens (12288 x 2048 at 512 tokens: 34.1 / 34.5 us; 2048 x 6144 at
+// 1024: 56.8 / 34.2; 2560 x 9728 at 512: 83.9 / 37.4; 19456 x 2560 at 1024: 93.7 / 127.0); within 15 % of them everywhere.  A 128 x 128 tile alone on its CU is 1.17 times as long as half of
+// two that share one.
+inline int wide_pick(int M, int N, int K, int n_cus) {
+    const double G = K / kGroup;
+    const auto fullest = [&](int tokens, int rows) {
+        const long tiles = (long)((M + tokens - 1) / tokens) * ((N + rows - 1) / rows);
+        return (double)((tiles + n_cus - 1) / n_cus);
+    };
+    const double c0 = fullest(128, 128);
+    const double t[kWideVariants] = {8.0 + 0.80 * G * (c0 < 1.17 ? 1.17 : c0),
+                                     4.5 + 0.16 * G * fullest(32, 64)};
+    int best = 0;
+    for (int v = 1; v < kWideVariants; ++v)
+        if (t[v] < t[best]) best = v;
+    return best;
+}
+
+// Launches one problem as variant v; -1 when it does not fit (the caller falls back).
+template <int BITS>
+int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream) {
+    const WideVariant &k = wide_kernel<BITS>(v);
+    const size_t lds = k.lds(q.K);
+    if (lds > (size_t)lds_limit || (long)k.rows * q.K > (1L << 30) || (long)k.tokens * q.K > (1L << 30)) return -1;
+    const int tm = (q.M + k.tokens - 1) / k.tokens, tn = (q.N + k.rows - 1) / k.rows;
+    if ((long)tm * tn > (1L << 28)) return -1;
+    const int per = (tm * tn + kWideXcds - 1) / kWideXcds;
+    const int flags = ((q.K / kGroup) % 4 == 0 && (reinterpret_cast<uintptr_t>(q.ws) & 7) == 0 ? 1 : 0) |
+                      (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0);
+    const int variant = out_kind == OUT_G32 ? 2 : scale_kind;
+    hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), lds, stream, q.A, q.B, q.out,
+                       q.s, reinterpret_cast<const uint16_t *>(q.ws), q.M, q.N, q.K, out_kind == OUT_F32 ? 1 : 0, tm,
+                       tn, flags);
+    note_kernel("gemv_wide_kernel", BITS, k.t[0], k.t[1], k.t[2], k.t[3], k.t[4], variant);
+    return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+}  // namespace bonsai
+#endif  // BONSAI_GEMV_WIDE_HIP_H
