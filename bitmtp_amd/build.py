@@ -98,21 +98,21 @@ def py_ops_path() -> str:
 
 
 def _build_host(source: str, out: str, extra: list[str]) -> None:
-    """Compiles a host source against the installed PyTorch and links it to the three C-ABI
+    """Compiles a host source against the installed PyTorch and links it to the C-ABI
     libraries it calls (found at run time next to it through $ORIGIN)."""
     import torch
     tdir = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     os.makedirs(os.path.dirname(out), exist_ok=True)
-    libdirs = [os.path.dirname(lib_path(s)) for s in ("t2g128_kernels.hip", "q1g128_kernels.hip", "act_quant.hip")]
+    libdirs = [os.path.dirname(lib_path(s)) for s in ("t2g128_kernels.hip", "q1g128_kernels.hip", "act_quant.hip", "decode_ops.hip")]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include", f"-I{rocm}/include",
            os.path.join(CSRC, source), "-o", out,
            f"-L{tdir}/lib", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip"] + extra
-    cmd += [f"-L{d}" for d in libdirs] + ["-lbonsai_t2", "-lbonsai_q1", "-lbonsai_actq",
-            "-Wl,-rpath,$ORIGIN/../t2g128_kernels:$ORIGIN/../q1g128_kernels:$ORIGIN/../act_quant"]
+    cmd += [f"-L{d}" for d in libdirs] + ["-lbonsai_t2", "-lbonsai_q1", "-lbonsai_actq", "-lbonsai_decode",
+            "-Wl,-rpath,$ORIGIN/../t2g128_kernels:$ORIGIN/../q1g128_kernels:$ORIGIN/../act_quant:$ORIGIN/../decode_ops"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"g++ failed for {source}:\n{proc.stdout}")

@@ -27,6 +27,7 @@
 #include <mutex>
 
 #include "../../include/bonsai_decode.h"
+#include "prefill_attn.hip.h"
 #include "wave_reduce.h"
 
 namespace {
@@ -1515,16 +1516,16 @@ int rows_per_wave(int M) {
 
 }  // namespace
 
-extern "C" int bonsai_qk_norm_rope_kv_write(const void *xqkv, const void *q_norm_w,
+static int launch_rope(const void *xqkv, const void *q_norm_w,
                                             const void *k_norm_w, float eps, const void *cos_table,
                                             const void *sin_table, const int32_t *positions,
                                             void *q_out, void *k_layer, void *v_layer, int M,
                                             int n_heads, int n_kv, int slots, int write_slot,
-                                            int max_pos, void *stream) {
+                                            int max_pos, int max_width, void *stream) {
     if (!xqkv || !q_norm_w || !k_norm_w || !cos_table || !sin_table || !positions || !q_out ||
         !k_layer || !v_layer)
         return BONSAI_DECODE_ERR_ARG;
-    if (M < 1 || M > BONSAI_MAX_WIDTH || n_heads < 1 || n_kv < 1 || max_pos < 1 || write_slot < 0 ||
+    if (M < 1 || M > max_width || n_heads < 1 || n_kv < 1 || max_pos < 1 || write_slot < 0 ||
         write_slot + M > slots)
         return BONSAI_DECODE_ERR_ARG;
     RopeArgs a;
@@ -1549,6 +1550,43 @@ extern "C" int bonsai_qk_norm_rope_kv_write(const void *xqkv, const void *q_norm
                        static_cast<hipStream_t>(stream), a.xqkv, a.qw, a.kw, a.cos_t, a.sin_t,
                        a.positions, a.q_out, a.k_layer, a.v_layer, a.eps, a.M, a.n_heads, a.n_kv,
                        a.slots, a.write_slot, a.max_pos);
+    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+}
+
+extern "C" int bonsai_qk_norm_rope_kv_write(const void *xqkv, const void *q_norm_w, const void *k_norm_w,
+                                            float eps, const void *cos_table, const void *sin_table,
+                                            const int32_t *positions, void *q_out, void *k_layer, void *v_layer,
+                                            int M, int n_heads, int n_kv, int slots, int write_slot, int max_pos,
+                                            void *stream) {
+    return launch_rope(xqkv, q_norm_w, k_norm_w, eps, cos_table, sin_table, positions, q_out, k_layer, v_layer, M,
+                       n_heads, n_kv, slots, write_slot, max_pos, BONSAI_MAX_WIDTH, stream);
+}
+
+extern "C" int bonsai_prefill_rope_kv_write(const void *xqkv, const void *q_norm_w, const void *k_norm_w,
+                                            float eps, const void *cos_table, const void *sin_table,
+                                            const int32_t *positions, void *q_out, void *k_layer, void *v_layer,
+                                            int M, int n_heads, int n_kv, int slots, int write_slot, int max_pos,
+                                            void *stream) {
+    return launch_rope(xqkv, q_norm_w, k_norm_w, eps, cos_table, sin_table, positions, q_out, k_layer, v_layer, M,
+                       n_heads, n_kv, slots, write_slot, max_pos, BONSAI_PREFILL_MAX_ROWS, stream);
+}
+
+extern "C" int bonsai_prefill_attention(const void *q, const void *k_layer, const void *v_layer, void *out_bf16,
+                                        float scale, int M, int n_heads, int n_kv, int slots, int base,
+                                        void *stream) {
+    namespace P = bonsai_prefill;
+    if (!q || !k_layer || !v_layer || !out_bf16) return BONSAI_DECODE_ERR_ARG;
+    if (M < 1 || M > BONSAI_PREFILL_MAX_ROWS || n_kv < 1 || n_heads < n_kv || n_heads % n_kv != 0 ||
+        n_heads / n_kv > P::kPairs || base < 0 || slots > (1 << 22) || base + M > slots)
+        return BONSAI_DECODE_ERR_ARG;
+    const int hpg = n_heads / n_kv;
+    const int tokens = P::kPairs / hpg;
+    const int tiles = (M + tokens - 1) / tokens;
+    hipLaunchKernelGGL(P::prefill_attn_kernel, dim3(tiles * n_kv), dim3(P::kWaves * 64), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(q),
+                       static_cast<const uint16_t *>(k_layer), static_cast<const uint16_t *>(v_layer),
+                       static_cast<uint16_t *>(out_bf16), scale * 1.44269504088896340736f, M, n_heads, n_kv, hpg,
+                       slots, base, tokens, tiles);
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }
 

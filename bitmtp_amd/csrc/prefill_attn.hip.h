@@ -1,0 +1,222 @@
+// Attention of a block of prompt rows over the history and themselves (causal), on the matrix cores.
+//
+// The decode step's chunk pass (attn_mfma_kernel) serves up to 32 rows: 16 (row, query head) pairs per
+// workgroup, partial results through memory.  A prompt has rows enough to keep the chip busy without
+// splitting the history, so here a workgroup of four waves owns 128 pairs of one kv head for good --
+// 128 / heads-per-group consecutive rows with all their query heads, 32 pairs a wave -- and walks the
+// 64-slot chunks they see; nothing is merged.
+//
+//   S^T = K Q^T   2 x 8 v_mfma_f32_32x32x16_bf16: a lane owns ONE query (column) and half of the
+//                 chunk's slots, so the softmax is in-lane but for one exchange of the maximum with
+//                 lane + 32; the running sum stays a half per lane until the end
+//   O^T += V^T P^T   4 x 4 more: the slots a lane half holds after S^T (4 h + 0..3 of every eight) are
+//                 the slots its B operand takes, so P goes from the softmax registers straight into the
+//                 matrix core (rounded to bf16 as everywhere); V^T is read with the same slot order
+//
+// K rows are staged as they are (pitch 272 bytes: 32 rows at one column meet every bank once), V
+// transposed 4 slots x 8 dims at a time in registers (16 v_perm per thread and chunk; pitch 136).  Two
+// buffers: the loads of chunk c + 2 are in flight and c + 1 is being parked while c is multiplied.
+// Both are shared by the four waves, which is what bounds the LDS traffic; the matrix cores and the
+// vector ALU (32 exponentials per lane and chunk) do not overlap on this part and take about half of
+// the time each.
+//
+// Longest rows first; the kv head is the low part of the block number, so that with eight of them an
+// XCD's L2 holds one head's history.
+// Reference: the prompt forward's causal attention, src/bonsai_sft/gpu/model.py:996-1005 with the mask
+// of fast_generate.py:949-953.
+#ifndef BONSAI_PREFILL_ATTN_HIP_H
+#define BONSAI_PREFILL_ATTN_HIP_H
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace bonsai_prefill {
+
+constexpr int kHead = 128;
+constexpr int kSlots = 64;             // slots of a chunk
+constexpr int kWaves = 4;
+constexpr int kPairs = 32 * kWaves;    // (row, query head) pairs of a workgroup
+constexpr int kKPitch = 2 * kHead + 16;
+constexpr int kVPitch = 2 * kSlots + 8;
+constexpr int kKBytes = kSlots * kKPitch, kVBytes = kHead * kVPitch;
+constexpr int kLds = 2 * (kKBytes + kVBytes);
+constexpr int kRawBuffer = 0x00020000;
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned int u32v4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ bf16x8 frag(u32v4 v) {
+    bf16x8 r;
+    __builtin_memcpy(&r, &v, 16);
+    return r;
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    const bf16x2 p = {(__bf16)a, (__bf16)b};
+    uint32_t u;
+    __builtin_memcpy(&u, &p, 4);
+    return u;
+}
+
+__global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_attn_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *v_layer, uint16_t *out,
+                    float scale_log2e, int M, int n_heads, int n_kv, int hpg, int slots, int base, int tokens,
+                    int tiles) {
+    __shared__ __align__(16) unsigned char smem[kLds];
+    const int kvh = (int)blockIdx.x % n_kv;
+    const int m0 = (tiles - 1 - (int)blockIdx.x / n_kv) * tokens;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, h = lane >> 5;
+
+    // ---- this lane's query
+    const int pair = wave * 32 + col;
+    const int tok = pair / hpg, g = pair - tok * hpg;
+    const bool valid = tok < tokens && m0 + tok < M;
+    const int m = valid ? m0 + tok : M - 1;
+    const int pos = base + m;
+    const size_t row = (size_t)m * n_heads * kHead + (size_t)(kvh * hpg + g) * kHead;
+    u32v4 qr[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) qr[j] = *reinterpret_cast<const u32v4 *>(q + row + 16 * j + 8 * h);
+
+    const int rows = M - m0 < tokens ? M - m0 : tokens;
+    const int seen = base + m0 + rows;                       // slots the last row sees
+    const int chunks = (seen + kSlots - 1) / kSlots;
+    const int masked_from = (base + m0 + 1) / kSlots;        // from here on some row does not see all slots
+
+    // slots from `seen` on read as zero
+    const size_t head = (size_t)kvh * slots * kHead;
+    const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(k_layer + head), 0, seen * 2 * kHead, kRawBuffer);
+    const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(v_layer + head), 0, seen * 2 * kHead, kRawBuffer);
+
+    const int k_slot = tid >> 4, k_col = tid & 15;           // K: 16-byte column of slots k_slot + 16 i
+    const int v_slot = (tid & 15) * 4, v_dim = (tid >> 4) * 8;  // V: a block of 4 slots x 8 dims
+    const int k_off = k_slot * 2 * kHead + k_col * 16;
+    const int v_off = v_slot * 2 * kHead + v_dim * 2;
+    u32v4 kr[4], vr[4];
+    const auto load = [&](int c) {
+        const int s = c * kSlots * 2 * kHead;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) kr[i] = __builtin_amdgcn_raw_buffer_load_b128(rK, k_off + i * 16 * 2 * kHead, s, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rV, v_off + i * 2 * kHead, s, 0);
+    };
+    const auto park = [&](int buf) {
+        unsigned char *kb = smem + buf * (kKBytes + kVBytes), *vb = kb + kKBytes;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<u32v4 *>(kb + (k_slot + 16 * i) * kKPitch + k_col * 16) = kr[i];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+            const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
+            uint2 v;
+            v.x = __builtin_amdgcn_perm(vr[1][d / 2], vr[0][d / 2], sel);
+            v.y = __builtin_amdgcn_perm(vr[3][d / 2], vr[2][d / 2], sel);
+            *reinterpret_cast<uint2 *>(vb + (v_dim + d) * kVPitch + v_slot * 2) = v;
+        }
+    };
+
+    f32x16 o[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    load(0);
+    park(0);
+    if (chunks > 1) load(1);
+    for (int c = 0; c < chunks; ++c) {
+        const int buf = c & 1;
+        // chunk c is parked, chunk c - 1 no longer read (loads for later chunks stay in flight)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (c + 1 < chunks) park(buf ^ 1);
+        if (c + 2 < chunks) load(c + 2);
+        const unsigned char *kb = smem + buf * (kKBytes + kVBytes), *vb = kb + kKBytes;
+
+        f32x16 s[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+            const unsigned char *kp = kb + (32 * t + col) * kKPitch + 16 * h;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(*reinterpret_cast<const u32v4 *>(kp + 32 * j)),
+                                                               frag(qr[j]), s[t], 0, 0, 0);
+        }
+        // s[t][r]: slot 64 c + 32 t + 8 (r / 4) + 4 h + r % 4
+        if (c >= masked_from) {
+            const int rel = pos - c * kSlots - 4 * h;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (32 * t + 8 * (r / 4) + r % 4 > rel) s[t][r] = -INFINITY;
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m_run, mx * scale_log2e);  // finite: every row sees slot 0
+        if (__any(m_new > m_run)) {
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            l_run *= alpha;
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+            m_run = m_new;
+        }
+        uint32_t p[2][8];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const float a = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r], scale_log2e, -m_run));
+                const float b = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r + 1], scale_log2e, -m_run));
+                p[t][r] = pack_bf16(a, b);
+                bf16x2 pv;
+                __builtin_memcpy(&pv, &p[t][r], 4);
+                const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
+                l_run = __builtin_amdgcn_fdot2_f32_bf16(pv, ones, l_run, false);
+            }
+        // K-step ks takes slots 16 ks + 4 h + 0..3 and 16 ks + 8 + 4 h + 0..3 of each lane half
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const uint32_t *pp = p[ks / 2] + 4 * (ks & 1);
+            const bf16x8 pf = frag(u32v4{pp[0], pp[1], pp[2], pp[3]});
+            const unsigned char *vp = vb + col * kVPitch + (16 * ks + 4 * h) * 2;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const uint2 lo = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch);
+                const uint2 hi = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch + 16);
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(u32v4{lo.x, lo.y, hi.x, hi.y}), pf, o[d], 0, 0, 0);
+            }
+        }
+    }
+
+    const float l = l_run + __shfl_xor(l_run, 32);
+    if (!valid) return;
+    const float inv = 1.0f / l;
+    // o[d][r]: dim 32 d + 8 (r / 4) + 4 h + r % 4
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            uint2 v;
+            v.x = pack_bf16(o[d][4 * k] * inv, o[d][4 * k + 1] * inv);
+            v.y = pack_bf16(o[d][4 * k + 2] * inv, o[d][4 * k + 3] * inv);
+            *reinterpret_cast<uint2 *>(out + row + 32 * d + 8 * k + 4 * h) = v;
+        }
+}
+
+}  // namespace bonsai_prefill
+#endif  // BONSAI_PREFILL_ATTN_HIP_H

@@ -21,7 +21,9 @@
 
 #include <optional>
 #include <string>
+#include <vector>
 
+#include "../../include/bonsai_decode.h"
 #include "../../include/bonsai_gemv.h"
 
 namespace {
@@ -291,6 +293,92 @@ PyObject *silu_mul_quant(PyObject *, PyObject *x_obj) {
     END_HANDLE_TH_ERRORS
 }
 
+// prefill_layers(device, dims, eps, scale, buffers, layers) -> 0 / 1: the layers of a decoder over a block
+// of prompt rows, ten launches each from one call (a launch costs the stream 2.5-3 us, a ctypes call as
+// much again).  Addresses and sizes as Python integers, laid out by bitmtp_amd/model.py:
+//   dims     (bits, M, base, dim, n_heads, n_kv, ffn, slots, max_pos, layers, kv_address)
+//   buffers  (h0, h1, a_q, a_s, xqkv, q, attn, o_q, o_s, proj, gate_up, i_q, i_s, positions, cos, sin)
+//   layers   per layer (wqkv, its scales, wo, scales, gate|up, scales, down, scales, input norm,
+//            post-attention norm, q norm, k norm)
+// Returns which of h0 / h1 holds the residual stream; the last MLP's output, still to be added, is in proj.
+PyObject *prefill_layers(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    constexpr int kDims = 11, kBufs = 16, kPerLayer = 12;
+    if (nargs != 6 || !PyTuple_CheckExact(args[1]) || PyTuple_GET_SIZE(args[1]) != kDims ||
+        !PyTuple_CheckExact(args[4]) || PyTuple_GET_SIZE(args[4]) != kBufs || !PyList_CheckExact(args[5]))
+        return fail("prefill_layers: bad arguments");
+    long long d[kDims];
+    for (int i = 0; i < kDims; ++i) d[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(args[1], i));
+    const int bits = (int)d[0], M = (int)d[1], base = (int)d[2], dim = (int)d[3], nh = (int)d[4], nkv = (int)d[5],
+              ffn = (int)d[6], slots = (int)d[7], max_pos = (int)d[8], n_layers = (int)d[9];
+    const float eps = (float)PyFloat_AsDouble(args[2]), scale = (float)PyFloat_AsDouble(args[3]);
+    char *b[kBufs];
+    for (int i = 0; i < kBufs; ++i) b[i] = static_cast<char *>(PyLong_AsVoidPtr(PyTuple_GET_ITEM(args[4], i)));
+    const Py_ssize_t count = PyList_GET_SIZE(args[5]);
+    std::vector<void *> w((size_t)count * kPerLayer);
+    for (Py_ssize_t l = 0; l < count; ++l) {
+        PyObject *t = PyList_GET_ITEM(args[5], l);
+        if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != kPerLayer) return fail("prefill_layers: bad layer");
+        for (int i = 0; i < kPerLayer; ++i) w[l * kPerLayer + i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(t, i));
+    }
+    if (PyErr_Occurred()) return nullptr;
+    if (count != n_layers) return fail("prefill_layers: layer count mismatch");
+    char *kv = reinterpret_cast<char *>(d[10]);
+    const long long head_bytes = (long long)slots * 256, layer_bytes = head_bytes * nkv;
+    const int q_dim = nh * BONSAI_HEAD_DIM, qkv = (nh + 2 * nkv) * BONSAI_HEAD_DIM;
+    const OnDevice on(c10::Device(c10::DeviceType::CUDA, (c10::DeviceIndex)PyLong_AsLong(args[0])));
+    void *st = on.stream();
+    int cur = 0;
+    const char *what = nullptr;
+    int rc = 0;
+    {
+        ReleaseGil unlocked;
+        const auto gemv = bits == 2 ? t2g128_gemv_ex : q1g128_gemv_ex;
+        const auto project = [&](char *a, char *s, void *wq, void *ws, char *out, int n, int k) {
+            return gemv(reinterpret_cast<const int8_t *>(a), static_cast<const uint8_t *>(wq), out,
+                        reinterpret_cast<const float *>(s), ws, M, n, k, BONSAI_OUT_BF16, BONSAI_SCALE_BF16, st);
+        };
+        char *h[2] = {b[0], b[1]};
+        char *a_q = b[2], *a_s = b[3], *xqkv = b[4], *q = b[5], *attn = b[6], *o_q = b[7], *o_s = b[8], *proj = b[9],
+             *gu = b[10], *i_q = b[11], *i_s = b[12];
+        const auto i8 = [](char *p) { return reinterpret_cast<int8_t *>(p); };
+        const auto f32 = [](char *p) { return reinterpret_cast<float *>(p); };
+        for (int l = 0; l < n_layers && rc == 0; ++l) {
+            void **x = w.data() + (size_t)l * kPerLayer;
+            char *kl = kv + l * layer_bytes, *vl = kv + (n_layers + l) * layer_bytes;
+#define STEP(name, call)          \
+    do {                          \
+        if (rc == 0) {            \
+            rc = (call);          \
+            if (rc != 0) what = name; \
+        }                         \
+    } while (0)
+            if (l == 0) {
+                STEP("norm", bonsai_rmsnorm_quant_int8(h[0], x[8], eps, i8(a_q), f32(a_s), M, dim, st));
+            } else {
+                STEP("norm", bonsai_add_rmsnorm_quant_int8(proj, h[cur], x[8], eps, h[cur ^ 1], i8(a_q), f32(a_s), M, dim, st));
+                cur ^= 1;
+            }
+            STEP("q|k|v", project(a_q, a_s, x[0], x[1], xqkv, qkv, dim));
+            STEP("rope", bonsai_prefill_rope_kv_write(xqkv, x[10], x[11], eps, b[14], b[15],
+                                                      reinterpret_cast<const int32_t *>(b[13]), q, kl, vl, M, nh, nkv,
+                                                      slots, base, max_pos, st));
+            STEP("attention", bonsai_prefill_attention(q, kl, vl, attn, scale, M, nh, nkv, slots, base, st));
+            STEP("quantiser", bonsai_act_quant_int8(attn, BONSAI_X_BF16, i8(o_q), f32(o_s), M, q_dim, st));
+            STEP("o", project(o_q, o_s, x[2], x[3], proj, dim, q_dim));
+            STEP("norm", bonsai_add_rmsnorm_quant_int8(h[cur], proj, x[9], eps, h[cur ^ 1], i8(a_q), f32(a_s), M, dim, st));
+            cur ^= 1;
+            STEP("gate|up", project(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim));
+            STEP("silu", bonsai_silu_mul_quant_int8(gu, i8(i_q), f32(i_s), M, ffn, st));
+            STEP("down", project(i_q, i_s, x[6], x[7], proj, dim, ffn));
+#undef STEP
+        }
+    }
+    if (rc != 0) return fail(std::string("prompt block: ") + what + " failed with status " + std::to_string(rc));
+    return PyLong_FromLong(cur);
+    END_HANDLE_TH_ERRORS
+}
+
 #define FASTCALL(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)), METH_FASTCALL
 PyMethodDef kMethods[] = {
     {"linear", FASTCALL(linear), "(bits, a_int8, b_packed, s, ws, allow_f16_scales) -> bf16 or None"},
@@ -298,6 +386,7 @@ PyMethodDef kMethods[] = {
     {"quant_input", quant_input, METH_O, "(x) -> (q, s) or None"},
     {"norm_quant", FASTCALL(norm_quant), "(x, w, eps) -> (q, s) or None"},
     {"add_norm_quant", FASTCALL(add_norm_quant), "(x, residual, w, eps) -> (h, q, s) or None"},
+    {"prefill_layers", FASTCALL(prefill_layers), "(device, dims, eps, scale, buffers, layers) -> residual buffer"},
     {"silu_mul_quant", silu_mul_quant, METH_O, "(gate_up) -> (q, s) or None"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_bonsai_py", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -48,6 +48,10 @@ def load_decode_kernel() -> None:
     lib.bonsai_decode_attention_rope_parts.argtypes = [vp, vp, vp, cf, vp, vp, vp, ci, vp, vp, vp, vp, vp,
                                                        vp, vp, cf, ci, ci, ci, ci, ci, vp]
     lib.bonsai_decode_attention_rope_parts.restype = ci
+    lib.bonsai_prefill_rope_kv_write.argtypes = lib.bonsai_qk_norm_rope_kv_write.argtypes
+    lib.bonsai_prefill_rope_kv_write.restype = ci
+    lib.bonsai_prefill_attention.argtypes = [vp, vp, vp, vp, cf, ci, ci, ci, ci, ci, vp]
+    lib.bonsai_prefill_attention.restype = ci
     lib.bonsai_decode_set_tuning.argtypes = [ci]
     lib.bonsai_decode_set_tuning.restype = None
     lib.bonsai_decode_set_attention_engine.argtypes = [ci]
@@ -275,6 +279,32 @@ def decode_attention_rope_parts(xqkv: torch.Tensor, q_norm_w: torch.Tensor, k_no
             _ptr(out_bf16), _ptr(out_amax), float(scale), m, n_heads, n_kv, slots, int(sigma),
             _stream(xqkv.device))
     _need(rc == 0, f"bonsai_decode_attention_rope_parts failed with status {rc}")
+
+
+def prefill_attention(q: torch.Tensor, k_layer: torch.Tensor, v_layer: torch.Tensor, base: int,
+                      out: Optional[torch.Tensor] = None, scale: Optional[float] = None) -> torch.Tensor:
+    """Causal attention of prompt rows ``base .. base + M - 1`` whose keys and values already sit in slots
+    of the same numbers: row i sees slots ``0 .. base + i`` (reference: the prompt forward,
+    fast_generate.py:949-953).  ``q`` bf16 ``[M, n_heads, 128]``, ``out`` bf16 ``[M, n_heads * 128]``."""
+    for t, name in ((q, "q"), (k_layer, "k_layer"), (v_layer, "v_layer")):
+        _check(t, torch.bfloat16, name)
+    _need(q.dim() == 3 and q.shape[2] == HEAD_DIM, "q must be [M, n_heads, 128]")
+    _need(k_layer.shape == v_layer.shape and k_layer.dim() == 3 and k_layer.shape[2] == HEAD_DIM,
+          "KV layer shape mismatch")
+    m, n_heads = q.shape[0], q.shape[1]
+    n_kv, slots = k_layer.shape[0], k_layer.shape[1]
+    if out is None:
+        out = torch.empty(m, n_heads * HEAD_DIM, dtype=torch.bfloat16, device=q.device)
+    else:
+        _check(out, torch.bfloat16, "out")
+        _need(out.numel() == m * n_heads * HEAD_DIM, "out size mismatch")
+    if scale is None:
+        scale = 1.0 / math.sqrt(HEAD_DIM)
+    with torch.cuda.device(q.device):
+        rc = decode_lib().bonsai_prefill_attention(_ptr(q), _ptr(k_layer), _ptr(v_layer), _ptr(out), float(scale), m,
+                                                   n_heads, n_kv, slots, int(base), _stream(q.device))
+    _need(rc == 0, f"bonsai_prefill_attention failed with status {rc}")
+    return out
 
 
 def kv_commit(kv: torch.Tensor, src_slot: int, dst_slot: int, n: int) -> None:

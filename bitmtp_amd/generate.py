@@ -18,9 +18,10 @@ Semantics kept from the reference:
   throughput is ``timed_decode_tokens / decode_time`` with prefill and the first token
   excluded (fast_generate.py:1001,1147-1148,1171).
 
-The prompt is prefilled with the same packed kernels: AR-causal replays of width
-``atlas.prefill_width`` over consecutive chunks (the reference uses a bf16 dequantised
-variable-shape forward, fast_generate.py:949-953).
+The prompt is prefilled with the same packed arithmetic: one AR-causal replay where it fits
+``atlas.prefill_width`` rows, otherwise wide blocks of rows straight into the history
+(``GraphAtlas.prefill_prompt``; the reference uses a bf16 dequantised variable-shape forward,
+fast_generate.py:949-953).
 """
 from __future__ import annotations
 
@@ -106,6 +107,8 @@ def prefill(atlas: GraphAtlas, prompt: Sequence[int], sigma: int) -> int:
     n = len(prompt)
     if n < 1:
         raise ValueError("empty prompt")
+    if n > W and hasattr(atlas, "prefill_prompt"):
+        return atlas.prefill_prompt(prompt, sigma)
     g = atlas.get_graph(W, sigma, "ar")
     cache_len = 0
     first = None

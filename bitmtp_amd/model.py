@@ -614,14 +614,31 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
 
     # the last MLP's result: still to be added (ffn_out + h_cur), or already in the stream (fused layers)
     last_x = ws.ffn_out[logits_start:] if plan is None else h_cur[logits_start:]
-    last_res = _vp(h_cur[logits_start:]) if plan is None else None
+    last_res = h_cur[logits_start:] if plan is None else None
+    project_rows(model, ws, last_x, last_res, logits_end - logits_start, threshold, io.tokens_out, io.conf,
+                 io.accept, head_mode)
 
-    rows = logits_end - logits_start
+
+def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: torch.Tensor, last_res: Optional[torch.Tensor],
+                 rows: int, threshold: float, tokens_out: torch.Tensor, conf: torch.Tensor,
+                 accept: torch.Tensor, head_mode: str = "native") -> None:
+    """Final norm of ``last_x (+ last_res)``, output projection and argmax / confidence chain of ``rows`` rows
+    (reference: model.py:1401-1403, fast_generate.py:111-130)."""
+    args = model.args
+    dim, eps = args.dim, float(args.norm_eps)
+    actq = ops.actq_lib()
+    stream = ctypes.c_void_p(torch.cuda.current_stream(model.device).cuda_stream)
+    res = _vp(last_res) if last_res is not None else None
+
+    def check(rc: int, what: str) -> None:
+        if rc != 0:
+            raise RuntimeError(f"{what} failed with status {rc}")
+
     if head_mode not in ("native", "fp8", "bf16_raw"):
         raise ValueError(f"unknown head_mode {head_mode!r}")
     if head_mode != "native" or model.head is None:
         # projections of the normalised bf16 rows (reference: model.py:1401-1403)
-        check(actq.bonsai_add_rmsnorm_bf16(_vp(last_x), last_res, _vp(model.norm), eps, _vp(ws.h_last),
+        check(actq.bonsai_add_rmsnorm_bf16(_vp(last_x), res, _vp(model.norm), eps, _vp(ws.h_last),
                                            _vp(ws.l_n), rows, dim, stream),
               "bonsai_add_rmsnorm_bf16")
         if head_mode == "fp8":
@@ -638,8 +655,8 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
             logits = ws.logits_view(rows, w.shape[0])
             decode_ops.bf16_linear(ws.l_n[:rows], w, logits)
     else:
-        if plan is None:
-            check(actq.bonsai_add_rmsnorm_quant_int8(_vp(last_x), last_res, _vp(model.norm), eps,
+        if res is not None:
+            check(actq.bonsai_add_rmsnorm_quant_int8(_vp(last_x), res, _vp(model.norm), eps,
                                                      _vp(ws.h_last), _vp(ws.l_q), _vp(ws.l_s), rows,
                                                      dim, stream),
                   "bonsai_add_rmsnorm_quant_int8")
@@ -650,5 +667,60 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
         logits = ws.logits_view(rows, model.head_rows)
         _gemv(ws.l_q, ws.l_s, model.head, logits, rows, stream)
     # (the attention scratch is free again by now and far larger than the chain needs)
-    decode_ops.draft_chain(logits, args.vocab_size, threshold, io.tokens_out, io.conf, io.accept,
+    decode_ops.draft_chain(logits, args.vocab_size, threshold, tokens_out, conf, accept,
                            scratch=ws.attn_scratch)
+
+
+# ---------------------------------------------------------------------------
+# Prompts
+# ---------------------------------------------------------------------------
+# Rows of one block: what the buffers below are sized for at most (a row takes about 70 KB with the 4B
+# shape).  A default segment's whole prompt is one block, so every weight is read once.
+PROMPT_BLOCK_MAX = 4096
+
+
+class PromptBuffers:
+    """Intermediate buffers of a prompt block of up to ``rows`` rows."""
+
+    def __init__(self, args: ModelArgs, rows: int, device):
+        def buf(width, dtype):
+            return torch.empty((rows, width), dtype=dtype, device=device)
+        bf, i8, f32 = torch.bfloat16, torch.int8, torch.float32
+        self.rows = rows
+        self.h = [buf(args.dim, bf), buf(args.dim, bf)]
+        self.proj = buf(args.dim, bf)
+        self._rest = [buf(args.dim, i8), buf(1, f32), buf(args.q_dim + 2 * args.kv_dim, bf), buf(args.q_dim, bf),
+                      buf(args.q_dim, bf), buf(args.q_dim, i8), buf(1, f32), buf(2 * args.ffn_dim, bf),
+                      buf(args.ffn_dim, i8), buf(1, f32)]
+        a_q, a_s, xqkv, q, attn, o_q, o_s, gu, i_q, i_s = (t.data_ptr() for t in self._rest)
+        self.addresses = (self.h[0].data_ptr(), self.h[1].data_ptr(), a_q, a_s, xqkv, q, attn, o_q, o_s,
+                          self.proj.data_ptr(), gu, i_q, i_s)
+
+
+def prompt_layers(model: BonsaiDecoder) -> List[Tuple[int, ...]]:
+    """Weight addresses of every layer, as ``prefill_layers`` of csrc/py_ops.cpp takes them."""
+    return [tuple(t.data_ptr() for t in (lw.wqkv.weight, lw.wqkv.weight_scale, lw.wo.weight, lw.wo.weight_scale,
+                                         lw.w_gu.weight, lw.w_gu.weight_scale, lw.w_down.weight,
+                                         lw.w_down.weight_scale, lw.input_layernorm, lw.post_attention_layernorm,
+                                         lw.q_norm, lw.k_norm)) for lw in model.layers]
+
+
+def enqueue_prompt_block(model: BonsaiDecoder, buffers: PromptBuffers, tokens: torch.Tensor, base: int,
+                         positions: torch.Tensor, kv: torch.Tensor,
+                         rope: Tuple[torch.Tensor, torch.Tensor]) -> int:
+    """Enqueue the layers over prompt rows ``base .. base + len(tokens) - 1``: their keys and values go to the
+    history slots of the same numbers of ``kv`` ``[2, n_layers, n_kv, slots, 128]``.  ``positions``: int32, those
+    rows' positions.  Returns which of ``buffers.h`` holds the residual stream; the last MLP's output is still
+    to be added to it from ``buffers.proj``.  The operations and rounding points are those of a step
+    (reference: the variable-shape prompt forward, fast_generate.py:949-953)."""
+    args = model.args
+    m = tokens.numel()
+    if m > buffers.rows or base + m > kv.shape[3] or m < 1:
+        raise ValueError("the prompt block does not fit its buffers or its segment")
+    torch.index_select(model.embed, 0, tokens, out=buffers.h[0][:m])
+    cos, sin = rope
+    dims = (model.layers[0].wo.bits, m, base, args.dim, args.n_heads, args.n_kv_heads, args.ffn_dim, kv.shape[3],
+            cos.shape[0], len(model.layers), kv.data_ptr())
+    return ops.native().prefill_layers(
+        model.device.index or 0, dims, float(args.norm_eps), 1.0 / math.sqrt(HEAD_DIM),
+        buffers.addresses + (positions.data_ptr(), cos.data_ptr(), sin.data_ptr()), prompt_layers(model))

@@ -222,6 +222,13 @@ def _load_native() -> None:
     _native = module
 
 
+def native():
+    """The extension module (csrc/py_ops.cpp)."""
+    if _native is None:
+        _load_native()
+    return _native
+
+
 def t2_lib() -> ctypes.CDLL:
     if _t2_lib is None:
         load_t2_kernel()

@@ -29,7 +29,8 @@ import numpy as np
 import torch
 
 from . import contracts, decode_ops, ops
-from .model import BonsaiDecoder, StepIO, Workspace, enqueue_step, rope_tables
+from .model import (PROMPT_BLOCK_MAX, BonsaiDecoder, PromptBuffers, StepIO, Workspace, enqueue_prompt_block,
+                    enqueue_step, project_rows, rope_tables)
 
 DEFAULT_SEGMENT_LADDER = (256, 1024, 4096)
 DEFAULT_M_SET = (1, 8, 9, 10, 12, 16, 17)
@@ -175,6 +176,8 @@ class GraphAtlas:
                                    logits_ld_max=model.max_logits_ld())
         self.rope = rope_tables(self.args, max_slots, self.device)
         self.graphs: Dict[Tuple[int, int, str], CapturedGraph] = {}
+        self._prompt: Optional[PromptBuffers] = None   # sized by the longest block so far
+        self._positions: Optional[torch.Tensor] = None
         self.replays = 0
 
     def synchronize(self) -> None:
@@ -302,6 +305,34 @@ class GraphAtlas:
                            logits_start=ls, logits_end=le)
         cg._eager = run
         return cg
+
+    # -- prompts -------------------------------------------------------------
+    def prefill_prompt(self, prompt: Sequence[int], sigma: int) -> int:
+        """Materialise a prompt's KV in segment sigma, in blocks of up to ``PROMPT_BLOCK_MAX`` rows, and return
+        the token after it.  A block reads every weight once and projects its last row only; the replayed
+        graphs do both for every ``prefill_width`` rows."""
+        n = len(prompt)
+        if n > sigma:
+            raise RuntimeError("history does not fit the segment")
+        kv = self.kv(sigma)
+        block = min(n, PROMPT_BLOCK_MAX)
+        with torch.inference_mode(False), torch.cuda.device(self.device):
+            if self._prompt is None or self._prompt.rows < block:
+                self._prompt = None
+                self._prompt = PromptBuffers(self.args, min(-(-block // 256) * 256, PROMPT_BLOCK_MAX), self.device)
+            if self._positions is None:
+                self._positions = torch.arange(self.rope[0].shape[0], dtype=torch.int32, device=self.device)
+                self._prompt_out = torch.zeros(4, dtype=torch.int32, device=self.device)
+            buffers, out = self._prompt, self._prompt_out
+            tokens = torch.from_numpy(np.asarray(prompt, dtype=np.int32)).to(self.device)
+            for base in range(0, n, block):
+                m = min(block, n - base)
+                cur = enqueue_prompt_block(self.model, buffers, tokens[base: base + m], base,
+                                           self._positions[base: base + m], kv, self.rope)
+            last = m - 1
+            project_rows(self.model, self.workspace, buffers.proj[last: m], buffers.h[cur][last: m], 1, self.threshold,
+                         out[:1], out[1:2].view(torch.float32), out[2:4])
+            return int(out[0].item())
 
     # -- one replay ----------------------------------------------------------
     def replay(self, g: CapturedGraph, tokens: Sequence[int], positions: Sequence[int],

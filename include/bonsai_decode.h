@@ -47,6 +47,7 @@ extern "C" {
 #define BONSAI_HEAD_DIM 128     /* the only head size of the Bonsai/Qwen3 family */
 #define BONSAI_MAX_WIDTH 32     /* rows per step (the reference uses at most 17) */
 #define BONSAI_ATTN_CHUNK 64    /* KV slots per attention work item */
+#define BONSAI_PREFILL_MAX_ROWS 65535 /* rows of a prompt block */
 
 /* Replaces `_fused_qkv_qknorm_rope_kv_write` (src/bonsai_sft/gpu/model.py:388-436).
  *   xqkv      bf16 [M, (n_heads + 2 n_kv) * 128]   merged q|k|v GEMV output
@@ -63,6 +64,23 @@ int bonsai_qk_norm_rope_kv_write(const void *xqkv, const void *q_norm_w, const v
                                  const int32_t *positions, void *q_out, void *k_layer,
                                  void *v_layer, int M, int n_heads, int n_kv, int slots,
                                  int write_slot, int max_pos, void *stream);
+
+/* ---- prompts -------------------------------------------------------------------------
+ * The two calls above for a block of prompt rows of any height (M <= BONSAI_PREFILL_MAX_ROWS) whose
+ * keys and values go straight into the history: rows base .. base + M - 1 of the sequence, in the
+ * slots of the same numbers.  bonsai_prefill_rope_kv_write takes write_slot = base;
+ * bonsai_prefill_attention lets row i see slots 0 .. base + i (causal, everything earlier visible):
+ *   q bf16 [M, n_heads, 128], k_layer / v_layer bf16 [n_kv, slots, 128], out bf16 [M, n_heads * 128].
+ * Reference: the variable-shape prompt forward (src/bonsai_sft/gpu/fast_generate.py:949-953 with
+ * model.py:388-436 and :996-1005). */
+int bonsai_prefill_rope_kv_write(const void *xqkv, const void *q_norm_w, const void *k_norm_w,
+                                 float eps, const void *cos_table, const void *sin_table,
+                                 const int32_t *positions, void *q_out, void *k_layer,
+                                 void *v_layer, int M, int n_heads, int n_kv, int slots,
+                                 int write_slot, int max_pos, void *stream);
+int bonsai_prefill_attention(const void *q, const void *k_layer, const void *v_layer, void *out_bf16,
+                             float scale, int M, int n_heads, int n_kv, int slots, int base,
+                             void *stream);
 
 /* Process-wide tuning of the attention launch geometry: query rows per wave (1..4), 0 =
  * built-in heuristic.  No counterpart in the reference; results do not depend on it. */

@@ -1,0 +1,98 @@
+"""The prompt path: causal attention of wide blocks against float64, and whole prompts against the same decoder
+stepped through its captured graphs."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("m,n_heads,n_kv,base,slots", [
+    (1, 16, 8, 0, 40), (64, 16, 8, 0, 96), (65, 16, 8, 63, 160), (127, 4, 4, 1, 128), (130, 32, 8, 190, 400),
+    (300, 6, 2, 77, 500), (33, 3, 1, 1000, 1100), (515, 16, 8, 0, 515)])
+def test_prefill_attention_against_float64(m, n_heads, n_kv, base, slots):
+    from bitmtp_amd import decode_ops
+    print(f"[case] prefill attention m={m} heads={n_heads}/{n_kv} base={base}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(m + base)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    q = rnd(m, n_heads, 128).to(torch.bfloat16)
+    k, v = rnd(n_kv, slots, 128).to(torch.bfloat16), rnd(n_kv, slots, 128).to(torch.bfloat16)
+    k[:, base + m:] = float("nan")   # slots behind the block are never read
+    v[:, base + m:] = float("nan")
+    out = decode_ops.prefill_attention(q, k, v, base)
+    torch.cuda.synchronize()
+    seen = base + m
+    hpg = n_heads // n_kv
+    qd = q.double().transpose(0, 1).reshape(n_kv, hpg * m, 128)
+    s = torch.bmm(qd, k[:, :seen].double().transpose(1, 2).contiguous()) / np.sqrt(128.0)
+    s = s.view(n_kv, hpg, m, seen)
+    ok = torch.arange(seen, device=DEV)[None, :] <= base + torch.arange(m, device=DEV)[:, None]
+    p = torch.softmax(s.masked_fill(~ok, float("-inf")), dim=-1)
+    want = torch.bmm(p.view(n_kv, hpg * m, seen), v[:, :seen].double()).view(n_heads, m, 128).transpose(0, 1)
+    got = out.view(m, n_heads, 128).double()
+    assert torch.isfinite(got).all()
+    assert ((got - want).abs() <= 2e-3 + 2e-2 * want.abs()).all()
+
+
+def test_prefill_attention_argument_checks():
+    from bitmtp_amd import decode_ops
+    q = torch.zeros(8, 4, 128, dtype=torch.bfloat16, device=DEV)
+    k = torch.zeros(2, 16, 128, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(RuntimeError):
+        decode_ops.prefill_attention(q, k, k, 9)          # runs past the slots
+    with pytest.raises(RuntimeError):
+        decode_ops.prefill_attention(q[:, :3].contiguous(), k, k, 0)   # heads not a multiple of the kv heads
+
+
+def _replayed(atlas, prompt, sigma):
+    """The prompt through width-32 replays of the captured AR graph; the last row's logits."""
+    W = atlas.prefill_width
+    g = atlas.get_graph(W, sigma, "ar")
+    for c in range(0, len(prompt), W):
+        take = min(W, len(prompt) - c)
+        atlas.replay(g, list(prompt[c:c + take]) + [0] * (W - take), [c + i for i in range(W)], c)
+        atlas.commit_kv(sigma, c, take)
+    atlas.read_outputs(g)
+    logits = atlas.workspace.logits_buf[: W * atlas.workspace.logits.shape[1]].view(W, -1)
+    return logits[take - 1].float().clone()
+
+
+@pytest.mark.parametrize("kind,head,n,block", [("t2g128", None, 33, None), ("t2g128", None, 200, 96),
+                                               ("q1", "bf16", 157, None), ("q1", "q1", 70, 64)])
+def test_prompt_block_against_replayed_steps(kind, head, n, block, monkeypatch):
+    """Keys, values and last-row logits of the prompt path are those of the stepped decoder: the first layer to the
+    bit (the same sums), deeper ones and the logits within the order of the attention's sums."""
+    from bitmtp_amd import generate, runtime
+    from bitmtp_amd.model import BonsaiDecoder, ModelArgs
+    from bitmtp_amd.runtime import GraphAtlas
+    print(f"[case] prompt {kind} head={head} n={n} block={block}", flush=True)
+    args = ModelArgs(dim=512, n_layers=3, n_heads=4, n_kv_heads=2, ffn_dim=1024, vocab_size=1000,
+                     mask_token_id=999, kernel_kind=kind)
+    model = BonsaiDecoder.random_init(args, seed=5, device=DEV, head_kind=head)
+    atlas = GraphAtlas(model, segment_ladder=(256,))
+    prompt = np.random.default_rng(n).integers(0, 1000, n).tolist()
+    want_logits = _replayed(atlas, prompt, 256)
+    want = atlas.kv(256)[:, :, :, :n].clone()
+    atlas.kv(256).fill_(float("nan"))
+    if block is not None:
+        monkeypatch.setattr(runtime, "PROMPT_BLOCK_MAX", block)
+    first = generate.prefill(atlas, prompt, 256)
+    got = atlas.kv(256)[:, :, :, :n]
+    logits = atlas.workspace.logits_buf[: want_logits.numel()].float()
+    scale = want_logits.abs().max()
+    assert (logits - want_logits).abs().max() <= 6e-2 * scale
+    assert first == int(logits[:1000].argmax())
+    d0 = (got[:, 0].float() - want[:, 0].float()).abs()
+    assert d0.max() <= 2e-2 * want[:, 0].float().abs().max() and (d0 > 0).float().mean() < 1e-2
+    assert (got.float() - want.float()).norm() <= 3e-2 * want.float().norm()
+
+
+def test_prompt_longer_than_its_segment_is_refused():
+    from bitmtp_amd import generate
+    from bitmtp_amd.model import BonsaiDecoder, ModelArgs
+    from bitmtp_amd.runtime import GraphAtlas
+    args = ModelArgs(dim=512, n_layers=1, n_heads=4, n_kv_heads=2, ffn_dim=1024, vocab_size=1000, mask_token_id=999)
+    atlas = GraphAtlas(BonsaiDecoder.random_init(args, seed=5, device=DEV), segment_ladder=(64,))
+    with pytest.raises(RuntimeError):
+        generate.prefill(atlas, [1] * 65, 64)
