@@ -360,16 +360,18 @@ int launch_grouped_mx_only(const GemvProblem &q, int out_kind, int scale_kind, i
 // the dot4 kernel they leave (12288 x 1920 at nine tokens: dot4 9.2 us).
 inline bool lean_any_k(int K) { return K % 512 != 0 && K > 512; }
 
-// Blocks the wide kernel takes.  The lean kernel's 16-token tiles are ahead up to about six of its
-// workgroups per CU (12288 x 2048 at 32 tokens 7.2 us against 7.3, at 48 12.7 / 9.3; 2048 x 2048 at 128
-// 5.8 / 7.2, at 256 10.3 / 7.6; 2560 x 9728 at 128 18.4 / 20.3, at 192 26.6 / 21.2), and at a few tokens
-// over 16 also above that (19456 x 2560 at 24 tokens 9.9 / 11.9, at 32 12.9 / 12.1).  What the lean kernel
-// does not take leaves only the dot4 kernel where K is not a multiple of 512 (19000 x 2688: dot4 9.1 us at
-// four tokens, 15.5 at nine, against 10.6 at any width up to 32).
+// Blocks the wide kernel takes: where it is expected to be faster than the lean kernel's 16-token tiles, whose
+// time is a fit to the same sweep as wide_estimate (12288 x 2048: 6.3 / 6.4 us at 17 tokens, 8.0 / 6.6 at 32;
+// 2048 x 2048: 4.7 / 6.3 at 64, 6.5 / 6.5 at 128; 2560 x 9728: 12.5 / 14.3 at 64, 16.6 / 15 at 96).  What the
+// lean kernel does not take leaves only the dot4 kernel where K is not a multiple of 512 (19000 x 2688: dot4
+// 9.1 us at four tokens, 15.5 at nine, against 10.6 at any width up to 32).
 inline bool wide_default(int M, int N, int K, int n_cus) {
     const long lean_tiles = (long)((M + kMfmaTokens - 1) / kMfmaTokens) * ((N + 15) / 16);
     if (K % 512 != 0 && (lean_tiles > 8L * n_cus || N > kLongMatrixRows || K < 512)) return M >= kWideMinRagged;
-    return M > 24 && lean_tiles > 6L * n_cus;
+    if (M <= kMfmaTokens) return false;
+    const double G = K / kGroup;
+    const double lean = 3.1 + G * (0.0087 + 0.051 * lean_tiles / n_cus);
+    return wide_estimate(wide_pick(M, N, K, n_cus), M, N, K, n_cus) < lean;
 }
 
 template <int BITS>

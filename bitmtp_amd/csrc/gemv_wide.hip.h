@@ -1,27 +1,33 @@
 // Matrix-core kernel for wide blocks (prompts, batches of requests): more than 16 tokens.
 //
 // Below 16 tokens a packed projection streams its weights and is bound by latency and bytes; here
-// every weight is multiplied with tens to thousands of tokens, and what bounds the kernel is the
-// vector ALU: per scale group (128 of K) and 16 x 16 results, two v_mfma_i32_16x16x64_i8 (32 clocks)
-// leave exact int32 group sums that must become fp32 and meet the group's scale -- eight vector
-// operations, 32 clocks as well -- beside the unpacking of the weights.  The token-tiled decode
-// kernels unpack every weight once per 16 tokens (14 operations per 16 x 16 results and group) and
-// re-read the activations for every 16 rows.  Here a wave holds MT x NT tiles of 16 tokens x 16 rows:
-// an unpacked operand serves MT tiles, an activation operand read from LDS serves NT, and the offset
-// term (two more MFMAs per 16 tokens and group against an operand of all -2 / -1, as in
-// gemv_mxl.hip.h) serves NT as well.
+// every weight is multiplied with tens to thousands of tokens, and what bounds the kernel is the issue
+// of vector instructions: per scale group (128 of K) the exact int32 sums must become fp32 and meet the
+// group's scale, two operations a result (eight per 16 x 16 results, against two matrix instructions),
+// beside unpacking the weights and arranging the activations.  On this part a wave that is alone on its
+// SIMD issues a vector operation every 8.7 clocks, two waves every 5.5, four every 4.7, and a matrix
+// instruction costs 8 of issue whatever its size.  So
+//   * v_mfma_i32_32x32x32_i8: half the matrix instructions of the 16 x 16 form;
+//   * weights are unpacked to 64 times their value (mfma_unpack64), which needs no offset term -- the
+//     other forms feed -2 sum(a) through the accumulator, 8 more matrix instructions per 16 x 64 x 64 --
+//     and the factor, a power of two, goes out with the division;
+//   * the accumulators start from the bits of 1.5 * 2^23, so that a sum is a float and one exact
+//     subtraction stands for the conversion;
+//   * 64 tokens x 32 rows a wave in 128 registers, four waves a SIMD, are ahead of 64 x 64 in 224.
+// 19456 x 2560 at 3001 tokens 254 -> 206 us (1.45 POP/s), 2560 x 9728 123 -> 97, 12288 x 2048 at 514
+// 35 -> 27, at 256 19.6 -> 16.8, 2048 x 2048 at 256 7.1 -> 6.6.
 //
-//   WM x WN waves share a staged block of WM*MT*16 tokens x WN*NT*16 rows; KS such sets of waves
+//   WM x WN waves share a staged block of WM*MT*32 tokens x WN*NT*32 rows; KS such sets of waves
 //   split K and add their fp32 results up in slice order (narrower blocks and few rows, where a
 //   tile per workgroup would leave most CUs idle).
 //
 // Per group a set stages 128 bytes of K for its tokens (4 x 4 byte transposes: operand order, see
-// gemv_core.h; 16-byte units XORed with the row number, so that a ds_read_b128 of 16 rows meets every
-// bank once) and the packed rows as they are (a wave's operand read is 512 contiguous bytes).  The
-// loads of group g + 2 are in flight and group g + 1 is being parked while group g is multiplied: one
-// barrier per group, none where a set is a single wave.  All scales of the row block (G x rows,
-// transposed) and the multipliers are staged once.  Rows past N and tokens past M read as zero through
-// the buffer range check.
+// gemv_core.h; 16-byte units XORed with half the row number, so that a ds_read_b128 of 16 rows meets
+// every bank once) and the packed rows, inverted where the unpacking wants it (a wave's operand read is
+// 512 or 1024 contiguous bytes).  The loads of group g + 2 are in flight and group g + 1 is being parked
+// while group g is multiplied: one barrier per group, none where a set is a single wave.  All scales of
+// the row block (G x rows, transposed), the multipliers and their reciprocals are staged once.  Rows past
+// N and tokens past M read as zero through the buffer range check.
 //
 // Arithmetic and rounding points are those of the other kernels: exact G, fp32 scale-accumulate with
 // groups in ascending order inside a slice, slices in order, division by s[m], bf16 RNE.
@@ -45,22 +51,22 @@ constexpr int kWideTokenGroup = 8;  // token tiles walked before the next row ti
 
 template <int BITS, int WM, int WN, int KS, int MT, int NT>
 struct WideShape {
-    static constexpr int kTokens = WM * MT * 16, kRows = WN * NT * 16;
+    static constexpr int kTokens = WM * MT * 32, kRows = WN * NT * 32;
     static constexpr int kSet = 64 * WM * WN;  // threads that share a staged block
     static constexpr int kThreads = kSet * KS;
     static constexpr bool kPrivate = WM * WN == 1;  // a set is one wave: program order is enough
     static constexpr int kBufs = kPrivate ? 1 : 2;
-    static constexpr int kAhead = kPrivate && MT <= 2 ? 2 : 1;  // register sets of staging loads in flight
+    static constexpr int kAhead = kPrivate ? 2 : 1;  // register sets of staging loads in flight
     static constexpr int kABytes = kTokens * 128, kBBytes = kRows * 16 * BITS;
     static constexpr int kSetBytes = kBufs * (kABytes + kBBytes);
-    static constexpr int kElems = MT * NT * 4;  // results per lane
+    static constexpr int kElems = MT * NT * 16;  // results per lane
     static constexpr int kOutPitch = kRows * 2 + 16;
     static constexpr int kShare = kElems / KS;  // results per lane that a K slice finishes
     static constexpr int kRedBytes = (KS - 1) * kSet * kElems * 4;
-    // scales [G][rows] u16, then multipliers [tokens] fp32 (they stay), then the staged blocks, whose
+    // scales [G][rows] u16, then multipliers and their reciprocals [tokens] (they stay), then the staged blocks, whose
     // space the K slices' partial sums and the outgoing tile take over
     static size_t lds_bytes(int K) {
-        const size_t keep = (size_t)(K / kGroup) * kRows * 2 + kTokens * 4;
+        const size_t keep = (size_t)(K / kGroup) * kRows * 2 + kTokens * 8;
         const size_t stage = (size_t)KS * kSetBytes;
         const size_t after = kRedBytes + (size_t)kTokens * kOutPitch;
         return keep + (stage > after ? stage : after);
@@ -74,7 +80,7 @@ __device__ __forceinline__ void wide_barrier() {
 }
 
 template <int BITS, int WM, int WN, int KS, int MT, int NT, bool SF16, bool G32>
-__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : 4)))
 gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
                  int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
     using S = WideShape<BITS, WM, WN, KS, MT, NT>;
@@ -102,10 +108,10 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     const int set = wave / (WM * WN), wsub = wave % (WM * WN);
     const int stid = tid - set * S::kSet;
     const int wm = wsub / WN, wn = wsub % WN;
-    const int op_row = lane & 15, kb = lane >> 4;
+    const int op_row = lane & 31, kb = lane >> 5;
 
     uint16_t *scales = reinterpret_cast<uint16_t *>(smem);
-    float *mult = reinterpret_cast<float *>(smem + (size_t)G * S::kRows * 2);
+    float2 *mult = reinterpret_cast<float2 *>(smem + (size_t)G * S::kRows * 2);
     unsigned char *work = reinterpret_cast<unsigned char *>(mult + S::kTokens);
     unsigned char *abuf = work + set * S::kSetBytes;
     unsigned char *bbuf = abuf + S::kBufs * S::kABytes;
@@ -126,11 +132,11 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     constexpr int QB = mfma_quarter_bytes<BITS>();
     constexpr int QW = QB / 16;
     constexpr int QPR = 128 / QB;                       // quarters of a token row
-    constexpr int AL = S::kTokens * QPR / S::kSet;      // quarters a thread stages
+    constexpr int AN_TASKS = S::kTokens * QPR;
+    constexpr int AL = (AN_TASKS + S::kSet - 1) / S::kSet;  // quarters a thread stages
     constexpr int BCH = BITS;                           // 16-byte chunks of a packed row
     constexpr int BN_TASKS = S::kRows * BCH;
     constexpr int BL = (BN_TASKS + S::kSet - 1) / S::kSet;
-    static_assert(AL * S::kSet == S::kTokens * QPR && AL >= 1, "staging tasks divide evenly");
     uint32_t a_off[AL], b_off[BL];
 #pragma unroll
     for (int i = 0; i < AL; ++i) {
@@ -146,8 +152,10 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     auto load = [&](auto &ar, auto &br, int g) {
 #pragma unroll
         for (int i = 0; i < AL; ++i)
+            if (AN_TASKS % S::kSet == 0 || stid + i * S::kSet < AN_TASKS) {
 #pragma unroll
-            for (int q = 0; q < QW; ++q) ar[i][q] = mxl_load_b128(rA, a_off[i] + q * 16, (uint32_t)(g * 128));
+                for (int q = 0; q < QW; ++q) ar[i][q] = mxl_load_b128(rA, a_off[i] + q * 16, (uint32_t)(g * 128));
+            }
 #pragma unroll
         for (int i = 0; i < BL; ++i)
             if (BN_TASKS % S::kSet == 0 || stid + i * S::kSet < BN_TASKS)
@@ -158,9 +166,10 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
 #pragma unroll
         for (int i = 0; i < AL; ++i) {
             const int task = stid + i * S::kSet;
+            if (AN_TASKS % S::kSet != 0 && task >= AN_TASKS) continue;
             const int row = task / QPR, q = task % QPR;
             u32x4 *dst = a + row * 8;
-            const int x = row & 7;
+            const int x = (row >> 1) & 7;
             if (BITS == 2) {
                 const u32x4 v = ar[i][0];
                 dst[q ^ x] = transpose4x4_bytes(v.x, v.y, v.z, v.w);
@@ -173,7 +182,8 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
         u32x4 *b = reinterpret_cast<u32x4 *>(bbuf + buf * S::kBBytes);
 #pragma unroll
         for (int i = 0; i < BL; ++i)
-            if (BN_TASKS % S::kSet == 0 || stid + i * S::kSet < BN_TASKS) b[stid + i * S::kSet] = br[i];
+            if (BN_TASKS % S::kSet == 0 || stid + i * S::kSet < BN_TASKS)
+                b[stid + i * S::kSet] = u32x4{mfma_flip<BITS>(br[i].x), mfma_flip<BITS>(br[i].y), mfma_flip<BITS>(br[i].z), mfma_flip<BITS>(br[i].w)};
     };
 
     load(ars[0], brs[0], gb < ge ? gb : 0);
@@ -182,12 +192,13 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     if (!G32) {
         const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint16_t *>(ws + (size_t)n0 * G), 0, nv * G * 2, kMxlBufferWord3);
-        if (flags & 1) {  // whole quads of groups, aligned
-            const int quads = G >> 2;
-            for (int i = tid; i < S::kRows * quads; i += S::kThreads) {
-                const int row = i / quads, q = i - row * quads;
-                typedef unsigned int v2u __attribute__((ext_vector_type(2)));
-                const v2u v = __builtin_amdgcn_raw_buffer_load_b64(rS, i * 8, 0, 0);
+        if (flags & 1) {  // whole quads of groups, aligned: a thread's quads are those of one row
+            typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+            constexpr int kPerRow = S::kThreads / S::kRows;
+            static_assert(kPerRow * S::kRows == S::kThreads, "threads divide among the rows");
+            const int row = tid % S::kRows;
+            for (int q = tid / S::kRows; q < G >> 2; q += kPerRow) {
+                const v2u v = __builtin_amdgcn_raw_buffer_load_b64(rS, row * (G * 2) + q * 8, 0, 0);
                 uint16_t *d = scales + (q * 4) * S::kRows + row;
                 d[0] = (uint16_t)v.x;
                 d[S::kRows] = (uint16_t)(v.x >> 16);
@@ -200,23 +211,28 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                 scales[g * S::kRows + row] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rS, i * 2, 0, 0);
             }
         }
-        for (int i = tid; i < S::kTokens; i += S::kThreads) mult[i] = s[m0 + (i < mv ? i : mv - 1)];
+        // (the sums come out 64 times too large, mfma_unpack64: so does what divides them)
+        for (int i = tid; i < S::kTokens; i += S::kThreads) {
+            const float d = s[m0 + (i < mv ? i : mv - 1)] * 64.0f;
+            mult[i] = make_float2(d, 1.0f / d);
+        }
     }
 
-    float acc[MT][NT][4];
+    typedef int v16i __attribute__((ext_vector_type(16)));
+    float acc[MT][NT][16];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
-    constexpr int kNegs = BITS == 2 ? (int)0xFEFEFEFEu : (int)0xFFFFFFFFu;
-    const v4i negs = {kNegs, kNegs, kNegs, kNegs};
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     // The accumulators start from the bits of 1.5 * 2^23 (|G| < 2^22): the sums then ARE floats,
     // 12582912 + G, and one exact subtraction at full rate takes the place of an int-to-float conversion.
     constexpr int kBias = 0x4B400000;
     constexpr float kBiasF = 12582912.0f;
-    const v4i bias4 = {kBias, kBias, kBias, kBias};
+    v16i bias16;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bias16[r] = kBias;
 
     if (S::kPrivate) {
         if (S::kAhead > 1 && gb + 1 < ge) load(ars[S::kAhead - 1], brs[S::kAhead - 1], gb + 1);
@@ -239,57 +255,61 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
             if (g + 2 < ge) load(ars[0], brs[0], g + 2);
         }
         if (g >= ge) return;  // (uniform in a set)
-        const u32x4 *a = reinterpret_cast<const u32x4 *>(abuf + buf * S::kABytes) + (wm * MT * 16 + op_row) * 8;
-        const unsigned char *b = bbuf + buf * S::kBBytes + (wn * NT * 16 + op_row) * (16 * BITS) + kb * (4 * BITS);
-        const int x = op_row & 7;
-        v4i va0[MT], va1[MT], vc[MT];
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            const u32x4 u0 = a[i * 128 + ((2 * kb) ^ x)], u1 = a[i * 128 + ((2 * kb + 1) ^ x)];
-            va0[i] = v4i{(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w};
-            va1[i] = v4i{(int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
-        }
-#pragma unroll
-        for (int i = 0; i < MT; ++i) vc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va0[i], negs, bias4, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) vc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va1[i], negs, vc[i], 0, 0, 0);
+        // lane half kb takes 16-byte units 4 kb + t of the group, t the number of the matrix instruction
+        const u32x4 *a = reinterpret_cast<const u32x4 *>(abuf + buf * S::kABytes) + (wm * MT * 32 + op_row) * 8;
+        const unsigned char *b = bbuf + buf * S::kBBytes + (wn * NT * 32 + op_row) * (16 * BITS) + kb * (8 * BITS);
+        const int x = (op_row >> 1) & 7;
+        v4i vb[NT][4];
+        float w[NT];
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            uint32_t p0, p1 = 0;
+            uint32_t p[4] = {0u, 0u, 0u, 0u};
             if (BITS == 2) {
-                const uint2 pp = *reinterpret_cast<const uint2 *>(b + j * 16 * 16 * BITS);
-                p0 = pp.x;
-                p1 = pp.y;
+                const u32x4 pp = *reinterpret_cast<const u32x4 *>(b + j * 32 * 16 * BITS);
+                p[0] = pp.x;
+                p[1] = pp.y;
+                p[2] = pp.z;
+                p[3] = pp.w;
             } else {
-                p0 = *reinterpret_cast<const uint32_t *>(b + j * 16 * 16 * BITS);
+                const uint2 pp = *reinterpret_cast<const uint2 *>(b + j * 32 * 16 * BITS);
+                p[0] = pp.x;
+                p[2] = pp.y;
             }
-            float w = 0.0f;
-            if (!G32) w = scale_to_f32<SF16>(scales[g * S::kRows + (wn * NT + j) * 16 + op_row]);
-            uint32_t b0[4], b1[4];
-            mfma_unpack<BITS>(p0, p1, b0, b1);
-            const v4i vb0 = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3]};
-            const v4i vb1 = {(int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
-            v4i dd[MT];
+            w[j] = G32 ? 0.0f : scale_to_f32<SF16>(scales[g * S::kRows + (wn * NT + j) * 32 + op_row]);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) dd[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va0[i], vb0, vc[i], 0, 0, 0);
+            for (int t = 0; t < 4; t += 2) {
+                uint32_t b0[4], b1[4];
+                mfma_unpack64<BITS>(p[t], p[t + 1], b0, b1);
+                vb[j][t] = v4i{(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3]};
+                vb[j][t + 1] = v4i{(int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
+            }
+        }
 #pragma unroll
-            for (int i = 0; i < MT; ++i) dd[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(va1[i], vb1, dd[i], 0, 0, 0);
-            if (G32) {
-                const int n = (wn * NT + j) * 16 + op_row;
+        for (int i = 0; i < MT; ++i) {
+            v4i va[4];
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
+            for (int t = 0; t < 4; ++t) {
+                const u32x4 u = a[i * 256 + ((4 * kb + t) ^ x)];
+                va[t] = v4i{(int)u.x, (int)u.y, (int)u.z, (int)u.w};
+            }
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int m = (wm * MT + i) * 16 + 4 * kb + r;
+            for (int j = 0; j < NT; ++j) {
+                v16i dd = bias16;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[t], vb[j][t], dd, 0, 0, 0);
+                if (G32) {
+                    const int n = (wn * NT + j) * 32 + op_row;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = (wm * MT + i) * 32 + 8 * (r / 4) + 4 * kb + r % 4;
                         if (m < mv && n < nv)
-                            reinterpret_cast<int32_t *>(out)[((size_t)(m0 + m) * N + n0 + n) * G + g] = dd[i][r] - kBias;
+                            reinterpret_cast<int32_t *>(out)[((size_t)(m0 + m) * N + n0 + n) * G + g] = (dd[r] - kBias) >> 6;
                     }
-                continue;
+                    continue;
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] += (__int_as_float(dd[r]) - kBiasF) * w[j];
             }
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[i][j][r] += (__int_as_float(dd[i][r]) - kBiasF) * w;
         }
     };
     for (int it = 0; it < iters; it += S::kAhead) {
@@ -306,13 +326,27 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     };
     __syncthreads();  // the staged blocks are free
     unsigned char *tile = work + S::kRedBytes;
-    const auto finish = [&](int i, int j, int r, float y, float d, float inv) {
-        const int m = (wm * MT + i) * 16 + 4 * kb + r, n = (wn * NT + j) * 16 + op_row;
-        y = divide(y, d, inv);
+    const auto place = [&](int i, int j, int r, int &m, int &n) {
+        m = (wm * MT + i) * 32 + 8 * (r / 4) + 4 * kb + r % 4;
+        n = (wn * NT + j) * 32 + op_row;
+    };
+    const auto finish = [&](int i, int j, int r, float y0, float y1) {  // results r, r + 1
+        int m, n;
+        place(i, j, r, m, n);
+        const float2 d0 = mult[m], d1 = mult[m + 1];
+        y0 = divide(y0, d0.x, d0.y);
+        y1 = divide(y1, d1.x, d1.y);
         if (out_f32) {
-            if (m < mv && n < nv) reinterpret_cast<float *>(out)[(size_t)(m0 + m) * N + n0 + n] = y;
+            float *o = reinterpret_cast<float *>(out) + (size_t)(m0 + m) * N + n0 + n;
+            if (m < mv && n < nv) o[0] = y0;
+            if (m + 1 < mv && n < nv) o[N] = y1;
         } else {
-            *reinterpret_cast<uint16_t *>(tile + m * S::kOutPitch + n * 2) = f32_to_bf16_rne_nobranch(y);
+            typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+            const bf2 p = {static_cast<__bf16>(y0), static_cast<__bf16>(y1)};  // round to nearest even
+            uint16_t u[2];
+            __builtin_memcpy(u, &p, 4);
+            *reinterpret_cast<uint16_t *>(tile + m * S::kOutPitch + n * 2) = u[0];
+            *reinterpret_cast<uint16_t *>(tile + (m + 1) * S::kOutPitch + n * 2) = u[1];
         }
     };
     if (KS > 1) {
@@ -329,7 +363,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
 #pragma unroll
                 for (int k = 0; k < S::kShare; ++k) {
                     const int e = z * S::kShare + k;
-                    slot(z, set, k) = acc[e / (NT * 4)][e / 4 % NT][e % 4];
+                    slot(z, set, k) = acc[e / (NT * 16)][e / 16 % NT][e % 16];
                 }
             }
         __syncthreads();
@@ -337,25 +371,27 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
         for (int z = 0; z < KS; ++z)
             if (z == set) {
 #pragma unroll
-                for (int k = 0; k < S::kShare; ++k) {
-                    const int e = z * S::kShare + k;
-                    const float own = acc[e / (NT * 4)][e / 4 % NT][e % 4];
-                    float y = z == 0 ? own : slot(z, 0, k);
+                for (int k = 0; k < S::kShare; k += 2) {
+                    float y[2];
 #pragma unroll
-                    for (int src = 1; src < KS; ++src) y += src == z ? own : slot(z, src, k);
-                    const float d = mult[(wm * MT + e / (NT * 4)) * 16 + 4 * kb + e % 4];
-                    finish(e / (NT * 4), e / 4 % NT, e % 4, y, d, 1.0f / d);
+                    for (int h = 0; h < 2; ++h) {
+                        const int e = z * S::kShare + k + h;
+                        const float own = acc[e / (NT * 16)][e / 16 % NT][e % 16];
+                        y[h] = z == 0 ? own : slot(z, 0, k + h);
+#pragma unroll
+                        for (int src = 1; src < KS; ++src) y[h] += src == z ? own : slot(z, src, k + h);
+                    }
+                    const int e = z * S::kShare + k;
+                    finish(e / (NT * 16), e / 16 % NT, e % 16, y[0], y[1]);
                 }
             }
     } else {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float d = mult[(wm * MT + i) * 16 + 4 * kb + r], inv = 1.0f / d;
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) finish(i, j, r, acc[i][j][r], d, inv);
-            }
+                for (int r = 0; r < 16; r += 2) finish(i, j, r, acc[i][j][r], acc[i][j][r + 1]);
     }
     if (out_f32) return;
     __syncthreads();
@@ -397,12 +433,14 @@ constexpr WideVariant wide_variant() {
                        S::kTokens, S::kRows, S::kThreads, S::lds_bytes, {WM, WN, KS, MT, NT}};
 }
 
-enum : int { WIDE_128x128 = 0, WIDE_32x64, kWideVariants };
+// (tokens x rows of a workgroup, K slices)
+enum : int { WIDE_64x256 = 0, WIDE_64x128_K2, WIDE_32x64_K4, WIDE_32x64_K8, WIDE_64x128_K4, WIDE_128x256, kWideVariants };
 
 template <int BITS>
 const WideVariant &wide_kernel(int v) {
-    static const WideVariant t[kWideVariants] = {wide_variant<BITS, 2, 2, 1, 4, 4>(),
-                                                 wide_variant<BITS, 1, 1, 4, 2, 4>()};
+    static const WideVariant t[kWideVariants] = {wide_variant<BITS, 1, 8, 1, 2, 1>(), wide_variant<BITS, 1, 4, 2, 2, 1>(),
+                                                 wide_variant<BITS, 1, 2, 4, 1, 1>(), wide_variant<BITS, 1, 1, 8, 1, 2>(),
+                                                 wide_variant<BITS, 1, 4, 4, 2, 1>(), wide_variant<BITS, 2, 4, 1, 2, 2>()};
     return t[v];
 }
 
@@ -416,23 +454,31 @@ int wide_init_device(int max_lds) {
     return 0;
 }
 
-// Which variant a shape gets: the smaller of the two estimates, in microseconds, of fixed cost plus
-// scale groups times tiles per CU in the fullest CU.  The constants are fits to sweeps over the 1.7B- and
-// 4B-shaped matrices at 17-3000 tokens (12288 x 2048 at 512 tokens: 34.1 / 34.5 us; 2048 x 6144 at
-// 1024: 56.8 / 34.2; 2560 x 9728 at 512: 83.9 / 37.4; 19456 x 2560 at 1024: 93.7 / 127.0); within 15 % of them everywhere.  A 128 x 128 tile alone on its CU is 1.17 times as long as half of
-// two that share one.
-inline int wide_pick(int M, int N, int K, int n_cus) {
-    const double G = K / kGroup;
-    const auto fullest = [&](int tokens, int rows) {
-        const long tiles = (long)((M + tokens - 1) / tokens) * ((N + rows - 1) / rows);
-        return (double)((tiles + n_cus - 1) / n_cus);
+// What a launch takes, in microseconds: a fixed part, the scale groups of a K slice times the length of one
+// -- bound by latency up to some tiles per CU, then by what they issue -- and a part per tile for its scales
+// and its results.  Fitted to 17 ... 4096 tokens of 13 matrices (1024 x 1024 ... 20000 x 9728): 4-9 % rms.
+inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
+    struct Cost {
+        int tokens, rows, slices;
+        double fixed, group_min, group_tile, tile;
     };
-    const double c0 = fullest(128, 128);
-    const double t[kWideVariants] = {8.0 + 0.80 * G * (c0 < 1.17 ? 1.17 : c0),
-                                     4.5 + 0.16 * G * fullest(32, 64)};
+    static constexpr Cost c[kWideVariants] = {{64, 256, 1, 3.5, 0.725, 0.61, 1.7},  {64, 128, 2, 3.15, 0.79, 0.625, 1.6},
+                                              {32, 64, 4, 3.5, 0.605, 0.475, 0.57}, {32, 64, 8, 1.9, 0.83, 0.86, 2.5},
+                                              {64, 128, 4, 1.5, 1.25, 1.25, 3.0},   {128, 256, 1, 0.0, 0.955, 1.09, 7.4}};
+    const Cost &k = c[v];
+    const int G = K / kGroup, unit = G % 4 == 0 ? 4 : 1;
+    const int groups = (G / unit + k.slices - 1) / k.slices * unit;
+    const long tiles = (long)((M + k.tokens - 1) / k.tokens) * ((N + k.rows - 1) / k.rows);
+    const double per_cu = (double)((tiles + n_cus - 1) / n_cus);
+    const double busy = k.group_tile * per_cu;
+    return k.fixed + groups * (busy > k.group_min ? busy : k.group_min) + k.tile * per_cu;
+}
+
+// The variant with the smallest estimate: 0.8 % behind the best of them in the mean over the same sweep.
+inline int wide_pick(int M, int N, int K, int n_cus) {
     int best = 0;
     for (int v = 1; v < kWideVariants; ++v)
-        if (t[v] < t[best]) best = v;
+        if (wide_estimate(v, M, N, K, n_cus) < wide_estimate(best, M, N, K, n_cus)) best = v;
     return best;
 }
 

@@ -1,4 +1,4 @@
-"""Blocks of more than 16 tokens (gemv_wide_kernel, both tiles) and rows that are no whole number of 512-wide K tiles
+"""Blocks of more than 16 tokens (gemv_wide_kernel, every tile) and rows that are no whole number of 512-wide K tiles
 (gemv_mxl_ragged_kernel) against a float64 product of the unpacked operands: int32 group sums exactly, the scaled value to fp32
 summation order, bf16 to its own rounding.  Sizes sit on the edges of tiles, slices and scale groups."""
 import pytest
@@ -38,7 +38,7 @@ def _check(m, n, k, bits, scale_dtype, family):
 
 @pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bits", [2, 1])
-@pytest.mark.parametrize("variant", [1, 2])
+@pytest.mark.parametrize("variant", [1, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 128), (17, 16, 256), (32, 64, 384), (33, 65, 512), (128, 128, 2048),
                                    (129, 131, 640), (257, 1000, 1152), (40, 136, 9728)])
 def test_wide_kernel(m, n, k, variant, bits, scale_dtype):
@@ -53,7 +53,7 @@ def test_wide_kernel(m, n, k, variant, bits, scale_dtype):
 
 
 @pytest.mark.parametrize("bits", [2, 1])
-@pytest.mark.parametrize("m,n,k,family", [(49, 12288, 2048, "gemv_wide_kernel<"), (32, 12288, 2048, "gemv_mxl_kernel<"),
+@pytest.mark.parametrize("m,n,k,family", [(49, 12288, 2048, "gemv_wide_kernel<"), (32, 2048, 2048, "gemv_mxl_kernel<"),
                                           (600, 700, 1664, "gemv_wide_kernel<"), (9, 20000, 896, "gemv_mxl_ragged_kernel<"),
                                           (5, 33000, 384, "gemv_wide_kernel<")])
 def test_built_in_choice(m, n, k, family, bits):
