@@ -145,6 +145,69 @@ qk_norm_rope_kernel(const uint16_t *pxqkv, const uint16_t *pqw, const uint16_t *
     dst[lane + 64] = (uint16_t)o1;
 }
 
+// The same for the rows of a prompt, where bytes count and not the length of one row's chain: sixteen lanes a
+// (token, head) row, lane j with dims 4 j .. + 3 and their partners 64 further, 8-byte loads and stores, rows in memory
+// order.  (One wave a row with 2-byte accesses: 29.8 us for 3001 rows of 48 heads, 2.5 TB/s.)
+__global__ void __launch_bounds__(256)
+prefill_rope_kernel(const uint16_t *xqkv, const uint16_t *qw, const uint16_t *kw, const uint16_t *cos_t,
+                    const uint16_t *sin_t, const int32_t *positions, uint16_t *q_out, uint16_t *k_layer,
+                    uint16_t *v_layer, float eps, int M, int n_heads, int n_kv, int slots, int write_slot, int max_pos) {
+    const int total_heads = n_heads + 2 * n_kv;
+    const long row = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+    const int m = (int)(row / total_heads), head = (int)(row - (long)m * total_heads);
+    if (m >= M) return;  // whole rows of sixteen lanes
+    const int d = 4 * (threadIdx.x & 15);
+    const uint16_t *x = xqkv + (size_t)row * kHd;
+    const uint2 lo = *reinterpret_cast<const uint2 *>(x + d), hi = *reinterpret_cast<const uint2 *>(x + d + 64);
+    uint16_t *dst;
+    if (head >= n_heads + n_kv) {
+        dst = v_layer + ((size_t)(head - n_heads - n_kv) * slots + write_slot + m) * kHd;
+        *reinterpret_cast<uint2 *>(dst + d) = lo;
+        *reinterpret_cast<uint2 *>(dst + d + 64) = hi;
+        return;
+    }
+    const bool is_q = head < n_heads;
+    int pos = positions[m];
+    pos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
+    const uint16_t *w = is_q ? qw : kw, *cr = cos_t + (size_t)pos * kHd, *sr = sin_t + (size_t)pos * kHd;
+    const auto four = [](const uint16_t *p, float *f) {
+        const uint2 v = *reinterpret_cast<const uint2 *>(p);
+        f[0] = bf16_bits_to_f32(v.x & 0xffffu);
+        f[1] = __uint_as_float(v.x & 0xffff0000u);
+        f[2] = bf16_bits_to_f32(v.y & 0xffffu);
+        f[3] = __uint_as_float(v.y & 0xffff0000u);
+    };
+    float w0[4], w1[4], c0[4], c1[4], s0[4], s1[4], f0[4], f1[4];
+    four(w + d, w0);
+    four(w + d + 64, w1);
+    four(cr + d, c0);
+    four(cr + d + 64, c1);
+    four(sr + d, s0);
+    four(sr + d + 64, s1);
+    four(x + d, f0);
+    four(x + d + 64, f1);
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss += (double)(f0[i] * f0[i]) + (double)(f1[i] * f1[i]);
+    ss += bonsai_wave::partner<bonsai_wave::kXor1>(ss);
+    ss += bonsai_wave::partner<bonsai_wave::kXor2>(ss);
+    ss += bonsai_wave::partner<bonsai_wave::kHalfMirror>(ss);
+    ss += bonsai_wave::partner<bonsai_wave::kMirror>(ss);
+    const float var = (float)ss / (float)kHd;
+    const float rs = 1.0f / sqrtf(var + eps);
+    uint32_t o0[4], o1[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // the rounding points of rope_row_math
+        const float n0 = bf16_round(w0[i] * bf16_round(f0[i] * rs)), n1 = bf16_round(w1[i] * bf16_round(f1[i] * rs));
+        o0[i] = f32_to_bf16_bits(bf16_round(n0 * c0[i]) + bf16_round(-n1 * s0[i]));
+        o1[i] = f32_to_bf16_bits(bf16_round(n1 * c1[i]) + bf16_round(n0 * s1[i]));
+    }
+    dst = is_q ? q_out + ((size_t)m * n_heads + head) * kHd
+               : k_layer + ((size_t)(head - n_heads) * slots + write_slot + m) * kHd;
+    *reinterpret_cast<uint2 *>(dst + d) = make_uint2(o0[0] | (o0[1] << 16), o0[2] | (o0[3] << 16));
+    *reinterpret_cast<uint2 *>(dst + d + 64) = make_uint2(o1[0] | (o1[1] << 16), o1[2] | (o1[3] << 16));
+}
+
 // ---------------------------------------------------------------------------
 // Attention, split over KV chunks.  One wave per (kv head, query head of the group,
 // chunk, row group of RW rows).  Logical sequence index t in [0, cache_len + M):
@@ -1546,6 +1609,20 @@ static int launch_rope(const void *xqkv, const void *q_norm_w,
     a.write_slot = write_slot;
     a.max_pos = max_pos;
     const int total_heads = n_heads + 2 * n_kv;
+    if (max_width > BONSAI_MAX_WIDTH) {  // a prompt
+        const uintptr_t all = reinterpret_cast<uintptr_t>(xqkv) | reinterpret_cast<uintptr_t>(q_norm_w) |
+                              reinterpret_cast<uintptr_t>(k_norm_w) | reinterpret_cast<uintptr_t>(cos_table) |
+                              reinterpret_cast<uintptr_t>(sin_table) | reinterpret_cast<uintptr_t>(q_out) |
+                              reinterpret_cast<uintptr_t>(k_layer) | reinterpret_cast<uintptr_t>(v_layer);
+        if ((all & 7) == 0) {
+            const long rows = (long)M * total_heads;
+            hipLaunchKernelGGL(prefill_rope_kernel, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0,
+                               static_cast<hipStream_t>(stream), a.xqkv, a.qw, a.kw, a.cos_t, a.sin_t, a.positions,
+                               a.q_out, a.k_layer, a.v_layer, a.eps, a.M, a.n_heads, a.n_kv, a.slots, a.write_slot,
+                               a.max_pos);
+            return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+        }
+    }
     hipLaunchKernelGGL(qk_norm_rope_kernel, dim3((total_heads + 3) / 4, M), dim3(256), 0,
                        static_cast<hipStream_t>(stream), a.xqkv, a.qw, a.kw, a.cos_t, a.sin_t,
                        a.positions, a.q_out, a.k_layer, a.v_layer, a.eps, a.M, a.n_heads, a.n_kv,
@@ -1571,6 +1648,20 @@ extern "C" int bonsai_prefill_rope_kv_write(const void *xqkv, const void *q_norm
                        n_heads, n_kv, slots, write_slot, max_pos, BONSAI_PREFILL_MAX_ROWS, stream);
 }
 
+// CUs of the current device, asked for once per device
+static int cu_count() {
+    constexpr int kDevices = 64;
+    static std::atomic<int> known[kDevices];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return 256;
+    int n = known[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+        known[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
 extern "C" int bonsai_prefill_attention(const void *q, const void *k_layer, const void *v_layer, void *out_bf16,
                                         float scale, int M, int n_heads, int n_kv, int slots, int base,
                                         void *stream) {
@@ -1580,9 +1671,12 @@ extern "C" int bonsai_prefill_attention(const void *q, const void *k_layer, cons
         n_heads / n_kv > P::kPairs || base < 0 || slots > (1 << 22) || base + M > slots)
         return BONSAI_DECODE_ERR_ARG;
     const int hpg = n_heads / n_kv;
-    const int tokens = P::kPairs / hpg;
+    // two rounds of the 32-pair form at most: above, its four-fold staging costs more than idle CUs (16 query heads,
+    // 512 rows 19.2 -> 11.8 us, 1024 33.2 -> 23.8, 2048 61.9 / 64.2; 32 heads, 512 rows 19.8 -> 17.6, 777 27.3 / 33.0)
+    const bool split = hpg <= 32 && (long)((M + 32 / hpg - 1) / (32 / hpg)) * n_kv <= 2L * cu_count();
+    const int tokens = (split ? 32 : P::kPairs) / hpg;
     const int tiles = (M + tokens - 1) / tokens;
-    hipLaunchKernelGGL(P::prefill_attn_kernel, dim3(tiles * n_kv), dim3(P::kWaves * 64), 0,
+    hipLaunchKernelGGL((split ? P::prefill_attn_split_kernel : P::prefill_attn_kernel), dim3(tiles * n_kv), dim3(P::kWaves * 64), 0,
                        static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(q),
                        static_cast<const uint16_t *>(k_layer), static_cast<const uint16_t *>(v_layer),
                        static_cast<uint16_t *>(out_bf16), scale * 1.44269504088896340736f, M, n_heads, n_kv, hpg,

@@ -218,5 +218,178 @@ prefill_attn_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *
         }
 }
 
+// Few rows: the kernel above has 128 pairs a workgroup, which leaves most CUs idle (256 rows of two query heads a
+// kv head: 32 workgroups) and one workgroup walks all chunks.  Here the four waves of a workgroup share 32 pairs
+// and take every fourth chunk each, staged by the wave for itself (program order instead of barriers); the four
+// results meet in LDS.  Same operations; the softmax's running maxima are those of a wave's own chunks.
+constexpr int kSplitStage = kKBytes + kVBytes;
+constexpr int kSplitLds = kWaves * kSplitStage;
+static_assert(kWaves * 64 * 64 * 4 + kWaves * 64 * 8 <= kSplitLds, "the merge reuses the staging areas");
+
+__global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1)))
+prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *v_layer, uint16_t *out,
+                          float scale_log2e, int M, int n_heads, int n_kv, int hpg, int slots, int base, int tokens,
+                          int tiles) {
+    __shared__ __align__(16) unsigned char smem[kSplitLds];
+    const int kvh = (int)blockIdx.x % n_kv;
+    const int m0 = (tiles - 1 - (int)blockIdx.x / n_kv) * tokens;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int col = lane & 31, h = lane >> 5;
+    const int tok = col / hpg, g = col - tok * hpg;
+    const bool valid = tok < tokens && m0 + tok < M;
+    const int m = valid ? m0 + tok : M - 1;
+    const int pos = base + m;
+    const size_t row = (size_t)m * n_heads * kHead + (size_t)(kvh * hpg + g) * kHead;
+    u32v4 qr[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) qr[j] = *reinterpret_cast<const u32v4 *>(q + row + 16 * j + 8 * h);
+    const int rows = M - m0 < tokens ? M - m0 : tokens;
+    const int seen = base + m0 + rows;
+    const int chunks = (seen + kSlots - 1) / kSlots;
+    const int masked_from = (base + m0 + 1) / kSlots;
+    const size_t head = (size_t)kvh * slots * kHead;
+    const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(k_layer + head), 0, seen * 2 * kHead, kRawBuffer);
+    const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(v_layer + head), 0, seen * 2 * kHead, kRawBuffer);
+    unsigned char *kb = smem + wave * kSplitStage, *vb = kb + kKBytes;
+    const int k_slot = lane >> 4, k_col = lane & 15;            // slots k_slot + 4 i
+    const int v_slot = (lane & 15) * 4, v_dim = (lane >> 4) * 8;  // dims v_dim + 32 i
+    u32v4 kr[16], vr[4][4];
+    const auto load = [&](int c) {
+        const int s = c * kSlots * 2 * kHead;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            kr[i] = __builtin_amdgcn_raw_buffer_load_b128(rK, (k_slot + 4 * i) * 2 * kHead + k_col * 16, s, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                vr[i][t] = __builtin_amdgcn_raw_buffer_load_b128(rV, (v_slot + t) * 2 * kHead + (v_dim + 32 * i) * 2, s, 0);
+    };
+
+    f32x16 o[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+    if (wave < chunks) load(wave);
+    for (int c = wave; c < chunks; c += kWaves) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) *reinterpret_cast<u32v4 *>(kb + (k_slot + 4 * i) * kKPitch + k_col * 16) = kr[i];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int d = 0; d < 8; ++d) {
+                const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
+                uint2 v;
+                v.x = __builtin_amdgcn_perm(vr[i][1][d / 2], vr[i][0][d / 2], sel);
+                v.y = __builtin_amdgcn_perm(vr[i][3][d / 2], vr[i][2][d / 2], sel);
+                *reinterpret_cast<uint2 *>(vb + (v_dim + 32 * i + d) * kVPitch + v_slot * 2) = v;
+            }
+        if (c + kWaves < chunks) load(c + kWaves);
+        f32x16 s[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+            const unsigned char *kp = kb + (32 * t + col) * kKPitch + 16 * h;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(*reinterpret_cast<const u32v4 *>(kp + 32 * j)),
+                                                               frag(qr[j]), s[t], 0, 0, 0);
+        }
+        if (c >= masked_from) {
+            const int rel = pos - c * kSlots - 4 * h;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (32 * t + 8 * (r / 4) + r % 4 > rel) s[t][r] = -INFINITY;
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m_run, mx * scale_log2e);
+        // (a row may see nothing of a chunk that is not its wave's first: its maximum is then still -inf)
+        const float shift = m_new == -INFINITY ? 0.0f : m_new;
+        if (__any(m_new > m_run)) {
+            const float alpha = __builtin_amdgcn_exp2f(m_run - shift);
+            l_run *= alpha;
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+            m_run = m_new;
+        }
+        uint32_t p[2][8];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const float a = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r], scale_log2e, -shift));
+                const float b = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r + 1], scale_log2e, -shift));
+                p[t][r] = pack_bf16(a, b);
+                bf16x2 pv;
+                __builtin_memcpy(&pv, &p[t][r], 4);
+                const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
+                l_run = __builtin_amdgcn_fdot2_f32_bf16(pv, ones, l_run, false);
+            }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const uint32_t *pp = p[ks / 2] + 4 * (ks & 1);
+            const bf16x8 pf = frag(u32v4{pp[0], pp[1], pp[2], pp[3]});
+            const unsigned char *vp = vb + col * kVPitch + (16 * ks + 4 * h) * 2;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const uint2 lo = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch);
+                const uint2 hi = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch + 16);
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(u32v4{lo.x, lo.y, hi.x, hi.y}), pf, o[d], 0, 0, 0);
+            }
+        }
+    }
+
+    // ---- the waves' results: [wave][register][lane], maxima and sums behind them
+    __syncthreads();
+    float *meet = reinterpret_cast<float *>(smem);
+    float *stat = meet + kWaves * 64 * 64;  // [wave][maximum, sum][lane]
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) meet[(wave * 64 + d * 16 + r) * 64 + lane] = o[d][r];
+    stat[wave * 128 + lane] = m_run;
+    stat[wave * 128 + 64 + lane] = l_run;
+    __syncthreads();
+    float top = -INFINITY, l = 0.0f, e[kWaves];
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) top = fmaxf(top, stat[w * 128 + lane]);  // finite: every row sees slot 0
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        e[w] = __builtin_amdgcn_exp2f(stat[w * 128 + lane] - top);
+        l = fmaf(e[w], stat[w * 128 + 64 + lane], l);
+    }
+    l += __shfl_xor(l, 32);
+    if (!valid) return;
+    const float inv = 1.0f / l;
+    // wave d finishes dims 32 d + 8 (r / 4) + 4 h + r % 4
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) sum = fmaf(e[w], meet[(w * 64 + wave * 16 + 4 * k + i) * 64 + lane], sum);
+            v[i] = sum * inv;
+        }
+        *reinterpret_cast<uint2 *>(out + row + 32 * wave + 8 * k + 4 * h) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+    }
+}
+
 }  // namespace bonsai_prefill
 #endif  // BONSAI_PREFILL_ATTN_HIP_H

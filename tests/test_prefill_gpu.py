@@ -1,5 +1,7 @@
 """The prompt path: causal attention of wide blocks against float64, and whole prompts against the same decoder
 stepped through its captured graphs."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -10,7 +12,8 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize("m,n_heads,n_kv,base,slots", [
     (1, 16, 8, 0, 40), (64, 16, 8, 0, 96), (65, 16, 8, 63, 160), (127, 4, 4, 1, 128), (130, 32, 8, 190, 400),
-    (300, 6, 2, 77, 500), (33, 3, 1, 1000, 1100), (515, 16, 8, 0, 515)])
+    (300, 6, 2, 77, 500), (33, 3, 1, 1000, 1100), (515, 16, 8, 0, 515), (1024, 16, 8, 0, 1024), (1030, 16, 8, 3, 1040),
+    (700, 32, 8, 64, 800)])
 def test_prefill_attention_against_float64(m, n_heads, n_kv, base, slots):
     from bitmtp_amd import decode_ops
     print(f"[case] prefill attention m={m} heads={n_heads}/{n_kv} base={base}", flush=True)
@@ -33,6 +36,30 @@ def test_prefill_attention_against_float64(m, n_heads, n_kv, base, slots):
     got = out.view(m, n_heads, 128).double()
     assert torch.isfinite(got).all()
     assert ((got - want).abs() <= 2e-3 + 2e-2 * want.abs()).all()
+
+
+@pytest.mark.parametrize("m,n_heads,n_kv", [(1, 4, 2), (33, 3, 1), (67, 16, 8)])
+def test_prompt_rows_rope_is_the_steps_own(m, n_heads, n_kv):
+    """q / k norm + RoPE + KV write of prompt rows: the bits of the step's entry point, 32 rows at a time."""
+    from bitmtp_amd import decode_ops
+    print(f"[case] prompt rope m={m} heads={n_heads}/{n_kv}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(m)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)
+    x, qw, kw, cos, sin = rnd(m, (n_heads + 2 * n_kv) * 128), rnd(128), rnd(128), rnd(90, 128), rnd(90, 128)
+    pos = torch.randint(-2, 95, (m,), generator=gen, device=DEV, dtype=torch.int32)
+    got, want = (torch.zeros(2, n_kv, m + 8, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    q_got, q_want = (torch.zeros(m, n_heads, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    lib, p = decode_ops.decode_lib(), lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rc = lib.bonsai_prefill_rope_kv_write(p(x), p(qw), p(kw), 1e-6, p(cos), p(sin), p(pos), p(q_got), p(got[0]), p(got[1]),
+                                          m, n_heads, n_kv, m + 8, 5, 90, stream)
+    assert rc == 0
+    for r in range(0, m, 32):
+        rows = min(32, m - r)
+        decode_ops.qk_norm_rope_kv_write(x[r:r + rows], qw, kw, 1e-6, cos, sin, pos[r:r + rows], q_want[r:r + rows], want[0],
+                                         want[1], n_heads, n_kv, 5 + r)
+    assert torch.equal(q_got.view(torch.int16), q_want.view(torch.int16))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
 def test_prefill_attention_argument_checks():
