@@ -39,11 +39,18 @@ constexpr int kPartStride = kHd + 4;  // 128 accumulators + running max + runnin
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
+// round to nearest even through the hardware conversion (v_cvt_pk_bf16_f32 on gfx950), one or two at a time
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x0040u;
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return u >> 16;
+    const __bf16 b = static_cast<__bf16>(f);
+    uint16_t u;
+    __builtin_memcpy(&u, &b, 2);
+    return u;
+}
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    const bf16x2_t p = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+    uint32_t u;
+    __builtin_memcpy(&u, &p, 4);
+    return u;
 }
 __device__ __forceinline__ float bf16_round(float f) { return bf16_bits_to_f32(f32_to_bf16_bits(f)); }
 
@@ -147,7 +154,8 @@ qk_norm_rope_kernel(const uint16_t *pxqkv, const uint16_t *pqw, const uint16_t *
 
 // The same for the rows of a prompt, where bytes count and not the length of one row's chain: sixteen lanes a
 // (token, head) row, lane j with dims 4 j .. + 3 and their partners 64 further, 8-byte loads and stores, rows in memory
-// order.  (One wave a row with 2-byte accesses: 29.8 us for 3001 rows of 48 heads, 2.5 TB/s.)
+// order, roundings two at a time (what bounds it otherwise).  (One wave a row with 2-byte accesses: 29.8 us for 3001
+// rows of 48 heads, 2.5 TB/s.)
 __global__ void __launch_bounds__(256)
 prefill_rope_kernel(const uint16_t *xqkv, const uint16_t *qw, const uint16_t *kw, const uint16_t *cos_t,
                     const uint16_t *sin_t, const int32_t *positions, uint16_t *q_out, uint16_t *k_layer,
@@ -195,17 +203,22 @@ prefill_rope_kernel(const uint16_t *xqkv, const uint16_t *qw, const uint16_t *kw
     ss += bonsai_wave::partner<bonsai_wave::kMirror>(ss);
     const float var = (float)ss / (float)kHd;
     const float rs = 1.0f / sqrtf(var + eps);
-    uint32_t o0[4], o1[4];
+    const auto lo_of = [](uint32_t v) { return __uint_as_float(v << 16); };
+    const auto hi_of = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
+    uint32_t o0[2], o1[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {  // the rounding points of rope_row_math
-        const float n0 = bf16_round(w0[i] * bf16_round(f0[i] * rs)), n1 = bf16_round(w1[i] * bf16_round(f1[i] * rs));
-        o0[i] = f32_to_bf16_bits(bf16_round(n0 * c0[i]) + bf16_round(-n1 * s0[i]));
-        o1[i] = f32_to_bf16_bits(bf16_round(n1 * c1[i]) + bf16_round(n0 * s1[i]));
+    for (int i = 0; i < 4; i += 2) {  // the rounding points of rope_row_math, two elements at a time
+        const uint32_t t0 = pack_bf16(f0[i] * rs, f0[i + 1] * rs), t1 = pack_bf16(f1[i] * rs, f1[i + 1] * rs);
+        const uint32_t n0 = pack_bf16(w0[i] * lo_of(t0), w0[i + 1] * hi_of(t0)), n1 = pack_bf16(w1[i] * lo_of(t1), w1[i + 1] * hi_of(t1));
+        const uint32_t a0 = pack_bf16(lo_of(n0) * c0[i], hi_of(n0) * c0[i + 1]), b0 = pack_bf16(-lo_of(n1) * s0[i], -hi_of(n1) * s0[i + 1]);
+        const uint32_t a1 = pack_bf16(lo_of(n1) * c1[i], hi_of(n1) * c1[i + 1]), b1 = pack_bf16(lo_of(n0) * s1[i], hi_of(n0) * s1[i + 1]);
+        o0[i / 2] = pack_bf16(lo_of(a0) + lo_of(b0), hi_of(a0) + hi_of(b0));
+        o1[i / 2] = pack_bf16(lo_of(a1) + lo_of(b1), hi_of(a1) + hi_of(b1));
     }
     dst = is_q ? q_out + ((size_t)m * n_heads + head) * kHd
                : k_layer + ((size_t)(head - n_heads) * slots + write_slot + m) * kHd;
-    *reinterpret_cast<uint2 *>(dst + d) = make_uint2(o0[0] | (o0[1] << 16), o0[2] | (o0[3] << 16));
-    *reinterpret_cast<uint2 *>(dst + d + 64) = make_uint2(o1[0] | (o1[1] << 16), o1[2] | (o1[3] << 16));
+    *reinterpret_cast<uint2 *>(dst + d) = make_uint2(o0[0], o0[1]);
+    *reinterpret_cast<uint2 *>(dst + d + 64) = make_uint2(o1[0], o1[1]);
 }
 
 // ---------------------------------------------------------------------------

@@ -456,15 +456,16 @@ int wide_init_device(int max_lds) {
 
 // What a launch takes, in microseconds: a fixed part, the scale groups of a K slice times the length of one
 // -- bound by latency up to some tiles per CU, then by what they issue -- and a part per tile for its scales
-// and its results.  Fitted to 17 ... 4096 tokens of 13 matrices (1024 x 1024 ... 20000 x 9728): 4-9 % rms.
+// and its results.  Fitted to 17 ... 4096 tokens of 13 matrices (1024 x 1024 ... 20000 x 9728): 4-9 % rms,
+// then moved within that for the choice between them.
 inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
     struct Cost {
         int tokens, rows, slices;
         double fixed, group_min, group_tile, tile;
     };
-    static constexpr Cost c[kWideVariants] = {{64, 256, 1, 3.5, 0.725, 0.61, 1.7},  {64, 128, 2, 3.15, 0.79, 0.625, 1.6},
-                                              {32, 64, 4, 3.5, 0.605, 0.475, 0.57}, {32, 64, 8, 1.9, 0.83, 0.86, 2.5},
-                                              {64, 128, 4, 1.5, 1.25, 1.25, 3.0},   {128, 256, 1, 0.0, 0.955, 1.09, 7.4}};
+    static constexpr Cost c[kWideVariants] = {{64, 256, 1, 3.7, 0.752, 0.571, 1.47},   {64, 128, 2, 2.94, 0.882, 0.577, 1.565},
+                                              {32, 64, 4, 3.27, 0.595, 0.498, 0.554},  {32, 64, 8, 1.87, 0.791, 0.889, 2.54},
+                                              {64, 128, 4, 1.5, 1.25, 1.25, 3.0},      {128, 256, 1, 2.56, 0.898, 1.032, 7.46}};
     const Cost &k = c[v];
     const int G = K / kGroup, unit = G % 4 == 0 ? 4 : 1;
     const int groups = (G / unit + k.slices - 1) / k.slices * unit;
@@ -474,7 +475,7 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
     return k.fixed + groups * (busy > k.group_min ? busy : k.group_min) + k.tile * per_cu;
 }
 
-// The variant with the smallest estimate: 0.8 % behind the best of them in the mean over the same sweep.
+// The variant with the smallest estimate: at most 2.4 % behind the best of them over the same sweep.
 inline int wide_pick(int M, int N, int K, int n_cus) {
     int best = 0;
     for (int v = 1; v < kWideVariants; ++v)
