@@ -529,6 +529,38 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
     id /= n_kv;
     const int part = id % parts;
     const int pt = id / parts;
+    const int pairs_total = M * G;
+
+    // ROPE (`q` is the merged projection [M][n_heads + 2 n_kv][128]): a job is one row: q row `job` of the tile, then
+    // K row (with its V row) job - n_q of the block.  A wave takes kRowsInFlight jobs at a time and issues all their
+    // loads first; those of the first jobs need nothing of the descriptor and go out before it is waited for, so that
+    // they come back, in order, before the K / V chunk whose addresses it gives.
+    constexpr int kRowsInFlight = ROPE ? 4 : 1;
+    const int wu = __builtin_amdgcn_readfirstlane(w);
+    const int n_q = min(kPairTile, pairs_total - pt * kPairTile);
+    RopeRowIn in[kRowsInFlight] = {};
+    uint16_t v0[kRowsInFlight] = {}, v1[kRowsInFlight] = {};
+    int jm[kRowsInFlight] = {};
+    const auto load_rows = [&](int base, int jobs) {
+        const int total_heads = n_heads + 2 * n_kv;
+#pragma unroll
+        for (int j = 0; j < kRowsInFlight; ++j) {
+            const int job = base + wu + j * kAttnWaves;
+            if (job >= jobs) break;  // uniform
+            const bool is_q = job < n_q;
+            const int qp = pt * kPairTile + job;
+            jm[j] = is_q ? qp / G : job - n_q;
+            const int src_head = is_q ? kvh * G + (qp - jm[j] * G) : n_heads + kvh;
+            in[j] = rope_row_load(q + ((size_t)jm[j] * total_heads + src_head) * kHd, is_q ? rope.qw : rope.kw,
+                                  rope.cos_t, rope.sin_t, rope.positions[jm[j]], rope.max_pos, lane);
+            if (!is_q) {
+                const uint16_t *xv = q + ((size_t)jm[j] * total_heads + n_heads + n_kv + kvh) * kHd;
+                v0[j] = xv[lane];
+                v1[j] = xv[lane + 64];
+            }
+        }
+    };
+    if constexpr (ROPE) load_rows(0, n_q + M);
 
     // a descriptor that does not fit the segment is clamped, never followed out of bounds
     const int cache_len = min(max(meta[0], 0), sigma);
@@ -539,7 +571,6 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
     const int c_begin = part * cpw;
     if (c_begin >= live_chunks) return;  // whole workgroup; the combine step counts the same parts
     const int c_end = min(c_begin + cpw, live_chunks);
-    const int pairs_total = M * G;
 
     // the four pairs whose results this lane holds (D layout: tile rows 4 kb + r)
     bool valid[4];
@@ -625,34 +656,11 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
 
     // the first chunk's loads travel while the q rows are fetched or derived
     ChunkRegs cur = load_chunk(c_begin);
-    // ROPE: `q` is the merged projection [M][n_heads + 2 n_kv][128]
     if constexpr (ROPE) {
         const bool own_rows = c_end * kChunk > cache_len;  // this workgroup reaches the block's rows
-        const int total_heads = n_heads + 2 * n_kv;
-        const int n_q = min(kPairTile, pairs_total - pt * kPairTile);
         const int n_jobs = n_q + (own_rows ? M : 0);
-        // a job is one row: q row `job` of the tile, then K row (with its V row) job - n_q of the
-        // block.  A wave takes kRowsInFlight jobs at a time and issues all their loads first.
-        constexpr int kRowsInFlight = 4;
-        const int wu = __builtin_amdgcn_readfirstlane(w);
         for (int base = 0; base < n_jobs; base += kRowsInFlight * kAttnWaves) {
-            RopeRowIn in[kRowsInFlight];
-            uint16_t v0[kRowsInFlight], v1[kRowsInFlight];
-            int jm[kRowsInFlight];
-#pragma unroll
-            for (int j = 0; j < kRowsInFlight; ++j) {
-                const int job = min(base + wu + j * kAttnWaves, n_jobs - 1);  // past the end: a repeat, unused
-                const bool is_q = job < n_q;
-                const int qp = pt * kPairTile + job;
-                jm[j] = is_q ? qp / G : job - n_q;
-                const int src_head = is_q ? kvh * G + (qp - jm[j] * G) : n_heads + kvh;
-                in[j] = rope_row_load(q + ((size_t)jm[j] * total_heads + src_head) * kHd,
-                                      is_q ? rope.qw : rope.kw, rope.cos_t, rope.sin_t,
-                                      rope.positions[jm[j]], rope.max_pos, lane);
-                const uint16_t *xv = q + ((size_t)jm[j] * total_heads + n_heads + n_kv + kvh) * kHd;
-                v0[j] = xv[lane];
-                v1[j] = xv[lane + 64];
-            }
+            if (base > 0) load_rows(base, n_jobs);
 #pragma unroll
             for (int j = 0; j < kRowsInFlight; ++j) {
                 const int job = base + wu + j * kAttnWaves;
@@ -685,7 +693,6 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
     // A operand of S: this lane's pair (tile row `col`), dims 32 j + 8 kb .. + 8
     uint4 qreg[4];
     if constexpr (ROPE) {
-        const int n_q = min(kPairTile, pairs_total - pt * kPairTile);
         const uint4 *qrow = reinterpret_cast<const uint4 *>(q_new[min(col, n_q - 1)]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) qreg[j] = qrow[4 * j + kb];
