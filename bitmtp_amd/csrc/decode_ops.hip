@@ -476,6 +476,12 @@ __device__ __forceinline__ void combine_head_slice(const float *part, int part_b
 #undef BONSAI_COMBINE_PART
 }
 
+// x / y for the small numbers of an attention launch, y as small_recip(y): exact while x y < 32768 (pairs of a tile row
+// by heads per kv head: below 1024 x 32; chunks by parts: below 160 x 16).  A division by a number the compiler does not
+// know is some twenty dependent instructions, 60 ns of a launch of 3 us.
+__host__ __device__ inline unsigned small_recip(unsigned y) { return (32768u + y - 1) / y; }
+__device__ __forceinline__ int small_div(int x, unsigned recip) { return (int)(((unsigned)x * recip) >> 15); }
+
 // live parts of a step: the live chunks split into runs of ceil(live / parts)
 __host__ __device__ inline int attn_chunks_per_part(int live_chunks, int parts) {
     return (live_chunks + parts - 1) / parts;
@@ -495,6 +501,16 @@ struct RopeIn {
     int max_pos;
 };
 
+// The sizes of a launch in two words, so that they and the pointers the first loads need fit the sixteen words of
+// arguments that a wave finds in its registers when it starts; the others cost it a memory round trip.
+struct AttnDims {
+    uint32_t sizes, recips;
+    AttnDims(int M, int G, int n_kv, int parts)
+        : sizes((uint32_t)M | (uint32_t)G << 8 | (uint32_t)n_kv << 16 | (uint32_t)parts << 24),
+          recips(small_recip(G) | small_recip(parts) << 16) {}
+};
+static_assert(BONSAI_MAX_WIDTH < 256 && kMaxParts < 256, "AttnDims: eight bits each");
+
 // FIN: no second launch.  A workgroup makes its partials visible to the device and counts itself
 // in on its kv head's arrival counter; the one that finds all the others there merges the
 // partials of its pair tile (combine_head_slice, what attn_combine_parts_kernel does), stores the
@@ -510,9 +526,13 @@ struct FinOut {
 
 template <bool ROPE, bool FIN>
 __global__ void __launch_bounds__(kAttnWaves * 64)
-attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
-                 const int32_t *meta, float *part_out, float scale_log2e, int M, int n_heads,
-                 int n_kv, int G, int slots, int sigma, int parts, const RopeIn rope, const FinOut fin) {
+attn_mfma_kernel(const uint16_t *q, const int32_t *meta, const int32_t *positions, const uint16_t *cos_t,
+                 const uint16_t *sin_t, const uint16_t *qw, uint32_t sizes, uint32_t recips, int sigma, int max_pos,
+                 const uint16_t *kw, uint16_t *k_layer, uint16_t *v_layer, float *part_out, float scale_log2e,
+                 float eps, int slots, const FinOut fin) {
+    const int M = sizes & 255, G = (sizes >> 8) & 255, n_kv = (sizes >> 16) & 255, parts = sizes >> 24;
+    const int n_heads = G * n_kv;
+    const unsigned g_recip = recips & 0xffffu, parts_recip = recips >> 16;
     __shared__ unsigned fin_last;
     __shared__ float fin_max[kPairTile];
     __shared__ __attribute__((aligned(16))) unsigned char v_lds[kChunk * kVPitch];
@@ -524,11 +544,7 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
     __shared__ __attribute__((aligned(16))) float st_sum[kAttnWaves][kPairTile];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int col = lane & 15, kb = lane >> 4;
-    int id = blockIdx.x;
-    const int kvh = id % n_kv;
-    id /= n_kv;
-    const int part = id % parts;
-    const int pt = id / parts;
+    const int kvh = blockIdx.x, part = blockIdx.y, pt = blockIdx.z;
     const int pairs_total = M * G;
 
     // ROPE (`q` is the merged projection [M][n_heads + 2 n_kv][128]): a job is one row: q row `job` of the tile, then
@@ -549,10 +565,10 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
             if (job >= jobs) break;  // uniform
             const bool is_q = job < n_q;
             const int qp = pt * kPairTile + job;
-            jm[j] = is_q ? qp / G : job - n_q;
+            jm[j] = is_q ? small_div(qp, g_recip) : job - n_q;
             const int src_head = is_q ? kvh * G + (qp - jm[j] * G) : n_heads + kvh;
-            in[j] = rope_row_load(q + ((size_t)jm[j] * total_heads + src_head) * kHd, is_q ? rope.qw : rope.kw,
-                                  rope.cos_t, rope.sin_t, rope.positions[jm[j]], rope.max_pos, lane);
+            in[j] = rope_row_load(q + ((size_t)jm[j] * total_heads + src_head) * kHd, is_q ? qw : kw,
+                                  cos_t, sin_t, positions[jm[j]], max_pos, lane);
             if (!is_q) {
                 const uint16_t *xv = q + ((size_t)jm[j] * total_heads + n_heads + n_kv + kvh) * kHd;
                 v0[j] = xv[lane];
@@ -567,7 +583,7 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
     const int hide = meta[1];
     const int total = cache_len + M;
     const int live_chunks = (total + kChunk - 1) / kChunk;
-    const int cpw = attn_chunks_per_part(live_chunks, parts);
+    const int cpw = small_div(live_chunks + parts - 1, parts_recip);  // attn_chunks_per_part
     const int c_begin = part * cpw;
     if (c_begin >= live_chunks) return;  // whole workgroup; the combine step counts the same parts
     const int c_end = min(c_begin + cpw, live_chunks);
@@ -581,7 +597,7 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
         const int pd = pt * kPairTile + 4 * kb + r;
         valid[r] = pd < pairs_total;
         const int pc = valid[r] ? pd : pairs_total - 1;
-        row_of[r] = pc / G;
+        row_of[r] = small_div(pc, g_recip);
         head_of[r] = kvh * G + (pc - row_of[r] * G);
         wmask[r] = (uint32_t)meta[2 + row_of[r]];
     }
@@ -668,7 +684,7 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
                 const bool is_q = job < n_q;
                 const int m = jm[j];
                 uint32_t o0, o1;
-                rope_row_math(in[j], rope.eps, o0, o1);
+                rope_row_math(in[j], eps, o0, o1);
                 uint16_t *dst = is_q ? q_new[job] : k_new[m];
                 dst[lane] = (uint16_t)o0;
                 dst[lane + 64] = (uint16_t)o1;
@@ -698,7 +714,7 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
         for (int j = 0; j < 4; ++j) qreg[j] = qrow[4 * j + kb];
     } else {
         const int qp = min(pt * kPairTile + col, pairs_total - 1);
-        const int qm = qp / G, qg = qp - qm * G;
+        const int qm = small_div(qp, g_recip), qg = qp - qm * G;
         const uint4 *qrow =
             reinterpret_cast<const uint4 *>(q + ((size_t)qm * n_heads + kvh * G + qg) * kHd);
 #pragma unroll
@@ -862,7 +878,7 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
         // as well, so nothing else needs to be written back or invalidated.
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        const int live = (live_chunks + cpw - 1) / cpw;  // workgroups of this kv head that got here
+        const int live = cpw == 1 ? live_chunks : (live_chunks + cpw - 1) / cpw;  // workgroups of this kv head that got here
         if (threadIdx.x == 0) {
             const unsigned old = __hip_atomic_fetch_add(&fin.arrivals[kvh], 1u, __ATOMIC_RELAXED,
                                                         __HIP_MEMORY_SCOPE_AGENT);
@@ -874,7 +890,7 @@ attn_mfma_kernel(const uint16_t *q, uint16_t *k_layer, uint16_t *v_layer,
         const int pr = threadIdx.x >> 4, j = threadIdx.x & 15;
         const bool mine = pr < pairs_total;
         const int pc = mine ? pr : pairs_total - 1;
-        const int row = pc / G, head = kvh * G + (pc - row * G);
+        const int row = small_div(pc, g_recip), head = kvh * G + (pc - row * G);
         float num[8];
         combine_head_slice<true>(part_out, part_bytes, (row * n_heads + head) * parts * kPartStride, live, j, num);
         uint32_t ob[8];
@@ -1040,14 +1056,14 @@ constexpr int kCombinePartsThreads = 512;
 
 __global__ void __launch_bounds__(kCombinePartsThreads)
 attn_combine_parts_kernel(const float *part, const int32_t *meta, uint16_t *out_bf16, int8_t *out_q,
-                          float *out_s, int M, int n_heads, int parts, int sigma) {
+                          float *out_s, int M, int n_heads, int parts, int sigma, unsigned parts_recip) {
     __shared__ float max_scratch[kCombinePartsThreads / 64];
     const int m = blockIdx.x;
     const int tid = threadIdx.x;
     const int total = min(max(meta[0], 0), sigma) + M;
     const int live_chunks = (total + kChunk - 1) / kChunk;
-    const int cpw = attn_chunks_per_part(live_chunks, parts);
-    const int live = (live_chunks + cpw - 1) / cpw;  // <= parts <= kMaxParts
+    const int cpw = small_div(live_chunks + parts - 1, parts_recip);  // attn_chunks_per_part
+    const int live = cpw == 1 ? live_chunks : (live_chunks + cpw - 1) / cpw;  // <= parts <= kMaxParts
     const int nvec = n_heads * (kHd / 8);
     const bool mine = tid < nvec;
     const int v = mine ? tid : nvec - 1;
@@ -1750,24 +1766,22 @@ static int launch_attention(const void *q, void *k_layer, void *v_layer, const i
     if (g_attn_engine == 0 || rope != nullptr) {
         parts = a.n_chunks < kMaxParts ? a.n_chunks : kMaxParts;
         const int tiles = (M * a.hpg + kPairTile - 1) / kPairTile;
-        const dim3 grid(n_kv * parts * tiles), block(kAttnWaves * 64);
+        const dim3 grid(n_kv, parts, tiles), block(kAttnWaves * 64);
+        const AttnDims dims(M, a.hpg, n_kv, parts);
+        const RopeIn r = rope != nullptr ? *rope : RopeIn{};
+#define ATTN_ARGS                                                                                        \
+    static_cast<const uint16_t *>(q), meta, r.positions, r.cos_t, r.sin_t, r.qw, dims.sizes, dims.recips, sigma, \
+        r.max_pos, r.kw, static_cast<uint16_t *>(k_layer), static_cast<uint16_t *>(v_layer), a.part,        \
+        a.scale_log2e, r.eps, slots
         if (fin != nullptr) {  // the one launch that also merges its partials (rope != nullptr, one tile)
-            hipLaunchKernelGGL((attn_mfma_kernel<true, true>), grid, block, 0, st,
-                               static_cast<const uint16_t *>(q), static_cast<uint16_t *>(k_layer),
-                               static_cast<uint16_t *>(v_layer), meta, a.part, a.scale_log2e, M,
-                               n_heads, n_kv, a.hpg, slots, sigma, parts, *rope, *fin);
+            hipLaunchKernelGGL((attn_mfma_kernel<true, true>), grid, block, 0, st, ATTN_ARGS, *fin);
             return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
         }
         if (rope != nullptr)
-            hipLaunchKernelGGL((attn_mfma_kernel<true, false>), grid, block, 0, st,
-                               static_cast<const uint16_t *>(q), static_cast<uint16_t *>(k_layer),
-                               static_cast<uint16_t *>(v_layer), meta, a.part, a.scale_log2e, M,
-                               n_heads, n_kv, a.hpg, slots, sigma, parts, *rope, FinOut{});
+            hipLaunchKernelGGL((attn_mfma_kernel<true, false>), grid, block, 0, st, ATTN_ARGS, FinOut{});
         else
-            hipLaunchKernelGGL((attn_mfma_kernel<false, false>), grid, block, 0, st,
-                               static_cast<const uint16_t *>(q), static_cast<uint16_t *>(k_layer),
-                               static_cast<uint16_t *>(v_layer), meta, a.part, a.scale_log2e, M,
-                               n_heads, n_kv, a.hpg, slots, sigma, parts, RopeIn{}, FinOut{});
+            hipLaunchKernelGGL((attn_mfma_kernel<false, false>), grid, block, 0, st, ATTN_ARGS, FinOut{});
+#undef ATTN_ARGS
     } else {
     const int rw = rows_per_wave(M);
     a.row_groups = (M + rw - 1) / rw;
@@ -1800,7 +1814,7 @@ static int launch_attention(const void *q, void *k_layer, void *v_layer, const i
     if (parts > 0)
         hipLaunchKernelGGL(attn_combine_parts_kernel, dim3(M), dim3(kCombinePartsThreads), 0, st,
                            c.part, c.meta, c.out_bf16, c.out_q, c.out_s, c.M, c.n_heads, parts,
-                           c.sigma);
+                           c.sigma, small_recip(parts));
     else
         hipLaunchKernelGGL(attn_combine_kernel, dim3(M), dim3(kCombineThreads), 0, st, c.part,
                            c.meta, c.out_bf16, c.out_q, c.out_s, c.M, c.n_heads, c.n_chunks,
