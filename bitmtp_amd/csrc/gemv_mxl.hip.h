@@ -78,17 +78,10 @@ __host__ __device__ constexpr size_t mxl_lds_bytes(int mmax, int waves) {
 // scale) instead of the scaled result; the scales and multipliers are not read.
 // RAGGED: some problem's K is not a multiple of 512 (kernel gemv_mxl_ragged_kernel).
 template <int BITS, int MR, bool SF16, int W, int NB, bool G32, bool RAGGED>
-__device__ __forceinline__ void gemv_mxl_body(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8,
-                                              int e9, int e10, int e11, int out_f32, int mmax, const MxlTable &tbl) {
+__device__ __forceinline__ void gemv_mxl_body(const MxlDesc &d, int out_f32, int mmax) {
     using MF = MfmaFmt<BITS>;
     extern __shared__ __align__(16) unsigned char smem[];
-
-    // ---- descriptor of this workgroup: (wg >= e) is the sign bit of e - 1 - wg (scalar)
     const int wg = (int)blockIdx.x;
-    const auto ge = [wg](int e) { return (int)((uint32_t)(e - 1 - wg) >> 31); };
-    const int di = ge(e0) + ge(e1) + ge(e2) + ge(e3) + ge(e4) + ge(e5) + ge(e6) + ge(e7) + ge(e8) +
-                   ge(e9) + ge(e10) + ge(e11);
-    const MxlDesc d = tbl.d[di];
     const int K = d.K, N = d.N, M = d.M;
     const int G = K >> 7;
     const int KT = RAGGED ? (K + 511) >> 9 : K >> 9;  // (ragged: the last tile may hold one to three groups)
@@ -280,11 +273,28 @@ __device__ __forceinline__ void gemv_mxl_body(int e0, int e1, int e2, int e3, in
     }
 }
 
+// descriptor of this workgroup: (wg >= e) is the sign bit of e - 1 - wg (scalar)
+__device__ __forceinline__ MxlDesc mxl_find(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8, int e9,
+                                            int e10, int e11, const MxlTable &tbl) {
+    const int wg = (int)blockIdx.x;
+    const auto ge = [wg](int e) { return (int)((uint32_t)(e - 1 - wg) >> 31); };
+    return tbl.d[ge(e0) + ge(e1) + ge(e2) + ge(e3) + ge(e4) + ge(e5) + ge(e6) + ge(e7) + ge(e8) + ge(e9) + ge(e10) +
+                 ge(e11)];
+}
+
 template <int BITS, int MR, bool SF16, int W, int NB, int OCC, bool G32 = false>
 __global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
 gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8, int e9,
                 int e10, int e11, int out_f32, int mmax, const MxlTable tbl) {
-    gemv_mxl_body<BITS, MR, SF16, W, NB, G32, false>(e0, e1, e2, e3, e4, e5, e6, e7, e8, e9, e10, e11, out_f32, mmax, tbl);
+    gemv_mxl_body<BITS, MR, SF16, W, NB, G32, false>(mxl_find(e0, e1, e2, e3, e4, e5, e6, e7, e8, e9, e10, e11, tbl), out_f32, mmax);
+}
+
+// A launch of one matrix: no descriptor to wait for, what the first loads need arrives in registers with the wave.
+template <int BITS, int MR, bool SF16, int W, int NB, int OCC>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
+gemv_mxl_kernel(const int8_t *A, const uint8_t *B, const uint16_t *ws, const float *s, void *out, int N, int K,
+                    int M, int out_f32) {
+    gemv_mxl_body<BITS, MR, SF16, W, NB, false, false>(MxlDesc{A, B, out, s, ws, M, N, K, 0, {0, 0}}, out_f32, M);
 }
 
 // Rows of any whole number of groups from four on: the dot4 kernel, the only other one that takes them, walks
@@ -294,7 +304,7 @@ template <int BITS, int MR, bool SF16, int W, int NB, int OCC, bool G32 = false>
 __global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
 gemv_mxl_ragged_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, int e8, int e9,
                        int e10, int e11, int out_f32, int mmax, const MxlTable tbl) {
-    gemv_mxl_body<BITS, MR, SF16, W, NB, G32, true>(e0, e1, e2, e3, e4, e5, e6, e7, e8, e9, e10, e11, out_f32, mmax, tbl);
+    gemv_mxl_body<BITS, MR, SF16, W, NB, G32, true>(mxl_find(e0, e1, e2, e3, e4, e5, e6, e7, e8, e9, e10, e11, tbl), out_f32, mmax);
 }
 
 // ---------------------------------------------------------------------------
@@ -302,28 +312,35 @@ gemv_mxl_ragged_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, i
 // ---------------------------------------------------------------------------
 using MxlKernelFn = void (*)(int, int, int, int, int, int, int, int, int, int, int, int, int, int,
                              const MxlTable);
+using MxlOneFn = void (*)(const int8_t *, const uint8_t *, const uint16_t *, const float *, void *, int, int, int, int);
+struct MxlKernels {
+    MxlKernelFn table;
+    MxlOneFn one;  // null: the table form takes single matrices too (ragged rows, group sums)
+};
 
 constexpr int kMxlWideWaves = 12;
 
 // width class: 0 = every block has one token, 1 = at most eight tokens, 2 = up to sixteen;
 // dense: more than four workgroups per CU to place (only matters for width class 2)
 template <int BITS, int MR, int W, int NB, int OCC>
-MxlKernelFn mxl_kernel_n(int scale_kind, bool ragged) {
+MxlKernels mxl_kernel_n(int scale_kind, bool ragged) {
     if (ragged) {
-        if (scale_kind == 2) return gemv_mxl_ragged_kernel<BITS, MR, false, W, NB, OCC, true>;
-        return scale_kind == 1 ? gemv_mxl_ragged_kernel<BITS, MR, true, W, NB, OCC> : gemv_mxl_ragged_kernel<BITS, MR, false, W, NB, OCC>;
+        if (scale_kind == 2) return {gemv_mxl_ragged_kernel<BITS, MR, false, W, NB, OCC, true>, nullptr};
+        return {scale_kind == 1 ? gemv_mxl_ragged_kernel<BITS, MR, true, W, NB, OCC> : gemv_mxl_ragged_kernel<BITS, MR, false, W, NB, OCC>,
+                nullptr};
     }
-    if (scale_kind == 2) return gemv_mxl_kernel<BITS, MR, false, W, NB, OCC, true>;  // int32 group sums from the same builds
-    return scale_kind == 1 ? gemv_mxl_kernel<BITS, MR, true, W, NB, OCC> : gemv_mxl_kernel<BITS, MR, false, W, NB, OCC>;
+    if (scale_kind == 2) return {gemv_mxl_kernel<BITS, MR, false, W, NB, OCC, true>, nullptr};  // int32 group sums from the same builds
+    if (scale_kind == 1) return {gemv_mxl_kernel<BITS, MR, true, W, NB, OCC>, gemv_mxl_kernel<BITS, MR, true, W, NB, OCC>};
+    return {gemv_mxl_kernel<BITS, MR, false, W, NB, OCC>, gemv_mxl_kernel<BITS, MR, false, W, NB, OCC>};
 }
 template <int BITS, int W, int OCC1, int OCC2>
-MxlKernelFn mxl_kernel_w(int scale_kind, int width_class, bool ragged) {
+MxlKernels mxl_kernel_w(int scale_kind, int width_class, bool ragged) {
     if (width_class == 0) return mxl_kernel_n<BITS, 1, W, 1, OCC1>(scale_kind, ragged);
     if (width_class == 1) return mxl_kernel_n<BITS, 4, W, 1, OCC1>(scale_kind, ragged);
     return mxl_kernel_n<BITS, 4, W, 2, OCC2>(scale_kind, ragged);
 }
 template <int BITS>
-MxlKernelFn mxl_kernel(int scale_kind, int width_class, bool wide, bool dense, bool ragged) {
+MxlKernels mxl_kernel(int scale_kind, int width_class, bool wide, bool dense, bool ragged) {
     if (wide) return mxl_kernel_w<BITS, kMxlWideWaves, 3, 3>(scale_kind, width_class, ragged);
     return dense ? mxl_kernel_w<BITS, kMxWaves, 5, 5>(scale_kind, width_class, ragged)
                  : mxl_kernel_w<BITS, kMxWaves, 5, 4>(scale_kind, width_class, ragged);
@@ -334,11 +351,13 @@ int mxl_init_device(int max_lds) {
     for (int sk = 0; sk < 3; ++sk)
         for (int wc = 0; wc < 3; ++wc)
             for (int wide = 0; wide < 2; ++wide)
-                for (int k = 0; k < 4; ++k)
-                    if (hipFuncSetAttribute(
-                            reinterpret_cast<const void *>(mxl_kernel<BITS>(sk, wc, wide != 0, (k & 1) != 0, (k & 2) != 0)),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, max_lds) != hipSuccess)
-                        return 2;
+                for (int k = 0; k < 4; ++k) {
+                    const MxlKernels fn = mxl_kernel<BITS>(sk, wc, wide != 0, (k & 1) != 0, (k & 2) != 0);
+                    for (const void *f : {reinterpret_cast<const void *>(fn.table), reinterpret_cast<const void *>(fn.one)})
+                        if (f != nullptr &&
+                            hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds) != hipSuccess)
+                            return 2;
+                }
     return 0;
 }
 
@@ -408,10 +427,17 @@ int launch_mxl(const GemvProblem *probs, int count, int out_kind, int scale_kind
     for (int i = count; i < kMxlMaxDesc; ++i) ends[i] = 0x7fffffff;
     const int width_class = one_token ? 0 : (mmax <= 8 ? 1 : 2);
     const int variant = out_kind == OUT_G32 ? 2 : scale_kind;
-    hipLaunchKernelGGL(mxl_kernel<BITS>(variant, width_class, wide, dense, ragged), dim3(wg, 1, 1), dim3(waves * 64, 1, 1),
-                       lds, stream, ends[0], ends[1], ends[2], ends[3], ends[4], ends[5], ends[6],
-                       ends[7], ends[8], ends[9], ends[10], ends[11], out_kind == OUT_F32 ? 1 : 0,
-                       mmax, tbl);
+    const MxlKernels fn = mxl_kernel<BITS>(variant, width_class, wide, dense, ragged);
+    const bool one = count == 1 && fn.one != nullptr;
+    if (one) {
+        const MxlDesc &d = tbl.d[0];
+        hipLaunchKernelGGL(fn.one, dim3(wg, 1, 1), dim3(waves * 64, 1, 1), lds, stream, d.A, d.B, d.ws, d.s, d.out, d.N, d.K,
+                           d.M, out_kind == OUT_F32 ? 1 : 0);
+    } else {
+        hipLaunchKernelGGL(fn.table, dim3(wg, 1, 1), dim3(waves * 64, 1, 1), lds, stream, ends[0], ends[1], ends[2], ends[3],
+                           ends[4], ends[5], ends[6], ends[7], ends[8], ends[9], ends[10], ends[11],
+                           out_kind == OUT_F32 ? 1 : 0, mmax, tbl);
+    }
     // <BITS, MR, SF16, W, NB, OCC, G32> as instantiated by mxl_kernel
     note_kernel(ragged ? "gemv_mxl_ragged_kernel" : "gemv_mxl_kernel", BITS, width_class == 0 ? 1 : 4, scale_kind == 1 && variant != 2, waves,
                 width_class == 2 ? 2 : 1, wide ? 3 : (width_class == 2 && !dense ? 4 : 5), variant == 2);
