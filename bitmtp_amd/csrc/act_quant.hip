@@ -198,9 +198,11 @@ __device__ __forceinline__ void unpack8_bf16(const uint4 raw, float out[8]) {
 template <bool ADD, int VPT>
 __global__ void __launch_bounds__(kMaxProducerThreads)
 rmsnorm_quant_kernel(const uint16_t *x, const uint16_t *residual, const uint16_t *w, float eps,
-                     uint16_t *h_out, uint16_t *n_out, int8_t *q, float *s, int K, int T) {
+                     int geom, uint16_t *h_out, uint16_t *n_out, int8_t *q, float *s) {
     // n_out (optional): the normalised row in bf16; q / s (optional): its quantisation.
-    // T = workgroup size, passed explicitly: reading blockDim costs a load at kernel start
+    // geom = K | waves << 26: the workgroup size passed explicitly (reading blockDim costs a load at kernel start), and
+    // sixteen dwords of arguments in all, which arrive with the wave; a seventeenth is a memory round trip
+    const int K = geom & 0x3ffffff, T = (int)((uint32_t)geom >> 26) * 64;
     __shared__ double sum_scratch[kMaxProducerWaves];
     __shared__ float max_scratch[kMaxProducerWaves];
     const int m = blockIdx.x;
@@ -352,10 +354,10 @@ void launch_rmsnorm(const uint16_t *x, const uint16_t *r, const uint16_t *w, flo
     const int nvec = K / 8;
     const dim3 grid(M), block(producer_threads(nvec));
     switch (producer_vpt(nvec)) {
-        case 1: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 1>), grid, block, 0, st, x, r, w, eps, h_out, n_out, q, s, K, (int)block.x); break;
-        case 2: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 2>), grid, block, 0, st, x, r, w, eps, h_out, n_out, q, s, K, (int)block.x); break;
-        case 4: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 4>), grid, block, 0, st, x, r, w, eps, h_out, n_out, q, s, K, (int)block.x); break;
-        default: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 8>), grid, block, 0, st, x, r, w, eps, h_out, n_out, q, s, K, (int)block.x); break;
+        case 1: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 1>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
+        case 2: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 2>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
+        case 4: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 4>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
+        default: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 8>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
     }
 }
 
