@@ -43,16 +43,28 @@ HBM_PEAK_GBPS = 8000.0
 MIN_DISTINCT_BYTES = 512 << 20   # every timed graph walks at least this much distinct weight data
 
 
+# what the grouped layer launch of one to sixteen tokens is compiled from and chosen by
+MEASURED_SOURCES = ("gemv_core.h", "gemv_dispatch.hip.h", "gemv_mfma.hip.h", "gemv_mx.hip.h", "gemv_mxl.hip.h",
+                    "packed_gemv.hip.h", "t2g128_kernels.hip", "wave_reduce.h")
+
+
+def code_of(source: str) -> str:
+    """C++ source without comments and with every run of blanks one blank: what can change a kernel."""
+    import re
+    keep = lambda m: " " if m.group(0).startswith("/") else m.group(0)
+    text = re.sub(r'//[^\n]*|/\*.*?\*/|"(?:\\.|[^"\\])*"', keep, source, flags=re.S)
+    return " ".join(text.split())
+
+
 def kernel_sources_digest() -> str:
-    """sha256 over the GEMV kernel sources (csrc/*.h, *.hip of the GEMV libraries), the key under
-    which profiles/traffic.json records what its counters were measured on."""
+    """sha256 over the code (comments aside) of the measured launch, the key under which
+    profiles/traffic.json records what its counters were measured on."""
     import hashlib
     csrc = os.path.join(ROOT, "bitmtp_amd", "csrc")
     h = hashlib.sha256()
-    for name in sorted(os.listdir(csrc)):
-        if name.startswith("gemv_") or name in ("packed_gemv.hip.h", "wave_reduce.h", "t2g128_kernels.hip"):
-            with open(os.path.join(csrc, name), "rb") as f:
-                h.update(name.encode() + b"\0" + f.read())
+    for name in MEASURED_SOURCES:
+        with open(os.path.join(csrc, name), encoding="utf-8") as f:
+            h.update(name.encode() + b"\0" + code_of(f.read()).encode())
     return h.hexdigest()[:16]
 
 

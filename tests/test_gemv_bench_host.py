@@ -60,6 +60,27 @@ def test_traffic_table_matches_the_layer_bytes():
     assert bench.LAYER_BYTES == sum(bench.t2_bytes(n, k) for _, n, k in bench.PROJECTIONS) == 13369344
 
 
+def test_traffic_key_follows_the_code_and_not_its_comments():
+    import bench
+    a = 'int f(int x) {\n  // twice\n  return 2 * x; /* "quoted" */ }\nconst char *s = "// kept";\n'
+    assert bench.code_of(a) == 'int f(int x) { return 2 * x; } const char *s = "// kept";'
+    assert bench.code_of(a.replace("twice", "two times")) == bench.code_of(a) != bench.code_of(a.replace("2 * x", "3 * x"))
+    import os
+    csrc = os.path.join(bench.ROOT, "bitmtp_amd", "csrc")
+    included = set()
+    todo = ["t2g128_kernels.hip"]
+    while todo:
+        name = todo.pop()
+        if name in included:
+            continue
+        included.add(name)
+        with open(os.path.join(csrc, name)) as f:
+            todo += [os.path.basename(l.split('"')[1]) for l in f if l.startswith('#include "') and "include/" not in l]
+    # kernels of other widths and matrices are the only sources of that library left out
+    assert included - set(bench.MEASURED_SOURCES) == {"gemv_wide.hip.h", "gemv_mxs.hip.h", "gemv_rowreg.hip.h"}
+    assert set(bench.MEASURED_SOURCES) <= included
+
+
 def test_kernel_choices_of_the_sweep_tool():
     from bitmtp_amd import gemv_bench
     assert gemv_bench.KERNELS["auto"] == (0, 0)
