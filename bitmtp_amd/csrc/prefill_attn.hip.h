@@ -60,39 +60,148 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
     return u;
 }
 
+// What a workgroup of `tokens` consecutive rows, the last of them m0 + tokens - 1 at most, sees and where its lanes' pairs sit.
+struct Rows {
+    int m0, seen, chunks, masked_from;
+    __device__ __forceinline__ Rows(int tile, int tokens, int M, int base) {
+        m0 = tile * tokens;
+        seen = base + (M - m0 < tokens ? M : m0 + tokens);  // slots the last row sees
+        chunks = (seen + kSlots - 1) / kSlots;
+        masked_from = (base + m0 + 1) / kSlots;             // from here on some row does not see all slots
+    }
+};
+
+// A lane's pair: (row, query head) number `pair` of the workgroup; pairs without a row repeat the block's last one.
+struct Pair {
+    u32v4 q[8];   // its query, dims 16 j + 8 h + 0..7
+    int pos;      // the last slot it sees
+    size_t row;   // element its output row starts at
+    bool valid;
+    __device__ __forceinline__ Pair(const uint16_t *qs, int pair, int h, int m0, int tokens, int M, int base, int n_heads,
+                                    int hpg, int kvh) {
+        const int tok = pair / hpg, g = pair - tok * hpg;
+        valid = tok < tokens && m0 + tok < M;
+        const int m = valid ? m0 + tok : M - 1;
+        pos = base + m;
+        row = (size_t)m * n_heads * kHead + (size_t)(kvh * hpg + g) * kHead;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = *reinterpret_cast<const u32v4 *>(qs + row + 16 * j + 8 * h);
+    }
+};
+
+// The running softmax of a lane's query: o[d][r] is dim 32 d + 8 (r / 4) + 4 h + r % 4, l the sum of the lane's half of
+// the slots, both against the maximum m.
+struct Softmax {
+    f32x16 o[4];
+    float m, l;
+    __device__ __forceinline__ Softmax() : m(-INFINITY), l(0.0f) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    }
+};
+
+// A block of 4 slots x 8 dims of V, transposed: 8 stores of 4 slots each.
+__device__ __forceinline__ void park_v(unsigned char *vb, const u32v4 (&v)[4], int dim, int slot) {
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
+        uint2 t;
+        t.x = __builtin_amdgcn_perm(v[1][d / 2], v[0][d / 2], sel);
+        t.y = __builtin_amdgcn_perm(v[3][d / 2], v[2][d / 2], sel);
+        *reinterpret_cast<uint2 *>(vb + (dim + d) * kVPitch + slot * 2) = t;
+    }
+}
+
+// Chunk c, parked at kb / vb, into the running softmax of a wave's 32 queries.
+__device__ __forceinline__ void attend(const unsigned char *kb, const unsigned char *vb, const Pair &p, int c,
+                                       int masked_from, int col, int h, float scale_log2e, Softmax &x) {
+    f32x16 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+        const unsigned char *kp = kb + (32 * t + col) * kKPitch + 16 * h;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(*reinterpret_cast<const u32v4 *>(kp + 32 * j)),
+                                                           frag(p.q[j]), s[t], 0, 0, 0);
+    }
+    // s[t][r]: slot 64 c + 32 t + 8 (r / 4) + 4 h + r % 4
+    if (c >= masked_from) {
+        const int rel = p.pos - c * kSlots - 4 * h;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (32 * t + 8 * (r / 4) + r % 4 > rel) s[t][r] = -INFINITY;
+    }
+    float mx = s[0][0];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(x.m, mx * scale_log2e);
+    // A row may have met nothing but -inf so far: a wave that does not start at slot 0 can see nothing of its first
+    // chunk, and scores themselves can be -inf.  Its exponentials are then 0 against any finite maximum.
+    const float shift = m_new == -INFINITY ? 0.0f : m_new;
+    if (__any(m_new > x.m)) {
+        const float alpha = __builtin_amdgcn_exp2f(x.m - shift);
+        x.l *= alpha;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) x.o[d][r] *= alpha;
+        x.m = m_new;
+    }
+    uint32_t e[2][8];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const float a = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r], scale_log2e, -shift));
+            const float b = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r + 1], scale_log2e, -shift));
+            e[t][r] = pack_bf16(a, b);
+            bf16x2 pv;
+            __builtin_memcpy(&pv, &e[t][r], 4);
+            const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
+            x.l = __builtin_amdgcn_fdot2_f32_bf16(pv, ones, x.l, false);
+        }
+    // K-step ks takes slots 16 ks + 4 h + 0..3 and 16 ks + 8 + 4 h + 0..3 of each lane half
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        const uint32_t *pp = e[ks / 2] + 4 * (ks & 1);
+        const bf16x8 pf = frag(u32v4{pp[0], pp[1], pp[2], pp[3]});
+        const unsigned char *vp = vb + col * kVPitch + (16 * ks + 4 * h) * 2;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const uint2 lo = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch);
+            const uint2 hi = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch + 16);
+            x.o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(u32v4{lo.x, lo.y, hi.x, hi.y}), pf, x.o[d], 0, 0, 0);
+        }
+    }
+}
+
+// A kv head's K or V, slots from `seen` on read as zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t history(const uint16_t *layer, int kvh, int slots, int seen) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(layer + (size_t)kvh * slots * kHead), 0, seen * 2 * kHead,
+                                             kRawBuffer);
+}
+
 __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 prefill_attn_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *v_layer, uint16_t *out,
                     float scale_log2e, int M, int n_heads, int n_kv, int hpg, int slots, int base, int tokens,
                     int tiles) {
     __shared__ __align__(16) unsigned char smem[kLds];
     const int kvh = (int)blockIdx.x % n_kv;
-    const int m0 = (tiles - 1 - (int)blockIdx.x / n_kv) * tokens;
+    const Rows w(tiles - 1 - (int)blockIdx.x / n_kv, tokens, M, base);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, h = lane >> 5;
-
-    // ---- this lane's query
-    const int pair = wave * 32 + col;
-    const int tok = pair / hpg, g = pair - tok * hpg;
-    const bool valid = tok < tokens && m0 + tok < M;
-    const int m = valid ? m0 + tok : M - 1;
-    const int pos = base + m;
-    const size_t row = (size_t)m * n_heads * kHead + (size_t)(kvh * hpg + g) * kHead;
-    u32v4 qr[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qr[j] = *reinterpret_cast<const u32v4 *>(q + row + 16 * j + 8 * h);
-
-    const int rows = M - m0 < tokens ? M - m0 : tokens;
-    const int seen = base + m0 + rows;                       // slots the last row sees
-    const int chunks = (seen + kSlots - 1) / kSlots;
-    const int masked_from = (base + m0 + 1) / kSlots;        // from here on some row does not see all slots
-
-    // slots from `seen` on read as zero
-    const size_t head = (size_t)kvh * slots * kHead;
-    const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t *>(k_layer + head), 0, seen * 2 * kHead, kRawBuffer);
-    const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t *>(v_layer + head), 0, seen * 2 * kHead, kRawBuffer);
+    const Pair p(q, wave * 32 + col, h, w.m0, tokens, M, base, n_heads, hpg, kvh);
+    const __amdgpu_buffer_rsrc_t rK = history(k_layer, kvh, slots, w.seen), rV = history(v_layer, kvh, slots, w.seen);
 
     const int k_slot = tid >> 4, k_col = tid & 15;           // K: 16-byte column of slots k_slot + 16 i
     const int v_slot = (tid & 15) * 4, v_dim = (tid >> 4) * 8;  // V: a block of 4 slots x 8 dims
@@ -107,114 +216,38 @@ prefill_attn_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *
         for (int i = 0; i < 4; ++i) vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rV, v_off + i * 2 * kHead, s, 0);
     };
     const auto park = [&](int buf) {
-        unsigned char *kb = smem + buf * (kKBytes + kVBytes), *vb = kb + kKBytes;
+        unsigned char *kb = smem + buf * (kKBytes + kVBytes);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             *reinterpret_cast<u32v4 *>(kb + (k_slot + 16 * i) * kKPitch + k_col * 16) = kr[i];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) {
-            const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
-            uint2 v;
-            v.x = __builtin_amdgcn_perm(vr[1][d / 2], vr[0][d / 2], sel);
-            v.y = __builtin_amdgcn_perm(vr[3][d / 2], vr[2][d / 2], sel);
-            *reinterpret_cast<uint2 *>(vb + (v_dim + d) * kVPitch + v_slot * 2) = v;
-        }
+        park_v(kb + kKBytes, vr, v_dim, v_slot);
     };
 
-    f32x16 o[4];
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
-    float m_run = -INFINITY, l_run = 0.0f;
-
+    Softmax x;
     load(0);
     park(0);
-    if (chunks > 1) load(1);
-    for (int c = 0; c < chunks; ++c) {
+    if (w.chunks > 1) load(1);
+    for (int c = 0; c < w.chunks; ++c) {
         const int buf = c & 1;
         // chunk c is parked, chunk c - 1 no longer read (loads for later chunks stay in flight)
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (c + 1 < chunks) park(buf ^ 1);
-        if (c + 2 < chunks) load(c + 2);
-        const unsigned char *kb = smem + buf * (kKBytes + kVBytes), *vb = kb + kKBytes;
-
-        f32x16 s[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
-            const unsigned char *kp = kb + (32 * t + col) * kKPitch + 16 * h;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(*reinterpret_cast<const u32v4 *>(kp + 32 * j)),
-                                                               frag(qr[j]), s[t], 0, 0, 0);
-        }
-        // s[t][r]: slot 64 c + 32 t + 8 (r / 4) + 4 h + r % 4
-        if (c >= masked_from) {
-            const int rel = pos - c * kSlots - 4 * h;
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (32 * t + 8 * (r / 4) + r % 4 > rel) s[t][r] = -INFINITY;
-        }
-        float mx = s[0][0];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m_run, mx * scale_log2e);  // finite: every row sees slot 0
-        if (__any(m_new > m_run)) {
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-            l_run *= alpha;
-#pragma unroll
-            for (int d = 0; d < 4; ++d)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
-            m_run = m_new;
-        }
-        uint32_t p[2][8];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const float a = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r], scale_log2e, -m_run));
-                const float b = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r + 1], scale_log2e, -m_run));
-                p[t][r] = pack_bf16(a, b);
-                bf16x2 pv;
-                __builtin_memcpy(&pv, &p[t][r], 4);
-                const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-                l_run = __builtin_amdgcn_fdot2_f32_bf16(pv, ones, l_run, false);
-            }
-        // K-step ks takes slots 16 ks + 4 h + 0..3 and 16 ks + 8 + 4 h + 0..3 of each lane half
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const uint32_t *pp = p[ks / 2] + 4 * (ks & 1);
-            const bf16x8 pf = frag(u32v4{pp[0], pp[1], pp[2], pp[3]});
-            const unsigned char *vp = vb + col * kVPitch + (16 * ks + 4 * h) * 2;
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const uint2 lo = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch);
-                const uint2 hi = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch + 16);
-                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(u32v4{lo.x, lo.y, hi.x, hi.y}), pf, o[d], 0, 0, 0);
-            }
-        }
+        if (c + 1 < w.chunks) park(buf ^ 1);
+        if (c + 2 < w.chunks) load(c + 2);
+        const unsigned char *kb = smem + buf * (kKBytes + kVBytes);
+        attend(kb, kb + kKBytes, p, c, w.masked_from, col, h, scale_log2e, x);
     }
 
-    const float l = l_run + __shfl_xor(l_run, 32);
-    if (!valid) return;
+    const float l = x.l + __shfl_xor(x.l, 32);
+    if (!p.valid) return;
     const float inv = 1.0f / l;
-    // o[d][r]: dim 32 d + 8 (r / 4) + 4 h + r % 4
 #pragma unroll
     for (int d = 0; d < 4; ++d)
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             uint2 v;
-            v.x = pack_bf16(o[d][4 * k] * inv, o[d][4 * k + 1] * inv);
-            v.y = pack_bf16(o[d][4 * k + 2] * inv, o[d][4 * k + 3] * inv);
-            *reinterpret_cast<uint2 *>(out + row + 32 * d + 8 * k + 4 * h) = v;
+            v.x = pack_bf16(x.o[d][4 * k] * inv, x.o[d][4 * k + 1] * inv);
+            v.y = pack_bf16(x.o[d][4 * k + 2] * inv, x.o[d][4 * k + 3] * inv);
+            *reinterpret_cast<uint2 *>(out + p.row + 32 * d + 8 * k + 4 * h) = v;
         }
 }
 
@@ -232,27 +265,12 @@ prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint
                           int tiles) {
     __shared__ __align__(16) unsigned char smem[kSplitLds];
     const int kvh = (int)blockIdx.x % n_kv;
-    const int m0 = (tiles - 1 - (int)blockIdx.x / n_kv) * tokens;
+    const Rows rows(tiles - 1 - (int)blockIdx.x / n_kv, tokens, M, base);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int col = lane & 31, h = lane >> 5;
-    const int tok = col / hpg, g = col - tok * hpg;
-    const bool valid = tok < tokens && m0 + tok < M;
-    const int m = valid ? m0 + tok : M - 1;
-    const int pos = base + m;
-    const size_t row = (size_t)m * n_heads * kHead + (size_t)(kvh * hpg + g) * kHead;
-    u32v4 qr[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qr[j] = *reinterpret_cast<const u32v4 *>(q + row + 16 * j + 8 * h);
-    const int rows = M - m0 < tokens ? M - m0 : tokens;
-    const int seen = base + m0 + rows;
-    const int chunks = (seen + kSlots - 1) / kSlots;
-    const int masked_from = (base + m0 + 1) / kSlots;
-    const size_t head = (size_t)kvh * slots * kHead;
-    const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t *>(k_layer + head), 0, seen * 2 * kHead, kRawBuffer);
-    const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t *>(v_layer + head), 0, seen * 2 * kHead, kRawBuffer);
+    const Pair p(q, col, h, rows.m0, tokens, M, base, n_heads, hpg, kvh);
+    const __amdgpu_buffer_rsrc_t rK = history(k_layer, kvh, slots, rows.seen), rV = history(v_layer, kvh, slots, rows.seen);
     unsigned char *kb = smem + wave * kSplitStage, *vb = kb + kKBytes;
     const int k_slot = lane >> 4, k_col = lane & 15;            // slots k_slot + 4 i
     const int v_slot = (lane & 15) * 4, v_dim = (lane >> 4) * 8;  // dims v_dim + 32 i
@@ -269,89 +287,15 @@ prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint
                 vr[i][t] = __builtin_amdgcn_raw_buffer_load_b128(rV, (v_slot + t) * 2 * kHead + (v_dim + 32 * i) * 2, s, 0);
     };
 
-    f32x16 o[4];
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
-    float m_run = -INFINITY, l_run = 0.0f;
-    if (wave < chunks) load(wave);
-    for (int c = wave; c < chunks; c += kWaves) {
+    Softmax x;
+    if (wave < rows.chunks) load(wave);
+    for (int c = wave; c < rows.chunks; c += kWaves) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) *reinterpret_cast<u32v4 *>(kb + (k_slot + 4 * i) * kKPitch + k_col * 16) = kr[i];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int d = 0; d < 8; ++d) {
-                const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
-                uint2 v;
-                v.x = __builtin_amdgcn_perm(vr[i][1][d / 2], vr[i][0][d / 2], sel);
-                v.y = __builtin_amdgcn_perm(vr[i][3][d / 2], vr[i][2][d / 2], sel);
-                *reinterpret_cast<uint2 *>(vb + (v_dim + 32 * i + d) * kVPitch + v_slot * 2) = v;
-            }
-        if (c + kWaves < chunks) load(c + kWaves);
-        f32x16 s[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
-            const unsigned char *kp = kb + (32 * t + col) * kKPitch + 16 * h;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(*reinterpret_cast<const u32v4 *>(kp + 32 * j)),
-                                                               frag(qr[j]), s[t], 0, 0, 0);
-        }
-        if (c >= masked_from) {
-            const int rel = pos - c * kSlots - 4 * h;
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (32 * t + 8 * (r / 4) + r % 4 > rel) s[t][r] = -INFINITY;
-        }
-        float mx = s[0][0];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m_run, mx * scale_log2e);
-        // (a row may see nothing of a chunk that is not its wave's first: its maximum is then still -inf)
-        const float shift = m_new == -INFINITY ? 0.0f : m_new;
-        if (__any(m_new > m_run)) {
-            const float alpha = __builtin_amdgcn_exp2f(m_run - shift);
-            l_run *= alpha;
-#pragma unroll
-            for (int d = 0; d < 4; ++d)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
-            m_run = m_new;
-        }
-        uint32_t p[2][8];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const float a = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r], scale_log2e, -shift));
-                const float b = __builtin_amdgcn_exp2f(fmaf(s[t][2 * r + 1], scale_log2e, -shift));
-                p[t][r] = pack_bf16(a, b);
-                bf16x2 pv;
-                __builtin_memcpy(&pv, &p[t][r], 4);
-                const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-                l_run = __builtin_amdgcn_fdot2_f32_bf16(pv, ones, l_run, false);
-            }
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const uint32_t *pp = p[ks / 2] + 4 * (ks & 1);
-            const bf16x8 pf = frag(u32v4{pp[0], pp[1], pp[2], pp[3]});
-            const unsigned char *vp = vb + col * kVPitch + (16 * ks + 4 * h) * 2;
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const uint2 lo = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch);
-                const uint2 hi = *reinterpret_cast<const uint2 *>(vp + 32 * d * kVPitch + 16);
-                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(u32v4{lo.x, lo.y, hi.x, hi.y}), pf, o[d], 0, 0, 0);
-            }
-        }
+        for (int i = 0; i < 4; ++i) park_v(vb, vr[i], v_dim + 32 * i, v_slot);
+        if (c + kWaves < rows.chunks) load(c + kWaves);
+        attend(kb, vb, p, c, rows.masked_from, col, h, scale_log2e, x);
     }
 
     // ---- the waves' results: [wave][register][lane], maxima and sums behind them
@@ -361,20 +305,20 @@ prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint
 #pragma unroll
     for (int d = 0; d < 4; ++d)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) meet[(wave * 64 + d * 16 + r) * 64 + lane] = o[d][r];
-    stat[wave * 128 + lane] = m_run;
-    stat[wave * 128 + 64 + lane] = l_run;
+        for (int r = 0; r < 16; ++r) meet[(wave * 64 + d * 16 + r) * 64 + lane] = x.o[d][r];
+    stat[wave * 128 + lane] = x.m;
+    stat[wave * 128 + 64 + lane] = x.l;
     __syncthreads();
     float top = -INFINITY, l = 0.0f, e[kWaves];
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) top = fmaxf(top, stat[w * 128 + lane]);  // finite: every row sees slot 0
+    for (int w = 0; w < kWaves; ++w) top = fmaxf(top, stat[w * 128 + lane]);
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
         e[w] = __builtin_amdgcn_exp2f(stat[w * 128 + lane] - top);
         l = fmaf(e[w], stat[w * 128 + 64 + lane], l);
     }
     l += __shfl_xor(l, 32);
-    if (!valid) return;
+    if (!p.valid) return;
     const float inv = 1.0f / l;
     // wave d finishes dims 32 d + 8 (r / 4) + 4 h + r % 4
 #pragma unroll
@@ -387,7 +331,7 @@ prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint
             for (int w = 0; w < kWaves; ++w) sum = fmaf(e[w], meet[(w * 64 + wave * 16 + 4 * k + i) * 64 + lane], sum);
             v[i] = sum * inv;
         }
-        *reinterpret_cast<uint2 *>(out + row + 32 * wave + 8 * k + 4 * h) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+        *reinterpret_cast<uint2 *>(out + p.row + 32 * wave + 8 * k + 4 * h) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
     }
 }
 

@@ -38,6 +38,36 @@ def test_prefill_attention_against_float64(m, n_heads, n_kv, base, slots):
     assert ((got - want).abs() <= 2e-3 + 2e-2 * want.abs()).all()
 
 
+def _assert_causal_attention(got, q, k, v, base):
+    """`got` [M, heads, 128] against float64, head by head: probabilities are rounded to bf16 and divided by their rounded
+    sum (2 * 2^-9 of sum p |v|), the row is rounded once more (2^-9); scores and sums are fp32."""
+    m, n_heads = q.shape[:2]
+    seen = base + m
+    ok = torch.arange(seen, device=DEV)[None, :] <= base + torch.arange(m, device=DEV)[:, None]
+    for h in range(n_heads):
+        kh, vh = (t[h // (n_heads // k.shape[0]), :seen].double() for t in (k, v))
+        p = torch.softmax((q[:, h].double() @ kh.T / np.sqrt(128.0)).masked_fill(~ok, float("-inf")), dim=-1)
+        want = p @ vh
+        bound = 2.0 ** -8 * (p @ vh.abs()) + 2.0 ** -9 * want.abs() + 1e-4
+        assert ((got[:, h].double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("m,n_heads,n_kv", [(40, 16, 8), (1030, 16, 8)])
+def test_prefill_attention_with_a_history_of_minus_infinity(m, n_heads, n_kv):
+    """Scores of -inf in the first slots (more than a whole 64-slot chunk of them) weigh nothing, in either kernel."""
+    from bitmtp_amd import decode_ops
+    print(f"[case] prefill attention, -inf scores, m={m}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(m)
+    base, hidden = 100, 70
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)
+    q, k, v = rnd(m, n_heads, 128), rnd(n_kv, base + m, 128), rnd(n_kv, base + m, 128)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[:, :hidden, 0] = float("-inf")
+    got = decode_ops.prefill_attention(q, k, v, base).view(m, n_heads, 128)
+    torch.cuda.synchronize()
+    _assert_causal_attention(got, q, k[:, hidden:], v[:, hidden:], base - hidden)
+
+
 @pytest.mark.parametrize("m,n_heads,n_kv", [(1, 4, 2), (33, 3, 1), (67, 16, 8)])
 def test_prompt_rows_rope_is_the_steps_own(m, n_heads, n_kv):
     """q / k norm + RoPE + KV write of prompt rows: the bits of the step's entry point, 32 rows at a time."""
