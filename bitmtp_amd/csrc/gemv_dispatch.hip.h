@@ -365,13 +365,15 @@ inline bool lean_any_k(int K) { return K % 512 != 0 && K > 512; }
 // 2048 x 2048: 4.7 / 6.3 at 64, 6.5 / 6.5 at 128; 2560 x 9728: 12.5 / 14.3 at 64, 16.6 / 15 at 96).  What the
 // lean kernel does not take leaves only the dot4 kernel where K is not a multiple of 512 (19000 x 2688: dot4
 // 9.1 us at four tokens, 15.5 at nine, against 10.6 at any width up to 32).
-inline bool wide_default(int M, int N, int K, int n_cus) {
+template <int BITS>
+bool wide_default(int M, int N, int K, int n_cus, int lds_limit) {
     const long lean_tiles = (long)((M + kMfmaTokens - 1) / kMfmaTokens) * ((N + 15) / 16);
     if (K % 512 != 0 && (lean_tiles > 8L * n_cus || N > kLongMatrixRows || K < 512)) return M >= kWideMinRagged;
     if (M <= kMfmaTokens) return false;
     const double G = K / kGroup;
     const double lean = 3.1 + G * (0.0087 + 0.051 * lean_tiles / n_cus);
-    return wide_estimate(wide_pick(M, N, K, n_cus), M, N, K, n_cus) < lean;
+    const int v = wide_pick<BITS>(M, N, K, n_cus, lds_limit);
+    return v >= 0 && wide_estimate(v, M, N, K, n_cus) < lean;
 }
 
 template <int BITS>
@@ -394,11 +396,11 @@ int launch_gemv(const int8_t *A, const uint8_t *B, void *out, const float *s, co
     const int lds_limit = st.lds_limit[dev];
 
     const MfmaTuning &mtu = mfma_tuning<BITS>();
-    if (mtu.engine == 7 || (mtu.engine == 0 && mtu.min_width <= 0 && wide_default(M, N, K, st.n_cus[dev]))) {
+    if (mtu.engine == 7 || (mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(M, N, K, st.n_cus[dev], lds_limit))) {
         const GemvProblem q{A, B, out, s, ws, M, N, K};
         const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % kWideVariants
-                                                           : wide_pick(M, N, K, st.n_cus[dev]);
-        const int rc = launch_wide<BITS>(v, q, out_kind, scale_kind, lds_limit, stream);
+                                                           : wide_pick<BITS>(M, N, K, st.n_cus[dev], lds_limit);
+        const int rc = v < 0 ? -1 : launch_wide<BITS>(v, q, out_kind, scale_kind, lds_limit, stream);
         if (rc != -1) return rc;
     }
     // two tokens go to the matrix cores for very long matrices and for long rows (K >= 4096: at
@@ -597,7 +599,7 @@ int launch_grouped(const GemvProblem *probs, int count, int out_kind, int scale_
         // token tiles of at most 16 (the staged activations are chunked along K: they always fit)
         const int cap = q.M < kMfmaTokens ? q.M : kMfmaTokens;
         if (q.M < min_width || !mx_problem_ok(q, out_kind == OUT_G32) ||
-            (tu.row_tiles == 0 && tu.max_wgs == 0 && wide_default(q.M, q.N, q.K, st.n_cus[dev]))) {
+            (tu.row_tiles == 0 && tu.max_wgs == 0 && wide_default<BITS>(q.M, q.N, q.K, st.n_cus[dev], lds_limit))) {
             const int rc = launch_gemv<BITS>(q.A, q.B, q.out, q.s, q.ws, q.M, q.N, q.K, out_kind,
                                              scale_kind, stream);
             if (rc != 0) return rc;

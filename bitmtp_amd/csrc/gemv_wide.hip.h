@@ -475,11 +475,24 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
     return k.fixed + groups * (busy > k.group_min ? busy : k.group_min) + k.tile * per_cu;
 }
 
-// The variant with the smallest estimate: at most 2.4 % behind the best of them over the same sweep.
-inline int wide_pick(int M, int N, int K, int n_cus) {
-    int best = 0;
-    for (int v = 1; v < kWideVariants; ++v)
-        if (wide_estimate(v, M, N, K, n_cus) < wide_estimate(best, M, N, K, n_cus)) best = v;
+// Whether variant v takes rows of K weights: all scales of its row block are staged at once, 2 bytes per row and group,
+// so that 64x128_K4 and 128x256 stop at K = 23,808, 64x256 at 32,384 and 64x128_K2 at 56,576 (160 KB of LDS), and
+// its offsets are 32-bit.
+template <int BITS>
+bool wide_fits(int v, int K, int lds_limit) {
+    const WideVariant &k = wide_kernel<BITS>(v);
+    return k.lds(K) <= (size_t)lds_limit && (long)k.rows * K <= (1L << 30) && (long)k.tokens * K <= (1L << 30);
+}
+
+// The variant with the smallest estimate among those that take rows of K weights: at most 2.4 % behind the best of
+// them over the same sweep.  -1: none does.
+template <int BITS>
+int wide_pick(int M, int N, int K, int n_cus, int lds_limit) {
+    int best = -1;
+    for (int v = 0; v < kWideVariants; ++v)
+        if (wide_fits<BITS>(v, K, lds_limit) &&
+            (best < 0 || wide_estimate(v, M, N, K, n_cus) < wide_estimate(best, M, N, K, n_cus)))
+            best = v;
     return best;
 }
 
@@ -487,15 +500,14 @@ inline int wide_pick(int M, int N, int K, int n_cus) {
 template <int BITS>
 int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream) {
     const WideVariant &k = wide_kernel<BITS>(v);
-    const size_t lds = k.lds(q.K);
-    if (lds > (size_t)lds_limit || (long)k.rows * q.K > (1L << 30) || (long)k.tokens * q.K > (1L << 30)) return -1;
+    if (!wide_fits<BITS>(v, q.K, lds_limit)) return -1;
     const int tm = (q.M + k.tokens - 1) / k.tokens, tn = (q.N + k.rows - 1) / k.rows;
     if ((long)tm * tn > (1L << 28)) return -1;
     const int per = (tm * tn + kWideXcds - 1) / kWideXcds;
     const int flags = ((q.K / kGroup) % 4 == 0 && (reinterpret_cast<uintptr_t>(q.ws) & 7) == 0 ? 1 : 0) |
                       (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0);
     const int variant = out_kind == OUT_G32 ? 2 : scale_kind;
-    hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), lds, stream, q.A, q.B, q.out,
+    hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), k.lds(q.K), stream, q.A, q.B, q.out,
                        q.s, reinterpret_cast<const uint16_t *>(q.ws), q.M, q.N, q.K, out_kind == OUT_F32 ? 1 : 0, tm,
                        tn, flags);
     note_kernel("gemv_wide_kernel", BITS, k.t[0], k.t[1], k.t[2], k.t[3], k.t[4], variant);

@@ -61,6 +61,20 @@ def test_built_in_choice(m, n, k, family, bits):
     _check(m, n, k, bits, torch.bfloat16, family)
 
 
+@pytest.mark.parametrize("bits", [2, 1])
+@pytest.mark.parametrize("m,n,k", [(600, 600, 23936), (300, 4100, 24064), (130, 1100, 32512), (70, 520, 56704), (33, 40, 65536)])
+def test_rows_too_long_for_some_tiles(m, n, k, bits):
+    """Rows whose staged scales leave no room for the tile that would be fastest take another one that fits."""
+    print(f"[case] long rows bits {bits} {m}x{n}x{k}", flush=True)
+    lib = ops.t2_lib() if bits == 2 else ops.q1_lib()
+    tune = lib.t2g128_set_mfma_tuning if bits == 2 else lib.q1g128_set_mfma_tuning
+    tune(0, 0, 0, 0, 7)   # the wide kernel, the tile its own choice
+    try:
+        _check(m, n, k, bits, torch.bfloat16, "gemv_wide_kernel<")
+    finally:
+        tune(0, 0, 0, 0, 0)
+
+
 @pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bits", [2, 1])
 @pytest.mark.parametrize("m,n,k", [(3, 16, 640), (4, 17, 768), (8, 100, 896), (9, 48, 640), (16, 333, 896), (16, 40, 1920),
