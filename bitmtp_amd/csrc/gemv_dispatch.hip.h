@@ -356,24 +356,56 @@ int launch_grouped_mx_only(const GemvProblem &q, int out_kind, int scale_kind, i
     return launch_mx<BITS>(batch, nb, out_kind, scale_kind, lds_limit, n_cus, stream);
 }
 
-// K for which the lean kernel stands in for the matrix-core kernels that want whole 512-wide tiles and for
-// the dot4 kernel they leave (12288 x 1920 at nine tokens: dot4 9.2 us).
-inline bool lean_any_k(int K) { return K % 512 != 0 && K > 512; }
+// ---- what a block goes to without the wide kernel ---------------------------------------------
+enum class Narrow { lean, matrix_core, dot4 };
 
-// Blocks the wide kernel takes: where it is expected to be faster than the lean kernel's 16-token tiles, whose
-// time is a fit to the same sweep as wide_estimate (12288 x 2048: 6.3 / 6.4 us at 17 tokens, 8.0 / 6.6 at 32;
-// 2048 x 2048: 4.7 / 6.3 at 64, 6.5 / 6.5 at 128; 2560 x 9728: 12.5 / 14.3 at 64, 16.6 / 15 at 96).  What the
-// lean kernel does not take leaves only the dot4 kernel where K is not a multiple of 512 (19000 x 2688: dot4
-// 9.1 us at four tokens, 15.5 at nine, against 10.6 at any width up to 32).
+inline long lean_tiles(int M, int N) { return (long)((M + kMfmaTokens - 1) / kMfmaTokens) * ((N + 15) / 16); }
+
+// Lean kernel: one descriptor per tile of up to 16 tokens, as long as its grid stays within eight workgroups per
+// CU.  Measured against the operand-loading and the staged kernel at widths 3-16: 8-15 % faster on the
+// K = 2048 / 2560 decode shapes of the 1.7B- and 4B-shaped models, 15-25 % on 12288 x 4096, 9728 x 9728,
+// 24576 x 4096 and 27648 x 5120, level on 4096 x 12288 (where the twelve-wave form of the same kernel runs).
+//   K not a multiple of 512: its ragged build, for as many token tiles as a table holds; the other matrix-core
+//     kernels want whole 512-wide tiles (12288 x 1920 at nine tokens: dot4 9.2 us, ragged 4.3)
+//   K = 512, 1024, 1536: some of its four waves have no K slice, so that its lead over the matrix-core kernels ends
+//     at 1 + K / 512 workgroups per CU and four token tiles (9728 x 1536 at 16 tokens 5.9 / 4.1 us, 4096 x 512 at
+//     48 3.5 / 3.8, 12288 x 1024 at 17 5.0 / 5.3, 1000 x 512 at 128 3.5 / 3.8)
+//   longer: up to 24 token tiles, from the thirteenth on as launches of the striding form
 template <int BITS>
-bool wide_default(int M, int N, int K, int n_cus, int lds_limit) {
-    const long lean_tiles = (long)((M + kMfmaTokens - 1) / kMfmaTokens) * ((N + 15) / 16);
-    if (K % 512 != 0 && (lean_tiles > 8L * n_cus || N > kLongMatrixRows || K < 512)) return M >= kWideMinRagged;
-    if (M <= kMfmaTokens) return false;
-    const double G = K / kGroup;
-    const double lean = 3.1 + G * (0.0087 + 0.051 * lean_tiles / n_cus);
-    const int v = wide_pick<BITS>(M, N, K, n_cus, lds_limit);
-    return v >= 0 && wide_estimate(v, M, N, K, n_cus) < lean;
+bool lean_takes(const GemvProblem &q, bool g32, int n_cus) {
+    const long tiles = lean_tiles(q.M, q.N);
+    if (q.N > kLongMatrixRows || tiles > 8L * n_cus || q.K < 512) return false;
+    if (q.K % 512 != 0) return q.M <= kMxlMaxDesc * kMfmaTokens;
+    if (q.K < 2048)
+        return q.M <= 4 * kMfmaTokens && tiles * 512 <= (512L + q.K) * n_cus &&
+               mfma_shape_ok(q.B, g32 ? nullptr : q.ws, q.K);
+    return q.M <= kMxMaxDesc * kMfmaTokens && mx_problem_ok(q, g32);
+}
+
+template <int BITS>
+Narrow narrow_kernel(const GemvProblem &q, bool g32, int n_cus) {
+    if (lean_takes<BITS>(q, g32, n_cus)) return Narrow::lean;
+    return mfma_shape_ok(q.B, g32 ? nullptr : q.ws, q.K) ? Narrow::matrix_core : Narrow::dot4;
+}
+
+// Blocks the wide kernel takes: where it is expected to be faster than what would run otherwise.  The lean kernel's
+// time is a fit to the same sweep as wide_estimate (12288 x 2048: 6.3 / 6.4 us at 17 tokens, 8.0 / 6.6 at 32;
+// 2048 x 2048: 4.7 / 6.3 at 64, 6.5 / 6.5 at 128; 2560 x 9728: 12.5 / 14.3 at 64, 16.6 / 15 at 96), the matrix-core
+// kernels' are fits to 17 ... 1024 tokens of K = 512, 1024 and 1536 by 1000 ... 32000 rows (6-7 % rms).  The dot4
+// kernel has no estimate: from five tokens on it is behind (19000 x 2688: dot4 9.1 us at four tokens, 15.5 at nine,
+// against 10.6 at any width up to 32; 1086 x 1152 at 245 tokens 24.5 against 5.6).
+template <int BITS>
+bool wide_default(const GemvProblem &q, bool g32, int n_cus, int lds_limit) {
+    if (q.M <= kMfmaTokens && q.K % 512 == 0) return false;
+    const Narrow other = narrow_kernel<BITS>(q, g32, n_cus);
+    if (other == Narrow::dot4) return q.M >= kWideMinRagged;
+    if (q.M <= kMfmaTokens) return false;
+    const double G = q.K / kGroup, per_cu = (double)lean_tiles(q.M, q.N) / n_cus;
+    const double narrow = other == Narrow::lean       ? 3.1 + G * (0.0087 + 0.051 * per_cu)
+                          : q.N <= kDirectMaxRows     ? 2.8 + G * 0.07 * per_cu
+                                                      : 2.6 + 0.08 * per_cu + G * (0.086 + 0.025 * per_cu);
+    const int v = wide_pick<BITS>(q.M, q.N, q.K, n_cus, lds_limit);
+    return v >= 0 && wide_estimate(v, q.M, q.N, q.K, n_cus) < narrow;
 }
 
 template <int BITS>
@@ -396,8 +428,9 @@ int launch_gemv(const int8_t *A, const uint8_t *B, void *out, const float *s, co
     const int lds_limit = st.lds_limit[dev];
 
     const MfmaTuning &mtu = mfma_tuning<BITS>();
-    if (mtu.engine == 7 || (mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(M, N, K, st.n_cus[dev], lds_limit))) {
-        const GemvProblem q{A, B, out, s, ws, M, N, K};
+    const GemvProblem q{A, B, out, s, ws, M, N, K};
+    const bool g32 = out_kind == OUT_G32;
+    if (mtu.engine == 7 || (mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(q, g32, st.n_cus[dev], lds_limit))) {
         const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % kWideVariants
                                                            : wide_pick<BITS>(M, N, K, st.n_cus[dev], lds_limit);
         const int rc = v < 0 ? -1 : launch_wide<BITS>(v, q, out_kind, scale_kind, lds_limit, stream);
@@ -411,7 +444,6 @@ int launch_gemv(const int8_t *A, const uint8_t *B, void *out, const float *s, co
     if constexpr (BITS == 2) {
         if (mtu.engine == 6 || mtu.engine == 0) {
             // one token against a very long matrix: activations in registers, v_dot8
-            const GemvProblem q{A, B, out, s, ws, M, N, K};
             if (rowreg_problem_ok(q, out_kind, mtu.engine == 6))
                 return launch_rowreg(q, out_kind, scale_kind, st.n_cus[dev],
                                      mxs_tuning<BITS>().wgs_per_cu, stream);
@@ -419,29 +451,15 @@ int launch_gemv(const int8_t *A, const uint8_t *B, void *out, const float *s, co
     }
     if (mtu.engine == 5 || mtu.engine == 0) {
         // very long matrices: the streaming kernel, at every width up to 16
-        const GemvProblem q{A, B, out, s, ws, M, N, K};
         if (mxs_problem_ok<BITS>(q, out_kind, lds_limit, st.n_cus[dev], mtu.engine == 5))
             return launch_mxs<BITS>(q, out_kind, scale_kind, lds_limit, st.n_cus[dev], stream);
     }
-    // Layer-sized matrices at three or more tokens: the lean grouped kernel with one descriptor per
-    // tile of up to 16 tokens, as long as its grid stays within eight workgroups per CU.  Measured
-    // against the operand-loading and the staged kernel at widths 3-16: 8-15 % faster on the
-    // K = 2048 / 2560 decode shapes of the 1.7B- and 4B-shaped models, 15-25 % on 12288 x 4096,
-    // 9728 x 9728, 24576 x 4096 and 27648 x 5120, level on 4096 x 12288 (where the twelve-wave
-    // form of the same kernel already ran).
-    const long lean_tiles = (long)((M + kMfmaTokens - 1) / kMfmaTokens) * ((N + 15) / 16);
-    const bool lean_default = mtu.engine == 0 && M >= min_width && N <= kLongMatrixRows &&
-                              lean_tiles <= 8L * st.n_cus[dev];
-    if ((mtu.engine == 4 || lean_default) && M >= min_width) {
-        // the grouped kernel with a single descriptor
-        const GemvProblem q{A, B, out, s, ws, M, N, K};
-        if (mx_problem_ok(q, out_kind == OUT_G32) || (lean_default && lean_any_k(K))) {
-            const int rc = launch_grouped_mx_only<BITS>(q, out_kind, scale_kind, lds_limit, st.n_cus[dev],
-                                                        stream);
-            if (rc >= 0) return rc;
-        }
+    // layer-sized matrices at three or more tokens: the lean grouped kernel (engine 4: the grouped kernels, forced)
+    if (M >= min_width && (mtu.engine == 4 ? mx_problem_ok(q, g32) : mtu.engine == 0 && lean_takes<BITS>(q, g32, st.n_cus[dev]))) {
+        const int rc = launch_grouped_mx_only<BITS>(q, out_kind, scale_kind, lds_limit, st.n_cus[dev], stream);
+        if (rc >= 0) return rc;
     }
-    if (M >= min_width && mfma_shape_ok(B, out_kind == OUT_G32 ? nullptr : ws, K)) {
+    if (M >= min_width && mfma_shape_ok(B, g32 ? nullptr : ws, K)) {
         int rc = -1;
         // operand-loaded activations win up to about 16k rows, staged ones above (measured)
         const int engine = mtu.engine != 0 ? mtu.engine : (N <= kDirectMaxRows ? 3 : 1);
@@ -599,7 +617,7 @@ int launch_grouped(const GemvProblem *probs, int count, int out_kind, int scale_
         // token tiles of at most 16 (the staged activations are chunked along K: they always fit)
         const int cap = q.M < kMfmaTokens ? q.M : kMfmaTokens;
         if (q.M < min_width || !mx_problem_ok(q, out_kind == OUT_G32) ||
-            (tu.row_tiles == 0 && tu.max_wgs == 0 && wide_default<BITS>(q.M, q.N, q.K, st.n_cus[dev], lds_limit))) {
+            (tu.row_tiles == 0 && tu.max_wgs == 0 && wide_default<BITS>(q, out_kind == OUT_G32, st.n_cus[dev], lds_limit))) {
             const int rc = launch_gemv<BITS>(q.A, q.B, q.out, q.s, q.ws, q.M, q.N, q.K, out_kind,
                                              scale_kind, stream);
             if (rc != 0) return rc;

@@ -62,6 +62,18 @@ def test_built_in_choice(m, n, k, family, bits):
 
 
 @pytest.mark.parametrize("bits", [2, 1])
+@pytest.mark.parametrize("m,n,k,family", [
+    (192, 1086, 1152, "gemv_mxl_ragged_kernel<"), (193, 1086, 1152, "gemv_wide_kernel<"),   # a table holds twelve token tiles
+    (16, 2048, 512, "gemv_mxl_kernel<"), (33, 4096, 512, "gemv_mfma_direct_kernel<"), (64, 1000, 1024, "gemv_mxl_kernel<"),
+    (65, 1000, 1024, "gemv_mfma_direct_kernel<"), (16, 12000, 1536, "gemv_mxl_kernel<"), (17, 20000, 1536, "gemv_mfma_kernel<"),
+    (80, 12288, 1024, "gemv_wide_kernel<")])
+def test_built_in_choice_is_among_kernels_that_run(m, n, k, family, bits):
+    """Where the lean kernel does not take the rows, the choice is between the wide kernel and what does."""
+    print(f"[case] choice bits {bits} {m}x{n}x{k}", flush=True)
+    _check(m, n, k, bits, torch.bfloat16, family)
+
+
+@pytest.mark.parametrize("bits", [2, 1])
 @pytest.mark.parametrize("m,n,k", [(600, 600, 23936), (300, 4100, 24064), (130, 1100, 32512), (70, 520, 56704), (33, 40, 65536)])
 def test_rows_too_long_for_some_tiles(m, n, k, bits):
     """Rows whose staged scales leave no room for the tile that would be fastest take another one that fits."""
