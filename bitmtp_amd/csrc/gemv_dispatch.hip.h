@@ -533,6 +533,44 @@ int launch_gemv_fused(const FusedGemv &d, hipStream_t stream) {
     return launch_gemv_dot4_fused<BITS>(d, lds_limit, n_cus, stream);
 }
 
+// Which problems of a grouped call leave the shared launches for one of their own (leaves[i]): blocks of more than
+// 16 tokens that the wide kernel serves in less than they add to the shared launch, and all of them where the wide
+// launches together take less than a shared launch for the rest.  What a problem adds is its row tiles times its
+// scale groups; a launch's fixed part is paid by whatever stays.  Fitted to the seven projections of a 1.7B- and a
+// 4B-shaped layer at 17 widths from 17 to 256 tokens, both formats, each with none, all and five other subsets of
+// them leaving: at most 9 % behind the best of these, 0.7 % in the mean.  (Against each problem's own launch, which
+// has a fixed part of its own, two large projections left much too early: 4B-shaped 17 tokens 27.0 -> 18.0 us, 32
+// tokens 30.9 -> 26.3, 1.7B-shaped 48 tokens 23.4 -> 19.5; level from 56 tokens on.)
+constexpr int kGroupedMax = 64;                                  // problems per call
+constexpr double kSharedLaunch = 2.5, kSharedGroupTile = 0.065;  // microseconds; the latter per CU
+
+template <int BITS>
+void grouped_leavers(const GemvProblem *probs, int count, int min_width, bool g32, int n_cus, int lds_limit, bool *leaves) {
+    double shared = 0.0, wide = 0.0;
+    int descs = 0;
+    bool others = false;  // a problem that stays whatever the wide kernel costs
+    for (int i = 0; i < count; ++i) {
+        const GemvProblem &q = probs[i];
+        leaves[i] = false;
+        if (q.M < min_width || !mx_problem_ok(q, g32)) continue;  // (never in a shared launch)
+        const int v = q.M > kMfmaTokens ? wide_pick<BITS>(q.M, q.N, q.K, n_cus, lds_limit) : -1;
+        if (v < 0) {
+            others = others || q.M > kDot4GroupMaxWidth;
+            continue;
+        }
+        const double adds = kSharedGroupTile * (q.K / kGroup) * lean_tiles(q.M, q.N) / n_cus;
+        const double alone = wide_estimate(v, q.M, q.N, q.K, n_cus);
+        leaves[i] = alone < adds;
+        if (leaves[i]) continue;
+        shared += adds;
+        wide += alone;
+        descs += (q.M + kMfmaTokens - 1) / kMfmaTokens;
+    }
+    if (others || wide >= shared + kSharedLaunch * ((descs + kMxMaxDesc - 1) / kMxMaxDesc)) return;
+    for (int i = 0; i < count; ++i)
+        leaves[i] = leaves[i] || (probs[i].M > kMfmaTokens && probs[i].M >= min_width && mx_problem_ok(probs[i], g32));
+}
+
 // Several GEMVs in one call (descriptors in host memory, read before the call returns).
 // Problems the grouped kernel takes (K % 512 == 0, aligned operands) share launches of up to
 // kMxMaxDesc descriptors each, blocks wider than 16 tokens as several token tiles; the rest
@@ -542,7 +580,7 @@ int launch_gemv_fused(const FusedGemv &d, hipStream_t stream) {
 template <int BITS>
 int launch_grouped(const GemvProblem *probs, int count, int out_kind, int scale_kind,
                    hipStream_t stream) {
-    if (probs == nullptr || count < 1) return 1;
+    if (probs == nullptr || count < 1 || count > kGroupedMax) return 1;
     if (out_kind < 0 || out_kind > 2 || scale_kind < 0 || scale_kind > 1) return 1;
     for (int i = 0; i < count; ++i) {
         const GemvProblem &q = probs[i];
@@ -604,6 +642,10 @@ int launch_grouped(const GemvProblem *probs, int count, int out_kind, int scale_
         return rc;
     };
     const size_t out_elt = out_kind == OUT_BF16 ? 2 : 4;
+    const bool g32 = out_kind == OUT_G32;
+    bool leaves[kGroupedMax] = {};
+    if (tu.row_tiles == 0 && tu.max_wgs == 0)
+        grouped_leavers<BITS>(probs, count, min_width, g32, st.n_cus[dev], lds_limit, leaves);
     for (int i = 0; i < count; ++i) {
         const GemvProblem &q = probs[i];
         if (narrow_on && q.M <= kDot4GroupMaxWidth) {
@@ -616,8 +658,7 @@ int launch_grouped(const GemvProblem *probs, int count, int out_kind, int scale_
         }
         // token tiles of at most 16 (the staged activations are chunked along K: they always fit)
         const int cap = q.M < kMfmaTokens ? q.M : kMfmaTokens;
-        if (q.M < min_width || !mx_problem_ok(q, out_kind == OUT_G32) ||
-            (tu.row_tiles == 0 && tu.max_wgs == 0 && wide_default<BITS>(q, out_kind == OUT_G32, st.n_cus[dev], lds_limit))) {
+        if (q.M < min_width || !mx_problem_ok(q, g32) || leaves[i]) {
             const int rc = launch_gemv<BITS>(q.A, q.B, q.out, q.s, q.ws, q.M, q.N, q.K, out_kind,
                                              scale_kind, stream);
             if (rc != 0) return rc;

@@ -103,6 +103,7 @@ void q1g128_set_mfma_tuning(int min_width, int row_tiles, int k_split, int passe
 int q1g128_gemv_grouped(const bonsai_gemv_desc *descs, int count, int out_kind, int scale_kind,
                         void *stream) {
     if (descs == nullptr || count < 1 || count > BONSAI_GROUPED_MAX) return BONSAI_ERR_ARG;
+    static_assert(BONSAI_GROUPED_MAX == kGroupedMax, "one limit");
     GemvProblem probs[BONSAI_GROUPED_MAX];
     for (int i = 0; i < count; ++i)
         probs[i] = GemvProblem{descs[i].A, descs[i].B, descs[i].out, descs[i].s, descs[i].ws,

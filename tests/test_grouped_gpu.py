@@ -57,6 +57,29 @@ def test_t2_17b_layer_in_one_call(oracle, M):
     check_group(oracle, probs, 2, f"1.7B layer M={M}")
 
 
+@pytest.mark.parametrize("bits", [2, 1])
+@pytest.mark.parametrize("layer,M,launches", [(LAYER_4B, 17, 1), (LAYER_4B, 32, 1), (LAYER_17B, 48, 1), (LAYER_17B, 64, 3),
+                                              (LAYER_4B, 192, 6), (LAYER_17B, 256, 7)])
+def test_wide_blocks_share_a_launch_while_that_is_faster(layer, M, launches, bits):
+    """Which problems of a call leave the shared launches is decided over all of them; the sums are those of single calls."""
+    import bitmtp_amd as ops
+    print(f"[case] grouped wide bits={bits} M={M} {layer}", flush=True)
+    gen = torch.Generator(device="cuda:0").manual_seed(M)
+    rnd = lambda lo, hi, *s: torch.randint(lo, hi, s, generator=gen, device="cuda:0", dtype=torch.int8)
+    probs = [(rnd(-128, 128, M, k), rnd(-128, 128, n, k * bits // 8), torch.rand(M, 1, generator=gen, device="cuda:0") * 40 + 1,
+              torch.rand(n, k // 128, generator=gen, device="cuda:0").to(torch.bfloat16)) for n, k in layer]
+    ops.init_kernels()
+    n0 = ops.launch_count(bits)
+    y = ops.packed_gemv_grouped(probs, bits=bits, out_kind=ops.OUT_F32)
+    assert ops.launch_count(bits) - n0 == launches
+    G = ops.packed_gemv_grouped([(a, b, None, None) for a, b, _, _ in probs], bits=bits, out_kind=ops.OUT_G32)
+    for (a, b, s, ws), g, v in zip(probs, G, y):
+        assert torch.equal(g, ops.packed_gemv_ex(a, b, None, None, bits=bits, out_kind=ops.OUT_G32))
+        terms = g.double() * ws.double() / s.double().unsqueeze(-1)
+        # fp32 sums of at most 76 terms in some order
+        assert ((v.double() - terms.sum(-1)).abs() <= 1e-6 * terms.abs().sum(-1) + 1e-30).all()
+
+
 @pytest.mark.parametrize("M", [1, 8, 16])
 def test_t2_4b_layer_in_one_call(oracle, M):
     """The 4B-shaped layer: K in {2560, 4096, 9728} (5, 8 and 19 K tiles over four waves)."""
