@@ -290,10 +290,13 @@ gemv_mxl_kernel(int e0, int e1, int e2, int e3, int e4, int e5, int e6, int e7, 
 }
 
 // A launch of one matrix: no descriptor to wait for, what the first loads need arrives in registers with the wave.
-template <int BITS, int MR, bool SF16, int W, int NB, int OCC>
+// (FORM tells it from the table form by name: false / true there, 2 here)
+constexpr int kMxlOne = 2;
+template <int BITS, int MR, bool SF16, int W, int NB, int OCC, int FORM>
 __global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
 gemv_mxl_kernel(const int8_t *A, const uint8_t *B, const uint16_t *ws, const float *s, void *out, int N, int K,
                     int M, int out_f32) {
+    static_assert(FORM == kMxlOne, "scaled results only");
     gemv_mxl_body<BITS, MR, SF16, W, NB, false, false>(MxlDesc{A, B, out, s, ws, M, N, K, 0, {0, 0}}, out_f32, M);
 }
 
@@ -330,8 +333,8 @@ MxlKernels mxl_kernel_n(int scale_kind, bool ragged) {
                 nullptr};
     }
     if (scale_kind == 2) return {gemv_mxl_kernel<BITS, MR, false, W, NB, OCC, true>, nullptr};  // int32 group sums from the same builds
-    if (scale_kind == 1) return {gemv_mxl_kernel<BITS, MR, true, W, NB, OCC>, gemv_mxl_kernel<BITS, MR, true, W, NB, OCC>};
-    return {gemv_mxl_kernel<BITS, MR, false, W, NB, OCC>, gemv_mxl_kernel<BITS, MR, false, W, NB, OCC>};
+    if (scale_kind == 1) return {gemv_mxl_kernel<BITS, MR, true, W, NB, OCC>, gemv_mxl_kernel<BITS, MR, true, W, NB, OCC, kMxlOne>};
+    return {gemv_mxl_kernel<BITS, MR, false, W, NB, OCC>, gemv_mxl_kernel<BITS, MR, false, W, NB, OCC, kMxlOne>};
 }
 template <int BITS, int W, int OCC1, int OCC2>
 MxlKernels mxl_kernel_w(int scale_kind, int width_class, bool ragged) {
@@ -438,9 +441,9 @@ int launch_mxl(const GemvProblem *probs, int count, int out_kind, int scale_kind
                            ends[4], ends[5], ends[6], ends[7], ends[8], ends[9], ends[10], ends[11],
                            out_kind == OUT_F32 ? 1 : 0, mmax, tbl);
     }
-    // <BITS, MR, SF16, W, NB, OCC, G32> as instantiated by mxl_kernel
+    // <BITS, MR, SF16, W, NB, OCC, G32 / FORM> as instantiated by mxl_kernel
     note_kernel(ragged ? "gemv_mxl_ragged_kernel" : "gemv_mxl_kernel", BITS, width_class == 0 ? 1 : 4, scale_kind == 1 && variant != 2, waves,
-                width_class == 2 ? 2 : 1, wide ? 3 : (width_class == 2 && !dense ? 4 : 5), variant == 2);
+                width_class == 2 ? 2 : 1, wide ? 3 : (width_class == 2 && !dense ? 4 : 5), one ? kMxlOne : variant == 2);
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

@@ -299,11 +299,13 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                 for (int t = 0; t < 4; ++t) dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[t], vb[j][t], dd, 0, 0, 0);
                 if (G32) {
                     const int n = (wn * NT + j) * 32 + op_row;
+                    int stride = N;
+                    asm volatile("" : "+s"(stride));  // addresses made here: 16 of them held over the loop would spill
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int m = (wm * MT + i) * 32 + 8 * (r / 4) + 4 * kb + r % 4;
                         if (m < mv && n < nv)
-                            reinterpret_cast<int32_t *>(out)[((size_t)(m0 + m) * N + n0 + n) * G + g] = (dd[r] - kBias) >> 6;
+                            reinterpret_cast<int32_t *>(out)[((size_t)(m0 + m) * stride + n0 + n) * G + g] = (dd[r] - kBias) >> 6;
                     }
                     continue;
                 }

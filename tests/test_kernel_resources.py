@@ -27,8 +27,9 @@ def _resource_report(source: str) -> dict:
     for line in demangle.splitlines():
         m = re.search(r"Function Name: (.*?) \[-Rpass", line)
         if m:
-            cur = re.sub(r"^void ", "", m.group(1))
+            cur = re.sub(r"^void ", "", m.group(1)).replace("(anonymous namespace)::", "")
             cur = re.sub(r"\(.*$", "", cur)          # drop the argument list
+            assert cur not in report, f"two kernels called {cur}"
             report[cur] = {}
             continue
         for key, tag in (("VGPRs", "vgprs"), (r"ScratchSize \[bytes/lane\]", "scratch"),
@@ -56,15 +57,26 @@ def test_default_kernels_do_not_spill(reports, bits):
     rep = reports[bits]
     hot = {}
     hot.update(_select(rep, r"gemv_mxl_kernel<"))                      # lean matrix-core kernel, every build
+    hot.update(_select(rep, r"gemv_mxl_ragged_kernel<"))               # rows of any length
+    hot.update(_select(rep, r"gemv_wide_kernel<"))                     # wide blocks, every tile and output kind
     hot.update(_select(rep, r"gemv_mxs_kernel<"))                      # streaming kernel
     hot.update(_select(rep, r"gemv_rowreg_kernel<"))                   # single-token head kernel (T2 only)
     hot.update(_select(rep, rf"gemv_dot4_grouped_kernel<{bits}, 1, "))  # grouped dot4, one token
     hot.update(_select(rep, rf"gemv_dot4_grouped_kernel<{bits}, 2, [12],"))
     hot.update(_select(rep, rf"gemv_dot4_kernel<{bits}, 1, \d, false"))  # single GEMV, one token
     hot.update(_select(rep, rf"gemv_dot4_kernel<{bits}, 2, [12], false"))
+    assert len(_select(hot, r"gemv_mxl_kernel<.*, 2>$")) == 14 and len(_select(hot, "gemv_wide")) == 18
     assert len(hot) >= 20
     spilled = {k: v["scratch"] for k, v in hot.items() if v["scratch"] != 0}
     assert not spilled, f"kernels with scratch memory: {spilled}"
+
+
+def test_prompt_kernels_do_not_spill():
+    rep = _select(_resource_report("decode_ops.hip"), "prefill_")
+    assert sorted(k.split("::")[-1] for k in rep) == ["prefill_attn_kernel", "prefill_attn_split_kernel", "prefill_rope_kernel"]
+    for name, v in rep.items():
+        assert v["scratch"] == 0, (name, v)
+        assert "split" in name or v["occupancy"] >= 2, (name, v)   # two workgroups of the 128-pair kernel share a CU
 
 
 @pytest.mark.parametrize("bits", [2, 1])
