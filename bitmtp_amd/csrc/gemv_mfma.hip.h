@@ -137,6 +137,7 @@ __global__ void __launch_bounds__(kMfmaThreads) gemv_mfma_kernel
         }
     };
     auto park_tile = [&](const TileRegs &tr) {
+        bonsai_wave::order_lds();  // the tile before is no longer read
 #pragma unroll
         for (int rt = 0; rt < R; ++rt)
 #pragma unroll
@@ -147,6 +148,7 @@ __global__ void __launch_bounds__(kMfmaThreads) gemv_mfma_kernel
                 d2[0] = make_uint2(tr.w[rt][h].x, tr.w[rt][h].y);
                 d2[1] = make_uint2(tr.w[rt][h].z, tr.w[rt][h].w);
             }
+        bonsai_wave::order_lds();
     };
 
     TileRegs cur;
@@ -413,6 +415,7 @@ gemv_mfma_direct_kernel
         }
     };
     auto park_tile = [&](const TileRegs &tr) {
+        bonsai_wave::order_lds();  // the tile before is no longer read
 #pragma unroll
         for (int rt = 0; rt < R; ++rt)
 #pragma unroll
@@ -423,6 +426,7 @@ gemv_mfma_direct_kernel
                 d2[0] = make_uint2(tr.w[rt][h].x, tr.w[rt][h].y);
                 d2[1] = make_uint2(tr.w[rt][h].z, tr.w[rt][h].w);
             }
+        bonsai_wave::order_lds();
     };
 
     TileRegs cur;

@@ -163,6 +163,7 @@ gemv_mx_kernel(const MxParams p) {
         }
     };
     auto park_tile = [&](const TileRegs &tr) {
+        bonsai_wave::order_lds();  // the tile before is no longer read
 #pragma unroll
         for (int rt = 0; rt < R; ++rt)
 #pragma unroll
@@ -173,6 +174,7 @@ gemv_mx_kernel(const MxParams p) {
                 d2[0] = make_uint2(tr.w[rt][h].x, tr.w[rt][h].y);
                 d2[1] = make_uint2(tr.w[rt][h].z, tr.w[rt][h].w);
             }
+        bonsai_wave::order_lds();
     };
 
     // ---- staging of one K tile of activations by one wave: 4x4 byte transposes into operand

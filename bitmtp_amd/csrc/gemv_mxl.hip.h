@@ -192,6 +192,7 @@ __device__ __forceinline__ void gemv_mxl_body(const MxlDesc &d, int out_f32, int
     const unsigned char *wsrc = wt + op_row * MF::kPitch;
 
     for (int kt = tb; kt < te; ++kt) {
+        bonsai_wave::order_lds();  // the tile before is no longer read
         act_store(acur, 0);
         if (NB > 1 && nbatch > 1) act_store(amore, 1);
 #pragma unroll
@@ -200,6 +201,7 @@ __device__ __forceinline__ void gemv_mxl_body(const MxlDesc &d, int out_f32, int
             d2[0] = make_uint2(w[h].x, w[h].y);
             d2[1] = make_uint2(w[h].z, w[h].w);
         }
+        bonsai_wave::order_lds();
         const int left = G - kt * kMxTileGroups;  // groups of this tile that exist (four or more: all)
         uint2 sc = scr;
         if (RAGGED) {

@@ -114,6 +114,7 @@ gemv_mxs_kernel(const MxsParams p) {
         if (!G32) tr.sc = *reinterpret_cast<const uint2 *>(bs + (last ? voff_sc_last : voff_sc));
     };
     auto park_tile = [&](const TileRegs &tr) {
+        bonsai_wave::order_lds();  // the tile before is no longer read
 #pragma unroll
         for (int h = 0; h < MF::kLoads; ++h) {
             unsigned char *dst = wt + (h * MF::kRowsPerLoad + ld_row) * MF::kPitch + ld_col * 16;
@@ -121,6 +122,7 @@ gemv_mxs_kernel(const MxsParams p) {
             d2[0] = make_uint2(tr.w[h].x, tr.w[h].y);
             d2[1] = make_uint2(tr.w[h].z, tr.w[h].w);
         }
+        bonsai_wave::order_lds();
     };
 
     // ---- activation staging, as in gemv_mx.hip.h, but once: wave w stages K tiles w, w + 4, ...

@@ -247,7 +247,9 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
         const int g = gb + it;
         const int buf = S::kPrivate ? 0 : (it & 1);
         if (S::kPrivate) {
+            bonsai_wave::order_lds();  // group g - 1 is no longer read
             if (g < ge) park(ars[R], brs[R], 0);
+            bonsai_wave::order_lds();
             if (g + S::kAhead < ge) load(ars[R], brs[R], g + S::kAhead);
         } else {
             if (it > 0) wide_barrier();  // group g is parked; group g - 1 is no longer read

@@ -30,6 +30,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "wave_reduce.h"
+
 namespace bonsai_prefill {
 
 constexpr int kHead = 128;
@@ -290,10 +292,12 @@ prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint
     Softmax x;
     if (wave < rows.chunks) load(wave);
     for (int c = wave; c < rows.chunks; c += kWaves) {
+        bonsai_wave::order_lds();  // the chunk before is no longer read
 #pragma unroll
         for (int i = 0; i < 16; ++i) *reinterpret_cast<u32v4 *>(kb + (k_slot + 4 * i) * kKPitch + k_col * 16) = kr[i];
 #pragma unroll
         for (int i = 0; i < 4; ++i) park_v(vb, vr[i], v_dim + 32 * i, v_slot);
+        bonsai_wave::order_lds();
         if (c + kWaves < rows.chunks) load(c + kWaves);
         attend(kb, vb, p, c, rows.masked_from, col, h, scale_log2e, x);
     }

@@ -14,6 +14,13 @@
 
 namespace bonsai_wave {
 
+// Between LDS stores of one lane and loads of them by another lane of the same wave, and before the stores of the
+// next round: a wave's LDS accesses are carried out in program order, so this emits nothing, but program order is
+// what the compiler must keep, and for a single lane the two touch different addresses.
+__device__ __forceinline__ void order_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 constexpr int kXor1 = 0xB1;         // quad_perm [1,0,3,2]
 constexpr int kXor2 = 0x4E;         // quad_perm [2,3,0,1]
 constexpr int kHalfMirror = 0x141;  // lane i <-> 7-i inside each 8 lanes
