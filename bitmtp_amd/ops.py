@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import warnings
 from typing import List, Optional, Sequence, Tuple
 
 import torch
@@ -201,8 +202,10 @@ def load_torch_ops():
 # checks, allocates and launches without Python in between (an operator call is a few
 # microseconds of GPU work; the checked ctypes path costs 11 us of host time).  It declines
 # anything but the plain case, and the checked path then decides and words the error.  It is
-# loaded by the first call that path has accepted, so a refused call still loads nothing.
+# loaded by the first call that path has accepted, so a refused call still loads nothing; where it
+# is not built, or not for this PyTorch, the checked path serves every call.
 _native = None
+_native_missing = False
 
 
 def py_ops_lib_path() -> str:
@@ -222,8 +225,21 @@ def _load_native() -> None:
     _native = module
 
 
+def _offer_native() -> None:
+    """Loads the extension for the calls after this one, if it can be: the operators only lose
+    their short host path without it (said once), the launches below it are the same."""
+    global _native_missing
+    if _native is not None or _native_missing:
+        return
+    try:
+        _load_native()
+    except (RuntimeError, ImportError) as e:
+        _native_missing = True
+        warnings.warn(f"operator calls take the slower host path: {e}", RuntimeWarning, stacklevel=3)
+
+
 def native():
-    """The extension module (csrc/py_ops.cpp)."""
+    """The extension module (csrc/py_ops.cpp); raises where it is missing."""
     if _native is None:
         _load_native()
     return _native
@@ -343,13 +359,12 @@ def t2g128_int8xint2_linear(a_int8: torch.Tensor, b_packed: torch.Tensor, s: tor
     out = torch.empty(*out_shape, dtype=torch.bfloat16, device=a_int8.device)
     # the checked form of the same entry point: the drop-in symbol returns nothing, and a
     # refused launch would hand back the uninitialised tensor
+    _offer_native()
     with torch.cuda.device(a_int8.device):
         rc = lib.t2g128_gemv_ex(_ptr(a_int8), _ptr(b_packed), _ptr(out), _ptr(s), _ptr(ws),
                                 m, n, k, OUT_BF16, SCALE_BF16, _stream(a_int8.device))
     if rc != 0:
         raise RuntimeError(f"t2g128: native launch failed with status {rc} (M={m}, N={n}, K={k})")
-    if _native is None:
-        _load_native()
     return out
 
 
@@ -367,13 +382,12 @@ def q1g128_int8xint1_linear(a_int8: torch.Tensor, b_packed: torch.Tensor, s: tor
     m, out_shape = _out_shape(a_int8, n, "q1g128")
     lib = q1_lib()
     out = torch.empty(*out_shape, dtype=torch.bfloat16, device=a_int8.device)
+    _offer_native()
     with torch.cuda.device(a_int8.device):
         rc = lib.q1g128_gemv_ex(_ptr(a_int8), _ptr(b_packed), _ptr(out), _ptr(s), _ptr(ws),
                                 m, n, k, OUT_BF16, SCALE_BF16, _stream(a_int8.device))
     if rc != 0:
         raise RuntimeError(f"q1: native launch failed with status {rc} (M={m}, N={n}, K={k})")
-    if _native is None:
-        _load_native()
     return out
 
 
@@ -448,13 +462,12 @@ def packed_gemv_ex(a_int8: torch.Tensor, b_packed: torch.Tensor, s: Optional[tor
         raise RuntimeError(f"{kind}: out must be a contiguous {dtype} tensor of shape {shape} on {dev}")
     scale_kind = SCALE_F16 if (ws is not None and ws.dtype == torch.float16) else SCALE_BF16
     fn = t2_lib().t2g128_gemv_ex if bits == 2 else q1_lib().q1g128_gemv_ex
+    _offer_native()
     with torch.cuda.device(dev):
         rc = fn(_ptr(a_int8), _ptr(b_packed), _ptr(out), _ptr(s), _ptr(ws), m, n, k, out_kind,
                 scale_kind, _stream(dev))
     if rc != 0:
         raise RuntimeError(f"{kind}: native launch failed with status {rc} (M={m}, N={n}, K={k})")
-    if _native is None:
-        _load_native()
     return out
 
 
@@ -632,12 +645,11 @@ def packed_gemv_grouped(problems: Sequence[Tuple[torch.Tensor, torch.Tensor, Opt
         raise RuntimeError(f"{kind}: the scales of a grouped call must share one dtype")
     scale_kind = scale_kinds.pop() if scale_kinds else SCALE_BF16
     fn = t2_lib().t2g128_gemv_grouped if bits == 2 else q1_lib().q1g128_gemv_grouped
+    _offer_native()
     with torch.cuda.device(dev):
         rc = fn(descs, len(problems), out_kind, scale_kind, _stream(dev))
     if rc != 0:
         raise RuntimeError(f"{kind}: grouped native launch failed with status {rc}")
-    if _native is None:
-        _load_native()
     return results
 
 
@@ -662,13 +674,12 @@ def quant_input(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     s = torch.empty(*x.shape[:-1], 1, dtype=torch.float32, device=x.device)
     if m == 0:
         return q, s
+    _offer_native()
     with torch.cuda.device(x.device):
         rc = actq_lib().bonsai_act_quant_int8(_ptr(x), _X_KIND[x.dtype], _ptr(q), _ptr(s), m, k,
                                               _stream(x.device))
     if rc != 0:
         raise RuntimeError(f"quant_input: native launch failed with status {rc}")
-    if _native is None:
-        _load_native()
     return q, s
 
 
@@ -692,13 +703,12 @@ def fused_norm_quant(x: torch.Tensor, w: torch.Tensor, eps: float) -> Tuple[torc
     m = x.numel() // k
     q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     s = torch.empty(*x.shape[:-1], 1, dtype=torch.float32, device=x.device)
+    _offer_native()
     with torch.cuda.device(x.device):
         rc = actq_lib().bonsai_rmsnorm_quant_int8(_ptr(x), _ptr(w), float(eps), _ptr(q), _ptr(s), m, k,
                                                   _stream(x.device))
     if rc != 0:
         raise RuntimeError(f"fused_norm_quant: native launch failed with status {rc}")
-    if _native is None:
-        _load_native()
     return q, s
 
 
@@ -718,14 +728,13 @@ def fused_add_norm_quant(x: torch.Tensor, residual: torch.Tensor, w: torch.Tenso
     h = torch.empty_like(x)
     q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     s = torch.empty(*x.shape[:-1], 1, dtype=torch.float32, device=x.device)
+    _offer_native()
     with torch.cuda.device(x.device):
         rc = actq_lib().bonsai_add_rmsnorm_quant_int8(_ptr(x), _ptr(residual), _ptr(w), float(eps),
                                                       _ptr(h), _ptr(q), _ptr(s), m, k,
                                                       _stream(x.device))
     if rc != 0:
         raise RuntimeError(f"fused_add_norm_quant: native launch failed with status {rc}")
-    if _native is None:
-        _load_native()
     return h, q, s
 
 
@@ -766,11 +775,10 @@ def silu_mul_quant(gate_up: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     m = gate_up.numel() // f2
     q = torch.empty(*gate_up.shape[:-1], f, dtype=torch.int8, device=gate_up.device)
     s = torch.empty(*gate_up.shape[:-1], 1, dtype=torch.float32, device=gate_up.device)
+    _offer_native()
     with torch.cuda.device(gate_up.device):
         rc = actq_lib().bonsai_silu_mul_quant_int8(_ptr(gate_up), _ptr(q), _ptr(s), m, f,
                                                    _stream(gate_up.device))
     if rc != 0:
         raise RuntimeError(f"silu_mul_quant: native launch failed with status {rc}")
-    if _native is None:
-        _load_native()
     return q, s

@@ -23,6 +23,41 @@ def test_declines_what_is_not_a_plain_gpu_tensor():
     assert n.add_norm_quant(x, x, w, 1e-6) is None and n.silu_mul_quant(x) is None
 
 
+def _without_extension(monkeypatch, tmp_path, broken=False):
+    so = tmp_path / "_bonsai_py.so"
+    if broken:
+        so.write_bytes(b"not a library")
+    monkeypatch.setattr(ops, "_native", None)
+    monkeypatch.setattr(ops, "_native_missing", False)
+    monkeypatch.setattr(ops, "py_ops_lib_path", lambda: str(so))
+
+
+@pytest.mark.parametrize("broken", [False, True])
+def test_only_the_prompt_path_needs_the_extension(monkeypatch, tmp_path, broken):
+    _without_extension(monkeypatch, tmp_path, broken)
+    with pytest.warns(RuntimeWarning, match="_bonsai_py.so"):
+        ops._offer_native()
+    import warnings
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        ops._offer_native()      # said once
+    with pytest.raises((RuntimeError, ImportError)):
+        ops.native()
+
+
+@pytest.mark.gpu
+def test_operators_run_without_the_extension(monkeypatch, tmp_path):
+    x = torch.randn(3, 512, device=DEV).to(torch.bfloat16)
+    b = torch.randint(-128, 128, (48, 128), device=DEV, dtype=torch.int8)
+    ws = torch.rand(48, 4, device=DEV).to(torch.bfloat16)
+    want = ops.t2g128_int8xint2_linear(*ops.quant_input(x)[:1], b, ops.quant_input(x)[1], ws)
+    _without_extension(monkeypatch, tmp_path)
+    with pytest.warns(RuntimeWarning, match="slower host path"):
+        q, s = ops.quant_input(x)
+    _same(ops.t2g128_int8xint2_linear(q, b, s, ws), want)
+    assert ops._native is None
+
+
 def _same(got, want):
     got, want = (g if isinstance(g, (tuple, list)) else (g,) for g in (got, want))
     assert len(got) == len(want)
