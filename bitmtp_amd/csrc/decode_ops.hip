@@ -1698,6 +1698,10 @@ static int cu_count() {
     return n;
 }
 
+static thread_local const char *t_prompt_attn = "none";
+
+extern "C" const char *bonsai_prefill_attention_kernel(void) { return t_prompt_attn; }
+
 extern "C" int bonsai_prefill_attention(const void *q, const void *k_layer, const void *v_layer, void *out_bf16,
                                         float scale, int M, int n_heads, int n_kv, int slots, int base,
                                         void *stream) {
@@ -1717,6 +1721,7 @@ extern "C" int bonsai_prefill_attention(const void *q, const void *k_layer, cons
                        static_cast<const uint16_t *>(k_layer), static_cast<const uint16_t *>(v_layer),
                        static_cast<uint16_t *>(out_bf16), scale * 1.44269504088896340736f, M, n_heads, n_kv, hpg,
                        slots, base, tokens, tiles);
+    t_prompt_attn = split ? "prefill_attn_split_kernel" : "prefill_attn_kernel";
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }
 

@@ -52,6 +52,8 @@ def load_decode_kernel() -> None:
     lib.bonsai_prefill_rope_kv_write.restype = ci
     lib.bonsai_prefill_attention.argtypes = [vp, vp, vp, vp, cf, ci, ci, ci, ci, ci, vp]
     lib.bonsai_prefill_attention.restype = ci
+    lib.bonsai_prefill_attention_kernel.argtypes = []
+    lib.bonsai_prefill_attention_kernel.restype = ctypes.c_char_p
     lib.bonsai_decode_set_tuning.argtypes = [ci]
     lib.bonsai_decode_set_tuning.restype = None
     lib.bonsai_decode_set_attention_engine.argtypes = [ci]
@@ -305,6 +307,11 @@ def prefill_attention(q: torch.Tensor, k_layer: torch.Tensor, v_layer: torch.Ten
                                                    n_heads, n_kv, slots, int(base), _stream(q.device))
     _need(rc == 0, f"bonsai_prefill_attention failed with status {rc}")
     return out
+
+
+def prefill_attention_kernel() -> str:
+    """Name of the kernel this thread's last :func:`prefill_attention` went to (diagnostics for tests)."""
+    return decode_lib().bonsai_prefill_attention_kernel().decode()
 
 
 def kv_commit(kv: torch.Tensor, src_slot: int, dst_slot: int, n: int) -> None:

@@ -82,6 +82,10 @@ int bonsai_prefill_attention(const void *q, const void *k_layer, const void *v_l
                              float scale, int M, int n_heads, int n_kv, int slots, int base,
                              void *stream);
 
+/* Name of the kernel the calling thread's last bonsai_prefill_attention went to ("none" before the first): a
+ * read-only diagnostic for tests; no reference counterpart. */
+const char *bonsai_prefill_attention_kernel(void);
+
 /* Process-wide tuning of the attention launch geometry: query rows per wave (1..4), 0 =
  * built-in heuristic.  No counterpart in the reference; results do not depend on it. */
 void bonsai_decode_set_tuning(int rows_per_wave);

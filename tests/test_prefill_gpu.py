@@ -68,6 +68,33 @@ def test_prefill_attention_with_a_history_of_minus_infinity(m, n_heads, n_kv):
     _assert_causal_attention(got, q, k[:, hidden:], v[:, hidden:], base - hidden)
 
 
+@pytest.mark.parametrize("m,n_heads,n_kv,base,slots,split", [
+    # two rounds of 32-pair workgroups on 256 CUs, and the first row count beyond
+    (1024, 16, 8, 5, 1040, True), (1025, 16, 8, 5, 1040, False),
+    # ratios that leave pairs of the 128 idle (3, 5, 7, 24), and one that has none to spare
+    (2571, 6, 2, 30, 2610, False), (1540, 20, 4, 0, 1540, False), (600, 56, 8, 65, 670, False), (200, 120, 5, 10, 210, False),
+    (1100, 16, 16, 63, 1200, False),
+    # more than 32 query heads a kv head: never the 32-pair kernel
+    (1, 33, 1, 0, 8, False), (70, 40, 1, 129, 200, False), (67, 128, 2, 0, 67, False), (131, 128, 1, 1, 140, False)])
+def test_which_prefill_attention_kernel_runs(m, n_heads, n_kv, base, slots, split):
+    from bitmtp_amd import decode_ops
+    hpg, cus = n_heads // n_kv, torch.cuda.get_device_properties(0).multi_processor_count
+    if cus == 256:  # (the line lies elsewhere on a part of another size; the results below hold there too)
+        assert split == (hpg <= 32 and -(-m // (32 // hpg)) * n_kv <= 2 * cus)
+    print(f"[case] prefill attention kernel m={m} heads={n_heads}/{n_kv} base={base}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(m + base)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)
+    q, k, v = rnd(m, n_heads, 128), rnd(n_kv, slots, 128), rnd(n_kv, slots, 128)
+    seen = base + m
+    k[:, seen:] = float("nan")
+    v[:, seen:] = float("nan")
+    got = decode_ops.prefill_attention(q, k, v, base).view(m, n_heads, 128)
+    torch.cuda.synchronize()
+    if cus == 256:
+        assert decode_ops.prefill_attention_kernel() == ("prefill_attn_split_kernel" if split else "prefill_attn_kernel")
+    _assert_causal_attention(got, q, k, v, base)
+
+
 @pytest.mark.parametrize("m,n_heads,n_kv", [(1, 4, 2), (33, 3, 1), (67, 16, 8)])
 def test_prompt_rows_rope_is_the_steps_own(m, n_heads, n_kv):
     """q / k norm + RoPE + KV write of prompt rows: the bits of the step's entry point, 32 rows at a time."""
@@ -119,7 +146,8 @@ def _replayed(atlas, prompt, sigma):
                                                ("q1", "bf16", 157, None), ("q1", "q1", 70, 64)])
 def test_prompt_block_against_replayed_steps(kind, head, n, block, monkeypatch):
     """Keys, values and last-row logits of the prompt path are those of the stepped decoder: the first layer to the
-    bit (the same sums), deeper ones and the logits within the order of the attention's sums."""
+    bit (K = 512 is one K slice in every kernel: the same sums), deeper ones and the logits within the order of the
+    attention's sums (which moves single int8 steps; equal to the bit as well at these sizes when this was written)."""
     from bitmtp_amd import generate, runtime
     from bitmtp_amd.model import BonsaiDecoder, ModelArgs
     from bitmtp_amd.runtime import GraphAtlas
@@ -138,11 +166,10 @@ def test_prompt_block_against_replayed_steps(kind, head, n, block, monkeypatch):
     got = atlas.kv(256)[:, :, :, :n]
     logits = atlas.workspace.logits_buf[: want_logits.numel()].float()
     scale = want_logits.abs().max()
-    assert (logits - want_logits).abs().max() <= 6e-2 * scale
+    assert (logits - want_logits).abs().max() <= 2e-2 * scale
     assert first == int(logits[:1000].argmax())
-    d0 = (got[:, 0].float() - want[:, 0].float()).abs()
-    assert d0.max() <= 2e-2 * want[:, 0].float().abs().max() and (d0 > 0).float().mean() < 1e-2
-    assert (got.float() - want.float()).norm() <= 3e-2 * want.float().norm()
+    assert torch.equal(got[:, 0].view(torch.int16), want[:, 0].view(torch.int16))
+    assert (got.float() - want.float()).norm() <= 2e-2 * want.float().norm()
 
 
 def test_prompt_longer_than_its_segment_is_refused():
