@@ -1,14 +1,14 @@
-// Entry-point logic shared by libbonsai_t2.so and libbonsai_q1.so: argument
-// checks, one-time device set-up and the choice among the kernels.  Measured on
-// MI355X: the dot4 kernel (packed_gemv.hip.h) is fastest for one and two tokens
-// on layer-sized matrices; from three tokens on (from two for very long matrices,
-// the lm_head) the int8 matrix-core kernels (gemv_mfma.hip.h) win: the one that
-// loads the activations straight as operands up to 16384 rows, the one that
-// stages them in LDS once per workgroup above; one token against a very long matrix
-// has a kernel of its own (gemv_rowreg.hip.h), wider blocks there take the streaming
-// matrix-core kernel (gemv_mxs.hip.h).  Shapes the matrix-core kernels do not take (K not a multiple of
-// 512, unaligned operands, token tiles that do not fit in LDS) go to the dot4
-// kernel.  Replaces the if-chain over registered (M, N, K) of the reference
+// Entry-point logic shared by libbonsai_t2.so and libbonsai_q1.so: argument checks, one-time device set-up and the
+// choice among the kernels.  Measured on MI355X, by block width:
+//   1, 2    dot4 (packed_gemv.hip.h); matrix cores at two tokens for long rows (K >= 4096) and very long matrices
+//   3-16    the lean matrix-core kernel (gemv_mxl.hip.h), one descriptor per tile of up to 16 tokens, also in grouped
+//           launches; lean_takes says which rows and grids
+//   17 on   the wide kernel (gemv_wide.hip.h) where it is expected to be faster than whatever would run otherwise
+//           (wide_default; grouped_leavers for the problems of one call), else as before
+//   very long matrices (the lm_head): one token gemv_rowreg.hip.h, up to 16 gemv_mxs.hip.h
+// What none of these takes goes to the matrix-core kernels of gemv_mfma.hip.h (short rows on many rows, K a multiple
+// of 512; operands loaded directly up to 16384 rows, staged above) and, with K no multiple of 512 at widths up to
+// four or unaligned scales, to dot4.  Replaces the if-chain over registered (M, N, K) of the reference
 // (src/bonsai_sft/gpu/t2g128_kernels/t2g128_kernels.cu:94-148).
 #ifndef BONSAI_GEMV_DISPATCH_HIP_H
 #define BONSAI_GEMV_DISPATCH_HIP_H

@@ -4,18 +4,20 @@
 // every weight is multiplied with tens to thousands of tokens, and what bounds the kernel is the issue
 // of vector instructions: per scale group (128 of K) the exact int32 sums must become fp32 and meet the
 // group's scale, two operations a result (eight per 16 x 16 results, against two matrix instructions),
-// beside unpacking the weights and arranging the activations.  On this part a wave that is alone on its
-// SIMD issues a vector operation every 8.7 clocks, two waves every 5.5, four every 4.7, and a matrix
-// instruction costs 8 of issue whatever its size.  So
+// beside unpacking the weights and arranging the activations.  Counters at 3001 tokens: the vector ALU is
+// busy in 82 % of the cycles with four waves a SIMD (19456 x 2560, 64x256) and in 60 % with two
+// (2560 rows, 128x256), the matrix cores in 30-37 %.  So
 //   * v_mfma_i32_32x32x32_i8: half the matrix instructions of the 16 x 16 form;
 //   * weights are unpacked to 64 times their value (mfma_unpack64), which needs no offset term -- the
 //     other forms feed -2 sum(a) through the accumulator, 8 more matrix instructions per 16 x 64 x 64 --
 //     and the factor, a power of two, goes out with the division;
 //   * the accumulators start from the bits of 1.5 * 2^23, so that a sum is a float and one exact
 //     subtraction stands for the conversion;
-//   * 64 tokens x 32 rows a wave in 128 registers, four waves a SIMD, are ahead of 64 x 64 in 224.
-// 19456 x 2560 at 3001 tokens 254 -> 206 us (1.45 POP/s), 2560 x 9728 123 -> 97, 12288 x 2048 at 514
-// 35 -> 27, at 256 19.6 -> 16.8, 2048 x 2048 at 256 7.1 -> 6.6.
+//   * 64 tokens x 32 rows a wave in 128 registers, four waves a SIMD, are ahead of 64 x 64 in 224
+//     where the rows fill the chip.
+// Back to back on random bytes, with 16 x 16 instructions before -> now: 19456 x 2560 at 3001 tokens 254 -> 203 us
+// (1.47 POP/s; 191 us and 1.56 within a prompt; PyTorch's int8 product reaches 1.99 at 16384^3), 2560 x 9728 123 -> 97,
+// 12288 x 2048 at 514 35 -> 26, at 256 19.6 -> 16.7, 2048 x 2048 at 256 7.1 -> 6.6.
 //
 //   WM x WN waves share a staged block of WM*MT*32 tokens x WN*NT*32 rows; KS such sets of waves
 //   split K and add their fp32 results up in slice order (narrower blocks and few rows, where a
@@ -460,8 +462,9 @@ int wide_init_device(int max_lds) {
 
 // What a launch takes, in microseconds: a fixed part, the scale groups of a K slice times the length of one
 // -- bound by latency up to some tiles per CU, then by what they issue -- and a part per tile for its scales
-// and its results.  Fitted to 17 ... 4096 tokens of 13 matrices (1024 x 1024 ... 20000 x 9728): 4-9 % rms,
-// then moved within that for the choice between them.
+// and its results.  Fitted to 17 ... 4096 tokens of 13 matrices (1024 x 1024 ... 20000 x 9728), then moved for
+// the choice between them.  Over 220 drawn blocks with weights from HBM each is off by 13-18 % rms, mostly by a
+// part that all share (9-16 % low).
 inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
     struct Cost {
         int tokens, rows, slices;
@@ -488,8 +491,9 @@ bool wide_fits(int v, int K, int lds_limit) {
     return k.lds(K) <= (size_t)lds_limit && (long)k.rows * K <= (1L << 30) && (long)k.tokens * K <= (1L << 30);
 }
 
-// The variant with the smallest estimate among those that take rows of K weights: at most 2.4 % behind the best of
-// them over the same sweep.  -1: none does.
+// The variant with the smallest estimate among those that take rows of K weights: over 220 drawn blocks 0.8 % behind
+// the best of them in the mean, within 0.8 % on nine in ten, 21 % at most (16586 x 2560 of sign weights at 89 tokens:
+// 64x128_K2 for 32x64_K4).  -1: none does.
 template <int BITS>
 int wide_pick(int M, int N, int K, int n_cus, int lds_limit) {
     int best = -1;

@@ -674,8 +674,9 @@ def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: torch.Tensor, last
 # ---------------------------------------------------------------------------
 # Prompts
 # ---------------------------------------------------------------------------
-# Rows of one block: what the buffers below are sized for at most (a row takes about 70 KB with the 4B
-# shape).  A default segment's whole prompt is one block, so every weight is read once.
+# Rows of one block: what the buffers below are sized for at most.  A row takes 99 KB with the 4B shape, so
+# 407 MB at 4096 rows, which the atlas keeps.  A default segment's whole prompt is one block, so every weight
+# is read once.
 PROMPT_BLOCK_MAX = 4096
 
 

@@ -244,7 +244,8 @@ int bonsai_silu_mul_quant_int8(const void *gate_up, int8_t *q, float *s, int M, 
  *   with activations loaded as operands, 4 = the grouped kernels with one descriptor (the lean
  *   form where it applies), 5 = the streaming kernel on any shape it can run (otherwise only on
  *   very long matrices), 6 = the single-token register kernel on any T2 matrix with K of 1024,
- *   2048 or 4096 (otherwise only on very long ones).
+ *   2048 or 4096 (otherwise only on very long ones), 7 = the wide-block kernel at any width,
+ *   where row_tiles is 1 + the number of its tile (0: its own choice).
  * set_grouped_tuning: the grouped kernels -- 16-row tiles per wave (1 or 2) and a cap on the
  *   workgroups of one launch (either one set selects the general grouped kernel instead of
  *   its lean form), smallest width sent to the matrix cores (a value above zero also keeps

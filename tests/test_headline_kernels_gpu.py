@@ -4,8 +4,10 @@ choose), ``gemv_dot4_grouped_kernel`` (one- and two-token grouped launches),
 ``gemv_mxs_kernel`` and ``gemv_rowreg_kernel`` (very long matrices) -- pinned on their own,
 through the C ABI, at the K of the real layers (2048, 2560, 6144, 9728):
 
-* the int32 group sums ``G`` come from the very kernel that produces the bf16 result
-  (asserted through the library's last-kernel record) and are bit-exact against the oracle on
+* the int32 group sums ``G`` come from the kernel that produces the bf16 result (asserted
+  through the library's last-kernel record; a launch of one matrix by the lean kernel is a build
+  whose arguments are not a table, and its sums come from the table build of the same body, so
+  there the scaled results below pin it) and are bit-exact against the oracle on
   every byte value (T2 code 0 = -2 included, rows of 0x00 and 0xFF) and activations over all of
   int8 with an all -128 and an all 127 row;
 * with every scale 1 the fp32 output equals the integer product ``unpack(B) @ A`` exactly (all
