@@ -73,6 +73,33 @@ def test_built_in_choice_is_among_kernels_that_run(m, n, k, family, bits):
     _check(m, n, k, bits, torch.bfloat16, family)
 
 
+@pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits", [2, 1])
+@pytest.mark.parametrize("m,n,k", [(3, 1, 512), (4, 17, 512), (8, 100, 1024), (9, 48, 1536), (16, 333, 1024), (33, 1000, 512),
+                                   (64, 700, 1536)])
+def test_lean_kernel_rows_of_one_to_three_tiles(m, n, k, bits, scale_dtype):
+    """Fewer K tiles than waves: some slices are empty."""
+    print(f"[case] lean short rows bits {bits} {m}x{n}x{k} {scale_dtype}", flush=True)
+    _check(m, n, k, bits, scale_dtype, "gemv_mxl_kernel<")
+
+
+@pytest.mark.parametrize("bits", [2, 1])
+@pytest.mark.parametrize("m,n,k", [(2, 40, 512), (5, 333, 1024), (16, 100, 2048), (17, 100, 2048), (200, 300, 512),
+                                   (70, 1000, 2176)])
+def test_scales_on_any_16_bit_address(m, n, k, bits):
+    """Scales that do not start on 8 bytes keep the kernels with wide scale loads out, alone and in a grouped call."""
+    print(f"[case] unaligned scales bits {bits} {m}x{n}x{k}", flush=True)
+    a, b, s, ws, groups, want = _problem(m, n, k, bits, m + n + k)
+    flat = torch.empty(ws.numel() + 1, dtype=ws.dtype, device=DEV)
+    odd = flat[1:].view(ws.shape)
+    odd.copy_(ws)
+    assert odd.data_ptr() % 8 == 2 and odd.is_contiguous()
+    scale = (groups.abs() * ws.double()).sum(-1) / s.double()
+    for y in (ops.packed_gemv_ex(a, b, s, odd, bits=bits, out_kind=ops.OUT_F32),
+              ops.packed_gemv_grouped([(a, b, s, odd), (a, b, s, ws)], bits=bits, out_kind=ops.OUT_F32)[0]):
+        assert ((y.double() - want).abs() <= 1e-6 * scale + 1e-30).all()
+
+
 @pytest.mark.parametrize("bits", [2, 1])
 @pytest.mark.parametrize("m,n,k", [(600, 600, 23936), (300, 4100, 24064), (130, 1100, 32512), (70, 520, 56704), (33, 40, 65536)])
 def test_rows_too_long_for_some_tiles(m, n, k, bits):
