@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the packed T2-g128 GEMV hot path on one MI355X.
 
-Workload (BASELINE.json configs[1]): all seven linear projections of one
+Workload: all seven linear projections of one
 Qwen3-1.7B-shaped decoder layer in T2-g128 -- q/o 2048x2048, k/v 1024x2048,
 gate/up 6144x2048, down 2048x6144 -- at widths 1, 4 and 8.  One STEP is that set
 once.  It is measured two ways:
@@ -18,9 +18,8 @@ HIP graph so that the Python launch cost is outside the measurement, as in the
 reference's graph-replayed decode.
 
 Beside the headline, `config` carries the rest of the target range on the same timing (one
-graph per figure over >= 512 MB of distinct weights): BASELINE.json configs[0] (one 6144 x 2048 GEMV
-at width 1), the 4B-shaped layer (K = 2560, 4096, 9728) grouped and as its four merged
-matrices, the Q1-g128 set of configs[4], both packed lm_heads, and the end-to-end decode runs.
+graph per figure over >= 512 MB of distinct weights): one 6144 x 2048 GEMV at width 1, the 4B-shaped layer (K = 2560, 4096, 9728) grouped and as its four merged
+matrices, the Q1-g128 set (K = 2560, 9728), both packed lm_heads, and the end-to-end decode runs.
 Every figure names the kernel that was launched (read back from the library, not written here).
 
 Prints ONE JSON line: the driver's fields (metric, value, unit, ...), `config`, `roofline` of the
@@ -418,7 +417,7 @@ def main() -> int:
                     help="skip the end-to-end decode tokens/s section")
     ap.add_argument("--no-head", action="store_true", help="skip the lm_head-sized extra measurements")
     ap.add_argument("--no-extra", action="store_true",
-                    help="skip configs[0], the 4B-shaped layer and the Q1 set (profiling runs)")
+                    help="skip the single 6144 x 2048 GEMV, the 4B-shaped layer and the Q1 set (profiling runs)")
     ap.add_argument("--widths", default=None,
                     help="comma list restricting the widths measured (profiling runs); default 1,4,8")
     ap.add_argument("--no-drop-in", action="store_true",
@@ -527,11 +526,11 @@ def main() -> int:
         "read_probe_us": per_width[dom]["read_probe_us"],
     }
 
-    # ---- the rest of the target range (T2 K = 2048..9728, Q1 configs[4])
+    # ---- the rest of the target range (T2 K = 2048..9728, Q1)
     config0 = layer_4b = q1_set = None
     if not args.no_extra:
         from bitmtp_amd import gemv_bench
-        # configs[0]: a single 6144 x 2048 GEMV at width 1 through the drop-in symbol
+        # a single 6144 x 2048 GEMV at width 1 through the drop-in symbol
         r0 = gemv_bench.sweep("t2", [(6144, 2048)], [1], pool_bytes=MIN_DISTINCT_BYTES, max_pool=512,
                               quiet=True)[0]
         config0 = {k: r0[k] for k in ("N", "K", "width", "bytes", "pool", "us_per_launch", "gbps",
@@ -559,7 +558,7 @@ def main() -> int:
         }
         run = run4
         del pool4
-        # configs[4]: Q1-g128, K in {2560, 9728} x N in {1024, 2560, 9728}, drop-in symbol
+        # Q1-g128, K in {2560, 9728} x N in {1024, 2560, 9728}, drop-in symbol
         q1_rows = gemv_bench.sweep("q1", gemv_bench.PRESETS["config4"], list(WIDTHS),
                                    pool_bytes=MIN_DISTINCT_BYTES, quiet=True)
         q1_set = {}
@@ -583,7 +582,7 @@ def main() -> int:
         torch.cuda.synchronize()
 
     # The other half of the headline metric: end-to-end decode tokens/s of the random-init
-    # 1.7B-shaped model (configs[2]), AR and D8 hybrid, by the reference's timing contract.
+    # 1.7B-shaped model, AR and D8 hybrid, by the reference's timing contract.
     decode = decode_bf16 = decode_4b = None
     if not args.no_decode:
         del run
@@ -596,7 +595,7 @@ def main() -> int:
         decode_bf16 = run_decode_bench("1.7b", prompt_len=256, new_tokens=512, repeats=1,
                                        head_kind="bf16")
         torch.cuda.empty_cache()
-        # configs[3]: the 4B-shaped model, 512-token prompt, 1024 new tokens
+        # the 4B-shaped model, 512-token prompt, 1024 new tokens
         decode_4b = run_decode_bench("4b", prompt_len=512, new_tokens=1024, repeats=1)
 
     cpu = cpu_baseline(args.cpu_seconds) if args.cpu_seconds > 0 else None
@@ -607,7 +606,7 @@ def main() -> int:
         "ms_per_step": round(ms_per_step, 5), "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "int8", "data": "synthetic",
         "config": {
-            "workload": "configs[1]: 7 T2-g128 projections of one Qwen3-1.7B-shaped layer at "
+            "workload": "7 T2-g128 projections of one Qwen3-1.7B-shaped layer at "
                         "widths 1,4,8, grouped: one t2g128_gemv_grouped launch per width "
                         "(3 launches/step), HBM-cold over a pool of distinct layers",
             "pool_layers": args.layers, "pool_bytes": args.layers * LAYER_BYTES,

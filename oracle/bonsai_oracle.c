@@ -1,6 +1,6 @@
 /*
  * CPU oracle for the packed low-bit GEMV path (T2-g128 ternary W2A8 and
- * Q1-g128 sign W1A8).  TEST INFRASTRUCTURE ONLY: this file is the checker the
+ * Q1-g128 sign W1A8).  TEST INFRASTRUCTURE ONLY: this file is what the
  * HIP kernels are compared against and the CPU baseline that gets timed.  The
  * shipped library never links or calls it.
  *
