@@ -25,6 +25,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/bonsai_decode.h"
 #include "prefill_attn.hip.h"
@@ -1613,6 +1614,8 @@ int rows_per_wave(int M) {
     return 4;
 }
 
+#include "step_one.hip.h"
+
 }  // namespace
 
 static int launch_rope(const void *xqkv, const void *q_norm_w,
@@ -1873,6 +1876,64 @@ extern "C" int bonsai_decode_attention_rope_parts(const void *xqkv, const void *
                      static_cast<uint16_t *>(out_amax), (n_kv + 7) & ~7};
     return launch_attention(xqkv, k_layer, v_layer, meta, scratch, nullptr, nullptr, nullptr, scale, M,
                             n_heads, n_kv, slots, sigma, &rope, &fin, static_cast<hipStream_t>(stream));
+}
+
+// ---- one launch for all layers of a one-token step (step_one.hip.h) ------------------------
+extern "C" int64_t bonsai_decode_step_one_bytes(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv) {
+    const step_one::Fit f = step_one::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
+    return f.build < 0 ? 0 : f.bytes;
+}
+
+extern "C" int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange,
+                                            void *stream) {
+    const step_one::Fit f = step_one::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
+    if (f.build < 0 || !exchange || (reinterpret_cast<uintptr_t>(exchange) & 127)) return BONSAI_DECODE_ERR_ARG;
+    const step_one::Rows lay(dim, ffn, n_heads, n_kv);
+    const size_t from = step_one::kControlBytes / 16, to = from + (size_t)2 * n_layers * lay.size / 16;
+    hipLaunchKernelGGL(step_one::exchange_reset_kernel, dim3(256), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<step_one::v4u *>(exchange), (size_t)f.bytes / 16, from, to);
+    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+}
+
+extern "C" int bonsai_decode_step_one(const bonsai_step_one_desc *d, void *stream) {
+    if (!d || !d->layers || !d->embed || !d->step_in || !d->kv || !d->cos_table || !d->sin_table || !d->exchange || !d->h_out ||
+        !d->status)
+        return BONSAI_DECODE_ERR_ARG;
+    if (d->slots < 1 || d->sigma < 0 || d->sigma >= d->slots || d->max_pos < 1 || d->vocab < 1 || d->slots > (1 << 22) ||
+        (reinterpret_cast<uintptr_t>(d->exchange) & 127) || (reinterpret_cast<uintptr_t>(d->embed) & 15) ||
+        (reinterpret_cast<uintptr_t>(d->kv) & 15) || (reinterpret_cast<uintptr_t>(d->layers) & 7) ||
+        (reinterpret_cast<uintptr_t>(d->step_in) & 3) || (reinterpret_cast<uintptr_t>(d->h_out) & 3))
+        return BONSAI_DECODE_ERR_ARG;
+    const int groups = cu_count();
+    const step_one::Fit f = step_one::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, groups);
+    if (f.build < 0) return BONSAI_DECODE_ERR_ARG;
+    step_one::Args a;
+    a.layers = static_cast<const step_one::Layer *>(d->layers);
+    a.embed = static_cast<const uint16_t *>(d->embed);
+    a.step_in = d->step_in;
+    a.kv = static_cast<uint16_t *>(d->kv);
+    a.cos_t = static_cast<const uint16_t *>(d->cos_table);
+    a.sin_t = static_cast<const uint16_t *>(d->sin_table);
+    a.exchange = static_cast<uint8_t *>(d->exchange);
+    a.h_out = static_cast<uint16_t *>(d->h_out);
+    a.status = d->status;
+    a.n_layers = d->n_layers;
+    a.dim = d->dim;
+    a.ffn = d->ffn;
+    a.n_heads = d->n_heads;
+    a.n_kv = d->n_kv;
+    a.slots = d->slots;
+    a.sigma = d->sigma;
+    a.max_pos = d->max_pos;
+    a.vocab = d->vocab;
+    a.groups = groups;
+    a.eps = d->eps;
+    a.scale = d->scale;
+    void *args[] = {&a};
+    if (hipLaunchKernel(step_one::kernel_of(f.build), dim3(groups), dim3(step_one::kThreads), args, (size_t)f.lds,
+                        static_cast<hipStream_t>(stream)) != hipSuccess)
+        return BONSAI_DECODE_ERR_LAUNCH;
+    return BONSAI_DECODE_OK;
 }
 
 extern "C" int bonsai_kv_commit(void *kv, int n_layers, int n_kv, int slots, int src_slot,

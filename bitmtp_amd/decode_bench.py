@@ -132,6 +132,8 @@ def run_slot_costs(model_name: str = "1.7b", cache_len: int = 500, device: str =
 
     saved = (mdl._gemv, decode_ops.qk_norm_rope_kv_write, decode_ops.decode_attention, ops.actq_lib,
              mdl._fused, os.environ.get("BONSAI_FUSED_STEP"))
+    one_launch = os.environ.get("BONSAI_ONE_LAUNCH_STEP")
+    os.environ["BONSAI_ONE_LAUNCH_STEP"] = "0"   # operators are left out of the separate launches
     out = {"model": model_name, "cache_len": cache_len, "widths": {}}
     try:
         for M, role in ((1, "ar"), (9, "verify")):
@@ -186,6 +188,10 @@ def run_slot_costs(model_name: str = "1.7b", cache_len: int = 500, device: str =
     finally:
         (mdl._gemv, decode_ops.qk_norm_rope_kv_write, decode_ops.decode_attention, ops.actq_lib,
          mdl._fused) = saved[:5]
+        if one_launch is None:
+            del os.environ["BONSAI_ONE_LAUNCH_STEP"]
+        else:
+            os.environ["BONSAI_ONE_LAUNCH_STEP"] = one_launch
         if saved[5] is None:
             os.environ.pop("BONSAI_FUSED_STEP", None)
         else:

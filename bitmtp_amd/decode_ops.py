@@ -21,6 +21,15 @@ ATTN_CHUNK = 64
 _lib = None
 
 
+class StepOneDesc(ctypes.Structure):
+    """``bonsai_step_one_desc`` of include/bonsai_decode.h."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("layers", "embed", "step_in", "kv", "cos_table", "sin_table", "exchange",
+                                                "h_out", "status")]
+                + [(n, ctypes.c_int) for n in ("bits", "n_layers", "dim", "ffn", "n_heads", "n_kv", "slots", "sigma",
+                                               "max_pos", "vocab")]
+                + [("eps", ctypes.c_float), ("scale", ctypes.c_float)])
+
+
 def decode_lib_path() -> str:
     return os.path.join(_HERE, "decode_ops", "libbonsai_decode.so")
 
@@ -76,6 +85,12 @@ def load_decode_kernel() -> None:
     lib.bonsai_fp8_quant_rows.restype = ci
     lib.bonsai_fp8_linear.argtypes = [vp, vp, vp, cf, vp, ci, ci, ci, vp]
     lib.bonsai_fp8_linear.restype = ci
+    lib.bonsai_decode_step_one_bytes.argtypes = [ci] * 6
+    lib.bonsai_decode_step_one_bytes.restype = ctypes.c_int64
+    lib.bonsai_decode_step_one_reset.argtypes = [ci] * 6 + [vp, vp]
+    lib.bonsai_decode_step_one_reset.restype = ci
+    lib.bonsai_decode_step_one.argtypes = [ctypes.POINTER(StepOneDesc), vp]
+    lib.bonsai_decode_step_one.restype = ci
     _lib = lib
 
 
@@ -312,6 +327,56 @@ def prefill_attention(q: torch.Tensor, k_layer: torch.Tensor, v_layer: torch.Ten
 def prefill_attention_kernel() -> str:
     """Name of the kernel this thread's last :func:`prefill_attention` went to (diagnostics for tests)."""
     return decode_lib().bonsai_prefill_attention_kernel().decode()
+
+
+class StepOne:
+    """All layers of a one-token step in one launch (``bonsai_decode_step_one``): the addresses of a model's weights
+    and the exchange memory its workgroups hand rows over in.  One launch at a time may use an object.  ``status`` is
+    nonzero, once the launches queued so far have ended, if one of them did not get the whole device: nothing those
+    launches wrote is of use, and ``reset`` makes the object ready again."""
+
+    def __init__(self, layers: torch.Tensor, shape, device):
+        """``layers``: int64 ``[n_layers, 12]`` on the device; ``shape``: (bits, n_layers, dim, ffn, n_heads, n_kv)."""
+        _check(layers, torch.int64, "layers")
+        _need(tuple(layers.shape) == (shape[1], 12), "layers must be [n_layers, 12]")
+        self.layers, self.shape, self.device = layers, tuple(shape), device
+        nbytes = self.exchange_bytes(shape, device)
+        _need(nbytes > 0, "this shape does not run as one launch")
+        self.exchange = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        self.status = torch.zeros(1, dtype=torch.int32).pin_memory()   # written by the device, only when it gives up
+        self.failed = self.status.numpy()
+        self.reset()
+
+    @staticmethod
+    def exchange_bytes(shape, device) -> int:
+        """Size of the exchange memory; 0 for shapes that do not run as one launch."""
+        with torch.cuda.device(device):
+            return int(decode_lib().bonsai_decode_step_one_bytes(*shape))
+
+    def reset(self) -> None:
+        self.failed[0] = 0
+        with torch.cuda.device(self.device):
+            rc = decode_lib().bonsai_decode_step_one_reset(*self.shape, _ptr(self.exchange), _stream(self.device))
+        _need(rc == 0, f"bonsai_decode_step_one_reset failed with status {rc}")
+
+    def enqueue(self, embed: torch.Tensor, step_in: torch.Tensor, kv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                sigma: int, eps: float, h_out: torch.Tensor) -> None:
+        bits, n_layers, dim, ffn, n_heads, n_kv = self.shape
+        for t, name in ((embed, "embed"), (kv, "kv"), (cos, "cos"), (sin, "sin"), (h_out, "h_out")):
+            _check(t, torch.bfloat16, name)
+        _check(step_in, torch.int32, "step_in")
+        _need(embed.dim() == 2 and embed.shape[1] == dim and h_out.numel() >= dim, "embed / h_out shape mismatch")
+        _need(kv.dim() == 5 and kv.shape[:3] == (2, n_layers, n_kv) and kv.shape[4] == HEAD_DIM, "kv shape mismatch")
+        _need(cos.shape == sin.shape and cos.dim() == 2 and cos.shape[1] == HEAD_DIM, "RoPE table shape mismatch")
+        _need(step_in.numel() >= 5, "step_in size mismatch")
+        d = StepOneDesc(layers=self.layers.data_ptr(), embed=embed.data_ptr(), step_in=step_in.data_ptr(), kv=kv.data_ptr(),
+                        cos_table=cos.data_ptr(), sin_table=sin.data_ptr(), exchange=self.exchange.data_ptr(),
+                        h_out=h_out.data_ptr(), status=self.status.data_ptr(), bits=bits, n_layers=n_layers, dim=dim, ffn=ffn,
+                        n_heads=n_heads, n_kv=n_kv, slots=kv.shape[3], sigma=int(sigma), max_pos=cos.shape[0],
+                        vocab=embed.shape[0], eps=float(eps), scale=1.0 / math.sqrt(HEAD_DIM))
+        with torch.cuda.device(self.device):
+            rc = decode_lib().bonsai_decode_step_one(ctypes.byref(d), _stream(self.device))
+        _need(rc == 0, f"bonsai_decode_step_one failed with status {rc}")
 
 
 def kv_commit(kv: torch.Tensor, src_slot: int, dst_slot: int, n: int) -> None:

@@ -491,6 +491,31 @@ def fused_plan(model: "BonsaiDecoder", m: int) -> Optional[FusedPlan]:
     return plan
 
 
+def step_one(model: "BonsaiDecoder") -> Optional["decode_ops.StepOne"]:
+    """What runs all layers of a one-token step in one launch, or ``None`` where the separate launches do: shapes that
+    launch does not take, BONSAI_ONE_LAUNCH_STEP=0, or a form of the separate launches asked for by name
+    (BONSAI_FUSED_STEP, BONSAI_ATTENTION_ONE_LAUNCH)."""
+    by_name = any(name in os.environ for name in ("BONSAI_FUSED_STEP", "BONSAI_ATTENTION_ONE_LAUNCH"))
+    if os.environ.get("BONSAI_ONE_LAUNCH_STEP", "0" if by_name else "1") == "0":
+        return None
+    args = model.args
+    rows = []
+    for lw in model.layers:
+        packed = (lw.wqkv, lw.wo, lw.w_gu, lw.w_down)
+        norms = (lw.input_layernorm, lw.post_attention_layernorm, lw.q_norm, lw.k_norm)
+        tensors = [p.weight for p in packed] + [p.weight_scale for p in packed] + list(norms)
+        if any(not t.is_contiguous() for t in tensors) or any(t.dtype != torch.bfloat16 for t in tensors[4:]) \
+                or any(t.data_ptr() % (4 if 4 <= i < 8 else 16) for i, t in enumerate(tensors)) \
+                or any(p.bits != lw.wo.bits for p in packed):
+            return None
+        rows.append([t.data_ptr() for t in tensors])
+    shape = (model.layers[0].wo.bits, len(rows), args.dim, args.ffn_dim, args.n_heads, args.n_kv_heads)
+    if not model.embed.is_contiguous() or model.embed.data_ptr() % 16 or \
+            decode_ops.StepOne.exchange_bytes(shape, model.device) == 0:
+        return None
+    return decode_ops.StepOne(torch.tensor(rows, dtype=torch.int64).to(model.device), shape, model.device)
+
+
 def _fused(w: PackedLinear, m: int, stream: ctypes.c_void_p, *, act, act_aux, act_kind: int, out,
            epi: int, act_parts: int = 0, norm_w=None, eps: float = 0.0, residual=None, out_aux=None) -> None:
     d = ops.FusedGemvDesc(act=act.data_ptr(), act_aux=act_aux.data_ptr(),
@@ -509,8 +534,8 @@ def _fused(w: PackedLinear, m: int, stream: ctypes.c_void_p, *, act, act_aux, ac
 
 def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tensor, sigma: int,
                  rope: Tuple[torch.Tensor, torch.Tensor], logits_start: int, logits_end: int,
-                 threshold: float, head_mode: str = "native") -> None:
-    """Enqueue one width-``io.M`` step on the current stream.
+                 threshold: float, head_mode: str = "native", one: Optional["decode_ops.StepOne"] = None) -> None:
+    """Enqueue one width-``io.M`` step on the current stream; with ``one``, of width 1, all layers of it as one launch.
 
     ``kv`` is the shared buffer ``[2, n_layers, n_kv, slots, 128]``; the new rows go to
     slots ``sigma .. sigma+M-1``.  Logit rows ``[logits_start, logits_end)`` are projected
@@ -531,6 +556,11 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
         if rc != 0:
             raise RuntimeError(f"{what} failed with status {rc}")
 
+    if one is not None:
+        h = ws.h[0][:1]
+        one.enqueue(model.embed, io.step_in, kv, cos, sin, sigma, eps, h)
+        project_rows(model, ws, h, None, logits_end - logits_start, threshold, io.tokens_out, io.conf, io.accept, head_mode)
+        return
     plan = fused_plan(model, M)
     # wider blocks keep the ten-launch layer; BONSAI_ROPE_IN_ATTENTION=1 drops its q / k norm + RoPE
     # launch (same bits; measured slower at nine rows, where every workgroup of the attention

@@ -30,7 +30,7 @@ import torch
 
 from . import contracts, decode_ops, ops
 from .model import (PROMPT_BLOCK_MAX, BonsaiDecoder, PromptBuffers, StepIO, Workspace, enqueue_prompt_block,
-                    enqueue_step, project_rows, rope_tables)
+                    enqueue_step, project_rows, rope_tables, step_one)
 
 DEFAULT_SEGMENT_LADDER = (256, 1024, 4096)
 DEFAULT_M_SET = (1, 8, 9, 10, 12, 16, 17)
@@ -136,6 +136,8 @@ class CapturedGraph:
     P: int
     logits_start: int
     logits_end: int
+    one: Optional[decode_ops.StepOne] = None            # its layers are one launch
+    separate: Optional["CapturedGraph"] = None          # the same step as separate launches, captured when first needed
 
 
 class GraphAtlas:
@@ -179,10 +181,39 @@ class GraphAtlas:
         self._prompt: Optional[PromptBuffers] = None   # sized by the longest block so far
         self._positions: Optional[torch.Tensor] = None
         self.replays = 0
+        # one-token steps as one launch (model.step_one; False: not asked for yet).  Such a launch gives up when it does
+        # not get the whole device; what was queued since the last read is kept until it is known that none did, so that
+        # it can be queued again with the separate launches
+        self._one = False
+        self._queued: List[Tuple] = []
+        self._separate_for = 0      # replays that keep to the separate launches after one gave up
+        self._back_off = 64
 
     def synchronize(self) -> None:
         """Wait for everything queued on the atlas's device (the loops' timing fences)."""
         torch.cuda.synchronize(self.device)
+        self._settle()
+
+    # -- steps that gave up ----------------------------------------------------
+    def _settle(self) -> None:
+        """Everything queued has ended: queue it again if a one-launch step among it gave up."""
+        if not self._queued:
+            return
+        queued, self._queued = self._queued, []
+        if not self._one or self._one.failed[0] == 0:
+            return
+        self._one.reset()
+        self._separate_for, self._back_off = self._back_off, min(2 * self._back_off, 1 << 20)
+        for what, args in queued:
+            (what or self._replay)(*args)
+        torch.cuda.synchronize(self.device)
+
+    def _note(self, what, *args) -> None:
+        """Something queued behind a one-launch step; ``what`` is None for a replay."""
+        self._queued.append((what, args))
+        if len(self._queued) > 256:
+            torch.cuda.current_stream(self.device).synchronize()
+            self._settle()
 
     # -- KV ------------------------------------------------------------------
     def kv(self, sigma: int) -> torch.Tensor:
@@ -213,12 +244,17 @@ class GraphAtlas:
         if cache_len + n_accept > sigma:
             raise RuntimeError("KV commit would run past the history segment")
         decode_ops.kv_commit(self.kv(sigma), sigma + first_row, cache_len, n_accept)
+        if self._queued:
+            self._note(decode_ops.kv_commit, self.kv(sigma), sigma + first_row, cache_len, n_accept)
 
     def migrate_segment(self, src_sigma: int, dst_sigma: int, cache_len: int) -> None:
         """Copy live history to another segment's buffer (fast_runtime.py:510-521)."""
         if src_sigma == dst_sigma:
             return
-        self.kv(dst_sigma)[:, :, :, :cache_len].copy_(self.kv(src_sigma)[:, :, :, :cache_len])
+        source, target = self.kv(src_sigma)[:, :, :, :cache_len], self.kv(dst_sigma)[:, :, :, :cache_len]
+        target.copy_(source)
+        if self._queued:
+            self._note(target.copy_, source)
 
     # -- graphs --------------------------------------------------------------
     def get_graph(self, M: int, sigma: int, role: str) -> CapturedGraph:
@@ -244,7 +280,8 @@ class GraphAtlas:
                         continue
                     self.get_graph(M, sigma, role)
 
-    def _capture_one(self, M: int, sigma: int, role: str) -> CapturedGraph:
+    def _capture_one(self, *what) -> CapturedGraph:
+        """``what``: the arguments of ``_capture_one_impl``."""
         # The cyclic garbage collector must not run while a stream is capturing: if it finds
         # an unreachable atlas, it destroys that atlas's graphs in the middle of this capture,
         # which aborts the process.  Collect first, then keep the collector off until the
@@ -255,12 +292,12 @@ class GraphAtlas:
         gc.disable()
         try:
             with torch.inference_mode(False):
-                return self._capture_one_impl(M, sigma, role)
+                return self._capture_one_impl(*what)
         finally:
             if gc_was_enabled:
                 gc.enable()
 
-    def _capture_one_impl(self, M: int, sigma: int, role: str) -> CapturedGraph:
+    def _capture_one_impl(self, M: int, sigma: int, role: str, separate: bool = False) -> CapturedGraph:
         if role not in contracts.GRAPH_ROLES:
             raise ValueError(f"unsupported graph role: {role!r}")
         if role not in self.roles:
@@ -280,10 +317,15 @@ class GraphAtlas:
         # the closure holds the pieces, not the atlas: no reference cycle through the graphs
         model, workspace, rope, threshold = self.model, self.workspace, self.rope, self.threshold
         head_mode = HEAD_MODE_OF_ROLE[role]
+        one = None
+        if M == 1 and not separate:
+            if self._one is False:
+                self._one = step_one(model)
+            one = self._one
 
         def run():
             enqueue_step(model, workspace, io, kv, sigma, rope, ls, le, threshold,
-                         head_mode=head_mode)
+                         head_mode=head_mode, one=one)
 
         graph = None
         if self.use_graphs:
@@ -302,7 +344,7 @@ class GraphAtlas:
                 run()
                 io.out_host.copy_(io.out, non_blocking=True)
         cg = CapturedGraph(graph=graph, io=io, M=M, sigma=sigma, role=role, P=M - self.D,
-                           logits_start=ls, logits_end=le)
+                           logits_start=ls, logits_end=le, one=one)
         cg._eager = run
         return cg
 
@@ -315,6 +357,8 @@ class GraphAtlas:
         if n > sigma:
             raise RuntimeError("history does not fit the segment")
         kv = self.kv(sigma)
+        if self._queued:
+            self.synchronize()
         block = min(n, PROMPT_BLOCK_MAX)
         with torch.inference_mode(False), torch.cuda.device(self.device):
             if self._prompt is None or self._prompt.rows < block:
@@ -343,24 +387,35 @@ class GraphAtlas:
             raise ValueError("tokens / positions must have exactly M entries")
         if cache_len + M > g.sigma + M or cache_len > g.sigma:
             raise RuntimeError("history does not fit the segment")
-        desc = step_descriptor(g.role, M, self.D, cache_len, n_pend)
+        inputs = step_descriptor(g.role, M, self.D, cache_len, n_pend) + list(positions) + list(tokens)
+        self._replay(g, inputs)
+        self.replays += 1
+        if g.one is not None or self._queued:
+            self._note(None, g, inputs)
+
+    def _replay(self, g: CapturedGraph, inputs: Sequence[int]) -> None:
+        io = g.io
+        if g.one is not None and self._separate_for > 0:
+            self._separate_for -= 1
+            if g.separate is None:
+                g.separate = self._capture_one(g.M, g.sigma, g.role, True)
+            g = g.separate
         # the previous upload from this pinned buffer must have left the host first
         g.io.uploaded.synchronize()
-        host = g.io.step_in_host.numpy()
-        host[: 2 + M] = desc
-        host[2 + M: 2 + 2 * M] = positions
-        host[2 + 2 * M:] = tokens
+        g.io.step_in_host.numpy()[:] = inputs
         stream = torch.cuda.current_stream(self.device)
         if g.graph is not None:
             g.graph.replay()          # uploads, runs the step, downloads the results
-            g.io.uploaded.record(stream)
             g.io.downloaded = True
         else:
             g.io.step_in.copy_(g.io.step_in_host, non_blocking=True)
-            g.io.uploaded.record(stream)
             g._eager()
             g.io.downloaded = False
-        self.replays += 1
+        g.io.uploaded.record(stream)
+        if g.io is not io:            # the results belong where the caller's graph leaves them
+            io.out.copy_(g.io.out)
+            io.uploaded.record(stream)
+            io.downloaded = False
 
     def read_outputs(self, g: CapturedGraph) -> Tuple[np.ndarray, np.ndarray, int]:
         """One device-to-host copy + synchronisation: (argmax tokens, confidences,
@@ -377,6 +432,13 @@ class GraphAtlas:
         else:
             g.io.out_host.copy_(g.io.out, non_blocking=True)
             torch.cuda.current_stream(self.device).synchronize()
+        if self._queued:
+            if next(args[0] for what, args in reversed(self._queued) if what is None) is not g:
+                torch.cuda.current_stream(self.device).synchronize()   # the reader has not waited for the last of them
+            self._settle()
+            if not g.io.downloaded:
+                g.io.out_host.copy_(g.io.out, non_blocking=True)
+                torch.cuda.current_stream(self.device).synchronize()
         rows = g.logits_end - g.logits_start
         out = g.io.out_host.numpy()
         toks = out[:rows].copy()

@@ -154,6 +154,39 @@ int bonsai_decode_attention_rope_parts(const void *xqkv, const void *q_norm_w, c
                                        int M, int n_heads, int n_kv, int slots, int sigma,
                                        void *stream);
 
+/* All layers of a one-token step in one launch: what q|k|v projection, q/k norm + RoPE + KV write, attention,
+ * o projection, gate|up projection and down projection of every layer do, with the residual adds, norms, SiLU * up and
+ * quantisations between them (`Transformer.forward_sdlm_decode_graph_kernel`, src/bonsai_sft/gpu/model.py:1386-1403,
+ * up to the final norm).  Takes the embedding row of step_in's token, writes the token's keys and values to slot
+ * `sigma` of every layer and the residual stream behind the last layer to `h_out`.
+ *
+ * One workgroup per compute unit stays for the whole launch and waits for the others, so a launch needs all units of
+ * the device.  Waits are bounded: if the units are not there within 5 ms, *status (int32, pinned host or device memory,
+ * zeroed by the caller) becomes nonzero, h_out and the slot hold nothing useful, the launches queued behind do the same at once, and
+ * the exchange memory has to be reset before the next use; the step can then be repeated by other means.
+ *
+ *   layers    device array of n_layers records of 12 pointers: packed weights of q|k|v, o, gate|up and down, their
+ *             bf16 group scales in the same order, input and post-attention norm weights, q and k norm weights;
+ *             weights and norm weights on 16 bytes, scales on 4
+ *   step_in   int32 [5]: meta[0 .. 2] as above, position, token
+ *   kv        bf16 [2, n_layers, n_kv, slots, 128]
+ *   exchange  bonsai_decode_step_one_bytes(...) bytes on 128 bytes, prepared by bonsai_decode_step_one_reset; one
+ *             launch at a time may use it
+ * bonsai_decode_step_one_bytes returns 0 for shapes it does not take. */
+typedef struct bonsai_step_one_desc {
+    const void *layers, *embed;
+    const int32_t *step_in;
+    void *kv;
+    const void *cos_table, *sin_table;
+    void *exchange, *h_out;
+    int32_t *status;
+    int bits, n_layers, dim, ffn, n_heads, n_kv, slots, sigma, max_pos, vocab;
+    float eps, scale;
+} bonsai_step_one_desc;
+int64_t bonsai_decode_step_one_bytes(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv);
+int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange, void *stream);
+int bonsai_decode_step_one(const bonsai_step_one_desc *desc, void *stream);
+
 /* Copies n KV rows of every layer and kv head from slot src to slot dst inside one
  * shared buffer [2, n_layers, n_kv, slots, 128] bf16 (commit_kv / commit_kv_from_verify,
  * src/bonsai_sft/gpu/fast_runtime.py:467-508).  Source and destination ranges must
