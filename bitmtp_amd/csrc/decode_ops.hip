@@ -1615,6 +1615,7 @@ int rows_per_wave(int M) {
 }
 
 #include "step_one.hip.h"
+#include "step_block.hip.h"
 
 }  // namespace
 
@@ -1895,15 +1896,18 @@ extern "C" int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }
 
-extern "C" int bonsai_decode_step_one(const bonsai_step_one_desc *d, void *stream) {
+static bool step_args_ok(const bonsai_step_one_desc *d) {
     if (!d || !d->layers || !d->embed || !d->step_in || !d->kv || !d->cos_table || !d->sin_table || !d->exchange || !d->h_out ||
         !d->status)
-        return BONSAI_DECODE_ERR_ARG;
-    if (d->slots < 1 || d->sigma < 0 || d->sigma >= d->slots || d->max_pos < 1 || d->vocab < 1 || d->slots > (1 << 22) ||
-        (reinterpret_cast<uintptr_t>(d->exchange) & 127) || (reinterpret_cast<uintptr_t>(d->embed) & 15) ||
-        (reinterpret_cast<uintptr_t>(d->kv) & 15) || (reinterpret_cast<uintptr_t>(d->layers) & 7) ||
-        (reinterpret_cast<uintptr_t>(d->step_in) & 3) || (reinterpret_cast<uintptr_t>(d->h_out) & 3))
-        return BONSAI_DECODE_ERR_ARG;
+        return false;
+    return d->slots >= 1 && d->sigma >= 0 && d->sigma < d->slots && d->max_pos >= 1 && d->vocab >= 1 && d->slots <= (1 << 22) &&
+           (reinterpret_cast<uintptr_t>(d->exchange) & 127) == 0 && (reinterpret_cast<uintptr_t>(d->embed) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(d->kv) & 15) == 0 && (reinterpret_cast<uintptr_t>(d->layers) & 7) == 0 &&
+           (reinterpret_cast<uintptr_t>(d->step_in) & 3) == 0 && (reinterpret_cast<uintptr_t>(d->h_out) & 3) == 0;
+}
+
+extern "C" int bonsai_decode_step_one(const bonsai_step_one_desc *d, void *stream) {
+    if (!step_args_ok(d)) return BONSAI_DECODE_ERR_ARG;
     const int groups = cu_count();
     const step_one::Fit f = step_one::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, groups);
     if (f.build < 0) return BONSAI_DECODE_ERR_ARG;
@@ -1931,6 +1935,58 @@ extern "C" int bonsai_decode_step_one(const bonsai_step_one_desc *d, void *strea
     a.scale = d->scale;
     void *args[] = {&a};
     if (hipLaunchKernel(step_one::kernel_of(f.build), dim3(groups), dim3(step_one::kThreads), args, (size_t)f.lds,
+                        static_cast<hipStream_t>(stream)) != hipSuccess)
+        return BONSAI_DECODE_ERR_LAUNCH;
+    return BONSAI_DECODE_OK;
+}
+
+// ---- the same for blocks (step_block.hip.h) -------------------------------------------------
+extern "C" int64_t bonsai_decode_step_block_bytes(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv) {
+    const step_block::Fit f = step_block::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
+    return f.build < 0 ? 0 : f.bytes;
+}
+
+extern "C" int bonsai_decode_step_block_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange,
+                                              void *stream) {
+    const step_block::Fit f = step_block::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
+    if (f.build < 0 || !exchange || (reinterpret_cast<uintptr_t>(exchange) & 127)) return BONSAI_DECODE_ERR_ARG;
+    if (hipFuncSetAttribute(step_block::kernel_of(f.build), hipFuncAttributeMaxDynamicSharedMemorySize, f.lds) != hipSuccess)
+        return BONSAI_DECODE_ERR_LAUNCH;
+    hipLaunchKernelGGL(step_block::reset_kernel, dim3(256), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<step_block::v4u *>(exchange), (size_t)f.bytes / 16, (size_t)f.clear / 16);
+    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+}
+
+extern "C" int bonsai_decode_step_block(const bonsai_step_one_desc *d, int rows, void *stream) {
+    if (!step_args_ok(d) || rows < 1 || rows > step_block::kRows || d->sigma + rows > d->slots) return BONSAI_DECODE_ERR_ARG;
+    const int groups = cu_count();
+    const step_block::Fit f = step_block::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, groups);
+    if (f.build < 0) return BONSAI_DECODE_ERR_ARG;
+    step_block::Args a;
+    a.layers = static_cast<const step_one::Layer *>(d->layers);
+    a.embed = static_cast<const uint16_t *>(d->embed);
+    a.step_in = d->step_in;
+    a.kv = static_cast<uint16_t *>(d->kv);
+    a.cos_t = static_cast<const uint16_t *>(d->cos_table);
+    a.sin_t = static_cast<const uint16_t *>(d->sin_table);
+    a.exchange = static_cast<uint8_t *>(d->exchange);
+    a.h_out = static_cast<uint16_t *>(d->h_out);
+    a.status = d->status;
+    a.rows = rows;
+    a.n_layers = d->n_layers;
+    a.dim = d->dim;
+    a.ffn = d->ffn;
+    a.n_heads = d->n_heads;
+    a.n_kv = d->n_kv;
+    a.slots = d->slots;
+    a.sigma = d->sigma;
+    a.max_pos = d->max_pos;
+    a.vocab = d->vocab;
+    a.groups = groups;
+    a.eps = d->eps;
+    a.scale = d->scale;
+    void *args[] = {&a};
+    if (hipLaunchKernel(step_block::kernel_of(f.build), dim3(groups), dim3(step_one::kThreads), args, (size_t)f.lds,
                         static_cast<hipStream_t>(stream)) != hipSuccess)
         return BONSAI_DECODE_ERR_LAUNCH;
     return BONSAI_DECODE_OK;

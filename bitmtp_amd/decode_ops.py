@@ -91,6 +91,12 @@ def load_decode_kernel() -> None:
     lib.bonsai_decode_step_one_reset.restype = ci
     lib.bonsai_decode_step_one.argtypes = [ctypes.POINTER(StepOneDesc), vp]
     lib.bonsai_decode_step_one.restype = ci
+    lib.bonsai_decode_step_block_bytes.argtypes = [ci] * 6
+    lib.bonsai_decode_step_block_bytes.restype = ctypes.c_int64
+    lib.bonsai_decode_step_block_reset.argtypes = [ci] * 6 + [vp, vp]
+    lib.bonsai_decode_step_block_reset.restype = ci
+    lib.bonsai_decode_step_block.argtypes = [ctypes.POINTER(StepOneDesc), ci, vp]
+    lib.bonsai_decode_step_block.restype = ci
     _lib = lib
 
 
@@ -335,6 +341,8 @@ class StepOne:
     nonzero, once the launches queued so far have ended, if one of them did not get the whole device: nothing those
     launches wrote is of use, and ``reset`` makes the object ready again."""
 
+    NAME, MAX_ROWS = "bonsai_decode_step_one", 1
+
     def __init__(self, layers: torch.Tensor, shape, device):
         """``layers``: int64 ``[n_layers, 12]`` on the device; ``shape``: (bits, n_layers, dim, ffn, n_heads, n_kv)."""
         _check(layers, torch.int64, "layers")
@@ -347,36 +355,48 @@ class StepOne:
         self.failed = self.status.numpy()
         self.reset()
 
-    @staticmethod
-    def exchange_bytes(shape, device) -> int:
+    @classmethod
+    def exchange_bytes(cls, shape, device) -> int:
         """Size of the exchange memory; 0 for shapes that do not run as one launch."""
         with torch.cuda.device(device):
-            return int(decode_lib().bonsai_decode_step_one_bytes(*shape))
+            return int(getattr(decode_lib(), cls.NAME + "_bytes")(*shape))
 
     def reset(self) -> None:
         self.failed[0] = 0
         with torch.cuda.device(self.device):
-            rc = decode_lib().bonsai_decode_step_one_reset(*self.shape, _ptr(self.exchange), _stream(self.device))
-        _need(rc == 0, f"bonsai_decode_step_one_reset failed with status {rc}")
+            rc = getattr(decode_lib(), self.NAME + "_reset")(*self.shape, _ptr(self.exchange), _stream(self.device))
+        _need(rc == 0, f"{self.NAME}_reset failed with status {rc}")
+
+    def _launch(self, desc: StepOneDesc, rows: int) -> int:
+        return decode_lib().bonsai_decode_step_one(ctypes.byref(desc), _stream(self.device))
 
     def enqueue(self, embed: torch.Tensor, step_in: torch.Tensor, kv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                sigma: int, eps: float, h_out: torch.Tensor) -> None:
+                sigma: int, eps: float, h_out: torch.Tensor, rows: int = 1) -> None:
         bits, n_layers, dim, ffn, n_heads, n_kv = self.shape
         for t, name in ((embed, "embed"), (kv, "kv"), (cos, "cos"), (sin, "sin"), (h_out, "h_out")):
             _check(t, torch.bfloat16, name)
         _check(step_in, torch.int32, "step_in")
-        _need(embed.dim() == 2 and embed.shape[1] == dim and h_out.numel() >= dim, "embed / h_out shape mismatch")
+        _need(embed.dim() == 2 and embed.shape[1] == dim and h_out.numel() >= rows * dim, "embed / h_out shape mismatch")
         _need(kv.dim() == 5 and kv.shape[:3] == (2, n_layers, n_kv) and kv.shape[4] == HEAD_DIM, "kv shape mismatch")
         _need(cos.shape == sin.shape and cos.dim() == 2 and cos.shape[1] == HEAD_DIM, "RoPE table shape mismatch")
-        _need(step_in.numel() >= 5, "step_in size mismatch")
+        _need(1 <= rows <= self.MAX_ROWS and step_in.numel() >= 2 + 3 * rows, "step_in size mismatch")
         d = StepOneDesc(layers=self.layers.data_ptr(), embed=embed.data_ptr(), step_in=step_in.data_ptr(), kv=kv.data_ptr(),
                         cos_table=cos.data_ptr(), sin_table=sin.data_ptr(), exchange=self.exchange.data_ptr(),
                         h_out=h_out.data_ptr(), status=self.status.data_ptr(), bits=bits, n_layers=n_layers, dim=dim, ffn=ffn,
                         n_heads=n_heads, n_kv=n_kv, slots=kv.shape[3], sigma=int(sigma), max_pos=cos.shape[0],
                         vocab=embed.shape[0], eps=float(eps), scale=1.0 / math.sqrt(HEAD_DIM))
         with torch.cuda.device(self.device):
-            rc = decode_lib().bonsai_decode_step_one(ctypes.byref(d), _stream(self.device))
-        _need(rc == 0, f"bonsai_decode_step_one failed with status {rc}")
+            rc = self._launch(d, rows)
+        _need(rc == 0, f"{self.NAME} failed with status {rc}")
+
+
+class StepBlock(StepOne):
+    """The same for a block of up to 16 rows (``bonsai_decode_step_block``)."""
+
+    NAME, MAX_ROWS = "bonsai_decode_step_block", 16
+
+    def _launch(self, desc: StepOneDesc, rows: int) -> int:
+        return decode_lib().bonsai_decode_step_block(ctypes.byref(desc), rows, _stream(self.device))
 
 
 def kv_commit(kv: torch.Tensor, src_slot: int, dst_slot: int, n: int) -> None:

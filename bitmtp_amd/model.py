@@ -491,11 +491,11 @@ def fused_plan(model: "BonsaiDecoder", m: int) -> Optional[FusedPlan]:
     return plan
 
 
-def step_one(model: "BonsaiDecoder") -> Optional["decode_ops.StepOne"]:
-    """What runs all layers of a one-token step in one launch, or ``None`` where the separate launches do: shapes that
-    launch does not take, BONSAI_ONE_LAUNCH_STEP=0, or a form of the separate launches asked for by name
-    (BONSAI_FUSED_STEP, BONSAI_ATTENTION_ONE_LAUNCH)."""
-    by_name = any(name in os.environ for name in ("BONSAI_FUSED_STEP", "BONSAI_ATTENTION_ONE_LAUNCH"))
+def step_one(model: "BonsaiDecoder", form: type = decode_ops.StepOne) -> Optional["decode_ops.StepOne"]:
+    """What runs all layers of a step in one launch (``form``: ``StepOne`` or, up to 16 rows, ``StepBlock``), or ``None`` where the separate
+    launches do: shapes that launch does not take, BONSAI_ONE_LAUNCH_STEP=0, or a form of the separate launches asked for by
+    name (BONSAI_FUSED_STEP, BONSAI_ATTENTION_ONE_LAUNCH, BONSAI_ROPE_IN_ATTENTION)."""
+    by_name = any(name in os.environ for name in ("BONSAI_FUSED_STEP", "BONSAI_ATTENTION_ONE_LAUNCH", "BONSAI_ROPE_IN_ATTENTION"))
     if os.environ.get("BONSAI_ONE_LAUNCH_STEP", "0" if by_name else "1") == "0":
         return None
     args = model.args
@@ -511,9 +511,9 @@ def step_one(model: "BonsaiDecoder") -> Optional["decode_ops.StepOne"]:
         rows.append([t.data_ptr() for t in tensors])
     shape = (model.layers[0].wo.bits, len(rows), args.dim, args.ffn_dim, args.n_heads, args.n_kv_heads)
     if not model.embed.is_contiguous() or model.embed.data_ptr() % 16 or \
-            decode_ops.StepOne.exchange_bytes(shape, model.device) == 0:
+            form.exchange_bytes(shape, model.device) == 0:
         return None
-    return decode_ops.StepOne(torch.tensor(rows, dtype=torch.int64).to(model.device), shape, model.device)
+    return form(torch.tensor(rows, dtype=torch.int64).to(model.device), shape, model.device)
 
 
 def _fused(w: PackedLinear, m: int, stream: ctypes.c_void_p, *, act, act_aux, act_kind: int, out,
@@ -535,7 +535,7 @@ def _fused(w: PackedLinear, m: int, stream: ctypes.c_void_p, *, act, act_aux, ac
 def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tensor, sigma: int,
                  rope: Tuple[torch.Tensor, torch.Tensor], logits_start: int, logits_end: int,
                  threshold: float, head_mode: str = "native", one: Optional["decode_ops.StepOne"] = None) -> None:
-    """Enqueue one width-``io.M`` step on the current stream; with ``one``, of width 1, all layers of it as one launch.
+    """Enqueue one width-``io.M`` step on the current stream; with ``one``, all layers of it as one launch.
 
     ``kv`` is the shared buffer ``[2, n_layers, n_kv, slots, 128]``; the new rows go to
     slots ``sigma .. sigma+M-1``.  Logit rows ``[logits_start, logits_end)`` are projected
@@ -557,9 +557,9 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
             raise RuntimeError(f"{what} failed with status {rc}")
 
     if one is not None:
-        h = ws.h[0][:1]
-        one.enqueue(model.embed, io.step_in, kv, cos, sin, sigma, eps, h)
-        project_rows(model, ws, h, None, logits_end - logits_start, threshold, io.tokens_out, io.conf, io.accept, head_mode)
+        h = ws.h[0][:M]
+        one.enqueue(model.embed, io.step_in, kv, cos, sin, sigma, eps, h, M)
+        project_rows(model, ws, h[logits_start:logits_end], None, logits_end - logits_start, threshold, io.tokens_out, io.conf, io.accept, head_mode)
         return
     plan = fused_plan(model, M)
     # wider blocks keep the ten-launch layer; BONSAI_ROPE_IN_ATTENTION=1 drops its q / k norm + RoPE

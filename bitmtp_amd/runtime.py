@@ -181,10 +181,10 @@ class GraphAtlas:
         self._prompt: Optional[PromptBuffers] = None   # sized by the longest block so far
         self._positions: Optional[torch.Tensor] = None
         self.replays = 0
-        # one-token steps as one launch (model.step_one; False: not asked for yet).  Such a launch gives up when it does
-        # not get the whole device; what was queued since the last read is kept until it is known that none did, so that
-        # it can be queued again with the separate launches
-        self._one = False
+        # steps of one token and of up to sixteen as one launch (model.step_one; False: not asked for yet).  Such a launch
+        # gives up when it does not get the whole device; what was queued since the last read is kept until it is known
+        # that none did, so that it can be queued again with the separate launches
+        self._one = self._block = False
         self._queued: List[Tuple] = []
         self._separate_for = 0      # replays that keep to the separate launches after one gave up
         self._back_off = 64
@@ -200,9 +200,11 @@ class GraphAtlas:
         if not self._queued:
             return
         queued, self._queued = self._queued, []
-        if not self._one or self._one.failed[0] == 0:
+        failed = [one for one in (self._one, self._block) if one and one.failed[0] != 0]
+        if not failed:
             return
-        self._one.reset()
+        for one in failed:
+            one.reset()
         self._separate_for, self._back_off = self._back_off, min(2 * self._back_off, 1 << 20)
         for what, args in queued:
             (what or self._replay)(*args)
@@ -322,6 +324,10 @@ class GraphAtlas:
             if self._one is False:
                 self._one = step_one(model)
             one = self._one
+        elif M <= decode_ops.StepBlock.MAX_ROWS and not separate:
+            if self._block is False:
+                self._block = step_one(model, decode_ops.StepBlock)
+            one = self._block
 
         def run():
             enqueue_step(model, workspace, io, kv, sigma, rope, ls, le, threshold,

@@ -187,6 +187,14 @@ int64_t bonsai_decode_step_one_bytes(int bits, int n_layers, int dim, int ffn, i
 int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange, void *stream);
 int bonsai_decode_step_one(const bonsai_step_one_desc *desc, void *stream);
 
+/* The same for a block of 1 to 16 rows (draft and verify steps): step_in as a step descriptor of `rows` rows, then
+ * `rows` positions and `rows` tokens; h_out bf16 [rows, dim]; the rows' keys and values go to slots sigma ..
+ * sigma + rows - 1.  Exchange memory of its own size and preparation; the preparation also sets a function attribute, so
+ * make it outside stream capture. */
+int64_t bonsai_decode_step_block_bytes(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv);
+int bonsai_decode_step_block_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange, void *stream);
+int bonsai_decode_step_block(const bonsai_step_one_desc *desc, int rows, void *stream);
+
 /* Copies n KV rows of every layer and kv head from slot src to slot dst inside one
  * shared buffer [2, n_layers, n_kv, slots, 128] bf16 (commit_kv / commit_kv_from_verify,
  * src/bonsai_sft/gpu/fast_runtime.py:467-508).  Source and destination ranges must
