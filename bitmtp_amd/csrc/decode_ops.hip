@@ -1950,7 +1950,7 @@ extern "C" int bonsai_decode_step_block_reset(int bits, int n_layers, int dim, i
                                               void *stream) {
     const step_block::Fit f = step_block::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
     if (f.build < 0 || !exchange || (reinterpret_cast<uintptr_t>(exchange) & 127)) return BONSAI_DECODE_ERR_ARG;
-    if (hipFuncSetAttribute(step_block::kernel_of(f.build), hipFuncAttributeMaxDynamicSharedMemorySize, f.lds) != hipSuccess)
+    if (hipFuncSetAttribute(step_block::kernel_of(f.build), hipFuncAttributeMaxDynamicSharedMemorySize, step_block::kMostLds) != hipSuccess)
         return BONSAI_DECODE_ERR_LAUNCH;
     hipLaunchKernelGGL(step_block::reset_kernel, dim3(256), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<step_block::v4u *>(exchange), (size_t)f.bytes / 16, (size_t)f.clear / 16);

@@ -15,17 +15,18 @@
 // instructions little of that.  To a row phase: two bf16 values and a tag (step and layer) in eight bytes, which nothing but
 // the value itself makes valid; few readers wait for them.  From a row phase: int8 rows and, stored with them, their
 // multipliers, in one of two sets of places, one for each layer, of which a step empties the other; no int8 row holds -128.
-// One wave of a workgroup looks for the multipliers (in eight copies: all 256 looking at one line took 0.3 us longer, all
-// looking at the rows themselves 4 us a layer), then all read their stretch of the rows.  Waits are bounded and handled as
-// in the one-token form.
+// One wave of a workgroup looks for a row's announcement (in eight copies: all 256 looking at one line took 0.3 us longer);
+// then the others look for their stretch of the rows and it for the multipliers.  (All looking at the rows from the start
+// took 4 us a layer more; only behind the multipliers, 1 % more of a step.)  Waits are bounded and handled as in the
+// one-token form.
 //
 // Projections: 16 rows of weights x 128 of K x 16 tokens are two v_mfma_i32_16x16x64_i8, exact group sums.  A back wave
 // owns a stretch of K for all rows of the workgroup and reads that stretch of the tokens once; the waves' results meet in
 // LDS in the order of K.
 //
-// Layers of nine rows, 1.7B / 4B shape, us at a history of 24, 300, 1500: 934 / 961 / 1034 -> 642 / 681 / 803 and
-// 1521 / 1543 / 1657 -> 1033 / 1136 / 1321; two rows (1.7B) 808 / 815 / 896 -> 587 / 622 / 733; sixteen 982 / 1007 / 1084 ->
-// 712 / 746 / 876.
+// Layers of nine rows, 1.7B / 4B shape, us at a history of 24, 300, 1500: 934 / 961 / 1034 -> 642 / 677 / 792 and
+// 1521 / 1543 / 1657 -> 1027 / 1125 / 1316; two rows (1.7B) 812 / 818 / 900 -> 586 / 614 / 728; sixteen 987 / 1011 / 1089 ->
+// 712 / 745 / 866.
 #ifndef BONSAI_STEP_BLOCK_HIP_H
 #define BONSAI_STEP_BLOCK_HIP_H
 
@@ -64,6 +65,7 @@ constexpr int kRows = 16;                   // rows of a block at most
 constexpr int kMaxSplits = 32;              // attention parts per head
 constexpr int kPartBytes = (kHd + 4) * 8;   // of a (head, part, row): 128 sums, maximum, sum, each with its tag
 constexpr int kControlBytes = 256;
+constexpr int kMostLds = 159 * 1024;        // beside what is declared in place
 constexpr uint32_t kEmpty = 0x80808080u;    // int8 rows hold no -128, a multiplier is positive
 constexpr int kCopies = 8;                  // of the multipliers' line, one for each XCD's workgroups
 constexpr int kNap = 1;                     // of 64 cycles, between two looks
@@ -133,7 +135,7 @@ struct Places {   // byte offsets in the exchange memory
         g8 = o8 + kRows * n_heads * kHd;
         d8 = g8 + kRows * dim;
         s8 = d8 + kRows * ffn;
-        layer8 = s8 + 4 * kCopies * 128;   // a line a phase and copy
+        layer8 = s8 + 8 * kCopies * 128;   // a line a phase and copy, multipliers and announcements
         size = q8 + 2 * (int64_t)n_layers * layer8;   // two sets, in turn
     }
 };
@@ -189,7 +191,6 @@ __device__ __forceinline__ bool look_singly(T &x, uint64_t limit, Ask ask, Good 
         __builtin_amdgcn_sched_barrier(0);
         if (good(x)) return true;
         if (timed_out(spins, since, limit)) return false;
-        __builtin_amdgcn_s_sleep(1);
     }
 }
 // Words of eight values of a row: word tid + 256 i into v[i] (zero past the end).
@@ -256,9 +257,11 @@ __device__ __forceinline__ void put_word(const __amdgpu_buffer_rsrc_t row, int w
             return w & 2 ? __builtin_amdgcn_perm(r, u, 0x07060302u) : __builtin_amdgcn_perm(u, r, 0x05040100u);
         };
         const uint32_t a = transpose(w0), b = transpose(w1);
-        const int at = wanted(ok, (w >> 2) * 32 + (w & 3) * 4);
-        __builtin_amdgcn_raw_buffer_store_b32(a, row, at, 0, kDeviceScope);
-        __builtin_amdgcn_raw_buffer_store_b32(b, row, at, 16, kDeviceScope);
+        // four lanes' first pieces, then their second ones, eight neighbouring bytes a lane: a line is written at once
+        using First = std::integral_constant<int, 0x88>;    // quad_perm [0, 2, 0, 2]
+        using Second = std::integral_constant<int, 0xDD>;   // quad_perm [1, 3, 1, 3]
+        const uint32_t a0 = from(a, First{}), a1 = from(a, Second{}), b0 = from(b, First{}), b1 = from(b, Second{});
+        __builtin_amdgcn_raw_buffer_store_b64(w & 2 ? v2u{b0, b1} : v2u{a0, a1}, row, wanted(ok, w * 8), 0, kDeviceScope);
     }
 }
 
@@ -300,13 +303,17 @@ struct Taken {   // weights of a wave's stretch: S groups of T row tiles
 __device__ __forceinline__ int key_of(int row) { return (row >> 1) & 7; }
 
 // From memory to LDS without registers: lane i's `BYTES` at `off` go to lds + BYTES i.  In assembly because the compiler would
-// wait for them before the next read of any LDS; who reads what has come waits by vmcnt and a barrier.
+// wait for them before the next read of any LDS; who reads what has come waits by vmcnt and a barrier.  (m0 is read when the
+// load is issued, and is left as it was.)
 template <int BYTES>
 __device__ __forceinline__ void fetch(const v4u from, int off, uint32_t lds) {
+    uint32_t m0;
     if constexpr (BYTES == 16)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(from) : "memory", "m0");
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+                     : "=&s"(m0) : "s"(lds), "v"(off), "s"(from) : "memory");
     else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(from) : "memory", "m0");
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dword %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+                     : "=&s"(m0) : "s"(lds), "v"(off), "s"(from) : "memory");
 }
 __device__ __forceinline__ v4u words_of(uintptr_t p, int bytes) {   // a buffer resource for it
     return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(p >> 32) & 0xffffu)),
@@ -458,7 +465,19 @@ __device__ __forceinline__ void store_part(const Common &c, uint32_t tag) {
     if (d == 0)
         __builtin_amdgcn_raw_buffer_store_b128(v4u{__float_as_uint(m), tag, __float_as_uint(sum), tag}, r, row * kPartBytes + kHd * 8, 0, kDeviceScope);
 }
-// Row workgroup: the parts of row `wg`, all heads, into the raw row.
+// Row workgroup: beside the row's int8 values its multiplier ..
+__device__ __forceinline__ void raise(const Common &c, int phase, uint8_t *rows8, float s) {
+    const int tid = afresh((int)threadIdx.x);
+    if (tid < kCopies)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s), rsrc_of(rows8 + c.s8 + phase * kCopies * 128, kCopies * 128), tid * 128 + c.wg * 4,
+                                              0, kDeviceScope);
+}
+// .. and, half a microsecond or more before it, that the row is about to come.  The back waves look for the rows from then on:
+// all 256 workgroups' looking from the start takes the memory's bandwidth from what they look for, and looking only behind
+// the multipliers costs a look.
+__device__ __forceinline__ void announce(const Common &c, int phase, uint8_t *rows8) { raise(c, 4 + phase, rows8, 0.0f); }
+
+// The parts of row `wg`, all heads, into the raw row.
 __device__ __forceinline__ bool merge_parts(const Common &c, uint32_t tag, uint64_t limit) {
     const int tid = afresh((int)threadIdx.x);
     const int d = (tid & 63) * 2;
@@ -518,6 +537,35 @@ __device__ __forceinline__ bool merge_parts(const Common &c, uint32_t tag, uint6
     return true;
 }
 
+// Int8 rows' lines of N groups: lanes 8 r .. 8 r + 7 have rows r and r + 8.
+template <int N>
+struct Lines {
+    v4u v[N][2];
+    __device__ __forceinline__ bool look_for(const __amdgpu_buffer_rsrc_t rows, int k, int m_rows, int group, int groups, uint64_t limit) {
+        const int lane = afresh((int)threadIdx.x & 63);
+        return look_singly(*this, limit, [&](Lines &t) {
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int row = (lane >> 3) + 8 * h;
+                    t.v[j][h] = __builtin_amdgcn_raw_buffer_load_b128(rows, wanted(row < m_rows && j < groups, row * k + (group + j) * 128 + (lane & 7) * 16),
+                                                                      0, kDeviceScope);
+                }
+        }, [](const Lines &t) {
+            uint32_t least = ~0u;
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    least = min(min(least, t.v[j][h].x ^ kEmpty), t.v[j][h].y ^ kEmpty);
+                    least = min(min(least, t.v[j][h].z ^ kEmpty), t.v[j][h].w ^ kEmpty);
+                }
+            return (bool)__all(least != 0u);
+        });
+    }
+};
+
 // ---- back waves ---------------------------------------------------------------------------------
 __device__ __forceinline__ float silu_mul(float g, float u) { return step_one::silu_mul(g, u); }
 
@@ -570,39 +618,8 @@ __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
 #pragma unroll
         for (int from = 0; from < S; from += kAhead) {
             if (from >= groups) break;
-            v4u x[kAhead][2];
-            const auto there = [&](auto scope_c) -> bool {
-                uint32_t least = ~0u;
-#pragma unroll
-                for (int j = 0; j < kAhead; ++j)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        x[j][h] = __builtin_amdgcn_raw_buffer_load_b128(
-                            ra, wanted(put_row + 8 * h < c.m_rows && from + j < groups, (put_row + 8 * h) * sh.k + (first + from + j) * 128 + (lane & 7) * 16), 0,
-                            decltype(scope_c)::value);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int j = 0; j < kAhead; ++j)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const v4u v = x[j][h];
-                        least = min(min(least, v.x ^ kEmpty), v.y ^ kEmpty);
-                        least = min(min(least, v.z ^ kEmpty), v.w ^ kEmpty);
-                    }
-                return (bool)__all(least != 0u);
-            };
-            // The multipliers have been seen, and the values, stored before them, are nearly always there: a first look by way
-            // of the L2, which the XCD's other workgroups share, and only then past it.
-            if (!there(std::integral_constant<int, 0>{})) {
-                uint64_t since = 0;
-                for (int spins = 1; !there(std::integral_constant<int, kDeviceScope>{}); ++spins) {
-                    if (timed_out(spins, since, limit)) {
-                        if (lane == 0) c.meet.bad = 1;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-            }
+            Lines<kAhead> x;
+            if (!x.look_for(ra, sh.k, c.m_rows, first + from, groups - from, limit) && lane == 0) c.meet.bad = 1;
 #pragma unroll
             for (int two = 0; two < kAhead; two += 2) {
                 if (from + two >= groups) break;
@@ -611,7 +628,7 @@ __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         const int r = put_row + 8 * h;
-                        *reinterpret_cast<v4u *>(mine + j * 2048 + r * 128 + ((lane & 7) ^ key_of(r)) * 16) = x[two + j][h];
+                        *reinterpret_cast<v4u *>(mine + j * 2048 + r * 128 + ((lane & 7) ^ key_of(r)) * 16) = x.v[two + j][h];
                     }
                 v4i a0[2], a1[2];
 #pragma unroll
@@ -693,8 +710,8 @@ __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
         fill(c.o8, c.q_dim);
         fill(c.g8, a.dim);
         fill(c.d8, a.ffn);
-        if (t < 4 * kCopies)
-            __builtin_amdgcn_raw_buffer_store_b32(kEmpty, rsrc_of(c.q8_next + (size_t)l * c.layer8 + c.s8, 4 * kCopies * 128), t * 128 + c.wg * 4, 0, kDeviceScope);
+        if (t < 8 * kCopies)
+            __builtin_amdgcn_raw_buffer_store_b32(kEmpty, rsrc_of(c.q8_next + (size_t)l * c.layer8 + c.s8, 8 * kCopies * 128), t * 128 + c.wg * 4, 0, kDeviceScope);
     };
     for (int layer = 0; layer < a.n_layers; ++layer) {
         const int l = afresh_scalar(layer);
@@ -824,12 +841,6 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
     const auto in = (const __attribute__((address_space(1))) int32_t *)(uintptr_t)a.step_in;
     const uint32_t sees = (lane & 15) < c.m_rows ? (uint32_t)in[2 + (lane & 15)] : 0u;
 
-    // row phases: beside the row's int8 values its multiplier
-    const auto raise = [&](int phase, uint8_t *rows8, float s) {
-        if (tid < kCopies)
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s), rsrc_of(rows8 + c.s8 + phase * kCopies * 128, kCopies * 128), tid * 128 + c.wg * 4,
-                                                  0, kDeviceScope);
-    };
     const auto norm_row = [&](const v4u *v, const v4u *w, bool ok, uint8_t *rows8, int at8, int phase) -> bool {
         double ss = 0.0;
         float f[UD][8];
@@ -870,7 +881,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
 #pragma unroll
         for (int i = 0; i < UD; ++i)
             put_word<BITS>(rsrc_of(rows8 + at8 + c.wg * a.dim, a.dim), t + i * kFront, f[i], s, t + i * kFront < (a.dim >> 3));
-        raise(phase, rows8, s);
+        raise(c, phase, rows8, s);
         return true;
     };
     const auto top_of = [&](const v4u *v, auto units_c) {
@@ -900,7 +911,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
             unpack_word(v[i], f);
             put_word<BITS>(rsrc_of(rows8 + at8 + c.wg * k, k), t + i * kFront, f, s, t + i * kFront < (k >> 3));
         }
-        raise(phase, rows8, s);
+        raise(c, phase, rows8, s);
         return true;
     };
     // all rows' multipliers
@@ -912,12 +923,13 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
     const auto project = [&](int phase, const uint8_t *rows8, uint64_t limit, auto meanwhile) -> bool {
         uint32_t x;
         __syncthreads();   // the weights are there
+        if (!ROW && wave == 0 && !wait_rows(4 + phase, rows8, x, limit) && lane == 0) c.meet.bad = 1;
+        __syncthreads();
+        if (given_up(c.meet)) return false;
         if (wave == 0) {
             if (!wait_rows(phase, rows8, x, limit) && lane == 0) c.meet.bad = 1;
             if (lane < kRows) c.mult[lane] = __uint_as_float(x);
         }
-        __syncthreads();
-        if (given_up(c.meet)) return false;
         meanwhile();
         __syncthreads();   // the back waves' units
         if (given_up(c.meet)) return false;
@@ -944,6 +956,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
             } else {
                 ok = receive<UD>(c.h + (size_t)c.wg * a.dim * 4, a.dim >> 3, tag, row, limit);
             }
+            announce(c, 0, rows8);
             if (!norm_row(row, ln1, ok, rows8, 0, 0)) return false;
             ask_norm(ln2, cur, 1);
         }
@@ -1037,6 +1050,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
         }
         if constexpr (ROW) {
             if (!merge_parts(c, tag, limit) && lane == 0) c.meet.bad = 1;
+            announce(c, 1, rows8);
             __syncthreads();   // the raw row
             if (given_up(c.meet)) return false;
             v4u row[UQ];
@@ -1051,6 +1065,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
         if constexpr (ROW) {
             v4u row[UD];
             const bool ok = receive<UD>(c.h2 + (size_t)c.wg * a.dim * 4, a.dim >> 3, tag, row, limit);
+            announce(c, 2, rows8);
             if (!norm_row(row, ln2, ok, rows8, c.g8, 2)) return false;
         }
         const auto ahead = [&] {   // what the next layer needs
@@ -1069,6 +1084,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
         if constexpr (ROW) {
             v4u row[UF];
             const bool ok = receive<UF>(c.inner + (size_t)c.wg * a.ffn * 4, a.ffn >> 3, tag, row, limit);
+            announce(c, 3, rows8);
             if (!quant_row(row, std::integral_constant<int, UF>{}, a.ffn, ok, rows8, c.d8, 3)) return false;
         }
         if (c.rows_d && !project(3, rows8, limit, [] {})) return false;
@@ -1195,7 +1211,7 @@ inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, 
             break;
         }
     }
-    if (f.build >= 0 && f.lds > 159 * 1024) f.build = -1;
+    if (f.build >= 0 && f.lds > kMostLds) f.build = -1;
     f.bytes = at.size;
     f.clear = at.q8;   // control and tags
     return f;
