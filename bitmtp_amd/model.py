@@ -406,7 +406,11 @@ class StepIO:
     out_host: torch.Tensor       # pinned mirror
     uploaded: "torch.cuda.Event"  # recorded once step_in_host has been consumed: after the
                                   # eager upload, or after the replay of a graph that carries it
-    downloaded: bool = False      # the last replay already copied `out` into `out_host`
+    downloaded: bool = False      # the last replay copies `out` into `out_host` itself
+    arrived: bool = False         # .. and has: its results were seen there
+
+    #: what no word of ``out`` is: a host that waits for a replay's results looks for words that are still this
+    PENDING = -2 ** 31
 
     @property
     def meta(self) -> torch.Tensor:

@@ -406,11 +406,14 @@ class GraphAtlas:
             if g.separate is None:
                 g.separate = self._capture_one(g.M, g.sigma, g.role, True)
             g = g.separate
-        # the previous upload from this pinned buffer must have left the host first
-        g.io.uploaded.synchronize()
+        # the previous upload from this pinned buffer must have left the host first (as it has where results came back)
+        if not g.io.arrived:
+            g.io.uploaded.synchronize()
         g.io.step_in_host.numpy()[:] = inputs
         stream = torch.cuda.current_stream(self.device)
+        g.io.arrived = False
         if g.graph is not None:
+            g.io.out_host.numpy()[:] = StepIO.PENDING
             g.graph.replay()          # uploads, runs the step, downloads the results
             g.io.downloaded = True
         else:
@@ -427,13 +430,16 @@ class GraphAtlas:
         """One device-to-host copy + synchronisation: (argmax tokens, confidences,
         device-side accepted-prefix length) of the projected rows."""
         if g.io.downloaded:
-            # the event after the replay: polling it returns sooner than a blocking
-            # synchronisation wakes the thread up
-            ev = g.io.uploaded
+            # The results themselves, as the replay's last node writes them: the event behind it is ready 17 us later, and a
+            # blocking synchronisation wakes the thread up later still.
+            out = g.io.out_host.numpy()
             deadline = time.perf_counter() + 0.05
-            while not ev.query():
+            while True:
+                if not (out == StepIO.PENDING).any():
+                    g.io.arrived = True
+                    break
                 if time.perf_counter() > deadline:  # a replay is a millisecond: stop spinning
-                    ev.synchronize()
+                    g.io.uploaded.synchronize()
                     break
         else:
             g.io.out_host.copy_(g.io.out, non_blocking=True)

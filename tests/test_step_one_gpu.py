@@ -179,3 +179,27 @@ def test_several_steps_before_a_read():
     assert np.array_equal(a, out)
     atlas.replay(gb, [10], [10], 10)
     assert np.array_equal(b, atlas.read_outputs(gb)[0]) and torch.equal(kv, atlas.kv(256)[:, :, :, :10])
+
+
+def test_results_that_look_as_if_they_had_not_come():
+    """Results are waited for by a mark in the pinned buffer; where a word keeps that value, by the event behind the replay.
+    Replays without a read in between, and reads without a replay."""
+    from bitmtp_amd.model import StepIO
+    from bitmtp_amd.runtime import GraphAtlas
+    atlas = GraphAtlas(_model(2, 1024, 512, 8, 4), segment_ladder=(64,))
+    g = atlas.get_graph(9, 64, "verify")
+    tokens, positions = list(range(9)), list(range(4, 13))
+    atlas.replay(g, tokens, positions, 5)
+    want = [np.copy(x) for x in atlas.read_outputs(g)]
+    assert g.io.arrived
+    for marked in (False, True):
+        atlas.replay(g, [7] * 9, positions, 5)
+        atlas.replay(g, tokens, positions, 5)
+        assert not g.io.arrived
+        torch.cuda.synchronize()
+        if marked:
+            g.io.out_host[8] = StepIO.PENDING
+        for _ in range(2):
+            got = atlas.read_outputs(g)
+            assert g.io.arrived != marked
+            assert all(np.array_equal(x[:8], y[:8]) for x, y in zip(got[:2], want[:2])) and got[2] == want[2]
