@@ -1958,7 +1958,7 @@ extern "C" int bonsai_decode_step_block_reset(int bits, int n_layers, int dim, i
 }
 
 extern "C" int bonsai_decode_step_block(const bonsai_step_one_desc *d, int rows, void *stream) {
-    if (!step_args_ok(d) || rows < 1 || rows > step_block::kRows || d->sigma + rows > d->slots) return BONSAI_DECODE_ERR_ARG;
+    if (!step_args_ok(d) || rows < 2 || rows > step_block::kRows || d->sigma + rows > d->slots) return BONSAI_DECODE_ERR_ARG;
     const int groups = cu_count();
     const step_block::Fit f = step_block::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, groups);
     if (f.build < 0) return BONSAI_DECODE_ERR_ARG;

@@ -391,7 +391,7 @@ class StepOne:
 
 
 class StepBlock(StepOne):
-    """The same for a block of up to 16 rows (``bonsai_decode_step_block``)."""
+    """The same for a block of 2 to 16 rows (``bonsai_decode_step_block``)."""
 
     NAME, MAX_ROWS = "bonsai_decode_step_block", 16
 

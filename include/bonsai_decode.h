@@ -187,7 +187,7 @@ int64_t bonsai_decode_step_one_bytes(int bits, int n_layers, int dim, int ffn, i
 int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange, void *stream);
 int bonsai_decode_step_one(const bonsai_step_one_desc *desc, void *stream);
 
-/* The same for a block of 1 to 16 rows (draft and verify steps): step_in as a step descriptor of `rows` rows, then
+/* The same for a block of 2 to 16 rows (draft and verify steps): step_in as a step descriptor of `rows` rows, then
  * `rows` positions and `rows` tokens; h_out bf16 [rows, dim]; the rows' keys and values go to slots sigma ..
  * sigma + rows - 1.  Exchange memory of its own size and preparation; the preparation also sets a function attribute, so
  * make it outside stream capture. */

@@ -106,7 +106,7 @@ def test_argument_checks():
     good = dict(layers=0x1000, embed=0x2000, step_in=0x3000, kv=0x4000, cos_table=0x5000, sin_table=0x6000, exchange=0x7000,
                 h_out=0x8000, status=0x9000, bits=2, n_layers=3, dim=2048, ffn=6144, n_heads=16, n_kv=8, slots=64, sigma=32,
                 max_pos=64, vocab=100, eps=1e-6, scale=0.1)
-    for rows, bad in ((0, {}), (17, {}), (9, dict(layers=0)), (9, dict(status=0)), (9, dict(exchange=0x7040)), (9, dict(kv=0x4008)),
+    for rows, bad in ((0, {}), (1, {}), (17, {}), (9, dict(layers=0)), (9, dict(status=0)), (9, dict(exchange=0x7040)), (9, dict(kv=0x4008)),
                       (9, dict(embed=0x2008)), (9, dict(sigma=56)), (9, dict(sigma=-1)), (9, dict(dim=2000)), (9, dict(n_layers=2)),
                       (9, dict(n_heads=17)), (9, dict(bits=4))):
         d = {**good, **bad}
