@@ -287,23 +287,25 @@ rmsnorm_quant_kernel(const uint16_t *x, const uint16_t *residual, const uint16_t
     }
 }
 
-// inner = bf16( fp32(bf16(silu(gate))) * up ), gate = gu[m][0..F), up = gu[m][F..2F)
-template <int VPT>
+// SILU: inner = bf16( fp32(bf16(silu(gate))) * up ), gate = x[m][0..F), up = x[m][F..2F); otherwise inner = x[m][0..F).
+// Latency at few rows, bytes at many: 3001 rows of 9728 take 32.7 us with the activation (3.9 TB/s of 2 x 2 + 1 bytes an
+// element) and 18.9 without it (4.6 TB/s of 2 + 1), which is why a prompt's gate|up applies it.
+template <int VPT, bool SILU>
 __global__ void __launch_bounds__(kMaxProducerThreads)
-silu_mul_quant_kernel(const uint16_t *gu, int8_t *q, float *s, int F, int T) {
+row_quant_kernel(const uint16_t *x, int8_t *q, float *s, int F, int T) {
     __shared__ float max_scratch[kMaxProducerWaves];
     const int m = blockIdx.x;
     const int tid = threadIdx.x;
     const int nvec = F / 8;
-    const uint4 *grow = reinterpret_cast<const uint4 *>(gu + (size_t)m * 2 * F);
-    const uint4 *urow = reinterpret_cast<const uint4 *>(gu + (size_t)m * 2 * F + F);
+    const uint4 *grow = reinterpret_cast<const uint4 *>(x + (size_t)m * (SILU ? 2 : 1) * F);
+    const uint4 *urow = reinterpret_cast<const uint4 *>(x + (size_t)m * 2 * F + F);
     uint4 gr[VPT], ur[VPT];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int v = tid + i * T;
         const int vc = v < nvec ? v : 0;
         gr[i] = grow[vc];
-        ur[i] = urow[vc];
+        if (SILU) ur[i] = urow[vc];
     }
     float nf[VPT][8];
     float amax = 0.0f;
@@ -312,6 +314,14 @@ silu_mul_quant_kernel(const uint16_t *gu, int8_t *q, float *s, int F, int T) {
         const int v = tid + i * T;
         float g[8], u[8];
         unpack8_bf16(gr[i], g);
+        if constexpr (!SILU) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                nf[i][e] = g[e];
+                if (v < nvec) amax = fmaxf(amax, fabsf(nf[i][e]));
+            }
+            continue;
+        }
         unpack8_bf16(ur[i], u);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -369,9 +379,22 @@ extern "C" int bonsai_act_quant_int8(const void *x, int x_kind, int8_t *q, float
     if (M < 1 || K < 8 || K % 8 != 0) return BONSAI_ERR_ARG;
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (x_kind) {
-        case BONSAI_X_BF16:
-            hipLaunchKernelGGL(act_quant_kernel<BONSAI_X_BF16>, dim3(M), dim3(kThreads), 0, st, x, q, s, K);
+        case BONSAI_X_BF16: {
+            if (K > kMaxProducerK) {
+                hipLaunchKernelGGL(act_quant_kernel<BONSAI_X_BF16>, dim3(M), dim3(kThreads), 0, st, x, q, s, K);
+                break;
+            }
+            // read once and kept in registers, as many threads as vectors where a workgroup has them
+            const dim3 grid(M), block(producer_threads(K / 8));
+            const uint16_t *row = reinterpret_cast<const uint16_t *>(x);
+            switch (producer_vpt(K / 8)) {
+                case 1: hipLaunchKernelGGL((row_quant_kernel<1, false>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+                case 2: hipLaunchKernelGGL((row_quant_kernel<2, false>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+                case 4: hipLaunchKernelGGL((row_quant_kernel<4, false>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+                default: hipLaunchKernelGGL((row_quant_kernel<8, false>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+            }
             break;
+        }
         case BONSAI_X_F16:
             hipLaunchKernelGGL(act_quant_kernel<BONSAI_X_F16>, dim3(M), dim3(kThreads), 0, st, x, q, s, K);
             break;
@@ -436,10 +459,10 @@ extern "C" int bonsai_silu_mul_quant_int8(const void *gate_up, int8_t *q, float 
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t *gu = reinterpret_cast<const uint16_t *>(gate_up);
     switch (producer_vpt(nvec)) {
-        case 1: hipLaunchKernelGGL(silu_mul_quant_kernel<1>, grid, block, 0, st, gu, q, s, F, (int)block.x); break;
-        case 2: hipLaunchKernelGGL(silu_mul_quant_kernel<2>, grid, block, 0, st, gu, q, s, F, (int)block.x); break;
-        case 4: hipLaunchKernelGGL(silu_mul_quant_kernel<4>, grid, block, 0, st, gu, q, s, F, (int)block.x); break;
-        default: hipLaunchKernelGGL(silu_mul_quant_kernel<8>, grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        case 1: hipLaunchKernelGGL((row_quant_kernel<1, true>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        case 2: hipLaunchKernelGGL((row_quant_kernel<2, true>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        case 4: hipLaunchKernelGGL((row_quant_kernel<4, true>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        default: hipLaunchKernelGGL((row_quant_kernel<8, true>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
     }
     return hipGetLastError() == hipSuccess ? BONSAI_OK : BONSAI_ERR_LAUNCH;
 }

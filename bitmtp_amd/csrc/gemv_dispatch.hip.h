@@ -408,6 +408,29 @@ bool wide_default(const GemvProblem &q, bool g32, int n_cus, int lds_limit) {
     return v >= 0 && wide_estimate(v, q.M, q.N, q.K, n_cus) < narrow;
 }
 
+// gate|up of a wide block with silu(gate) * up behind it: out bf16 [M, N / 2]; -1 where the projection is not the wide
+// kernel's (the caller then runs projection and producer as two launches).
+template <int BITS>
+int launch_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K,
+                     hipStream_t stream) {
+    if (A == nullptr || B == nullptr || out == nullptr || s == nullptr || ws == nullptr) return 1;
+    if (M < 1 || N < 2 || N % 2 != 0 || K < kGroup || K % kGroup != 0) return 1;
+    if ((long)M * N > 0x7fffffffL / 2) return 1;
+    if (!operands_aligned(A, B, out, s, ws, OUT_BF16)) return 1;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 2;
+    LibState<BITS> &st = lib_state<BITS>();
+    const int rc = ensure_ready<BITS>(dev, stream);
+    if (rc != 0) return rc;
+    const int lds_limit = st.lds_limit[dev];
+    const MfmaTuning &mtu = mfma_tuning<BITS>();
+    const GemvProblem q{A, B, out, s, ws, M, N, K};
+    if (mtu.engine != 7 && !(mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(q, false, st.n_cus[dev], lds_limit))) return -1;
+    const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % kWideVariants
+                                                       : wide_pick<BITS>(M, N, K, st.n_cus[dev], lds_limit);
+    return v < 0 ? -1 : launch_wide<BITS>(v, q, OUT_BF16, 0, lds_limit, stream, true);
+}
+
 template <int BITS>
 int launch_gemv(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws,
                 int M, int N, int K, int out_kind, int scale_kind, hipStream_t stream) {

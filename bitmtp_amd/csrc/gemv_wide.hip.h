@@ -34,6 +34,10 @@
 // Arithmetic and rounding points are those of the other kernels: exact G, fp32 scale-accumulate with
 // groups in ascending order inside a slice, slices in order, division by s[m], bf16 RNE.
 //
+// gate|up of a prompt (`pairs`): a tile has gate rows and their up rows, and silu(gate) * up leaves the tile instead, 16 bytes
+// a lane as before: half the bytes out, and what follows reads half (3001 tokens of the 4B shape: 191.2 us as without it,
+// the activation launch behind it 32.7 -> 18.9; 256 tokens of the 1.7B one: 18.4 and 4.5 us, level).
+//
 // Block numbers go round the eight XCDs, so an XCD takes a contiguous range of tiles, eight token
 // tiles by consecutive row tiles: its L2 sees the same activations and the same rows again.
 //
@@ -100,9 +104,19 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     const int gm = tiles_m - mg * kWideTokenGroup < kWideTokenGroup ? tiles_m - mg * kWideTokenGroup : kWideTokenGroup;
     const int tn = rem / gm;
     const int m0 = (mg * kWideTokenGroup + rem - tn * gm) * S::kTokens;
-    const int n0 = tn * S::kRows;
+    // pairs: the tile's rows are kRows / 2 gate rows and, behind them, their up rows, of N / 2 each
+    const bool pairs = flags & 4;
+    constexpr int kHalf = S::kRows / 2;
+    const int n0 = tn * (pairs ? kHalf : S::kRows);
     const int mv = M - m0 < S::kTokens ? M - m0 : S::kTokens;
-    const int nv = N - n0 < S::kRows ? N - n0 : S::kRows;
+    const int nv = pairs ? (N / 2 - n0 < kHalf ? N / 2 - n0 : kHalf) : (N - n0 < S::kRows ? N - n0 : S::kRows);
+    // row r of the tile as a row of what rB and rS cover (a pair's matrix whole: rows past its end repeat the last)
+    const auto at_row = [&](int r) {
+        if (!pairs) return r;
+        const int p = r < kHalf ? r : r - kHalf;
+        return n0 + (p < nv ? p : nv - 1) + (r < kHalf ? 0 : N / 2);
+    };
+    const int base_row = pairs ? 0 : n0, rows_there = pairs ? N : nv;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -121,7 +135,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t *>(A + (size_t)m0 * K), 0, mv * K, kMxlBufferWord3);
     const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t *>(B + (size_t)n0 * row_bytes), 0, nv * row_bytes, kMxlBufferWord3);
+        const_cast<uint8_t *>(B + (size_t)base_row * row_bytes), 0, rows_there * row_bytes, kMxlBufferWord3);
 
     // ---- K slice of this set (whole 512-wide tiles where K has them: the slices of gemv_mxl.hip.h)
     const int unit = (G & 3) == 0 ? 4 : 1;
@@ -148,7 +162,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
 #pragma unroll
     for (int i = 0; i < BL; ++i) {
         const int task = stid + i * S::kSet;
-        b_off[i] = (uint32_t)(task / BCH) * (uint32_t)row_bytes + (uint32_t)((task % BCH) * 16);
+        b_off[i] = (uint32_t)at_row(task / BCH) * (uint32_t)row_bytes + (uint32_t)((task % BCH) * 16);
     }
     u32x4 ars[S::kAhead][AL][QW], brs[S::kAhead][BL];
     auto load = [&](auto &ar, auto &br, int g) {
@@ -193,14 +207,14 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     // ---- scales of the row block, transposed, and the multipliers
     if (!G32) {
         const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t *>(ws + (size_t)n0 * G), 0, nv * G * 2, kMxlBufferWord3);
+            const_cast<uint16_t *>(ws + (size_t)base_row * G), 0, rows_there * G * 2, kMxlBufferWord3);
         if (flags & 1) {  // whole quads of groups, aligned: a thread's quads are those of one row
             typedef unsigned int v2u __attribute__((ext_vector_type(2)));
             constexpr int kPerRow = S::kThreads / S::kRows;
             static_assert(kPerRow * S::kRows == S::kThreads, "threads divide among the rows");
             const int row = tid % S::kRows;
             for (int q = tid / S::kRows; q < G >> 2; q += kPerRow) {
-                const v2u v = __builtin_amdgcn_raw_buffer_load_b64(rS, row * (G * 2) + q * 8, 0, 0);
+                const v2u v = __builtin_amdgcn_raw_buffer_load_b64(rS, at_row(row) * (G * 2) + q * 8, 0, 0);
                 uint16_t *d = scales + (q * 4) * S::kRows + row;
                 d[0] = (uint16_t)v.x;
                 d[S::kRows] = (uint16_t)(v.x >> 16);
@@ -210,7 +224,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
         } else {
             for (int i = tid; i < S::kRows * G; i += S::kThreads) {
                 const int row = i / G, g = i - row * G;
-                scales[g * S::kRows + row] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rS, i * 2, 0, 0);
+                scales[g * S::kRows + row] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rS, (at_row(row) * G + g) * 2, 0, 0);
             }
         }
         // (the sums come out 64 times too large, mfma_unpack64: so does what divides them)
@@ -402,8 +416,25 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     if (out_f32) return;
     __syncthreads();
     // ---- the tile leaves in 16-byte pieces of whole rows
-    constexpr int CPR = S::kRows / 8;
     uint16_t *o = reinterpret_cast<uint16_t *>(out);
+    if (pairs) {   // .. as bf16(bf16(silu(gate)) * up)
+        constexpr int kPairs = kHalf / 8;
+        for (int i = tid; i < S::kTokens * kPairs; i += S::kThreads) {
+            const int m = i / kPairs, c = (i % kPairs) * 8;
+            if (m >= mv || c >= nv) continue;
+            const uint16_t *gate = reinterpret_cast<const uint16_t *>(tile + m * S::kOutPitch) + c, *up = gate + kHalf;
+            const u32x4 g = *reinterpret_cast<const u32x4 *>(gate), u = *reinterpret_cast<const u32x4 *>(up);
+            const auto two = [](uint32_t x, uint32_t y) {   // (the products are rounded already)
+                const float lo = silu_mul_bf16(__uint_as_float(x << 16), __uint_as_float(y << 16));
+                const float hi = silu_mul_bf16(__uint_as_float(x & 0xffff0000u), __uint_as_float(y & 0xffff0000u));
+                return (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
+            };
+            const u32x4 r = u32x4{two(g.x, u.x), two(g.y, u.y), two(g.z, u.z), two(g.w, u.w)};
+            *reinterpret_cast<u32x4 *>(o + (size_t)(m0 + m) * (N / 2) + n0 + c) = r;
+        }
+        return;
+    }
+    constexpr int CPR = S::kRows / 8;
     for (int i = tid; i < S::kTokens * CPR; i += S::kThreads) {
         const int m = i / CPR, c = (i % CPR) * 8;
         if (m >= mv || c >= nv) continue;
@@ -506,14 +537,19 @@ int wide_pick(int M, int N, int K, int n_cus, int lds_limit) {
 
 // Launches one problem as variant v; -1 when it does not fit (the caller falls back).
 template <int BITS>
-int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream) {
+int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream, bool pairs = false) {
     const WideVariant &k = wide_kernel<BITS>(v);
     if (!wide_fits<BITS>(v, q.K, lds_limit)) return -1;
-    const int tm = (q.M + k.tokens - 1) / k.tokens, tn = (q.N + k.rows - 1) / k.rows;
+    // pairs: N / 2 gate rows, N / 2 up rows -> silu(gate) * up, 16-byte pieces of whole rows; one resource over all of B
+    if (pairs && (out_kind != OUT_BF16 || q.N % 16 != 0 || (reinterpret_cast<uintptr_t>(q.out) & 15) != 0 ||
+                  (long)q.N * q.K * BITS / 8 > (1L << 30)))
+        return -1;
+    const int tile_rows = pairs ? k.rows / 2 : k.rows, all_rows = pairs ? q.N / 2 : q.N;
+    const int tm = (q.M + k.tokens - 1) / k.tokens, tn = (all_rows + tile_rows - 1) / tile_rows;
     if ((long)tm * tn > (1L << 28)) return -1;
     const int per = (tm * tn + kWideXcds - 1) / kWideXcds;
     const int flags = ((q.K / kGroup) % 4 == 0 && (reinterpret_cast<uintptr_t>(q.ws) & 7) == 0 ? 1 : 0) |
-                      (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0);
+                      (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0) | (pairs ? 4 : 0);
     const int variant = out_kind == OUT_G32 ? 2 : scale_kind;
     hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), k.lds(q.K), stream, q.A, q.B, q.out,
                        q.s, reinterpret_cast<const uint16_t *>(q.ws), q.M, q.N, q.K, out_kind == OUT_F32 ? 1 : 0, tm,

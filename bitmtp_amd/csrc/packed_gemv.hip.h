@@ -150,7 +150,7 @@ __device__ __forceinline__ float bf16_round_f32(float f) {
 }
 
 // bf16(bf16(silu(g)) * u) with silu through the hardware exp2 and reciprocal, exactly as
-// silu_mul_quant_kernel (act_quant.hip) evaluates it.
+// row_quant_kernel (act_quant.hip) evaluates it.
 __device__ __forceinline__ float silu_mul_bf16(float g, float u) {
     const float ex = __builtin_amdgcn_exp2f(g * -1.44269504088896341f);
     const float sg = bf16_round_f32(g * __builtin_amdgcn_rcpf(1.0f + ex));

@@ -369,8 +369,20 @@ PyObject *prefill_layers(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             STEP("o", project(o_q, o_s, x[2], x[3], proj, dim, q_dim));
             STEP("norm", bonsai_add_rmsnorm_quant_int8(h[cur], proj, x[9], eps, h[cur ^ 1], i8(a_q), f32(a_s), M, dim, st));
             cur ^= 1;
-            STEP("gate|up", project(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim));
-            STEP("silu", bonsai_silu_mul_quant_int8(gu, i8(i_q), f32(i_s), M, ffn, st));
+            // silu(gate) * up leaves with the projection where the wide kernel takes it: half the bytes
+            if (rc == 0) {
+                rc = (bits == 2 ? t2g128_gemv_silu : q1g128_gemv_silu)(i8(a_q), static_cast<const uint8_t *>(x[4]), gu, f32(a_s), x[5], M,
+                                                                       2 * ffn, dim, st);
+                if (rc == 0) {
+                    STEP("quantiser", bonsai_act_quant_int8(gu, BONSAI_X_BF16, i8(i_q), f32(i_s), M, ffn, st));
+                } else if (rc == -1) {
+                    rc = 0;
+                    STEP("gate|up", project(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim));
+                    STEP("silu", bonsai_silu_mul_quant_int8(gu, i8(i_q), f32(i_s), M, ffn, st));
+                } else {
+                    what = "gate|up";
+                }
+            }
             STEP("down", project(i_q, i_s, x[6], x[7], proj, dim, ffn));
 #undef STEP
         }

@@ -124,6 +124,11 @@ void q1g128_set_stream_tuning(int min_bytes, int wgs_per_cu) {
     t.wgs_per_cu = wgs_per_cu;
 }
 
+int q1g128_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K,
+                     void *stream) {
+    return launch_gemv_silu<1>(A, B, out, s, ws, M, N, K, static_cast<hipStream_t>(stream));
+}
+
 int q1g128_gemv_ex(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws,
                    int M, int N, int K, int out_kind, int scale_kind, void *stream) {
     return launch_gemv<1>(A, B, out, s, ws, M, N, K, out_kind, scale_kind,

@@ -94,6 +94,8 @@ def load_t2_kernel() -> None:
     lib.t2g128_int8xint2_linear.restype = None
     lib.t2g128_gemv_ex.argtypes = _GEMV_EX_ARGTYPES
     lib.t2g128_gemv_ex.restype = ctypes.c_int
+    lib.t2g128_gemv_silu.argtypes = [ctypes.c_void_p] * 5 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
+    lib.t2g128_gemv_silu.restype = ctypes.c_int
     lib.t2g128_init.argtypes = []
     lib.t2g128_init.restype = ctypes.c_int
     lib.t2g128_set_tuning.argtypes = [ctypes.c_int] * 3
@@ -130,6 +132,8 @@ def load_q1_kernel() -> None:
     lib.q1g128_w1a16_linear.restype = None
     lib.q1g128_gemv_ex.argtypes = _GEMV_EX_ARGTYPES
     lib.q1g128_gemv_ex.restype = ctypes.c_int
+    lib.q1g128_gemv_silu.argtypes = [ctypes.c_void_p] * 5 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
+    lib.q1g128_gemv_silu.restype = ctypes.c_int
     lib.q1g128_init.argtypes = []
     lib.q1g128_init.restype = ctypes.c_int
     lib.q1g128_set_tuning.argtypes = [ctypes.c_int] * 3

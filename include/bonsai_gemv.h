@@ -88,6 +88,14 @@ int t2g128_gemv_ex(const int8_t *A, const uint8_t *B, void *out, const float *s,
 int q1g128_gemv_ex(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws,
                    int M, int N, int K, int out_kind, int scale_kind, void *stream);
 
+/* gate|up of a prompt with the activation behind it: B and ws (bf16) hold the merged rows [gate (N/2 rows); up (N/2 rows)],
+ * out is bf16 [M, N/2] = bf16(bf16(silu(gate)) * up) of the bf16 projections, bit for bit what *_gemv_ex followed by the
+ * first half of bonsai_silu_mul_quant_int8 gives.  -1 (nothing launched) for what the wide-block kernel does not take. */
+int t2g128_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K,
+                     void *stream);
+int q1g128_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K,
+                     void *stream);
+
 /* ---- several GEMVs in one launch ------------------------------------------ */
 /* No counterpart in the reference, which launches one kernel per projection
  * (src/bonsai_sft/gpu/model.py:977,1006,1058,1062 through t2g128_kernels.cu:94-100).  A
