@@ -15,11 +15,13 @@
 //
 // K rows are staged as they are (pitch 272 bytes: 32 rows at one column meet every bank once), V
 // transposed 4 slots x 8 dims at a time in registers (16 v_perm per thread and chunk; pitch 136).  Two
-// buffers: the loads of chunk c + 2 are in flight and c + 1 is being parked while c is multiplied.
-// Both are shared by the four waves, which is what bounds the LDS traffic.  3001 rows of 32 query heads:
-// 103 us, 0.72 PFLOP/s over the slots seen; matrix cores and vector ALU are each busy for a third of the
-// cycles at 1.7 waves a SIMD: what bounds it is a wave's chain scores -> maximum -> exponentials -> product,
-// which two waves a SIMD that meet at a barrier every chunk do not cover.
+// buffers of each, shared by the four waves, which is what bounds the LDS traffic.  Keys run a chunk ahead of values:
+// chunk c + 1's scores are multiplied in front of chunk c's softmax, so that a wave's matrix instructions run beside its
+// exponentials; keys c + 2 and values c + 1 are parked meanwhile and the loads of the ones after them are in flight.
+// 3001 rows of 32 query heads: 105 us with each chunk in turn (matrix cores and vector ALU busy for a third of the cycles:
+// two waves a SIMD that meet at a barrier every chunk do not cover a wave's chain scores -> maximum -> exponentials ->
+// product), 96 so, 0.78 PFLOP/s over the slots seen.  (Half the scores beside the maximum and half beside the exponentials:
+// 97; the order of the two kinds of instructions prescribed: 103.)
 //
 // Longest rows first; the kv head is the low part of the block number, so that with eight of them an
 // XCD's L2 holds one head's history.
@@ -117,10 +119,8 @@ __device__ __forceinline__ void park_v(unsigned char *vb, const u32v4 (&v)[4], i
     }
 }
 
-// Chunk c, parked at kb / vb, into the running softmax of a wave's 32 queries.
-__device__ __forceinline__ void attend(const unsigned char *kb, const unsigned char *vb, const Pair &p, int c,
-                                       int masked_from, int col, int h, float scale_log2e, Softmax &x) {
-    f32x16 s[2];
+// Scores of a chunk's keys, parked at kb: s[t][r] is slot 32 t + 8 (r / 4) + 4 h + r % 4 of it.
+__device__ __forceinline__ void scores(const unsigned char *kb, const Pair &p, int col, int h, f32x16 (&s)[2]) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
@@ -131,7 +131,10 @@ __device__ __forceinline__ void attend(const unsigned char *kb, const unsigned c
             s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(*reinterpret_cast<const u32v4 *>(kp + 32 * j)),
                                                            frag(p.q[j]), s[t], 0, 0, 0);
     }
-    // s[t][r]: slot 64 c + 32 t + 8 (r / 4) + 4 h + r % 4
+}
+// Chunk c with its scores and its values, parked at vb, into the running softmax of a wave's 32 queries.
+__device__ __forceinline__ void take(f32x16 (&s)[2], const unsigned char *vb, const Pair &p, int c, int masked_from, int col,
+                                     int h, float scale_log2e, Softmax &x) {
     if (c >= masked_from) {
         const int rel = p.pos - c * kSlots - 4 * h;
 #pragma unroll
@@ -211,33 +214,53 @@ prefill_attn_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *
     const int k_off = k_slot * 2 * kHead + k_col * 16;
     const int v_off = v_slot * 2 * kHead + v_dim * 2;
     u32v4 kr[4], vr[4];
-    const auto load = [&](int c) {
-        const int s = c * kSlots * 2 * kHead;
+    const auto load_k = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) kr[i] = __builtin_amdgcn_raw_buffer_load_b128(rK, k_off + i * 16 * 2 * kHead, s, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rV, v_off + i * 2 * kHead, s, 0);
+        for (int i = 0; i < 4; ++i) kr[i] = __builtin_amdgcn_raw_buffer_load_b128(rK, k_off + i * 16 * 2 * kHead, c * kSlots * 2 * kHead, 0);
     };
-    const auto park = [&](int buf) {
-        unsigned char *kb = smem + buf * (kKBytes + kVBytes);
+    const auto load_v = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rV, v_off + i * 2 * kHead, c * kSlots * 2 * kHead, 0);
+    };
+    unsigned char *const kbs = smem, *const vbs = smem + 2 * kKBytes;
+    const auto park_k = [&](int c) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<u32v4 *>(kb + (k_slot + 16 * i) * kKPitch + k_col * 16) = kr[i];
-        park_v(kb + kKBytes, vr, v_dim, v_slot);
+            *reinterpret_cast<u32v4 *>(kbs + (c & 1) * kKBytes + (k_slot + 16 * i) * kKPitch + k_col * 16) = kr[i];
     };
+    const auto park = [&](int c) { park_v(vbs + (c & 1) * kVBytes, vr, v_dim, v_slot); };
+    // (loads for later chunks stay in flight)
+    const auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
+    // Keys are a chunk ahead of values: chunk c + 1's scores are multiplied while chunk c's softmax is computed.
     Softmax x;
-    load(0);
+    f32x16 s[2];
+    load_k(0);
+    load_v(0);
+    park_k(0);
     park(0);
-    if (w.chunks > 1) load(1);
+    if (w.chunks > 1) load_k(1);
+    meet();
+    scores(kbs, p, col, h, s);
+    if (w.chunks > 1) {
+        park_k(1);
+        load_v(1);
+    }
+    if (w.chunks > 2) load_k(2);
     for (int c = 0; c < w.chunks; ++c) {
-        const int buf = c & 1;
-        // chunk c is parked, chunk c - 1 no longer read (loads for later chunks stay in flight)
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (c + 1 < w.chunks) park(buf ^ 1);
-        if (c + 2 < w.chunks) load(c + 2);
-        const unsigned char *kb = smem + buf * (kKBytes + kVBytes);
-        attend(kb, kb + kKBytes, p, c, w.masked_from, col, h, scale_log2e, x);
+        // keys c + 1 and values c are parked; keys c and values c - 1 are no longer read
+        meet();
+        if (c + 1 < w.chunks) park(c + 1);
+        if (c + 2 < w.chunks) {
+            park_k(c + 2);
+            load_v(c + 2);
+        }
+        if (c + 3 < w.chunks) load_k(c + 3);
+        f32x16 ahead[2];
+        scores(kbs + ((c + 1) & 1) * kKBytes, p, col, h, ahead);   // (behind the last chunk: of what lies there, not used)
+        take(s, vbs + (c & 1) * kVBytes, p, c, w.masked_from, col, h, scale_log2e, x);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) s[t] = ahead[t];
     }
 
     const float l = x.l + __shfl_xor(x.l, 32);
@@ -300,7 +323,9 @@ prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint
         for (int i = 0; i < 4; ++i) park_v(vb, vr[i], v_dim + 32 * i, v_slot);
         bonsai_wave::order_lds();
         if (c + kWaves < rows.chunks) load(c + kWaves);
-        attend(kb, vb, p, c, rows.masked_from, col, h, scale_log2e, x);
+        f32x16 s[2];
+        scores(kb, p, col, h, s);
+        take(s, vb, p, c, rows.masked_from, col, h, scale_log2e, x);
     }
 
     // ---- the waves' results: [wave][register][lane], maxima and sums behind them
