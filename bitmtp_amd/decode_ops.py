@@ -9,7 +9,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
-from typing import Optional
+from typing import List, Optional, Sequence
 
 import torch
 
@@ -336,24 +336,35 @@ def prefill_attention_kernel() -> str:
 
 
 class StepOne:
-    """All layers of a one-token step in one launch (``bonsai_decode_step_one``): the addresses of a model's weights
-    and the exchange memory its workgroups hand rows over in.  One launch at a time may use an object.  ``status`` is
-    nonzero, once the launches queued so far have ended, if one of them did not get the whole device: nothing those
-    launches wrote is of use, and ``reset`` makes the object ready again."""
+    """All layers of a one-token step in one launch (``bonsai_decode_step_one``): a model's weights and the exchange
+    memory its workgroups hand rows over in.  One launch at a time may use that memory.  ``status`` is nonzero, once the
+    launches queued so far have ended, if one of them did not get the whole device: nothing those launches wrote is of
+    use, and ``reset`` makes the object ready again."""
 
     NAME, MAX_ROWS = "bonsai_decode_step_one", 1
 
-    def __init__(self, layers: torch.Tensor, shape, device):
-        """``layers``: int64 ``[n_layers, 12]`` on the device; ``shape``: (bits, n_layers, dim, ffn, n_heads, n_kv)."""
-        _check(layers, torch.int64, "layers")
-        _need(tuple(layers.shape) == (shape[1], 12), "layers must be [n_layers, 12]")
-        self.layers, self.shape, self.device = layers, tuple(shape), device
+    def __init__(self, weights: Sequence[Sequence[torch.Tensor]], shape, device, like: Optional["StepOne"] = None):
+        """``weights``: the twelve tensors of every layer in the order of the C entry's records; they are read at their
+        addresses, so the object holds them.  ``shape``: (bits, n_layers, dim, ffn, n_heads, n_kv).  ``like``: another
+        object, whose exchange memory this one shares where the shape is the same."""
+        _need(len(weights) == shape[1] and all(len(row) == 12 for row in weights), "weights must be [n_layers][12]")
+        self.weights = tuple(tuple(row) for row in weights)
+        self.addresses = self.addresses_of(weights)
+        self.layers = torch.tensor(self.addresses, dtype=torch.int64).to(device)
+        self.shape, self.device = tuple(shape), device
+        if like is not None and type(like) is type(self) and like.shape == self.shape and like.device == device:
+            self.exchange, self.status, self.failed = like.exchange, like.status, like.failed
+            return
         nbytes = self.exchange_bytes(shape, device)
         _need(nbytes > 0, "this shape does not run as one launch")
         self.exchange = torch.empty(nbytes, dtype=torch.uint8, device=device)
         self.status = torch.zeros(1, dtype=torch.int32).pin_memory()   # written by the device, only when it gives up
         self.failed = self.status.numpy()
         self.reset()
+
+    @staticmethod
+    def addresses_of(weights) -> List[List[int]]:
+        return [[t.data_ptr() for t in row] for row in weights]
 
     @classmethod
     def exchange_bytes(cls, shape, device) -> int:

@@ -18,10 +18,11 @@ PyTorch supplies device memory, the embedding gather and graph capture only.
 """
 from __future__ import annotations
 
+import copy
 import ctypes
 import os
 import math
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -234,6 +235,14 @@ class BonsaiDecoder:
         if self.head is None:
             return "bf16"
         return "t2" if self.head.bits == 2 else "q1"
+
+    def snapshot(self) -> "BonsaiDecoder":
+        """The same tensors in records of its own: what this model is given later does not reach it."""
+        other = copy.copy(self)
+        other.layers = [replace(lw, wqkv=replace(lw.wqkv), wo=replace(lw.wo), w_gu=replace(lw.w_gu), w_down=replace(lw.w_down))
+                        for lw in self.layers]
+        other.head = None if self.head is None else replace(self.head)
+        return other
 
     def _lm_head_weight(self) -> torch.Tensor:
         """The bf16 output matrix ``[vocab, dim]``: the tied embedding (which a packed head
@@ -495,29 +504,40 @@ def fused_plan(model: "BonsaiDecoder", m: int) -> Optional[FusedPlan]:
     return plan
 
 
-def step_one(model: "BonsaiDecoder", form: type = decode_ops.StepOne) -> Optional["decode_ops.StepOne"]:
+def step_one(model: "BonsaiDecoder", form: type = decode_ops.StepOne,
+             have: Optional["decode_ops.StepOne"] = None) -> Optional["decode_ops.StepOne"]:
     """What runs all layers of a step in one launch (``form``: ``StepOne`` or, up to 16 rows, ``StepBlock``), or ``None`` where the separate
     launches do: shapes that launch does not take, BONSAI_ONE_LAUNCH_STEP=0, or a form of the separate launches asked for by
-    name (BONSAI_FUSED_STEP, BONSAI_ATTENTION_ONE_LAUNCH, BONSAI_ROPE_IN_ATTENTION)."""
+    name (BONSAI_FUSED_STEP, BONSAI_ATTENTION_ONE_LAUNCH, BONSAI_ROPE_IN_ATTENTION).  ``have``: what an earlier call
+    returned; it is what this one returns too, if it reads the weights that the model has now."""
     by_name = any(name in os.environ for name in ("BONSAI_FUSED_STEP", "BONSAI_ATTENTION_ONE_LAUNCH", "BONSAI_ROPE_IN_ATTENTION"))
     if os.environ.get("BONSAI_ONE_LAUNCH_STEP", "0" if by_name else "1") == "0":
         return None
     args = model.args
+    bits = model.layers[0].wo.bits
+    dims = [(args.q_dim + 2 * args.kv_dim, args.dim), (args.dim, args.q_dim), (2 * args.ffn_dim, args.dim), (args.dim, args.ffn_dim)]
+    # the launch takes these for granted
+    shapes = ([(n, k * bits // 8) for n, k in dims] + [(n, k // GROUP_SIZE) for n, k in dims]
+              + [(args.dim,), (args.dim,), (HEAD_DIM,), (HEAD_DIM,)])
     rows = []
     for lw in model.layers:
         packed = (lw.wqkv, lw.wo, lw.w_gu, lw.w_down)
         norms = (lw.input_layernorm, lw.post_attention_layernorm, lw.q_norm, lw.k_norm)
         tensors = [p.weight for p in packed] + [p.weight_scale for p in packed] + list(norms)
-        if any(not t.is_contiguous() for t in tensors) or any(t.dtype != torch.bfloat16 for t in tensors[4:]) \
+        if any(not t.is_contiguous() or t.device != model.device for t in tensors) or any(t.dtype != torch.bfloat16 for t in tensors[4:]) \
+                or any(t.element_size() != 1 for t in tensors[:4]) or [tuple(t.shape) for t in tensors] != shapes \
                 or any(t.data_ptr() % (4 if 4 <= i < 8 else 16) for i, t in enumerate(tensors)) \
-                or any(p.bits != lw.wo.bits for p in packed):
+                or any(p.bits != bits for p in packed):
             return None
-        rows.append([t.data_ptr() for t in tensors])
-    shape = (model.layers[0].wo.bits, len(rows), args.dim, args.ffn_dim, args.n_heads, args.n_kv_heads)
-    if not model.embed.is_contiguous() or model.embed.data_ptr() % 16 or \
-            form.exchange_bytes(shape, model.device) == 0:
+        rows.append(tensors)
+    shape = (bits, len(rows), args.dim, args.ffn_dim, args.n_heads, args.n_kv_heads)
+    if not model.embed.is_contiguous() or model.embed.data_ptr() % 16:
         return None
-    return form(torch.tensor(rows, dtype=torch.int64).to(model.device), shape, model.device)
+    if have is not None and have.shape == shape and have.addresses == have.addresses_of(rows):
+        return have
+    if form.exchange_bytes(shape, model.device) == 0:
+        return None
+    return form(rows, shape, model.device, have)
 
 
 def _fused(w: PackedLinear, m: int, stream: ctypes.c_void_p, *, act, act_aux, act_kind: int, out,

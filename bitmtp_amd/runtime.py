@@ -137,6 +137,7 @@ class CapturedGraph:
     logits_start: int
     logits_end: int
     one: Optional[decode_ops.StepOne] = None            # its layers are one launch
+    model: Optional[BonsaiDecoder] = None               # the weights it was captured with (without a graph: the atlas's own model)
     separate: Optional["CapturedGraph"] = None          # the same step as separate launches, captured when first needed
 
 
@@ -181,10 +182,11 @@ class GraphAtlas:
         self._prompt: Optional[PromptBuffers] = None   # sized by the longest block so far
         self._positions: Optional[torch.Tensor] = None
         self.replays = 0
-        # steps of one token and of up to sixteen as one launch (model.step_one; False: not asked for yet).  Such a launch
-        # gives up when it does not get the whole device; what was queued since the last read is kept until it is known
-        # that none did, so that it can be queued again with the separate launches
-        self._one = self._block = False
+        # steps of one token and of up to sixteen as one launch (model.step_one), with the weights of the last capture or,
+        # without graphs, of the last step.  Such a launch gives up when it does not get the whole device; what was queued
+        # since the last read is kept until it is known that none did, so that it can be queued again with the separate
+        # launches
+        self._one = self._block = None
         self._queued: List[Tuple] = []
         self._separate_for = 0      # replays that keep to the separate launches after one gave up
         self._back_off = 64
@@ -200,7 +202,7 @@ class GraphAtlas:
         if not self._queued:
             return
         queued, self._queued = self._queued, []
-        failed = [one for one in (self._one, self._block) if one and one.failed[0] != 0]
+        failed = [one for one in {args[0].one for what, args in queued if what is None} if one is not None and one.failed[0] != 0]
         if not failed:
             return
         for one in failed:
@@ -299,7 +301,17 @@ class GraphAtlas:
             if gc_was_enabled:
                 gc.enable()
 
-    def _capture_one_impl(self, M: int, sigma: int, role: str, separate: bool = False) -> CapturedGraph:
+    def _one_launch(self, M: int) -> Optional[decode_ops.StepOne]:
+        """What runs the layers of an M-row step of the model, as its weights are now, in one launch."""
+        if M == 1:
+            self._one = step_one(self.model, have=self._one)
+            return self._one
+        if M <= decode_ops.StepBlock.MAX_ROWS:
+            self._block = step_one(self.model, decode_ops.StepBlock, self._block)
+            return self._block
+        return None
+
+    def _capture_one_impl(self, M: int, sigma: int, role: str, separate_of: Optional[CapturedGraph] = None) -> CapturedGraph:
         if role not in contracts.GRAPH_ROLES:
             raise ValueError(f"unsupported graph role: {role!r}")
         if role not in self.roles:
@@ -318,18 +330,12 @@ class GraphAtlas:
 
         # the closure holds the pieces, not the atlas: no reference cycle through the graphs
         model, workspace, rope, threshold = self.model, self.workspace, self.rope, self.threshold
+        if self.use_graphs:   # what is captured reads these tensors for good
+            model = model.snapshot() if separate_of is None else separate_of.model
         head_mode = HEAD_MODE_OF_ROLE[role]
-        one = None
-        if M == 1 and not separate:
-            if self._one is False:
-                self._one = step_one(model)
-            one = self._one
-        elif M <= decode_ops.StepBlock.MAX_ROWS and not separate:
-            if self._block is False:
-                self._block = step_one(model, decode_ops.StepBlock)
-            one = self._block
+        one = self._one_launch(M) if separate_of is None else None
 
-        def run():
+        def run(one):
             enqueue_step(model, workspace, io, kv, sigma, rope, ls, le, threshold,
                          head_mode=head_mode, one=one)
 
@@ -338,7 +344,7 @@ class GraphAtlas:
             side = torch.cuda.Stream(device=self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
             with torch.cuda.stream(side):
-                run()  # warm-up outside capture: lazy library set-up happens here
+                run(one)  # warm-up outside capture: lazy library set-up happens here
             torch.cuda.current_stream(self.device).wait_stream(side)
             torch.cuda.synchronize(self.device)
             # the graph carries its own upload of the step inputs and download of the results
@@ -347,10 +353,10 @@ class GraphAtlas:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 io.step_in.copy_(io.step_in_host, non_blocking=True)
-                run()
+                run(one)
                 io.out_host.copy_(io.out, non_blocking=True)
         cg = CapturedGraph(graph=graph, io=io, M=M, sigma=sigma, role=role, P=M - self.D,
-                           logits_start=ls, logits_end=le, one=one)
+                           logits_start=ls, logits_end=le, one=one, model=model)
         cg._eager = run
         return cg
 
@@ -394,6 +400,8 @@ class GraphAtlas:
         if cache_len + M > g.sigma + M or cache_len > g.sigma:
             raise RuntimeError("history does not fit the segment")
         inputs = step_descriptor(g.role, M, self.D, cache_len, n_pend) + list(positions) + list(tokens)
+        if g.graph is None and g.one is not None:
+            g.one = self._one_launch(M)
         self._replay(g, inputs)
         self.replays += 1
         if g.one is not None or self._queued:
@@ -404,7 +412,7 @@ class GraphAtlas:
         if g.one is not None and self._separate_for > 0:
             self._separate_for -= 1
             if g.separate is None:
-                g.separate = self._capture_one(g.M, g.sigma, g.role, True)
+                g.separate = self._capture_one(g.M, g.sigma, g.role, g)
             g = g.separate
         # the previous upload from this pinned buffer must have left the host first (as it has where results came back)
         if not g.io.arrived:
@@ -418,7 +426,7 @@ class GraphAtlas:
             g.io.downloaded = True
         else:
             g.io.step_in.copy_(g.io.step_in_host, non_blocking=True)
-            g._eager()
+            g._eager(g.one)
             g.io.downloaded = False
         g.io.uploaded.record(stream)
         if g.io is not io:            # the results belong where the caller's graph leaves them
