@@ -1110,7 +1110,7 @@ step_block_kernel(const Args a) {
     };
     const int rows_q = mine(sq, n_qkv), rows_o = mine(so, a.dim), rows_g = mine(sg, 2 * a.ffn), rows_d = mine(sd, a.dim);
     const auto in = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)a.step_in;
-    const int n = in[0];
+    const int n = in[0] < 0 ? 0 : (in[0] < a.sigma ? in[0] : a.sigma);   // as everywhere: a history within its slots
     // a head's slots: the history and, behind it, the block's rows, in parts of at least 64
     const int back_wg = groups - 1 - wg;   // the rows' workgroups have none
     const int kvh = back_wg % a.n_kv, unit = back_wg / a.n_kv, split = unit / gqa;

@@ -1034,7 +1034,7 @@ step_one_kernel(const Args a) {
     // memory) of one head, or a part of them.  A workgroup a query head rather than a kv head: the chain is shorter, and
     // the heads' second reads of keys and values come from their common L2.
     const auto in = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)a.step_in;
-    const int n = in[0];
+    const int n = in[0] < 0 ? 0 : (in[0] < a.sigma ? in[0] : a.sigma);   // as everywhere: a history within its slots
     const int kvh = wg % a.n_kv, unit = wg / a.n_kv, split = unit / gqa;
     const int head = kvh * gqa + unit - split * gqa;
     const int room = groups / (a.n_kv * gqa);

@@ -86,6 +86,33 @@ def test_long_histories(n_heads, n_kv, monkeypatch):
     _compare(_model(2, 1024, 1024, n_heads, n_kv), 4096, (300, 511, 512, 1000, 1023, 1024, 2047, 3333, 4095), monkeypatch)
 
 
+@pytest.mark.parametrize("width", [1, 9])
+def test_history_lengths_outside_the_segment(width):
+    """``cache_len`` below 0 is an empty history and above the segment a full one, as for every other attention kernel."""
+    from bitmtp_amd.runtime import GraphAtlas, step_descriptor
+    model, sigma = _model(2, 1024, 512, 8, 4), 200
+    atlas = GraphAtlas(model, segment_ladder=(sigma,))
+    g = atlas.get_graph(width, sigma, "ar")
+    assert g.one is not None
+    kv = atlas.kv(sigma)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    hist = (torch.randn(tuple(kv.shape), generator=gen, device=DEV) * 0.5).to(torch.bfloat16)
+    outs = {}
+    for n in (0, -1, -1000, -2 ** 31, sigma, sigma + 1, sigma + 70, 2 ** 31 - 1):
+        kv.copy_(hist)
+        inputs = [n] + step_descriptor("ar", width, model.args.block_size, 0)[1:] + list(range(width)) + list(range(width))
+        g.io.step_in.copy_(torch.tensor(inputs, dtype=torch.int32))
+        h = atlas.workspace.h[0][:width]
+        g.one.enqueue(model.embed, g.io.step_in, kv, *atlas.rope, sigma, 1e-6, h, width)
+        torch.cuda.synchronize()
+        assert g.one.failed[0] == 0
+        outs[n] = (h.clone(), kv.clone())
+    for n, (h, after) in outs.items():
+        want = outs[0 if n < 0 else min(n, sigma)]
+        assert torch.equal(h, want[0]) and torch.equal(after, want[1]), n
+    assert not torch.equal(outs[0][0], outs[sigma][0])
+
+
 def test_shapes_that_keep_the_separate_launches(monkeypatch):
     from bitmtp_amd import decode_ops
     from bitmtp_amd.model import step_one
