@@ -1616,6 +1616,7 @@ int rows_per_wave(int M) {
 
 #include "step_one.hip.h"
 #include "step_block.hip.h"
+#include "step_finish.hip.h"
 
 }  // namespace
 
@@ -1880,19 +1881,18 @@ extern "C" int bonsai_decode_attention_rope_parts(const void *xqkv, const void *
 }
 
 // ---- one launch for all layers of a one-token step (step_one.hip.h) ------------------------
+// Behind the exchange memory lie the rows of a step that is done again (step_finish.hip.h).
 extern "C" int64_t bonsai_decode_step_one_bytes(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv) {
     const step_one::Fit f = step_one::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
-    return f.build < 0 ? 0 : f.bytes;
+    return f.build < 0 ? 0 : f.bytes + step_finish::Places(1, dim, ffn, n_heads, n_kv).size;
 }
 
 extern "C" int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange,
                                             void *stream) {
     const step_one::Fit f = step_one::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
     if (f.build < 0 || !exchange || (reinterpret_cast<uintptr_t>(exchange) & 127)) return BONSAI_DECODE_ERR_ARG;
-    const step_one::Rows lay(dim, ffn, n_heads, n_kv);
-    const size_t from = step_one::kControlBytes / 16, to = from + (size_t)2 * n_layers * lay.size / 16;
     hipLaunchKernelGGL(step_one::exchange_reset_kernel, dim3(256), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       static_cast<step_one::v4u *>(exchange), (size_t)f.bytes / 16, from, to);
+                       static_cast<step_one::v4u *>(exchange), (size_t)f.bytes / 16, (size_t)step_one::kControlBytes / 16, (size_t)f.marked / 16);
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }
 
@@ -1906,12 +1906,8 @@ static bool step_args_ok(const bonsai_step_one_desc *d) {
            (reinterpret_cast<uintptr_t>(d->step_in) & 3) == 0 && (reinterpret_cast<uintptr_t>(d->h_out) & 3) == 0;
 }
 
-extern "C" int bonsai_decode_step_one(const bonsai_step_one_desc *d, void *stream) {
-    if (!step_args_ok(d)) return BONSAI_DECODE_ERR_ARG;
-    const int groups = cu_count();
-    const step_one::Fit f = step_one::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, groups);
-    if (f.build < 0) return BONSAI_DECODE_ERR_ARG;
-    step_one::Args a;
+template <class Args>
+static void step_args(Args &a, const bonsai_step_one_desc *d) {
     a.layers = static_cast<const step_one::Layer *>(d->layers);
     a.embed = static_cast<const uint16_t *>(d->embed);
     a.step_in = d->step_in;
@@ -1930,20 +1926,62 @@ extern "C" int bonsai_decode_step_one(const bonsai_step_one_desc *d, void *strea
     a.sigma = d->sigma;
     a.max_pos = d->max_pos;
     a.vocab = d->vocab;
-    a.groups = groups;
     a.eps = d->eps;
     a.scale = d->scale;
+}
+
+static bool final_norm_ok(const bonsai_step_one_desc *d, int rows) {
+    if (d->norm_rows == 0) return true;
+    const auto on = [](const void *p, uintptr_t bytes) { return p != nullptr && (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; };
+    return d->norm_rows > 0 && d->norm_first >= 0 && d->norm_rows <= rows - d->norm_first && on(d->norm_w, 16) && on(d->h_out, 16) &&
+           (d->norm_out ? on(d->norm_out, 16) : on(d->norm_q, 8) && on(d->norm_s, 4));
+}
+
+// The step's own launch and, behind it, the one that finishes it.
+template <class Args, class Fit>
+static int launch_step(const bonsai_step_one_desc *d, int rows, const void *kernel, Args &a, const Fit &f, size_t mark_from, uint32_t mark,
+                       hipStream_t stream) {
+    const auto ticks = [](int wait, uint32_t by_default) { return wait == 0 ? by_default : (wait < 0 ? 0u : (uint32_t)wait); };
+    step_args(a, d);
+    a.groups = cu_count();
+    a.first_wait = ticks(d->first_wait, step_one::kStartTicks);
+    a.later_wait = ticks(d->later_wait, step_one::kRunTicks);
     void *args[] = {&a};
-    if (hipLaunchKernel(step_one::kernel_of(f.build), dim3(groups), dim3(step_one::kThreads), args, (size_t)f.lds,
-                        static_cast<hipStream_t>(stream)) != hipSuccess)
+    if (hipLaunchKernel(kernel, dim3(a.groups), dim3(step_one::kThreads), args, (size_t)f.lds, stream) != hipSuccess)
         return BONSAI_DECODE_ERR_LAUNCH;
-    return BONSAI_DECODE_OK;
+    step_finish::Args b;
+    step_args(b, d);
+    b.rows_at = b.exchange + f.bytes;
+    b.words = (uint32_t)(f.bytes / 16);
+    b.mark_from = (uint32_t)(mark_from / 16);
+    b.mark_to = (uint32_t)(f.marked / 16);
+    b.mark = mark;
+    b.rows = rows;
+    b.norm_w = static_cast<const uint16_t *>(d->norm_w);
+    b.norm_q = static_cast<int8_t *>(d->norm_q);
+    b.norm_s = d->norm_s;
+    b.norm_out = static_cast<uint16_t *>(d->norm_out);
+    b.norm_first = d->norm_first;
+    b.norm_rows = d->norm_rows;
+    if (d->bits == 2)
+        hipLaunchKernelGGL(step_finish::finish_kernel<2>, dim3(step_finish::kGroups), dim3(step_finish::kThreads), 0, stream, b);
+    else
+        hipLaunchKernelGGL(step_finish::finish_kernel<1>, dim3(step_finish::kGroups), dim3(step_finish::kThreads), 0, stream, b);
+    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+}
+
+extern "C" int bonsai_decode_step_one(const bonsai_step_one_desc *d, void *stream) {
+    if (!step_args_ok(d) || !final_norm_ok(d, 1)) return BONSAI_DECODE_ERR_ARG;
+    const step_one::Fit f = step_one::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, cu_count());
+    if (f.build < 0) return BONSAI_DECODE_ERR_ARG;
+    step_one::Args a;
+    return launch_step(d, 1, step_one::kernel_of(f.build), a, f, step_one::kControlBytes, step_one::kEmpty, static_cast<hipStream_t>(stream));
 }
 
 // ---- the same for blocks (step_block.hip.h) -------------------------------------------------
 extern "C" int64_t bonsai_decode_step_block_bytes(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv) {
     const step_block::Fit f = step_block::fit(bits, n_layers, dim, ffn, n_heads, n_kv, cu_count());
-    return f.build < 0 ? 0 : f.bytes;
+    return f.build < 0 ? 0 : f.bytes + step_finish::Places(step_block::kRows, dim, ffn, n_heads, n_kv).size;
 }
 
 extern "C" int bonsai_decode_step_block_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange,
@@ -1958,38 +1996,13 @@ extern "C" int bonsai_decode_step_block_reset(int bits, int n_layers, int dim, i
 }
 
 extern "C" int bonsai_decode_step_block(const bonsai_step_one_desc *d, int rows, void *stream) {
-    if (!step_args_ok(d) || rows < 2 || rows > step_block::kRows || d->sigma + rows > d->slots) return BONSAI_DECODE_ERR_ARG;
-    const int groups = cu_count();
-    const step_block::Fit f = step_block::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, groups);
+    if (!step_args_ok(d) || rows < 2 || rows > step_block::kRows || d->sigma + rows > d->slots || !final_norm_ok(d, rows))
+        return BONSAI_DECODE_ERR_ARG;
+    const step_block::Fit f = step_block::fit(d->bits, d->n_layers, d->dim, d->ffn, d->n_heads, d->n_kv, cu_count());
     if (f.build < 0) return BONSAI_DECODE_ERR_ARG;
     step_block::Args a;
-    a.layers = static_cast<const step_one::Layer *>(d->layers);
-    a.embed = static_cast<const uint16_t *>(d->embed);
-    a.step_in = d->step_in;
-    a.kv = static_cast<uint16_t *>(d->kv);
-    a.cos_t = static_cast<const uint16_t *>(d->cos_table);
-    a.sin_t = static_cast<const uint16_t *>(d->sin_table);
-    a.exchange = static_cast<uint8_t *>(d->exchange);
-    a.h_out = static_cast<uint16_t *>(d->h_out);
-    a.status = d->status;
     a.rows = rows;
-    a.n_layers = d->n_layers;
-    a.dim = d->dim;
-    a.ffn = d->ffn;
-    a.n_heads = d->n_heads;
-    a.n_kv = d->n_kv;
-    a.slots = d->slots;
-    a.sigma = d->sigma;
-    a.max_pos = d->max_pos;
-    a.vocab = d->vocab;
-    a.groups = groups;
-    a.eps = d->eps;
-    a.scale = d->scale;
-    void *args[] = {&a};
-    if (hipLaunchKernel(step_block::kernel_of(f.build), dim3(groups), dim3(step_one::kThreads), args, (size_t)f.lds,
-                        static_cast<hipStream_t>(stream)) != hipSuccess)
-        return BONSAI_DECODE_ERR_LAUNCH;
-    return BONSAI_DECODE_OK;
+    return launch_step(d, rows, step_block::kernel_of(f.build), a, f, (size_t)f.clear, step_block::kEmpty, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int bonsai_kv_commit(void *kv, int n_layers, int n_kv, int slots, int src_slot,

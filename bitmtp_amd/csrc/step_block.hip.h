@@ -41,8 +41,6 @@ using step_one::kBackWaves;
 using step_one::kFront;
 using step_one::kFrontWaves;
 using step_one::kOob;
-using step_one::kRunTicks;
-using step_one::kStartTicks;
 using step_one::kThreads;
 using step_one::Layer;
 using step_one::Meet;
@@ -50,7 +48,6 @@ using step_one::multiplier;
 using step_one::pair16;
 using step_one::pair32;
 using step_one::rsrc_of;
-using step_one::timed_out;
 using step_one::top_of_64;
 using step_one::unpack_word;
 using step_one::v2u;
@@ -82,6 +79,7 @@ struct Args {
     int32_t *status;
     int rows, n_layers, dim, ffn, n_heads, n_kv, slots, sigma, max_pos, vocab, groups;
     float eps, scale;
+    uint32_t first_wait, later_wait;
 };
 
 // ---- sizes --------------------------------------------------------------------------------
@@ -158,11 +156,18 @@ struct Lds {
 __device__ __forceinline__ void hand_over(const __amdgpu_buffer_rsrc_t rows, int value, uint32_t d, uint32_t tag) {
     __builtin_amdgcn_raw_buffer_store_b64(v2u{d, tag}, rows, value * 4, 0, kDeviceScope);
 }
+// (The check of the limit on its own, before the spins: with first_spin of step_one.hip.h in its place, which is right as
+// well, a nine-row step of the 1.7B shape takes 643 us instead of 612.  A one-token step has it the other way round: 396
+// with first_spin, 401 with this.)
+__device__ __forceinline__ bool timed_out(int spins, uint32_t &since, uint32_t limit) {
+    if (limit == 0) return true;
+    return step_one::timed_out(spins, since, limit);
+}
 // Looks until good(x), two looks under way, half of one's time apart: for what few look at.
 template <class T, class Ask, class Good>
-__device__ __forceinline__ bool look(T &x, uint64_t limit, Ask ask, Good good) {
+__device__ __forceinline__ bool look(T &x, uint32_t limit, Ask ask, Good good) {
     T y;
-    uint64_t since = 0;
+    uint32_t since = 0;
     ask(x);
     for (int spins = 1;; ++spins) {
         __builtin_amdgcn_s_sleep(kNap);
@@ -183,8 +188,8 @@ __device__ __forceinline__ bool look(T &x, uint64_t limit, Ask ask, Good good) {
 }
 // .. and one, for what takes many registers.
 template <class T, class Ask, class Good>
-__device__ __forceinline__ bool look_singly(T &x, uint64_t limit, Ask ask, Good good) {
-    uint64_t since = 0;
+__device__ __forceinline__ bool look_singly(T &x, uint32_t limit, Ask ask, Good good) {
+    uint32_t since = 0;
     for (int spins = 1;; ++spins) {
         asm volatile("" ::: "memory");
         ask(x);
@@ -195,7 +200,7 @@ __device__ __forceinline__ bool look_singly(T &x, uint64_t limit, Ask ask, Good 
 }
 // Words of eight values of a row: word tid + 256 i into v[i] (zero past the end).
 template <int U>
-__device__ __forceinline__ bool receive(const uint8_t *row, int words, uint32_t tag, v4u *v, uint64_t limit) {
+__device__ __forceinline__ bool receive(const uint8_t *row, int words, uint32_t tag, v4u *v, uint32_t limit) {
     const int tid = afresh((int)threadIdx.x);
     const __amdgpu_buffer_rsrc_t r = rsrc_of(row, words * 32);
     struct Both {
@@ -394,7 +399,7 @@ __device__ __forceinline__ double sum32(double v) {
 }
 // Wave `wave` of the workgroup brings row `wave` of the block: the query, normed and rotated, and where the part holds rows
 // of the block itself, key and value, which the first query head's workgroup also stores to the workspace.
-__device__ __forceinline__ bool head_rows(const Common &c, int l, int wave, const Rope &rope, uint32_t tag, uint64_t limit) {
+__device__ __forceinline__ bool head_rows(const Common &c, int l, int wave, const Rope &rope, uint32_t tag, uint32_t limit) {
     uint32_t *q_lds = reinterpret_cast<uint32_t *>(c.smem), *k_lds = q_lds + kRows * kHd / 2, *v_lds = k_lds + kRows * kHd / 2;
     if (wave >= c.m_rows) return true;
     const int lane = c.lane, word = lane & 31;
@@ -478,7 +483,7 @@ __device__ __forceinline__ void raise(const Common &c, int phase, uint8_t *rows8
 __device__ __forceinline__ void announce(const Common &c, int phase, uint8_t *rows8) { raise(c, 4 + phase, rows8, 0.0f); }
 
 // The parts of row `wg`, all heads, into the raw row.
-__device__ __forceinline__ bool merge_parts(const Common &c, uint32_t tag, uint64_t limit) {
+__device__ __forceinline__ bool merge_parts(const Common &c, uint32_t tag, uint32_t limit) {
     const int tid = afresh((int)threadIdx.x);
     const int d = (tid & 63) * 2;
     const size_t part = (size_t)kRows * kPartBytes;
@@ -541,7 +546,7 @@ __device__ __forceinline__ bool merge_parts(const Common &c, uint32_t tag, uint6
 template <int N>
 struct Lines {
     v4u v[N][2];
-    __device__ __forceinline__ bool look_for(const __amdgpu_buffer_rsrc_t rows, int k, int m_rows, int group, int groups, uint64_t limit) {
+    __device__ __forceinline__ bool look_for(const __amdgpu_buffer_rsrc_t rows, int k, int m_rows, int group, int groups, uint32_t limit) {
         const int lane = afresh((int)threadIdx.x & 63);
         return look_singly(*this, limit, [&](Lines &t) {
 #pragma unroll
@@ -601,7 +606,7 @@ __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
     // The tokens come from the int8 rows at `rows8` as whole lines and go by the wave's own LDS into the matrix cores' order (lane
     // by lane each row's piece took 0.8 us at K = 2048 and 1.9 us at 6144, whatever cache they came from), the results to
     // the same LDS, [wave][tile][token][row].
-    const auto multiply = [&](const auto &wt, const Share &sh, const uint8_t *rows8, uint64_t limit) {
+    const auto multiply = [&](const auto &wt, const Share &sh, const uint8_t *rows8, uint32_t limit) {
         constexpr int S = std::decay_t<decltype(wt)>::kGroups, T = std::decay_t<decltype(wt)>::kTiles;
         constexpr int kAhead = S < 4 ? (S + 1) / 2 * 2 : 4;   // groups requested together
         const int lane = afresh(c.lane);
@@ -662,7 +667,7 @@ __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
     };
     // A projection of the int8 rows `rows8`: W neighbouring rows of a token, added up over the waves, are one thread's,
     // done(token, row, values, the token's multiplier).
-    const auto project = [&](auto wt_c, auto w_c, const Share &sh, int rows, const uint8_t *rows8, const uint8_t *w, uint64_t limit,
+    const auto project = [&](auto wt_c, auto w_c, const Share &sh, int rows, const uint8_t *rows8, const uint8_t *w, uint32_t limit,
                              auto done) -> bool {
         constexpr int W = decltype(w_c)::value;
         typedef float Vec __attribute__((ext_vector_type(W)));
@@ -715,7 +720,7 @@ __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
     };
     for (int layer = 0; layer < a.n_layers; ++layer) {
         const int l = afresh_scalar(layer);
-        const uint64_t limit = l == 0 ? kStartTicks : kRunTicks;
+        const uint32_t limit = l == 0 ? a.first_wait : a.later_wait;
         const int more = l + 1 < a.n_layers;
         const v2u nxt = ask_layer(a, more ? l + 1 : l);
         const uint32_t tag = c.epoch * (uint32_t)a.n_layers + (uint32_t)l + 1u;
@@ -915,12 +920,12 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
         return true;
     };
     // all rows' multipliers
-    const auto wait_rows = [&](int phase, const uint8_t *rows8, uint32_t &x, uint64_t limit) -> bool {
+    const auto wait_rows = [&](int phase, const uint8_t *rows8, uint32_t &x, uint32_t limit) -> bool {
         const __amdgpu_buffer_rsrc_t r = rsrc_of(rows8 + c.s8 + (phase * kCopies + c.wg % kCopies) * 128, kRows * 4);
         return look(x, limit, [&](uint32_t &t) { t = __builtin_amdgcn_raw_buffer_load_b32(r, wanted(lane < c.m_rows, lane * 4), 0, kDeviceScope); },
                     [](const uint32_t &t) { return (bool)__all(t != kEmpty); });
     };
-    const auto project = [&](int phase, const uint8_t *rows8, uint64_t limit, auto meanwhile) -> bool {
+    const auto project = [&](int phase, const uint8_t *rows8, uint32_t limit, auto meanwhile) -> bool {
         uint32_t x;
         __syncthreads();   // the weights are there
         if (!ROW && wave == 0 && !wait_rows(4 + phase, rows8, x, limit) && lane == 0) c.meet.bad = 1;
@@ -939,7 +944,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
 
     for (int layer = 0; layer < a.n_layers; ++layer) {
         const int l = afresh_scalar(layer);
-        const uint64_t limit = l == 0 ? kStartTicks : kRunTicks;
+        const uint32_t limit = l == 0 ? a.first_wait : a.later_wait;
         const int more = l + 1 < a.n_layers;
         const v2u nxt = ask_layer(a, more ? l + 1 : l);
         const uint32_t tag = c.epoch * (uint32_t)a.n_layers + (uint32_t)l + 1u;
@@ -1186,7 +1191,7 @@ constexpr Build kBuilds[] = {
 };
 struct Fit {
     int build = -1, lds = 0;
-    int64_t bytes = 0, clear = 0;
+    int64_t bytes = 0, clear = 0, marked = 0;   // exchange memory; cleared up to `clear`, from there to `marked` (its end) empty rows
 };
 inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, int groups) {
     Fit f;
@@ -1212,7 +1217,7 @@ inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, 
         }
     }
     if (f.build >= 0 && f.lds > kMostLds) f.build = -1;
-    f.bytes = at.size;
+    f.bytes = f.marked = at.size;
     f.clear = at.q8;   // control and tags
     return f;
 }

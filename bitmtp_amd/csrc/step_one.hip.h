@@ -32,9 +32,9 @@
 // last phases depend on all of them, given two layers).  Parts of the attention carry a tag instead (step and layer).
 //
 // Waits are bounded.  A workgroup that waits longer than kStartTicks in the first layer (the launch did not get all of
-// its compute units) or kRunTicks later leaves, marks the exchange memory so that launches queued behind leave at once,
-// and sets *status; the caller repeats the step with the separate launches.  A step writes nothing but its workspace
-// slot, its exchange memory and its output row, so it can be repeated.
+// its compute units) or kRunTicks later leaves, marks the exchange memory so that workgroups that start late leave at
+// once, and sets *status.  A step writes nothing but its workspace slot, its exchange memory and its output row, so it
+// can be repeated: the launch behind this one does so where it finds the mark (step_finish.hip.h).
 //
 // Arithmetic: operations and rounding points of the stand-alone producers; group sums exact (see Codes), scaled and summed
 // in fp32 over K: two or four groups a unit, then the units of a row.  The attention keeps its probabilities in fp32.
@@ -50,8 +50,8 @@ constexpr int kMaxSplits = 32;             // attention parts per head
 constexpr int kSingle = 128;               // slots one workgroup takes alone: up to here no parts to merge
 constexpr int kRounds = 2;                 // rounds of eight slots a wave requests ahead
 constexpr int kPartEntries = kHd + 4;      // 8-byte entries of a part: 128 sums, maximum, sum, pad
-constexpr uint64_t kStartTicks = 500000;   // 5 ms of the 100 MHz counter
-constexpr uint64_t kRunTicks = 20000000;   // 200 ms
+constexpr uint32_t kStartTicks = 500000;   // 5 ms of the 100 MHz counter
+constexpr uint32_t kRunTicks = 20000000;   // 200 ms
 constexpr int kPauseRow = 8, kPauseLong = 10;  // s_sleep(1) steps before the first poll (27 ns each)
 constexpr int kBufFlags = 0x00020000;
 constexpr int kOob = 0x7ffffff0;           // an offset no buffer reaches: loads give 0, stores are dropped
@@ -73,6 +73,7 @@ struct Args {
     int32_t *status;
     int n_layers, dim, ffn, n_heads, n_kv, slots, sigma, max_pos, vocab, groups;
     float eps, scale;
+    uint32_t first_wait, later_wait;   // ticks, in the first layer and in the others
 };
 
 // ---- sizes --------------------------------------------------------------------------------
@@ -194,20 +195,21 @@ __device__ __forceinline__ float lanes_on(float v) {
 }
 
 // ---- hand-over ----------------------------------------------------------------------------
-__device__ __forceinline__ bool timed_out(int spins, uint64_t &since, uint64_t limit) {
+__device__ __forceinline__ int first_spin(uint32_t limit) { return limit ? 1 : 64; }   // (0: does not wait at all)
+__device__ __forceinline__ bool timed_out(int spins, uint32_t &since, uint32_t limit) {
     if (spins & 63) return false;
-    const uint64_t now = wall_clock64();
+    const uint32_t now = (uint32_t)wall_clock64() | 1u;
     if (since == 0) since = now;
-    return now - since > limit;
+    return now - since >= limit;
 }
 
 // A row of `words` 16-byte words at `from`: word tid + 256 i into v[i] (zero past the end), once all of them have arrived.
 template <int U>
-__device__ __forceinline__ bool receive(const __amdgpu_buffer_rsrc_t r, int from, int words, v4u *v, int pause, uint64_t limit) {
+__device__ __forceinline__ bool receive(const __amdgpu_buffer_rsrc_t r, int from, int words, v4u *v, int pause, uint32_t limit) {
     const int tid = afresh((int)threadIdx.x);
     for (int z = 0; z < pause; ++z) __builtin_amdgcn_s_sleep(1);
-    uint64_t since = 0;
-    for (int spins = 1;; ++spins) {
+    uint32_t since = 0;
+    for (int spins = first_spin(limit);; ++spins) {
         bool ok = true;
 #pragma unroll
         for (int i = 0; i < U; ++i)
@@ -719,7 +721,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
 
     for (int layer = 0; layer < a.n_layers; ++layer) {
         const int l = afresh_scalar(layer);
-        const uint64_t limit = l == 0 ? kStartTicks : kRunTicks;
+        const uint32_t limit = l == 0 ? a.first_wait : a.later_wait;
         const int row0 = l * c.lay.size;   // of the layer's rows in a set
         const int more = l + 1 < a.n_layers;
         const int nl = more ? l + 1 : l;
@@ -742,9 +744,9 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
                 const int row = wave == 0 ? c.head : (wave == 1 ? a.n_heads : a.n_heads + a.n_kv) + c.kvh;
                 const int from = row0 + c.lay.qkv + row * 256;
                 uint32_t d = kEmpty;
-                uint64_t since = 0;
+                uint32_t since = 0;
                 for (int z = 0; z < kPauseRow; ++z) __builtin_amdgcn_s_sleep(1);
-                for (int spins = 1;; ++spins) {
+                for (int spins = first_spin(limit);; ++spins) {
                     d = __builtin_amdgcn_raw_buffer_load_b32(c.here, lane * 4, from, kDeviceScope);
                     if (__all(d != kEmpty)) break;
                     if (timed_out(spins, since, limit)) {
@@ -897,11 +899,11 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
             const __amdgpu_buffer_rsrc_t r = rsrc_of(c.parts + (size_t)c.head * kMaxSplits * (kPartEntries * 8), kMaxSplits * kPartEntries * 8);
             const int d = tid & 127, q = tid >> 7;
             bool ok = true;
-            uint64_t since = 0;
+            uint32_t since = 0;
             v2u o[kMaxSplits / 2];
             v4u ml;
             for (int z = 0; z < kPauseRow; ++z) __builtin_amdgcn_s_sleep(1);
-            for (int spins = 1;; ++spins) {
+            for (int spins = first_spin(limit);; ++spins) {
 #pragma unroll
                 for (int i = 0; i < kMaxSplits / 2; ++i)
                     o[i] = __builtin_amdgcn_raw_buffer_load_b64(r, wanted(q + 2 * i < c.splits, ((q + 2 * i) * kPartEntries + d) * 8), 0, kDeviceScope);
@@ -1095,7 +1097,7 @@ constexpr Build kBuilds[] = {
 };
 struct Fit {
     int build = -1, lds = 0;
-    int64_t bytes = 0;
+    int64_t bytes = 0, marked = 0;   // exchange memory; behind the control words, up to here, marks of empty rows
 };
 inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, int groups) {
     Fit f;
@@ -1118,7 +1120,8 @@ inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, 
     if (f.lds > 58 * 1024) return f;
     const Rows lay(dim, ffn, n_heads, n_kv);
     if ((int64_t)n_layers * lay.size > 0x7fffffff) return f;
-    f.bytes = kControlBytes + 2 * (int64_t)n_layers * lay.size + (int64_t)n_heads * kMaxSplits * kPartEntries * 8;
+    f.marked = kControlBytes + 2 * (int64_t)n_layers * lay.size;
+    f.bytes = f.marked + (int64_t)n_heads * kMaxSplits * kPartEntries * 8;
     const auto words = [](int k) { return (k / 8 + kFront - 1) / kFront; };
     for (int i = 0; i < (int)(sizeof kBuilds / sizeof kBuilds[0]); ++i) {
         const Build &b = kBuilds[i];

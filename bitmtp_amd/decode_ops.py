@@ -9,7 +9,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
-from typing import List, Optional, Sequence
+from typing import List, NamedTuple, Optional, Sequence
 
 import torch
 
@@ -27,7 +27,20 @@ class StepOneDesc(ctypes.Structure):
                                                 "h_out", "status")]
                 + [(n, ctypes.c_int) for n in ("bits", "n_layers", "dim", "ffn", "n_heads", "n_kv", "slots", "sigma",
                                                "max_pos", "vocab")]
-                + [("eps", ctypes.c_float), ("scale", ctypes.c_float)])
+                + [("eps", ctypes.c_float), ("scale", ctypes.c_float), ("first_wait", ctypes.c_int), ("later_wait", ctypes.c_int)]
+                + [(n, ctypes.c_void_p) for n in ("norm_w", "norm_q", "norm_s", "norm_out")]
+                + [("norm_first", ctypes.c_int), ("norm_rows", ctypes.c_int)])
+
+
+class FinalNorm(NamedTuple):
+    """Rows ``first .. first + rows - 1`` of a step, normed for the output projection: bf16 to ``out`` or, without it,
+    quantised to ``q`` and ``s``."""
+    weight: torch.Tensor                  # bf16 [dim]
+    first: int
+    rows: int
+    q: Optional[torch.Tensor] = None      # int8 [>= rows, dim]
+    s: Optional[torch.Tensor] = None      # fp32 [>= rows]
+    out: Optional[torch.Tensor] = None    # bf16 [>= rows, dim]
 
 
 def decode_lib_path() -> str:
@@ -337,11 +350,12 @@ def prefill_attention_kernel() -> str:
 
 class StepOne:
     """All layers of a one-token step in one launch (``bonsai_decode_step_one``): a model's weights and the exchange
-    memory its workgroups hand rows over in.  One launch at a time may use that memory.  ``status`` is nonzero, once the
-    launches queued so far have ended, if one of them did not get the whole device: nothing those launches wrote is of
-    use, and ``reset`` makes the object ready again."""
+    memory its workgroups hand rows over in.  One step at a time may use that memory.  A step that does not get the whole
+    device takes longer, tens of milliseconds, and raises ``status``, which nobody but the reader clears; its results are
+    right all the same."""
 
     NAME, MAX_ROWS = "bonsai_decode_step_one", 1
+    waits = (0, 0)   # of the C entry: how long, in the first layer and later ones, a step waits for the whole device
 
     def __init__(self, weights: Sequence[Sequence[torch.Tensor]], shape, device, like: Optional["StepOne"] = None):
         """``weights``: the twelve tensors of every layer in the order of the C entry's records; they are read at their
@@ -382,7 +396,7 @@ class StepOne:
         return decode_lib().bonsai_decode_step_one(ctypes.byref(desc), _stream(self.device))
 
     def enqueue(self, embed: torch.Tensor, step_in: torch.Tensor, kv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                sigma: int, eps: float, h_out: torch.Tensor, rows: int = 1) -> None:
+                sigma: int, eps: float, h_out: torch.Tensor, rows: int = 1, norm: Optional[FinalNorm] = None) -> None:
         bits, n_layers, dim, ffn, n_heads, n_kv = self.shape
         for t, name in ((embed, "embed"), (kv, "kv"), (cos, "cos"), (sin, "sin"), (h_out, "h_out")):
             _check(t, torch.bfloat16, name)
@@ -395,7 +409,22 @@ class StepOne:
                         cos_table=cos.data_ptr(), sin_table=sin.data_ptr(), exchange=self.exchange.data_ptr(),
                         h_out=h_out.data_ptr(), status=self.status.data_ptr(), bits=bits, n_layers=n_layers, dim=dim, ffn=ffn,
                         n_heads=n_heads, n_kv=n_kv, slots=kv.shape[3], sigma=int(sigma), max_pos=cos.shape[0],
-                        vocab=embed.shape[0], eps=float(eps), scale=1.0 / math.sqrt(HEAD_DIM))
+                        vocab=embed.shape[0], eps=float(eps), scale=1.0 / math.sqrt(HEAD_DIM), first_wait=self.waits[0],
+                        later_wait=self.waits[1])
+        if norm is not None:
+            _check(norm.weight, torch.bfloat16, "norm weight")
+            _need(norm.weight.numel() == dim, "norm weight shape mismatch")
+            for t, dtype, size, name in ((norm.q, torch.int8, dim, "norm q"), (norm.s, torch.float32, 1, "norm s"),
+                                         (norm.out, torch.bfloat16, dim, "norm out")):
+                if t is not None:
+                    _check(t, dtype, name)
+                    _need(t.numel() >= norm.rows * size, f"{name} too small")
+            d.norm_w, d.norm_first, d.norm_rows = norm.weight.data_ptr(), norm.first, norm.rows
+            if norm.out is not None:
+                d.norm_out = norm.out.data_ptr()
+            else:
+                _need(norm.q is not None and norm.s is not None, "the normed rows have nowhere to go")
+                d.norm_q, d.norm_s = norm.q.data_ptr(), norm.s.data_ptr()
         with torch.cuda.device(self.device):
             rc = self._launch(d, rows)
         _need(rc == 0, f"{self.NAME} failed with status {rc}")

@@ -531,7 +531,7 @@ def step_one(model: "BonsaiDecoder", form: type = decode_ops.StepOne,
             return None
         rows.append(tensors)
     shape = (bits, len(rows), args.dim, args.ffn_dim, args.n_heads, args.n_kv_heads)
-    if not model.embed.is_contiguous() or model.embed.data_ptr() % 16:
+    if any(not t.is_contiguous() or t.data_ptr() % 16 or t.dtype != torch.bfloat16 for t in (model.embed, model.norm)):
         return None
     if have is not None and have.shape == shape and have.addresses == have.addresses_of(rows):
         return have
@@ -581,9 +581,11 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
             raise RuntimeError(f"{what} failed with status {rc}")
 
     if one is not None:
-        h = ws.h[0][:M]
-        one.enqueue(model.embed, io.step_in, kv, cos, sin, sigma, eps, h, M)
-        project_rows(model, ws, h[logits_start:logits_end], None, logits_end - logits_start, threshold, io.tokens_out, io.conf, io.accept, head_mode)
+        to = dict(out=ws.l_n) if _bf16_rows(model, head_mode) else dict(q=ws.l_q, s=ws.l_s)
+        rows = logits_end - logits_start
+        one.enqueue(model.embed, io.step_in, kv, cos, sin, sigma, eps, ws.h[0][:M], M,
+                    decode_ops.FinalNorm(model.norm, logits_start, rows, **to))
+        project_rows(model, ws, None, None, rows, threshold, io.tokens_out, io.conf, io.accept, head_mode)
         return
     plan = fused_plan(model, M)
     # wider blocks keep the ten-launch layer; BONSAI_ROPE_IN_ATTENTION=1 drops its q / k norm + RoPE
@@ -673,11 +675,18 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
                  io.accept, head_mode)
 
 
-def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: torch.Tensor, last_res: Optional[torch.Tensor],
+def _bf16_rows(model: BonsaiDecoder, head_mode: str) -> bool:
+    """Whether the output projection takes normed rows in bf16 (reference: model.py:1401-1403) instead of quantised."""
+    if head_mode not in ("native", "fp8", "bf16_raw"):
+        raise ValueError(f"unknown head_mode {head_mode!r}")
+    return head_mode != "native" or model.head is None
+
+
+def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: Optional[torch.Tensor], last_res: Optional[torch.Tensor],
                  rows: int, threshold: float, tokens_out: torch.Tensor, conf: torch.Tensor,
                  accept: torch.Tensor, head_mode: str = "native") -> None:
     """Final norm of ``last_x (+ last_res)``, output projection and argmax / confidence chain of ``rows`` rows
-    (reference: model.py:1401-1403, fast_generate.py:111-130)."""
+    (reference: model.py:1401-1403, fast_generate.py:111-130); without ``last_x`` of rows that the workspace has normed."""
     args = model.args
     dim, eps = args.dim, float(args.norm_eps)
     actq = ops.actq_lib()
@@ -688,13 +697,11 @@ def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: torch.Tensor, last
         if rc != 0:
             raise RuntimeError(f"{what} failed with status {rc}")
 
-    if head_mode not in ("native", "fp8", "bf16_raw"):
-        raise ValueError(f"unknown head_mode {head_mode!r}")
-    if head_mode != "native" or model.head is None:
-        # projections of the normalised bf16 rows (reference: model.py:1401-1403)
-        check(actq.bonsai_add_rmsnorm_bf16(_vp(last_x), res, _vp(model.norm), eps, _vp(ws.h_last),
-                                           _vp(ws.l_n), rows, dim, stream),
-              "bonsai_add_rmsnorm_bf16")
+    if _bf16_rows(model, head_mode):
+        if last_x is not None:
+            check(actq.bonsai_add_rmsnorm_bf16(_vp(last_x), res, _vp(model.norm), eps, _vp(ws.h_last),
+                                               _vp(ws.l_n), rows, dim, stream),
+                  "bonsai_add_rmsnorm_bf16")
         if head_mode == "fp8":
             if model.head_fp8 is None:
                 raise RuntimeError("the FP8 draft projection was not prepared")
@@ -714,7 +721,7 @@ def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: torch.Tensor, last
                                                      _vp(ws.h_last), _vp(ws.l_q), _vp(ws.l_s), rows,
                                                      dim, stream),
                   "bonsai_add_rmsnorm_quant_int8")
-        else:
+        elif last_x is not None:
             check(actq.bonsai_rmsnorm_quant_int8(_vp(last_x), _vp(model.norm), eps, _vp(ws.l_q),
                                                  _vp(ws.l_s), rows, dim, stream),
                   "bonsai_rmsnorm_quant_int8")

@@ -183,41 +183,16 @@ class GraphAtlas:
         self._positions: Optional[torch.Tensor] = None
         self.replays = 0
         # steps of one token and of up to sixteen as one launch (model.step_one), with the weights of the last capture or,
-        # without graphs, of the last step.  Such a launch gives up when it does not get the whole device; what was queued
-        # since the last read is kept until it is known that none did, so that it can be queued again with the separate
-        # launches
+        # without graphs, of the last step
         self._one = self._block = None
-        self._queued: List[Tuple] = []
-        self._separate_for = 0      # replays that keep to the separate launches after one gave up
+        # Such a launch that does not get the whole device has its step done again behind it, the slow way.  It says so, and
+        # then the separate launches stay for a while, twice as long every time.
+        self._separate_for = 0                  # replays that keep to the separate launches
         self._back_off = 64
 
     def synchronize(self) -> None:
         """Wait for everything queued on the atlas's device (the loops' timing fences)."""
         torch.cuda.synchronize(self.device)
-        self._settle()
-
-    # -- steps that gave up ----------------------------------------------------
-    def _settle(self) -> None:
-        """Everything queued has ended: queue it again if a one-launch step among it gave up."""
-        if not self._queued:
-            return
-        queued, self._queued = self._queued, []
-        failed = [one for one in {args[0].one for what, args in queued if what is None} if one is not None and one.failed[0] != 0]
-        if not failed:
-            return
-        for one in failed:
-            one.reset()
-        self._separate_for, self._back_off = self._back_off, min(2 * self._back_off, 1 << 20)
-        for what, args in queued:
-            (what or self._replay)(*args)
-        torch.cuda.synchronize(self.device)
-
-    def _note(self, what, *args) -> None:
-        """Something queued behind a one-launch step; ``what`` is None for a replay."""
-        self._queued.append((what, args))
-        if len(self._queued) > 256:
-            torch.cuda.current_stream(self.device).synchronize()
-            self._settle()
 
     # -- KV ------------------------------------------------------------------
     def kv(self, sigma: int) -> torch.Tensor:
@@ -248,17 +223,12 @@ class GraphAtlas:
         if cache_len + n_accept > sigma:
             raise RuntimeError("KV commit would run past the history segment")
         decode_ops.kv_commit(self.kv(sigma), sigma + first_row, cache_len, n_accept)
-        if self._queued:
-            self._note(decode_ops.kv_commit, self.kv(sigma), sigma + first_row, cache_len, n_accept)
 
     def migrate_segment(self, src_sigma: int, dst_sigma: int, cache_len: int) -> None:
         """Copy live history to another segment's buffer (fast_runtime.py:510-521)."""
         if src_sigma == dst_sigma:
             return
-        source, target = self.kv(src_sigma)[:, :, :, :cache_len], self.kv(dst_sigma)[:, :, :, :cache_len]
-        target.copy_(source)
-        if self._queued:
-            self._note(target.copy_, source)
+        self.kv(dst_sigma)[:, :, :, :cache_len].copy_(self.kv(src_sigma)[:, :, :, :cache_len])
 
     # -- graphs --------------------------------------------------------------
     def get_graph(self, M: int, sigma: int, role: str) -> CapturedGraph:
@@ -369,8 +339,6 @@ class GraphAtlas:
         if n > sigma:
             raise RuntimeError("history does not fit the segment")
         kv = self.kv(sigma)
-        if self._queued:
-            self.synchronize()
         block = min(n, PROMPT_BLOCK_MAX)
         with torch.inference_mode(False), torch.cuda.device(self.device):
             if self._prompt is None or self._prompt.rows < block:
@@ -400,17 +368,10 @@ class GraphAtlas:
         if cache_len + M > g.sigma + M or cache_len > g.sigma:
             raise RuntimeError("history does not fit the segment")
         inputs = step_descriptor(g.role, M, self.D, cache_len, n_pend) + list(positions) + list(tokens)
+        io = g.io
         if g.graph is None and g.one is not None:
             g.one = self._one_launch(M)
-        self._replay(g, inputs)
-        self.replays += 1
-        if g.one is not None or self._queued:
-            self._note(None, g, inputs)
-
-    def _replay(self, g: CapturedGraph, inputs: Sequence[int]) -> None:
-        io = g.io
-        if g.one is not None and self._separate_for > 0:
-            self._separate_for -= 1
+        if g.one is not None and self._keeps_separate(g.one):
             if g.separate is None:
                 g.separate = self._capture_one(g.M, g.sigma, g.role, g)
             g = g.separate
@@ -420,6 +381,26 @@ class GraphAtlas:
         g.io.step_in_host.numpy()[:] = inputs
         stream = torch.cuda.current_stream(self.device)
         g.io.arrived = False
+        self._launch(g, stream)
+        if g.io is not io:            # the results belong where the caller's graph leaves them
+            io.out.copy_(g.io.out)
+            io.uploaded.record(stream)
+            io.downloaded = False
+        self.replays += 1
+
+    def _keeps_separate(self, one: decode_ops.StepOne) -> bool:
+        """Whether this replay keeps to the separate launches, after a step that did not get the whole device."""
+        if one.failed[0] != 0:
+            if one.failed[0] != 1:
+                raise RuntimeError("a decode step did not end")
+            one.failed[0] = 0
+            self._separate_for, self._back_off = self._back_off, min(2 * self._back_off, 1 << 20)
+        if self._separate_for > 0:
+            self._separate_for -= 1
+            return True
+        return False
+
+    def _launch(self, g: CapturedGraph, stream: "torch.cuda.Stream") -> None:
         if g.graph is not None:
             g.io.out_host.numpy()[:] = StepIO.PENDING
             g.graph.replay()          # uploads, runs the step, downloads the results
@@ -429,10 +410,6 @@ class GraphAtlas:
             g._eager(g.one)
             g.io.downloaded = False
         g.io.uploaded.record(stream)
-        if g.io is not io:            # the results belong where the caller's graph leaves them
-            io.out.copy_(g.io.out)
-            io.uploaded.record(stream)
-            io.downloaded = False
 
     def read_outputs(self, g: CapturedGraph) -> Tuple[np.ndarray, np.ndarray, int]:
         """One device-to-host copy + synchronisation: (argmax tokens, confidences,
@@ -452,13 +429,8 @@ class GraphAtlas:
         else:
             g.io.out_host.copy_(g.io.out, non_blocking=True)
             torch.cuda.current_stream(self.device).synchronize()
-        if self._queued:
-            if next(args[0] for what, args in reversed(self._queued) if what is None) is not g:
-                torch.cuda.current_stream(self.device).synchronize()   # the reader has not waited for the last of them
-            self._settle()
-            if not g.io.downloaded:
-                g.io.out_host.copy_(g.io.out, non_blocking=True)
-                torch.cuda.current_stream(self.device).synchronize()
+        if g.one is not None and g.one.failed[0] > 1:
+            raise RuntimeError("a decode step did not end")
         rows = g.logits_end - g.logits_start
         out = g.io.out_host.numpy()
         toks = out[:rows].copy()

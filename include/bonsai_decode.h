@@ -161,9 +161,12 @@ int bonsai_decode_attention_rope_parts(const void *xqkv, const void *q_norm_w, c
  * `sigma` of every layer and the residual stream behind the last layer to `h_out`.
  *
  * One workgroup per compute unit stays for the whole launch and waits for the others, so a launch needs all units of
- * the device.  Waits are bounded: if the units are not there within 5 ms, *status (int32, pinned host or device memory,
- * zeroed by the caller) becomes nonzero, h_out and the slot hold nothing useful, the launches queued behind do the same at once, and
- * the exchange memory has to be reset before the next use; the step can then be repeated by other means.
+ * the device.  Waits are bounded: if the units are not there within 5 ms, the launch leaves and *status (int32, pinned host
+ * or device memory, zeroed by the caller) becomes 1.  A second launch behind it norms the rows that are projected onto the
+ * vocabulary and, where the first one left, does the step again before that, with whatever workgroups it gets.  So
+ * all results are right in stream order either way; *status says that it took milliseconds, and that separate launches may
+ * serve better while something else runs on the device.  (2: that launch waited 20 s for a workgroup of its own, and the
+ * results are not there.)
  *
  *   layers    device array of n_layers records of 12 pointers: packed weights of q|k|v, o, gate|up and down, their
  *             bf16 group scales in the same order, input and post-attention norm weights, q and k norm weights;
@@ -171,7 +174,12 @@ int bonsai_decode_attention_rope_parts(const void *xqkv, const void *q_norm_w, c
  *   step_in   int32 [5]: meta[0 .. 2] as above, position, token
  *   kv        bf16 [2, n_layers, n_kv, slots, 128]
  *   exchange  bonsai_decode_step_one_bytes(...) bytes on 128 bytes, prepared by bonsai_decode_step_one_reset; one
- *             launch at a time may use it
+ *             step at a time may use it
+ *   first_wait, later_wait   how long a workgroup waits for others, in units of 10 ns, in the first layer and in the
+ *             later ones; 0: 5 ms and 200 ms; negative: it does not wait where it finds nothing
+ *   norm_*    final norm with weights norm_w of rows norm_first .. norm_first + norm_rows - 1 of h_out (none: 0): bf16 to
+ *             norm_out or, where that is null, quantised to norm_q int8 [norm_rows, dim] and norm_s fp32 [norm_rows], as
+ *             bonsai_add_rmsnorm_bf16 and bonsai_rmsnorm_quant_int8 do it; norm_w, norm_out and h_out on 16 bytes
  * bonsai_decode_step_one_bytes returns 0 for shapes it does not take. */
 typedef struct bonsai_step_one_desc {
     const void *layers, *embed;
@@ -182,6 +190,12 @@ typedef struct bonsai_step_one_desc {
     int32_t *status;
     int bits, n_layers, dim, ffn, n_heads, n_kv, slots, sigma, max_pos, vocab;
     float eps, scale;
+    int first_wait, later_wait;
+    const void *norm_w;
+    void *norm_q;
+    float *norm_s;
+    void *norm_out;
+    int norm_first, norm_rows;
 } bonsai_step_one_desc;
 int64_t bonsai_decode_step_one_bytes(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv);
 int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, void *exchange, void *stream);

@@ -116,8 +116,8 @@ def test_argument_checks():
     assert lib.bonsai_decode_step_block(None, 9, None) != 0
 
 
-def test_steps_are_repeated_after_a_launch_that_gave_up(monkeypatch):
-    """The flag such a launch raises is raised from the host, one of a one-token step between two blocks with it."""
+def test_steps_are_repeated_after_a_launch_that_gave_up():
+    """Marks of launches that gave up, for a block and a one-token step behind it, with nothing read in between."""
     from bitmtp_amd.runtime import GraphAtlas
     model = _model(2, 1024, 1024, 8, 4)
     atlas = GraphAtlas(model, segment_ladder=(256,))
@@ -128,17 +128,14 @@ def test_steps_are_repeated_after_a_launch_that_gave_up(monkeypatch):
     for lost in (False, True):
         atlas.kv(sigma).zero_()
         for n in range(1, 28, 9):
+            if lost and n == 10:
+                for one in (atlas._one, atlas._block):
+                    one.exchange[4:8].view(torch.int32).fill_(1)
             atlas.replay(verify, list(range(n, n + 9)), list(range(n - 1, n + 8)), n)
             atlas.commit_kv(sigma, n, 4)
             atlas.replay(ar, [n], [n + 4], n + 4)
             atlas.commit_kv(sigma, n + 4, 1)
-            if lost and n == 10:   # nothing of these steps arrived
-                torch.cuda.synchronize()
-                atlas.kv(sigma)[:, :, :, n:].zero_()
-                verify.io.out.zero_()
-                atlas._one.failed[0] = atlas._block.failed[0] = 1
             toks, conf, accept = atlas.read_outputs(verify)
-            assert not atlas._queued and atlas._one.failed[0] == 0 and atlas._block.failed[0] == 0
         results.append((toks, accept, atlas.kv(sigma)[:, :, :, :24].float().clone()))
     assert verify.separate is not None and ar.separate is not None
     (t0, c0, k0), (t1, c1, k1) = results
