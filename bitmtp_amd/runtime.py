@@ -20,6 +20,7 @@ Differences from the reference, by design:
 from __future__ import annotations
 
 import gc
+import threading
 import time
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -137,8 +138,27 @@ class CapturedGraph:
     logits_start: int
     logits_end: int
     one: Optional[decode_ops.StepOne] = None            # its layers are one launch
-    model: Optional[BonsaiDecoder] = None               # the weights it was captured with (without a graph: the atlas's own model)
-    separate: Optional["CapturedGraph"] = None          # the same step as separate launches, captured when first needed
+
+
+class _WholeDevice:
+    """Steps in one launch need every compute unit of a device.  Two of them on two streams would each get some and wait for
+    the rest until both give up, so a step waits, on its stream, for the last one of another stream."""
+
+    def __init__(self):
+        self.lock = threading.Lock()
+        self.last: Dict[int, Tuple[int, "torch.cuda.Event"]] = {}   # device: stream, what is recorded behind the step
+
+    def launch(self, stream: "torch.cuda.Stream", done: "torch.cuda.Event", step, *args) -> None:
+        """``step(*args)``, which queues a step on ``stream`` and records ``done`` behind it."""
+        with self.lock:
+            last = self.last.get(stream.device_index)
+            if last is not None and last[0] != stream.cuda_stream:
+                stream.wait_event(last[1])
+            step(*args)
+            self.last[stream.device_index] = (stream.cuda_stream, done)
+
+
+_whole_device = _WholeDevice()
 
 
 class GraphAtlas:
@@ -186,9 +206,13 @@ class GraphAtlas:
         # without graphs, of the last step
         self._one = self._block = None
         # Such a launch that does not get the whole device has its step done again behind it, the slow way.  It says so, and
-        # then the separate launches stay for a while, twice as long every time.
+        # then the separate launches stay for a while, twice as long every time until the one launch has run undisturbed again.
         self._separate_for = 0                  # replays that keep to the separate launches
-        self._back_off = 64
+        self._back_off = self.BACK_OFF
+        self._undisturbed = 0                   # replays as one launch since
+
+    #: replays with separate launches after a step that did not get the whole device
+    BACK_OFF = 64
 
     def synchronize(self) -> None:
         """Wait for everything queued on the atlas's device (the loops' timing fences)."""
@@ -281,7 +305,7 @@ class GraphAtlas:
             return self._block
         return None
 
-    def _capture_one_impl(self, M: int, sigma: int, role: str, separate_of: Optional[CapturedGraph] = None) -> CapturedGraph:
+    def _capture_one_impl(self, M: int, sigma: int, role: str) -> CapturedGraph:
         if role not in contracts.GRAPH_ROLES:
             raise ValueError(f"unsupported graph role: {role!r}")
         if role not in self.roles:
@@ -301,9 +325,9 @@ class GraphAtlas:
         # the closure holds the pieces, not the atlas: no reference cycle through the graphs
         model, workspace, rope, threshold = self.model, self.workspace, self.rope, self.threshold
         if self.use_graphs:   # what is captured reads these tensors for good
-            model = model.snapshot() if separate_of is None else separate_of.model
+            model = model.snapshot()
         head_mode = HEAD_MODE_OF_ROLE[role]
-        one = self._one_launch(M) if separate_of is None else None
+        one = self._one_launch(M)
 
         def run(one):
             enqueue_step(model, workspace, io, kv, sigma, rope, ls, le, threshold,
@@ -313,8 +337,9 @@ class GraphAtlas:
         if self.use_graphs:
             side = torch.cuda.Stream(device=self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
-            with torch.cuda.stream(side):
-                run(one)  # warm-up outside capture: lazy library set-up happens here
+            with torch.cuda.stream(side):   # warm-up outside capture: lazy library set-up happens here
+                warm = torch.cuda.Event()
+                _whole_device.launch(side, warm, lambda: (run(one), warm.record(side)))
             torch.cuda.current_stream(self.device).wait_stream(side)
             torch.cuda.synchronize(self.device)
             # the graph carries its own upload of the step inputs and download of the results
@@ -326,7 +351,7 @@ class GraphAtlas:
                 run(one)
                 io.out_host.copy_(io.out, non_blocking=True)
         cg = CapturedGraph(graph=graph, io=io, M=M, sigma=sigma, role=role, P=M - self.D,
-                           logits_start=ls, logits_end=le, one=one, model=model)
+                           logits_start=ls, logits_end=le, one=one)
         cg._eager = run
         return cg
 
@@ -368,24 +393,19 @@ class GraphAtlas:
         if cache_len + M > g.sigma + M or cache_len > g.sigma:
             raise RuntimeError("history does not fit the segment")
         inputs = step_descriptor(g.role, M, self.D, cache_len, n_pend) + list(positions) + list(tokens)
-        io = g.io
         if g.graph is None and g.one is not None:
             g.one = self._one_launch(M)
-        if g.one is not None and self._keeps_separate(g.one):
-            if g.separate is None:
-                g.separate = self._capture_one(g.M, g.sigma, g.role, g)
-            g = g.separate
+        separate = g.one is None or self._keeps_separate(g.one)
         # the previous upload from this pinned buffer must have left the host first (as it has where results came back)
         if not g.io.arrived:
             g.io.uploaded.synchronize()
         g.io.step_in_host.numpy()[:] = inputs
         stream = torch.cuda.current_stream(self.device)
         g.io.arrived = False
-        self._launch(g, stream)
-        if g.io is not io:            # the results belong where the caller's graph leaves them
-            io.out.copy_(g.io.out)
-            io.uploaded.record(stream)
-            io.downloaded = False
+        if separate:
+            self._launch(g, stream, None)
+        else:
+            _whole_device.launch(stream, g.io.uploaded, self._launch, g, stream, g.one)
         self.replays += 1
 
     def _keeps_separate(self, one: decode_ops.StepOne) -> bool:
@@ -395,19 +415,25 @@ class GraphAtlas:
                 raise RuntimeError("a decode step did not end")
             one.failed[0] = 0
             self._separate_for, self._back_off = self._back_off, min(2 * self._back_off, 1 << 20)
+            self._undisturbed = 0
         if self._separate_for > 0:
             self._separate_for -= 1
             return True
+        self._undisturbed += 1
+        if self._undisturbed == self.BACK_OFF:   # (they may still be queued: one that gives up later is seen then)
+            self._back_off = self.BACK_OFF
         return False
 
-    def _launch(self, g: CapturedGraph, stream: "torch.cuda.Stream") -> None:
-        if g.graph is not None:
+    def _launch(self, g: CapturedGraph, stream: "torch.cuda.Stream", one: Optional[decode_ops.StepOne]) -> None:
+        # (a step in one launch keeps to separate ones without a graph of theirs: capturing one here, in the middle of a
+        # program's work, would disturb its other threads)
+        if g.graph is not None and one is g.one:
             g.io.out_host.numpy()[:] = StepIO.PENDING
             g.graph.replay()          # uploads, runs the step, downloads the results
             g.io.downloaded = True
         else:
             g.io.step_in.copy_(g.io.step_in_host, non_blocking=True)
-            g._eager(g.one)
+            g._eager(one)
             g.io.downloaded = False
         g.io.uploaded.record(stream)
 

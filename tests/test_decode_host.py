@@ -343,3 +343,26 @@ def test_graph_capture_runs_with_the_garbage_collector_off():
         assert not gc.isenabled()      # a caller's own setting is left alone
     finally:
         gc.enable()
+
+
+def test_separate_launches_stay_for_a_while_after_a_disturbed_step():
+    """64 replays, twice as many each time, and 64 again once as many steps in one launch were not disturbed."""
+    atlas = R.GraphAtlas.__new__(R.GraphAtlas)
+    atlas._separate_for, atlas._back_off, atlas._undisturbed = 0, R.GraphAtlas.BACK_OFF, 0
+    one = SimpleNamespace(failed=np.zeros(1, dtype=np.int32))
+
+    def separate_after(undisturbed):
+        assert not any(atlas._keeps_separate(one) for _ in range(undisturbed))
+        one.failed[0] = 1
+        n = 0
+        while atlas._keeps_separate(one):
+            n += 1
+        assert one.failed[0] == 0
+        return n
+    assert [separate_after(5), separate_after(0), separate_after(62)] == [64, 128, 256]
+    assert separate_after(63) == 64       # (the replay that ends a wait is undisturbed too)
+    assert [separate_after(0) for _ in range(3)] == [128, 256, 512]
+    assert separate_after(1000) == 64
+    for _ in range(13):
+        separate_after(0)
+    assert atlas._back_off == 1 << 20     # (the longest)

@@ -1,6 +1,8 @@
 """Steps in one launch that did not get the whole device (``csrc/step_finish.hip.h``): their results are right in stream
 order, without a read in between, and the exchange memory serves the next step.  The device gives up by its own bounded
 waits, which are told not to wait at all."""
+import threading
+
 import pytest
 import torch
 
@@ -99,6 +101,73 @@ def test_the_exchange_memory_serves_the_next_step(width):
             want = got
         for x, y in zip(got, want):
             assert torch.equal(x, y) if what == "" else float((x - y).norm() / y.norm()) <= 4e-2, what
+
+
+def test_atlases_on_two_streams_take_turns():
+    """Steps of two atlases on two streams, made to start together, don't keep each other from the device."""
+    from bitmtp_amd.runtime import GraphAtlas
+    model = _model(2, 1024, 512, 8, 4)
+    atlases = [GraphAtlas(model, segment_ladder=(256,)) for _ in range(2)]
+    graphs = [(a.get_graph(1, 256, "ar"), a.get_graph(9, 256, "verify")) for a in atlases]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for n in range(1, 41):
+        torch.cuda._sleep(200000)
+        start = torch.cuda.Event()
+        start.record()
+        for a, (ar, verify), stream in zip(atlases, graphs, streams):
+            with torch.cuda.stream(stream):
+                stream.wait_event(start)
+                if n % 2:
+                    a.replay(ar, [n], [n], n)
+                    a.commit_kv(256, n, 1)
+                else:
+                    a.replay(verify, [n] * 9, list(range(n, n + 9)), n)
+                    a.commit_kv(256, n, 1, 1)
+    results = [a.read_outputs(verify)[0] for a, (_, verify) in zip(atlases, graphs)]
+    torch.cuda.synchronize()
+    for a in atlases:
+        assert a._one.failed[0] == 0 and a._block.failed[0] == 0 and a._separate_for == 0
+    assert (results[0] == results[1]).all() and torch.equal(atlases[0].kv(256)[:, :, :, :41], atlases[1].kv(256)[:, :, :, :41])
+
+
+@pytest.mark.parametrize("waits", [(0, 0), (-1, 0)])
+def test_atlases_in_two_threads(waits, monkeypatch):
+    """The same, queued by two threads, undisturbed and where the steps give up and the separate launches take over."""
+    from bitmtp_amd import decode_ops
+    from bitmtp_amd.runtime import GraphAtlas
+    monkeypatch.setattr(decode_ops.StepOne, "waits", waits)
+    model = _model(2, 1024, 512, 8, 4)
+    atlases = [GraphAtlas(model, segment_ladder=(256,)) for _ in range(2)]
+    graphs = [(a.get_graph(1, 256, "ar"), a.get_graph(9, 256, "verify")) for a in atlases]
+    results, errors = [None, None], []
+
+    def steps(i, stream):
+        try:
+            a, (ar, verify) = atlases[i], graphs[i]
+            with torch.cuda.stream(stream):
+                for n in range(1, 61):
+                    a.replay(ar, [n], [n], n)
+                    a.commit_kv(256, n, 1)
+                    a.replay(verify, [n] * 9, list(range(n, n + 9)), n + 1)
+                results[i] = a.read_outputs(verify)[0].copy(), a.kv(256)[:, :, :, :61].clone()
+                stream.synchronize()
+        except Exception as e:   # noqa: BLE001 - reported by the test
+            errors.append(e)
+
+    threads = [threading.Thread(target=steps, args=(i, torch.cuda.Stream())) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for a in atlases:
+        assert (a._separate_for > 0 or a._one.failed[0] + a._block.failed[0] > 0) == (waits != (0, 0))
+    (t0, k0), (t1, k1) = results
+    if waits == (0, 0):
+        assert (t0 == t1).all() and torch.equal(k0, k1)
+    else:   # (which steps were separate launches depends on when the flag was seen)
+        assert float((k0.float() - k1.float()).norm() / k0.float().norm()) <= 4e-2
 
 
 @pytest.mark.parametrize("bits,dim,ffn,n_heads,n_kv,width,first,rows", [

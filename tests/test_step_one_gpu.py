@@ -169,7 +169,7 @@ def test_steps_are_repeated_after_a_launch_that_gave_up(use_graphs, monkeypatch)
         n += 1
         token = int(atlas.read_outputs(g)[0][0])
         out.append(token)
-        assert atlas._one.failed[0] == (step == 5) and (g.separate is not None) == (step > 5)
+        assert atlas._one.failed[0] == (step == 5) and atlas._separate_for == (64 - (step - 5) if step > 5 else 0)
     assert out == want
     for _ in range(atlas._separate_for):
         atlas.replay(g, [token], [n], n)
