@@ -34,9 +34,11 @@
 // Arithmetic and rounding points are those of the other kernels: exact G, fp32 scale-accumulate with
 // groups in ascending order inside a slice, slices in order, division by s[m], bf16 RNE.
 //
-// gate|up of a prompt (`pairs`): a tile has gate rows and their up rows, and silu(gate) * up leaves the tile instead, 16 bytes
+// gate|up of a prompt (`PAIRS`): a tile has gate rows and their up rows, and silu(gate) * up leaves the tile instead, 16 bytes
 // a lane as before: half the bytes out, and what follows reads half (3001 tokens of the 4B shape: 191.2 us as without it,
-// the activation launch behind it 32.7 -> 18.9; 256 tokens of the 1.7B one: 18.4 and 4.5 us, level).
+// the activation launch behind it 32.7 -> 18.9; 256 tokens of the 1.7B one: 18.4 and 4.5 us, level).  Builds of their own: with
+// a flag for it, all the others were slower, 4096 x 2048 at 128 tokens 6.59 us instead of 6.45, 2048 x 2048 at 514 10.5
+// instead of 10.2, long ones level.
 //
 // Block numbers go round the eight XCDs, so an XCD takes a contiguous range of tiles, eight token
 // tiles by consecutive row tiles: its L2 sees the same activations and the same rows again.
@@ -85,7 +87,7 @@ __device__ __forceinline__ void wide_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int BITS, int WM, int WN, int KS, int MT, int NT, bool SF16, bool G32>
+template <int BITS, int WM, int WN, int KS, int MT, int NT, bool SF16, bool G32, bool PAIRS>
 __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : 4)))
 gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
                  int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
@@ -104,19 +106,18 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     const int gm = tiles_m - mg * kWideTokenGroup < kWideTokenGroup ? tiles_m - mg * kWideTokenGroup : kWideTokenGroup;
     const int tn = rem / gm;
     const int m0 = (mg * kWideTokenGroup + rem - tn * gm) * S::kTokens;
-    // pairs: the tile's rows are kRows / 2 gate rows and, behind them, their up rows, of N / 2 each
-    const bool pairs = flags & 4;
+    // PAIRS: the tile's rows are kRows / 2 gate rows and, behind them, their up rows, of N / 2 each
     constexpr int kHalf = S::kRows / 2;
-    const int n0 = tn * (pairs ? kHalf : S::kRows);
+    const int n0 = tn * (PAIRS ? kHalf : S::kRows);
     const int mv = M - m0 < S::kTokens ? M - m0 : S::kTokens;
-    const int nv = pairs ? (N / 2 - n0 < kHalf ? N / 2 - n0 : kHalf) : (N - n0 < S::kRows ? N - n0 : S::kRows);
+    const int nv = PAIRS ? (N / 2 - n0 < kHalf ? N / 2 - n0 : kHalf) : (N - n0 < S::kRows ? N - n0 : S::kRows);
     // row r of the tile as a row of what rB and rS cover (a pair's matrix whole: rows past its end repeat the last)
     const auto at_row = [&](int r) {
-        if (!pairs) return r;
+        if (!PAIRS) return r;
         const int p = r < kHalf ? r : r - kHalf;
         return n0 + (p < nv ? p : nv - 1) + (r < kHalf ? 0 : N / 2);
     };
-    const int base_row = pairs ? 0 : n0, rows_there = pairs ? N : nv;
+    const int base_row = PAIRS ? 0 : n0, rows_there = PAIRS ? N : nv;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -417,7 +418,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     __syncthreads();
     // ---- the tile leaves in 16-byte pieces of whole rows
     uint16_t *o = reinterpret_cast<uint16_t *>(out);
-    if (pairs) {   // .. as bf16(bf16(silu(gate)) * up)
+    if constexpr (PAIRS) {   // .. as bf16(bf16(silu(gate)) * up)
         constexpr int kPairs = kHalf / 8;
         for (int i = tid; i < S::kTokens * kPairs; i += S::kThreads) {
             const int m = i / kPairs, c = (i % kPairs) * 8;
@@ -455,7 +456,7 @@ using WideKernelFn = void (*)(const int8_t *, const uint8_t *, void *, const flo
                               int, int, int, int, int);
 
 struct WideVariant {
-    WideKernelFn fn[3];  // bf16 scales, fp16 scales, group sums
+    WideKernelFn fn[4];  // bf16 scales, fp16 scales, group sums, pairs (bf16 scales)
     int tokens, rows, threads;
     size_t (*lds)(int K);
     int t[5];  // template arguments, for the launch record
@@ -464,9 +465,10 @@ struct WideVariant {
 template <int BITS, int WM, int WN, int KS, int MT, int NT>
 constexpr WideVariant wide_variant() {
     using S = WideShape<BITS, WM, WN, KS, MT, NT>;
-    return WideVariant{{gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false>,
-                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, true, false>,
-                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, true>},
+    return WideVariant{{gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, false>,
+                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, true, false, false>,
+                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, true, false>,
+                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, true>},
                        S::kTokens, S::kRows, S::kThreads, S::lds_bytes, {WM, WN, KS, MT, NT}};
 }
 
@@ -484,7 +486,7 @@ const WideVariant &wide_kernel(int v) {
 template <int BITS>
 int wide_init_device(int max_lds) {
     for (int v = 0; v < kWideVariants; ++v)
-        for (int k = 0; k < 3; ++k)
+        for (int k = 0; k < 4; ++k)
             if (hipFuncSetAttribute(reinterpret_cast<const void *>(wide_kernel<BITS>(v).fn[k]),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, max_lds) != hipSuccess)
                 return 2;
@@ -541,7 +543,7 @@ int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int l
     const WideVariant &k = wide_kernel<BITS>(v);
     if (!wide_fits<BITS>(v, q.K, lds_limit)) return -1;
     // pairs: N / 2 gate rows, N / 2 up rows -> silu(gate) * up, 16-byte pieces of whole rows; one resource over all of B
-    if (pairs && (out_kind != OUT_BF16 || q.N % 16 != 0 || (reinterpret_cast<uintptr_t>(q.out) & 15) != 0 ||
+    if (pairs && (out_kind != OUT_BF16 || scale_kind != 0 || q.N % 16 != 0 || (reinterpret_cast<uintptr_t>(q.out) & 15) != 0 ||
                   (long)q.N * q.K * BITS / 8 > (1L << 30)))
         return -1;
     const int tile_rows = pairs ? k.rows / 2 : k.rows, all_rows = pairs ? q.N / 2 : q.N;
@@ -549,8 +551,8 @@ int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int l
     if ((long)tm * tn > (1L << 28)) return -1;
     const int per = (tm * tn + kWideXcds - 1) / kWideXcds;
     const int flags = ((q.K / kGroup) % 4 == 0 && (reinterpret_cast<uintptr_t>(q.ws) & 7) == 0 ? 1 : 0) |
-                      (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0) | (pairs ? 4 : 0);
-    const int variant = out_kind == OUT_G32 ? 2 : scale_kind;
+                      (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0);
+    const int variant = pairs ? 3 : (out_kind == OUT_G32 ? 2 : scale_kind);
     hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), k.lds(q.K), stream, q.A, q.B, q.out,
                        q.s, reinterpret_cast<const uint16_t *>(q.ws), q.M, q.N, q.K, out_kind == OUT_F32 ? 1 : 0, tm,
                        tn, flags);
