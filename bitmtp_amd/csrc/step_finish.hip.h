@@ -179,7 +179,6 @@ __device__ __forceinline__ void project(const int8_t *q8, const float *s8, int r
     const int8_t *const x = q8 + (size_t)token * k + kb * 32;
     const uint8_t *const wr = w + (size_t)row * groups * (16 * BITS) + kb * (4 * BITS);
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
     for (int g = 0; g < groups; ++g) {
         uint32_t p0, p1;
         if constexpr (BITS == 2) {
@@ -229,7 +228,6 @@ __device__ __forceinline__ void attend(const uint16_t *query, const uint16_t *k_
         sum = sum * keep + wave_sum(p);
         o0 *= keep;
         o1 *= keep;
-#pragma unroll 8
         for (int e = 0; e < 64; ++e) {   // (behind the last slot the last one, with a probability of 0)
             const float pe = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(p), e));
             const uint32_t v = *reinterpret_cast<const uint32_t *>(v_head + slot_of(base + e < total ? base + e : total - 1) + 2 * lane);
