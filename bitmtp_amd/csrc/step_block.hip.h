@@ -1196,9 +1196,8 @@ struct Fit {
 inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, int groups) {
     Fit f;
     const int q_dim = n_heads * kHd;
-    // (Two layers are for looking at: separate launches leave every stage of the last one in the step's buffers, one launch
-    // does not.  It would take 59 us instead of 72 for nine rows of two layers of the 1.7B shape.)
-    if ((bits != 1 && bits != 2) || n_layers < 3 || n_kv < 1 || n_heads < 1 || n_heads % n_kv != 0 || (groups - kRows) / n_heads < 1 ||
+    // (One layer: workgroup 0 may be done, and advance the counter, before every other one has read it.)
+    if ((bits != 1 && bits != 2) || n_layers < 2 || n_kv < 1 || n_heads < 1 || n_heads % n_kv != 0 || (groups - kRows) / n_heads < 1 ||
         groups > 65535 || dim < 128 || ffn < 128 || dim % 128 != 0 || ffn % 128 != 0)
         return f;
     const int64_t n_qkv = (int64_t)(n_heads + 2 * n_kv) * kHd;

@@ -131,9 +131,63 @@ def _oracle_weights(model, atlas):
     }
 
 
+@pytest.mark.parametrize("waits", [(0, 0), (-1, 0)])   # as one launch, and done again behind one that gave up
+@pytest.mark.parametrize("name,M,role", [("1.7b", 1, "ar"), ("1.7b", 9, "verify"), ("4b", 1, "ar"), ("4b", 16, "draft")])
+def test_two_layer_step_in_one_launch_at_real_dims(name, M, role, waits, monkeypatch):
+    """Two layers of the real width and the real head in one launch, against the CPU composition of the oracles."""
+    from oracle import decode_oracle as DO
+    from oracle import oracle as O
+    from bitmtp_amd import decode_ops, runtime
+    from bitmtp_amd.model import BonsaiDecoder
+    from bitmtp_amd.runtime import GraphAtlas
+    O.build()
+    monkeypatch.setattr(decode_ops.StepOne, "waits", waits)
+    sigma, cache_len = 256, 131
+    model = BonsaiDecoder.random_init(_args(name, n_layers=2), seed=5, device=DEV)
+    for lw in model.layers:   # layers that add a small part to the residual stream, as trained ones do
+        lw.wo.weight_scale.mul_(2.0 ** -10)
+        lw.w_down.weight_scale.mul_(2.0 ** -10)
+    atlas = GraphAtlas(model, segment_ladder=(sigma,), threshold=0.9)
+    a = model.args
+    rng = np.random.default_rng(3)
+    kv = atlas.kv(sigma)
+    kv.copy_((torch.randn(tuple(kv.shape), device=DEV) * 0.5).to(torch.bfloat16))
+    kv_bits = bf16_bits(kv)
+    tokens = rng.integers(0, a.vocab_size, M).tolist()
+    positions = [cache_len + i for i in range(M)]
+    n_pend = 3 if role == "draft" else 0
+    g = atlas.get_graph(M, sigma, role)
+    assert g.one is not None
+    print(f"[case] {name} two-layer step in one launch, M={M}, {role}, waits {waits}", flush=True)
+    g.one.failed[0] = 0   # (raised by the launch that warms up)
+    atlas.replay(g, tokens, positions, cache_len, n_pend)
+    atlas.read_outputs(g)
+    assert g.one.failed[0] == (waits != (0, 0))
+    got = O.bf16_bits_to_f32(bf16_bits(atlas.workspace.logits[:g.logits_end - g.logits_start]))[:, :a.vocab_size]
+    vis = runtime.dense_visibility(runtime.step_descriptor(role, M, atlas.D, cache_len, n_pend), M, sigma)
+    kk, vv = kv_bits[0].copy(), kv_bits[1].copy()
+    want_bits = DO.decode_step(_oracle_weights(model, atlas), kk, vv, tokens, positions, vis, sigma, g.logits_start, g.logits_end)
+    want = O.bf16_bits_to_f32(want_bits)[:, :a.vocab_size]
+    new = bf16_bits(kv)
+    for plane, ref, steps in ((0, kk, 2), (1, vv, 1)):
+        # layer 0 sees no attention: one bf16 step from the order of a projection's sums, which a key's norm and rotation
+        # (four roundings of values that cancel) can make two of the larger operand's
+        x, y = (O.bf16_bits_to_f32(t[0][:, sigma:sigma + M]) for t in (new[plane], ref))
+        assert (np.abs(x - y) <= steps * 2.0 ** -7 * np.maximum(np.abs(y), 2.0 ** -3)).all()
+        assert np.array_equal(new[plane][:, :, :sigma], kv_bits[plane][:, :, :sigma])
+    for x, y in ((got, want),) + tuple((O.bf16_bits_to_f32(new[p][1][:, sigma:sigma + M]), O.bf16_bits_to_f32(r[1][:, sigma:sigma + M]))
+                                       for p, r in ((0, kk), (1, vv))):
+        # one whole int8 step of every value of a normal row (1 / 127 of its maximum of about 3.5 rms) is 2.8e-2, and a
+        # bf16 step of the row itself 4e-3 a layer
+        err = np.linalg.norm(x - y) / np.linalg.norm(y)
+        print(f"[info] {err:.3e}", flush=True)
+        assert err <= 4e-2
+
+
 @pytest.mark.parametrize("name", ["1.7b", "4b"])
-def test_two_layer_step_at_real_dims_stage_by_stage(name):
-    """Two layers of the real width and the real head.  The whole step is compared with the
+def test_two_layer_step_at_real_dims_stage_by_stage(name, monkeypatch):
+    """Two layers of the real width and the real head, as separate launches: a step in one launch does not leave its
+    stages in the workspace.  The whole step is compared with the
     CPU composition of the oracles, and -- much sharper -- every stage of the LAST layer and of
     the head with the oracle applied to the GPU's own input of that stage, which the step's
     workspace still holds.  A wiring mistake (a swapped norm weight, a missing residual, the
@@ -147,6 +201,7 @@ def test_two_layer_step_at_real_dims_stage_by_stage(name):
     from bitmtp_amd.model import BonsaiDecoder
     from bitmtp_amd.runtime import GraphAtlas
     O.build()
+    monkeypatch.setenv("BONSAI_ONE_LAUNCH_STEP", "0")
     sigma, cache_len, M, role = 256, 131, 9, "verify"
     model = BonsaiDecoder.random_init(_args(name, n_layers=2), seed=5, device=DEV)
     atlas = GraphAtlas(model, segment_ladder=(sigma,), threshold=0.9)

@@ -89,7 +89,8 @@ def test_shapes_and_widths_that_keep_the_separate_launches():
     from bitmtp_amd import decode_ops
     from bitmtp_amd.runtime import GraphAtlas
     assert decode_ops.StepBlock.exchange_bytes((2, 3, 2048, 6144, 16, 8), torch.device(DEV)) > 0
-    for shape in ((2, 2, 2048, 6144, 16, 8),        # two layers
+    assert decode_ops.StepBlock.exchange_bytes((2, 2, 2048, 6144, 16, 8), torch.device(DEV)) > 0
+    for shape in ((2, 1, 2048, 6144, 16, 8),        # one layer
                   (2, 3, 1088, 6144, 16, 8),        # half a group of K
                   (2, 3, 8192, 28672, 64, 8),       # more rows than the LDS has room for
                   (2, 3, 2048, 6144, 15, 8),
@@ -107,7 +108,7 @@ def test_argument_checks():
                 h_out=0x8000, status=0x9000, bits=2, n_layers=3, dim=2048, ffn=6144, n_heads=16, n_kv=8, slots=64, sigma=32,
                 max_pos=64, vocab=100, eps=1e-6, scale=0.1)
     for rows, bad in ((0, {}), (1, {}), (17, {}), (9, dict(layers=0)), (9, dict(status=0)), (9, dict(exchange=0x7040)), (9, dict(kv=0x4008)),
-                      (9, dict(embed=0x2008)), (9, dict(sigma=56)), (9, dict(sigma=-1)), (9, dict(dim=2000)), (9, dict(n_layers=2)),
+                      (9, dict(embed=0x2008)), (9, dict(sigma=56)), (9, dict(sigma=-1)), (9, dict(dim=2000)), (9, dict(n_layers=1)),
                       (9, dict(n_heads=17)), (9, dict(bits=4))):
         d = {**good, **bad}
         if set(bad) & {"dim", "n_layers", "n_heads", "bits"}:   # not to be launched with these addresses
