@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from test_step_one_gpu import DEV, _model
+from test_step_one_gpu import BAD_ARGUMENTS, DEV, _model, _refused
 
 pytestmark = pytest.mark.gpu
 
@@ -101,20 +101,9 @@ def test_shapes_and_widths_that_keep_the_separate_launches():
 
 
 def test_argument_checks():
-    import ctypes
     from bitmtp_amd import decode_ops
-    lib = decode_ops.decode_lib()
-    good = dict(layers=0x1000, embed=0x2000, step_in=0x3000, kv=0x4000, cos_table=0x5000, sin_table=0x6000, exchange=0x7000,
-                h_out=0x8000, status=0x9000, bits=2, n_layers=3, dim=2048, ffn=6144, n_heads=16, n_kv=8, slots=64, sigma=32,
-                max_pos=64, vocab=100, eps=1e-6, scale=0.1)
-    for rows, bad in ((0, {}), (1, {}), (17, {}), (9, dict(layers=0)), (9, dict(status=0)), (9, dict(exchange=0x7040)), (9, dict(kv=0x4008)),
-                      (9, dict(embed=0x2008)), (9, dict(sigma=56)), (9, dict(sigma=-1)), (9, dict(dim=2000)), (9, dict(n_layers=1)),
-                      (9, dict(n_heads=17)), (9, dict(bits=4))):
-        d = {**good, **bad}
-        if set(bad) & {"dim", "n_layers", "n_heads", "bits"}:   # not to be launched with these addresses
-            assert decode_ops.StepBlock.exchange_bytes([d[k] for k in ("bits", "n_layers", "dim", "ffn", "n_heads", "n_kv")], torch.device(DEV)) == 0
-        assert lib.bonsai_decode_step_block(ctypes.byref(decode_ops.StepOneDesc(**d)), rows, None) != 0, (rows, bad)
-    assert lib.bonsai_decode_step_block(None, 9, None) != 0
+    _refused(9, [(0, {}), (1, {}), (17, {})] + [(9, bad) for bad in BAD_ARGUMENTS + [dict(sigma=88), dict(dim=2000)]])
+    assert decode_ops.decode_lib().bonsai_decode_step_block(None, 9, None) != 0
 
 
 def test_steps_are_repeated_after_a_launch_that_gave_up():

@@ -130,18 +130,42 @@ def test_shapes_that_keep_the_separate_launches(monkeypatch):
     assert step_one(_model(2, 1024, 512, 8, 4)) is None
 
 
-def test_argument_checks():
+def _refused(width, cases):
+    """Every case is refused by the host.  The other arguments are those of a step that could run, in its own memory, and a
+    shape is known to be refused before the call."""
     import ctypes
     from bitmtp_amd import decode_ops
-    lib = decode_ops.decode_lib()
-    good = dict(layers=0x1000, embed=0x2000, step_in=0x3000, kv=0x4000, cos_table=0x5000, sin_table=0x6000, exchange=0x7000,
-                h_out=0x8000, status=0x9000, bits=2, n_layers=3, dim=2048, ffn=6144, n_heads=16, n_kv=8, slots=64, sigma=32,
-                max_pos=64, vocab=100, eps=1e-6, scale=0.1)
-    for bad in (dict(layers=0), dict(status=0), dict(exchange=0x7040), dict(kv=0x4008), dict(embed=0x2008), dict(sigma=64),
-                dict(sigma=-1), dict(vocab=0), dict(max_pos=0), dict(dim=640), dict(n_layers=1), dict(n_heads=17), dict(bits=4)):
-        d = decode_ops.StepOneDesc(**{**good, **bad})
-        assert lib.bonsai_decode_step_one(ctypes.byref(d), None) != 0, bad
-    assert lib.bonsai_decode_step_one(None, None) != 0
+    from bitmtp_amd.runtime import GraphAtlas
+    model = _model(2, 256, 256, 2, 1)
+    atlas = GraphAtlas(model, segment_ladder=(64,))
+    g = atlas.get_graph(width, 64, "ar")
+    seen = []
+    g.one._launch = lambda d, rows: seen.append(d) or 0    # the arguments of a step, which is not queued
+    norm = decode_ops.FinalNorm(model.norm, 0, width, q=atlas.workspace.l_q, s=atlas.workspace.l_s)
+    g.one.enqueue(model.embed, g.io.step_in, atlas.kv(64), *atlas.rope, 64, 1e-6, atlas.workspace.h[0][:width], width, norm)
+    good = {name: getattr(seen[0], name) for name, _ in decode_ops.StepOneDesc._fields_}
+    for rows, change in cases:
+        d = dict(good)
+        for name, value in change.items():
+            d[name] = good[name] + int(value[1:]) if isinstance(value, str) else value
+        if set(change) & {"dim", "n_layers", "n_heads", "bits"}:
+            shape = [d[k] for k in ("bits", "n_layers", "dim", "ffn", "n_heads", "n_kv")]
+            assert g.one.exchange_bytes(shape, torch.device(DEV)) == 0, shape
+        assert type(g.one)._launch(g.one, decode_ops.StepOneDesc(**d), rows) != 0, (rows, change)
+
+
+#: addresses that are not there or not aligned ("+4": four bytes on), sizes, and the final norm's
+BAD_ARGUMENTS = [dict(layers=0), dict(status=0), dict(exchange="+64"), dict(kv="+8"), dict(embed="+8"), dict(sigma=96),
+                 dict(sigma=-1), dict(vocab=0), dict(max_pos=0), dict(n_layers=1), dict(n_heads=0), dict(bits=4),
+                 dict(norm_w=0), dict(norm_w="+8"), dict(norm_q=0), dict(norm_q="+4"), dict(norm_s=0), dict(norm_s="+2"),
+                 dict(h_out="+4"), dict(norm_out=1 << 40 | 8), dict(norm_rows=-1), dict(norm_first=-1), dict(norm_first=1),
+                 dict(norm_rows=17)]
+
+
+def test_argument_checks():
+    from bitmtp_amd import decode_ops
+    _refused(1, [(1, bad) for bad in BAD_ARGUMENTS + [dict(dim=640)]])
+    assert decode_ops.decode_lib().bonsai_decode_step_one(None, None) != 0
 
 
 @pytest.mark.parametrize("use_graphs", [True, False])
