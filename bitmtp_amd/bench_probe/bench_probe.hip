@@ -8,6 +8,9 @@
 //   * bonsai_probe_grid_barrier    a device-wide barrier among resident workgroups through one
 //                                  counter (what a hand-over inside a persistent kernel costs);
 //                                  the wait is bounded, so every wave exits whatever happens
+//   * bonsai_probe_hand_over       rows passed on among resident workgroups by marks in the rows themselves, without a
+//                                  counter or a fence (what steps in one launch do); bounded waits as well
+//   * bonsai_probe_load_rows       16-byte loads whose 64 lanes touch a given number of rows (cost of a request)
 // Declared in include/bonsai_probe.h.  No reference counterpart.
 #include <hip/hip_runtime.h>
 
@@ -85,9 +88,93 @@ __global__ void __launch_bounds__(256) probe_last_arriver_kernel(unsigned *recor
     if (threadIdx.x == 0 && mode == 1) __hip_atomic_store(&state[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+constexpr int kHandWords = 3;          // 16-byte words of a row a thread looks at, at most
+constexpr int kHandThreads = 512;
+constexpr int kHandSpinLimit = 20000;
+constexpr unsigned kHandEmpty = 0xffffffffu;
+constexpr int kPastL2 = 16;            // sc1
+
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+// Phase p: every workgroup looks for all of row p and then stores its own dwords of row p + 1, `waves` of its waves a part
+// each.  Every wait ends: after kHandSpinLimit looks a workgroup notes it in *error and leaves, and so do the others.
+__global__ void __launch_bounds__(kHandThreads)
+probe_hand_over_kernel(unsigned *rows, unsigned *error, int phases, int dwords, int pause, int waves) {
+    __shared__ int s_bad;
+    const int tid = threadIdx.x, mine = (dwords + (int)gridDim.x - 1) / (int)gridDim.x, first = (int)blockIdx.x * mine;
+    const int piece = (mine + waves - 1) / waves;   // dwords a wave stores
+    const int own = (tid >> 6) * piece + (tid & 63);
+    const bool stores = (tid >> 6) < waves && (tid & 63) < piece && own < mine && first + own < dwords;
+    if (tid == 0) s_bad = 0;
+    __syncthreads();
+    for (int p = 0; p < phases; ++p) {
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(rows + (size_t)p * dwords, 0, 2 * dwords * 4, 0x00020000);
+        for (int z = 0; p > 0 && z < pause; ++z) __builtin_amdgcn_s_sleep(1);
+        v4u v[kHandWords];
+        bool ok = false;
+        for (int spins = 0; !ok && spins < kHandSpinLimit; ++spins) {
+            if (spins) __builtin_amdgcn_s_sleep(1);
+            ok = true;
+#pragma unroll
+            for (int i = 0; i < kHandWords; ++i)
+                v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, tid + i * kHandThreads < dwords / 4 ? (tid + i * kHandThreads) * 16 : 0, 0, kPastL2);
+#pragma unroll
+            for (int i = 0; i < kHandWords; ++i)
+                ok = ok && v[i].x != kHandEmpty && v[i].y != kHandEmpty && v[i].z != kHandEmpty && v[i].w != kHandEmpty;
+            ok = __all(ok);
+        }
+        if (!ok) s_bad = 1;
+        __syncthreads();
+        if (s_bad) break;
+        if (stores) __builtin_amdgcn_raw_buffer_store_b32((v[0].x + (unsigned)p) & 0x7fffffffu, r, (dwords + first + own) * 4, 0, kPastL2);
+        __syncthreads();
+    }
+    if (s_bad && tid == 0) atomicOr(error, 1u);
+}
+
+// `loads` 16-byte loads a lane, 64 / rows lanes a row of 1024 bytes: neighbouring ones or, `turned`, every rows-th one. All in
+// the first 64 KB.
+__global__ void __launch_bounds__(1024) probe_load_rows_kernel(const unsigned *src, int loads, int rows, int turned, unsigned *sink) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned *>(src), 0, 65536, 0x00020000);
+    const int lane = threadIdx.x & 63, per = 64 / rows;
+    const int at = turned ? (lane % rows) * 1024 + (lane / rows) * 16 : (lane / per) * 1024 + (lane % per) * 16;
+    unsigned acc = 0;
+    for (int i = 0; i < loads; i += 8) {
+        v4u v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = __builtin_amdgcn_raw_buffer_load_b128(r, at, (((i >> 3) & 1) * 8 + j) * 64 % 1024, 0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc |= v[j].x ^ v[j].w;
+    }
+    if (acc == 0x12345678u) *sink = acc;
+}
+
 }  // namespace
 
 extern "C" {
+
+int bonsai_probe_hand_over(int workgroups, int values, int phases, int pause, int waves, void *rows, void *error, void *stream) {
+    int dev = 0, cus = 0;
+    if (workgroups < 1 || values < 8 || values % 8 != 0 || values / 8 > kHandWords * kHandThreads || phases < 1 || phases > 1000 || pause < 0 ||
+        pause > 100 || waves < 1 || waves > kHandThreads / 64 || rows == nullptr || error == nullptr || (reinterpret_cast<uintptr_t>(rows) & 15) != 0)
+        return 1;
+    const int mine = (values / 2 + workgroups - 1) / workgroups;
+    if ((mine + waves - 1) / waves > 64) return 1;   // a dword a lane
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 2;
+    if (workgroups > cus) return 1;   // resident at once
+    hipLaunchKernelGGL(probe_hand_over_kernel, dim3(workgroups), dim3(kHandThreads), 0, static_cast<hipStream_t>(stream),
+                       static_cast<unsigned *>(rows), static_cast<unsigned *>(error), phases, values / 2, pause, waves);
+    return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+int bonsai_probe_load_rows(int workgroups, int threads, int loads, int rows, int turned, const void *src, void *sink, void *stream) {
+    if (workgroups < 1 || workgroups > 65536 || threads < 64 || threads > 1024 || threads % 64 != 0 || loads < 8 || loads % 8 != 0 || rows < 1 ||
+        rows > 64 || 64 % rows != 0 || src == nullptr || sink == nullptr || (reinterpret_cast<uintptr_t>(src) & 15) != 0)
+        return 1;
+    hipLaunchKernelGGL(probe_load_rows_kernel, dim3(workgroups), dim3(threads), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const unsigned *>(src), loads, rows, turned, static_cast<unsigned *>(sink));
+    return hipGetLastError() == hipSuccess ? 0 : 2;
+}
 
 int bonsai_probe_last_arriver(int launches, int workgroups, int words, int mode, void *records,
                               void *state, void *stream) {

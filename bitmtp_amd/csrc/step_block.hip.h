@@ -11,7 +11,7 @@
 // and the attention between the first projection and the second row phase, a query head or a part of its slots a workgroup,
 // from the last workgroup on, so that the rows' ones, which everybody waits for, have none of it, of o or of down.
 //
-// Hand-overs, eight a layer of 0.8 - 1.4 us each, are what bounds it now: the nine-row step takes 23 us a layer, and bytes and
+// Hand-overs, eight a layer of 1.0 - 1.4 us each, are what bounds it now: the nine-row step takes 23 us a layer, and bytes and
 // instructions little of that.  To a row phase: two bf16 values and a tag (step and layer) in eight bytes, which nothing but
 // the value itself makes valid; few readers wait for them.  From a row phase: int8 rows and, stored with them, their
 // multipliers, in one of two sets of places, one for each layer, of which a step empties the other; no int8 row holds -128.
@@ -325,7 +325,8 @@ __device__ __forceinline__ v4u words_of(uintptr_t p, int bytes) {   // a buffer 
                (uint32_t)__builtin_amdgcn_readfirstlane(bytes), 0x00020000u};
 }
 // A workgroup's weights and scales of a projection to `lds`, whole lines by eight lanes a row.  (Each lane its own row's pieces,
-// into registers, took 40 cycles of the compute unit's address path a request, 5 us a layer, and everything else waited.)
+// into registers, takes the compute unit's address path 27 ns a request instead of 7, and everything else waited: 5 us a
+// layer.)
 __device__ __forceinline__ void fetch_share(uintptr_t weights, uintptr_t scales, const Share &sh, int bw, int row0, int rows, int n, int on,
                                             uint32_t lds) {
     if (!on || rows <= 0) return;

@@ -8,8 +8,8 @@
 //     shape, 105 KB with the 4B one), and only while no row is on its way: what shares the memory system with a
 //     hand-over delays it (1 us each);
 //   * a row goes from one phase to the next through memory, without a barrier: the producer stores it past its L2 (sc1),
-//     the consumer reads it past its own until every dword has arrived.  Measured between 256 workgroups: 0.8 to 1.2 us
-//     for 2048 to 9728 values, 1.6 to 3 us where everybody polls from the start or a workgroup's values go out in several
+//     the consumer reads it past its own until every dword has arrived.  Measured between 256 workgroups: 1.0 to 1.2 us
+//     for 2048 to 9728 values, 1.9 where everybody polls from the start, 1.5 where a workgroup's values go out in several
 //     stores (a line that is being polled has to be taken out of eight L2s for each of them), hence one store a workgroup
 //     and a pause before the first poll;
 //   * what needs a value of the whole row (the norm's sum of squares, the maximum the quantisation scales by) is computed

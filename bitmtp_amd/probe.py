@@ -42,6 +42,10 @@ def probe_lib() -> ctypes.CDLL:
         lib.bonsai_probe_grid_barrier.restype = ci
         lib.bonsai_probe_last_arriver.argtypes = [ci, ci, ci, ci, vp, vp, vp]
         lib.bonsai_probe_last_arriver.restype = ci
+        lib.bonsai_probe_hand_over.argtypes = [ci, ci, ci, ci, ci, vp, vp, vp]
+        lib.bonsai_probe_hand_over.restype = ci
+        lib.bonsai_probe_load_rows.argtypes = [ci, ci, ci, ci, ci, vp, vp, vp]
+        lib.bonsai_probe_load_rows.restype = ci
         _lib = lib
     return _lib
 
@@ -169,6 +173,78 @@ def last_arriver_us(torch, dev, workgroups: int, words: int, launches: int = 500
     return out
 
 
+def hand_over_us(torch, dev, workgroups: int, values: int, pause: int = 8, waves: int = 1, phases: int = 201) -> float:
+    """Microseconds per row of ``values`` bf16 that ``workgroups`` resident workgroups pass on, each its share, by marks in
+    the rows: (time of a launch of ``phases`` - time of one) / (phases - 1).  Raises if a workgroup's looks ran out."""
+    lib = probe_lib()
+    rows = torch.empty(phases + 1, values // 2, dtype=torch.int32, device=dev)
+    error = torch.zeros(1, dtype=torch.int32, device=dev)
+
+    def run(n):
+        best = float("inf")
+        for _ in range(6):
+            rows.fill_(-1)
+            rows[0] = 1
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            rc = lib.bonsai_probe_hand_over(workgroups, values, n, pause, waves, rows.data_ptr(), error.data_ptr(), _stream_ptr(torch))
+            if rc != 0:
+                raise RuntimeError(f"bonsai_probe_hand_over returned {rc}")
+            e1.record()
+            torch.cuda.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 1e3)
+        if int(error.item()) != 0:
+            raise RuntimeError("hand-over probe: a workgroup's looks ran out")
+        return best
+
+    return (run(phases) - run(1)) / (phases - 1)
+
+
+def load_ns(torch, dev, rows: int, turned: bool, loads: int = 4096) -> float:
+    """Nanoseconds a compute unit takes for one 16-byte load of a wave whose lanes touch ``rows`` rows, neighbouring lanes
+    the same one or (``turned``) different ones, from cache, with sixteen waves on it."""
+    lib = probe_lib()
+    src = torch.zeros(65536 // 4, dtype=torch.int32, device=dev)
+    sink = torch.zeros(1, dtype=torch.int32, device=dev)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+
+    def run(n):
+        def once():
+            rc = lib.bonsai_probe_load_rows(cus, 1024, n, rows, int(turned), src.data_ptr(), sink.data_ptr(), _stream_ptr(torch))
+            if rc != 0:
+                raise RuntimeError(f"bonsai_probe_load_rows returned {rc}")
+        return _time_us(torch, once)
+
+    return (run(loads) - run(loads // 4)) / (loads - loads // 4) / 16 * 1e3
+
+
+def result_lag_us(torch, dev, rounds: int = 50) -> float:
+    """Microseconds from a graph's results in pinned memory to the event behind the graph, as the host sees both."""
+    import time
+    word = torch.zeros(1024, dtype=torch.int32, device=dev)
+    host = torch.zeros(1024, dtype=torch.int32).pin_memory()
+    seen = host.numpy()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        word.add_(1)
+        host.copy_(word, non_blocking=True)
+    done, lags = torch.cuda.Event(), []
+    for _ in range(rounds):
+        torch.cuda.synchronize()
+        before = int(seen[0])
+        g.replay()
+        done.record()
+        until = time.perf_counter() + 1.0
+        while seen[0] == before and time.perf_counter() < until:
+            pass
+        t = time.perf_counter()
+        while not done.query() and time.perf_counter() < until:
+            pass
+        lags.append((time.perf_counter() - t) * 1e6)
+    return sorted(lags)[len(lags) // 2]
+
+
 def main() -> int:
     import torch
     if not torch.cuda.is_available():
@@ -200,6 +276,15 @@ def main() -> int:
     # bf16) per workgroup, nine tokens 64+ (capped)
     for wgs, words in ((128, 8), (128, 64), (768, 8)):
         emit("last_arriver", workgroups=wgs, words_per_record=words, **last_arriver_us(torch, dev, wgs, words))
+    # what steps in one launch are made of: a row from everybody to everybody, the first look behind the data or at once,
+    # a workgroup's values in one store or in several; two workgroups alone
+    for wgs, values, pause, waves in ((2, 128, 0, 1), (256, 2048, 8, 1), (256, 2048, 0, 1), (256, 2048, 8, 4), (256, 6144, 8, 1),
+                                      (256, 9728, 8, 1), (256, 9728, 0, 1), (256, 9728, 8, 8)):
+        emit("hand_over", workgroups=wgs, values=values, pause=pause, waves=waves,
+             us=hand_over_us(torch, dev, wgs, values, pause, waves))
+    for rows in (1, 4, 8, 16, 32, 64):
+        emit("load", rows_of_a_load=rows, ns=load_ns(torch, dev, rows, False), turned_ns=load_ns(torch, dev, rows, True))
+    emit("result_lag", us=result_lag_us(torch, dev))
     return 0
 
 

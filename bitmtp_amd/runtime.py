@@ -441,7 +441,7 @@ class GraphAtlas:
         """One device-to-host copy + synchronisation: (argmax tokens, confidences,
         device-side accepted-prefix length) of the projected rows."""
         if g.io.downloaded:
-            # The results themselves, as the replay's last node writes them: the event behind it is ready 17 us later, and a
+            # The results themselves, as the replay's last node writes them: the event behind it is ready 7 - 11 us later, and a
             # blocking synchronisation wakes the thread up later still.
             out = g.io.out_host.numpy()
             deadline = time.perf_counter() + 0.05

@@ -55,6 +55,19 @@ int bonsai_probe_grid_barrier(int workgroups, int barriers, void *state, void *s
 int bonsai_probe_last_arriver(int launches, int workgroups, int words, int mode, void *records,
                               void *state, void *stream);
 
+/* One launch of `workgroups` persistent workgroups of 512 threads (at most one per CU, else status 1) that pass a row of
+ * `values` bf16 (a multiple of 8, at most 12288) on, `phases` (1..1000) times: each looks for all of row p, past its L2, until no
+ * dword holds 0xffffffff, and stores its share of row p + 1, by `waves` (1..8) of its waves.  A first look comes
+ * `pause` (0..100) sleeps of 64 cycles after the own store.  `rows` holds phases + 1 rows back to back, 16-byte aligned, the
+ * first one of other values and the others of 0xffffffff; `error` is a zeroed word, set to 1 when a workgroup's looks ran
+ * out (all then leave: the kernel always ends). */
+int bonsai_probe_hand_over(int workgroups, int values, int phases, int pause, int waves, void *rows, void *error, void *stream);
+
+/* `loads` (a multiple of 8) 16-byte loads a lane by `workgroups` workgroups of `threads` threads, from the 64 KB at `src`
+ * (16-byte aligned): `rows` (a power of two up to 64) rows of a wave's load, 64 / rows lanes a row, neighbouring ones or,
+ * with `turned`, every rows-th one.  `sink` is 4 writable device bytes (practically never written). */
+int bonsai_probe_load_rows(int workgroups, int threads, int loads, int rows, int turned, const void *src, void *sink, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
