@@ -35,6 +35,7 @@ namespace step_block {
 using step_one::address;
 using step_one::afresh;
 using step_one::afresh_scalar;
+using step_one::ask_layer;
 using step_one::given_up;
 using step_one::kBack;
 using step_one::kBackWaves;
@@ -48,7 +49,7 @@ using step_one::multiplier;
 using step_one::pair16;
 using step_one::pair32;
 using step_one::rsrc_of;
-using step_one::top_of_64;
+using step_one::top_of;
 using step_one::unpack_word;
 using step_one::v2u;
 using step_one::v4f;
@@ -365,12 +366,6 @@ struct Common {
     uint8_t *h, *h2, *qkv, *inner, *parts, *q8, *q8_next;
     int layer8, o8, g8, d8, s8;
 };
-
-__device__ __forceinline__ v2u ask_layer(const Args &a, int l) {
-    const int i = afresh((int)threadIdx.x & 63);
-    return __builtin_amdgcn_raw_buffer_load_b64(rsrc_of(a.layers, a.n_layers * (int)sizeof(Layer)),
-                                                wanted(i < (int)sizeof(Layer) / 8, l * (int)sizeof(Layer) + i * 8), 0, 0);
-}
 
 // ---- all waves: head rows of the attention ---------------------------------------------------
 // Two rows a wave, a query's by lanes 0 - 31 and the key's by 32 - 63; lane i has dims 2 i, 2 i + 1 and, 64 further, their
@@ -848,40 +843,8 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
     const uint32_t sees = (lane & 15) < c.m_rows ? (uint32_t)in[2 + (lane & 15)] : 0u;
 
     const auto norm_row = [&](const v4u *v, const v4u *w, bool ok, uint8_t *rows8, int at8, int phase) -> bool {
-        double ss = 0.0;
         float f[UD][8];
-#pragma unroll
-        for (int i = 0; i < UD; ++i) {
-            unpack_word(v[i], f[i]);
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) ss += (double)(f[i][j] * f[i][j]) + (double)(f[i][j + 1] * f[i][j + 1]);
-        }
-        const double wsum = bonsai_wave::sum64(ss);
-        if (lane == 0) {
-            c.meet.sumsq[wave] = wsum;
-            if (!ok) c.meet.bad = 1;
-        }
-        __syncthreads();
-        if (given_up(c.meet)) return false;
-        double total = 0.0;
-#pragma unroll
-        for (int i = 0; i < kFrontWaves; ++i) total += c.meet.sumsq[i];
-        const float var = (float)total / (float)a.dim;
-        const float rs = 1.0f / sqrtf(var + a.eps);
-        float top = 0.0f;
-#pragma unroll
-        for (int i = 0; i < UD; ++i) {
-            float wf[8];
-            unpack_word(w[i], wf);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                f[i][j] = bf16_round(wf[j] * bf16_round(f[i][j] * rs));
-                top = fmaxf(top, fabsf(f[i][j]));
-            }
-        }
-        top = top_of_64(top);
-        if (lane == 0) c.meet.top[wave] = top;
-        __syncthreads();
+        if (!step_one::norm<UD>(c.meet, v, w, a.dim, a.eps, wave, lane, ok, f)) return false;
         const float s = multiplier(c.meet);
         const int t = afresh(tid);
 #pragma unroll
@@ -890,19 +853,8 @@ __device__ __forceinline__ bool front(const Common &c, int wave, Rope rope) {
         raise(c, phase, rows8, s);
         return true;
     };
-    const auto top_of = [&](const v4u *v, auto units_c) {
-        float top = 0.0f;
-#pragma unroll
-        for (int i = 0; i < decltype(units_c)::value; ++i) {
-            float f[8];
-            unpack_word(v[i], f);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) top = fmaxf(top, fabsf(f[j]));
-        }
-        return top_of_64(top);
-    };
     const auto quant_row = [&](const v4u *v, auto units_c, int k, bool ok, uint8_t *rows8, int at8, int phase) -> bool {
-        const float top = top_of(v, units_c);
+        const float top = top_of<decltype(units_c)::value>(v);
         if (lane == 0) {
             c.meet.top[wave] = top;
             if (!ok) c.meet.bad = 1;

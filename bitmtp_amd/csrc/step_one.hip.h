@@ -298,6 +298,59 @@ __device__ __forceinline__ float multiplier(const Meet &m) {
     return recip * 127.0f;
 }
 
+// Words v of a row, a front wave's share of it, normed with weights w into f; their maximum is one of meet.top's when the
+// waves have met.  false: give up.
+template <int U>
+__device__ __forceinline__ bool norm(Meet &meet, const v4u *v, const v4u *w, int dim, float eps, int wave, int lane, bool ok, float (*f)[8]) {
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        unpack_word(v[i], f[i]);
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) ss += (double)(f[i][j] * f[i][j]) + (double)(f[i][j + 1] * f[i][j + 1]);
+    }
+    const double wsum = bonsai_wave::sum64(ss);
+    if (lane == 0) {
+        meet.sumsq[wave] = wsum;
+        if (!ok) meet.bad = 1;
+    }
+    __syncthreads();
+    if (given_up(meet)) return false;
+    double total = 0.0;
+#pragma unroll
+    for (int i = 0; i < kFrontWaves; ++i) total += meet.sumsq[i];
+    const float var = (float)total / (float)dim;
+    const float rs = 1.0f / sqrtf(var + eps);
+    float top = 0.0f;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        float wf[8];
+        unpack_word(w[i], wf);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            f[i][j] = bf16_round(wf[j] * bf16_round(f[i][j] * rs));
+            top = fmaxf(top, fabsf(f[i][j]));
+        }
+    }
+    top = top_of_64(top);
+    if (lane == 0) meet.top[wave] = top;
+    __syncthreads();
+    return true;
+}
+// Maximum of |value| over a wave's words.
+template <int U>
+__device__ __forceinline__ float top_of(const v4u *v) {
+    float top = 0.0f;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        float f[8];
+        unpack_word(v[i], f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) top = fmaxf(top, fabsf(f[j]));
+    }
+    return top_of_64(top);
+}
+
 // ---- the projections ----------------------------------------------------------------------
 // A lane's loads for one projection.
 template <int N>
@@ -423,6 +476,7 @@ struct Common {
 };
 
 // a layer's addresses, one a lane
+template <class Args>
 __device__ __forceinline__ v2u ask_layer(const Args &a, int l) {
     const int i = afresh((int)threadIdx.x & 63);
     return __builtin_amdgcn_raw_buffer_load_b64(rsrc_of(a.layers, a.n_layers * (int)sizeof(Layer)),
@@ -663,40 +717,8 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
 
     // norm + quantisation of a row of dim values; false: give up
     const auto stage_norm = [&](const v4u *v, const v4u *w, bool ok) -> bool {
-        double ss = 0.0;
         float f[UD][8];
-#pragma unroll
-        for (int i = 0; i < UD; ++i) {
-            unpack_word(v[i], f[i]);
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) ss += (double)(f[i][j] * f[i][j]) + (double)(f[i][j + 1] * f[i][j + 1]);
-        }
-        const double wsum = bonsai_wave::sum64(ss);
-        if (lane == 0) {
-            c.meet.sumsq[wave] = wsum;
-            if (!ok) c.meet.bad = 1;
-        }
-        __syncthreads();
-        if (given_up(c.meet)) return false;
-        double total = 0.0;
-#pragma unroll
-        for (int i = 0; i < kFrontWaves; ++i) total += c.meet.sumsq[i];
-        const float var = (float)total / (float)a.dim;
-        const float rs = 1.0f / sqrtf(var + a.eps);
-        float top = 0.0f;
-#pragma unroll
-        for (int i = 0; i < UD; ++i) {
-            float wf[8];
-            unpack_word(w[i], wf);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                f[i][j] = bf16_round(wf[j] * bf16_round(f[i][j] * rs));
-                top = fmaxf(top, fabsf(f[i][j]));
-            }
-        }
-        top = top_of_64(top);
-        if (lane == 0) c.meet.top[wave] = top;
-        __syncthreads();
+        if (!norm<UD>(c.meet, v, w, a.dim, a.eps, wave, lane, ok, f)) return false;
         const float s = multiplier(c.meet);
         const int t = afresh(tid);
 #pragma unroll
@@ -705,18 +727,6 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
         __syncthreads();   // the back waves' units
         __syncthreads();   // and their results
         return true;
-    };
-    const auto wave_top = [&](const v4u *v, auto units_c) {   // maximum of |value| over the wave's words
-        constexpr int U = decltype(units_c)::value;
-        float top = 0.0f;
-#pragma unroll
-        for (int i = 0; i < U; ++i) {
-            float f[8];
-            unpack_word(v[i], f);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) top = fmaxf(top, fabsf(f[j]));
-        }
-        return top_of_64(top);
     };
 
     for (int layer = 0; layer < a.n_layers; ++layer) {
@@ -949,7 +959,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
             v4u row_a[UQ];
             if (c.rows_o) {
                 const bool ok = receive<UQ>(c.here, row0 + c.lay.att, c.q_dim >> 3, row_a, kPauseLong, limit);
-                const float top = wave_top(row_a, std::integral_constant<int, UQ>{});
+                const float top = top_of<UQ>(row_a);
                 if (lane == 0) {
                     c.meet.top[wave] = top;
                     if (!ok) c.meet.bad = 1;
@@ -991,7 +1001,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
 #pragma unroll
                 for (int i = 0; i < UF; ++i)
                     if (t + i * kFront < (a.ffn >> 3)) *reinterpret_cast<v4u *>(c.raw + (t + i * kFront) * 8) = row_f[i];
-                const float top = wave_top(row_f, std::integral_constant<int, UF>{});
+                const float top = top_of<UF>(row_f);
                 if (lane == 0) {
                     c.meet.top[wave] = top;
                     if (!ok) c.meet.bad = 1;
