@@ -297,13 +297,17 @@ class GraphAtlas:
 
     def _one_launch(self, M: int) -> Optional[decode_ops.StepOne]:
         """What runs the layers of an M-row step of the model, as its weights are now, in one launch."""
+        if M > decode_ops.StepBlock.MAX_ROWS:
+            return None
+        have = self._one if M == 1 else self._block
+        one = step_one(self.model, decode_ops.StepOne if M == 1 else decode_ops.StepBlock, have)
+        if have is not None and one is not have and not self.use_graphs:
+            torch.cuda.synchronize(self.device)   # steps that read the old weights and their table are still queued
         if M == 1:
-            self._one = step_one(self.model, have=self._one)
-            return self._one
-        if M <= decode_ops.StepBlock.MAX_ROWS:
-            self._block = step_one(self.model, decode_ops.StepBlock, self._block)
-            return self._block
-        return None
+            self._one = one
+        else:
+            self._block = one
+        return one
 
     def _capture_one_impl(self, M: int, sigma: int, role: str) -> CapturedGraph:
         if role not in contracts.GRAPH_ROLES:

@@ -79,6 +79,22 @@ def test_a_snapshot_keeps_what_the_model_had():
     assert before.layers[1].w_gu.weight is not model.layers[1].w_gu.weight and before.head.weight is model.head.weight
 
 
+@pytest.mark.parametrize("use_graphs", [False, True])
+def test_old_weights_are_dropped_when_no_step_reads_them(use_graphs, plain, monkeypatch):
+    """Without graphs the step before may still be queued, on whatever stream; a graph holds what it reads."""
+    from bitmtp_amd import runtime
+    atlas = runtime.GraphAtlas.__new__(runtime.GraphAtlas)
+    atlas.model, atlas.device, atlas.use_graphs, atlas._one, atlas._block = _model("cpu"), torch.device("cpu"), use_graphs, None, None
+    waits = []
+    monkeypatch.setattr(torch.cuda, "synchronize", waits.append)
+    monkeypatch.setattr(decode_ops, "StepOne", Recorded)
+    first = atlas._one_launch(1)
+    assert atlas._one_launch(1) is first and not waits
+    atlas.model.layers[1].wo = _other(atlas.model.layers[1].wo, 5)
+    assert atlas._one_launch(1) is not first and atlas._one is not first
+    assert waits == ([] if use_graphs else [atlas.device])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("width", [1, 9])
 def test_steps_follow_replaced_weights(width, plain, monkeypatch):
