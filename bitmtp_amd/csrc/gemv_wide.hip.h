@@ -5,8 +5,8 @@
 // of vector instructions: per scale group (128 of K) the exact int32 sums must become fp32 and meet the
 // group's scale, two operations a result (eight per 16 x 16 results, against two matrix instructions),
 // beside unpacking the weights and arranging the activations.  Counters at 3001 tokens: the vector ALU is
-// busy in 82 % of the cycles with four waves a SIMD (19456 x 2560, 64x256) and in 60 % with two
-// (2560 rows, 128x256), the matrix cores in 30-37 %.  So
+// busy in 85 % of the cycles with four waves a SIMD (gate|up 19456 x 2560, 64x256) and in 60 % with two
+// (2560 rows, 128x256), the matrix cores in 30-36 %.  So
 //   * v_mfma_i32_32x32x32_i8: half the matrix instructions of the 16 x 16 form;
 //   * weights are unpacked to 64 times their value (mfma_unpack64), which needs no offset term -- the
 //     other forms feed -2 sum(a) through the accumulator, 8 more matrix instructions per 16 x 64 x 64 --
