@@ -90,6 +90,37 @@ def test_ar_tokens_do_not_depend_on_the_layer_form_at_full_size(full, monkeypatc
         assert torch.equal(logits.view(torch.int16), runs[0][1].view(torch.int16))
 
 
+@pytest.mark.parametrize("name,n_prompt,n_new", [("1.7b", 256, 200), ("4b", 1000, 120)])
+def test_ar_tokens_of_steps_in_one_launch_at_full_size(name, n_prompt, n_new, monkeypatch):
+    """Greedy AR decoding with each step in one launch and with separate launches, of a decoder that predicts with a margin:
+    layers that add a small part to the residual stream, a successor for every token.  The same tokens; of the logits behind
+    the last one, as in the comparisons of test_step_one_gpu, at most a whole int8 step of every value of a row (2.8e-2)
+    and bf16 steps of the row."""
+    from bitmtp_amd import generate
+    from bitmtp_amd.model import BonsaiDecoder
+    from bitmtp_amd.runtime import GraphAtlas
+    model = BonsaiDecoder.random_init(_args(name), seed=3, device=DEV)
+    for lw in model.layers:
+        lw.wo.weight_scale.mul_(2.0 ** -10)
+        lw.w_down.weight_scale.mul_(2.0 ** -10)
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    model.embed = model.embed[torch.randperm(model.args.vocab_size, generator=gen, device=DEV)].contiguous()
+    prompt = np.random.default_rng(29).integers(0, model.args.vocab_size, n_prompt).tolist()
+    runs = []
+    for flag in ("1", "0"):
+        monkeypatch.setenv("BONSAI_ONE_LAUNCH_STEP", flag)
+        atlas = GraphAtlas(model, segment_ladder=(2048,), threshold=0.9, roles=("ar",))
+        print(f"[case] {name}: AR {n_new} tokens, BONSAI_ONE_LAUNCH_STEP={flag}", flush=True)
+        toks, _ = generate.ar_generate(atlas, prompt, max_gen_len=n_new)
+        g = atlas.get_graph(1, 2048, "ar")
+        assert (g.one is not None) == (flag == "1") and (g.one is None or g.one.failed[0] == 0)
+        runs.append((toks, atlas.workspace.logits[0, :model.args.vocab_size].float()))
+        del atlas, g
+    (t1, l1), (t0, l0) = runs
+    assert t1 == t0 and len(set(t1)) > n_new // 2
+    assert float((l1 - l0).norm() / l0.norm()) <= 4e-2
+
+
 def test_graph_replay_equals_eager_at_full_size(full):
     from bitmtp_amd.runtime import GraphAtlas
     name, sigma, model, atlas = full
