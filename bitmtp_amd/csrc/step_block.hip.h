@@ -11,7 +11,7 @@
 // and the attention between the first projection and the second row phase, a query head or a part of its slots a workgroup,
 // from the last workgroup on, so that the rows' ones, which everybody waits for, have none of it, of o or of down.
 //
-// Hand-overs, eight a layer of 1.0 - 1.4 us each, are what bounds it now: the nine-row step takes 23 us a layer, and bytes and
+// Hand-overs, eight a layer of 1.0 - 1.4 us each, are what bounds it now: the nine-row step takes 22 us a layer, and bytes and
 // instructions little of that.  To a row phase: two bf16 values and a tag (step and layer) in eight bytes, which nothing but
 // the value itself makes valid; few readers wait for them.  From a row phase: int8 rows and, stored with them, their
 // multipliers, in one of two sets of places, one for each layer, of which a step empties the other; no int8 row holds -128.
@@ -24,9 +24,9 @@
 // owns a stretch of K for all rows of the workgroup and reads that stretch of the tokens once; the waves' results meet in
 // LDS in the order of K.
 //
-// Layers of nine rows, 1.7B / 4B shape, us at a history of 24, 300, 1500: 934 / 961 / 1034 -> 642 / 677 / 792 and
-// 1521 / 1543 / 1657 -> 1027 / 1125 / 1316; two rows (1.7B) 812 / 818 / 900 -> 586 / 614 / 728; sixteen 987 / 1011 / 1089 ->
-// 712 / 745 / 866.
+// Layers of nine rows, 1.7B / 4B shape, us at a history of 24, 300, 1500: 934 / 961 / 1034 -> 608 / 654 / 773 and
+// 1521 / 1543 / 1657 -> 1004 / 1107 / 1298; two rows (1.7B) 812 / 818 / 900 -> 555 / 597 / 716; sixteen 987 / 1011 / 1089 ->
+// 658 / 705 / 830.
 #ifndef BONSAI_STEP_BLOCK_HIP_H
 #define BONSAI_STEP_BLOCK_HIP_H
 
