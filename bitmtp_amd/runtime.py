@@ -457,8 +457,10 @@ class GraphAtlas:
                     g.io.uploaded.synchronize()
                     break
         else:
+            stream = torch.cuda.current_stream(self.device)
+            stream.wait_event(g.io.uploaded)   # (the step may be on another one)
             g.io.out_host.copy_(g.io.out, non_blocking=True)
-            torch.cuda.current_stream(self.device).synchronize()
+            stream.synchronize()
         if g.one is not None and g.one.failed[0] > 1:
             raise RuntimeError("a decode step did not end")
         rows = g.logits_end - g.logits_start

@@ -205,3 +205,29 @@ def test_final_norm(bits, dim, ffn, n_heads, n_kv, width, first, rows):
         torch.cuda.synchronize()
         assert torch.equal(q, want_q) and torch.equal(s, want_s) and torch.equal(out, want_out)
         assert g.one.failed[0] == (waits != (0, 0))
+
+
+@pytest.mark.parametrize("use_graphs", [True, False])
+def test_results_read_on_another_stream(use_graphs):
+    """Where separate launches stand in for a step, too, its results are those of that step on whatever stream they are read."""
+    from bitmtp_amd.runtime import GraphAtlas
+    atlas = GraphAtlas(_model(2, 1024, 512, 8, 4), segment_ladder=(64,), use_graphs=use_graphs)
+    g = atlas.get_graph(9, 64, "verify")
+    tokens, positions = list(range(9)), list(range(4, 13))
+    want = []
+    for first in (7, 0):
+        atlas.replay(g, [first] + tokens[1:], positions, 5)
+        want.append(atlas.read_outputs(g)[0].copy())
+    assert (want[0] != want[1]).any()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    for separate in (0, 1):
+        atlas._separate_for = separate
+        atlas.replay(g, tokens, positions, 5)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(20000000)
+            atlas._separate_for = separate
+            atlas.replay(g, [7] + tokens[1:], positions, 5)
+        assert (atlas.read_outputs(g)[0] == want[0]).all(), separate
+        stream.synchronize()
