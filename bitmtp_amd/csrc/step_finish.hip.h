@@ -32,6 +32,7 @@ constexpr int kWaves = 8, kThreads = kWaves * 64;
 constexpr int kGroups = 64;                    // workgroups: the rows of a norm, the tasks of a repeated step
 constexpr int kRows = 16;
 constexpr uint32_t kLongest = 2000000000;      // 20 s, which no task waits unless an earlier one is lost
+constexpr uint32_t kLost = 2;                  // the mark and the status then: the tasks' numbers are of no use to later steps
 enum { kEpoch, kGaveUp, kDrawn, kDone, kLeft, kControlWords };   // words of the exchange memory, with those of the step's launch
 
 struct Places {   // byte offsets of the rows of a repeated step, behind the exchange memory (its residual stream is h_out)
@@ -418,7 +419,10 @@ __device__ __forceinline__ void step_again(const Args &a, Meet &meet) {
         }
         __syncthreads();
         if (__builtin_amdgcn_readfirstlane(meet.lost)) {
-            if (tid == 0) *a.status = 2;
+            if (tid == 0) {
+                control[kGaveUp] = kLost;
+                *a.status = (int32_t)kLost;
+            }
             return;
         }
         __threadfence();   // what earlier tasks stored, wherever they ran
@@ -443,8 +447,13 @@ finish_kernel(const Args a) {
         x = word_of(a.h_out + (size_t)(a.norm_first + row) * a.dim, threadIdx.x);
         w = word_of(a.norm_w, threadIdx.x);
     }
-    if (control[kGaveUp] == 0) {
+    const uint32_t mark = control[kGaveUp];
+    if (mark == 0) {
         if (row < a.norm_rows) final_norm(a, meet, row, x, w);
+        return;
+    }
+    if (mark == kLost) {
+        if (row == 0 && threadIdx.x == 0) *a.status = (int32_t)kLost;   // (over the 1 of the step's own launch)
         return;
     }
     step_again<BITS>(a, meet);

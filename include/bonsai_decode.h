@@ -166,7 +166,7 @@ int bonsai_decode_attention_rope_parts(const void *xqkv, const void *q_norm_w, c
  * vocabulary and, where the first one left, does the step again before that, with whatever workgroups it gets.  So
  * all results are right in stream order either way; *status says that it took milliseconds, and that separate launches may
  * serve better while something else runs on the device.  (2: that launch waited 20 s for a workgroup of its own, and the
- * results are not there.)
+ * results are not there; nor are those of later steps, until the exchange memory is reset.)
  *
  *   layers    device array of n_layers records of 12 pointers: packed weights of q|k|v, o, gate|up and down, their
  *             bf16 group scales in the same order, input and post-attention norm weights, q and k norm weights;

@@ -207,6 +207,30 @@ def test_final_norm(bits, dim, ffn, n_heads, n_kv, width, first, rows):
         assert g.one.failed[0] == (waits != (0, 0))
 
 
+@pytest.mark.parametrize("width", [1, 9])
+def test_a_step_that_did_not_end_is_told_until_the_memory_is_reset(width):
+    """Behind a step of which a task was lost (the mark is set from the host) no step pretends to have results."""
+    from bitmtp_amd.runtime import GraphAtlas
+    atlas = GraphAtlas(_model(2, 1024, 512, 8, 4), segment_ladder=(64,))
+    g = atlas.get_graph(width, 64, "ar")
+    step = (g, list(range(width)), list(range(5, 5 + width)), 5)
+    atlas.replay(*step)
+    want = atlas.read_outputs(g)[0].copy()
+    g.one.exchange[4:8].view(torch.int32).fill_(2)
+    for _ in range(2):
+        g.one.failed[0] = 0
+        atlas.replay(*step)
+        torch.cuda.synchronize()
+        assert g.one.failed[0] == 2
+        with pytest.raises(RuntimeError, match="did not end"):
+            atlas.read_outputs(g)
+        with pytest.raises(RuntimeError, match="did not end"):
+            atlas.replay(*step)
+    g.one.reset()
+    atlas.replay(*step)
+    assert (atlas.read_outputs(g)[0] == want).all() and g.one.failed[0] == 0
+
+
 @pytest.mark.parametrize("use_graphs", [True, False])
 def test_results_read_on_another_stream(use_graphs):
     """Where separate launches stand in for a step, too, its results are those of that step on whatever stream they are read."""
