@@ -1893,7 +1893,8 @@ extern "C" int bonsai_decode_step_one_reset(int bits, int n_layers, int dim, int
     if (f.build < 0 || !exchange || (reinterpret_cast<uintptr_t>(exchange) & 127)) return BONSAI_DECODE_ERR_ARG;
     hipLaunchKernelGGL(step_one::exchange_reset_kernel, dim3(256), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<step_one::v4u *>(exchange), (size_t)f.bytes / 16, (size_t)step_one::kControlBytes / 16, (size_t)f.marked / 16);
-    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+    return step_one::look_at_dies(exchange, n_kv, cu_count(), static_cast<hipStream_t>(stream)) == hipSuccess ? BONSAI_DECODE_OK
+                                                                                                             : BONSAI_DECODE_ERR_LAUNCH;
 }
 
 static bool step_args_ok(const bonsai_step_one_desc *d) {
@@ -1992,7 +1993,8 @@ extern "C" int bonsai_decode_step_block_reset(int bits, int n_layers, int dim, i
         return BONSAI_DECODE_ERR_LAUNCH;
     hipLaunchKernelGGL(step_block::reset_kernel, dim3(256), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<step_block::v4u *>(exchange), (size_t)f.bytes / 16, (size_t)f.clear / 16);
-    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+    return step_one::look_at_dies(exchange, n_kv, cu_count(), static_cast<hipStream_t>(stream)) == hipSuccess ? BONSAI_DECODE_OK
+                                                                                                             : BONSAI_DECODE_ERR_LAUNCH;
 }
 
 extern "C" int bonsai_decode_step_block(const bonsai_step_one_desc *d, int rows, void *stream) {

@@ -24,9 +24,12 @@
 // owns a stretch of K for all rows of the workgroup and reads that stretch of the tokens once; the waves' results meet in
 // LDS in the order of K.
 //
-// Layers of nine rows, 1.7B / 4B shape, us at a history of 24, 300, 1500: 934 / 961 / 1034 -> 608 / 654 / 773 and
-// 1521 / 1543 / 1657 -> 1004 / 1107 / 1298; two rows (1.7B) 812 / 818 / 900 -> 555 / 597 / 716; sixteen 987 / 1011 / 1089 ->
-// 658 / 705 / 830.
+// The rows of q|k|v are dealt out by kv head, so that the hand-over to the attention stays within a die (near_heads of
+// step_one.hip.h): nine rows 610 -> 594 us (1.7B shape), 1006 -> 992 (4B), sixteen 661 -> 636.
+//
+// Layers of nine rows, 1.7B / 4B shape, us at a history of 24, 300, 1500: 934 / 961 / 1034 -> 590 / 645 / 761 and
+// 1521 / 1543 / 1657 -> 988 / 1092 / 1289; two rows (1.7B) 812 / 818 / 900 -> 539 / 581 / 702; sixteen 987 / 1011 / 1089 ->
+// 637 / 692 / 817.
 #ifndef BONSAI_STEP_BLOCK_HIP_H
 #define BONSAI_STEP_BLOCK_HIP_H
 
@@ -37,6 +40,7 @@ using step_one::afresh;
 using step_one::afresh_scalar;
 using step_one::ask_layer;
 using step_one::given_up;
+using step_one::HeadOrder;
 using step_one::kBack;
 using step_one::kBackWaves;
 using step_one::kFront;
@@ -67,6 +71,9 @@ constexpr int kMostLds = 159 * 1024;        // beside what is declared in place
 constexpr uint32_t kEmpty = 0x80808080u;    // int8 rows hold no -128, a multiplier is positive
 constexpr int kCopies = 8;                  // of the multipliers' line, one for each XCD's workgroups
 constexpr int kNap = 1;                     // of 64 cycles, between two looks
+// .. and before a row's workgroup looks for its row (27 ns each): none 593, 10 588, 20 589 us a nine-row step (1.7B shape), 991,
+// 984 and 993 with the 4B one.
+constexpr int kPause = 10;
 constexpr int kVPitch = 272, kOPitch = 132; // bytes of a slot's values, floats of a row's sums in LDS
 
 struct Args {
@@ -157,6 +164,12 @@ struct Lds {
 __device__ __forceinline__ void hand_over(const __amdgpu_buffer_rsrc_t rows, int value, uint32_t d, uint32_t tag) {
     __builtin_amdgcn_raw_buffer_store_b64(v2u{d, tag}, rows, value * 4, 0, kDeviceScope);
 }
+__device__ __forceinline__ void hand_over_near(const __amdgpu_buffer_rsrc_t rows, int value, uint32_t d, uint32_t tag, bool near) {
+    if (near)
+        __builtin_amdgcn_raw_buffer_store_b64(v2u{d, tag}, rows, value * 4, 0, 0);
+    else
+        hand_over(rows, value, d, tag);
+}
 // (The check of the limit on its own, before the spins: with first_spin of step_one.hip.h in its place, which is right as
 // well, a nine-row step of the 1.7B shape takes 643 us instead of 612.  A one-token step has it the other way round: 396
 // with first_spin, 401 with this.)
@@ -204,6 +217,7 @@ template <int U>
 __device__ __forceinline__ bool receive(const uint8_t *row, int words, uint32_t tag, v4u *v, uint32_t limit) {
     const int tid = afresh((int)threadIdx.x);
     const __amdgpu_buffer_rsrc_t r = rsrc_of(row, words * 32);
+    for (int z = 0; z < kPause; ++z) __builtin_amdgcn_s_sleep(1);
     struct Both {
         v4u x[U], y[U];
     } both;
@@ -328,23 +342,27 @@ __device__ __forceinline__ v4u words_of(uintptr_t p, int bytes) {   // a buffer 
 // A workgroup's weights and scales of a projection to `lds`, whole lines by eight lanes a row.  (Each lane its own row's pieces,
 // into registers, takes the compute unit's address path 27 ns a request instead of 7, and everything else waited: 5 us a
 // layer.)
-__device__ __forceinline__ void fetch_share(uintptr_t weights, uintptr_t scales, const Share &sh, int bw, int row0, int rows, int n, int on,
+// Row i of the share is row place(i) of n; the scales of its first `run` rows are those of neighbouring rows, of the others as
+// well (pairs: of the gate rows, of the up rows).
+template <class Place>
+__device__ __forceinline__ void fetch_share(uintptr_t weights, uintptr_t scales, const Share &sh, int bw, int rows, int run, int n, Place place, int on,
                                             uint32_t lds) {
     if (!on || rows <= 0) return;
     const int lane = afresh((int)threadIdx.x & 63);
-    const int row_bytes = sh.chunks * 16, half_n = sh.pairs ? n >> 1 : n, first = sh.pairs ? row0 >> 1 : row0;
+    const int row_bytes = sh.chunks * 16;
     const v4u rw = words_of(weights, n * row_bytes), rs = words_of(scales, n * sh.groups * 2);
     const int recip = 65536 / sh.blocks + 1;
     for (int i = bw; i < sh.tiles * sh.blocks * 2; i += kBackWaves) {
         const int tile = ((i >> 1) * recip) >> 16, block = (i >> 1) - tile * sh.blocks;
         const int r = (i & 1) * 8 + (lane >> 3), row = tile * 16 + r, chunk = block * 8 + ((lane & 7) ^ key_of(r));
-        const int at = first + (sh.pairs ? (row & 1) * half_n + (row >> 1) : row);
-        fetch<16>(rw, wanted(row < rows && chunk < sh.chunks, at * row_bytes + chunk * 16), (uint32_t)__builtin_amdgcn_readfirstlane((int)lds + i * 1024));
+        fetch<16>(rw, wanted(row < rows && chunk < sh.chunks, place(row) * row_bytes + chunk * 16), (uint32_t)__builtin_amdgcn_readfirstlane((int)lds + i * 1024));
     }
-    const int bytes = (sh.pairs ? rows >> 1 : rows) * sh.groups * 2, parts = sh.part_bytes >> 8;
+    const int row_scales = sh.groups * 2, bytes = (sh.pairs ? rows >> 1 : rows) * row_scales, parts = sh.part_bytes >> 8;
+    const int from[2] = {place(0) * row_scales, place(sh.pairs ? 1 : run) * row_scales}, next = run * row_scales;
     for (int i = bw; i < (sh.pairs ? 2 * parts : parts); i += kBackWaves) {
         const int up = i >= parts, at = (i - up * parts) * 256 + lane * 4;
-        fetch<4>(rs, wanted(at < bytes, (first + up * half_n) * sh.groups * 2 + at),
+        const bool behind = !sh.pairs && at >= next;
+        fetch<4>(rs, wanted(at < bytes, (up || behind ? from[1] : from[0]) + (behind ? at - next : at)),
                  (uint32_t)__builtin_amdgcn_readfirstlane((int)lds + sh.weight_bytes + i * 256));
     }
 }
@@ -355,8 +373,10 @@ struct Common {
     Share sq, so, sg, sd;
     int rows_q, rows_o, rows_g, rows_d;
     uint32_t epoch;
-    bool attends, is_row;
+    bool attends, is_row, near;
     int n, hide, kvh, unit, split, head, per, splits, room;
+    HeadOrder order;
+    int head_row0;   // of the kv head's rows of q|k|v, the workgroup's first
     uint8_t *smem;
     int wave_bytes;
     const uint8_t *once, *gate;
@@ -401,14 +421,15 @@ __device__ __forceinline__ bool head_rows(const Common &c, int l, int wave, cons
     const int lane = c.lane, word = lane & 31;
     const bool key = lane >= 32, own = (c.split + 1) * c.per > c.n;
     const __amdgpu_buffer_rsrc_t r = rsrc_of(c.qkv + (size_t)wave * c.n_qkv * 4, c.n_qkv * 4);
-    const int at = (key ? c.a.n_heads + c.kvh : c.head) * 512 + word * 8;
+    const int of_head = c.kvh * c.order.rows() * 4;
+    const int at = of_head + (key ? c.gqa : c.head - c.kvh * c.gqa) * 512 + word * 8;
     struct In {
         v2u lo, hi, v;
     } in;
     if (!look(in, limit, [&](In &t) {
             t.lo = __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, kDeviceScope);
             t.hi = __builtin_amdgcn_raw_buffer_load_b64(r, at, 256, kDeviceScope);
-            t.v = __builtin_amdgcn_raw_buffer_load_b64(r, lane * 8, (c.a.n_heads + c.a.n_kv + c.kvh) * 512, kDeviceScope);
+            t.v = __builtin_amdgcn_raw_buffer_load_b64(r, lane * 8, of_head + (c.gqa + 1) * 512, kDeviceScope);
         }, [&](const In &t) { return (bool)__all(((t.lo.y == tag) & (t.hi.y == tag) & (t.v.y == tag)) | (!own & (key | ((t.lo.y == tag) & (t.hi.y == tag))))); }))
         return false;
     const auto lo_of = [](uint32_t p) { return __uint_as_float(p << 16); };
@@ -574,10 +595,13 @@ template <int BITS, int SQ, int TQ, int SO, int SG, int TG, int SD>
 __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
     const Args &a = c.a;
     const auto lds_of = [](const uint8_t *p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)p; };
-    const auto fetch_q = [&](const v2u &t, int on) { fetch_share(address(t, 0), address(t, 4), c.sq, bw, (c.wg - c.sq.first) * c.sq.rows, c.rows_q, c.n_qkv, on, lds_of(c.once)); };
-    const auto fetch_o = [&](const v2u &t) { fetch_share(address(t, 1), address(t, 5), c.so, bw, (c.wg - c.so.first) * c.so.rows, c.rows_o, a.dim, 1, lds_of(c.once)); };
-    const auto fetch_g = [&](const v2u &t) { fetch_share(address(t, 2), address(t, 6), c.sg, bw, (c.wg - c.sg.first) * c.sg.rows, c.rows_g, 2 * a.ffn, 1, lds_of(c.gate)); };
-    const auto fetch_d = [&](const v2u &t) { fetch_share(address(t, 3), address(t, 7), c.sd, bw, (c.wg - c.sd.first) * c.sd.rows, c.rows_d, a.dim, 1, lds_of(c.once)); };
+    const auto from = [&](const Share &sh) { return [&](int row) { return (c.wg - sh.first) * sh.rows + row; }; };
+    const auto head_row = [&](int row) { return c.order.row_of(c.kvh, c.head_row0 + row); };
+    const auto in_turn = [&](int row) { return c.wg * c.sg.rows / 2 + (row & 1) * a.ffn + (row >> 1); };   // gate, up
+    const auto fetch_q = [&](const v2u &t, int on) { fetch_share(address(t, 0), address(t, 4), c.sq, bw, c.rows_q, kHd - c.head_row0 % kHd, c.n_qkv, head_row, on, lds_of(c.once)); };
+    const auto fetch_o = [&](const v2u &t) { fetch_share(address(t, 1), address(t, 5), c.so, bw, c.rows_o, c.rows_o, a.dim, from(c.so), 1, lds_of(c.once)); };
+    const auto fetch_g = [&](const v2u &t) { fetch_share(address(t, 2), address(t, 6), c.sg, bw, c.rows_g, c.rows_g, 2 * a.ffn, in_turn, 1, lds_of(c.gate)); };
+    const auto fetch_d = [&](const v2u &t) { fetch_share(address(t, 3), address(t, 7), c.sd, bw, c.rows_d, c.rows_d, a.dim, from(c.sd), 1, lds_of(c.once)); };
     v2u cur = ask_layer(a, 0);
     fetch_q(cur, 1);
     rope.ask(cur);
@@ -730,9 +754,10 @@ __device__ __forceinline__ bool back(const Common &c, int bw, Rope rope) {
         }
         if (c.rows_q) {
             const __amdgpu_buffer_rsrc_t to = rsrc_of(c.qkv, kRows * c.n_qkv * 4);
+            const int at_q = c.kvh * c.order.rows() + c.head_row0;
             if (!project(Taken<BITS, SQ, TQ>{}, Two{}, c.sq, c.rows_q, rows8, c.once, limit,
                          [&](int token, int row, auto v, float s) {
-                             hand_over(to, token * c.n_qkv + c.wg * c.sq.rows + row, pack_bf16(v[0] / s, v[1] / s), tag);
+                             hand_over_near(to, token * c.n_qkv + at_q + row, pack_bf16(v[0] / s, v[1] / s), tag, c.near);
                          }))
                 return false;
         }
@@ -1059,19 +1084,20 @@ step_block_kernel(const Args a) {
     __shared__ Meet meet;
     const int groups = a.groups, gqa = a.n_heads / a.n_kv;
     const int q_dim = a.n_heads * kHd, n_qkv = (a.n_heads + 2 * a.n_kv) * kHd;
-    const Share sq(BITS, a.dim, n_qkv, groups, false, false), so(BITS, q_dim, a.dim, groups, false, true), sg(BITS, a.dim, 2 * a.ffn, groups, true, false),
-        sd(BITS, a.ffn, a.dim, groups, false, true);
-    const auto mine = [wg](const Share &s, int n) {
-        if (wg < s.first) return 0;
-        const int left = n - (wg - s.first) * s.rows;
+    const HeadOrder order{a.n_heads, a.n_kv, gqa};
+    const Share sq(BITS, a.dim, order.rows(), groups / a.n_kv, false, false), so(BITS, q_dim, a.dim, groups, false, true),
+        sg(BITS, a.dim, 2 * a.ffn, groups, true, false), sd(BITS, a.ffn, a.dim, groups, false, true);
+    const auto part = [](const Share &s, int n, int i) {
+        const int left = n - i * s.rows;
         return left < 0 ? 0 : (left < s.rows ? left : s.rows);
     };
-    const int rows_q = mine(sq, n_qkv), rows_o = mine(so, a.dim), rows_g = mine(sg, 2 * a.ffn), rows_d = mine(sd, a.dim);
+    const auto mine = [wg, part](const Share &s, int n) { return wg < s.first ? 0 : part(s, n, wg - s.first); };
+    const int back_wg = groups - 1 - wg;   // the rows' workgroups have no part of the attention
+    const int kvh = back_wg % a.n_kv, unit = back_wg / a.n_kv, split = unit / gqa;
+    const int rows_q = part(sq, order.rows(), unit), rows_o = mine(so, a.dim), rows_g = mine(sg, 2 * a.ffn), rows_d = mine(sd, a.dim);
     const auto in = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)a.step_in;
     const int n = in[0] < 0 ? 0 : (in[0] < a.sigma ? in[0] : a.sigma);   // as everywhere: a history within its slots
     // a head's slots: the history and, behind it, the block's rows, in parts of at least 64
-    const int back_wg = groups - 1 - wg;   // the rows' workgroups have none
-    const int kvh = back_wg % a.n_kv, unit = back_wg / a.n_kv, split = unit / gqa;
     const int head = kvh * gqa + unit - split * gqa;
     const int room = room_of(groups, a.n_heads);
     const int total = n + a.rows;
@@ -1091,7 +1117,7 @@ step_block_kernel(const Args a) {
     const Lds lds(sq, so, sg, sd, q_dim, TQ > TG ? TQ : TG);
     const size_t set8 = (size_t)a.n_layers * at.layer8;
     const Common c{a, wg, tid & 63, gqa, q_dim, n_qkv, a.rows, sq, so, sg, sd, rows_q, rows_o, rows_g, rows_d, epoch, attends, is_row,
-                   n, in[1], kvh, unit, split, head, per, splits, room, smem, lds.wave, smem + lds.once, smem + lds.gate, reinterpret_cast<uint16_t *>(smem),
+                   step_one::near_heads(state, wg), n, in[1], kvh, unit, split, head, per, splits, room, order, unit * sq.rows, smem, lds.wave, smem + lds.once, smem + lds.gate, reinterpret_cast<uint16_t *>(smem),
                    reinterpret_cast<float *>(smem + lds.resid), reinterpret_cast<float *>(smem + lds.mult), meet, a.exchange + at.h, a.exchange + at.h2,
                    a.exchange + at.qkv, a.exchange + at.inner, a.exchange + at.parts, a.exchange + at.q8 + (epoch & 1) * set8, a.exchange + at.q8 + (~epoch & 1) * set8, at.layer8, at.o8, at.g8, at.d8, at.s8};
     if (tid == 0) meet.bad = 0;
@@ -1155,7 +1181,8 @@ inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, 
         return f;
     const int64_t n_qkv = (int64_t)(n_heads + 2 * n_kv) * kHd;
     if (2 * (int64_t)ffn * dim >= kOob || n_qkv * dim >= kOob) return f;   // 32-bit offsets into a matrix
-    const Share sq(bits, dim, (int)n_qkv, groups, false, false), so(bits, q_dim, dim, groups, false, true), sg(bits, dim, 2 * ffn, groups, true, false),
+    const HeadOrder order{n_heads, n_kv, n_heads / n_kv};
+    const Share sq(bits, dim, order.rows(), groups / n_kv, false, false), so(bits, q_dim, dim, groups, false, true), sg(bits, dim, 2 * ffn, groups, true, false),
         sd(bits, ffn, dim, groups, false, true);
     const Places at(n_layers, dim, ffn, n_heads, n_kv, groups);
     const auto words = [](int k) { return (k / 8 + kFront - 1) / kFront; };

@@ -387,10 +387,10 @@ __device__ __forceinline__ void do_task(const Args &a, Meet &meet, const Task &t
             final_norm(a, meet, t.index, word_of(a.h_out + (size_t)(a.norm_first + t.index) * a.dim, word), word_of(a.norm_w, word));
             break;
         }
-        default:   // (all but the control words, the first one of which others still look at)
+        default:   // (all but the control words: others still look at the first ones, and where the dies are stays)
             for (uint32_t i = (uint32_t)(t.index * kThreads + tid); i < a.words; i += kGroups * kThreads) {
                 const uint32_t v = i >= a.mark_from && i < a.mark_to ? a.mark : 0u;
-                if (i >= (kControlWords + 3) / 4) reinterpret_cast<v4u *>(a.exchange)[i] = v4u{v, v, v, v};
+                if (i >= step_one::kControlBytes / 16) reinterpret_cast<v4u *>(a.exchange)[i] = v4u{v, v, v, v};
             }
     }
 }

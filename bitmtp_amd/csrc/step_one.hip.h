@@ -12,6 +12,9 @@
 //     for 2048 to 9728 values, 1.9 where everybody polls from the start, 1.5 where a workgroup's values go out in several
 //     stores (a line that is being polled has to be taken out of eight L2s for each of them), hence one store a workgroup
 //     and a pause before the first poll;
+//   * q|k|v's rows are dealt out by kv head, so that the hand-over to the attention, and of its parts, stays within a die's
+//     L2 (near_heads): 0.2 us instead of 0.6 between two workgroups.  With the pauses that fit it the 1.7B shape takes 379 /
+//     432 / 483 us at a history of 24 / 300 / 1500 (before: 386 / 455 / 517), the 4B one 698 / 771 / 871 (720 / 803 / 902);
 //   * what needs a value of the whole row (the norm's sum of squares, the maximum the quantisation scales by) is computed
 //     by every workgroup from the row it has read anyway.
 // What bounds it now is the length of the chain: per phase a hand-over, about 0.8 us for norm and quantisation, 0.5 us
@@ -52,7 +55,14 @@ constexpr int kRounds = 2;                 // rounds of eight slots a wave reque
 constexpr int kPartEntries = kHd + 4;      // 8-byte entries of a part: 128 sums, maximum, sum, pad
 constexpr uint32_t kStartTicks = 500000;   // 5 ms of the 100 MHz counter
 constexpr uint32_t kRunTicks = 20000000;   // 200 ms
-constexpr int kPauseRow = 8, kPauseLong = 10;  // s_sleep(1) steps before the first poll (27 ns each)
+// s_sleep(1) steps (27 ns each) before the first look.  One that comes too early costs a look, about 1 us with those of 255
+// others on their way, and delays what it looks for; one that comes too late costs what it is late by.  By sweep, us a step at a
+// history of 24 / 300 / 900, from 8 (10 for the attention's row and the down projection's) everywhere: gate|up's row 12 steps and
+// the down projection's 18 382 / 439 / 458 -> 377 / 431 / 438 (1.7B shape), 729 / 802 / 854 -> 705 / 779 / 830 (4B); q|k|v's row
+// 12 level and 698 / 772 / 825, 16 1 % behind and 692 / 766 / 817; two more or fewer of any: within 1 %.
+constexpr int kPauseHead = 4, kPauseParts = 2;   // near hand-overs
+constexpr int kPauseAtt = 10, kPauseH2 = 12, kPauseInner = 18;
+__host__ __device__ constexpr int pause_row(int words) { return 8 + 4 * words; }   // words a lane of a row of dim
 constexpr int kBufFlags = 0x00020000;
 constexpr int kOob = 0x7ffffff0;           // an offset no buffer reaches: loads give 0, stores are dropped
 
@@ -95,6 +105,17 @@ struct Share {
     __host__ __device__ int results() const { return (rows + 15) / 16 * 16 * pitch(); }
 };
 
+// q|k|v's rows in the order of the kv heads: a head's queries, its key, its value.  A kv head's rows are computed and attended
+// to by the same workgroups, those whose number is the head's modulo n_kv.
+struct HeadOrder {
+    int n_heads, n_kv, gqa;
+    __host__ __device__ int rows() const { return (gqa + 2) * kHd; }   // of a kv head
+    __device__ int row_of(int kvh, int i) const {                     // its i-th one, as a row of the matrix
+        const int which = (uint32_t)i / kHd;
+        return (which < gqa ? kvh * gqa + which : n_heads + (which - gqa) * n_kv + kvh) * kHd + (int)((uint32_t)i % kHd);
+    }
+};
+
 __host__ __device__ inline int align128(int bytes) { return (bytes + 127) & ~127; }
 struct Rows {   // byte offsets of a layer's rows in a set
     int qkv, att, h2, inner, size;
@@ -107,6 +128,9 @@ struct Rows {   // byte offsets of a layer's rows in a set
     }
 };
 constexpr int kControlBytes = 256;
+// Control words beside those of step_finish.hip.h, which leaves these: whether the workgroups of a kv head share a die, and the
+// dies of the workgroups with the same number modulo eight, a bit each.
+enum { kDiesShared = 16, kDieOf = 24, kDies = 8 };
 
 // LDS: planes of the row (two bytes a value), its group sums, results of all units, raw row of the down projection
 struct Lds {
@@ -228,6 +252,23 @@ __device__ __forceinline__ bool receive(const __amdgpu_buffer_rsrc_t r, int from
 __device__ __forceinline__ void hand_over(const __amdgpu_buffer_rsrc_t set, int row, int off, uint32_t d) {
     d = d == kEmpty ? 0x7fff7fffu : d;
     __builtin_amdgcn_raw_buffer_store_b32(d, set, off, row, kDeviceScope);
+}
+// What only workgroups of the same die wait for stays in its L2: from one workgroup to another 0.21 us instead of 0.57 to
+// another die (0.38 on the same one past the L2).  `near`: see near_heads.
+__device__ __forceinline__ void hand_over_near(const __amdgpu_buffer_rsrc_t set, int row, int off, uint32_t d, bool near) {
+    d = d == kEmpty ? 0x7fff7fffu : d;
+    if (near)
+        __builtin_amdgcn_raw_buffer_store_b32(d, set, off, row, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b32(d, set, off, row, kDeviceScope);
+}
+// Workgroups go round the dies in the order of their numbers, so that those of a kv head (n_kv a multiple of eight) share
+// one.  The exchange memory's reset has looked whether they do (dies_kernel), and a workgroup that is not where it was then
+// stores past its L2, which all see.
+__device__ __forceinline__ bool near_heads(const __attribute__((address_space(4))) uint32_t *control, int wg) {
+    uint32_t die;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(die));
+    return control[kDiesShared] != 0 && ((control[kDieOf + wg % kDies] >> die) & 1u) != 0;
 }
 // `values` values of a row from `first` on, for the next launch
 __device__ __forceinline__ void empty(const __amdgpu_buffer_rsrc_t set, int row, int first, int values) {
@@ -358,23 +399,21 @@ struct Weights {
     v4u w[N];
     uint32_t s[N];   // two group scales
 
-    // Loads FROM .. TO - 1 of back wave `bw`: rows [row0, row0 + rows) of n (pairs: of gate row0 / 2 .. and up row0 / 2 ..,
-    // alternating).  `on` = 0 asks for nothing.
-    template <int BITS, int FROM, int TO>
-    __device__ __forceinline__ void ask(uintptr_t weights, uintptr_t scales, const Share &sh, int bw, int row0, int rows, int n,
-                                        bool pairs, int on) {
+    // Loads FROM .. TO - 1 of back wave `bw`: `rows` rows, i-th one row place(i) of n.  `on` = 0 asks for nothing.
+    template <int BITS, int FROM, int TO, class Place>
+    __device__ __forceinline__ void ask(uintptr_t weights, uintptr_t scales, const Share &sh, int bw, int rows, int n, Place place,
+                                        int on) {
         const int total = on ? n * sh.units : 0;
         const __amdgpu_buffer_rsrc_t rw = rsrc_of(reinterpret_cast<const void *>(weights), total * 64);
         const __amdgpu_buffer_rsrc_t rs = rsrc_of(reinterpret_cast<const void *>(scales), total * (BITS == 2 ? 4 : 8));
         const int lane = afresh((int)threadIdx.x & 63);
         const int recip = 65536 / sh.units + 1;
-        const int first = pairs ? row0 >> 1 : row0;
 #pragma unroll
         for (int i = FROM; i < TO; ++i) {
             const int idx = bw + i * kBackWaves;
             const int tile = (idx * recip) >> 16, u = idx - tile * sh.units;
             const int row = tile * 16 + (lane & 15);
-            const int at = (first + (pairs ? (row & 1) * (n >> 1) + (row >> 1) : row)) * sh.units + u;
+            const int at = place(row) * sh.units + u;
             const int off = wanted(row < rows, at * 64 + (lane >> 4) * 16);
             w[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0);
             const int o = BITS == 2 ? (off >> 6) * 4 : (off >> 6) * 8 + ((off >> 2) & 4);
@@ -466,8 +505,11 @@ struct Common {
     __amdgpu_buffer_rsrc_t here, other;   // this launch's set and the other one
     uint8_t *parts;
     uint32_t epoch;
-    bool attends, merges;
+    bool attends, merges, near;
     int n, hide, sees_itself, position, token, kvh, unit, split, head, per, splits;
+    HeadOrder order;
+    int head_row0;   // of the kv head's rows of q|k|v, the workgroup's first
+    __device__ int qkv_at() const { return kvh * order.rows() + head_row0; }   // .. in the exchange memory
     unsigned char *planes;
     float *sums, *red, *resid;
     uint16_t *raw;
@@ -497,11 +539,14 @@ __device__ __forceinline__ bool back(const Common &c, int bw) {
     Weights<NG> w_g;
     Weights<ND> w_d;
     constexpr int kHalfG = (NG + 1) / 2;
-    const auto ask_q = [&](const v2u &t, int on) { w_q.template ask<BITS, 0, NQ>(address(t, 0), address(t, 4), c.sq, bw, c.wg * c.sq.rows, c.rows_q, c.n_qkv, false, on); };
-    const auto ask_o = [&](const v2u &t, int on) { w_o.template ask<BITS, 0, NO>(address(t, 1), address(t, 5), c.so, bw, c.wg * c.so.rows, c.rows_o, a.dim, false, on); };
-    const auto ask_g1 = [&](const v2u &t, int on) { w_g.template ask<BITS, 0, kHalfG>(address(t, 2), address(t, 6), c.sg, bw, c.wg * c.sg.rows, c.rows_g, 2 * a.ffn, true, on); };
-    const auto ask_g2 = [&](const v2u &t, int on) { w_g.template ask<BITS, kHalfG, NG>(address(t, 2), address(t, 6), c.sg, bw, c.wg * c.sg.rows, c.rows_g, 2 * a.ffn, true, on); };
-    const auto ask_d = [&](const v2u &t, int on) { w_d.template ask<BITS, 0, ND>(address(t, 3), address(t, 7), c.sd, bw, c.wg * c.sd.rows, c.rows_d, a.dim, false, on); };
+    const auto head_row = [&](int row) { return c.order.row_of(c.kvh, c.head_row0 + row); };
+    const auto from = [&](const Share &sh) { return [&](int row) { return c.wg * sh.rows + row; }; };
+    const auto in_turn = [&](int row) { return c.wg * c.sg.rows / 2 + (row & 1) * a.ffn + (row >> 1); };   // gate, up
+    const auto ask_q = [&](const v2u &t, int on) { w_q.template ask<BITS, 0, NQ>(address(t, 0), address(t, 4), c.sq, bw, c.rows_q, c.n_qkv, head_row, on); };
+    const auto ask_o = [&](const v2u &t, int on) { w_o.template ask<BITS, 0, NO>(address(t, 1), address(t, 5), c.so, bw, c.rows_o, a.dim, from(c.so), on); };
+    const auto ask_g1 = [&](const v2u &t, int on) { w_g.template ask<BITS, 0, kHalfG>(address(t, 2), address(t, 6), c.sg, bw, c.rows_g, 2 * a.ffn, in_turn, on); };
+    const auto ask_g2 = [&](const v2u &t, int on) { w_g.template ask<BITS, kHalfG, NG>(address(t, 2), address(t, 6), c.sg, bw, c.rows_g, 2 * a.ffn, in_turn, on); };
+    const auto ask_d = [&](const v2u &t, int on) { w_d.template ask<BITS, 0, ND>(address(t, 3), address(t, 7), c.sd, bw, c.rows_d, a.dim, from(c.sd), on); };
     v2u cur = ask_layer(a, 0);
     ask_q(cur, 1);
     ask_o(cur, 1);
@@ -575,7 +620,7 @@ __device__ __forceinline__ bool back(const Common &c, int bw) {
             __syncthreads();   // maximum
             project(w_q, std::integral_constant<int, NQ>{}, std::integral_constant<int, TQ>{}, c.sq, c.rows_q, s, [&](int row, float v) {
                 const float y = v / s, z = lanes_on<TQ>(y);
-                if ((lane & (2 * TQ - 1)) == 0 && row < c.rows_q) hand_over(c.here, row0 + c.lay.qkv, (c.wg * c.sq.rows + row) * 2, pack_bf16(y, z));
+                if ((lane & (2 * TQ - 1)) == 0 && row < c.rows_q) hand_over_near(c.here, row0 + c.lay.qkv, (c.qkv_at() + row) * 2, pack_bf16(y, z), c.near);
             });
         }
 
@@ -606,7 +651,7 @@ __device__ __forceinline__ bool back(const Common &c, int bw) {
         };
         if (c.rows_o) __syncthreads();   // maximum
         ask_q(nxt, more);
-        if (bw == 1) empty(c.other, row0 + c.lay.qkv, c.wg * c.sq.rows, c.rows_q);
+        if (bw == 1) empty(c.other, row0 + c.lay.qkv, c.qkv_at(), c.rows_q);
         if (c.rows_o) {
             if (given_up(c.meet)) return false;
             project(w_o, std::integral_constant<int, NO>{}, std::integral_constant<int, TO>{}, c.so, c.rows_o, s,
@@ -740,7 +785,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
         // ---- q | k | v
         {
             bool ok = true;
-            if (l > 0 && c.rows_q) ok = receive<UD>(c.here, row0, a.dim >> 3, row_d, kPauseRow, limit);
+            if (l > 0 && c.rows_q) ok = receive<UD>(c.here, row0, a.dim >> 3, row_d, pause_row(UD), limit);
             nxt = ask_layer(a, nl);
             if (c.rows_q && !stage_norm(row_d, ln1, ok)) return false;
         }
@@ -751,11 +796,11 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
             const bool has_token = n >= c.split * c.per && n < (c.split + 1) * c.per;   // the part that holds the token itself
             bool ok = true;
             if (wave < (has_token ? 3 : 1)) {
-                const int row = wave == 0 ? c.head : (wave == 1 ? a.n_heads : a.n_heads + a.n_kv) + c.kvh;
-                const int from = row0 + c.lay.qkv + row * 256;
+                const int row = wave == 0 ? c.head - c.kvh * c.gqa : c.gqa + wave - 1;   // of the kv head's
+                const int from = row0 + c.lay.qkv + (c.kvh * (c.gqa + 2) + row) * 256;
                 uint32_t d = kEmpty;
                 uint32_t since = 0;
-                for (int z = 0; z < kPauseRow; ++z) __builtin_amdgcn_s_sleep(1);
+                for (int z = 0; z < kPauseHead; ++z) __builtin_amdgcn_s_sleep(1);
                 for (int spins = first_spin(limit);; ++spins) {
                     d = __builtin_amdgcn_raw_buffer_load_b32(c.here, lane * 4, from, kDeviceScope);
                     if (__all(d != kEmpty)) break;
@@ -897,9 +942,15 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
                 } else {
                     const uint32_t tag = c.epoch * (uint32_t)a.n_layers + (uint32_t)l + 1u;
                     const __amdgpu_buffer_rsrc_t r = rsrc_of(c.parts + (size_t)(c.head * kMaxSplits + c.split) * (kPartEntries * 8), kPartEntries * 8);
-                    __builtin_amdgcn_raw_buffer_store_b64(v2u{__float_as_uint(o), tag}, r, tid * 8, 0, kDeviceScope);
-                    if (tid < 2)
-                        __builtin_amdgcn_raw_buffer_store_b64(v2u{__float_as_uint(tid ? sum : m), tag}, r, (kHd + tid) * 8, 0, kDeviceScope);
+                    const v2u part = v2u{__float_as_uint(o), tag}, of_all = v2u{__float_as_uint(tid ? sum : m), tag};
+                    const int last = wanted(tid < 2, (kHd + tid) * 8);
+                    if (c.near) {
+                        __builtin_amdgcn_raw_buffer_store_b64(part, r, tid * 8, 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b64(of_all, r, last, 0, 0);
+                    } else {
+                        __builtin_amdgcn_raw_buffer_store_b64(part, r, tid * 8, 0, kDeviceScope);
+                        __builtin_amdgcn_raw_buffer_store_b64(of_all, r, last, 0, kDeviceScope);
+                    }
                 }
             }
         }
@@ -912,7 +963,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
             uint32_t since = 0;
             v2u o[kMaxSplits / 2];
             v4u ml;
-            for (int z = 0; z < kPauseRow; ++z) __builtin_amdgcn_s_sleep(1);
+            for (int z = 0; z < kPauseParts; ++z) __builtin_amdgcn_s_sleep(1);
             for (int spins = first_spin(limit);; ++spins) {
 #pragma unroll
                 for (int i = 0; i < kMaxSplits / 2; ++i)
@@ -958,7 +1009,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
         {
             v4u row_a[UQ];
             if (c.rows_o) {
-                const bool ok = receive<UQ>(c.here, row0 + c.lay.att, c.q_dim >> 3, row_a, kPauseLong, limit);
+                const bool ok = receive<UQ>(c.here, row0 + c.lay.att, c.q_dim >> 3, row_a, kPauseAtt, limit);
                 const float top = top_of<UQ>(row_a);
                 if (lane == 0) {
                     c.meet.top[wave] = top;
@@ -983,7 +1034,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
         // ---- gate | up
         {
             bool ok = true;
-            if (c.rows_g) ok = receive<UD>(c.here, row0 + c.lay.h2, a.dim >> 3, row_d, kPauseRow, limit);
+            if (c.rows_g) ok = receive<UD>(c.here, row0 + c.lay.h2, a.dim >> 3, row_d, kPauseH2, limit);
             ask_row(ln1, norm_weights(nxt, 0));
             ask_head(nxt);
             ask_history(nl, slot0, c.attends && more);
@@ -994,7 +1045,7 @@ __device__ __forceinline__ bool front(const Common &c, int wave) {
         {
             v4u row_f[UF];
             bool ok = true;
-            if (c.rows_d) ok = receive<UF>(c.here, row0 + c.lay.inner, a.ffn >> 3, row_f, kPauseLong, limit);
+            if (c.rows_d) ok = receive<UF>(c.here, row0 + c.lay.inner, a.ffn >> 3, row_f, kPauseInner, limit);
             ask_row(ln2, norm_weights(nxt, 1));
             if (c.rows_d) {
                 const int t = afresh(tid);
@@ -1034,20 +1085,22 @@ step_one_kernel(const Args a) {
     __shared__ float resid[256];
     const int groups = a.groups, gqa = a.n_heads / a.n_kv;
     const int q_dim = a.n_heads * kHd, n_qkv = (a.n_heads + 2 * a.n_kv) * kHd;
-    const Share sq(a.dim, n_qkv, groups, BITS, false), so(q_dim, a.dim, groups, BITS, false),
+    const HeadOrder order{a.n_heads, a.n_kv, gqa};
+    const Share sq(a.dim, order.rows(), groups / a.n_kv, BITS, false), so(q_dim, a.dim, groups, BITS, false),
         sg(a.dim, 2 * a.ffn, groups, BITS, true), sd(a.ffn, a.dim, groups, BITS, false);
-    const auto mine = [wg](const Share &s, int n) {
-        const int left = n - wg * s.rows;
+    const auto mine = [](const Share &s, int n, int i) {
+        const int left = n - i * s.rows;
         return left < 0 ? 0 : (left < s.rows ? left : s.rows);
     };
-    const int rows_q = mine(sq, n_qkv), rows_o = mine(so, a.dim), rows_g = mine(sg, 2 * a.ffn), rows_d = mine(sd, a.dim);
+    const int kvh = wg % a.n_kv, unit = wg / a.n_kv;
+    const int rows_q = mine(sq, order.rows(), unit), rows_o = mine(so, a.dim, wg), rows_g = mine(sg, 2 * a.ffn, wg), rows_d = mine(sd, a.dim, wg);
 
     // The attention's share: the slots [0, n] (slot n is the token itself, whose key and value come from the exchange
     // memory) of one head, or a part of them.  A workgroup a query head rather than a kv head: the chain is shorter, and
     // the heads' second reads of keys and values come from their common L2.
     const auto in = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)a.step_in;
     const int n = in[0] < 0 ? 0 : (in[0] < a.sigma ? in[0] : a.sigma);   // as everywhere: a history within its slots
-    const int kvh = wg % a.n_kv, unit = wg / a.n_kv, split = unit / gqa;
+    const int split = unit / gqa;
     const int head = kvh * gqa + unit - split * gqa;
     const int room = groups / (a.n_kv * gqa);
     const int max_splits = room < kMaxSplits ? room : kMaxSplits;
@@ -1073,7 +1126,8 @@ step_one_kernel(const Args a) {
     const Lds at(k_max, results, a.ffn);
     const Common c{a, wg, tid & 63, gqa, q_dim, n_qkv, sq, so, sg, sd, lay, rows_q, rows_o, rows_g, rows_d,
                    rsrc_of(sets + (size_t)(epoch & 1) * set_bytes, set_bytes), rsrc_of(sets + (size_t)((epoch & 1) ^ 1) * set_bytes, set_bytes), sets + (size_t)2 * set_bytes,
-                   epoch, attends, merges, n, in[1], in[2] & 1, in[3], in[4], kvh, unit, split, head, per, splits, smem,
+                   epoch, attends, merges, near_heads(state, wg), n, in[1], in[2] & 1, in[3], in[4], kvh, unit, split, head, per, splits, order,
+                   unit * sq.rows, smem,
                    reinterpret_cast<float *>(smem + at.sums), reinterpret_cast<float *>(smem + at.red), resid,
                    reinterpret_cast<uint16_t *>(smem + at.raw), 2 * k_max, meet};
     if (tid == 0) meet.bad = 0;
@@ -1094,7 +1148,25 @@ __global__ void __launch_bounds__(256) exchange_reset_kernel(v4u *p, size_t word
         p[i] = i >= rows_from && i < rows_to ? v4u{kEmpty, kEmpty, kEmpty, kEmpty} : v4u{0, 0, 0, 0};
 }
 
+// The dies of the workgroups of a launch, then whether those with the same number modulo eight share one.
+__global__ void __launch_bounds__(64) dies_kernel(uint32_t *control) {
+    uint32_t die;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(die));
+    if (threadIdx.x == 0) __hip_atomic_fetch_or(control + kDieOf + blockIdx.x % kDies, 1u << die, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__global__ void __launch_bounds__(64) dies_shared_kernel(uint32_t *control, int n_kv) {
+    const uint32_t dies = control[kDieOf + threadIdx.x % kDies];
+    const bool one = __all(dies != 0 && (dies & (dies - 1)) == 0);
+    if (threadIdx.x == 0) control[kDiesShared] = one && n_kv % kDies == 0;
+}
+
 // ---- host ---------------------------------------------------------------------------------
+inline hipError_t look_at_dies(void *exchange, int n_kv, int groups, hipStream_t stream) {
+    uint32_t *control = static_cast<uint32_t *>(exchange);
+    hipLaunchKernelGGL(dies_kernel, dim3(groups), dim3(64), 0, stream, control);
+    hipLaunchKernelGGL(dies_shared_kernel, dim3(1), dim3(64), 0, stream, control, n_kv);
+    return hipGetLastError();
+}
 // The builds: loads a lane per projection and words a lane per row that each of them holds.
 struct Build {
     int bits, nq, no, ng, nd, ud, uq, uf;
@@ -1118,7 +1190,8 @@ inline Fit fit(int bits, int n_layers, int dim, int ffn, int n_heads, int n_kv, 
     const int64_t n_qkv = (int64_t)(n_heads + 2 * n_kv) * kHd;
     // 32-bit offsets into a matrix
     if (2 * (int64_t)ffn * dim >= kOob || n_qkv * dim >= kOob) return f;
-    const Share s[4] = {{dim, (int)n_qkv, groups, bits, false}, {q_dim, dim, groups, bits, false},
+    const HeadOrder order{n_heads, n_kv, n_heads / n_kv};
+    const Share s[4] = {{dim, order.rows(), groups / n_kv, bits, false}, {q_dim, dim, groups, bits, false},
                         {dim, 2 * ffn, groups, bits, true}, {ffn, dim, groups, bits, false}};
     int results = 0;
     for (const Share &x : s) {
