@@ -1127,6 +1127,49 @@ __global__ void __launch_bounds__(256) kv_commit_kernel(uint4 *kv, int planes, i
 }
 
 // ---------------------------------------------------------------------------
+// Steps behind a step, without the host in between (its turn-round is 25 us, the launches and copies around a step as much
+// again).  All rows that a step needs from the one before it are on the device when that one ends:
+//   step_next_kernel    one token after another: the row of the step before to the history, whose length the step's own last
+//                       launch has advanced (DraftExtra::step)
+//   step_after_kernel   a block that verifies a drafted one: inputs from pinned host memory, marked tokens (INT32_MIN + i)
+//                       from the draft, and the commit of the draft's pending rows
+// 4.3 and 5.2 us each.  64 tokens greedily behind a short prompt 28641 us without them, 28397 with one step to a graph (14 us pass
+// between two graphs, also of one stream) and 27792 with four; 48 speculatively 36380 and, both blocks' commits here, 35800 - 35980.
+// ---------------------------------------------------------------------------
+constexpr int kCommitGroups = 32;   // 8192 threads: a row of the 1.7B shape is 7168 pieces of 16 bytes, of the 4B one 9216
+__device__ __forceinline__ void commit_rows(uint4 *kv, int planes, int slots, int src, int dst, int n) {
+    if (n <= 0 || src < 0 || dst < 0 || n > slots || src > slots - n || dst > slots - n) return;
+    constexpr int kPieces = kHd * 2 / 16;
+    const int per_plane = n * kPieces;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < planes * per_plane; i += kCommitGroups * 256) {
+        const int plane = i / per_plane, off = i - plane * per_plane;
+        uint4 *base = kv + (size_t)plane * slots * kPieces;
+        base[(size_t)dst * kPieces + off] = base[(size_t)src * kPieces + off];
+    }
+}
+__global__ void __launch_bounds__(256) step_next_kernel(const int32_t *step_in, uint4 *kv, int planes, int slots, int sigma) {
+    const int n = step_in[0];
+    if (n <= sigma) commit_rows(kv, planes, slots, sigma, n - 1, 1);
+}
+__device__ __forceinline__ int32_t from_host(const int32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+__global__ void __launch_bounds__(256) step_after_kernel(const int32_t *from, int32_t *to, int words, const int32_t *drafted, int drafts,
+                                                         uint4 *kv, int planes, int slots) {
+    __shared__ int32_t rows[3];
+    const int tid = threadIdx.x;
+    // behind the inputs: source and destination slot and number of the rows; one trip over the bus for all of it
+    const int at = tid < 3 ? words + tid : tid - 3;
+    if (at < words + 3 && (tid < 3 || blockIdx.x == 0)) {
+        const int32_t v = from_host(from + at);
+        if (tid < 3)
+            rows[tid] = v;
+        else
+            to[at] = at >= words - words / 3 && (uint32_t)v - 0x80000000u < (uint32_t)drafts ? drafted[v - INT32_MIN] : v;   // (the last third are tokens)
+    }
+    __syncthreads();
+    commit_rows(kv, planes, slots, rows[0], rows[1], rows[2]);
+}
+
+// ---------------------------------------------------------------------------
 // Draft chain.  One workgroup of 1024 threads per logits row: running (max, index)
 // and the sum of exp(x - max) in one pass with 16-byte loads; conf = 1 / sum.
 // ---------------------------------------------------------------------------
@@ -1307,7 +1350,11 @@ draft_rows_split_kernel(const uint16_t *logits, int ld, int vocab, int splits, f
 
 __global__ void __launch_bounds__(1024)
 draft_merge_accept_kernel(const float *scratch, int rows, int splits, float threshold,
-                          int32_t *tokens, float *conf, int32_t *accept) {
+                          int32_t *tokens, float *conf, int32_t *accept, const bonsai_draft_extra extra) {
+    // Results in pinned memory: the reader looks at every word, so they need no order.  (In place of a copy node: 4 us.)
+    const auto tell = [&extra](int i, int32_t v) {
+        if (extra.host != nullptr) __hip_atomic_store(extra.host + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    };
     __shared__ float conf_lds[BONSAI_MAX_WIDTH];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int row = w; row < rows; row += 16) {  // rows <= 32: every wave runs the same two rounds at most
@@ -1324,9 +1371,20 @@ draft_merge_accept_kernel(const float *scratch, int rows, int splits, float thre
         st = wave_merge(st);
         if (lane == 0) {
             const float c = st.sum > 0.0f ? 1.0f / st.sum : 0.0f;
-            tokens[row] = st.idx == 0x7fffffff ? 0 : st.idx;
+            const int32_t token = st.idx == 0x7fffffff ? 0 : st.idx;
+            tokens[row] = token;
             conf[row] = c;
             conf_lds[row] = c;
+            tell(row, token);
+            tell(extra.conf_at + row, __float_as_int(c));
+            if (extra.tokens_too != nullptr) extra.tokens_too[row] = token;
+            if (extra.step != nullptr && row == 0) {   // the next one-token step: history length, position, token
+                const int32_t n = extra.step[0];
+                __hip_atomic_store(extra.ring + (uint32_t)n % (uint32_t)extra.ring_words, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                extra.step[0] = n + 1;
+                extra.step[3] += 1;
+                extra.step[4] = token;
+            }
         }
     }
     __syncthreads();
@@ -1338,6 +1396,8 @@ draft_merge_accept_kernel(const float *scratch, int rows, int splits, float thre
         }
         accept[0] = n;
         accept[1] = rows;
+        tell(extra.accept_at, n);
+        tell(extra.accept_at + 1, rows);
     }
 }
 
@@ -2023,6 +2083,26 @@ extern "C" int bonsai_kv_commit(void *kv, int n_layers, int n_kv, int slots, int
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }
 
+static bool kv_planes_ok(const void *kv, int n_layers, int n_kv, int slots) {
+    return kv && n_layers >= 1 && n_kv >= 1 && slots >= 1 && 2LL * n_layers * n_kv * slots * (kHd * 2 / 16) <= 0x7fffffffLL;
+}
+
+extern "C" int bonsai_step_next(const int32_t *step_in, void *kv, int n_layers, int n_kv, int slots, int sigma, void *stream) {
+    if (!step_in || !kv_planes_ok(kv, n_layers, n_kv, slots) || sigma < 0 || sigma >= slots) return BONSAI_DECODE_ERR_ARG;
+    hipLaunchKernelGGL(step_next_kernel, dim3(kCommitGroups), dim3(256), 0, static_cast<hipStream_t>(stream), step_in,
+                       static_cast<uint4 *>(kv), 2 * n_layers * n_kv, slots, sigma);
+    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+}
+
+extern "C" int bonsai_step_after(const int32_t *from, int32_t *step_in, int rows, const int32_t *drafted, int drafts, void *kv,
+                                 int n_layers, int n_kv, int slots, void *stream) {
+    if (!from || !step_in || !drafted || rows < 1 || rows > BONSAI_MAX_WIDTH || drafts < 0 || !kv_planes_ok(kv, n_layers, n_kv, slots))
+        return BONSAI_DECODE_ERR_ARG;
+    hipLaunchKernelGGL(step_after_kernel, dim3(kCommitGroups), dim3(256), 0, static_cast<hipStream_t>(stream), from, step_in, 2 + 3 * rows,
+                       drafted, drafts, static_cast<uint4 *>(kv), 2 * n_layers * n_kv, slots);
+    return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
+}
+
 extern "C" int bonsai_draft_chain(const void *logits, int rows, int ld, int vocab, float threshold,
                                   int32_t *tokens, float *conf, int32_t *accept, void *stream) {
     if (!logits || !tokens || !conf || !accept) return BONSAI_DECODE_ERR_ARG;
@@ -2042,7 +2122,15 @@ extern "C" int64_t bonsai_draft_chain_scratch_bytes(int rows) {
 extern "C" int bonsai_draft_chain_ws(const void *logits, int rows, int ld, int vocab, float threshold,
                                      int32_t *tokens, float *conf, int32_t *accept, void *scratch,
                                      void *stream) {
+    return bonsai_draft_chain_extra(logits, rows, ld, vocab, threshold, tokens, conf, accept, scratch, nullptr, stream);
+}
+
+extern "C" int bonsai_draft_chain_extra(const void *logits, int rows, int ld, int vocab, float threshold, int32_t *tokens, float *conf,
+                                        int32_t *accept, void *scratch, const bonsai_draft_extra *also, void *stream) {
     if (!logits || !tokens || !conf || !accept || !scratch) return BONSAI_DECODE_ERR_ARG;
+    const bonsai_draft_extra extra = also ? *also : bonsai_draft_extra{};
+    if ((extra.host && (extra.conf_at < 0 || extra.accept_at < 0)) || (extra.step && (!extra.ring || extra.ring_words < 1 || rows != 1)))
+        return BONSAI_DECODE_ERR_ARG;
     if (rows < 1 || rows > BONSAI_MAX_WIDTH || vocab < 1 || ld < vocab || ld % 8 != 0)
         return BONSAI_DECODE_ERR_ARG;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -2052,7 +2140,7 @@ extern "C" int bonsai_draft_chain_ws(const void *logits, int rows, int ld, int v
     if (hipGetLastError() != hipSuccess) return BONSAI_DECODE_ERR_LAUNCH;
     hipLaunchKernelGGL(draft_merge_accept_kernel, dim3(1), dim3(1024), 0, st,
                        static_cast<const float *>(scratch), rows, kDraftSplits, threshold, tokens,
-                       conf, accept);
+                       conf, accept, extra);
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }
 
@@ -2109,7 +2197,7 @@ extern "C" int bonsai_draft_chain_static(const void *logits, int rows, int ld, i
     if (hipGetLastError() != hipSuccess) return BONSAI_DECODE_ERR_LAUNCH;
     hipLaunchKernelGGL(draft_merge_accept_kernel, dim3(1), dim3(1024), 0, st,
                        static_cast<const float *>(ws), rows, kDraftSplits, threshold, tokens, conf,
-                       accept);
+                       accept, bonsai_draft_extra{});
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }
 

@@ -32,6 +32,12 @@ class StepOneDesc(ctypes.Structure):
                 + [("norm_first", ctypes.c_int), ("norm_rows", ctypes.c_int)])
 
 
+class DraftExtra(ctypes.Structure):
+    """``bonsai_draft_extra`` of include/bonsai_decode.h."""
+    _fields_ = [("host", ctypes.c_void_p), ("conf_at", ctypes.c_int), ("accept_at", ctypes.c_int), ("tokens_too", ctypes.c_void_p),
+                ("step", ctypes.c_void_p), ("ring", ctypes.c_void_p), ("ring_words", ctypes.c_int)]
+
+
 class FinalNorm(NamedTuple):
     """Rows ``first .. first + rows - 1`` of a step, normed for the output projection: bf16 to ``out`` or, without it,
     quantised to ``q`` and ``s``."""
@@ -86,6 +92,12 @@ def load_decode_kernel() -> None:
     lib.bonsai_draft_chain.restype = ci
     lib.bonsai_draft_chain_ws.argtypes = [vp, ci, ci, ci, cf, vp, vp, vp, vp, vp]
     lib.bonsai_draft_chain_ws.restype = ci
+    lib.bonsai_draft_chain_extra.argtypes = [vp, ci, ci, ci, cf, vp, vp, vp, vp, ctypes.POINTER(DraftExtra), vp]
+    lib.bonsai_draft_chain_extra.restype = ci
+    lib.bonsai_step_next.argtypes = [vp, vp, ci, ci, ci, ci, vp]
+    lib.bonsai_step_next.restype = ci
+    lib.bonsai_step_after.argtypes = [vp, vp, ci, vp, ci, vp, ci, ci, ci, vp]
+    lib.bonsai_step_after.restype = ci
     lib.bonsai_draft_chain_static.argtypes = [vp, ci, ci, ci, cf, vp, vp, vp, vp]
     lib.bonsai_draft_chain_static.restype = ci
     lib.bonsai_decode_init.argtypes = []
@@ -453,13 +465,68 @@ def kv_commit(kv: torch.Tensor, src_slot: int, dst_slot: int, n: int) -> None:
     _need(rc == 0, f"bonsai_kv_commit failed with status {rc}")
 
 
+def _check_kv(kv: torch.Tensor) -> None:
+    _check(kv, torch.bfloat16, "kv")
+    _need(kv.dim() == 5 and kv.shape[0] == 2 and kv.shape[4] == HEAD_DIM, "kv must be [2, n_layers, n_kv, slots, 128]")
+
+
+def _pinned(t: torch.Tensor, size: int) -> bool:
+    return t.dtype == torch.int32 and t.is_pinned() and t.is_contiguous() and t.numel() >= size
+
+
+def step_next(step_in: torch.Tensor, kv: torch.Tensor, sigma: int) -> None:
+    """Behind a one-token step that has advanced ``step_in``: its row, slot ``sigma`` of ``kv``, becomes the history's last."""
+    _check(step_in, torch.int32, "step_in")
+    _check_kv(kv)
+    with torch.cuda.device(kv.device):
+        rc = decode_lib().bonsai_step_next(_ptr(step_in), _ptr(kv), kv.shape[1], kv.shape[2], kv.shape[3], int(sigma), _stream(kv.device))
+    _need(rc == 0, f"bonsai_step_next failed with status {rc}")
+
+
+def step_after(inputs: torch.Tensor, step_in: torch.Tensor, drafted: torch.Tensor, kv: torch.Tensor) -> None:
+    """Step inputs from ``inputs`` (pinned) to ``step_in`` ``[2 + 3 rows]``, tokens ``-2**31 + i`` as ``drafted[i]``; then, as the three
+    pinned words behind them ask (source slot, destination slot, rows), rows of ``kv`` to the history."""
+    _check(step_in, torch.int32, "step_in")
+    _check(drafted, torch.int32, "drafted")
+    _check_kv(kv)
+    n = step_in.numel()
+    _need(n >= 5 and n % 3 == 2 and _pinned(inputs, n + 3), "step inputs must be 2 + 3 rows words, pinned with three more")
+    with torch.cuda.device(kv.device):
+        rc = decode_lib().bonsai_step_after(_ptr(inputs), _ptr(step_in), (n - 2) // 3, _ptr(drafted), drafted.numel(), _ptr(kv), kv.shape[1],
+                                            kv.shape[2], kv.shape[3], _stream(kv.device))
+    _need(rc == 0, f"bonsai_step_after failed with status {rc}")
+
+
+class AlsoTo(NamedTuple):
+    """Where a captured step's results go as well."""
+    host: torch.Tensor                           # pinned int32: tokens at 0, accept and confidences at these words
+    accept_at: int
+    conf_at: int
+    tokens: Optional[torch.Tensor] = None        # int32 on the device
+    step: Optional[torch.Tensor] = None          # the inputs of a one-token step, which become the next one's,
+    ring: Optional[torch.Tensor] = None          # and pinned words its token goes to, by the length of its history
+
+    def extra(self, rows: int) -> DraftExtra:
+        _need(_pinned(self.host, self.conf_at + rows) and rows <= self.accept_at <= self.conf_at - 2, "host results do not fit")
+        x = DraftExtra(host=self.host.data_ptr(), conf_at=self.conf_at, accept_at=self.accept_at)
+        if self.tokens is not None:
+            _check(self.tokens, torch.int32, "tokens")
+            _need(self.tokens.numel() >= rows, "tokens too small")
+            x.tokens_too = self.tokens.data_ptr()
+        if self.step is not None:
+            _check(self.step, torch.int32, "step")
+            _need(rows == 1 and self.step.numel() == 5 and self.ring is not None and _pinned(self.ring, 1), "only one-token steps go on")
+            x.step, x.ring, x.ring_words = self.step.data_ptr(), self.ring.data_ptr(), self.ring.numel()
+        return x
+
+
 def draft_chain(logits: torch.Tensor, vocab: int, threshold: float, tokens: torch.Tensor,
                 conf: torch.Tensor, accept: torch.Tensor,
-                scratch: Optional[torch.Tensor] = None) -> None:
+                scratch: Optional[torch.Tensor] = None, also: Optional[AlsoTo] = None) -> None:
     """Row argmax, confidence ``exp(max - logsumexp)`` and the accepted-prefix length
     ``1 + longest prefix of rows 1.. with conf > threshold`` (reference:
     fast_generate.py:111-130).  ``logits`` bf16 ``[rows, ld]``; outputs are pre-allocated
-    int32 ``[rows]``, fp32 ``[rows]`` and int32 ``[2]``."""
+    int32 ``[rows]``, fp32 ``[rows]`` and int32 ``[2]``.  ``also``: where results go as well (with ``scratch``)."""
     _check(logits, torch.bfloat16, "logits")
     _check(tokens, torch.int32, "tokens")
     _check(conf, torch.float32, "conf")
@@ -467,15 +534,16 @@ def draft_chain(logits: torch.Tensor, vocab: int, threshold: float, tokens: torc
     rows, ld = logits.shape
     _need(tokens.numel() >= rows and conf.numel() >= rows and accept.numel() >= 2,
           "draft_chain output buffers too small")
+    _need(also is None or scratch is not None, "draft_chain needs scratch for further outputs")
+    extra = None if also is None else ctypes.byref(also.extra(rows))
     with torch.cuda.device(logits.device):
         if scratch is not None:
             # rows split over several workgroups, partial statistics through `scratch`
             need = int(decode_lib().bonsai_draft_chain_scratch_bytes(rows))
             _need(scratch.is_cuda and scratch.is_contiguous()
                   and scratch.numel() * scratch.element_size() >= need, "draft_chain scratch too small")
-            rc = decode_lib().bonsai_draft_chain_ws(_ptr(logits), rows, ld, int(vocab),
-                                                    float(threshold), _ptr(tokens), _ptr(conf),
-                                                    _ptr(accept), _ptr(scratch), _stream(logits.device))
+            rc = decode_lib().bonsai_draft_chain_extra(_ptr(logits), rows, ld, int(vocab), float(threshold), _ptr(tokens), _ptr(conf),
+                                                       _ptr(accept), _ptr(scratch), extra, _stream(logits.device))
         else:
             rc = decode_lib().bonsai_draft_chain(_ptr(logits), rows, ld, int(vocab), float(threshold),
                                                  _ptr(tokens), _ptr(conf), _ptr(accept),

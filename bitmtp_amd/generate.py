@@ -4,7 +4,11 @@ counterparts of ``fast_ar_generate`` and ``fast_hybrid_generate``
 
 Semantics kept from the reference:
 
-* AR: one width-1 replay per token; the new KV row is committed after each replay.
+* AR: one width-1 replay per token; the new KV row is committed after each replay.  Where the
+  atlas can, a step is queued before the token of the one in front of it has been read
+  (``GraphAtlas.step_ahead``), several at once where no end-of-text token can come: behind one,
+  one step too many runs, whose row is not committed.  A verification that comes whatever is
+  drafted is queued behind the draft in the same way (``GraphAtlas.verify_drafted``).
 * Hybrid: a draft replay of width ``M = select_M_for_pending(n_pend)`` carries the
   pending committed tokens, the anchor (a repeat of the last pending token) and D-1 mask
   tokens.  Row 0 of the D draft predictions is always committed; the confidence chain
@@ -153,8 +157,11 @@ def ar_generate(atlas: GraphAtlas, input_ids: Sequence[int], max_gen_len: int = 
         return [], st
     gen = [next_tok]
     g = atlas.get_graph(1, sigma, "ar")
+    step_ahead = getattr(atlas, "step_ahead", lambda g, most: 0)
+    longest = atlas.segment_ladder[-1]
+    eos_found = False
     t1 = time.time()
-    while len(gen) < max_gen_len:
+    while len(gen) < max_gen_len and not eos_found:
         if cache_len + atlas.M_max > sigma:
             new_sigma = atlas.select_segment(cache_len + atlas.M_max + 64)
             if new_sigma != sigma:
@@ -162,14 +169,26 @@ def ar_generate(atlas: GraphAtlas, input_ids: Sequence[int], max_gen_len: int = 
                 sigma = new_sigma
                 g = atlas.get_graph(1, sigma, "ar")
         atlas.replay(g, [next_tok], [cache_len], cache_len)
-        atlas.commit_kv(sigma, cache_len, 1)
-        cache_len += 1
-        out, _, _ = atlas.read_outputs(g)
-        next_tok = int(out[0])
-        if eos_set and next_tok in eos_set:
-            break
-        gen.append(next_tok)
-        if cache_len + 1 > atlas.segment_ladder[-1]:
+        # the steps that this segment has room for; the next ones are queued while the last one before them is waited for
+        steps = min(max_gen_len - len(gen), max(1, (longest if sigma == longest else sigma - atlas.M_max + 1) - cache_len))
+        queued, read = 1, 0
+        while read < queued:
+            if queued == read + 1:
+                more = step_ahead(g, min(steps - queued, 1 if eos_set else steps))
+                if not more:
+                    atlas.commit_kv(sigma, cache_len, 1)
+                queued += more
+            if queued > 1:
+                next_tok = atlas.read_step(g, cache_len)
+            else:
+                next_tok = int(atlas.read_outputs(g)[0][0])
+            cache_len += 1
+            read += 1
+            if eos_set and next_tok in eos_set:
+                eos_found = True
+                break
+            gen.append(next_tok)
+        if cache_len + 1 > longest:
             break
     atlas.synchronize()
     decode_time = max(time.time() - t1, 1e-9)
@@ -227,6 +246,10 @@ def hybrid_generate(atlas: GraphAtlas, input_ids: Sequence[int], threshold: floa
     MASK = args.mask_token_id
     if hybrid_m is None:
         hybrid_m = default_hybrid_m(D)
+    # (the loop replays a block, settles or synchronises before anything reads the history)
+    commit_kv = getattr(atlas, "commit_with_next", atlas.commit_kv)
+    # a chain is at most D tokens long
+    always_verifies = hybrid_m > D and not exact_m1_verify and hasattr(atlas, "verify_drafted")
     eos_set = set(int(e) for e in eos_ids)
     prompt = [int(t) for t in input_ids]
     seq_len = len(prompt)
@@ -271,12 +294,17 @@ def hybrid_generate(atlas: GraphAtlas, input_ids: Sequence[int], threshold: floa
                 sigma = new_sigma
 
         # ---- draft replay: [pending | pad | anchor | MASK x (D-1)]
+        if always_verifies:
+            gv = atlas.get_graph(M_verify, sigma, role_v)   # (before the draft: a capture uses the workspace)
         gd = atlas.get_graph(M_draft, sigma, role_d)
         toks = pending + [0] * (P - n_pend) + [pending[-1]] + [MASK] * (D - 1)
         pos = [cache_len + i for i in range(n_pend)] + [0] * (P - n_pend) + \
               [cache_len + n_pend - 1 + i for i in range(D)]
         atlas.replay(gd, toks, pos, cache_len, n_pend=n_pend)
-        atlas.commit_kv(sigma, cache_len, n_pend)
+        verifying = always_verifies and atlas.verify_drafted(
+            gv, gd, pending[-1], [cache_len + n_pend - 1 + i for i in range(M_verify)], cache_len + n_pend, n_pend)
+        if not verifying:
+            atlas.commit_kv(sigma, cache_len, n_pend)
         cache_len += n_pend
         d_tokens, d_conf, _ = atlas.read_outputs(gd)
         draft_tokens = [int(t) for t in d_tokens[:D]]
@@ -292,16 +320,17 @@ def hybrid_generate(atlas: GraphAtlas, input_ids: Sequence[int], threshold: floa
                 accept_count, cache_len, bonus = _exact_m1_verify(
                     atlas, sigma, cache_len, pending, draft_tokens)
             else:
-                gv = atlas.get_graph(M_verify, sigma, role_v)
-                vt = [pending[-1]] + draft_tokens
-                vp = [cache_len - 1 + i for i in range(M_verify)]
-                atlas.replay(gv, vt, vp, cache_len)
+                if not verifying:
+                    gv = atlas.get_graph(M_verify, sigma, role_v)
+                    vt = [pending[-1]] + draft_tokens
+                    vp = [cache_len - 1 + i for i in range(M_verify)]
+                    atlas.replay(gv, vt, vp, cache_len)
                 v_tokens, _, _ = atlas.read_outputs(gv)
                 accept_count = verify_accept(draft_tokens, v_tokens, D)
                 bonus = int(v_tokens[accept_count])
                 if accept_count > 0:
                     # rows 1..accept_count of the verify workspace are AR-correct
-                    atlas.commit_kv(sigma, cache_len, accept_count, first_row=1)
+                    commit_kv(sigma, cache_len, accept_count, first_row=1)
                     cache_len += accept_count
             commit = draft_tokens[:accept_count] + [bonus]
             accepted_this_iter, bonus_this_iter = accept_count, 1

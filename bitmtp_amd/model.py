@@ -25,6 +25,7 @@ import math
 from dataclasses import dataclass, replace
 from typing import Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import decode_ops, ops
@@ -407,7 +408,7 @@ class StepIO:
     """Per-graph inputs and outputs.  ``step_in`` is one int32 vector
     ``[meta (2+M) | positions (M) | tokens (M)]`` so a replay needs a single
     host-to-device copy; ``out`` is ``[argmax tokens (M) | accept (2) | conf bits (M)]``
-    so the results come back in a single device-to-host copy."""
+    so the results come back in a single device-to-host copy, or by the stores of a captured step's last launch."""
     M: int
     step_in: torch.Tensor        # int32 [3M+2] device
     step_in_host: torch.Tensor   # pinned mirror
@@ -415,11 +416,21 @@ class StepIO:
     out_host: torch.Tensor       # pinned mirror
     uploaded: "torch.cuda.Event"  # recorded once step_in_host has been consumed: after the
                                   # eager upload, or after the replay of a graph that carries it
-    downloaded: bool = False      # the last replay copies `out` into `out_host` itself
+    inputs_host: torch.Tensor    # `step_in_host` and three words more: rows to commit before the step (decode_ops.step_after)
+    downloaded: bool = False      # the last replay stores its results into `out_host` itself
     arrived: bool = False         # .. and has: its results were seen there
 
     #: what no word of ``out`` is: a host that waits for a replay's results looks for words that are still this
     PENDING = -2 ** 31
+
+    def pending(self, rows: int) -> np.ndarray:
+        """``out_host`` while the results of ``rows`` projected rows are waited for."""
+        words = np.zeros(2 * self.M + 2, dtype=np.int32)
+        words[:rows] = words[self.M: self.M + 2 + rows] = self.PENDING
+        return words
+
+    def also_to(self, **more) -> "decode_ops.AlsoTo":
+        return decode_ops.AlsoTo(self.out_host, self.M, self.M + 2, **more)
 
     @property
     def meta(self) -> torch.Tensor:
@@ -447,9 +458,10 @@ class StepIO:
 
     @classmethod
     def allocate(cls, M: int, device) -> "StepIO":
+        inputs = torch.zeros(3 * M + 5, dtype=torch.int32).pin_memory()
         return cls(M=M,
                    step_in=torch.zeros(3 * M + 2, dtype=torch.int32, device=device),
-                   step_in_host=torch.zeros(3 * M + 2, dtype=torch.int32).pin_memory(),
+                   step_in_host=inputs[:3 * M + 2], inputs_host=inputs,
                    out=torch.zeros(2 * M + 2, dtype=torch.int32, device=device),
                    out_host=torch.zeros(2 * M + 2, dtype=torch.int32).pin_memory(),
                    uploaded=torch.cuda.Event())
@@ -558,7 +570,8 @@ def _fused(w: PackedLinear, m: int, stream: ctypes.c_void_p, *, act, act_aux, ac
 
 def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tensor, sigma: int,
                  rope: Tuple[torch.Tensor, torch.Tensor], logits_start: int, logits_end: int,
-                 threshold: float, head_mode: str = "native", one: Optional["decode_ops.StepOne"] = None) -> None:
+                 threshold: float, head_mode: str = "native", one: Optional["decode_ops.StepOne"] = None,
+                 also: Optional["decode_ops.AlsoTo"] = None) -> None:
     """Enqueue one width-``io.M`` step on the current stream; with ``one``, all layers of it as one launch.
 
     ``kv`` is the shared buffer ``[2, n_layers, n_kv, slots, 128]``; the new rows go to
@@ -566,7 +579,7 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
     through the packed head; their argmax, confidence and accepted-prefix length land in
     ``io.tokens_out / io.conf / io.accept`` (rows counted from ``logits_start``).
     ``head_mode``: "native" (the backbone's own projection), "fp8" or "bf16_raw" (the
-    approximate draft projections, model.py:1268-1282; prepared beforehand).
+    approximate draft projections, model.py:1268-1282; prepared beforehand).  ``also``: where the results go as well.
     """
     args = model.args
     M = io.M
@@ -585,7 +598,7 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
         rows = logits_end - logits_start
         one.enqueue(model.embed, io.step_in, kv, cos, sin, sigma, eps, ws.h[0][:M], M,
                     decode_ops.FinalNorm(model.norm, logits_start, rows, **to))
-        project_rows(model, ws, None, None, rows, threshold, io.tokens_out, io.conf, io.accept, head_mode)
+        project_rows(model, ws, None, None, rows, threshold, io.tokens_out, io.conf, io.accept, head_mode, also)
         return
     plan = fused_plan(model, M)
     # wider blocks keep the ten-launch layer; BONSAI_ROPE_IN_ATTENTION=1 drops its q / k norm + RoPE
@@ -672,7 +685,7 @@ def enqueue_step(model: BonsaiDecoder, ws: Workspace, io: StepIO, kv: torch.Tens
     last_x = ws.ffn_out[logits_start:] if plan is None else h_cur[logits_start:]
     last_res = h_cur[logits_start:] if plan is None else None
     project_rows(model, ws, last_x, last_res, logits_end - logits_start, threshold, io.tokens_out, io.conf,
-                 io.accept, head_mode)
+                 io.accept, head_mode, also)
 
 
 def _bf16_rows(model: BonsaiDecoder, head_mode: str) -> bool:
@@ -684,7 +697,7 @@ def _bf16_rows(model: BonsaiDecoder, head_mode: str) -> bool:
 
 def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: Optional[torch.Tensor], last_res: Optional[torch.Tensor],
                  rows: int, threshold: float, tokens_out: torch.Tensor, conf: torch.Tensor,
-                 accept: torch.Tensor, head_mode: str = "native") -> None:
+                 accept: torch.Tensor, head_mode: str = "native", also: Optional["decode_ops.AlsoTo"] = None) -> None:
     """Final norm of ``last_x (+ last_res)``, output projection and argmax / confidence chain of ``rows`` rows
     (reference: model.py:1401-1403, fast_generate.py:111-130); without ``last_x`` of rows that the workspace has normed."""
     args = model.args
@@ -729,7 +742,7 @@ def project_rows(model: BonsaiDecoder, ws: Workspace, last_x: Optional[torch.Ten
         _gemv(ws.l_q, ws.l_s, model.head, logits, rows, stream)
     # (the attention scratch is free again by now and far larger than the chain needs)
     decode_ops.draft_chain(logits, args.vocab_size, threshold, tokens_out, conf, accept,
-                           scratch=ws.attn_scratch)
+                           scratch=ws.attn_scratch, also=also)
 
 
 # ---------------------------------------------------------------------------

@@ -14,7 +14,9 @@ Differences from the reference, by design:
   the attention kernel evaluates, so attention reads ``cache_len + M`` slots instead
   of ``sigma + M``;
 * tokens, positions and the descriptor travel in one host-to-device copy per replay and
-  argmax / confidence come back in one device-to-host copy;
+  argmax / confidence are stored to pinned memory by its last launch;
+* a greedy step can be queued behind the one before it, and a verifying block behind its draft, before the host has seen
+  their results (``step_ahead``, ``verify_drafted``);
 * intermediate buffers are shared by all graphs; graphs are captured on first use.
 """
 from __future__ import annotations
@@ -138,6 +140,11 @@ class CapturedGraph:
     logits_start: int
     logits_end: int
     one: Optional[decode_ops.StepOne] = None            # its layers are one launch
+    pending: Optional[np.ndarray] = None                # the pinned results while they are waited for
+    # of one-token steps: graphs of so many steps behind the last one, and the pinned words their tokens go to, by history length
+    next: Optional[Dict[int, "torch.cuda.CUDAGraph"]] = None
+    ring: Optional[torch.Tensor] = None
+    at: int = 0                                         # history length of the last of them
 
 
 class _WholeDevice:
@@ -201,6 +208,9 @@ class GraphAtlas:
         self.graphs: Dict[Tuple[int, int, str], CapturedGraph] = {}
         self._prompt: Optional[PromptBuffers] = None   # sized by the longest block so far
         self._positions: Optional[torch.Tensor] = None
+        self._drafted = torch.zeros(max(self.M_max, self.D), dtype=torch.int32, device=self.device)   # the last draft's tokens
+        self._last: Optional[CapturedGraph] = None   # whose replay was the last use of the workspace, as a graph
+        self._owed: Optional[Tuple[int, int, int, int]] = None   # segment, first row, cache_len, rows: see commit_with_next
         self.replays = 0
         # steps of one token and of up to sixteen as one launch (model.step_one), with the weights of the last capture or,
         # without graphs, of the last step
@@ -213,15 +223,21 @@ class GraphAtlas:
 
     #: replays with separate launches after a step that did not get the whole device
     BACK_OFF = 64
+    #: tokens of one-token steps that the host has not read yet, at most
+    RING = 16
+    #: steps that a graph queues at once behind another (14 us pass between two graphs)
+    AHEAD = (4, 1)
 
     def synchronize(self) -> None:
         """Wait for everything queued on the atlas's device (the loops' timing fences)."""
+        self.settle()
         torch.cuda.synchronize(self.device)
 
     # -- KV ------------------------------------------------------------------
     def kv(self, sigma: int) -> torch.Tensor:
         """Shared buffer of segment sigma, allocated on first use
         (reference: ``_allocate_shared_kv``, fast_runtime.py:130-138)."""
+        self.settle()
         buf = self.kv_buffers.get(sigma)
         if buf is None:
             if sigma not in self.segment_ladder:
@@ -247,6 +263,24 @@ class GraphAtlas:
         if cache_len + n_accept > sigma:
             raise RuntimeError("KV commit would run past the history segment")
         decode_ops.kv_commit(self.kv(sigma), sigma + first_row, cache_len, n_accept)
+
+    def commit_with_next(self, sigma: int, cache_len: int, n_accept: int, first_row: int = 0) -> None:
+        """``commit_kv``, by the first launch of the next replay where that reads the segment's inputs anyway (blocks).  Whoever asks
+        the atlas for the history before, or waits for it (``kv``, ``synchronize``, ``settle``), has it committed first; a tensor
+        that ``kv`` returned earlier is behind until then."""
+        if n_accept <= 0:
+            return
+        if cache_len + n_accept > sigma:
+            raise RuntimeError("KV commit would run past the history segment")
+        self.settle()
+        self._owed = (sigma, first_row, cache_len, n_accept)
+
+    def settle(self) -> None:
+        """Commit what ``commit_with_next`` has left for the next replay."""
+        owed, self._owed = self._owed, None
+        if owed is not None:
+            sigma, first_row, cache_len, n_accept = owed
+            decode_ops.kv_commit(self.kv_buffers[sigma], sigma + first_row, cache_len, n_accept)
 
     def migrate_segment(self, src_sigma: int, dst_sigma: int, cache_len: int) -> None:
         """Copy live history to another segment's buffer (fast_runtime.py:510-521)."""
@@ -310,6 +344,7 @@ class GraphAtlas:
         return one
 
     def _capture_one_impl(self, M: int, sigma: int, role: str) -> CapturedGraph:
+        self._last = None
         if role not in contracts.GRAPH_ROLES:
             raise ValueError(f"unsupported graph role: {role!r}")
         if role not in self.roles:
@@ -333,11 +368,14 @@ class GraphAtlas:
         head_mode = HEAD_MODE_OF_ROLE[role]
         one = self._one_launch(M)
 
-        def run(one):
+        def run(one, also=None):
             enqueue_step(model, workspace, io, kv, sigma, rope, ls, le, threshold,
-                         head_mode=head_mode, one=one)
+                         head_mode=head_mode, one=one, also=also)
 
-        graph = None
+        goes_on = M == 1 and role == "ar"
+        ring = torch.zeros(self.RING, dtype=torch.int32).pin_memory() if goes_on else None
+        drafted = self._drafted
+        graph = graph_next = None
         if self.use_graphs:
             side = torch.cuda.Stream(device=self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
@@ -346,16 +384,26 @@ class GraphAtlas:
                 _whole_device.launch(side, warm, lambda: (run(one), warm.record(side)))
             torch.cuda.current_stream(self.device).wait_stream(side)
             torch.cuda.synchronize(self.device)
-            # the graph carries its own upload of the step inputs and download of the results
-            # (copy nodes between the pinned mirrors and the device vectors): a replay is one
-            # launch call on the host
+            # the graph carries its own upload of the step inputs and stores the results to the
+            # pinned mirror: a replay is one launch call on the host
+            also = io.also_to(**(dict(step=io.step_in, ring=ring) if goes_on else dict(tokens=drafted) if role in DRAFT_ROLES else {}))
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
-                io.step_in.copy_(io.step_in_host, non_blocking=True)
-                run(one)
-                io.out_host.copy_(io.out, non_blocking=True)
-        cg = CapturedGraph(graph=graph, io=io, M=M, sigma=sigma, role=role, P=M - self.D,
-                           logits_start=ls, logits_end=le, one=one)
+                if role == "ar":
+                    io.step_in.copy_(io.step_in_host, non_blocking=True)
+                else:
+                    decode_ops.step_after(io.inputs_host, io.step_in, drafted, kv)
+                run(one, also)
+            if goes_on:
+                graph_next = {}
+                for steps in self.AHEAD:
+                    graph_next[steps] = torch.cuda.CUDAGraph()
+                    with torch.cuda.graph(graph_next[steps]):
+                        for _ in range(steps):
+                            decode_ops.step_next(io.step_in, kv, sigma)
+                            run(one, also)
+        cg = CapturedGraph(graph=graph, io=io, M=M, sigma=sigma, role=role, P=M - self.D, logits_start=ls, logits_end=le, one=one,
+                           pending=io.pending(le - ls), next=graph_next, ring=ring)
         cg._eager = run
         return cg
 
@@ -368,6 +416,7 @@ class GraphAtlas:
         if n > sigma:
             raise RuntimeError("history does not fit the segment")
         kv = self.kv(sigma)
+        self._last = None
         block = min(n, PROMPT_BLOCK_MAX)
         with torch.inference_mode(False), torch.cuda.device(self.device):
             if self._prompt is None or self._prompt.rows < block:
@@ -404,6 +453,16 @@ class GraphAtlas:
         if not g.io.arrived:
             g.io.uploaded.synchronize()
         g.io.step_in_host.numpy()[:] = inputs
+        owed = self._owed
+        if separate or g.role == "ar" or owed is None or owed[0] != g.sigma:
+            self.settle()
+            g.io.inputs_host.numpy()[-1] = 0
+        else:
+            self._owed = None
+            g.io.inputs_host.numpy()[-3:] = (owed[0] + owed[1], owed[2], owed[3])
+        self._queue(g, separate)
+
+    def _queue(self, g: CapturedGraph, separate: bool) -> None:
         stream = torch.cuda.current_stream(self.device)
         g.io.arrived = False
         if separate:
@@ -411,6 +470,71 @@ class GraphAtlas:
         else:
             _whole_device.launch(stream, g.io.uploaded, self._launch, g, stream, g.one)
         self.replays += 1
+
+    # -- steps behind steps that the host has not seen the results of -----------
+    def _behind(self, g: CapturedGraph) -> bool:
+        """Whether a step of ``g`` can be queued without its inputs: as the graph of one launch, which separate launches do not stand
+        in for."""
+        return g.graph is not None and g.one is not None and self._separate_for == 0 and g.one.failed[0] == 0
+
+    def step_ahead(self, g: CapturedGraph, most: int = 1) -> int:
+        """Queue one-token steps behind the last one of ``g``, up to ``most``, each on the token of the one before it and with that
+        one's row committed.  Returns how many; 0 where the step has to wait for the host (``replay``).  Their tokens: ``read_step``, at
+        most ``RING`` behind."""
+        most = min(most, g.sigma - g.at)   # (each commits a row first)
+        if g.next is None or self._last is not g or most < 1 or not self._behind(g):
+            return 0
+        self.settle()
+        self._keeps_separate(g.one)   # (counts it)
+        steps = max(n for n in self.AHEAD if n <= most)
+        for _ in range(steps):
+            g.at += 1
+            g.ring.numpy()[g.at % self.RING] = StepIO.PENDING
+        stream = torch.cuda.current_stream(self.device)
+
+        def launch():
+            g.next[steps].replay()
+            g.io.uploaded.record(stream)
+
+        _whole_device.launch(stream, g.io.uploaded, launch)
+        self.replays += steps
+        return steps
+
+    def read_step(self, g: CapturedGraph, cache_len: int) -> int:
+        """The token of the step of ``g`` over ``cache_len`` slots, once it has arrived."""
+        word = cache_len % self.RING
+        ring = g.ring.numpy()
+        deadline = time.perf_counter() + 0.05
+        while ring[word] == StepIO.PENDING:
+            if time.perf_counter() > deadline:
+                g.io.uploaded.synchronize()
+                break
+        if g.one is not None and g.one.failed[0] > 1:
+            raise RuntimeError("a decode step did not end")
+        g.io.arrived = True   # its inputs have left the host, too
+        return int(ring[word])
+
+    def verify_drafted(self, g: CapturedGraph, drafted: CapturedGraph, anchor: int, positions: Sequence[int], cache_len: int,
+                       n_pend: int) -> bool:
+        """``replay`` the verify graph ``g`` on ``anchor`` and the tokens that the draft queued last will have, over ``cache_len`` slots,
+        the last ``n_pend`` of which are the draft's first rows, committed here.  False, and nothing queued, where that has to wait
+        for the host."""
+        if g.role != "verify" or g.graph is None or drafted.role not in DRAFT_ROLES or self._last is not drafted or \
+                drafted.sigma != g.sigma or (g.one is not None and not self._behind(g)):
+            return False
+        if len(positions) != g.M or g.M - 1 > drafted.logits_end - drafted.logits_start:
+            raise ValueError("positions / drafted tokens must be those of the verified block")
+        if cache_len > g.sigma or not 0 <= n_pend <= min(cache_len, drafted.M):
+            raise RuntimeError("history does not fit the segment")
+        self.settle()
+        if not g.io.arrived:
+            g.io.uploaded.synchronize()
+        g.io.inputs_host.numpy()[:] = (step_descriptor(g.role, g.M, self.D, cache_len) + list(positions) + [int(anchor)]
+                                       + [-2 ** 31 + i for i in range(g.M - 1)] + [g.sigma, cache_len - n_pend, n_pend])
+        if g.one is not None:
+            self._keeps_separate(g.one)   # (counts it)
+        self._queue(g, g.one is None)
+        return True
 
     def _keeps_separate(self, one: decode_ops.StepOne) -> bool:
         """Whether this replay keeps to the separate launches, after a step that did not get the whole device."""
@@ -432,10 +556,15 @@ class GraphAtlas:
         # (a step in one launch keeps to separate ones without a graph of theirs: capturing one here, in the middle of a
         # program's work, would disturb its other threads)
         if g.graph is not None and one is g.one:
-            g.io.out_host.numpy()[:] = StepIO.PENDING
+            g.io.out_host.numpy()[:] = g.pending
+            if g.ring is not None:
+                g.at = int(g.io.step_in_host[0])
+                g.ring.numpy()[g.at % self.RING] = StepIO.PENDING
             g.graph.replay()          # uploads, runs the step, downloads the results
             g.io.downloaded = True
+            self._last = g
         else:
+            self._last = None
             g.io.step_in.copy_(g.io.step_in_host, non_blocking=True)
             g._eager(one)
             g.io.downloaded = False
@@ -445,8 +574,8 @@ class GraphAtlas:
         """One device-to-host copy + synchronisation: (argmax tokens, confidences,
         device-side accepted-prefix length) of the projected rows."""
         if g.io.downloaded:
-            # The results themselves, as the replay's last node writes them: the event behind it is ready 7 - 11 us later, and a
-            # blocking synchronisation wakes the thread up later still.
+            # The results themselves, as the replay's last launch writes them: the event behind it is ready 7 - 11 us later,
+            # and a blocking synchronisation wakes the thread up later still.
             out = g.io.out_host.numpy()
             deadline = time.perf_counter() + 0.05
             while True:

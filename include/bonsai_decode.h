@@ -216,6 +216,16 @@ int bonsai_decode_step_block(const bonsai_step_one_desc *desc, int rows, void *s
 int bonsai_kv_commit(void *kv, int n_layers, int n_kv, int slots, int src_slot, int dst_slot,
                      int n, void *stream);
 
+/* Steps whose inputs are on the device when the step before them ends (no counterpart in the reference).
+ * bonsai_step_next: behind a one-token step whose draft chain advanced step_in (bonsai_draft_extra): its row, slot sigma of one
+ * shared buffer, becomes history slot step_in[0] - 1.
+ * bonsai_step_after: copies the 2 + 3 * rows step inputs from `from` (pinned host memory, read when the launch runs) to step_in,
+ * a token INT32_MIN + i as drafted[i] (i < drafts), and the three words behind them {src slot, dst slot, n} as bonsai_kv_commit does
+ * (n <= 0 or slots outside the buffer: nothing). */
+int bonsai_step_next(const int32_t *step_in, void *kv, int n_layers, int n_kv, int slots, int sigma, void *stream);
+int bonsai_step_after(const int32_t *from, int32_t *step_in, int rows, const int32_t *drafted, int drafts, void *kv, int n_layers,
+                      int n_kv, int slots, void *stream);
+
 /* Row argmax + confidence of the draft logits (`_fused_draft_chain`,
  * src/bonsai_sft/gpu/fast_generate.py:111-130):
  *   logits bf16 [rows, ld], the first `vocab` columns of each row are used
@@ -236,6 +246,18 @@ int64_t bonsai_draft_chain_scratch_bytes(int rows);
 int bonsai_draft_chain_ws(const void *logits, int rows, int ld, int vocab, float threshold,
                           int32_t *tokens, float *conf, int32_t *accept, void *scratch,
                           void *stream);
+
+/* .. with the results stored elsewhere as well; null pointers: not. */
+typedef struct {
+    int32_t *host;           /* pinned host memory: token r at word r, the bits of confidence r at conf_at + r, accept at accept_at */
+    int conf_at, accept_at;
+    int32_t *tokens_too;     /* device memory: token r at word r */
+    int32_t *step;           /* the inputs of the one-token step these are the results of (one row): become those of the next one, */
+    int32_t *ring;           /* whose token goes to word step[0] % ring_words (step[0] as it was) of this pinned host memory */
+    int ring_words;
+} bonsai_draft_extra;
+int bonsai_draft_chain_extra(const void *logits, int rows, int ld, int vocab, float threshold, int32_t *tokens, float *conf,
+                             int32_t *accept, void *scratch, const bonsai_draft_extra *also, void *stream);
 
 /* The split chain for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the

@@ -115,3 +115,99 @@ def test_long_generation_migrates_between_segments():
         assert out == want, fn.__name__
         assert len(calls) >= 3, fn.__name__
     assert MASK > VOCAB
+
+
+class QueueingAtlas(SymbolicAtlas):
+    """Steps queued before the results of the one in front of them are read, as ``GraphAtlas`` queues them; every third one has
+    to wait for the host."""
+    RING = 8
+
+    def __init__(self, *args, refuses=3, **kw):
+        super().__init__(*args, **kw)
+        self.refuses, self.asked, self.ring, self.last = refuses, 0, {}, None
+
+    def _refused(self):
+        self.asked += 1
+        return self.refuses and self.asked % self.refuses == 0
+
+    owed = None
+
+    def commit_with_next(self, *what, **more):
+        self.settle()
+        self.owed = what, more
+
+    def settle(self):
+        what, self.owed = self.owed, None
+        if what is not None:
+            super().commit_kv(*what[0], **what[1])
+
+    def commit_kv(self, *args, **kw):
+        self.settle()
+        return super().commit_kv(*args, **kw)
+
+    def migrate_segment(self, *args):
+        self.settle()
+        return super().migrate_segment(*args)
+
+    def synchronize(self):
+        self.settle()
+
+    def replay(self, g, tokens, positions, cache_len, n_pend=0):
+        self.settle()
+        super().replay(g, tokens, positions, cache_len, n_pend)
+        self.last = g
+        if g.M == 1:
+            g.at = cache_len
+            self.ring[cache_len % self.RING] = int(g.out[0][0])
+
+    def step_ahead(self, g, most=1):
+        if self.last is not g or most < 1 or self._refused():
+            return 0
+        steps = 4 if most >= 4 else 1
+        for _ in range(steps):
+            self.commit_kv(g.sigma, g.at, 1)
+            self.replay(g, [self.ring[g.at % self.RING]], [g.at + 1], g.at + 1)
+        return steps
+
+    def read_step(self, g, cache_len):
+        assert 0 <= g.at - cache_len <= 4
+        return self.ring[cache_len % self.RING]
+
+    def verify_drafted(self, g, drafted, anchor, positions, cache_len, n_pend):
+        if self.last is not drafted or self._refused():
+            return False
+        assert self.owed is None
+        self.commit_kv(g.sigma, cache_len - n_pend, n_pend)
+        super().replay(g, [anchor] + [int(t) for t in drafted.out[0][: g.M - 1]], positions, cache_len)
+        self.last = g
+        return True
+
+
+@pytest.mark.parametrize("refuses", [0, 1, 3])
+@pytest.mark.parametrize("prompt", PROMPTS + [list(range(5, 5 + 200))], ids=lambda p: f"prompt{len(p)}")
+def test_steps_queued_before_the_results_are_read(prompt, refuses):
+    """The same tokens, histories and accounting, across segments and up to the end of the longest, with and without an end-of-text
+    token, behind which one step more may have run."""
+    for fn, kw in ((G.ar_generate, {}), (G.speculative_generate, {}), (G.hybrid_generate, {"threshold": 0.9}),
+                   (G.hybrid_generate, {"threshold": 0.9, "hybrid_m": 9})):
+        ladder = (64, 128, 256)
+        for length in (1, 2, 9, 45, 300):
+            for eos in ((), greedy(prompt, 20)[17:18]):
+                plain, queued = SymbolicAtlas(segment_ladder=ladder), QueueingAtlas(segment_ladder=ladder, refuses=refuses)
+                results = []
+                for atlas in (plain, queued):
+                    try:
+                        results.append(fn(atlas, prompt, max_gen_len=length, eos_ids=eos, **kw))
+                    except (AssertionError, RuntimeError) as e:   # no room left: in both
+                        results.append(type(e))
+                if isinstance(results[0], type):
+                    assert results[0] is results[1]
+                    continue
+                (want, st), (got, sq) = results
+                assert got == want and {k: v for k, v in st.items() if "time" not in k and k != "ttft"} == \
+                    {k: v for k, v in sq.items() if "time" not in k and k != "ttft"}
+                assert len(queued.log) - len(plain.log) in ((0, 1) if eos and fn is G.ar_generate else (0,))
+                assert queued.owed is None
+                for s in ladder:   # history: all that was committed
+                    held = len(prompt) + len(want) - 1
+                    assert queued.kv[s][:min(s, held)] == plain.kv[s][:min(s, held)]

@@ -1,0 +1,163 @@
+"""Steps queued behind steps whose results the host has not seen: one-token steps one after the other, a verification behind its
+draft, and results that a captured step stores to pinned memory itself."""
+import numpy as np
+import pytest
+import torch
+
+from test_step_one_gpu import DEV, _model
+
+pytestmark = pytest.mark.gpu
+
+
+def _atlas(ladder=(64, 256), **kw):
+    from bitmtp_amd.runtime import GraphAtlas
+    return GraphAtlas(_model(2, 1024, 512, 8, 4), segment_ladder=ladder, **kw)
+
+
+def _history(atlas, tokens):
+    sigma = max(s for s in atlas.kv_buffers)
+    return atlas.kv(sigma)[:, :, :, :tokens].clone()
+
+
+@pytest.mark.parametrize("loop", ["ar", "speculative"])
+@pytest.mark.parametrize("prompt,length", [(1, 2), (17, 3), (20, 40), (50, 90), (150, 60)])
+def test_the_same_tokens_and_history_as_steps_that_wait(loop, prompt, length, monkeypatch):
+    """Across segments, with and without an end-of-text token, several times with the same graphs."""
+    from bitmtp_amd import generate
+    fn = generate.ar_generate if loop == "ar" else generate.speculative_generate
+    atlas = _atlas()
+    tokens = [(7 * i + 3) % 990 for i in range(prompt)]
+    plain = {}
+    with monkeypatch.context() as m:
+        m.setattr(atlas, "step_ahead", lambda g, most: 0)
+        m.setattr(atlas, "verify_drafted", lambda *a: False)
+        full = fn(atlas, tokens, max_gen_len=length)[0]
+        for eos in ((), (full[len(full) * 2 // 3],)):
+            out, st = fn(atlas, tokens, max_gen_len=length, eos_ids=eos)
+            plain[eos] = (out, st["n_iters"], _history(atlas, prompt + len(out) - 1))
+    for _ in range(2):
+        for eos, (want, n_iters, history) in plain.items():
+            out, st = fn(atlas, tokens, max_gen_len=length, eos_ids=eos)
+            assert out == want and st["n_iters"] == n_iters
+            assert torch.equal(_history(atlas, prompt + len(out) - 1), history)
+            assert all(one is None or one.failed[0] == 0 for one in (atlas._one, atlas._block))
+
+
+@pytest.mark.parametrize("loop", ["ar", "speculative"])
+def test_a_step_that_gave_up_with_others_behind_it(loop):
+    """What is queued behind it reads its results, which the launch behind it makes; then separate launches take over."""
+    from bitmtp_amd import generate
+    fn = generate.ar_generate if loop == "ar" else generate.speculative_generate
+    atlas = _atlas((256,))
+    prompt = list(range(3, 20))
+    fn(atlas, prompt, max_gen_len=4)
+    want, _ = fn(atlas, prompt, max_gen_len=12)
+    one = atlas._one if loop == "ar" else atlas._block
+    one.exchange[4:8].view(torch.int32).fill_(1)   # the mark of a launch that did not get the whole device
+    out, _ = fn(atlas, prompt, max_gen_len=12)
+    assert len(out) == 12 and atlas._separate_for > 0 and out[0] == want[0]
+    atlas._separate_for = 0
+    assert fn(atlas, prompt, max_gen_len=12)[0] == want
+
+
+def test_steps_that_have_to_wait_for_the_host():
+    """After another use of the workspace, without graphs, with separate launches, in another segment."""
+    atlas = _atlas()
+    ar, draft, verify = atlas.get_graph(1, 64, "ar"), atlas.get_graph(9, 64, "draft"), atlas.get_graph(9, 64, "verify")
+    far = atlas.get_graph(9, 256, "verify")
+    positions = list(range(3, 12))
+    assert not atlas.step_ahead(ar)
+    atlas.replay(ar, [5], [3], 3)
+    atlas.replay(draft, [5] + [999] * 8, positions, 3, 1)
+    assert not atlas.step_ahead(ar) and not atlas.step_ahead(draft)
+    assert not atlas.verify_drafted(far, draft, 5, positions, 4, 1) and not atlas.verify_drafted(draft, draft, 5, positions, 4, 1)
+    with pytest.raises(RuntimeError):
+        atlas.verify_drafted(verify, draft, 5, positions, 65, 1)
+    with pytest.raises(ValueError):
+        atlas.verify_drafted(verify, draft, 5, positions[:3], 4, 1)
+    atlas._separate_for = 1
+    assert not atlas.verify_drafted(verify, draft, 5, positions, 4, 1) and not atlas.step_ahead(ar)
+    atlas.replay(ar, [5], [3], 3)
+    assert atlas._separate_for == 0 and not atlas.step_ahead(ar)   # separate launches have not advanced its inputs
+    atlas.replay(ar, [5], [3], 3)
+    assert atlas.step_ahead(ar) == 1 and atlas.step_ahead(ar, 7) == 4
+    atlas.replay(ar, [5], [61], 61)
+    assert atlas.step_ahead(ar, 7) == 1   # the segment ends
+    kv = atlas.kv(64)
+    torch.cuda.synchronize()
+    assert atlas.step_ahead(ar, 7) == 1
+    atlas.commit_with_next(64, 7, 1)   # is committed before the next step's row replaces it
+    row = kv[:, :, :, 64].clone()
+    assert atlas.step_ahead(ar, 7) == 1 and torch.equal(atlas.kv(64)[:, :, :, 7], row)
+    assert atlas.step_ahead(ar, 7) == 0
+    atlas.prefill_prompt(list(range(40)), 64)
+    assert not atlas.step_ahead(ar)
+    eager = _atlas(use_graphs=False)
+    g = eager.get_graph(1, 64, "ar")
+    eager.replay(g, [5], [3], 3)
+    assert not eager.step_ahead(g)
+
+
+@pytest.mark.parametrize("width,role", [(1, "ar"), (9, "draft"), (9, "verify"), (32, "ar")])
+def test_commits_with_the_next_replay(width, role):
+    """The same history as commits of their own, at its first and last slots, one row and all of them, replay after replay."""
+    sigma = 64
+    atlas = _atlas((sigma, 128))
+    g, other = atlas.get_graph(width, sigma, role), atlas.get_graph(9, 128, "verify")
+    kv = atlas.kv(sigma)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    start = (torch.randn(tuple(kv.shape), generator=gen, device=DEV) * 0.5).to(torch.bfloat16)
+    commits = [(1, 1, 0), (5, width, 0), (sigma - width, width, 0), (sigma - 1, 1, width - 1), (7, max(1, width // 2), width // 2)]
+    histories = []
+    for commit in (atlas.commit_kv, atlas.commit_with_next):
+        kv.copy_(start)
+        for i, (at, n, first) in enumerate(commits * 3):
+            atlas._separate_for = 1 if i == 7 else 0   # (separate launches for one of them)
+            atlas.replay(g, [(3 * i + j) % 1000 for j in range(width)], list(range(2, 2 + width)), 2, 1 if role == "draft" else 0)
+            commit(sigma, at, n, first)
+            if i % 4 == 3:
+                atlas.read_outputs(g)
+            if i % 5 == 4:
+                atlas.replay(other, list(range(9)), list(range(3, 12)), 4)   # another segment's
+        histories.append(atlas.kv(sigma).clone())   # (what is owed is committed when the history is asked for)
+        assert atlas._owed is None
+    assert torch.equal(*histories) and not torch.equal(histories[0][:, :, :, :sigma], start[:, :, :, :sigma])
+    with pytest.raises(RuntimeError):
+        atlas.commit_with_next(sigma, sigma - width + 1, width)
+
+
+@pytest.mark.parametrize("commit", [(64, 0, 0), (64, 0, -1), (-1, 0, 1), (0, -1, 1), (64, 90, 8), (90, 0, 8), (0, 0, 2 ** 31 - 1)])
+def test_rows_outside_the_buffer_are_not_committed(commit):
+    from bitmtp_amd import decode_ops
+    kv = torch.arange(2 * 2 * 2 * 96 * 128, device=DEV).remainder(251).to(torch.bfloat16).view(2, 2, 2, 96, 128)
+    before = kv.clone()
+    inputs = torch.tensor([10, 9, 1, 2, 3, 3, 4, 5, -1, -2 ** 31, -2 ** 31 + 2] + list(commit), dtype=torch.int32).pin_memory()
+    step_in = torch.zeros(11, dtype=torch.int32, device=DEV)
+    drafted = torch.tensor([100, 101, 102], dtype=torch.int32, device=DEV)
+    decode_ops.step_after(inputs, step_in, drafted, kv)
+    assert torch.equal(kv, before) and step_in.tolist() == [10, 9, 1, 2, 3, 3, 4, 5, -1, 100, 102]
+    for n in (-5, 0, 65, 2 ** 31 - 1):   # behind a step over no slots, and past the segment
+        step_in[0] = n
+        decode_ops.step_next(step_in, kv, 64)
+        assert torch.equal(kv, before)
+    step_in[0] = 64
+    decode_ops.step_next(step_in, kv, 64)
+    before[:, :, :, 63] = before[:, :, :, 64]
+    assert torch.equal(kv, before)
+
+
+@pytest.mark.parametrize("width,role", [(1, "ar"), (9, "draft"), (12, "draft"), (9, "verify"), (32, "ar")])
+def test_results_in_pinned_memory_are_those_on_the_device(width, role):
+    atlas = _atlas((64,))
+    g = atlas.get_graph(width, 64, role)
+    rows = g.logits_end - g.logits_start
+    for i in range(4):
+        atlas.replay(g, [(i + 7 * j) % 1000 for j in range(width)], list(range(3, 3 + width)), 3, 1 if role == "draft" else 0)
+        tokens, conf, accept = atlas.read_outputs(g)
+        assert g.io.arrived
+        torch.cuda.synchronize()
+        out = g.io.out.cpu().numpy()
+        assert np.array_equal(tokens, out[:rows]) and accept == out[width]
+        assert np.array_equal(conf.view(np.int32), out[width + 2: width + 2 + rows])
+        if role == "draft":
+            assert np.array_equal(atlas._drafted[:rows].cpu().numpy(), out[:rows])
