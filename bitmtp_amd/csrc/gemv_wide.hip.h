@@ -4,20 +4,23 @@
 // every weight is multiplied with tens to thousands of tokens, and what bounds the kernel is the issue
 // of vector instructions: per scale group (128 of K) the exact int32 sums must become fp32 and meet the
 // group's scale, two operations a result (eight per 16 x 16 results, against two matrix instructions),
-// beside unpacking the weights and arranging the activations.  Counters at 3001 tokens: the vector ALU is
-// busy in 85 % of the cycles with four waves a SIMD (gate|up 19456 x 2560, 64x256) and in 60 % with two
-// (2560 rows, 128x256), the matrix cores in 30-36 %.  So
+// beside unpacking the weights and arranging the activations.  (A wave alone issues a vector instruction
+// every 2.25 ns, whichever it is, two or more together one every 1.15 ns -- left shifts, byte permutations and
+// three-operand integer ones every 1.9; a matrix instruction takes 13.6.)  So
 //   * v_mfma_i32_32x32x32_i8: half the matrix instructions of the 16 x 16 form;
 //   * weights are unpacked to 64 times their value (mfma_unpack64), which needs no offset term -- the
 //     other forms feed -2 sum(a) through the accumulator, 8 more matrix instructions per 16 x 64 x 64 --
 //     and the factor, a power of two, goes out with the division;
 //   * the accumulators start from the bits of 1.5 * 2^23, so that a sum is a float and one exact
 //     subtraction stands for the conversion;
-//   * 64 tokens x 32 rows a wave in 128 registers, four waves a SIMD, are ahead of 64 x 64 in 224
-//     where the rows fill the chip.
-// Back to back on random bytes, with 16 x 16 instructions before -> now: 19456 x 2560 at 3001 tokens 254 -> 203 us
-// (1.47 POP/s; 191 us and 1.56 within a prompt; PyTorch's int8 product reaches 1.99 at 16384^3), 2560 x 9728 123 -> 97,
-// 12288 x 2048 at 514 35 -> 26, at 256 19.6 -> 16.7, 2048 x 2048 at 256 7.1 -> 6.6.
+//   * 64 tokens x 32 rows a wave in 128 registers, four waves a SIMD, are ahead where the rows fill the
+//     chip; where they do not, 128 tokens x 32 rows, two waves a SIMD, unpack a weight once for twice the tokens.
+//     They run as a pipeline (gemv_wide_kernel): waves that keep step at the barriers otherwise all read LDS, all
+//     multiply and all add at the same time.  64 x 64 a wave without it before -> now: 2560 x 9728 at 3001 tokens 94 -> 87 us,
+//     2560 x 4096 45 -> 41, 2560 x 9728 at 2048 91 -> 78; 12288 x 2048 at 514 (64 x 256 tiles then) 24.7 -> 23.5.
+// Back to back on random bytes, with 16 x 16 instructions before -> now: 19456 x 2560 at 3001 tokens 254 -> 194 us
+// (1.54 POP/s; PyTorch's int8 product reaches 1.99 at 16384^3), 2560 x 9728 123 -> 87,
+// 12288 x 2048 at 514 35 -> 23.5, at 256 19.6 -> 16.7, 2048 x 2048 at 256 7.1 -> 6.6.
 //
 //   WM x WN waves share a staged block of WM*MT*32 tokens x WN*NT*32 rows; KS such sets of waves
 //   split K and add their fp32 results up in slice order (narrower blocks and few rows, where a
@@ -63,8 +66,8 @@ struct WideShape {
     static constexpr int kSet = 64 * WM * WN;  // threads that share a staged block
     static constexpr int kThreads = kSet * KS;
     static constexpr bool kPrivate = WM * WN == 1;  // a set is one wave: program order is enough
+    static constexpr bool kPiped = KS == 1 && WM == 1 && NT == 1 && MT % 2 == 0 && MT > 2;  // (all but group sums)
     static constexpr int kBufs = kPrivate ? 1 : 2;
-    static constexpr int kAhead = kPrivate ? 2 : 1;  // register sets of staging loads in flight
     static constexpr int kABytes = kTokens * 128, kBBytes = kRows * 16 * BITS;
     static constexpr int kSetBytes = kBufs * (kABytes + kBBytes);
     static constexpr int kElems = MT * NT * 16;  // results per lane
@@ -93,6 +96,8 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                  int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
     using S = WideShape<BITS, WM, WN, KS, MT, NT>;
     extern __shared__ __align__(16) unsigned char smem[];
+    constexpr bool kPiped = S::kPiped && !G32;
+    constexpr int kAhead = S::kPrivate ? 2 : 1;  // register sets of staging loads in flight
     const int G = K >> 7;
     const int row_bytes = K * BITS / 8;
 
@@ -165,7 +170,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
         const int task = stid + i * S::kSet;
         b_off[i] = (uint32_t)at_row(task / BCH) * (uint32_t)row_bytes + (uint32_t)((task % BCH) * 16);
     }
-    u32x4 ars[S::kAhead][AL][QW], brs[S::kAhead][BL];
+    u32x4 ars[kAhead][AL][QW], brs[kAhead][BL];
     auto load = [&](auto &ar, auto &br, int g) {
 #pragma unroll
         for (int i = 0; i < AL; ++i)
@@ -250,12 +255,13 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     v16i bias16;
 #pragma unroll
     for (int r = 0; r < 16; ++r) bias16[r] = kBias;
+    if (kPiped) asm volatile("" : "+v"(bias16));  // in registers for good: no copies in front of the products
 
     if (S::kPrivate) {
-        if (S::kAhead > 1 && gb + 1 < ge) load(ars[S::kAhead - 1], brs[S::kAhead - 1], gb + 1);
+        if (kAhead > 1 && gb + 1 < ge) load(ars[kAhead - 1], brs[kAhead - 1], gb + 1);
     } else {
         park(ars[0], brs[0], 0);
-        if (gb + 1 < ge) load(ars[0], brs[0], gb + 1);
+        if (gb + 1 < ge) load(ars[kAhead - 1], brs[kAhead - 1], gb + 1);
     }
     __syncthreads();
 
@@ -267,7 +273,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
             bonsai_wave::order_lds();  // group g - 1 is no longer read
             if (g < ge) park(ars[R], brs[R], 0);
             bonsai_wave::order_lds();
-            if (g + S::kAhead < ge) load(ars[R], brs[R], g + S::kAhead);
+            if (g + kAhead < ge) load(ars[R], brs[R], g + kAhead);
         } else {
             if (it > 0) wide_barrier();  // group g is parked; group g - 1 is no longer read
             if (g + 1 < ge) park(ars[0], brs[0], buf ^ 1);
@@ -333,9 +339,95 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
             }
         }
     };
-    for (int it = 0; it < iters; it += S::kAhead) {
-        step(it, std::integral_constant<int, 0>{});
-        if (S::kAhead > 1) step(it + 1, std::integral_constant<int, S::kAhead - 1>{});
+    if constexpr (kPiped) {
+        // A wave's token tiles one after another, as a pipeline.  While the four products of a tile run, the sums of the tile
+        // before join their results, the activations of the tile behind are on their way from LDS, and group g + 1 is parked; the
+        // barrier stands in front of the last tile, which has its operands, so that the first ones of group g + 1 arrive
+        // under it.  (sched_barrier and the empty asm hold the order: left alone, the compiler keeps all sums to the end.)
+        v4i va[2][4], vb[4];
+        v16i dd[2];
+        uint32_t packed[4] = {0u, 0u, 0u, 0u};
+        float w[2] = {0.0f, 0.0f};
+        const int x = (op_row >> 1) & 7;
+        const unsigned char *a0 = abuf + op_row * 128, *b0 = bbuf + (wn * 32 + op_row) * (16 * BITS) + kb * (8 * BITS);
+        const uint16_t *sc = scales + wn * 32 + op_row;
+        const auto read_a = [&](int i, int buf) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const u32x4 u = *reinterpret_cast<const u32x4 *>(a0 + buf * S::kABytes + i * 4096 + ((4 * kb + t) ^ x) * 16);
+                va[i & 1][t] = v4i{(int)u.x, (int)u.y, (int)u.z, (int)u.w};
+            }
+        };
+        const auto read_b = [&](int g, int buf, float &scale) {  // (behind the last group: what stands there, unused)
+            if (BITS == 2) {
+                const u32x4 p = *reinterpret_cast<const u32x4 *>(b0 + buf * S::kBBytes);
+                packed[0] = p.x;
+                packed[1] = p.y;
+                packed[2] = p.z;
+                packed[3] = p.w;
+            } else {
+                const uint2 p = *reinterpret_cast<const uint2 *>(b0 + buf * S::kBBytes);
+                packed[0] = p.x;
+                packed[2] = p.y;
+            }
+            scale = scale_to_f32<SF16>(sc[g * S::kRows]);
+        };
+        const auto unpack = [&](int t) {
+            uint32_t u[2][4];
+            mfma_unpack64<BITS>(packed[t & ~1], packed[t | 1], u[0], u[1]);
+            vb[t] = v4i{(int)u[t & 1][0], (int)u[t & 1][1], (int)u[t & 1][2], (int)u[t & 1][3]};
+            asm volatile("" : "+v"(vb[t]));
+        };
+        const auto join = [&](int i, float scale, int from, int to) {
+#pragma unroll
+            for (int r = from; r < to; ++r) {
+                acc[i][0][r] += (__int_as_float(dd[i & 1][r]) - kBiasF) * scale;
+                asm volatile("" : "+v"(acc[i][0][r]));
+            }
+        };
+        const auto group = [&](int g, auto parity) {
+            constexpr int P = decltype(parity)::value;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (i + 1 < MT) {
+                    read_a(i + 1, P);
+                } else {
+                    wide_barrier();  // group g + 1 is parked; group g is no longer read
+                    read_b(g + 1, P ^ 1, w[P ^ 1]);
+                    read_a(0, P ^ 1);
+                }
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    dd[i & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[i & 1][t], vb[t], t ? dd[i & 1] : bias16, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (t == 0) {
+                        if (i == 0 && g + 1 < ge) park(ars[0], brs[0], P ^ 1);
+                        if (i == 1 && g + 2 < ge) load(ars[0], brs[0], g + 2);
+                    } else {
+                        join(i ? i - 1 : MT - 1, w[i ? P : P ^ 1], t * 5 - 5, t == 3 ? 16 : t * 5);
+                        if (i == MT - 1) unpack(t - 1);  // (the product before has taken its operand)
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            unpack(3);
+        };
+        read_b(0, 0, w[0]);
+        read_a(0, 0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) unpack(t);
+        dd[(MT - 1) & 1] = bias16;  // "group -1": nothing, at scale 0
+        for (int g = 0; g < ge; g += 2) {
+            group(g, std::integral_constant<int, 0>{});
+            if (g + 1 < ge) group(g + 1, std::integral_constant<int, 1>{});
+        }
+        join(MT - 1, w[(ge - 1) & 1], 0, 16);
+    } else {
+        for (int it = 0; it < iters; it += kAhead) {
+            step(it, std::integral_constant<int, 0>{});
+            if (kAhead > 1) step(it + 1, std::integral_constant<int, kAhead - 1>{});
+        }
     }
     if (G32) return;
 
@@ -479,7 +571,7 @@ template <int BITS>
 const WideVariant &wide_kernel(int v) {
     static const WideVariant t[kWideVariants] = {wide_variant<BITS, 1, 8, 1, 2, 1>(), wide_variant<BITS, 1, 4, 2, 2, 1>(),
                                                  wide_variant<BITS, 1, 2, 4, 1, 1>(), wide_variant<BITS, 1, 1, 8, 1, 2>(),
-                                                 wide_variant<BITS, 1, 4, 4, 2, 1>(), wide_variant<BITS, 2, 4, 1, 2, 2>()};
+                                                 wide_variant<BITS, 1, 4, 4, 2, 1>(), wide_variant<BITS, 1, 8, 1, 4, 1>()};
     return t[v];
 }
 
@@ -505,7 +597,7 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
     };
     static constexpr Cost c[kWideVariants] = {{64, 256, 1, 3.7, 0.752, 0.571, 1.47},   {64, 128, 2, 2.94, 0.882, 0.577, 1.565},
                                               {32, 64, 4, 3.27, 0.595, 0.498, 0.554},  {32, 64, 8, 1.87, 0.791, 0.889, 2.54},
-                                              {64, 128, 4, 1.5, 1.25, 1.25, 3.0},      {128, 256, 1, 2.56, 0.898, 1.032, 7.46}};
+                                              {64, 128, 4, 1.5, 1.25, 1.25, 3.0},      {128, 256, 1, 2.0, 0.88, 1.03, 6.0}};
     const Cost &k = c[v];
     const int G = K / kGroup, unit = G % 4 == 0 ? 4 : 1;
     const int groups = (G / unit + k.slices - 1) / k.slices * unit;
