@@ -410,11 +410,12 @@ bool wide_default(const GemvProblem &q, bool g32, int n_cus, int lds_limit) {
 
 // gate|up of a wide block with silu(gate) * up behind it: out bf16 [M, N / 2]; -1 where the projection is not the wide
 // kernel's (the caller then runs projection and producer as two launches).
+// ordered: activations in operand order, with or without silu.  ask: 0 or -1 for the same call, without it.
 template <int BITS>
 int launch_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K,
-                     hipStream_t stream) {
+                     hipStream_t stream, bool silu = true, bool ordered = false, bool ask = false) {
     if (A == nullptr || B == nullptr || out == nullptr || s == nullptr || ws == nullptr) return 1;
-    if (M < 1 || N < 2 || N % 2 != 0 || K < kGroup || K % kGroup != 0) return 1;
+    if (M < 1 || N < 1 || (silu && N % 2 != 0) || K < kGroup || K % kGroup != 0) return 1;
     if ((long)M * N > 0x7fffffffL / 2) return 1;
     if (!operands_aligned(A, B, out, s, ws, OUT_BF16)) return 1;
     int dev = 0;
@@ -428,7 +429,7 @@ int launch_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *
     if (mtu.engine != 7 && !(mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(q, false, st.n_cus[dev], lds_limit))) return -1;
     const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % kWideVariants
                                                        : wide_pick<BITS>(M, N, K, st.n_cus[dev], lds_limit);
-    return v < 0 ? -1 : launch_wide<BITS>(v, q, OUT_BF16, 0, lds_limit, stream, true);
+    return v < 0 ? -1 : launch_wide<BITS>(v, q, OUT_BF16, 0, lds_limit, stream, silu, ordered, ask);
 }
 
 template <int BITS>

@@ -26,6 +26,11 @@
 //   split K and add their fp32 results up in slice order (narrower blocks and few rows, where a
 //   tile per workgroup would leave most CUs idle).
 //
+// Activations that a quantiser has left in operand order (ORDERED: a prompt's) go from memory to LDS without passing
+// registers, and nothing is transposed here: once per weight row tile it was, and is once now, by the quantiser.
+// Before -> now, us at 3001 tokens: 6144 x 2560 72 -> 65, 19456 x 2560 197 -> 180, 2560 x 4096 42 -> 40, 2560 x 9728 88 -> 83;
+// at 256: 12288 x 2048 16.1 -> 14.3, 4096 x 2048 8.6 -> 7.6, 2048 x 6144 12.0 -> 10.5, 2048 x 2048 6.3 -> 5.7.
+//
 // Per group a set stages 128 bytes of K for its tokens (4 x 4 byte transposes: operand order, see
 // gemv_core.h; 16-byte units XORed with half the row number, so that a ds_read_b128 of 16 rows meets
 // every bank once) and the packed rows, inverted where the unpacking wants it (a wave's operand read is
@@ -90,10 +95,22 @@ __device__ __forceinline__ void wide_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int BITS, int WM, int WN, int KS, int MT, int NT, bool SF16, bool G32, bool PAIRS>
-__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : 4)))
-gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
-                 int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
+// .. and what was sent to LDS has arrived
+__device__ __forceinline__ void wide_barrier_landed() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// 16 bytes a lane from memory to LDS, a wave's 1 KB from `lds` on (wave-uniform)
+__device__ __forceinline__ void wide_load_to_lds(__amdgpu_buffer_rsrc_t r, unsigned char *lds, uint32_t voffset, uint32_t soffset) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)lds, 16, voffset, soffset, 0, 0);
+#endif
+}
+
+// ORDERED: activations in operand order, as bonsai_*_quant_ordered write them
+template <int BITS, int WM, int WN, int KS, int MT, int NT, bool SF16, bool G32, bool PAIRS, bool ORDERED>
+__device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws,
+                                               int M, int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
     using S = WideShape<BITS, WM, WN, KS, MT, NT>;
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr bool kPiped = S::kPiped && !G32;
@@ -159,11 +176,18 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     constexpr int BCH = BITS;                           // 16-byte chunks of a packed row
     constexpr int BN_TASKS = S::kRows * BCH;
     constexpr int BL = (BN_TASKS + S::kSet - 1) / S::kSet;
-    uint32_t a_off[AL], b_off[BL];
+    // Activations in operand order need no registers on their way (a set of one wave, in program order, keeps them): whole
+    // blocks go from memory to LDS, 64 units of 16 bytes a wave and load, each lane reading the unit that belongs where it writes.
+    constexpr bool SENT = ORDERED && !S::kPrivate;
+    constexpr int UL = S::kTokens * 8 / S::kSet;
+    static_assert(UL * S::kSet == S::kTokens * 8 && UL >= AL && BN_TASKS % 64 == 0, "whole waves");
+    uint32_t a_off[UL], b_off[BL];
 #pragma unroll
-    for (int i = 0; i < AL; ++i) {
+    for (int i = 0; i < UL; ++i) {
         const int task = stid + i * S::kSet;
-        a_off[i] = (uint32_t)(task / QPR) * (uint32_t)K + (uint32_t)((task % QPR) * QB);
+        a_off[i] = SENT
+                       ? (uint32_t)(task >> 3) * (uint32_t)K + (uint32_t)((task & 7) ^ ((task >> 4) & 7)) * 16
+                       : (uint32_t)(task / QPR) * (uint32_t)K + (uint32_t)((task % QPR) * QB);
     }
 #pragma unroll
     for (int i = 0; i < BL; ++i) {
@@ -192,7 +216,10 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
             const int row = task / QPR, q = task % QPR;
             u32x4 *dst = a + row * 8;
             const int x = (row >> 1) & 7;
-            if (BITS == 2) {
+            if (ORDERED) {
+#pragma unroll
+                for (int u = 0; u < QW; ++u) dst[(QW * q + u) ^ x] = ar[i][u];
+            } else if (BITS == 2) {
                 const u32x4 v = ar[i][0];
                 dst[q ^ x] = transpose4x4_bytes(v.x, v.y, v.z, v.w);
             } else {
@@ -208,7 +235,20 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                 b[stid + i * S::kSet] = u32x4{mfma_flip<BITS>(br[i].x), mfma_flip<BITS>(br[i].y), mfma_flip<BITS>(br[i].z), mfma_flip<BITS>(br[i].w)};
     };
 
-    load(ars[0], brs[0], gb < ge ? gb : 0);
+    const auto send = [&](int g, int buf) {
+#pragma unroll
+        for (int i = 0; i < UL; ++i)
+            wide_load_to_lds(rA, abuf + buf * S::kABytes + (i * S::kSet + wsub * 64) * 16, a_off[i], (uint32_t)(g * 128));
+#pragma unroll
+        for (int i = 0; i < BL; ++i)
+            if (BN_TASKS % S::kSet == 0 || wsub * 64 + i * S::kSet < BN_TASKS)
+                wide_load_to_lds(rB, bbuf + buf * S::kBBytes + (i * S::kSet + wsub * 64) * 16, b_off[i], (uint32_t)(g * 16 * BITS));
+    };
+    if (SENT) {
+        if (gb < ge) send(gb, 0);
+    } else {
+        load(ars[0], brs[0], gb < ge ? gb : 0);
+    }
 
     // ---- scales of the row block, transposed, and the multipliers
     if (!G32) {
@@ -240,6 +280,10 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
         }
     }
 
+    const auto flip = [](uint32_t (&p)[4]) {  // (as parking does for the others)
+#pragma unroll
+        for (int t = 0; t < 4; t += BITS == 2 ? 1 : 2) p[t] = mfma_flip<BITS>(p[t]);
+    };
     typedef int v16i __attribute__((ext_vector_type(16)));
     float acc[MT][NT][16];
 #pragma unroll
@@ -255,15 +299,19 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     v16i bias16;
 #pragma unroll
     for (int r = 0; r < 16; ++r) bias16[r] = kBias;
-    if (kPiped) asm volatile("" : "+v"(bias16));  // in registers for good: no copies in front of the products
-
+    if (kPiped || SENT) asm volatile("" : "+v"(bias16));  // in registers for good: no copies in front of the products
     if (S::kPrivate) {
         if (kAhead > 1 && gb + 1 < ge) load(ars[kAhead - 1], brs[kAhead - 1], gb + 1);
-    } else {
+    } else if (!SENT) {
         park(ars[0], brs[0], 0);
-        if (gb + 1 < ge) load(ars[kAhead - 1], brs[kAhead - 1], gb + 1);
+        if (gb + 1 < ge) load(ars[0], brs[0], gb + 1);
     }
-    __syncthreads();
+    if (SENT) {
+        wide_barrier_landed();
+        if (kPiped && gb + 1 < ge) send(gb + 1, 1);
+    } else {
+        __syncthreads();
+    }
 
     const auto step = [&](int it, auto set_of) {
         constexpr int R = decltype(set_of)::value;  // register set of this group
@@ -274,6 +322,9 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
             if (g < ge) park(ars[R], brs[R], 0);
             bonsai_wave::order_lds();
             if (g + kAhead < ge) load(ars[R], brs[R], g + kAhead);
+        } else if (SENT) {
+            if (it > 0) wide_barrier_landed();  // group g is there; group g - 1 is no longer read
+            if (g + 1 < ge) send(g + 1, buf ^ 1);
         } else {
             if (it > 0) wide_barrier();  // group g is parked; group g - 1 is no longer read
             if (g + 1 < ge) park(ars[0], brs[0], buf ^ 1);
@@ -300,6 +351,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                 p[0] = pp.x;
                 p[2] = pp.y;
             }
+            if (SENT) flip(p);
             w[j] = G32 ? 0.0f : scale_to_f32<SF16>(scales[g * S::kRows + (wn * NT + j) * 32 + op_row]);
 #pragma unroll
             for (int t = 0; t < 4; t += 2) {
@@ -370,6 +422,7 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                 packed[0] = p.x;
                 packed[2] = p.y;
             }
+            if (SENT) flip(packed);
             scale = scale_to_f32<SF16>(sc[g * S::kRows]);
         };
         const auto unpack = [&](int t) {
@@ -393,7 +446,12 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                 if (i + 1 < MT) {
                     read_a(i + 1, P);
                 } else {
-                    wide_barrier();  // group g + 1 is parked; group g is no longer read
+                    if (SENT) {
+                        wide_barrier_landed();  // group g + 1 is there; group g is no longer read
+                        if (g + 2 < ge) send(g + 2, P);
+                    } else {
+                        wide_barrier();  // group g + 1 is parked; group g is no longer read
+                    }
                     read_b(g + 1, P ^ 1, w[P ^ 1]);
                     read_a(0, P ^ 1);
                 }
@@ -402,8 +460,8 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
                     dd[i & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[i & 1][t], vb[t], t ? dd[i & 1] : bias16, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                     if (t == 0) {
-                        if (i == 0 && g + 1 < ge) park(ars[0], brs[0], P ^ 1);
-                        if (i == 1 && g + 2 < ge) load(ars[0], brs[0], g + 2);
+                        if (!SENT && i == 0 && g + 1 < ge) park(ars[0], brs[0], P ^ 1);
+                        if (!SENT && i == 1 && g + 2 < ge) load(ars[0], brs[0], g + 2);
                     } else {
                         join(i ? i - 1 : MT - 1, w[i ? P : P ^ 1], t * 5 - 5, t == 3 ? 16 : t * 5);
                         if (i == MT - 1) unpack(t - 1);  // (the product before has taken its operand)
@@ -541,6 +599,20 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     }
 }
 
+template <int BITS, int WM, int WN, int KS, int MT, int NT, bool SF16, bool G32, bool PAIRS>
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : 4)))
+gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
+                 int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
+    gemv_wide_tile<BITS, WM, WN, KS, MT, NT, SF16, G32, PAIRS, false>(A, B, out, s, ws, M, N, K, out_f32, tiles_m, tiles_n, flags);
+}
+
+template <int BITS, int WM, int WN, int KS, int MT, int NT, bool PAIRS>
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : 4)))
+gemv_wide_ordered_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
+                         int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
+    gemv_wide_tile<BITS, WM, WN, KS, MT, NT, false, false, PAIRS, true>(A, B, out, s, ws, M, N, K, out_f32, tiles_m, tiles_n, flags);
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -548,7 +620,7 @@ using WideKernelFn = void (*)(const int8_t *, const uint8_t *, void *, const flo
                               int, int, int, int, int);
 
 struct WideVariant {
-    WideKernelFn fn[4];  // bf16 scales, fp16 scales, group sums, pairs (bf16 scales)
+    WideKernelFn fn[6];  // bf16 scales, fp16 scales, group sums, pairs (bf16 scales); bf16 scales and pairs on ordered activations
     int tokens, rows, threads;
     size_t (*lds)(int K);
     int t[5];  // template arguments, for the launch record
@@ -560,7 +632,9 @@ constexpr WideVariant wide_variant() {
     return WideVariant{{gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, false>,
                         gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, true, false, false>,
                         gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, true, false>,
-                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, true>},
+                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, true>,
+                        gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, false>,
+                        gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, true>},
                        S::kTokens, S::kRows, S::kThreads, S::lds_bytes, {WM, WN, KS, MT, NT}};
 }
 
@@ -578,7 +652,7 @@ const WideVariant &wide_kernel(int v) {
 template <int BITS>
 int wide_init_device(int max_lds) {
     for (int v = 0; v < kWideVariants; ++v)
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < 6; ++k)
             if (hipFuncSetAttribute(reinterpret_cast<const void *>(wide_kernel<BITS>(v).fn[k]),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, max_lds) != hipSuccess)
                 return 2;
@@ -629,9 +703,10 @@ int wide_pick(int M, int N, int K, int n_cus, int lds_limit) {
     return best;
 }
 
-// Launches one problem as variant v; -1 when it does not fit (the caller falls back).
+// Launches one problem as variant v; -1 when it does not fit (the caller falls back).  ask: the answer alone, 0 or -1
 template <int BITS>
-int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream, bool pairs = false) {
+int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream, bool pairs = false,
+                bool ordered = false, bool ask = false) {
     const WideVariant &k = wide_kernel<BITS>(v);
     if (!wide_fits<BITS>(v, q.K, lds_limit)) return -1;
     // pairs: N / 2 gate rows, N / 2 up rows -> silu(gate) * up, 16-byte pieces of whole rows; one resource over all of B
@@ -641,14 +716,15 @@ int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int l
     const int tile_rows = pairs ? k.rows / 2 : k.rows, all_rows = pairs ? q.N / 2 : q.N;
     const int tm = (q.M + k.tokens - 1) / k.tokens, tn = (all_rows + tile_rows - 1) / tile_rows;
     if ((long)tm * tn > (1L << 28)) return -1;
+    if (ask) return 0;
     const int per = (tm * tn + kWideXcds - 1) / kWideXcds;
     const int flags = ((q.K / kGroup) % 4 == 0 && (reinterpret_cast<uintptr_t>(q.ws) & 7) == 0 ? 1 : 0) |
                       (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0);
-    const int variant = pairs ? 3 : (out_kind == OUT_G32 ? 2 : scale_kind);
+    const int variant = ordered ? (pairs ? 5 : 4) : (pairs ? 3 : (out_kind == OUT_G32 ? 2 : scale_kind));
     hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), k.lds(q.K), stream, q.A, q.B, q.out,
                        q.s, reinterpret_cast<const uint16_t *>(q.ws), q.M, q.N, q.K, out_kind == OUT_F32 ? 1 : 0, tm,
                        tn, flags);
-    note_kernel("gemv_wide_kernel", BITS, k.t[0], k.t[1], k.t[2], k.t[3], k.t[4], variant);
+    note_kernel(ordered ? "gemv_wide_ordered_kernel" : "gemv_wide_kernel", BITS, k.t[0], k.t[1], k.t[2], k.t[3], k.t[4], variant);
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
