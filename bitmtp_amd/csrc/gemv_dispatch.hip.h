@@ -429,7 +429,7 @@ int launch_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *
     if (mtu.engine != 7 && !(mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(q, false, st.n_cus[dev], lds_limit))) return -1;
     const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % kWideVariants
                                                        : wide_pick<BITS>(M, N, K, st.n_cus[dev], lds_limit);
-    return v < 0 ? -1 : launch_wide<BITS>(v, q, OUT_BF16, 0, lds_limit, stream, silu, ordered, ask);
+    return v < 0 ? -1 : launch_wide<BITS>(v, q, OUT_BF16, 0, lds_limit, stream, silu, ordered, ask, st.n_cus[dev]);
 }
 
 template <int BITS>

@@ -75,15 +75,16 @@ struct WideShape {
     static constexpr int kBufs = kPrivate ? 1 : 2;
     static constexpr int kABytes = kTokens * 128, kBBytes = kRows * 16 * BITS;
     static constexpr int kSetBytes = kBufs * (kABytes + kBBytes);
+    static constexpr bool kDeep = !kPrivate && KS > 1 && WM * WN * KS <= 8;  // has three buffers of ordered activations where they fit
     static constexpr int kElems = MT * NT * 16;  // results per lane
     static constexpr int kOutPitch = kRows * 2 + 16;
     static constexpr int kShare = kElems / KS;  // results per lane that a K slice finishes
     static constexpr int kRedBytes = (KS - 1) * kSet * kElems * 4;
     // scales [G][rows] u16, then multipliers and their reciprocals [tokens] (they stay), then the staged blocks, whose
     // space the K slices' partial sums and the outgoing tile take over
-    static size_t lds_bytes(int K) {
+    static size_t lds_bytes(int K, bool deep) {
         const size_t keep = (size_t)(K / kGroup) * kRows * 2 + kTokens * 8;
-        const size_t stage = (size_t)KS * kSetBytes;
+        const size_t stage = (size_t)KS * (kSetBytes + (deep && kDeep ? kABytes + kBBytes : 0));
         const size_t after = kRedBytes + (size_t)kTokens * kOutPitch;
         return keep + (stage > after ? stage : after);
     }
@@ -98,6 +99,12 @@ __device__ __forceinline__ void wide_barrier() {
 // .. and what was sent to LDS has arrived
 __device__ __forceinline__ void wide_barrier_landed() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// .. but for the last N loads (or fewer: what is waited for is older than the last block, of N loads at least)
+template <int N>
+__device__ __forceinline__ void wide_barrier_landed_but() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 // 16 bytes a lane from memory to LDS, a wave's 1 KB from `lds` on (wave-uniform)
@@ -152,8 +159,10 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
     uint16_t *scales = reinterpret_cast<uint16_t *>(smem);
     float2 *mult = reinterpret_cast<float2 *>(smem + (size_t)G * S::kRows * 2);
     unsigned char *work = reinterpret_cast<unsigned char *>(mult + S::kTokens);
-    unsigned char *abuf = work + set * S::kSetBytes;
-    unsigned char *bbuf = abuf + S::kBufs * S::kABytes;
+    // three buffers (SENT): two groups are on their way while one is multiplied
+    const int bufs = ORDERED && S::kDeep && (flags & 4) != 0 ? 3 : S::kBufs;
+    unsigned char *abuf = work + set * (bufs * (S::kABytes + S::kBBytes));
+    unsigned char *bbuf = abuf + bufs * S::kABytes;
 
     const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t *>(A + (size_t)m0 * K), 0, mv * K, kMxlBufferWord3);
@@ -308,23 +317,31 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
     }
     if (SENT) {
         wide_barrier_landed();
-        if (kPiped && gb + 1 < ge) send(gb + 1, 1);
+        if ((kPiped || (S::kDeep && bufs == 3)) && gb + 1 < ge) send(gb + 1, 1);
     } else {
         __syncthreads();
     }
 
+    int now = 0;  // buffer of the group, of three
     const auto step = [&](int it, auto set_of) {
         constexpr int R = decltype(set_of)::value;  // register set of this group
         const int g = gb + it;
-        const int buf = S::kPrivate ? 0 : (it & 1);
+        const int buf = S::kPrivate ? 0 : (SENT && S::kDeep ? now : it & 1);
         if (S::kPrivate) {
             bonsai_wave::order_lds();  // group g - 1 is no longer read
             if (g < ge) park(ars[R], brs[R], 0);
             bonsai_wave::order_lds();
             if (g + kAhead < ge) load(ars[R], brs[R], g + kAhead);
         } else if (SENT) {
-            if (it > 0) wide_barrier_landed();  // group g is there; group g - 1 is no longer read
-            if (g + 1 < ge) send(g + 1, buf ^ 1);
+            // group g is there; group g - 1 is no longer read
+            if (S::kDeep && bufs == 3 && g + 1 < ge) {
+                if (it > 0) wide_barrier_landed_but<UL + (BN_TASKS % S::kSet == 0 ? BL : 0)>();
+                if (g + 2 < ge) send(g + 2, now == 0 ? 2 : now - 1);
+            } else {
+                if (it > 0) wide_barrier_landed();
+                if (bufs != 3 && g + 1 < ge) send(g + 1, buf ^ 1);
+            }
+            if (S::kDeep) now = now + 1 == bufs ? 0 : now + 1;
         } else {
             if (it > 0) wide_barrier();  // group g is parked; group g - 1 is no longer read
             if (g + 1 < ge) park(ars[0], brs[0], buf ^ 1);
@@ -622,7 +639,8 @@ using WideKernelFn = void (*)(const int8_t *, const uint8_t *, void *, const flo
 struct WideVariant {
     WideKernelFn fn[6];  // bf16 scales, fp16 scales, group sums, pairs (bf16 scales); bf16 scales and pairs on ordered activations
     int tokens, rows, threads;
-    size_t (*lds)(int K);
+    size_t (*lds)(int K, bool deep);
+    bool deep;
     int t[5];  // template arguments, for the launch record
 };
 
@@ -635,7 +653,7 @@ constexpr WideVariant wide_variant() {
                         gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, true>,
                         gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, false>,
                         gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, true>},
-                       S::kTokens, S::kRows, S::kThreads, S::lds_bytes, {WM, WN, KS, MT, NT}};
+                       S::kTokens, S::kRows, S::kThreads, S::lds_bytes, S::kDeep, {WM, WN, KS, MT, NT}};
 }
 
 // (tokens x rows of a workgroup, K slices)
@@ -687,7 +705,7 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
 template <int BITS>
 bool wide_fits(int v, int K, int lds_limit) {
     const WideVariant &k = wide_kernel<BITS>(v);
-    return k.lds(K) <= (size_t)lds_limit && (long)k.rows * K <= (1L << 30) && (long)k.tokens * K <= (1L << 30);
+    return k.lds(K, false) <= (size_t)lds_limit && (long)k.rows * K <= (1L << 30) && (long)k.tokens * K <= (1L << 30);
 }
 
 // The variant with the smallest estimate among those that take rows of K weights: over 220 drawn blocks 0.8 % behind
@@ -706,7 +724,7 @@ int wide_pick(int M, int N, int K, int n_cus, int lds_limit) {
 // Launches one problem as variant v; -1 when it does not fit (the caller falls back).  ask: the answer alone, 0 or -1
 template <int BITS>
 int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream, bool pairs = false,
-                bool ordered = false, bool ask = false) {
+                bool ordered = false, bool ask = false, int n_cus = 0) {
     const WideVariant &k = wide_kernel<BITS>(v);
     if (!wide_fits<BITS>(v, q.K, lds_limit)) return -1;
     // pairs: N / 2 gate rows, N / 2 up rows -> silu(gate) * up, 16-byte pieces of whole rows; one resource over all of B
@@ -720,10 +738,15 @@ int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int l
     const int per = (tm * tn + kWideXcds - 1) / kWideXcds;
     const int flags = ((q.K / kGroup) % 4 == 0 && (reinterpret_cast<uintptr_t>(q.ws) & 7) == 0 ? 1 : 0) |
                       (q.N % 8 == 0 && (reinterpret_cast<uintptr_t>(q.out) & 15) == 0 ? 2 : 0);
+    // Weights from HBM and activations that another die has written take longer than a group: three buffers where no second
+    // workgroup on the CU fills the wait.  256 tokens within a prompt, us, two -> three: 2048 x 6144 (256 tiles) 13.0 -> 11.2, 2048 x 2048
+    // level; 4096 x 2048 (512 tiles) 8.7 -> 9.0, gate|up 12288 x 2048 (384 tiles) 16.1 -> 16.4.
+    const size_t three = k.lds(q.K, true);
+    const bool deep = ordered && k.deep && tm * tn <= n_cus && three <= (size_t)lds_limit;
     const int variant = ordered ? (pairs ? 5 : 4) : (pairs ? 3 : (out_kind == OUT_G32 ? 2 : scale_kind));
-    hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), k.lds(q.K), stream, q.A, q.B, q.out,
+    hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), deep ? three : k.lds(q.K, false), stream, q.A, q.B, q.out,
                        q.s, reinterpret_cast<const uint16_t *>(q.ws), q.M, q.N, q.K, out_kind == OUT_F32 ? 1 : 0, tm,
-                       tn, flags);
+                       tn, flags | (deep ? 4 : 0));
     note_kernel(ordered ? "gemv_wide_ordered_kernel" : "gemv_wide_kernel", BITS, k.t[0], k.t[1], k.t[2], k.t[3], k.t[4], variant);
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
