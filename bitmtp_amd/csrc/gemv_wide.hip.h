@@ -28,8 +28,8 @@
 //
 // Activations that a quantiser has left in operand order (ORDERED: a prompt's) go from memory to LDS without passing
 // registers, and nothing is transposed here: once per weight row tile it was, and is once now, by the quantiser.
-// Before -> now, us at 3001 tokens: 6144 x 2560 72 -> 65, 19456 x 2560 197 -> 180, 2560 x 4096 42 -> 40, 2560 x 9728 88 -> 83;
-// at 256: 12288 x 2048 16.1 -> 14.3, 4096 x 2048 8.6 -> 7.6, 2048 x 6144 12.0 -> 10.5, 2048 x 2048 6.3 -> 5.7.
+// From -> to operand order, us at 3001 tokens: 6144 x 2560 72 -> 65, 19456 x 2560 197 -> 180, 2560 x 4096 42 -> 40, 2560 x 9728
+// 88 -> 83; at 256: 12288 x 2048 16.1 -> 14.3, 4096 x 2048 8.6 -> 7.6, 2048 x 6144 12.0 -> 10.5, 2048 x 2048 6.3 -> 5.7.
 //
 // Per group a set stages 128 bytes of K for its tokens (4 x 4 byte transposes: operand order, see
 // gemv_core.h; 16-byte units XORed with half the row number, so that a ds_read_b128 of 16 rows meets
@@ -64,6 +64,30 @@ namespace bonsai {
 
 constexpr int kWideXcds = 8;
 constexpr int kWideTokenGroup = 8;  // token tiles walked before the next row tile
+
+// mfma_unpack64 for two dwords at a time: one shift of 64 bits for both (left shifts run at half the rate of other instructions, and this one
+// at that of a 32-bit one; what crosses from one dword to the other is masked): 6144 x 2560 at 3001 ordered tokens 63.9 -> 62.9 us,
+// 2560 x 9728 82.0 -> 81.3; at 256 12288 x 2048 14.6 -> 14.5, 4096 x 2048 7.4 -> 7.2, 2048 x 6144 10.4 -> 10.0.  H: which two operands, and from which dwords --
+// T2 2H and 2H + 1 from the dwords of those numbers, Q1 H and H + 2 from dwords 0 and 2.
+template <int BITS, int H, typename V>
+__device__ __forceinline__ void wide_unpack(const uint32_t (&p)[4], V (&vb)[4]) {
+    const uint64_t q = BITS == 2 ? (uint64_t)p[2 * H + 1] << 32 | p[2 * H] : (uint64_t)p[2] << 32 | p[0];
+    V &lo = vb[BITS == 2 ? 2 * H : H], &hi = vb[BITS == 2 ? 2 * H + 1 : H + 2];
+    const auto place = [&](int k, uint64_t x) {
+        lo[k] = (int)(BITS == 2 ? (uint32_t)x & 0xC0C0C0C0u : ((uint32_t)x & 0x80808080u) | 0x40404040u);
+        hi[k] = (int)(BITS == 2 ? (uint32_t)(x >> 32) & 0xC0C0C0C0u : ((uint32_t)(x >> 32) & 0x80808080u) | 0x40404040u);
+    };
+    const auto shifted = [&](auto by) {
+        uint64_t x = q << decltype(by)::value;
+        if (decltype(by)::value != 0) asm("" : "+v"(x));  // (or the masks would let the compiler split it into two)
+        return x;
+    };
+    constexpr int from = BITS == 2 ? 6 : (H == 0 ? 7 : 3), step = BITS == 2 ? 2 : 1;
+    place(0, shifted(std::integral_constant<int, from>{}));
+    place(1, shifted(std::integral_constant<int, from - step>{}));
+    place(2, shifted(std::integral_constant<int, from - 2 * step>{}));
+    place(3, shifted(std::integral_constant<int, from - 3 * step>{}));
+}
 
 template <int BITS, int WM, int WN, int KS, int MT, int NT>
 struct WideShape {
@@ -370,13 +394,8 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
             }
             if (SENT) flip(p);
             w[j] = G32 ? 0.0f : scale_to_f32<SF16>(scales[g * S::kRows + (wn * NT + j) * 32 + op_row]);
-#pragma unroll
-            for (int t = 0; t < 4; t += 2) {
-                uint32_t b0[4], b1[4];
-                mfma_unpack64<BITS>(p[t], p[t + 1], b0, b1);
-                vb[j][t] = v4i{(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3]};
-                vb[j][t + 1] = v4i{(int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
-            }
+            wide_unpack<BITS, 0>(p, vb[j]);
+            wide_unpack<BITS, 1>(p, vb[j]);
         }
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
@@ -442,12 +461,6 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
             if (SENT) flip(packed);
             scale = scale_to_f32<SF16>(sc[g * S::kRows]);
         };
-        const auto unpack = [&](int t) {
-            uint32_t u[2][4];
-            mfma_unpack64<BITS>(packed[t & ~1], packed[t | 1], u[0], u[1]);
-            vb[t] = v4i{(int)u[t & 1][0], (int)u[t & 1][1], (int)u[t & 1][2], (int)u[t & 1][3]};
-            asm volatile("" : "+v"(vb[t]));
-        };
         const auto join = [&](int i, float scale, int from, int to) {
 #pragma unroll
             for (int r = from; r < to; ++r) {
@@ -481,17 +494,23 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
                         if (!SENT && i == 1 && g + 2 < ge) load(ars[0], brs[0], g + 2);
                     } else {
                         join(i ? i - 1 : MT - 1, w[i ? P : P ^ 1], t * 5 - 5, t == 3 ? 16 : t * 5);
-                        if (i == MT - 1) unpack(t - 1);  // (the product before has taken its operand)
+                        if (i == MT - 1 && t > 1) {  // (operands that the products so far have taken)
+                            if (t == 2)
+                                wide_unpack<BITS, 0>(packed, vb);
+                            else
+                                wide_unpack<BITS, 1>(packed, vb);
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(vb[u]));
+                        }
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            unpack(3);
         };
         read_b(0, 0, w[0]);
         read_a(0, 0);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) unpack(t);
+        wide_unpack<BITS, 0>(packed, vb);
+        wide_unpack<BITS, 1>(packed, vb);
         dd[(MT - 1) & 1] = bias16;  // "group -1": nothing, at scale 0
         for (int g = 0; g < ge; g += 2) {
             group(g, std::integral_constant<int, 0>{});
@@ -623,8 +642,10 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     gemv_wide_tile<BITS, WM, WN, KS, MT, NT, SF16, G32, PAIRS, false>(A, B, out, s, ws, M, N, K, out_f32, tiles_m, tiles_n, flags);
 }
 
+// (six waves a SIMD where a wave has one tile of T2: three workgroups a CU.  4096 x 2048 at 256 tokens level, 6144 x 2560 at 3001
+// 117 -> 99 us.  In the kernel above, with its staging registers, that spills: 8.1 -> 9.1.)
 template <int BITS, int WM, int WN, int KS, int MT, int NT, bool PAIRS>
-__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : 4)))
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : (MT * NT == 1 && BITS == 2 ? 6 : 4))))
 gemv_wide_ordered_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
                          int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
     gemv_wide_tile<BITS, WM, WN, KS, MT, NT, false, false, PAIRS, true>(A, B, out, s, ws, M, N, K, out_f32, tiles_m, tiles_n, flags);
