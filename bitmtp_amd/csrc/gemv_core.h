@@ -248,25 +248,9 @@ BONSAI_HD void mfma_unpack(uint32_t p0, uint32_t p1, uint32_t b0[4], uint32_t b1
 
 // The same slots holding 64 times the weights themselves: a code's two bits at the top of a byte, the upper
 // one inverted, ARE the signed byte 64 (code - 2); a sign bit inverted above a one is +-64.  `p` is a packed
-// dword with its inversions done (mfma_flip: once per dword, however often it is unpacked).
+// dword with its inversions done (mfma_flip: once per dword, however often it is unpacked -- wide_unpack, gemv_wide.hip.h).
 template <int BITS>
 BONSAI_HD uint32_t mfma_flip(uint32_t p) { return BITS == 2 ? p ^ 0xAAAAAAAAu : ~p; }
-template <int BITS>
-BONSAI_HD void mfma_unpack64(uint32_t p0, uint32_t p1, uint32_t b0[4], uint32_t b1[4]) {
-    if (BITS == 2) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            b0[j] = (p0 << (6 - 2 * j)) & 0xC0C0C0C0u;
-            b1[j] = (p1 << (6 - 2 * j)) & 0xC0C0C0C0u;
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            b0[j] = ((p0 << (7 - j)) & 0x80808080u) | 0x40404040u;
-            b1[j] = ((p0 << (3 - j)) & 0x80808080u) | 0x40404040u;
-        }
-    }
-}
 
 // Staged activations of the MFMA path: token-major, one 16-byte unit per (group,
 // kb, t) in natural K order, each token padded by one unit so that the sixteen

@@ -395,7 +395,7 @@ Narrow narrow_kernel(const GemvProblem &q, bool g32, int n_cus) {
 // kernel has no estimate: from five tokens on it is behind (19000 x 2688: dot4 9.1 us at four tokens, 15.5 at nine,
 // against 10.6 at any width up to 32; 1086 x 1152 at 245 tokens 24.5 against 5.6).
 template <int BITS>
-bool wide_default(const GemvProblem &q, bool g32, int n_cus, int lds_limit) {
+bool wide_default(const GemvProblem &q, bool g32, int n_cus, int lds_limit, bool ordered = false) {
     if (q.M <= kMfmaTokens && q.K % 512 == 0) return false;
     const Narrow other = narrow_kernel<BITS>(q, g32, n_cus);
     if (other == Narrow::dot4) return q.M >= kWideMinRagged;
@@ -404,8 +404,8 @@ bool wide_default(const GemvProblem &q, bool g32, int n_cus, int lds_limit) {
     const double narrow = other == Narrow::lean       ? 3.1 + G * (0.0087 + 0.051 * per_cu)
                           : q.N <= kDirectMaxRows     ? 2.8 + G * 0.07 * per_cu
                                                       : 2.6 + 0.08 * per_cu + G * (0.086 + 0.025 * per_cu);
-    const int v = wide_pick<BITS>(q.M, q.N, q.K, n_cus, lds_limit);
-    return v >= 0 && wide_estimate(v, q.M, q.N, q.K, n_cus) < narrow;
+    const int v = wide_pick<BITS>(q.M, q.N, q.K, n_cus, lds_limit, ordered);
+    return v >= 0 && wide_estimate(v, q.M, q.N, q.K, n_cus, ordered) < narrow;
 }
 
 // gate|up of a wide block with silu(gate) * up behind it: out bf16 [M, N / 2]; -1 where the projection is not the wide
@@ -426,9 +426,10 @@ int launch_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *
     const int lds_limit = st.lds_limit[dev];
     const MfmaTuning &mtu = mfma_tuning<BITS>();
     const GemvProblem q{A, B, out, s, ws, M, N, K};
-    if (mtu.engine != 7 && !(mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(q, false, st.n_cus[dev], lds_limit))) return -1;
-    const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % kWideVariants
-                                                       : wide_pick<BITS>(M, N, K, st.n_cus[dev], lds_limit);
+    if (mtu.engine != 7 && !(mtu.engine == 0 && mtu.min_width <= 0 && wide_default<BITS>(q, false, st.n_cus[dev], lds_limit, ordered)))
+        return -1;
+    const int v = mtu.engine == 7 && mtu.row_tiles > 0 ? (mtu.row_tiles - 1) % (ordered ? kOrderedVariants : kWideVariants)
+                                                       : wide_pick<BITS>(M, N, K, st.n_cus[dev], lds_limit, ordered);
     return v < 0 ? -1 : launch_wide<BITS>(v, q, OUT_BF16, 0, lds_limit, stream, silu, ordered, ask, st.n_cus[dev]);
 }
 

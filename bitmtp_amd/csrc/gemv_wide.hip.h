@@ -8,7 +8,7 @@
 // every 2.25 ns, whichever it is, two or more together one every 1.15 ns -- left shifts, byte permutations and
 // three-operand integer ones every 1.9; a matrix instruction takes 13.6.)  So
 //   * v_mfma_i32_32x32x32_i8: half the matrix instructions of the 16 x 16 form;
-//   * weights are unpacked to 64 times their value (mfma_unpack64), which needs no offset term -- the
+//   * weights are unpacked to 64 times their value (wide_unpack), which needs no offset term -- the
 //     other forms feed -2 sum(a) through the accumulator, 8 more matrix instructions per 16 x 64 x 64 --
 //     and the factor, a power of two, goes out with the division;
 //   * the accumulators start from the bits of 1.5 * 2^23, so that a sum is a float and one exact
@@ -65,10 +65,11 @@ namespace bonsai {
 constexpr int kWideXcds = 8;
 constexpr int kWideTokenGroup = 8;  // token tiles walked before the next row tile
 
-// mfma_unpack64 for two dwords at a time: one shift of 64 bits for both (left shifts run at half the rate of other instructions, and this one
-// at that of a 32-bit one; what crosses from one dword to the other is masked): 6144 x 2560 at 3001 ordered tokens 63.9 -> 62.9 us,
-// 2560 x 9728 82.0 -> 81.3; at 256 12288 x 2048 14.6 -> 14.5, 4096 x 2048 7.4 -> 7.2, 2048 x 6144 10.4 -> 10.0.  H: which two operands, and from which dwords --
-// T2 2H and 2H + 1 from the dwords of those numbers, Q1 H and H + 2 from dwords 0 and 2.
+// Weights as 64 times their value (mfma_flip), two dwords at a time: one shift of 64 bits for both (left shifts run at half the rate
+// of other instructions, and this one at that of a 32-bit one; what crosses from one dword to the other is masked): 6144 x 2560 at
+// 3001 ordered tokens 63.9 -> 62.9 us, 2560 x 9728 82.0 -> 81.3; at 256 12288 x 2048 14.6 -> 14.5, 4096 x 2048 7.4 -> 7.2,
+// 2048 x 6144 10.4 -> 10.0.  H: which two operands, and from which dwords -- T2 2H and 2H + 1 from the dwords of those numbers,
+// Q1 H and H + 2 from dwords 0 and 2.
 template <int BITS, int H, typename V>
 __device__ __forceinline__ void wide_unpack(const uint32_t (&p)[4], V (&vb)[4]) {
     const uint64_t q = BITS == 2 ? (uint64_t)p[2 * H + 1] << 32 | p[2 * H] : (uint64_t)p[2] << 32 | p[0];
@@ -99,7 +100,7 @@ struct WideShape {
     static constexpr int kBufs = kPrivate ? 1 : 2;
     static constexpr int kABytes = kTokens * 128, kBBytes = kRows * 16 * BITS;
     static constexpr int kSetBytes = kBufs * (kABytes + kBBytes);
-    static constexpr bool kDeep = !kPrivate && KS > 1 && WM * WN * KS <= 8;  // has three buffers of ordered activations where they fit
+    static constexpr bool kDeep = !kPrivate && KS > 1;  // has three buffers of ordered activations where they fit
     static constexpr int kElems = MT * NT * 16;  // results per lane
     static constexpr int kOutPitch = kRows * 2 + 16;
     static constexpr int kShare = kElems / KS;  // results per lane that a K slice finishes
@@ -183,7 +184,7 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
     uint16_t *scales = reinterpret_cast<uint16_t *>(smem);
     float2 *mult = reinterpret_cast<float2 *>(smem + (size_t)G * S::kRows * 2);
     unsigned char *work = reinterpret_cast<unsigned char *>(mult + S::kTokens);
-    // three buffers (SENT): two groups are on their way while one is multiplied
+    // three buffers (ORDERED): two groups are on their way while one is multiplied
     const int bufs = ORDERED && S::kDeep && (flags & 4) != 0 ? 3 : S::kBufs;
     unsigned char *abuf = work + set * (bufs * (S::kABytes + S::kBBytes));
     unsigned char *bbuf = abuf + bufs * S::kABytes;
@@ -209,16 +210,16 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
     constexpr int BCH = BITS;                           // 16-byte chunks of a packed row
     constexpr int BN_TASKS = S::kRows * BCH;
     constexpr int BL = (BN_TASKS + S::kSet - 1) / S::kSet;
-    // Activations in operand order need no registers on their way (a set of one wave, in program order, keeps them): whole
-    // blocks go from memory to LDS, 64 units of 16 bytes a wave and load, each lane reading the unit that belongs where it writes.
-    constexpr bool SENT = ORDERED && !S::kPrivate;
+    // Activations in operand order need no registers on their way: whole blocks go from memory to LDS, 64 units of 16 bytes a
+    // wave and load, each lane reading the unit that belongs where it writes.
+    static_assert(!ORDERED || !S::kPrivate, "sets of one wave have one buffer");
     constexpr int UL = S::kTokens * 8 / S::kSet;
     static_assert(UL * S::kSet == S::kTokens * 8 && UL >= AL && BN_TASKS % 64 == 0, "whole waves");
     uint32_t a_off[UL], b_off[BL];
 #pragma unroll
     for (int i = 0; i < UL; ++i) {
         const int task = stid + i * S::kSet;
-        a_off[i] = SENT
+        a_off[i] = ORDERED
                        ? (uint32_t)(task >> 3) * (uint32_t)K + (uint32_t)((task & 7) ^ ((task >> 4) & 7)) * 16
                        : (uint32_t)(task / QPR) * (uint32_t)K + (uint32_t)((task % QPR) * QB);
     }
@@ -249,10 +250,7 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
             const int row = task / QPR, q = task % QPR;
             u32x4 *dst = a + row * 8;
             const int x = (row >> 1) & 7;
-            if (ORDERED) {
-#pragma unroll
-                for (int u = 0; u < QW; ++u) dst[(QW * q + u) ^ x] = ar[i][u];
-            } else if (BITS == 2) {
+            if (BITS == 2) {
                 const u32x4 v = ar[i][0];
                 dst[q ^ x] = transpose4x4_bytes(v.x, v.y, v.z, v.w);
             } else {
@@ -277,7 +275,7 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
             if (BN_TASKS % S::kSet == 0 || wsub * 64 + i * S::kSet < BN_TASKS)
                 wide_load_to_lds(rB, bbuf + buf * S::kBBytes + (i * S::kSet + wsub * 64) * 16, b_off[i], (uint32_t)(g * 16 * BITS));
     };
-    if (SENT) {
+    if (ORDERED) {
         if (gb < ge) send(gb, 0);
     } else {
         load(ars[0], brs[0], gb < ge ? gb : 0);
@@ -306,7 +304,7 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
                 scales[g * S::kRows + row] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rS, (at_row(row) * G + g) * 2, 0, 0);
             }
         }
-        // (the sums come out 64 times too large, mfma_unpack64: so does what divides them)
+        // (the sums come out 64 times too large, wide_unpack: so does what divides them)
         for (int i = tid; i < S::kTokens; i += S::kThreads) {
             const float d = s[m0 + (i < mv ? i : mv - 1)] * 64.0f;
             mult[i] = make_float2(d, 1.0f / d);
@@ -332,14 +330,14 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
     v16i bias16;
 #pragma unroll
     for (int r = 0; r < 16; ++r) bias16[r] = kBias;
-    if (kPiped || SENT) asm volatile("" : "+v"(bias16));  // in registers for good: no copies in front of the products
+    if (kPiped || ORDERED) asm volatile("" : "+v"(bias16));  // in registers for good: no copies in front of the products
     if (S::kPrivate) {
         if (kAhead > 1 && gb + 1 < ge) load(ars[kAhead - 1], brs[kAhead - 1], gb + 1);
-    } else if (!SENT) {
+    } else if (!ORDERED) {
         park(ars[0], brs[0], 0);
         if (gb + 1 < ge) load(ars[0], brs[0], gb + 1);
     }
-    if (SENT) {
+    if (ORDERED) {
         wide_barrier_landed();
         if ((kPiped || (S::kDeep && bufs == 3)) && gb + 1 < ge) send(gb + 1, 1);
     } else {
@@ -350,13 +348,13 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
     const auto step = [&](int it, auto set_of) {
         constexpr int R = decltype(set_of)::value;  // register set of this group
         const int g = gb + it;
-        const int buf = S::kPrivate ? 0 : (SENT && S::kDeep ? now : it & 1);
+        const int buf = S::kPrivate ? 0 : (S::kDeep && ORDERED ? now : it & 1);
         if (S::kPrivate) {
             bonsai_wave::order_lds();  // group g - 1 is no longer read
             if (g < ge) park(ars[R], brs[R], 0);
             bonsai_wave::order_lds();
             if (g + kAhead < ge) load(ars[R], brs[R], g + kAhead);
-        } else if (SENT) {
+        } else if (ORDERED) {
             // group g is there; group g - 1 is no longer read
             if (S::kDeep && bufs == 3 && g + 1 < ge) {
                 if (it > 0) wide_barrier_landed_but<UL + (BN_TASKS % S::kSet == 0 ? BL : 0)>();
@@ -392,7 +390,7 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
                 p[0] = pp.x;
                 p[2] = pp.y;
             }
-            if (SENT) flip(p);
+            if (ORDERED) flip(p);
             w[j] = G32 ? 0.0f : scale_to_f32<SF16>(scales[g * S::kRows + (wn * NT + j) * 32 + op_row]);
             wide_unpack<BITS, 0>(p, vb[j]);
             wide_unpack<BITS, 1>(p, vb[j]);
@@ -458,7 +456,7 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
                 packed[0] = p.x;
                 packed[2] = p.y;
             }
-            if (SENT) flip(packed);
+            if (ORDERED) flip(packed);
             scale = scale_to_f32<SF16>(sc[g * S::kRows]);
         };
         const auto join = [&](int i, float scale, int from, int to) {
@@ -476,7 +474,7 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
                 if (i + 1 < MT) {
                     read_a(i + 1, P);
                 } else {
-                    if (SENT) {
+                    if (ORDERED) {
                         wide_barrier_landed();  // group g + 1 is there; group g is no longer read
                         if (g + 2 < ge) send(g + 2, P);
                     } else {
@@ -490,8 +488,8 @@ __device__ __forceinline__ void gemv_wide_tile(const int8_t *A, const uint8_t *B
                     dd[i & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[i & 1][t], vb[t], t ? dd[i & 1] : bias16, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                     if (t == 0) {
-                        if (!SENT && i == 0 && g + 1 < ge) park(ars[0], brs[0], P ^ 1);
-                        if (!SENT && i == 1 && g + 2 < ge) load(ars[0], brs[0], g + 2);
+                        if (!ORDERED && i == 0 && g + 1 < ge) park(ars[0], brs[0], P ^ 1);
+                        if (!ORDERED && i == 1 && g + 2 < ge) load(ars[0], brs[0], g + 2);
                     } else {
                         join(i ? i - 1 : MT - 1, w[i ? P : P ^ 1], t * 5 - 5, t == 3 ? 16 : t * 5);
                         if (i == MT - 1 && t > 1) {  // (operands that the products so far have taken)
@@ -658,7 +656,7 @@ using WideKernelFn = void (*)(const int8_t *, const uint8_t *, void *, const flo
                               int, int, int, int, int);
 
 struct WideVariant {
-    WideKernelFn fn[6];  // bf16 scales, fp16 scales, group sums, pairs (bf16 scales); bf16 scales and pairs on ordered activations
+    WideKernelFn fn[4];  // bf16 scales, fp16 scales, group sums, pairs (bf16 scales); on ordered activations the first and the last
     int tokens, rows, threads;
     size_t (*lds)(int K, bool deep);
     bool deep;
@@ -671,8 +669,14 @@ constexpr WideVariant wide_variant() {
     return WideVariant{{gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, false>,
                         gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, true, false, false>,
                         gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, true, false>,
-                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, true>,
-                        gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, false>,
+                        gemv_wide_kernel<BITS, WM, WN, KS, MT, NT, false, false, true>},
+                       S::kTokens, S::kRows, S::kThreads, S::lds_bytes, S::kDeep, {WM, WN, KS, MT, NT}};
+}
+
+template <int BITS, int WM, int WN, int KS, int MT, int NT>
+constexpr WideVariant wide_ordered_variant() {
+    using S = WideShape<BITS, WM, WN, KS, MT, NT>;
+    return WideVariant{{gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, false>, nullptr, nullptr,
                         gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, true>},
                        S::kTokens, S::kRows, S::kThreads, S::lds_bytes, S::kDeep, {WM, WN, KS, MT, NT}};
 }
@@ -688,13 +692,31 @@ const WideVariant &wide_kernel(int v) {
     return t[v];
 }
 
+// On ordered activations: without staging registers and instructions smaller tiles are ahead, and these five stand for all (over 123
+// sizes 0.7 % behind the best of nine in the mean, 6 % at most; the six above, by their estimates, 3.4 % and 22 %).
+enum : int { ORDERED_32x64_K4 = 0, ORDERED_128x256, ORDERED_64x64_K2, ORDERED_64x128, ORDERED_64x64_K4, kOrderedVariants };
+
+template <int BITS>
+const WideVariant &wide_kernel_ordered(int v) {
+    static const WideVariant t[kOrderedVariants] = {wide_ordered_variant<BITS, 1, 2, 4, 1, 1>(), wide_ordered_variant<BITS, 1, 8, 1, 4, 1>(),
+                                                    wide_ordered_variant<BITS, 1, 2, 2, 2, 1>(), wide_ordered_variant<BITS, 1, 4, 1, 2, 1>(),
+                                                    wide_ordered_variant<BITS, 1, 2, 4, 2, 1>()};
+    return t[v];
+}
+
 template <int BITS>
 int wide_init_device(int max_lds) {
+    const auto init = [&](const WideVariant &k) {
+        for (WideKernelFn fn : k.fn)
+            if (fn != nullptr && hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     max_lds) != hipSuccess)
+                return false;
+        return true;
+    };
     for (int v = 0; v < kWideVariants; ++v)
-        for (int k = 0; k < 6; ++k)
-            if (hipFuncSetAttribute(reinterpret_cast<const void *>(wide_kernel<BITS>(v).fn[k]),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, max_lds) != hipSuccess)
-                return 2;
+        if (!init(wide_kernel<BITS>(v))) return 2;
+    for (int v = 0; v < kOrderedVariants; ++v)
+        if (!init(wide_kernel_ordered<BITS>(v))) return 2;
     return 0;
 }
 
@@ -703,15 +725,19 @@ int wide_init_device(int max_lds) {
 // and its results.  Fitted to 17 ... 4096 tokens of 13 matrices (1024 x 1024 ... 20000 x 9728), then moved for
 // the choice between them.  Over 220 drawn blocks with weights from HBM each is off by 13-18 % rms, mostly by a
 // part that all share (9-16 % low).
-inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
+// Those on ordered activations are fitted to 123 sizes from 17 to 3500 tokens (5-11 % rms).
+inline double wide_estimate(int v, int M, int N, int K, int n_cus, bool ordered = false) {
     struct Cost {
         int tokens, rows, slices;
         double fixed, group_min, group_tile, tile;
     };
+    static constexpr Cost o[kOrderedVariants] = {{32, 64, 4, 2.83, 0.625, 0.471, 0.189}, {128, 256, 1, 1.66, 0.288, 0.943, 6.336},
+                                                 {64, 64, 2, 3.46, 0.555, 0.316, 0.847}, {64, 128, 1, 4.27, 0.483, 0.284, 0.651},
+                                                 {64, 64, 4, 1.36, 0.883, 0.884, 1.924}};
     static constexpr Cost c[kWideVariants] = {{64, 256, 1, 3.7, 0.752, 0.571, 1.47},   {64, 128, 2, 2.94, 0.882, 0.577, 1.565},
                                               {32, 64, 4, 3.27, 0.595, 0.498, 0.554},  {32, 64, 8, 1.87, 0.791, 0.889, 2.54},
                                               {64, 128, 4, 1.5, 1.25, 1.25, 3.0},      {128, 256, 1, 2.0, 0.88, 1.03, 6.0}};
-    const Cost &k = c[v];
+    const Cost &k = ordered ? o[v] : c[v];
     const int G = K / kGroup, unit = G % 4 == 0 ? 4 : 1;
     const int groups = (G / unit + k.slices - 1) / k.slices * unit;
     const long tiles = (long)((M + k.tokens - 1) / k.tokens) * ((N + k.rows - 1) / k.rows);
@@ -724,8 +750,8 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus) {
 // so that 64x128_K4 and 128x256 stop at K = 23,808, 64x256 at 32,384 and 64x128_K2 at 56,576 (160 KB of LDS), and
 // its offsets are 32-bit.
 template <int BITS>
-bool wide_fits(int v, int K, int lds_limit) {
-    const WideVariant &k = wide_kernel<BITS>(v);
+bool wide_fits(int v, int K, int lds_limit, bool ordered = false) {
+    const WideVariant &k = ordered ? wide_kernel_ordered<BITS>(v) : wide_kernel<BITS>(v);
     return k.lds(K, false) <= (size_t)lds_limit && (long)k.rows * K <= (1L << 30) && (long)k.tokens * K <= (1L << 30);
 }
 
@@ -733,11 +759,11 @@ bool wide_fits(int v, int K, int lds_limit) {
 // the best of them in the mean, within 0.8 % on nine in ten, 21 % at most (16586 x 2560 of sign weights at 89 tokens:
 // 64x128_K2 for 32x64_K4).  -1: none does.
 template <int BITS>
-int wide_pick(int M, int N, int K, int n_cus, int lds_limit) {
+int wide_pick(int M, int N, int K, int n_cus, int lds_limit, bool ordered = false) {
     int best = -1;
-    for (int v = 0; v < kWideVariants; ++v)
-        if (wide_fits<BITS>(v, K, lds_limit) &&
-            (best < 0 || wide_estimate(v, M, N, K, n_cus) < wide_estimate(best, M, N, K, n_cus)))
+    for (int v = 0; v < (ordered ? kOrderedVariants : kWideVariants); ++v)
+        if (wide_fits<BITS>(v, K, lds_limit, ordered) &&
+            (best < 0 || wide_estimate(v, M, N, K, n_cus, ordered) < wide_estimate(best, M, N, K, n_cus, ordered)))
             best = v;
     return best;
 }
@@ -746,8 +772,8 @@ int wide_pick(int M, int N, int K, int n_cus, int lds_limit) {
 template <int BITS>
 int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream, bool pairs = false,
                 bool ordered = false, bool ask = false, int n_cus = 0) {
-    const WideVariant &k = wide_kernel<BITS>(v);
-    if (!wide_fits<BITS>(v, q.K, lds_limit)) return -1;
+    const WideVariant &k = ordered ? wide_kernel_ordered<BITS>(v) : wide_kernel<BITS>(v);
+    if (!wide_fits<BITS>(v, q.K, lds_limit, ordered)) return -1;
     // pairs: N / 2 gate rows, N / 2 up rows -> silu(gate) * up, 16-byte pieces of whole rows; one resource over all of B
     if (pairs && (out_kind != OUT_BF16 || scale_kind != 0 || q.N % 16 != 0 || (reinterpret_cast<uintptr_t>(q.out) & 15) != 0 ||
                   (long)q.N * q.K * BITS / 8 > (1L << 30)))
@@ -764,7 +790,7 @@ int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int l
     // level; 4096 x 2048 (512 tiles) 8.7 -> 9.0, gate|up 12288 x 2048 (384 tiles) 16.1 -> 16.4.
     const size_t three = k.lds(q.K, true);
     const bool deep = ordered && k.deep && tm * tn <= n_cus && three <= (size_t)lds_limit;
-    const int variant = ordered ? (pairs ? 5 : 4) : (pairs ? 3 : (out_kind == OUT_G32 ? 2 : scale_kind));
+    const int variant = pairs ? 3 : (out_kind == OUT_G32 ? 2 : scale_kind);
     hipLaunchKernelGGL(k.fn[variant], dim3(per * kWideXcds, 1, 1), dim3(k.threads, 1, 1), deep ? three : k.lds(q.K, false), stream, q.A, q.B, q.out,
                        q.s, reinterpret_cast<const uint16_t *>(q.ws), q.M, q.N, q.K, out_kind == OUT_F32 ? 1 : 0, tm,
                        tn, flags | (deep ? 4 : 0));

@@ -99,7 +99,7 @@ int q1g128_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *
 /* bf16 results on bf16 scales from activations in OPERAND ORDER, the order in which the matrix cores of wide blocks take them
  * (bonsai_act_quant_ordered and bonsai_norm_quant_ordered write it): 16 activations (T2) e = 0 .. 15 of a token as the four
  * dwords {e, e + 4, e + 8, e + 12}, e = 0 .. 3; 32 (Q1) as the eight dwords {e, e + 8, e + 16, e + 24}, e = 0 .. 7.  silu: as *_gemv_silu.
- * -1, and nothing launched, where such a call is not the wide kernel's, as *_gemv_ex and *_gemv_silu choose it (then they take the
+ * -1, and nothing launched, where another kernel than the wide one is expected to be faster (*_gemv_ex and *_gemv_silu take the
  * activations in their own order).  ask: the answer (0 or -1) without the launch.  Same results as from the other order. */
 int t2g128_gemv_ordered(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K, int silu,
                         int ask, void *stream);
