@@ -1785,7 +1785,7 @@ extern "C" int bonsai_prefill_attention(const void *q, const void *k_layer, cons
                        static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(q),
                        static_cast<const uint16_t *>(k_layer), static_cast<const uint16_t *>(v_layer),
                        static_cast<uint16_t *>(out_bf16), scale * 1.44269504088896340736f, M, n_heads, n_kv, hpg,
-                       slots, base, tokens, tiles);
+                       slots, base, tokens, tiles, cu_count() / n_kv);   // (tiles a head of one workgroup a CU)
     t_prompt_attn = split ? "prefill_attn_split_kernel" : "prefill_attn_kernel";
     return hipGetLastError() == hipSuccess ? BONSAI_DECODE_OK : BONSAI_DECODE_ERR_LAUNCH;
 }

@@ -23,7 +23,9 @@
 // product), 96 so, 0.78 PFLOP/s over the slots seen.  (Half the scores beside the maximum and half beside the exponentials:
 // 97; the order of the two kinds of instructions prescribed: 103.)
 //
-// Longest rows first; the kv head is the low part of the block number, so that with eight of them an
+// Longest rows first, but the second workgroup of each CU the other way round: the longest rows' CUs get the shorter ones of that
+// batch beside them (us, all longest first -> so: 32 heads, 2048 rows 58.0 -> 54.4, 3001 level, 4096 171 -> 161; 16 heads, 3001
+// 76.7 -> 74.0, 4096 106 -> 99.6; every other batch the other way round 4096 165).  The kv head is the low part of the block number, so that with eight of them an
 // XCD's L2 holds one head's history.
 // Reference: the prompt forward's causal attention, src/bonsai_sft/gpu/model.py:996-1005 with the mask
 // of fast_generate.py:949-953.
@@ -75,6 +77,12 @@ struct Rows {
         masked_from = (base + m0 + 1) / kSlots;             // from here on some row does not see all slots
     }
 };
+
+// Which of `tiles` tiles, longest first, comes at place `i`: places batch .. 2 batch - 1 the other way round.
+__device__ __forceinline__ int turn_of(int i, int tiles, int batch) {
+    if (i < batch || i >= 2 * batch) return i;
+    return batch + (tiles < 2 * batch ? tiles : 2 * batch) - 1 - i;
+}
 
 // A lane's pair: (row, query head) number `pair` of the workgroup; pairs without a row repeat the block's last one.
 struct Pair {
@@ -199,10 +207,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t history(const uint16_t *layer,
 __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 prefill_attn_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *v_layer, uint16_t *out,
                     float scale_log2e, int M, int n_heads, int n_kv, int hpg, int slots, int base, int tokens,
-                    int tiles) {
+                    int tiles, int batch) {
     __shared__ __align__(16) unsigned char smem[kLds];
     const int kvh = (int)blockIdx.x % n_kv;
-    const Rows w(tiles - 1 - (int)blockIdx.x / n_kv, tokens, M, base);
+    const Rows w(tiles - 1 - turn_of((int)blockIdx.x / n_kv, tiles, batch), tokens, M, base);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, h = lane >> 5;
@@ -288,7 +296,7 @@ static_assert(kWaves * 64 * 64 * 4 + kWaves * 64 * 8 <= kSplitLds, "the merge re
 __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1)))
 prefill_attn_split_kernel(const uint16_t *q, const uint16_t *k_layer, const uint16_t *v_layer, uint16_t *out,
                           float scale_log2e, int M, int n_heads, int n_kv, int hpg, int slots, int base, int tokens,
-                          int tiles) {
+                          int tiles, int) {
     __shared__ __align__(16) unsigned char smem[kSplitLds];
     const int kvh = (int)blockIdx.x % n_kv;
     const Rows rows(tiles - 1 - (int)blockIdx.x / n_kv, tokens, M, base);
