@@ -177,16 +177,16 @@ __device__ __forceinline__ float block_max_f32(float v, float *scratch, int wave
     return t;
 }
 
-// ORDER: 0 as they come, 2 / 1 operand order of the T2 / Q1 matrix-core kernels (bonsai_gemv.h), which two / four neighbouring
-// lanes make between them (all of them have a vector then: K is a multiple of 128).
-template <int ORDER>
+// ORDERED: in operand order of the wide T2 kernel (bonsai_gemv.h), which two neighbouring lanes make between them (both have a
+// vector: K is a multiple of 128).
+template <bool ORDERED>
 __device__ __forceinline__ void store_q8(int8_t *qrow, int v, const float nf[8], float sval) {
     uint2 o;
     o.x = quant1(nf[0], sval) | (quant1(nf[1], sval) << 8) | (quant1(nf[2], sval) << 16) |
           (quant1(nf[3], sval) << 24);
     o.y = quant1(nf[4], sval) | (quant1(nf[5], sval) << 8) | (quant1(nf[6], sval) << 16) |
           (quant1(nf[7], sval) << 24);
-    if (ORDER == 2) {
+    if (ORDERED) {
         // vector h of a pair holds bytes 2h and 2h + 1 of each dword; the first lane stores dwords 0 and 1, the second 2 and 3
         const bool second = (v & 1) != 0;
         const uint32_t d01 = __builtin_amdgcn_perm(o.y, o.x, 0x05010400u), d23 = __builtin_amdgcn_perm(o.y, o.x, 0x07030602u);
@@ -195,21 +195,6 @@ __device__ __forceinline__ void store_q8(int8_t *qrow, int v, const float nf[8],
         const uint32_t lo = second ? other : own, hi = second ? own : other;
         o.x = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
         o.y = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
-    }
-    if (ORDER == 1) {
-        // vector b of four holds byte b of each of the eight dwords; lane b stores dwords b and b + 4
-        const uint32_t lane = (uint32_t)v & 3u, pick = lane | (lane + 4u) << 8;
-        const auto across = [&](uint32_t x) {
-            const uint32_t l0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x00, 0xf, 0xf, false);
-            const uint32_t l1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x55, 0xf, 0xf, false);
-            const uint32_t l2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xAA, 0xf, 0xf, false);
-            const uint32_t l3 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xFF, 0xf, 0xf, false);
-            return __builtin_amdgcn_perm(__builtin_amdgcn_perm(l3, l2, pick), __builtin_amdgcn_perm(l1, l0, pick), 0x05040100u);
-        };
-        uint32_t *q = reinterpret_cast<uint32_t *>(qrow) + (v >> 2) * 8 + lane;
-        q[0] = across(o.x);
-        q[4] = across(o.y);
-        return;
     }
     reinterpret_cast<uint2 *>(qrow)[v] = o;
 }
@@ -223,7 +208,7 @@ __device__ __forceinline__ void unpack8_bf16(const uint4 raw, float out[8]) {
     }
 }
 
-template <bool ADD, int VPT, int ORDER>
+template <bool ADD, int VPT, bool ORDERED>
 __global__ void __launch_bounds__(kMaxProducerThreads)
 rmsnorm_quant_kernel(const uint16_t *x, const uint16_t *residual, const uint16_t *w, float eps,
                      int geom, uint16_t *h_out, uint16_t *n_out, int8_t *q, float *s) {
@@ -311,14 +296,14 @@ rmsnorm_quant_kernel(const uint16_t *x, const uint16_t *residual, const uint16_t
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int v = tid + i * T;
-        if (v < nvec) store_q8<ORDER>(qrow, v, h[i], sval);
+        if (v < nvec) store_q8<ORDERED>(qrow, v, h[i], sval);
     }
 }
 
 // SILU: inner = bf16( fp32(bf16(silu(gate))) * up ), gate = x[m][0..F), up = x[m][F..2F); otherwise inner = x[m][0..F).
 // Latency at few rows, bytes at many: 3001 rows of 9728 take 32.7 us with the activation (3.9 TB/s of 2 x 2 + 1 bytes an
 // element) and 18.9 without it (4.6 TB/s of 2 + 1), which is why a prompt's gate|up applies it.
-template <int VPT, bool SILU, int ORDER>
+template <int VPT, bool SILU, bool ORDERED>
 __global__ void __launch_bounds__(kMaxProducerThreads)
 row_quant_kernel(const uint16_t *x, int8_t *q, float *s, int F, int T) {
     __shared__ float max_scratch[kMaxProducerWaves];
@@ -370,7 +355,7 @@ row_quant_kernel(const uint16_t *x, int8_t *q, float *s, int F, int T) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int v = tid + i * T;
-        if (v < nvec) store_q8<ORDER>(qrow, v, nf[i], sval);
+        if (v < nvec) store_q8<ORDERED>(qrow, v, nf[i], sval);
     }
 }
 
@@ -385,34 +370,34 @@ inline int producer_vpt(int nvec) {
 
 constexpr int kMaxProducerK = 8 * kMaxProducerThreads * 8;  // VPT <= 8
 
-template <bool ADD, int ORDER = 0>
+template <bool ADD, bool ORDERED = false>
 void launch_rmsnorm(const uint16_t *x, const uint16_t *r, const uint16_t *w, float eps,
                     uint16_t *h_out, uint16_t *n_out, int8_t *q, float *s, int M, int K,
                     hipStream_t st) {
     const int nvec = K / 8;
     const dim3 grid(M), block(producer_threads(nvec));
     switch (producer_vpt(nvec)) {
-        case 1: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 1, ORDER>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
-        case 2: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 2, ORDER>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
-        case 4: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 4, ORDER>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
-        default: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 8, ORDER>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
+        case 1: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 1, ORDERED>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
+        case 2: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 2, ORDERED>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
+        case 4: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 4, ORDERED>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
+        default: hipLaunchKernelGGL((rmsnorm_quant_kernel<ADD, 8, ORDERED>), grid, block, 0, st, x, r, w, eps, K | (int)block.x << 20, h_out, n_out, q, s); break;
     }
 }
 
 // bf16 rows: read once and kept in registers, as many threads as vectors where a workgroup has them
-template <int ORDER>
+template <bool ORDERED>
 void launch_row_quant(const void *x, int8_t *q, float *s, int M, int K, hipStream_t st) {
     const dim3 grid(M), block(producer_threads(K / 8));
     const uint16_t *row = reinterpret_cast<const uint16_t *>(x);
     switch (producer_vpt(K / 8)) {
-        case 1: hipLaunchKernelGGL((row_quant_kernel<1, false, ORDER>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
-        case 2: hipLaunchKernelGGL((row_quant_kernel<2, false, ORDER>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
-        case 4: hipLaunchKernelGGL((row_quant_kernel<4, false, ORDER>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
-        default: hipLaunchKernelGGL((row_quant_kernel<8, false, ORDER>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+        case 1: hipLaunchKernelGGL((row_quant_kernel<1, false, ORDERED>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+        case 2: hipLaunchKernelGGL((row_quant_kernel<2, false, ORDERED>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+        case 4: hipLaunchKernelGGL((row_quant_kernel<4, false, ORDERED>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
+        default: hipLaunchKernelGGL((row_quant_kernel<8, false, ORDERED>), grid, block, 0, st, row, q, s, K, (int)block.x); break;
     }
 }
 
-bool order_ok(int M, int K, int bits) { return M >= 1 && K >= 128 && K % 128 == 0 && K <= kMaxProducerK && (bits == 1 || bits == 2); }
+bool order_ok(int M, int K) { return M >= 1 && K >= 128 && K % 128 == 0 && K <= kMaxProducerK; }
 
 }  // namespace
 
@@ -427,7 +412,7 @@ extern "C" int bonsai_act_quant_int8(const void *x, int x_kind, int8_t *q, float
                 hipLaunchKernelGGL(act_quant_kernel<BONSAI_X_BF16>, dim3(M), dim3(kThreads), 0, st, x, q, s, K);
                 break;
             }
-            launch_row_quant<0>(x, q, s, M, K, st);
+            launch_row_quant<false>(x, q, s, M, K, st);
             break;
         }
         case BONSAI_X_F16:
@@ -494,27 +479,26 @@ extern "C" int bonsai_silu_mul_quant_int8(const void *gate_up, int8_t *q, float 
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t *gu = reinterpret_cast<const uint16_t *>(gate_up);
     switch (producer_vpt(nvec)) {
-        case 1: hipLaunchKernelGGL((row_quant_kernel<1, true, 0>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
-        case 2: hipLaunchKernelGGL((row_quant_kernel<2, true, 0>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
-        case 4: hipLaunchKernelGGL((row_quant_kernel<4, true, 0>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
-        default: hipLaunchKernelGGL((row_quant_kernel<8, true, 0>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        case 1: hipLaunchKernelGGL((row_quant_kernel<1, true, false>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        case 2: hipLaunchKernelGGL((row_quant_kernel<2, true, false>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        case 4: hipLaunchKernelGGL((row_quant_kernel<4, true, false>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
+        default: hipLaunchKernelGGL((row_quant_kernel<8, true, false>), grid, block, 0, st, gu, q, s, F, (int)block.x); break;
     }
     return hipGetLastError() == hipSuccess ? BONSAI_OK : BONSAI_ERR_LAUNCH;
 }
 
 extern "C" int bonsai_norm_quant_ordered(const void *x, const void *residual, const void *w, float eps, void *h_out, int8_t *q,
-                                         float *s, int M, int K, int bits, void *stream) {
+                                         float *s, int M, int K, void *stream) {
     if (x == nullptr || w == nullptr || q == nullptr || s == nullptr || (residual == nullptr) != (h_out == nullptr)) return BONSAI_ERR_ARG;
-    if (!order_ok(M, K, bits)) return BONSAI_ERR_ARG;
-    const auto launch = residual != nullptr ? (bits == 2 ? launch_rmsnorm<true, 2> : launch_rmsnorm<true, 1>)
-                                            : (bits == 2 ? launch_rmsnorm<false, 2> : launch_rmsnorm<false, 1>);
+    if (!order_ok(M, K)) return BONSAI_ERR_ARG;
+    const auto launch = residual != nullptr ? launch_rmsnorm<true, true> : launch_rmsnorm<false, true>;
     launch(reinterpret_cast<const uint16_t *>(x), reinterpret_cast<const uint16_t *>(residual), reinterpret_cast<const uint16_t *>(w), eps,
            reinterpret_cast<uint16_t *>(h_out), nullptr, q, s, M, K, static_cast<hipStream_t>(stream));
     return hipGetLastError() == hipSuccess ? BONSAI_OK : BONSAI_ERR_LAUNCH;
 }
 
-extern "C" int bonsai_act_quant_ordered(const void *x, int8_t *q, float *s, int M, int K, int bits, void *stream) {
-    if (x == nullptr || q == nullptr || s == nullptr || !order_ok(M, K, bits)) return BONSAI_ERR_ARG;
-    (bits == 2 ? launch_row_quant<2> : launch_row_quant<1>)(x, q, s, M, K, static_cast<hipStream_t>(stream));
+extern "C" int bonsai_act_quant_ordered(const void *x, int8_t *q, float *s, int M, int K, void *stream) {
+    if (x == nullptr || q == nullptr || s == nullptr || !order_ok(M, K)) return BONSAI_ERR_ARG;
+    launch_row_quant<true>(x, q, s, M, K, static_cast<hipStream_t>(stream));
     return hipGetLastError() == hipSuccess ? BONSAI_OK : BONSAI_ERR_LAUNCH;
 }

@@ -640,10 +640,10 @@ gemv_wide_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, c
     gemv_wide_tile<BITS, WM, WN, KS, MT, NT, SF16, G32, PAIRS, false>(A, B, out, s, ws, M, N, K, out_f32, tiles_m, tiles_n, flags);
 }
 
-// (six waves a SIMD where a wave has one tile of T2: three workgroups a CU.  4096 x 2048 at 256 tokens level, 6144 x 2560 at 3001
+// (six waves a SIMD where a wave has one tile: three workgroups a CU.  4096 x 2048 at 256 tokens level, 6144 x 2560 at 3001
 // 117 -> 99 us.  In the kernel above, with its staging registers, that spills: 8.1 -> 9.1.)
 template <int BITS, int WM, int WN, int KS, int MT, int NT, bool PAIRS>
-__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : (MT * NT == 1 && BITS == 2 ? 6 : 4))))
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(MT * NT >= 4 || WM * WN == 1 ? 2 : (MT * NT == 1 ? 6 : 4))))
 gemv_wide_ordered_kernel(const int8_t *A, const uint8_t *B, void *out, const float *s, const uint16_t *ws, int M,
                          int N, int K, int out_f32, int tiles_m, int tiles_n, int flags) {
     gemv_wide_tile<BITS, WM, WN, KS, MT, NT, false, false, PAIRS, true>(A, B, out, s, ws, M, N, K, out_f32, tiles_m, tiles_n, flags);
@@ -673,11 +673,11 @@ constexpr WideVariant wide_variant() {
                        S::kTokens, S::kRows, S::kThreads, S::lds_bytes, S::kDeep, {WM, WN, KS, MT, NT}};
 }
 
-template <int BITS, int WM, int WN, int KS, int MT, int NT>
+template <int WM, int WN, int KS, int MT, int NT>
 constexpr WideVariant wide_ordered_variant() {
-    using S = WideShape<BITS, WM, WN, KS, MT, NT>;
-    return WideVariant{{gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, false>, nullptr, nullptr,
-                        gemv_wide_ordered_kernel<BITS, WM, WN, KS, MT, NT, true>},
+    using S = WideShape<2, WM, WN, KS, MT, NT>;
+    return WideVariant{{gemv_wide_ordered_kernel<2, WM, WN, KS, MT, NT, false>, nullptr, nullptr,
+                        gemv_wide_ordered_kernel<2, WM, WN, KS, MT, NT, true>},
                        S::kTokens, S::kRows, S::kThreads, S::lds_bytes, S::kDeep, {WM, WN, KS, MT, NT}};
 }
 
@@ -692,16 +692,22 @@ const WideVariant &wide_kernel(int v) {
     return t[v];
 }
 
-// On ordered activations: without staging registers and instructions smaller tiles are ahead, and these five stand for all (over 123
+// On ordered activations (T2 alone: half the weight bytes leave Q1 little to gain, 0.3 % over 131 sizes; T2 9 %): without staging registers and instructions smaller tiles are ahead, and these five stand for all (over 123
 // sizes 0.7 % behind the best of nine in the mean, 6 % at most; the six above, by their estimates, 3.4 % and 22 %).
 enum : int { ORDERED_32x64_K4 = 0, ORDERED_128x256, ORDERED_64x64_K2, ORDERED_64x128, ORDERED_64x64_K4, kOrderedVariants };
 
-template <int BITS>
-const WideVariant &wide_kernel_ordered(int v) {
-    static const WideVariant t[kOrderedVariants] = {wide_ordered_variant<BITS, 1, 2, 4, 1, 1>(), wide_ordered_variant<BITS, 1, 8, 1, 4, 1>(),
-                                                    wide_ordered_variant<BITS, 1, 2, 2, 2, 1>(), wide_ordered_variant<BITS, 1, 4, 1, 2, 1>(),
-                                                    wide_ordered_variant<BITS, 1, 2, 4, 2, 1>()};
+inline const WideVariant &wide_kernel_ordered(int v) {
+    static const WideVariant t[kOrderedVariants] = {wide_ordered_variant<1, 2, 4, 1, 1>(), wide_ordered_variant<1, 8, 1, 4, 1>(),
+                                                    wide_ordered_variant<1, 2, 2, 2, 1>(), wide_ordered_variant<1, 4, 1, 2, 1>(),
+                                                    wide_ordered_variant<1, 2, 4, 2, 1>()};
     return t[v];
+}
+
+template <int BITS>
+const WideVariant &wide_of(int v, bool ordered) {
+    if constexpr (BITS == 2)
+        if (ordered) return wide_kernel_ordered(v);
+    return wide_kernel<BITS>(v);
 }
 
 template <int BITS>
@@ -715,8 +721,9 @@ int wide_init_device(int max_lds) {
     };
     for (int v = 0; v < kWideVariants; ++v)
         if (!init(wide_kernel<BITS>(v))) return 2;
-    for (int v = 0; v < kOrderedVariants; ++v)
-        if (!init(wide_kernel_ordered<BITS>(v))) return 2;
+    if constexpr (BITS == 2)
+        for (int v = 0; v < kOrderedVariants; ++v)
+            if (!init(wide_kernel_ordered(v))) return 2;
     return 0;
 }
 
@@ -751,7 +758,7 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus, bool ordered 
 // its offsets are 32-bit.
 template <int BITS>
 bool wide_fits(int v, int K, int lds_limit, bool ordered = false) {
-    const WideVariant &k = ordered ? wide_kernel_ordered<BITS>(v) : wide_kernel<BITS>(v);
+    const WideVariant &k = wide_of<BITS>(v, ordered);
     return k.lds(K, false) <= (size_t)lds_limit && (long)k.rows * K <= (1L << 30) && (long)k.tokens * K <= (1L << 30);
 }
 
@@ -772,7 +779,7 @@ int wide_pick(int M, int N, int K, int n_cus, int lds_limit, bool ordered = fals
 template <int BITS>
 int launch_wide(int v, const GemvProblem &q, int out_kind, int scale_kind, int lds_limit, hipStream_t stream, bool pairs = false,
                 bool ordered = false, bool ask = false, int n_cus = 0) {
-    const WideVariant &k = ordered ? wide_kernel_ordered<BITS>(v) : wide_kernel<BITS>(v);
+    const WideVariant &k = wide_of<BITS>(v, ordered);
     if (!wide_fits<BITS>(v, q.K, lds_limit, ordered)) return -1;
     // pairs: N / 2 gate rows, N / 2 up rows -> silu(gate) * up, 16-byte pieces of whole rows; one resource over all of B
     if (pairs && (out_kind != OUT_BF16 || scale_kind != 0 || q.N % 16 != 0 || (reinterpret_cast<uintptr_t>(q.out) & 15) != 0 ||

@@ -342,12 +342,14 @@ PyObject *prefill_layers(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         char *h[2] = {b[0], b[1]};
         char *a_q = b[2], *a_s = b[3], *xqkv = b[4], *q = b[5], *attn = b[6], *o_q = b[7], *o_s = b[8], *proj = b[9],
              *gu = b[10], *i_q = b[11], *i_s = b[12];
-        // activations in operand order where the wide kernel takes them so (what is asked is what is launched later)
-        const auto ordered = bits == 2 ? t2g128_gemv_ordered : q1g128_gemv_ordered;
+        // T2: activations in operand order where the wide kernel takes them so (what is asked is what is launched later)
         const auto wide = [&](char *a, char *s, void *wq, void *ws, char *out, int n, int k, bool silu, bool ask) {
-            return ordered(reinterpret_cast<const int8_t *>(a), static_cast<const uint8_t *>(wq), out,
-                           reinterpret_cast<const float *>(s), ws, M, n, k, silu, ask, st);
+            return t2g128_gemv_ordered(reinterpret_cast<const int8_t *>(a), static_cast<const uint8_t *>(wq), out,
+                                       reinterpret_cast<const float *>(s), ws, M, n, k, silu, ask, st);
         };
+        struct {
+            bool known, qkv, o, pairs, down;
+        } takes = {};
         const auto i8 = [](char *p) { return reinterpret_cast<int8_t *>(p); };
         const auto f32 = [](char *p) { return reinterpret_cast<float *>(p); };
         for (int l = 0; l < n_layers && rc == 0; ++l) {
@@ -360,10 +362,20 @@ PyObject *prefill_layers(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             if (rc != 0) what = name; \
         }                         \
     } while (0)
-            const bool qkv_wide = wide(a_q, a_s, x[0], x[1], xqkv, qkv, dim, false, true) == 0;
-            if (qkv_wide) {
+            // the answers depend on sizes and alignment: those of one aligned layer are those of all (112 asked for in
+            // front of 280 launches cost a short prompt, which waits for the host, 1.5 %)
+            uintptr_t low = 0;
+            for (int i = 0; i < 8; ++i) low |= reinterpret_cast<uintptr_t>(x[i]) & 15;
+            if (bits == 2 && (low != 0 || !takes.known)) {
+                takes.qkv = wide(a_q, a_s, x[0], x[1], xqkv, qkv, dim, false, true) == 0;
+                takes.o = wide(o_q, o_s, x[2], x[3], proj, dim, q_dim, false, true) == 0;
+                takes.pairs = wide(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim, true, true) == 0;
+                takes.down = takes.pairs && wide(i_q, i_s, x[6], x[7], proj, dim, ffn, false, true) == 0;
+                takes.known = low == 0;
+            }
+            if (takes.qkv) {
                 STEP("norm", bonsai_norm_quant_ordered(l == 0 ? h[0] : proj, l == 0 ? nullptr : h[cur], x[8], eps,
-                                                       l == 0 ? nullptr : h[cur ^ 1], i8(a_q), f32(a_s), M, dim, bits, st));
+                                                       l == 0 ? nullptr : h[cur ^ 1], i8(a_q), f32(a_s), M, dim, st));
                 STEP("q|k|v", wide(a_q, a_s, x[0], x[1], xqkv, qkv, dim, false, false));
             } else {
                 if (l == 0)
@@ -377,32 +389,39 @@ PyObject *prefill_layers(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
                                                       reinterpret_cast<const int32_t *>(b[13]), q, kl, vl, M, nh, nkv,
                                                       slots, base, max_pos, st));
             STEP("attention", bonsai_prefill_attention(q, kl, vl, attn, scale, M, nh, nkv, slots, base, st));
-            if (wide(o_q, o_s, x[2], x[3], proj, dim, q_dim, false, true) == 0) {
-                STEP("quantiser", bonsai_act_quant_ordered(attn, i8(o_q), f32(o_s), M, q_dim, bits, st));
+            if (takes.o) {
+                STEP("quantiser", bonsai_act_quant_ordered(attn, i8(o_q), f32(o_s), M, q_dim, st));
                 STEP("o", wide(o_q, o_s, x[2], x[3], proj, dim, q_dim, false, false));
             } else {
                 STEP("quantiser", bonsai_act_quant_int8(attn, BONSAI_X_BF16, i8(o_q), f32(o_s), M, q_dim, st));
                 STEP("o", project(o_q, o_s, x[2], x[3], proj, dim, q_dim));
             }
-            const bool pairs_wide = wide(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim, true, true) == 0;
-            const bool down_wide = pairs_wide && wide(i_q, i_s, x[6], x[7], proj, dim, ffn, false, true) == 0;
-            if (pairs_wide)
-                STEP("norm", bonsai_norm_quant_ordered(h[cur], proj, x[9], eps, h[cur ^ 1], i8(a_q), f32(a_s), M, dim, bits, st));
+            if (takes.pairs)
+                STEP("norm", bonsai_norm_quant_ordered(h[cur], proj, x[9], eps, h[cur ^ 1], i8(a_q), f32(a_s), M, dim, st));
             else
                 STEP("norm", bonsai_add_rmsnorm_quant_int8(h[cur], proj, x[9], eps, h[cur ^ 1], i8(a_q), f32(a_s), M, dim, st));
             cur ^= 1;
             // silu(gate) * up leaves with the projection where the wide kernel takes it: half the bytes
-            if (pairs_wide) {
+            if (takes.pairs) {
                 STEP("gate|up", wide(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim, true, false));
-                if (down_wide)
-                    STEP("quantiser", bonsai_act_quant_ordered(gu, i8(i_q), f32(i_s), M, ffn, bits, st));
+                if (takes.down)
+                    STEP("quantiser", bonsai_act_quant_ordered(gu, i8(i_q), f32(i_s), M, ffn, st));
                 else
                     STEP("quantiser", bonsai_act_quant_int8(gu, BONSAI_X_BF16, i8(i_q), f32(i_s), M, ffn, st));
-            } else {
-                STEP("gate|up", project(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim));
-                STEP("silu", bonsai_silu_mul_quant_int8(gu, i8(i_q), f32(i_s), M, ffn, st));
+            } else if (rc == 0) {
+                rc = (bits == 2 ? t2g128_gemv_silu : q1g128_gemv_silu)(i8(a_q), static_cast<const uint8_t *>(x[4]), gu, f32(a_s), x[5], M,
+                                                                       2 * ffn, dim, st);
+                if (rc == 0) {
+                    STEP("quantiser", bonsai_act_quant_int8(gu, BONSAI_X_BF16, i8(i_q), f32(i_s), M, ffn, st));
+                } else if (rc == -1) {
+                    rc = 0;
+                    STEP("gate|up", project(a_q, a_s, x[4], x[5], gu, 2 * ffn, dim));
+                    STEP("silu", bonsai_silu_mul_quant_int8(gu, i8(i_q), f32(i_s), M, ffn, st));
+                } else {
+                    what = "gate|up";
+                }
             }
-            if (down_wide)
+            if (takes.down)
                 STEP("down", wide(i_q, i_s, x[6], x[7], proj, dim, ffn, false, false));
             else
                 STEP("down", project(i_q, i_s, x[6], x[7], proj, dim, ffn));

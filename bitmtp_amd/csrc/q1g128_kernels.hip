@@ -129,11 +129,6 @@ int q1g128_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *
     return launch_gemv_silu<1>(A, B, out, s, ws, M, N, K, static_cast<hipStream_t>(stream));
 }
 
-int q1g128_gemv_ordered(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K,
-                        int silu, int ask, void *stream) {
-    return launch_gemv_silu<1>(A, B, out, s, ws, M, N, K, static_cast<hipStream_t>(stream), silu != 0, true, ask != 0);
-}
-
 int q1g128_gemv_ex(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws,
                    int M, int N, int K, int out_kind, int scale_kind, void *stream) {
     return launch_gemv<1>(A, B, out, s, ws, M, N, K, out_kind, scale_kind,

@@ -1,4 +1,4 @@
-"""Activations in operand order (bonsai_*_quant_ordered, *_gemv_ordered): the quantisers' bytes are those of the other order, moved; the
+"""Activations in operand order (bonsai_*_quant_ordered, t2g128_gemv_ordered): the quantisers' bytes are those of the other order, moved; the
 products are the same bits, on every tile, and what the wide kernel does not take is refused.  Sizes sit on the edges of tiles, slices and
 scale groups."""
 import ctypes
@@ -13,56 +13,51 @@ DEV = "cuda:0"
 p = lambda t: ctypes.c_void_p(0 if t is None else t.data_ptr())   # noqa: E731
 
 
-def _ordered(q, bits):
+def _ordered(q):
     m, k = q.shape
-    return (q.view(m, k // 16, 4, 4) if bits == 2 else q.view(m, k // 32, 4, 8)).transpose(2, 3).reshape(m, k).contiguous()
+    return q.view(m, k // 16, 4, 4).transpose(2, 3).reshape(m, k).contiguous()
 
 
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-@pytest.mark.parametrize("bits", [2, 1])
 @pytest.mark.parametrize("m,k", [(1, 128), (3, 384), (5, 2048), (2, 8192), (2, 8320), (1, 9728), (1, 40960), (1, 65536)])
-def test_quantisers(m, k, bits):
+def test_quantisers(m, k):
     gen = torch.Generator(device=DEV).manual_seed(k + m)
     x, r = ((torch.randn(m, k, generator=gen, device=DEV) * 3).to(torch.bfloat16) for _ in range(2))
     w = (1 + 0.1 * torch.randn(k, generator=gen, device=DEV)).to(torch.bfloat16)
     lib = ops.actq_lib()
     q, s, h = torch.empty(m, k, dtype=torch.int8, device=DEV), torch.empty(m, device=DEV), torch.empty_like(x)
     eps = ctypes.c_float(1e-6)
-    assert lib.bonsai_act_quant_ordered(p(x), p(q), p(s), m, k, bits, _stream()) == 0
+    assert lib.bonsai_act_quant_ordered(p(x), p(q), p(s), m, k, _stream()) == 0
     want, scale = ops.quant_input(x)
-    assert torch.equal(q, _ordered(want, bits)) and torch.equal(s.view(-1), scale.view(-1))
-    assert lib.bonsai_norm_quant_ordered(p(x), None, p(w), eps, None, p(q), p(s), m, k, bits, _stream()) == 0
+    assert torch.equal(q, _ordered(want)) and torch.equal(s.view(-1), scale.view(-1))
+    assert lib.bonsai_norm_quant_ordered(p(x), None, p(w), eps, None, p(q), p(s), m, k, _stream()) == 0
     want, scale = ops.fused_norm_quant(x, w, 1e-6)
-    assert torch.equal(q, _ordered(want, bits)) and torch.equal(s.view(-1), scale.view(-1))
-    assert lib.bonsai_norm_quant_ordered(p(x), p(r), p(w), eps, p(h), p(q), p(s), m, k, bits, _stream()) == 0
+    assert torch.equal(q, _ordered(want)) and torch.equal(s.view(-1), scale.view(-1))
+    assert lib.bonsai_norm_quant_ordered(p(x), p(r), p(w), eps, p(h), p(q), p(s), m, k, _stream()) == 0
     rows, want, scale = ops.fused_add_norm_quant(x, r, w, 1e-6)
-    assert torch.equal(h, rows) and torch.equal(q, _ordered(want, bits)) and torch.equal(s.view(-1), scale.view(-1))
-    for rc in (lib.bonsai_act_quant_ordered(p(x), p(q), p(s), m, k - 64, bits, _stream()),
-               lib.bonsai_act_quant_ordered(p(x), p(q), p(s), m, k, 3, _stream()),
-               lib.bonsai_norm_quant_ordered(p(x), p(r), p(w), eps, None, p(q), p(s), m, k, bits, _stream())):
+    assert torch.equal(h, rows) and torch.equal(q, _ordered(want)) and torch.equal(s.view(-1), scale.view(-1))
+    for rc in (lib.bonsai_act_quant_ordered(p(x), p(q), p(s), m, k - 64, _stream()),
+               lib.bonsai_norm_quant_ordered(p(x), p(r), p(w), eps, None, p(q), p(s), m, k, _stream())):
         assert rc != 0
 
 
-@pytest.mark.parametrize("bits", [2, 1])
 @pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 128), (17, 32, 256), (33, 80, 384), (64, 256, 512), (129, 272, 640), (128, 128, 2048),
                                    (257, 1008, 1152), (40, 144, 9728)])
-def test_products(m, n, k, variant, bits):
-    print(f"[case] ordered variant {variant} bits {bits} {m}x{n}x{k}", flush=True)
+def test_products(m, n, k, variant):
+    print(f"[case] ordered variant {variant} {m}x{n}x{k}", flush=True)
     gen = torch.Generator(device=DEV).manual_seed(m + n + k)
     a = torch.randint(-128, 128, (m, k), generator=gen, device=DEV, dtype=torch.int8)
-    b = torch.randint(-128, 128, (n, k * bits // 8), generator=gen, device=DEV, dtype=torch.int8)
+    b = torch.randint(-128, 128, (n, k // 4), generator=gen, device=DEV, dtype=torch.int8)
     ws = torch.exp(torch.randn(n, k // 128, generator=gen, device=DEV) * 0.5 - 4).to(torch.bfloat16)
     s = torch.rand(m, generator=gen, device=DEV) * 40 + 1
     s[0] = 1e-30   # (infinite results)
-    lib = ops.t2_lib() if bits == 2 else ops.q1_lib()
-    name = "t2g128" if bits == 2 else "q1g128"
-    tune, plain = getattr(lib, name + "_set_mfma_tuning"), getattr(lib, name + "_gemv_ex")
-    silu, ordered = getattr(lib, name + "_gemv_silu"), getattr(lib, name + "_gemv_ordered")
-    order = _ordered(a, bits)
+    lib = ops.t2_lib()
+    tune, plain, silu, ordered = (getattr(lib, "t2g128_" + f) for f in ("set_mfma_tuning", "gemv_ex", "gemv_silu", "gemv_ordered"))
+    order = _ordered(a)
     tune(0, variant, 0, 0, 7 if variant else 0)
     try:
         for pairs in (0, 1):
@@ -83,7 +78,7 @@ def test_products(m, n, k, variant, bits):
             assert ordered(p(order), *args, pairs, 0, _stream()) == (0 if wide else -1)
             assert wide or variant == 0
             if wide:
-                assert ops.last_kernel(bits).startswith("gemv_wide_ordered_kernel<")
+                assert ops.last_kernel(2).startswith("gemv_wide_ordered_kernel<")
                 if want is None:
                     torch.testing.assert_close(got[1:].float(), (torch.nn.functional.silu(gate) * up)[1:].float(), rtol=2 ** -6, atol=1e-3)
                 else:
