@@ -28,8 +28,10 @@
 //
 // Activations that a quantiser has left in operand order (ORDERED: a prompt's) go from memory to LDS without passing
 // registers, and nothing is transposed here: once per weight row tile it was, and is once now, by the quantiser.
-// From -> to operand order, us at 3001 tokens: 6144 x 2560 72 -> 65, 19456 x 2560 197 -> 180, 2560 x 4096 42 -> 40, 2560 x 9728
-// 88 -> 83; at 256: 12288 x 2048 16.1 -> 14.3, 4096 x 2048 8.6 -> 7.6, 2048 x 6144 12.0 -> 10.5, 2048 x 2048 6.3 -> 5.7.
+// From -> to operand order on the same tile, us at 3001 tokens: 6144 x 2560 72 -> 65, 19456 x 2560 197 -> 180, 2560 x 4096 42 -> 40,
+// 2560 x 9728 88 -> 83; at 256: 12288 x 2048 16.1 -> 14.3, 4096 x 2048 8.6 -> 7.6, 2048 x 6144 12.0 -> 10.5, 2048 x 2048 6.3 -> 5.7.
+// With its own tiles, within a prompt: at 3001 tokens 71.6 -> 59.5, with SiLU 198 -> 176.5 (1.69 POP/s), 46.2 -> 38.7, 98 -> 80 (1.87);
+// at 256 with SiLU 18.1 -> 15.3, 10.1 -> 8.6, 13.8 -> 12.6, 7.1 -> 6.8.
 //
 // Per group a set stages 128 bytes of K for its tokens (4 x 4 byte transposes: operand order, see
 // gemv_core.h; 16-byte units XORed with half the row number, so that a ds_read_b128 of 16 rows meets
