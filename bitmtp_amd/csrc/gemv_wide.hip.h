@@ -694,14 +694,15 @@ const WideVariant &wide_kernel(int v) {
     return t[v];
 }
 
-// On ordered activations (T2 alone: half the weight bytes leave Q1 little to gain, 0.3 % over 131 sizes; T2 9 %): without staging registers and instructions smaller tiles are ahead, and these five stand for all (over 123
-// sizes 0.7 % behind the best of nine in the mean, 6 % at most; the six above, by their estimates, 3.4 % and 22 %).
-enum : int { ORDERED_32x64_K4 = 0, ORDERED_128x256, ORDERED_64x64_K2, ORDERED_64x128, ORDERED_64x64_K4, kOrderedVariants };
+// On ordered activations (T2 alone: half the weight bytes leave Q1 little to gain, 0.3 % over 131 sizes; T2 9 %): without staging
+// registers and instructions smaller tiles are ahead, and these six stand for all (over 267 sizes 0.6 % behind the best of
+// nine in the mean, 10 % at most; the six above, by their estimates, 3.4 % and 22 %; without the last one 1.2 % and 20 %).
+enum : int { ORDERED_32x64_K4 = 0, ORDERED_128x256, ORDERED_64x64_K2, ORDERED_64x128, ORDERED_64x64_K4, ORDERED_64x128_K4, kOrderedVariants };
 
 inline const WideVariant &wide_kernel_ordered(int v) {
     static const WideVariant t[kOrderedVariants] = {wide_ordered_variant<1, 2, 4, 1, 1>(), wide_ordered_variant<1, 8, 1, 4, 1>(),
                                                     wide_ordered_variant<1, 2, 2, 2, 1>(), wide_ordered_variant<1, 4, 1, 2, 1>(),
-                                                    wide_ordered_variant<1, 2, 4, 2, 1>()};
+                                                    wide_ordered_variant<1, 2, 4, 2, 1>(), wide_ordered_variant<1, 4, 4, 2, 1>()};
     return t[v];
 }
 
@@ -734,15 +735,16 @@ int wide_init_device(int max_lds) {
 // and its results.  Fitted to 17 ... 4096 tokens of 13 matrices (1024 x 1024 ... 20000 x 9728), then moved for
 // the choice between them.  Over 220 drawn blocks with weights from HBM each is off by 13-18 % rms, mostly by a
 // part that all share (9-16 % low).
-// Those on ordered activations are fitted to 123 sizes from 17 to 3500 tokens (5-11 % rms).
+// Those on ordered activations are fitted to 267 sizes from 17 to 3500 tokens and moved, by a tenth at most, for the choice (7-8 %
+// rms where they are near the best).
 inline double wide_estimate(int v, int M, int N, int K, int n_cus, bool ordered = false) {
     struct Cost {
         int tokens, rows, slices;
         double fixed, group_min, group_tile, tile;
     };
-    static constexpr Cost o[kOrderedVariants] = {{32, 64, 4, 2.83, 0.625, 0.471, 0.189}, {128, 256, 1, 1.66, 0.288, 0.943, 6.336},
-                                                 {64, 64, 2, 3.46, 0.555, 0.316, 0.847}, {64, 128, 1, 4.27, 0.483, 0.284, 0.651},
-                                                 {64, 64, 4, 1.36, 0.883, 0.884, 1.924}};
+    static constexpr Cost o[kOrderedVariants] = {{32, 64, 4, 2.993, 0.581, 0.424, 0.468}, {128, 256, 1, 2.101, 0.737, 0.846, 7.022},
+                                                 {64, 64, 2, 3.2, 0.539, 0.314, 0.827},   {64, 128, 1, 5.267, 0.422, 0.263, 0.599},
+                                                 {64, 64, 4, 1.752, 0.784, 0.833, 1.975}, {64, 128, 4, 1.026, 1.161, 1.141, 3.872}};
     static constexpr Cost c[kWideVariants] = {{64, 256, 1, 3.7, 0.752, 0.571, 1.47},   {64, 128, 2, 2.94, 0.882, 0.577, 1.565},
                                               {32, 64, 4, 3.27, 0.595, 0.498, 0.554},  {32, 64, 8, 1.87, 0.791, 0.889, 2.54},
                                               {64, 128, 4, 1.5, 1.25, 1.25, 3.0},      {128, 256, 1, 2.0, 0.88, 1.03, 6.0}};

@@ -44,7 +44,7 @@ def test_quantisers(m, k):
         assert rc != 0
 
 
-@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 128), (17, 32, 256), (33, 80, 384), (64, 256, 512), (129, 272, 640), (128, 128, 2048),
                                    (257, 1008, 1152), (40, 144, 9728)])
 def test_products(m, n, k, variant):
