@@ -454,7 +454,8 @@ class GraphAtlas:
             g.io.uploaded.synchronize()
         g.io.step_in_host.numpy()[:] = inputs
         owed = self._owed
-        if separate or g.role == "ar" or owed is None or owed[0] != g.sigma:
+        # (only the first launch of a captured block reads the words behind the inputs)
+        if separate or g.graph is None or g.role == "ar" or owed is None or owed[0] != g.sigma:
             self.settle()
             g.io.inputs_host.numpy()[-1] = 0
         else:

@@ -161,3 +161,19 @@ def test_results_in_pinned_memory_are_those_on_the_device(width, role):
         assert np.array_equal(conf.view(np.int32), out[width + 2: width + 2 + rows])
         if role == "draft":
             assert np.array_equal(atlas._drafted[:rows].cpu().numpy(), out[:rows])
+
+
+@pytest.mark.parametrize("loop,kw", [("speculative", {}), ("hybrid", {"threshold": 2.0}), ("hybrid", {"threshold": 2.0, "hybrid_m": 9})])
+def test_loops_without_graphs_keep_what_was_verified(loop, kw, monkeypatch):
+    """Verifications that accept drafts: the tokens and the history of the loop whose steps are graphs."""
+    from bitmtp_amd import generate
+    monkeypatch.setattr(generate, "verify_accept", lambda draft, verify, D: int(draft[0]) % 4)   # (random weights agree on few)
+    model, prompt, results = _model(2, 1024, 512, 8, 4), list(range(3, 33)), []
+    from bitmtp_amd.runtime import GraphAtlas
+    for use_graphs in (True, False):
+        atlas = GraphAtlas(model, segment_ladder=(64, 256), use_graphs=use_graphs)
+        out, st = getattr(generate, loop + "_generate")(atlas, prompt, max_gen_len=60, **kw)
+        results.append((out, st["accepted_drafts"], _history(atlas, len(prompt) + len(out) - 10)))
+        assert st["accepted_drafts"] > 9
+    assert results[0][:2] == results[1][:2]
+    assert torch.equal(results[0][2], results[1][2])

@@ -1,0 +1,143 @@
+"""The host side of queued steps: ``GraphAtlas`` itself over a device that does what was queued when it is waited for, no sooner.
+Which rows become history, and whose results the host reads."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+import torch
+
+from bitmtp_amd import runtime as R
+from bitmtp_amd.model import StepIO
+
+SIGMA, OTHER, D = 64, 128, 8
+
+
+class Device:
+    """Launches in the order they were queued, on streams that an event orders where the program asks for it."""
+
+    def __init__(self):
+        self.queue, self.step = [], 0
+        self.stream = SimpleNamespace(cuda_stream=1, device_index=0, wait_event=lambda e: None, synchronize=self.run)
+
+    def run(self, until=None):
+        while self.queue and (until is None or until in self.queue):
+            launch = self.queue.pop(0)
+            if callable(launch):
+                launch()
+
+
+class Event:
+    def __init__(self, device):
+        self.device, self.mark = device, None
+
+    def record(self, stream):
+        self.mark = SimpleNamespace(at=self)
+        self.device.queue.append(self.mark)
+
+    def synchronize(self):
+        if self.mark in self.device.queue:
+            self.device.run(self.mark)
+
+
+def token_of(step):
+    return 100 + step
+
+
+@pytest.fixture
+def device(monkeypatch):
+    dev = Device()
+    monkeypatch.setattr(R.torch.cuda, "current_stream", lambda d=None: dev.stream)
+    monkeypatch.setattr(R.torch.cuda, "synchronize", lambda d=None: dev.run())
+
+    def commit(kv, src, dst, n):
+        def launch():
+            kv[:, :, :, dst:dst + n] = kv[:, :, :, src:src + n].clone()
+        dev.queue.append(launch)
+    monkeypatch.setattr(R.decode_ops, "kv_commit", commit)
+    monkeypatch.setattr(R, "_whole_device", R._WholeDevice())
+    dev.commit = commit
+    return dev
+
+
+def _atlas(dev):
+    atlas = R.GraphAtlas.__new__(R.GraphAtlas)
+    atlas.device, atlas.D, atlas.M_max = "cuda:0", D, 32
+    atlas.segment_ladder = (SIGMA, OTHER)
+    atlas.kv_buffers = {s: torch.zeros(2, 1, 1, s + 32, 1, dtype=torch.int32) for s in atlas.segment_ladder}
+    atlas._last = atlas._owed = None
+    atlas.replays = atlas._separate_for = atlas._undisturbed = 0
+    atlas._back_off = atlas.BACK_OFF
+    atlas.dev = dev
+    return atlas
+
+
+def _graph(atlas, M, sigma, role, captured=True, one_launch=True):
+    """As ``GraphAtlas.get_graph`` returns it.  A step leaves its number in its rows of the buffer and ``token_of`` it as its tokens."""
+    dev, kv = atlas.dev, atlas.kv_buffers[sigma]
+    ls, le = R.logits_rows(role, M, D)
+    inputs = torch.zeros(3 * M + 5, dtype=torch.int32)
+    io = StepIO(M=M, step_in=torch.zeros(3 * M + 2, dtype=torch.int32), step_in_host=inputs[:3 * M + 2], inputs_host=inputs,
+                out=torch.zeros(2 * M + 2, dtype=torch.int32), out_host=torch.zeros(2 * M + 2, dtype=torch.int32), uploaded=Event(dev))
+    one = SimpleNamespace(failed=np.zeros(1, dtype=np.int32)) if one_launch else None
+    ring = torch.zeros(R.GraphAtlas.RING, dtype=torch.int32) if M == 1 and role == "ar" else None
+    g = R.CapturedGraph(graph=None, io=io, M=M, sigma=sigma, role=role, P=M - D, logits_start=ls, logits_end=le, one=one,
+                        pending=io.pending(le - ls), ring=ring)
+
+    def layers(outs):
+        dev.step += 1
+        kv[:, :, :, sigma:sigma + M] = dev.step * 100 + torch.arange(M).view(1, 1, 1, M, 1)
+        for out in outs:
+            out[:le - ls] = token_of(dev.step)
+            out[M:M + 2 + le - ls] = 1
+        if ring is not None and len(outs) == 2:   # (a captured one-token step)
+            ring[io.step_in[0] % len(ring)] = token_of(dev.step)
+            io.step_in[0] += 1
+
+    def replay():
+        io.step_in.copy_(io.step_in_host)
+        if role != "ar":                          # step_after
+            src, dst, n = (int(v) for v in inputs[-3:])
+            if n > 0:
+                kv[:, :, :, dst:dst + n] = kv[:, :, :, src:src + n].clone()
+        layers((io.out, io.out_host))
+
+    def further(steps):
+        for _ in range(steps):
+            n = int(io.step_in[0])
+            kv[:, :, :, n - 1] = kv[:, :, :, sigma].clone()
+            layers((io.out, io.out_host))
+    if captured:
+        g.graph = SimpleNamespace(replay=lambda: dev.queue.append(replay))
+        if ring is not None:
+            g.next = {n: SimpleNamespace(replay=lambda n=n: dev.queue.append(lambda: further(n))) for n in R.GraphAtlas.AHEAD}
+    g._eager = lambda one: dev.queue.append(lambda: layers((io.out,)))
+    atlas._one_launch = lambda M: one
+    return g
+
+
+@pytest.mark.parametrize("captured,one_launch", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("M,role", [(1, "ar"), (9, "draft"), (9, "verify"), (16, "draft")])
+def test_rows_left_for_the_next_replay_become_history(device, M, role, captured, one_launch):
+    """With graphs and without, with steps in one launch and separate ones, by a replay of the same segment or another one: the
+    history of commits of their own, by the time that the next step has run."""
+    histories = []
+    for name in ("commit_kv", "commit_with_next"):
+        device.step = 0
+        atlas = _atlas(device)
+        g = _graph(atlas, M, SIGMA, role, captured, one_launch)
+        other = _graph(atlas, 9, OTHER, "verify", captured, one_launch)
+        seen = []
+        for i in range(9):
+            step = other if i % 4 == 2 else g
+            atlas._separate_for = 1 if i == 5 else 0
+            atlas.replay(step, [i] * step.M, list(range(step.M)), 3, 1 if role == "draft" and step is g else 0)
+            device.run()
+            seen.append([atlas.kv_buffers[s][:, :, :, :s].clone() for s in atlas.segment_ladder])
+            rows = min(step.M, 1 + i % 3)
+            getattr(atlas, name)(step.sigma, 4 + 2 * i, rows, min(i % 2, step.M - rows))
+        atlas.synchronize()
+        seen.append([atlas.kv_buffers[s][:, :, :, :s].clone() for s in atlas.segment_ladder])
+        histories.append(seen)
+    for i, (want, got) in enumerate(zip(*histories)):
+        assert all(torch.equal(*pair) for pair in zip(want, got)), f"behind step {i}"
+    assert (histories[0][-1][0] != 0).sum() >= 2 * 6
