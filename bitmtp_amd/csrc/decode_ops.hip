@@ -1158,7 +1158,7 @@ __global__ void __launch_bounds__(256) step_after_kernel(const int32_t *from, in
     const int tid = threadIdx.x;
     // behind the inputs: source and destination slot and number of the rows; one trip over the bus for all of it
     const int at = tid < 3 ? words + tid : tid - 3;
-    if (at < words + 3 && (tid < 3 || blockIdx.x == 0)) {
+    if (tid < 3 || (blockIdx.x == 0 && at < words)) {
         const int32_t v = from_host(from + at);
         if (tid < 3)
             rows[tid] = v;

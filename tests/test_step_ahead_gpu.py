@@ -177,3 +177,17 @@ def test_loops_without_graphs_keep_what_was_verified(loop, kw, monkeypatch):
         assert st["accepted_drafts"] > 9
     assert results[0][:2] == results[1][:2]
     assert torch.equal(results[0][2], results[1][2])
+
+
+@pytest.mark.parametrize("rows", [1, 9, 32])
+def test_inputs_of_a_step_are_all_that_is_written(rows):
+    """``step_in`` in the middle of a larger buffer."""
+    from bitmtp_amd import decode_ops
+    words = 2 + 3 * rows
+    inputs = torch.arange(words + 3, dtype=torch.int32)
+    inputs[-3:] = 0
+    memory = torch.full((words + 64,), -7, dtype=torch.int32, device=DEV)
+    kv = torch.zeros(2, 1, 1, 40, 128, dtype=torch.bfloat16, device=DEV)
+    decode_ops.step_after(inputs.pin_memory(), memory[32:32 + words], torch.zeros(1, dtype=torch.int32, device=DEV), kv)
+    assert torch.equal(memory[32:32 + words].cpu(), inputs[:words])
+    assert (memory[:32] == -7).all() and (memory[32 + words:] == -7).all()
