@@ -145,6 +145,7 @@ class CapturedGraph:
     next: Optional[Dict[int, "torch.cuda.CUDAGraph"]] = None
     ring: Optional[torch.Tensor] = None
     at: int = 0                                         # history length of the last of them
+    ahead: int = 0                                      # how many of them since the last replay
 
 
 class _WholeDevice:
@@ -449,8 +450,9 @@ class GraphAtlas:
         if g.graph is None and g.one is not None:
             g.one = self._one_launch(M)
         separate = g.one is None or self._keeps_separate(g.one)
-        # the previous upload from this pinned buffer must have left the host first (as it has where results came back)
-        if not g.io.arrived:
+        # the previous upload from this pinned buffer must have left the host first (as it has where results came back), and
+        # steps behind the previous replay store their results where this one's are waited for
+        if not g.io.arrived or g.ahead:
             g.io.uploaded.synchronize()
         g.io.step_in_host.numpy()[:] = inputs
         owed = self._owed
@@ -466,6 +468,7 @@ class GraphAtlas:
     def _queue(self, g: CapturedGraph, separate: bool) -> None:
         stream = torch.cuda.current_stream(self.device)
         g.io.arrived = False
+        g.ahead = 0
         if separate:
             self._launch(g, stream, None)
         else:
@@ -491,6 +494,7 @@ class GraphAtlas:
         for _ in range(steps):
             g.at += 1
             g.ring.numpy()[g.at % self.RING] = StepIO.PENDING
+        g.ahead += steps
         stream = torch.cuda.current_stream(self.device)
 
         def launch():
@@ -512,7 +516,6 @@ class GraphAtlas:
                 break
         if g.one is not None and g.one.failed[0] > 1:
             raise RuntimeError("a decode step did not end")
-        g.io.arrived = True   # its inputs have left the host, too
         return int(ring[word])
 
     def verify_drafted(self, g: CapturedGraph, drafted: CapturedGraph, anchor: int, positions: Sequence[int], cache_len: int,
@@ -573,8 +576,10 @@ class GraphAtlas:
 
     def read_outputs(self, g: CapturedGraph) -> Tuple[np.ndarray, np.ndarray, int]:
         """One device-to-host copy + synchronisation: (argmax tokens, confidences,
-        device-side accepted-prefix length) of the projected rows."""
+        device-side accepted-prefix length) of the projected rows; behind ``step_ahead`` those of the last step."""
         if g.io.downloaded:
+            if g.ahead:   # (each stores to the same words)
+                g.io.uploaded.synchronize()
             # The results themselves, as the replay's last launch writes them: the event behind it is ready 7 - 11 us later,
             # and a blocking synchronisation wakes the thread up later still.
             out = g.io.out_host.numpy()

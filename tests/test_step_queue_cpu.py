@@ -31,7 +31,7 @@ class Event:
         self.device, self.mark = device, None
 
     def record(self, stream):
-        self.mark = SimpleNamespace(at=self)
+        self.mark = object()
         self.device.queue.append(self.mark)
 
     def synchronize(self):
@@ -141,3 +141,32 @@ def test_rows_left_for_the_next_replay_become_history(device, M, role, captured,
     for i, (want, got) in enumerate(zip(*histories)):
         assert all(torch.equal(*pair) for pair in zip(want, got)), f"behind step {i}"
     assert (histories[0][-1][0] != 0).sum() >= 2 * 6
+
+
+@pytest.mark.parametrize("steps", [1, 4])
+def test_results_behind_steps_that_nobody_has_read(device, steps):
+    """A replay behind queued steps, one of which has been read: its own token, not one of theirs that is stored late."""
+    atlas = _atlas(device)
+    g = _graph(atlas, 1, SIGMA, "ar")
+    atlas.replay(g, [5], [3], 3)
+    first = g.io.uploaded.mark
+    assert atlas.step_ahead(g, steps) == steps
+    queued = g.io.uploaded.mark
+    device.run(first)
+    assert atlas.read_step(g, 3) == token_of(1)
+    atlas.replay(g, [9], [20], 20)
+    device.run(queued)                            # the older steps end now, if they have not by now
+    tokens, _, _ = atlas.read_outputs(g)
+    assert tokens.tolist() == [token_of(steps + 2)]
+    assert device.step == steps + 2
+
+
+def test_outputs_behind_queued_steps_are_those_of_the_last(device):
+    atlas = _atlas(device)
+    g = _graph(atlas, 1, SIGMA, "ar")
+    atlas.replay(g, [5], [3], 3)
+    first = g.io.uploaded.mark
+    assert atlas.step_ahead(g) == 1
+    device.run(first)
+    assert atlas.read_outputs(g)[0].tolist() == [token_of(2)]
+    assert atlas.read_step(g, 3) == token_of(1) and atlas.read_step(g, 4) == token_of(2)
