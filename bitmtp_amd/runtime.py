@@ -146,6 +146,7 @@ class CapturedGraph:
     ring: Optional[torch.Tensor] = None
     at: int = 0                                         # history length of the last of them
     ahead: int = 0                                      # how many of them since the last replay
+    read: int = 0                                       # history length of the last step whose token the host has read
 
 
 class _WholeDevice:
@@ -483,9 +484,9 @@ class GraphAtlas:
 
     def step_ahead(self, g: CapturedGraph, most: int = 1) -> int:
         """Queue one-token steps behind the last one of ``g``, up to ``most``, each on the token of the one before it and with that
-        one's row committed.  Returns how many; 0 where the step has to wait for the host (``replay``).  Their tokens: ``read_step``, at
-        most ``RING`` behind."""
-        most = min(most, g.sigma - g.at)   # (each commits a row first)
+        one's row committed.  Returns how many; 0 where the step has to wait for the host (``replay``), or the host for a token: there is
+        room for ``RING`` that ``read_step`` has not read."""
+        most = min(most, g.sigma - g.at, self.RING - (g.at - g.read))   # (each commits a row first)
         if g.next is None or self._last is not g or most < 1 or not self._behind(g):
             return 0
         self.settle()
@@ -507,6 +508,9 @@ class GraphAtlas:
 
     def read_step(self, g: CapturedGraph, cache_len: int) -> int:
         """The token of the step of ``g`` over ``cache_len`` slots, once it has arrived."""
+        if not g.at - g.ahead <= cache_len <= g.at or cache_len <= g.at - self.RING:
+            raise ValueError(f"no step over {cache_len} slots is waited for")
+        g.read = max(g.read, cache_len)
         word = cache_len % self.RING
         ring = g.ring.numpy()
         deadline = time.perf_counter() + 0.05
@@ -563,6 +567,7 @@ class GraphAtlas:
             g.io.out_host.numpy()[:] = g.pending
             if g.ring is not None:
                 g.at = int(g.io.step_in_host[0])
+                g.read = g.at - 1
                 g.ring.numpy()[g.at % self.RING] = StepIO.PENDING
             g.graph.replay()          # uploads, runs the step, downloads the results
             g.io.downloaded = True

@@ -170,3 +170,18 @@ def test_outputs_behind_queued_steps_are_those_of_the_last(device):
     device.run(first)
     assert atlas.read_outputs(g)[0].tolist() == [token_of(2)]
     assert atlas.read_step(g, 3) == token_of(1) and atlas.read_step(g, 4) == token_of(2)
+
+
+def test_no_more_tokens_on_their_way_than_there_are_words_for(device):
+    atlas = _atlas(device)
+    g = _graph(atlas, 1, OTHER, "ar")
+    atlas.replay(g, [5], [3], 3)
+    while atlas.step_ahead(g, 7):
+        pass
+    assert g.at - 3 + 1 == atlas.RING
+    for n in range(3, 3 + 2 * atlas.RING):        # each token read makes room for another one
+        assert atlas.read_step(g, n) == token_of(n - 2)
+        assert atlas.step_ahead(g) == 1
+    for n in (2, g.at - atlas.RING, g.at + 1):    # not one of these steps, one whose word is taken, not queued
+        with pytest.raises(ValueError):
+            atlas.read_step(g, n)
