@@ -480,7 +480,7 @@ class GraphAtlas:
     def _behind(self, g: CapturedGraph) -> bool:
         """Whether a step of ``g`` can be queued without its inputs: as the graph of one launch, which separate launches do not stand
         in for."""
-        return g.graph is not None and g.one is not None and self._separate_for == 0 and g.one.failed[0] == 0
+        return g.graph is not None and g.one is not None and self._separate_for == 0 and not self._gave_up(g.one)
 
     def step_ahead(self, g: CapturedGraph, most: int = 1) -> int:
         """Queue one-token steps behind the last one of ``g``, up to ``most``, each on the token of the one before it and with that
@@ -490,7 +490,7 @@ class GraphAtlas:
         if g.next is None or self._last is not g or most < 1 or not self._behind(g):
             return 0
         self.settle()
-        self._keeps_separate(g.one)   # (counts it)
+        self._as_one_launch()
         steps = max(n for n in self.AHEAD if n <= most)
         for _ in range(steps):
             g.at += 1
@@ -540,24 +540,35 @@ class GraphAtlas:
         g.io.inputs_host.numpy()[:] = (step_descriptor(g.role, g.M, self.D, cache_len) + list(positions) + [int(anchor)]
                                        + [-2 ** 31 + i for i in range(g.M - 1)] + [g.sigma, cache_len - n_pend, n_pend])
         if g.one is not None:
-            self._keeps_separate(g.one)   # (counts it)
+            self._as_one_launch()
         self._queue(g, g.one is None)
         return True
 
-    def _keeps_separate(self, one: decode_ops.StepOne) -> bool:
-        """Whether this replay keeps to the separate launches, after a step that did not get the whole device."""
-        if one.failed[0] != 0:
-            if one.failed[0] != 1:
-                raise RuntimeError("a decode step did not end")
-            one.failed[0] = 0
-            self._separate_for, self._back_off = self._back_off, min(2 * self._back_off, 1 << 20)
-            self._undisturbed = 0
-        if self._separate_for > 0:
-            self._separate_for -= 1
-            return True
+    def _gave_up(self, one: decode_ops.StepOne) -> bool:
+        """Whether a step did not get the whole device; separate launches stay for a while then."""
+        failed = int(one.failed[0])   # (read once: the device may set it at any time)
+        if failed == 0:
+            return False
+        if failed != 1:
+            raise RuntimeError("a decode step did not end")
+        one.failed[0] = 0
+        self._separate_for, self._back_off = self._back_off, min(2 * self._back_off, 1 << 20)
+        self._undisturbed = 0
+        return True
+
+    def _as_one_launch(self) -> None:
+        """A step that does not keep to the separate launches."""
         self._undisturbed += 1
         if self._undisturbed == self.BACK_OFF:   # (they may still be queued: one that gives up later is seen then)
             self._back_off = self.BACK_OFF
+
+    def _keeps_separate(self, one: decode_ops.StepOne) -> bool:
+        """Whether this replay keeps to the separate launches."""
+        self._gave_up(one)
+        if self._separate_for > 0:
+            self._separate_for -= 1
+            return True
+        self._as_one_launch()
         return False
 
     def _launch(self, g: CapturedGraph, stream: "torch.cuda.Stream", one: Optional[decode_ops.StepOne]) -> None:

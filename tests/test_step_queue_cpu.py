@@ -185,3 +185,41 @@ def test_no_more_tokens_on_their_way_than_there_are_words_for(device):
     for n in (2, g.at - atlas.RING, g.at + 1):    # not one of these steps, one whose word is taken, not queued
         with pytest.raises(ValueError):
             atlas.read_step(g, n)
+
+
+class GivesUpBetween:
+    """A step's mark that the device sets between two looks of the host."""
+
+    def __init__(self, looks):
+        self.looks, self.value = looks, 0
+
+    def __getitem__(self, i):
+        self.looks -= 1
+        if self.looks < 0:
+            self.value, self.looks = 1, 1 << 30
+        return self.value
+
+    def __setitem__(self, i, value):
+        self.value = value
+
+
+@pytest.mark.parametrize("looks", [0, 1, 2, 3])
+@pytest.mark.parametrize("role", ["ar", "verify"])
+def test_no_step_goes_as_one_launch_once_another_was_seen_to_give_up(device, role, looks):
+    atlas = _atlas(device)
+    draft = _graph(atlas, 9, SIGMA, "draft")
+    g = _graph(atlas, 1 if role == "ar" else 9, SIGMA, role)
+    queued = 0
+    for i in range(6):
+        if i == 1:
+            g.one.failed = GivesUpBetween(looks)
+        if role == "ar":
+            atlas.replay(g, [5], [3], 3)
+            ahead = atlas._separate_for == 0 and atlas.step_ahead(g)
+        else:
+            atlas.replay(draft, [5] * 9, list(range(9)), 3, 1)
+            ahead = atlas.verify_drafted(g, draft, 5, list(range(9)), 4, 1)
+        assert not ahead or atlas._separate_for == 0
+        queued += bool(ahead)
+        device.run()
+    assert queued < 6 and atlas._back_off == 2 * atlas.BACK_OFF
