@@ -211,7 +211,8 @@ class GraphAtlas:
         self._prompt: Optional[PromptBuffers] = None   # sized by the longest block so far
         self._positions: Optional[torch.Tensor] = None
         self._drafted = torch.zeros(max(self.M_max, self.D), dtype=torch.int32, device=self.device)   # the last draft's tokens
-        self._last: Optional[CapturedGraph] = None   # whose replay was the last use of the workspace, as a graph
+        self._last: Optional[CapturedGraph] = None   # whose replay was the last use of the workspace, as a graph,
+        self._last_stream = 0                        # .. and on which stream
         self._owed: Optional[Tuple[int, int, int, int]] = None   # segment, first row, cache_len, rows: see commit_with_next
         self.replays = 0
         # steps of one token and of up to sixteen as one launch (model.step_one), with the weights of the last capture or,
@@ -541,6 +542,9 @@ class GraphAtlas:
                                        + [-2 ** 31 + i for i in range(g.M - 1)] + [g.sigma, cache_len - n_pend, n_pend])
         if g.one is not None:
             self._as_one_launch()
+        stream = torch.cuda.current_stream(self.device)
+        if stream.cuda_stream != self._last_stream:
+            stream.wait_event(drafted.io.uploaded)
         self._queue(g, g.one is None)
         return True
 
@@ -582,7 +586,7 @@ class GraphAtlas:
                 g.ring.numpy()[g.at % self.RING] = StepIO.PENDING
             g.graph.replay()          # uploads, runs the step, downloads the results
             g.io.downloaded = True
-            self._last = g
+            self._last, self._last_stream = g, stream.cuda_stream
         else:
             self._last = None
             g.io.step_in.copy_(g.io.step_in_host, non_blocking=True)

@@ -65,6 +65,7 @@ def _atlas(dev):
     atlas.segment_ladder = (SIGMA, OTHER)
     atlas.kv_buffers = {s: torch.zeros(2, 1, 1, s + 32, 1, dtype=torch.int32) for s in atlas.segment_ladder}
     atlas._last = atlas._owed = None
+    atlas._last_stream = 0
     atlas.replays = atlas._separate_for = atlas._undisturbed = 0
     atlas._back_off = atlas.BACK_OFF
     atlas.dev = dev
@@ -223,3 +224,17 @@ def test_no_step_goes_as_one_launch_once_another_was_seen_to_give_up(device, rol
         queued += bool(ahead)
         device.run()
     assert queued < 6 and atlas._back_off == 2 * atlas.BACK_OFF
+
+
+@pytest.mark.parametrize("draft_one,verify_one", [(True, True), (True, False), (False, True), (False, False)])
+def test_a_verification_on_another_stream_waits_for_its_draft(device, draft_one, verify_one):
+    atlas = _atlas(device)
+    draft, g = _graph(atlas, 16, SIGMA, "draft", one_launch=draft_one), _graph(atlas, 9, SIGMA, "verify", one_launch=verify_one)
+    waits = []
+    for other in (device.stream, SimpleNamespace(cuda_stream=2, device_index=0, wait_event=waits.append)):
+        first = device.stream
+        atlas.replay(draft, [5] * 16, list(range(16)), 3, 1)
+        device.stream = other
+        assert atlas.verify_drafted(g, draft, 5, list(range(9)), 4, 1)
+        device.run()
+        assert (draft.io.uploaded in waits) == (other is not first)
