@@ -397,7 +397,8 @@ void launch_row_quant(const void *x, int8_t *q, float *s, int M, int K, hipStrea
     }
 }
 
-bool order_ok(int M, int K) { return M >= 1 && K >= 128 && K % 128 == 0 && K <= kMaxProducerK; }
+static_assert(BONSAI_ORDERED_MAX_K == kMaxProducerK, "what a product in operand order takes can be quantised so");
+bool order_ok(int M, int K) { return M >= 1 && K >= 128 && K % 128 == 0 && K <= BONSAI_ORDERED_MAX_K; }
 
 }  // namespace
 

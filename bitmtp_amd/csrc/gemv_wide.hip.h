@@ -60,6 +60,7 @@
 
 #include <type_traits>
 
+#include "../../include/bonsai_gemv.h"
 #include "gemv_mxl.hip.h"
 
 namespace bonsai {
@@ -763,6 +764,7 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus, bool ordered 
 template <int BITS>
 bool wide_fits(int v, int K, int lds_limit, bool ordered = false) {
     const WideVariant &k = wide_of<BITS>(v, ordered);
+    if (ordered && K > BONSAI_ORDERED_MAX_K) return false;  // (no quantiser writes such rows)
     return k.lds(K, false) <= (size_t)lds_limit && (long)k.rows * K <= (1L << 30) && (long)k.tokens * K <= (1L << 30);
 }
 

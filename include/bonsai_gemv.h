@@ -96,14 +96,16 @@ int t2g128_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *
 int q1g128_gemv_silu(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K,
                      void *stream);
 
+/* Longest row that the quantisers write in operand order. */
+#define BONSAI_ORDERED_MAX_K 65536
+
 /* bf16 results on bf16 scales from activations in OPERAND ORDER, the order in which the matrix cores of wide T2 blocks take them
  * (bonsai_act_quant_ordered and bonsai_norm_quant_ordered write it): every 16 activations of a token as the four
  * dwords {e, e + 4, e + 8, e + 12}, e = 0 .. 3.  silu: as *_gemv_silu.
- * -1, and nothing launched, where another kernel than the wide one is expected to be faster (*_gemv_ex and *_gemv_silu take the
- * activations in their own order).  ask: the answer (0 or -1) without the launch.  Same results as from the other order. */
+ * -1, and nothing launched, where another kernel than the wide one is expected to be faster or K is above BONSAI_ORDERED_MAX_K
+ * (*_gemv_ex and *_gemv_silu take the activations in their own order).  ask: the answer (0 or -1) without the launch.  Same results as from the other order. */
 int t2g128_gemv_ordered(const int8_t *A, const uint8_t *B, void *out, const float *s, const void *ws, int M, int N, int K, int silu,
                         int ask, void *stream);
-
 
 /* ---- several GEMVs in one launch ------------------------------------------ */
 /* No counterpart in the reference, which launches one kernel per projection
@@ -228,7 +230,7 @@ int bonsai_add_rmsnorm_quant_int8(const void *x, const void *residual, const voi
                                   void *h_out, int8_t *q, float *s, int M, int K, void *stream);
 
 /* The two above (x bf16; residual and h_out NULL: no addition) and bonsai_act_quant_int8 (x bf16) with q in operand order
- * (t2g128_gemv_ordered): the same bytes, moved within 16 of a token.  K a multiple of 128. */
+ * (t2g128_gemv_ordered): the same bytes, moved within 16 of a token.  K a multiple of 128, at most BONSAI_ORDERED_MAX_K. */
 int bonsai_norm_quant_ordered(const void *x, const void *residual, const void *w, float eps, void *h_out, int8_t *q, float *s, int M,
                               int K, void *stream);
 int bonsai_act_quant_ordered(const void *x, int8_t *q, float *s, int M, int K, void *stream);
