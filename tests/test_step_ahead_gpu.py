@@ -1,5 +1,7 @@
 """Steps queued behind steps whose results the host has not seen: one-token steps one after the other, a verification behind its
 draft, and results that a captured step stores to pinned memory itself."""
+import itertools
+
 import numpy as np
 import pytest
 import torch
@@ -58,6 +60,95 @@ def test_a_step_that_gave_up_with_others_behind_it(loop):
     assert len(out) == 12 and atlas._separate_for > 0 and out[0] == want[0]
     atlas._separate_for = 0
     assert fn(atlas, prompt, max_gen_len=12)[0] == want
+
+
+def _disturbed(one, launches):
+    """``launches`` on a device that is still busy, the first one a step of ``one`` that does not get all of it."""
+    one.failed[0] = 0
+    torch.cuda._sleep(5000000)   # (nothing has begun when the last one is queued)
+    one.exchange[4:8].view(torch.int32).fill_(1)
+    return launches()
+
+
+def _successors(ladder, **kw):
+    """An atlas whose model has another token behind each token than itself (the tied head of ``_model`` repeats its input)."""
+    from bitmtp_amd.runtime import GraphAtlas
+    model = _model(2, 1024, 512, 8, 4)
+    model.embed = torch.roll(model.embed, 37, 0)
+    return GraphAtlas(model, segment_ladder=ladder, **kw)
+
+
+def _random_history(atlas, sigma):
+    kv = atlas.kv(sigma)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    return kv, (torch.randn(tuple(kv.shape), generator=gen, device=DEV) * 0.5).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("steps", [1, 4])
+def test_steps_behind_one_that_was_done_again(steps):
+    """They go on from its token and with its row in the history: to the bit what steps give that wait for each other."""
+    sigma, n = 256, 20
+    atlas = _successors((sigma,))
+    g, (kv, hist) = atlas.get_graph(1, sigma, "ar"), _random_history(atlas, sigma)
+
+    def step(token, at):
+        atlas.replay(g, [token], [at], at)
+        return int(atlas.read_outputs(g)[0][0])
+
+    kv.copy_(hist)
+    tokens, rows = [_disturbed(g.one, lambda: step(5, n))], [kv[:, :, :, sigma].clone()]
+    torch.cuda.synchronize()
+    assert g.one.failed[0] == 1
+    g.one.failed[0] = 0
+    for i in range(1, steps + 1):
+        atlas.commit_kv(sigma, n + i - 1, 1)
+        tokens.append(step(tokens[-1], n + i))
+        rows.append(kv[:, :, :, sigma].clone())
+    assert g.one.failed[0] == 0 and len(set([5] + tokens)) == steps + 2
+    kv.copy_(hist)
+
+    def queue():
+        atlas.replay(g, [5], [n], n)
+        assert atlas.step_ahead(g, steps) == steps
+    _disturbed(g.one, queue)
+    assert [atlas.read_step(g, n + i) for i in range(steps + 1)] == tokens
+    torch.cuda.synchronize()
+    assert g.one.failed[0] == 1
+    for i, row in enumerate(rows):
+        assert torch.equal(kv[:, :, :, n + i if i < steps else sigma], row), f"row of step {i}"
+
+
+def test_a_verification_behind_a_draft_that_was_done_again():
+    sigma, n, pending, mask = 256, 20, 5, 999
+    atlas = _successors((sigma,))
+    draft, verify = atlas.get_graph(9, sigma, "draft"), atlas.get_graph(9, sigma, "verify")
+    kv, hist = _random_history(atlas, sigma)
+    block = ([pending, pending] + [mask] * 7, [n] + [n + i for i in range(8)], n, 1)
+    positions = [n + i for i in range(9)]
+    assert draft.one is verify.one
+    kv.copy_(hist)
+    _disturbed(draft.one, lambda: atlas.replay(draft, *block))
+    want = [atlas.read_outputs(draft)]
+    torch.cuda.synchronize()
+    assert draft.one.failed[0] == 1
+    draft.one.failed[0] = 0
+    atlas.commit_kv(sigma, n, 1)
+    atlas.replay(verify, [pending] + [int(t) for t in want[0][0][:8]], positions, n + 1)
+    want.append(atlas.read_outputs(verify))
+    after = kv.clone()
+    assert draft.one.failed[0] == 0
+    kv.copy_(hist)
+
+    def queue():
+        atlas.replay(draft, *block)
+        assert atlas.verify_drafted(verify, draft, pending, positions, n + 1, 1)
+    _disturbed(draft.one, queue)
+    got = [atlas.read_outputs(draft), atlas.read_outputs(verify)]
+    torch.cuda.synchronize()
+    assert draft.one.failed[0] == 1
+    for (x, y) in zip(want, got):
+        assert all(np.array_equal(a, b) for a, b in zip(x, y))
+    assert torch.equal(kv, after)
 
 
 def test_steps_that_have_to_wait_for_the_host():
@@ -167,14 +258,14 @@ def test_results_in_pinned_memory_are_those_on_the_device(width, role):
 def test_loops_without_graphs_keep_what_was_verified(loop, kw, monkeypatch):
     """Verifications that accept drafts: the tokens and the history of the loop whose steps are graphs."""
     from bitmtp_amd import generate
-    monkeypatch.setattr(generate, "verify_accept", lambda draft, verify, D: int(draft[0]) % 4)   # (random weights agree on few)
-    model, prompt, results = _model(2, 1024, 512, 8, 4), list(range(3, 33)), []
-    from bitmtp_amd.runtime import GraphAtlas
+    prompt, results = list(range(3, 33)), []
     for use_graphs in (True, False):
-        atlas = GraphAtlas(model, segment_ladder=(64, 256), use_graphs=use_graphs)
+        accepted = itertools.cycle((2, 0, 3, 7))   # (random weights agree on few)
+        monkeypatch.setattr(generate, "verify_accept", lambda draft, verify, D: next(accepted))
+        atlas = _successors((64, 256), use_graphs=use_graphs)
         out, st = getattr(generate, loop + "_generate")(atlas, prompt, max_gen_len=60, **kw)
         results.append((out, st["accepted_drafts"], _history(atlas, len(prompt) + len(out) - 10)))
-        assert st["accepted_drafts"] > 9
+        assert st["accepted_drafts"] > 9 and len(set(out)) > 2
     assert results[0][:2] == results[1][:2]
     assert torch.equal(results[0][2], results[1][2])
 
