@@ -18,8 +18,8 @@
 //     They run as a pipeline (gemv_wide_kernel): waves that keep step at the barriers otherwise all read LDS, all
 //     multiply and all add at the same time.  64 x 64 a wave without it before -> now: 2560 x 9728 at 3001 tokens 94 -> 87 us,
 //     2560 x 4096 45 -> 41, 2560 x 9728 at 2048 91 -> 78; 12288 x 2048 at 514 (64 x 256 tiles then) 24.7 -> 23.5.
-// Back to back on random bytes, with 16 x 16 instructions before -> now: 19456 x 2560 at 3001 tokens 254 -> 194 us
-// (1.54 POP/s; PyTorch's int8 product reaches 1.99 at 16384^3), 2560 x 9728 123 -> 87,
+// Back to back on random bytes, activations in their own order, with 16 x 16 instructions before -> now: 19456 x 2560 at 3001 tokens
+// 254 -> 194 us (1.54 POP/s; PyTorch's int8 product reaches 1.99 at 16384^3), 2560 x 9728 123 -> 87,
 // 12288 x 2048 at 514 35 -> 23.5, at 256 19.6 -> 16.7, 2048 x 2048 at 256 7.1 -> 6.6.
 //
 //   WM x WN waves share a staged block of WM*MT*32 tokens x WN*NT*32 rows; KS such sets of waves
@@ -28,16 +28,16 @@
 //
 // Activations that a quantiser has left in operand order (ORDERED: a prompt's) go from memory to LDS without passing
 // registers, and nothing is transposed here: once per weight row tile it was, and is once now, by the quantiser.
-// From -> to operand order on the same tile, us at 3001 tokens: 6144 x 2560 72 -> 65, 19456 x 2560 197 -> 180, 2560 x 4096 42 -> 40,
-// 2560 x 9728 88 -> 83; at 256: 12288 x 2048 16.1 -> 14.3, 4096 x 2048 8.6 -> 7.6, 2048 x 6144 12.0 -> 10.5, 2048 x 2048 6.3 -> 5.7.
-// With its own tiles, within a prompt: at 3001 tokens 71.6 -> 59.5, with SiLU 198 -> 176.5 (1.69 POP/s), 46.2 -> 38.7, 98 -> 80 (1.87);
-// at 256 with SiLU 18.1 -> 15.3, 10.1 -> 8.6, 13.8 -> 12.6, 7.1 -> 6.8.
+// Own order -> operand order, each on its own tiles, within a prompt, us: at 3001 tokens 6144 x 2560 71.6 -> 59.5, 19456 x 2560 with SiLU
+// 198 -> 176.5 (1.69 POP/s), 2560 x 4096 46.2 -> 38.7, 2560 x 9728 98 -> 80 (1.87); at 256 12288 x 2048 with SiLU 18.1 -> 15.3,
+// 4096 x 2048 10.1 -> 8.6, 2048 x 6144 13.8 -> 12.6, 2048 x 2048 7.1 -> 6.8.
 //
-// Per group a set stages 128 bytes of K for its tokens (4 x 4 byte transposes: operand order, see
-// gemv_core.h; 16-byte units XORed with half the row number, so that a ds_read_b128 of 16 rows meets
-// every bank once) and the packed rows, inverted where the unpacking wants it (a wave's operand read is
-// 512 or 1024 contiguous bytes).  The loads of group g + 2 are in flight and group g + 1 is being parked
-// while group g is multiplied: one barrier per group, none where a set is a single wave.  All scales of
+// Per group a set stages 128 bytes of K for its tokens (16-byte units XORed with half the row number, so that a ds_read_b128 of
+// 16 rows meets every bank once) and the packed rows (a wave's operand read is 512 or 1024 contiguous bytes).  In their own order
+// activations pass registers (4 x 4 byte transposes: operand order, see gemv_core.h), and rows are inverted there where the
+// unpacking wants it: the loads of group g + 2 are in flight and group g + 1 is being parked while group g is multiplied.  In
+// operand order group g + 1 is on its way, with three buffers g + 2 as well, and rows are inverted behind their read.  One barrier
+// per group, none where a set is a single wave.  All scales of
 // the row block (G x rows, transposed), the multipliers and their reciprocals are staged once.  Rows past
 // N and tokens past M read as zero through the buffer range check.
 //
@@ -759,8 +759,8 @@ inline double wide_estimate(int v, int M, int N, int K, int n_cus, bool ordered 
 }
 
 // Whether variant v takes rows of K weights: all scales of its row block are staged at once, 2 bytes per row and group,
-// so that 64x128_K4 and 128x256 stop at K = 23,808, 64x256 at 32,384 and 64x128_K2 at 56,576 (160 KB of LDS), and
-// its offsets are 32-bit.
+// so that 64x128_K4 and 128x256 stop at K = 23,808, 64x256 at 32,384 and 64x128_K2 at 56,576 (160 KB of LDS; the other tiles of
+// ordered activations take all rows that there are), and its offsets are 32-bit.
 template <int BITS>
 bool wide_fits(int v, int K, int lds_limit, bool ordered = false) {
     const WideVariant &k = wide_of<BITS>(v, ordered);

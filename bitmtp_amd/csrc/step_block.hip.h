@@ -25,7 +25,8 @@
 // LDS in the order of K.
 //
 // The rows of q|k|v are dealt out by kv head, so that the hand-over to the attention stays within a die (near_heads of
-// step_one.hip.h): nine rows 610 -> 594 us (1.7B shape), 1006 -> 992 (4B), sixteen 661 -> 636.
+// step_one.hip.h): nine rows 610 -> 594 us (1.7B shape), 1006 -> 992 (4B), sixteen 661 -> 636, of which the near stores are 6 and 11 us
+// at nine rows.
 //
 // Layers of nine rows, 1.7B / 4B shape, us at a history of 24, 300, 1500: 934 / 961 / 1034 -> 590 / 645 / 761 and
 // 1521 / 1543 / 1657 -> 988 / 1092 / 1289; two rows (1.7B) 812 / 818 / 900 -> 539 / 581 / 702; sixteen 987 / 1011 / 1089 ->
@@ -71,8 +72,8 @@ constexpr int kMostLds = 159 * 1024;        // beside what is declared in place
 constexpr uint32_t kEmpty = 0x80808080u;    // int8 rows hold no -128, a multiplier is positive
 constexpr int kCopies = 8;                  // of the multipliers' line, one for each XCD's workgroups
 constexpr int kNap = 1;                     // of 64 cycles, between two looks
-// .. and before a row's workgroup looks for its row (27 ns each): none 593, 10 588, 20 589 us a nine-row step (1.7B shape), 991,
-// 984 and 993 with the 4B one.
+// .. and before a row's workgroup looks for its row (27 ns each): none 593, 10 588, 20 589 us a nine-row step (1.7B shape, 24 slots), 991,
+// 984 and 993 with the 4B one; none and 10 level at 300 and 900 slots, and at all three with 1024 x 3072 and 2304 x 6400.
 constexpr int kPause = 10;
 constexpr int kVPitch = 272, kOPitch = 132; // bytes of a slot's values, floats of a row's sums in LDS
 

@@ -14,7 +14,8 @@
 //     and a pause before the first poll;
 //   * q|k|v's rows are dealt out by kv head, so that the hand-over to the attention, and of its parts, stays within a die's
 //     L2 (near_heads): 0.2 us instead of 0.6 between two workgroups.  With the pauses that fit it the 1.7B shape takes 379 /
-//     432 / 483 us at a history of 24 / 300 / 1500 (before: 386 / 455 / 517), the 4B one 698 / 771 / 871 (720 / 803 / 902);
+//     432 / 483 us at a history of 24 / 300 / 1500 (before: 386 / 455 / 517), the 4B one 698 / 771 / 871 (720 / 803 / 902).  At 300
+//     slots, us without both / near alone / the pauses alone / both: 451 / 448 / 439 / 426 and 814 / 811 / 773 / 764;
 //   * what needs a value of the whole row (the norm's sum of squares, the maximum the quantisation scales by) is computed
 //     by every workgroup from the row it has read anyway.
 // What bounds it now is the length of the chain: per phase a hand-over, about 0.8 us for norm and quantisation, 0.5 us
@@ -59,7 +60,10 @@ constexpr uint32_t kRunTicks = 20000000;   // 200 ms
 // others on their way, and delays what it looks for; one that comes too late costs what it is late by.  By sweep, us a step at a
 // history of 24 / 300 / 900, from 8 (10 for the attention's row and the down projection's) everywhere: gate|up's row 12 steps and
 // the down projection's 18 382 / 439 / 458 -> 377 / 431 / 438 (1.7B shape), 729 / 802 / 854 -> 705 / 779 / 830 (4B); q|k|v's row
-// 12 level and 698 / 772 / 825, 16 1 % behind and 692 / 766 / 817; two more or fewer of any: within 1 %.
+// 12 level and 698 / 772 / 825, 16 1 % behind and 692 / 766 / 817; two more or fewer of any: within 1 %.  They are numbers that
+// fit these two shapes: how long others take depends on every row, and only the norm's pause follows one.  On two other shapes each
+// of them is within 1 % of the best at any of those histories (1024 x 3072 352 / 404 / 407, 2304 x 6400 542 / 594 / 636; from 8 and 10
+// everywhere 361 / 422 / 433 and 547 / 606 / 649).
 constexpr int kPauseHead = 4, kPauseParts = 2;   // near hand-overs
 constexpr int kPauseAtt = 10, kPauseH2 = 12, kPauseInner = 18;
 __host__ __device__ constexpr int pause_row(int words) { return 8 + 4 * words; }   // words a lane of a row of dim
@@ -263,8 +267,9 @@ __device__ __forceinline__ void hand_over_near(const __amdgpu_buffer_rsrc_t set,
         __builtin_amdgcn_raw_buffer_store_b32(d, set, off, row, kDeviceScope);
 }
 // Workgroups go round the dies in the order of their numbers, so that those of a kv head (n_kv a multiple of eight) share
-// one.  The exchange memory's reset has looked whether they do (dies_kernel), and a workgroup that is not where it was then
-// stores past its L2, which all see.
+// one.  The exchange memory's reset has looked whether they do (dies_kernel).  A workgroup that is not where it was then
+// stores past its L2, which all see; what the others leave in theirs it does not see, and a step in which it would have to
+// ends at its limit and is done again (step_finish.hip.h).
 __device__ __forceinline__ bool near_heads(const __attribute__((address_space(4))) uint32_t *control, int wg) {
     uint32_t die;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(die));
