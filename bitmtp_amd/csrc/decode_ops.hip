@@ -1140,9 +1140,10 @@ constexpr int kCommitGroups = 32;   // 8192 threads: a row of the 1.7B shape is 
 __device__ __forceinline__ void commit_rows(uint4 *kv, int planes, int slots, int src, int dst, int n) {
     if (n <= 0 || src < 0 || dst < 0 || n > slots || src > slots - n || dst > slots - n) return;
     constexpr int kPieces = kHd * 2 / 16;
-    const int per_plane = n * kPieces;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < planes * per_plane; i += kCommitGroups * 256) {
-        const int plane = i / per_plane, off = i - plane * per_plane;
+    if ((int64_t)planes * n * kPieces > 0x7fffffff) return;   // (as bonsai_kv_commit)
+    const uint32_t per_plane = (uint32_t)(n * kPieces), all = (uint32_t)planes * per_plane;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < all; i += kCommitGroups * 256) {
+        const uint32_t plane = i / per_plane, off = i - plane * per_plane;
         uint4 *base = kv + (size_t)plane * slots * kPieces;
         base[(size_t)dst * kPieces + off] = base[(size_t)src * kPieces + off];
     }
@@ -2084,7 +2085,7 @@ extern "C" int bonsai_kv_commit(void *kv, int n_layers, int n_kv, int slots, int
 }
 
 static bool kv_planes_ok(const void *kv, int n_layers, int n_kv, int slots) {
-    return kv && n_layers >= 1 && n_kv >= 1 && slots >= 1 && 2LL * n_layers * n_kv * slots * (kHd * 2 / 16) <= 0x7fffffffLL;
+    return kv && n_layers >= 1 && n_kv >= 1 && slots >= 1 && 2LL * n_layers * n_kv * (kHd * 2 / 16) <= 0x7fffffffLL;   // a row's pieces
 }
 
 extern "C" int bonsai_step_next(const int32_t *step_in, void *kv, int n_layers, int n_kv, int slots, int sigma, void *stream) {

@@ -221,7 +221,7 @@ int bonsai_kv_commit(void *kv, int n_layers, int n_kv, int slots, int src_slot, 
  * shared buffer, becomes history slot step_in[0] - 1.
  * bonsai_step_after: copies the 2 + 3 * rows step inputs from `from` (pinned host memory, read when the launch runs) to step_in,
  * a token INT32_MIN + i as drafted[i] (i < drafts), and the three words behind them {src slot, dst slot, n} as bonsai_kv_commit does
- * (n <= 0 or slots outside the buffer: nothing). */
+ * (n <= 0, slots outside the buffer or more than bonsai_kv_commit takes: nothing). */
 int bonsai_step_next(const int32_t *step_in, void *kv, int n_layers, int n_kv, int slots, int sigma, void *stream);
 int bonsai_step_after(const int32_t *from, int32_t *step_in, int rows, const int32_t *drafted, int drafts, void *kv, int n_layers,
                       int n_kv, int slots, void *stream);

@@ -1,4 +1,4 @@
-"""What ``step_after_kernel`` writes, thread by thread on the CPU: the step inputs, words beside them not."""
+"""What ``step_after_kernel`` writes, thread by thread on the CPU: the step inputs, words beside them not.  Which buffers it takes."""
 import ctypes
 import os
 import re
@@ -29,6 +29,7 @@ extern "C" void run(const int32_t *from, int32_t *to, int words, const int32_t *
             for (threadIdx.x = 0; threadIdx.x < 256; ++threadIdx.x)
                 step_after_kernel(from, to, words, drafted, drafts, (uint4 *)kv, planes, slots);
 }
+extern "C" int planes_ok(const void *kv, int n_layers, int n_kv, int slots) { return kv_planes_ok(kv, n_layers, n_kv, slots); }
 """
 
 
@@ -37,11 +38,11 @@ def step_after(tmp_path_factory):
     src = open(os.path.join(os.path.dirname(__file__), "..", "bitmtp_amd", "csrc", "decode_ops.hip")).read()
     body = [re.search(what, src, re.S | re.M).group(0) for what in (
         r"^constexpr int kCommitGroups = .*?$", r"^__device__ __forceinline__ void commit_rows\(.*?^\}",
-        r"^__global__ [^\n]*step_after_kernel\(.*?^\}")]
+        r"^__global__ [^\n]*step_after_kernel\(.*?^\}", r"^static bool kv_planes_ok\(.*?^\}")]
     out = tmp_path_factory.mktemp("step_after")
     (out / "t.cpp").write_text(STUBS + "\n".join(body) + RUN)
     subprocess.run(["g++", "-O1", "-shared", "-fPIC", str(out / "t.cpp"), "-o", str(out / "t.so")], check=True)
-    return ctypes.CDLL(str(out / "t.so")).run
+    return ctypes.CDLL(str(out / "t.so"))
 
 
 @pytest.mark.parametrize("rows", [1, 2, 9, 16, 31, 32])
@@ -57,8 +58,29 @@ def test_words_beside_the_inputs_stay(step_after, rows):
     want = kv.copy()
     want[:, 5:8] = kv[:, 20:23]
     p = lambda a: a.ctypes.data_as(ctypes.c_void_p)   # noqa: E731
-    step_after(p(inputs), p(memory[20:]), words, p(drafted), len(drafted), p(kv), planes, slots)
+    step_after.run(p(inputs), p(memory[20:]), words, p(drafted), len(drafted), p(kv), planes, slots)
     got = memory[20:20 + words]
     assert np.array_equal(got[:words - rows + 1], inputs[:words - rows + 1]) and np.array_equal(got[words - rows + 1:], drafted[:rows - 1])
     assert (memory[:20] == -7).all() and (memory[20 + words:] == -7).all()
     assert np.array_equal(kv, want)
+
+
+@pytest.mark.parametrize("n_layers,n_kv,slots,ok", [
+    (36, 8, 240000, True),            # 4B shape: 2 ** 31 pieces of 16 bytes and more
+    (28, 8, 1 << 22, True),           # the longest segment that steps take
+    (2 ** 25, 1, 1, True), (2 ** 26, 1, 1, False), (2 ** 20, 2 ** 12, 1, False),   # a row's pieces are counted in 32 bits
+    (0, 8, 64, False), (36, 0, 64, False), (36, 8, 0, False)])
+def test_buffers_of_any_length_are_taken(step_after, n_layers, n_kv, slots, ok):
+    assert step_after.planes_ok(ctypes.c_void_p(64), n_layers, n_kv, slots) == ok
+    assert not step_after.planes_ok(None, n_layers, n_kv, slots)
+
+
+def test_more_pieces_than_are_counted_are_not_committed(step_after):
+    """As ``bonsai_kv_commit`` refuses them."""
+    words, planes, slots, n = 5, 576, 600000, 233017   # n * planes * 16 just above 2 ** 31
+    inputs = np.array([1, 2, 3, 4, 5, 300000, 0, n], dtype=np.int32)
+    to, drafted = np.zeros(words, dtype=np.int32), np.zeros(1, dtype=np.int32)
+    kv = np.full(4096, 7, dtype=np.int32)             # nothing beside its start would be there
+    p = lambda a: a.ctypes.data_as(ctypes.c_void_p)   # noqa: E731
+    step_after.run(p(inputs), p(to), words, p(drafted), 1, p(kv), planes, slots)
+    assert (kv == 7).all() and np.array_equal(to, inputs[:words])

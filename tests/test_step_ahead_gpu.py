@@ -282,3 +282,21 @@ def test_inputs_of_a_step_are_all_that_is_written(rows):
     decode_ops.step_after(inputs.pin_memory(), memory[32:32 + words], torch.zeros(1, dtype=torch.int32, device=DEV), kv)
     assert torch.equal(memory[32:32 + words].cpu(), inputs[:words])
     assert (memory[:32] == -7).all() and (memory[32 + words:] == -7).all()
+
+
+def test_rows_are_committed_in_buffers_of_more_than_32_gib():
+    """One that the graphs of a long segment have: its last planes, by both launches."""
+    from bitmtp_amd import decode_ops
+    slots = 240032
+    kv = torch.empty(2, 36, 8, slots, 128, dtype=torch.bfloat16, device=DEV)
+    rows = torch.arange(2 * 36 * 8 * 2 * 128, device=DEV).remainder(251).to(torch.bfloat16).view(2, 36, 8, 2, 128)
+    kv[:, :, :, 240000:240002] = rows
+    step_in = torch.zeros(5, dtype=torch.int32, device=DEV)
+    inputs = torch.tensor([1, 2, 3, 4, 5, 240000, 239000, 2], dtype=torch.int32).pin_memory()
+    decode_ops.step_after(inputs, step_in, torch.zeros(1, dtype=torch.int32, device=DEV), kv)
+    assert torch.equal(kv[:, :, :, 239000:239002], rows) and step_in.tolist() == [1, 2, 3, 4, 5]
+    step_in[0] = 777
+    decode_ops.step_next(step_in, kv, 240000)
+    assert torch.equal(kv[:, :, :, 776:777], rows[:, :, :, :1])
+    del kv
+    torch.cuda.empty_cache()
