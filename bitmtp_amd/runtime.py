@@ -273,8 +273,8 @@ class GraphAtlas:
         that ``kv`` returned earlier is behind until then."""
         if n_accept <= 0:
             return
-        if cache_len + n_accept > sigma:
-            raise RuntimeError("KV commit would run past the history segment")
+        if sigma not in self.kv_buffers or not 0 <= cache_len <= sigma - n_accept or not 0 <= first_row <= self.M_max - n_accept:
+            return self.commit_kv(sigma, cache_len, n_accept, first_row)   # (refuses what cannot be)
         self.settle()
         self._owed = (sigma, first_row, cache_len, n_accept)
 

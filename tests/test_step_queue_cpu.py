@@ -50,6 +50,9 @@ def device(monkeypatch):
     monkeypatch.setattr(R.torch.cuda, "synchronize", lambda d=None: dev.run())
 
     def commit(kv, src, dst, n):
+        if min(src, dst) < 0 or max(src, dst) + n > kv.shape[3]:
+            raise RuntimeError("bonsai_kv_commit failed")
+
         def launch():
             kv[:, :, :, dst:dst + n] = kv[:, :, :, src:src + n].clone()
         dev.queue.append(launch)
@@ -142,6 +145,19 @@ def test_rows_left_for_the_next_replay_become_history(device, M, role, captured,
     for i, (want, got) in enumerate(zip(*histories)):
         assert all(torch.equal(*pair) for pair in zip(want, got)), f"behind step {i}"
     assert (histories[0][-1][0] != 0).sum() >= 2 * 6
+
+
+@pytest.mark.parametrize("sigma,cache_len,n,first_row", [(SIGMA, -1, 1, 0), (SIGMA, 60, 5, 0), (SIGMA, 3, 1, 32),
+                                                         (SIGMA, 3, 9, 24), (SIGMA + 1, 3, 1, 0)])
+def test_commits_that_cannot_be_are_refused_at_once(device, sigma, cache_len, n, first_row):
+    """As a commit of its own refuses them; the one before is still to come."""
+    atlas = _atlas(device)
+    atlas.commit_with_next(SIGMA, 4, 2, 1)
+    with pytest.raises((RuntimeError, KeyError)):
+        atlas.commit_with_next(sigma, cache_len, n, first_row)
+    atlas.kv_buffers[SIGMA][:, :, :, SIGMA:] = 7
+    atlas.synchronize()
+    assert atlas._owed is None and (atlas.kv_buffers[SIGMA][:, :, :, :SIGMA].flatten(0, 3) == 7).sum() == 2 * 2
 
 
 @pytest.mark.parametrize("steps", [1, 4])
