@@ -1133,8 +1133,9 @@ __global__ void __launch_bounds__(256) kv_commit_kernel(uint4 *kv, int planes, i
 //                       launch has advanced (DraftExtra::step)
 //   step_after_kernel   a block that verifies a drafted one: inputs from pinned host memory, marked tokens (INT32_MIN + i)
 //                       from the draft, and the commit of the draft's pending rows
-// 4.6 and 6.1 us each in a decode run (1.7B shape).  64 tokens greedily behind a short prompt 28641 us without them, 28397 with one step to a graph (14 us pass
-// between two graphs, also of one stream) and 27792 with four; 48 speculatively 36380 and, both blocks' commits here, 35800 - 35980.
+// 4.6 and 6.1 us each in a decode run (1.7B shape).  64 tokens greedily behind a short prompt 28641 us without them, 28397 with one
+// step to a graph (14 us pass between two graphs, also of one stream) and 27792 with four; 48 speculatively 36370, with the
+// verification queued behind its draft 36160, with verified rows committed by the next block's launch 36120, with both 35900.
 // ---------------------------------------------------------------------------
 constexpr int kCommitGroups = 32;   // 8192 threads: a row of the 1.7B shape is 7168 pieces of 16 bytes, of the 4B one 9216
 __device__ __forceinline__ void commit_rows(uint4 *kv, int planes, int slots, int src, int dst, int n) {
